@@ -13,6 +13,11 @@
 //     works on ONE 16-pair block at a time -- the block's rows, its columns of W[k] and the next block's rows are
 //     all it holds -- so it stays far below 128 registers and a SIMD holds four waves: while one waits for rows
 //     or adds a block into its partial tile, the matrix core runs the others' blocks.
+//   * With few rows a tile per unit would be short (2 259 rows: 9), its pair lists mostly padding, and every unit would
+//     still read all 442 KB of W for it.  Up to 10 240 rows on 256 units two, up to 3 072 rows four workgroups share a
+//     tile, each taking a half or a quarter of the columns with 8 or 16 offset groups (wide_log2_split()).  Measured,
+//     launches back to back: 64 -> 64 at 2 259 rows 14.2 -> 9.9 us, at 3 476 rows 14.3 -> 11.4, at 8 615 rows 20.1 -> 19.1;
+//     at 16 914 rows unsplit tiles are the faster ones (29.5 us).
 // Pair lists, operand order (the packed weights are conv_mfma.hip's), partial tiles in LDS (one per group and
 // column quarter, private to a wave, so the sum order is fixed), fixed-order reduction, fused scale/shift/ReLU and
 // the optional dense scatter are as in conv_mfma.hip; results are bit-identical run to run.
@@ -55,16 +60,16 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
           const int32_t* __restrict__ tiles, DenseTarget dt) {
     constexpr int G = CIN / 16;     // 16-channel chunks of the inner dimension
     constexpr int NBT = COUT / 16;  // 16-column blocks of the layer
-    constexpr int kCS = 4;               // waves of a group (column quarters)
-    constexpr int kKG = kWaves / kCS;    // groups the offsets are dealt to
-    constexpr int NB = NBT / kCS;   // column blocks of one wave
-    constexpr int CW = COUT / kCS;  // columns of one wave
+    constexpr int kQ = 4;          // a wave takes a quarter of the layer's columns
+    constexpr int NB = NBT / kQ;   // column blocks of one wave
+    constexpr int CW = COUT / kQ;  // columns of one wave
     constexpr int LDP = CW + 4;     // padded row stride of a partial tile
     static_assert(kTileRows <= 128 && kTileRows % 16 == 0, "the lists are staged in two halves of 64 rows");
     constexpr int kVecPerRow = COUT / 4;
     constexpr int kThreads = kWaves * 64;
-    static_assert(CIN % 16 == 0 && NBT % kCS == 0, "channel counts must fill whole MFMA chunks per wave");
+    static_assert(CIN % 16 == 0 && NBT % kQ == 0, "channel counts must fill whole MFMA chunks per wave");
     static_assert(kThreads % kVecPerRow == 0, "a thread must keep its columns from row to row");
+    static_assert(COUT == 64, "the split below counts in quarters of 16 columns");
     __shared__ int32_t s_in[kMaxK * kTileRows];   // compacted pair lists: input row ...
     __shared__ uint8_t s_row[kMaxK * kTileRows];  // ... and local output row of pair j of offset k
     __shared__ int32_t s_cnt[kMaxK + 5];          // pairs per offset
@@ -73,20 +78,41 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
 
     int n = *num_out;
     const int cut_count = tiles ? tiles[0] : 0;
-    const int cut_begin = tiles ? tiles[4 + blockIdx.x] : 0;
-    const int cut_end = tiles ? tiles[5 + blockIdx.x] : 0;
+    // the cuts of this workgroup's first tile under each split it may be part of: requested beside the row count
+    int cut_begin[3], cut_end[3];
+    int tile_of[3] = {(int)blockIdx.x, (int)blockIdx.x, (int)blockIdx.x};
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+#pragma unroll
+        for (int part = 1; part < 1 << s; ++part) tile_of[s] -= (int)blockIdx.x >= part * (num_cu >> s) ? num_cu >> s : 0;
+        cut_begin[s] = tiles ? tiles[4 + tile_of[s]] : 0;
+        cut_end[s] = tiles ? tiles[5 + tile_of[s]] : 0;
+    }
     n = n < 0 ? 0 : (n > max_voxels ? max_voxels : n);
+    // Column parts: 1 << lsplit workgroups share a tile.  The parts of a tile are row_groups apart in the grid, which
+    // puts them on one XCD (workgroups are dealt round robin over eight): they read the same rows.
+    const int lsplit = wide_log2_split(n, K, num_cu);
+    const int row_groups = num_cu >> lsplit;  // workgroups of one column part
+    const int first_tile = lsplit == 0 ? tile_of[0] : (lsplit == 1 ? tile_of[1] : tile_of[2]);
+    int part_id = 0;
+#pragma unroll
+    for (int part = 1; part < 4; ++part) part_id += (int)blockIdx.x >= part * row_groups ? 1 : 0;
+    const int lcs = 2 - lsplit, cs = 1 << lcs;                // waves of a group: the column quarters of this part
+    const int lkg = 4 - lcs, kg = 1 << lkg;                   // groups the offsets are dealt to
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (tells the compiler that it is wave-uniform)
-    const int kgrp = wave / kCS;   // offsets are dealt to this group ...
-    const int chalf = wave % kCS;  // ... and this wave computes this part of their columns
+    const int kgrp = wave >> lcs;                                // offsets are dealt to this group ...
+    const int quarter = (part_id << lcs) + (wave & (cs - 1));  // ... and this wave computes these columns of them
     float epi_scale = 1.f, epi_shift = 0.f;
     if (tid < COUT) {
         if (scale) epi_scale = scale[tid];
         if (shift) epi_shift = shift[tid];
     }
-    const int ec4 = (tid % kVecPerRow) * 4;  // this thread's epilogue columns, the same for every row it stores
+    // this thread's epilogue columns (the same for every row it stores): within the part, and of the layer
+    const int lvec = 4 - lsplit;  // log2 of the part's 4-column vectors
+    const int pc4 = (tid & ((1 << lvec) - 1)) * 4, ec4 = part_id * (COUT >> lsplit) + pc4;
+    static_assert(kVecPerRow == 16, "lvec");
 
     // rows >= n: the reference zero-fills them (then BN+ReLU): epilogue(0), spread over all workgroups
     if (write_pad) {
@@ -108,10 +134,13 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
             }
     }
     // The grid is one workgroup per compute unit (a workgroup takes most of a unit's LDS, so workgroups with no
-    // tile would queue behind the busy ones just to return); workgroup b walks tiles b, b + grid, ...: runs of rows
-    // from the rulebook's equal-work cuts, or runs of equal length.
-    const TilePlan plan = tile_plan(n, num_cu, kTileRows);
+    // tile would queue behind the busy ones just to return); a workgroup walks tiles first_tile, first_tile +
+    // row_groups, ...: runs of rows from the rulebook's equal-work cuts, or runs of equal length.
+    TilePlan plan = {0, 0};
+    if (cut_count == 0) plan = tile_plan(n, row_groups, kTileRows);
     const int tile_count = cut_count > 0 ? cut_count : (n > 0 ? plan.count : 0);
+    const int first_begin = lsplit == 0 ? cut_begin[0] : (lsplit == 1 ? cut_begin[1] : cut_begin[2]);
+    const int first_end = lsplit == 0 ? cut_end[0] : (lsplit == 1 ? cut_end[1] : cut_end[2]);
     const int i = lane & 15;  // pair inside a 16-pair block
     const int q = lane >> 4;  // channel group inside a 16-channel chunk
     const __amdgpu_buffer_rsrc_t rs_in = __builtin_amdgcn_make_buffer_rsrc(
@@ -119,11 +148,11 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
     const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<void*>(Wp), 0, (int)((size_t)K * CIN * COUT * sizeof(float)), kRawBuffer);
 
-    for (int tile = blockIdx.x; tile < tile_count; tile += gridDim.x) {
+    for (int tile = first_tile; tile < tile_count; tile += row_groups) {
     int run_begin, run_end;
     if (cut_count > 0) {
-        run_begin = tile == (int)blockIdx.x ? cut_begin : tiles[4 + tile];
-        run_end = tile == (int)blockIdx.x ? cut_end : tiles[5 + tile];
+        run_begin = tile == first_tile ? first_begin : tiles[4 + tile];
+        run_end = tile == first_tile ? first_end : tiles[5 + tile];
     } else {
         run_begin = tile * plan.height;
         run_end = run_begin + plan.height < n ? run_begin + plan.height : n;
@@ -185,8 +214,8 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
             if (b == size) rank = ahead + __popcll(m & below);
             ahead += __popcll(m);
         }
-        const int r2 = rank % (2 * kKG);
-        const int w = r2 < kKG ? r2 : 2 * kKG - 1 - r2;
+        const int r2 = rank & (2 * kg - 1);
+        const int w = r2 < kg ? r2 : 2 * kg - 1 - r2;
         my_mask = (uint32_t)__ballot(b > 0 && w == kgrp);
     }
 
@@ -217,7 +246,7 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
     };
     // chunk g of this wave's columns of W[k] -> operand registers (k < 0: nothing to fetch)
     auto load_b = [&](int k, int g, float4 (&b)[NB]) {
-        const unsigned at = k >= 0 ? (unsigned)(((((k * G + g) * NBT + chalf * NB) * 64) + lane) * 16) : kOutOfRange;
+        const unsigned at = k >= 0 ? (unsigned)(((((k * G + g) * NBT + quarter * NB) * 64) + lane) * 16) : kOutOfRange;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) b[nb] = buffer_load16(rs_w, at + nb * 64 * 16u);
     };
@@ -285,17 +314,22 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
     __syncthreads();
 
     // fixed-order sum of the groups' partial tiles, epilogue, coalesced stores
-    for (int v = tid; v < rows * kVecPerRow; v += kThreads) {
-        const int r = v / kVecPerRow;
-        const float* col = s_part + ((ec4 / CW) * kTileRows + r) * LDP + ec4 % CW;
+    for (int v = tid; v < rows << lvec; v += kThreads) {
+        const int r = v >> lvec;
+        const float* col = s_part + ((pc4 / CW) * kTileRows + r) * LDP + pc4 % CW;
         float4 acc4 = *reinterpret_cast<const float4*>(col);
-#pragma unroll
-        for (int w = 1; w < kKG; ++w) {
-            const float4 p4 = *reinterpret_cast<const float4*>(col + w * kCS * kTileRows * LDP);
+        auto add = [&](int w) {
+            const float4 p4 = *reinterpret_cast<const float4*>(col + (w << lcs) * kTileRows * LDP);
             acc4.x += p4.x;
             acc4.y += p4.y;
             acc4.z += p4.z;
             acc4.w += p4.w;
+        };
+#pragma unroll
+        for (int w = 1; w < 4; ++w) add(w);
+        for (int w0 = 4; w0 < kg; w0 += 4) {  // (8 or 16 groups under a column split)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) add(w0 + w);
         }
         float o[4] = {acc4.x, acc4.y, acc4.z, acc4.w};
 #pragma unroll

@@ -50,16 +50,27 @@ __host__ __device__ inline TilePlan tile_plan(int n, int num_cu, int target) {
     p.height = (n + p.count - 1) / p.count;
     return p;
 }
+// The one-tile-per-unit FP32 kernel (conv_wide.hip) with few rows: the 64 output columns of a tile are dealt to `split`
+// workgroups, so that the tiles stay tall enough to fill their 16-pair blocks while every compute unit has work and
+// reads only its columns of the weights.  At the bounds a tile has 48 (split 4) and 80 rows (split 2): beyond them
+// the blocks of the unsplit tiles are full enough.  A kernel volume with fewer offsets than the groups of a split
+// tile could be dealt (the 3x1x1 layer) is not split.
+constexpr int kWideSplit4Rows = 48, kWideSplit2Rows = 80, kWideSplitMinOffsets = 16;
+__host__ __device__ inline int wide_log2_split(int n, int K, int num_cu) {
+    if (num_cu % 4 || K < kWideSplitMinOffsets) return 0;
+    return n <= num_cu / 4 * kWideSplit4Rows ? 2 : (n <= num_cu / 2 * kWideSplit2Rows ? 1 : 0);
+}
 // tile capacity (rows) of the MFMA kernel that serves this layer shape
 int gemm_tile_rows(int cin, int cout, int dtype);
 int gemm_compute_units();
 
 // equal-work tile cuts for the MFMA kernel, written into `region` (tile_cut_bytes() bytes of the layer's
 // workspace; its first word must be zero before the launch and stays zero when there are no active rows);
-// target_rows >= kGemmMinTileRows is the tile height aimed at
+// target_rows >= kGemmMinTileRows is the tile height aimed at; `wide`: for the
+// one-tile-per-unit kernel, whose workgroups may share a tile (wide_log2_split())
 size_t tile_cut_bytes(int max_voxels);
 int launch_tile_cuts(const int32_t* nbr, const int32_t* num_out, int K, int max_voxels, int target_rows, int row_weight,
-                     void* region, hipStream_t stream);
+                     bool wide, void* region, hipStream_t stream);
 
 // picks the kernel for the layer shape; returns SESSD_E_UNSUPPORTED for dtype pairs not covered, and when a
 // dense target is set but the layer does not run on the MFMA kernel (see gemm_runs_on_mfma)

@@ -116,6 +116,8 @@ class ConvPluginBase {
     int tileRows() const;
     // weight of a row beside its pairs in those cuts
     int tileRowWeight() const;
+    // whether they are cut for the one-tile-per-unit kernel (wide_log2_split())
+    bool tilesWide() const;
     int exportRulebook(const int32_t* nbr, const int32_t* num_out, void* scratch,
                        int32_t* indice_pairs, uint32_t* indice_num, hipStream_t stream) const;
     int freeDevice();

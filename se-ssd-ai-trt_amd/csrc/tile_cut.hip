@@ -70,7 +70,7 @@ tile_weights(const int32_t* __restrict__ nbr, const int32_t* __restrict__ num_ou
 }
 
 __global__ void __launch_bounds__(kBlock)
-tile_cuts(const int32_t* __restrict__ num_out, int max_voxels, int num_cu, int target, int row_weight, const int32_t* __restrict__ w,
+tile_cuts(const int32_t* __restrict__ num_out, int max_voxels, int K, int num_cu, int target, int row_weight, int wide, const int32_t* __restrict__ w,
           const int32_t* __restrict__ bsum, int32_t* __restrict__ hdr) {
     __shared__ int32_t s_before[kBlock / 64], s_total[kBlock / 64], s_wave[kBlock / 64];
     int n = *num_out;
@@ -110,7 +110,7 @@ tile_cuts(const int32_t* __restrict__ num_out, int max_voxels, int num_cu, int t
     total = s_total[0] + s_total[1] + s_total[2] + s_total[3];
     for (int v = 0; v < wave; ++v) before += s_wave[v];
     const int excl = before + inc - mine;  // weight of all rows before this one
-    const int tiles = tile_plan(n, num_cu, target).count;
+    const int tiles = tile_plan(n, wide ? num_cu >> wide_log2_split(n, K, num_cu) : num_cu, target).count;
     // W is kept above the heaviest possible row: a row then advances the tile id by at most one, so every id
     // up to the last gets its start written (with few rows -- fewer than tiles -- total / tiles would fall
     // below a row's weight, ids would skip, and the skipped entries of the table would be read unwritten)
@@ -138,15 +138,15 @@ size_t tile_cut_bytes(int max_voxels) {
 }
 
 int launch_tile_cuts(const int32_t* nbr, const int32_t* num_out, int K, int max_voxels, int target_rows, int row_weight,
-                     void* region, hipStream_t stream) {
+                     bool wide, void* region, hipStream_t stream) {
     if (target_rows < kGemmMinTileRows) return fail(SESSD_E_INVALID, "tile cuts: target of %d rows is below %d", target_rows, kGemmMinTileRows);
     int32_t* hdr = static_cast<int32_t*>(region);
     int32_t* w = hdr + 4 + max_tiles(max_voxels) + 1;
     int32_t* bsum = w + max_voxels;
     const int blocks = ceil_div(max_voxels, kBlock);
     hipLaunchKernelGGL(tile_weights, dim3(blocks), dim3(kBlock * kSplit), 0, stream, nbr, num_out, max_voxels, K, row_weight, w, bsum);
-    hipLaunchKernelGGL(tile_cuts, dim3(blocks), dim3(kBlock), 0, stream, num_out, max_voxels, gemm_compute_units(), target_rows, row_weight, w,
-                       bsum, hdr);
+    hipLaunchKernelGGL(tile_cuts, dim3(blocks), dim3(kBlock), 0, stream, num_out, max_voxels, K, gemm_compute_units(), target_rows, row_weight, (int)wide,
+                       w, bsum, hdr);
     SESSD_HIP_TRY(hipGetLastError());
     return SESSD_OK;
 }

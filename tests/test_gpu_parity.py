@@ -799,3 +799,10 @@ def test_wide_fp32_kernel_tall_tiles_and_two_tiles_per_workgroup(n, clustered, c
     (tiles of uneven length from the equal-work cuts, two or three per workgroup), against the oracle on 16
     threads."""
     _fp32_subm_wide_against_oracle(n, 51200, (21, 400, 352), 5000 + n, clustered=clustered, threads=16, cin=cin)
+
+
+@pytest.mark.parametrize("cin", [64, 32])
+@pytest.mark.parametrize("n", [3071, 3072, 3073, 10239, 10240, 10241])
+def test_wide_fp32_kernel_around_the_row_counts_of_its_column_splits(n, cin):
+    """On 256 compute units a tile's columns are dealt to four workgroups up to 3 072 rows, to two up to 10 240."""
+    _fp32_subm_wide_against_oracle(n, n + 7, (11, 200, 176), 900 + n, threads=8, cin=cin)
