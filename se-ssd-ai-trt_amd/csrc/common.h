@@ -91,47 +91,7 @@ inline size_t dtype_size(int32_t t) { return t == SESSD_HALF ? 2 : 4; }
 
 constexpr uint32_t kEmpty = 0xFFFFFFFFu;
 
-// ---------------------------------------------------------------------------------------------
-// device side: open-addressing hash over linearised cell keys
-// ---------------------------------------------------------------------------------------------
-// keys[cap] (cap a power of two) start as kEmpty.  Multiplicative hashing spreads the strongly
-// correlated keys of neighbouring cells; linear probing keeps a probe sequence inside one or two
-// cache lines.  Every loop is bounded by the capacity: a full table is reported, never spun on.
-struct HashTable {
-    uint32_t* keys;
-    uint32_t* vals;
-    uint32_t mask;   // cap - 1
-    int32_t shift;   // 32 - log2(cap)
-};
-
 #ifdef __HIPCC__
-__device__ __forceinline__ uint32_t hash_slot0(const HashTable& t, uint32_t key) {
-    return (key * 2654435769u) >> t.shift;
-}
-
-// -> slot holding `key` (claimed now or earlier), or -1 when the table is full
-__device__ __forceinline__ int32_t hash_insert(const HashTable& t, uint32_t key) {
-    uint32_t slot = hash_slot0(t, key);
-    for (uint32_t probe = 0; probe <= t.mask; ++probe) {
-        uint32_t prev = atomicCAS(&t.keys[slot], kEmpty, key);
-        if (prev == kEmpty || prev == key) return (int32_t)slot;
-        slot = (slot + 1) & t.mask;
-    }
-    return -1;
-}
-
-// -> slot holding `key`, or -1 when absent
-__device__ __forceinline__ int32_t hash_find(const HashTable& t, uint32_t key) {
-    uint32_t slot = hash_slot0(t, key);
-    for (uint32_t probe = 0; probe <= t.mask; ++probe) {
-        uint32_t k = t.keys[slot];
-        if (k == key) return (int32_t)slot;
-        if (k == kEmpty) return -1;
-        slot = (slot + 1) & t.mask;
-    }
-    return -1;
-}
-
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 
 // number of set bits of `m` below this lane (wave64)
@@ -139,26 +99,6 @@ __device__ __forceinline__ uint32_t rank_in_wave(uint64_t m) {
     return __popcll(m & ((1ull << lane_id()) - 1ull));
 }
 #endif
-
-inline HashTable make_hash(uint32_t* keys, uint32_t* vals, uint32_t cap) {
-    HashTable t;
-    t.keys = keys;
-    t.vals = vals;
-    t.mask = cap - 1;
-    t.shift = 32 - ilog2(cap);
-    return t;
-}
-
-// The neighbour table of the SubM layer that comes next on a coors tensor, as the kernel that CREATES the rows
-// of that tensor sees it: it writes "no neighbour" into entries [first_offset, K) of every row it creates, so
-// that the SubM build can run its symmetric lookup (which writes those entries only where a neighbour exists)
-// without the whole K x max_voxels table being cleared per frame.
-struct MirrorInit {
-    int32_t* nbr = nullptr;  // [K][stride]
-    int stride = 0;          // max_voxels of the SubM layer
-    int first_offset = 0;    // 14 for a 3x3x3 kernel: offsets 14..26 are the mirrored ones
-    int K = 0;
-};
 
 // Optional second destination of a gather-GEMM's epilogue: the dense tensor of the sparse2Dense step that
 // would follow (sparse2Dense.cu:182-207: dense[(c*D + z)][y][x] = feat[row][c], here with the zero border of

@@ -1,0 +1,892 @@
+// coord.hip -- the passes of the coordinate side (coord.h) and their launches.
+//
+//   vg_insert     point -> cell table, each cell keeping its smallest point index
+//   vg_flags      "am I the first point of my cell" -> wave64 ballot words + counts per 256 points; the others are kept
+//                 behind the first one, the S - 1 smallest of them
+//   vg_finalize   prefix over the words = voxel row in first-appearance order; coordinate and mean
+//   sp_insert     ticket (input row, candidate) -> table of output cells, each keeping its smallest ticket
+//   sp_flags      "am I the first ticket of my cell" -> ballot words + counts per 256 tickets
+//   sp_number     prefix over the words = output row in first-seen order; out coors + voxel_num
+//   lookups       nbr[k][row] for all offsets of a row, and the rows' weights for the tile cuts
+//   tile cuts     equal-work tile boundaries from those weights (tile_cut.hip describes them)
+//
+// A pass that creates rows (vg_finalize, sp_number) holds their coordinates and numbers in registers: it inserts the
+// next strided layer's tickets right away, and what only needs finished tables (lookups, cuts) shares a launch with the
+// next step of the chain.  For the reference's backbone that is 12 launches a frame in place of 35.
+#include "coord.h"
+#include "fill.h"
+
+namespace sessd {
+
+namespace {
+
+constexpr uint32_t kSlotBits = 26;
+constexpr uint32_t kSlotMask = (1u << kSlotBits) - 1u;
+
+// ---------------------------------------------------------------------------------------------
+// voxelizer
+// ---------------------------------------------------------------------------------------------
+// -> key of the cell the point lies in, kEmpty when it lies in none
+__device__ __forceinline__ uint32_t point_cell(const VgPart& p, float x, float y, float z, int& ix, int& iy, int& iz) {
+    // voxelGenerator.cu:363-367: half-open range test
+    if (!(x >= p.min_x && x < p.max_x && y >= p.min_y && y < p.max_y && z >= p.min_z && z < p.max_z)) return kEmpty;
+    // voxelGenerator.cu:369-371: IEEE FP32 division (never a reciprocal multiply)
+    ix = (int)floorf((x - p.min_x) / p.vx);
+    iy = (int)floorf((y - p.min_y) / p.vy);
+    iz = (int)floorf((z - p.min_z) / p.vz);
+    // voxelGenerator.cu:375: a value just below max can still land on the grid size
+    if (!(ix >= 0 && ix < p.gx && iy >= 0 && iy < p.gy && iz >= 0 && iz < p.gz)) return kEmpty;
+    return ((uint32_t)iz * (uint32_t)p.gy + (uint32_t)iy) * (uint32_t)p.gx + (uint32_t)ix;
+}
+
+// cells of a stage's rows of the frame before -> empty
+__device__ __forceinline__ void clean_pass(const CleanPart& P, int block) {
+    const int n = clamp_rows(P.num, P.max_voxels);
+    for (int row = block * kCoordBlock + (int)threadIdx.x; row < n; row += P.blocks * kCoordBlock) {
+        const int4 c = reinterpret_cast<const int4*>(P.coors)[row];
+        static_cast<uint32_t*>(P.t.base)[((uint32_t)c.y * (uint32_t)P.t.gy + (uint32_t)c.z) * (uint32_t)P.t.gx + (uint32_t)c.w] = kEmpty;
+    }
+}
+
+struct Cleans {
+    CleanPart c[kMaxCleans];
+    int n;
+};
+
+template <int N>
+__global__ void __launch_bounds__(kCoordBlock) vg_insert(VgPart p, Cleans cleans, FillPlan<N> also) {
+    if ((int)blockIdx.x >= p.n_blocks) {
+        int b = blockIdx.x - p.n_blocks;
+        for (int i = 0; i < cleans.n; ++i) {
+            if (b < cleans.c[i].blocks) return clean_pass(cleans.c[i], b);
+            b -= cleans.c[i].blocks;
+        }
+        return fill_pass(also, b);
+    }
+    const int i = blockIdx.x * kCoordBlock + threadIdx.x;
+    const int n = clamp_rows(p.points_size, p.max_points);
+    if (i >= n) return;
+    const float* pt = p.points + (size_t)i * p.pf;
+    int ix, iy, iz;
+    const uint32_t key = point_cell(p, pt[0], pt[1], pt[2], ix, iy, iz);
+    int32_t slot = -1;
+    if (key != kEmpty) {
+        slot = insert_min(open_table(p.t, n), key, (uint32_t)i);
+        if (slot < 0) atomicOr(&p.status[1], SESSD_STATUS_HASH_FULL);
+    }
+    p.pt_slot[i] = slot;
+}
+
+// The table names every cell's first point f now.  A later point of the cell is offered to the S - 1 places behind f,
+// which keep the smallest indices in ascending order: every place ends up with the minimum of what was offered to it and
+// passes the rest on, so the final state does not depend on the order in which the threads arrive.
+template <int N>
+__global__ void __launch_bounds__(kCoordBlock) vg_flags(VgPart p, FillPlan<N> also) {
+    if ((int)blockIdx.x >= p.n_blocks) return fill_pass(also, blockIdx.x - p.n_blocks);
+    __shared__ uint32_t lds4[4];
+    const int i = blockIdx.x * kCoordBlock + threadIdx.x;
+    const int n = clamp_rows(p.points_size, p.max_points);
+    bool first = false;
+    if (i < n) {
+        const int32_t slot = p.pt_slot[i];
+        if (slot >= 0) {
+            const uint32_t f = value_at(open_table(p.t, n), slot);
+            first = f == (uint32_t)i;
+            if (!first) {
+                uint32_t* s = p.slots + (size_t)f * (p.max_pts - 1);
+                uint32_t cur = (uint32_t)i;
+                for (int q = 0; q < p.max_pts - 1; ++q) {
+                    const uint32_t old = atomicMin(&s[q], cur);
+                    if (old == kEmpty) break;
+                    cur = old > cur ? old : cur;
+                }
+            }
+        }
+    }
+    const uint64_t m = __ballot(first);
+    if ((threadIdx.x & 63) == 0) {
+        p.words[i >> 6] = m;
+        lds4[threadIdx.x >> 6] = __popcll(m);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) p.counts[blockIdx.x] = lds4[0] + lds4[1] + lds4[2] + lds4[3];
+}
+
+// ---------------------------------------------------------------------------------------------
+// strided layers: tickets
+// ---------------------------------------------------------------------------------------------
+// x / s truncating toward zero, s >= 1
+__device__ __forceinline__ int div_trunc(int x, int s) {
+    if (s == 1) return x;
+    if (s == 2) return (x - (x >> 31)) >> 1;
+    return x / s;
+}
+// e / c for the short candidate lists (e < 27)
+__device__ __forceinline__ int div_small(int e, int c) {
+    return c == 1 ? e : (c == 2 ? e >> 1 : (c == 3 ? (e * 43) >> 7 : e / c));
+}
+
+// getValidOutPosKernel (sparseConv3dlayer.cu:310-386), one enumeration step: candidate `e` of the input cell c.  Integer
+// divisions truncate toward zero exactly as in the reference; dilation is 1.
+// -> false when e is past the enumeration or the output cell is outside the grid
+__device__ __forceinline__ bool sp_candidate(const int c[3], const SpPart& P, int e, int o[3], int& offset) {
+    int up[3], cs[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const int lo = div_trunc(c[a] - (P.k[a] - 1) - 1 + P.s[a] + P.p[a], P.s[a]);
+        up[a] = div_trunc(c[a] + P.p[a], P.s[a]);
+        cs[a] = up[a] - lo + 1;
+    }
+    if (cs[0] <= 0 || cs[1] <= 0 || cs[2] <= 0 || e >= cs[0] * cs[1] * cs[2]) return false;
+    const int e1 = div_small(e, cs[2]), e0 = div_small(e1, cs[1]);
+    const int cnt[3] = {e0, e1 - e0 * cs[1], e - e1 * cs[2]};  // x fastest
+    bool valid = true;
+    int m = 1;
+    offset = 0;
+#pragma unroll
+    for (int a = 2; a >= 0; --a) {
+        o[a] = up[a] - cnt[a];
+        if (o[a] < 0 || o[a] > P.os[a] - 1) valid = false;
+        offset += m * (c[a] - o[a] * P.s[a] + P.p[a]);
+        m *= P.k[a];
+    }
+    return valid;
+}
+
+// Rows that follow each other name the same output cells again and again (eight input cells share an output cell of a
+// 3x3x3 stride-2 layer, and neighbours in space are mostly neighbours in the row order), and device-wide atomics are what
+// this pass is made of.  A block therefore gathers the cells of kTicketsAtOnce tickets in an LDS table first (cell ->
+// smallest ticket of the block), and one thread per distinct cell goes to the table in memory.
+constexpr int kPerThread = 2;
+constexpr int kTicketsAtOnce = kPerThread * kCoordBlock;
+constexpr int kLocalBits = 10, kLocalSlots = 1 << kLocalBits;  // twice the tickets
+struct InsertLds {
+    uint32_t key[kLocalSlots], val[kLocalSlots];
+};
+
+// the tickets of m rows (row, z, y, x) in LDS; the whole block takes part
+__device__ __forceinline__ void sp_insert_rows(const SpPart& P, const CellView& t, const int4* rows, int m, InsertLds& L) {
+    const int total = m * P.Kc;
+    for (int base = 0; base < total; base += kTicketsAtOnce) {
+        for (int i = threadIdx.x; i < kLocalSlots; i += kCoordBlock) {
+            L.key[i] = kEmpty;
+            L.val[i] = kEmpty;
+        }
+        __syncthreads();
+        uint32_t key[kPerThread], tk[kPerThread];
+        int local[kPerThread], offset[kPerThread];
+        bool live[kPerThread], owner[kPerThread];
+#pragma unroll
+        for (int j = 0; j < kPerThread; ++j) {
+            const int item = base + j * kCoordBlock + threadIdx.x;
+            live[j] = item < total;
+            owner[j] = false;
+            local[j] = -1;
+            offset[j] = 0;
+            key[j] = tk[j] = kEmpty;
+            if (!live[j]) continue;
+            const int r = P.Kc == 8 ? item >> 3 : item / P.Kc, e = item - r * P.Kc;
+            const int4 row = rows[r];
+            const int c[3] = {row.y, row.z, row.w};
+            tk[j] = (uint32_t)row.x * (uint32_t)P.Kc + (uint32_t)e;
+            int o[3];
+            // A negative coordinate makes the truncating divisions of getValidOutPos yield kernel offsets outside
+            // [0, K) (c = -2, k = 3, s = 2, p = 1: o = 0, offset term -1), with which the reference indexes its
+            // rulebook.  Such a row contributes nothing here and raises BAD_COORD; the offset is checked as well, so
+            // that nothing a caller passes can make sp_scatter store outside the neighbour table.
+            const bool bad = c[0] < 0 || c[1] < 0 || c[2] < 0;
+            if (bad && e == 0) atomicOr(&P.meta[2], SESSD_STATUS_BAD_COORD);
+            if (bad || !sp_candidate(c, P, e, o, offset[j]) || offset[j] < 0 || offset[j] >= P.K) continue;
+            key[j] = ((uint32_t)o[0] * (uint32_t)P.os[1] + (uint32_t)o[1]) * (uint32_t)P.os[2] + (uint32_t)o[2];
+            uint32_t ls = (key[j] * 2654435769u) >> (32 - kLocalBits);
+            for (;;) {  // (at most kTicketsAtOnce keys in twice as many slots: room is always found)
+                const uint32_t prev = atomicCAS(&L.key[ls], kEmpty, key[j]);
+                if (prev == kEmpty || prev == key[j]) {
+                    owner[j] = prev == kEmpty;
+                    break;
+                }
+                ls = (ls + 1) & (kLocalSlots - 1);
+            }
+            local[j] = (int)ls;
+            atomicMin(&L.val[ls], tk[j]);
+        }
+        __syncthreads();
+        // the thread that claimed a cell's LDS entry carries the block's smallest ticket to memory
+        if (t.d) {
+#pragma unroll
+            for (int j = 0; j < kPerThread; ++j)
+                if (owner[j]) atomicMin(&t.d[key[j]], L.val[local[j]]);
+        } else {
+            EntryGroup g[kPerThread];
+            uint32_t at[kPerThread];
+            unsigned long long prev[kPerThread];
+#pragma unroll
+            for (int j = 0; j < kPerThread; ++j)
+                if (owner[j]) g[j] = load_group(t, first_slot(t, key[j]));
+#pragma unroll
+            for (int j = 0; j < kPerThread; ++j)
+                if (owner[j]) {
+                    at[j] = likely_slot(t, key[j], g[j]);
+                    prev[j] = atomicCAS(&t.h[at[j]], kEmptyEntry, make_entry(key[j], L.val[local[j]]));
+                }
+#pragma unroll
+            for (int j = 0; j < kPerThread; ++j)
+                if (owner[j]) {
+                    const int32_t slot = finish_insert_min(t, key[j], L.val[local[j]], at[j], prev[j]);
+                    if (slot < 0) {
+                        atomicOr(&P.meta[2], SESSD_STATUS_HASH_FULL);
+                        L.key[local[j]] = kEmpty;  // (read below as "no slot")
+                    } else {
+                        L.val[local[j]] = (uint32_t)slot;
+                    }
+                }
+            __syncthreads();
+        }
+#pragma unroll
+        for (int j = 0; j < kPerThread; ++j)
+            if (live[j]) {
+                uint32_t c = kEmpty;
+                if (local[j] >= 0 && L.key[local[j]] != kEmpty)
+                    c = ((uint32_t)offset[j] << kSlotBits) | (t.d ? key[j] : L.val[local[j]]);
+                P.cand[tk[j]] = c;
+            }
+        if (base + kTicketsAtOnce < total) __syncthreads();
+    }
+}
+
+// Points per block of vg_finalize: with a strided layer behind it, a wave of points gives the block's four waves about
+// one round of tickets.
+constexpr int kFinalPoints = 64;
+constexpr int kAhead = 4;  // further points of a cell that are requested ahead (the reference averages five)
+
+__global__ void __launch_bounds__(kCoordBlock) vg_finalize(VgPart p, SpPart next, int has_next) {
+    __shared__ uint32_t lds4[4];
+    __shared__ int4 s_rows[kFinalPoints];
+    __shared__ int s_m;
+    __shared__ InsertLds L;
+    const int n = clamp_rows(p.points_size, p.max_points);
+    const int n_blocks = (n + kCoordBlock - 1) / kCoordBlock;  // 256-point blocks that hold points
+    const int first_point = blockIdx.x * kFinalPoints;
+    if (first_point >= n && blockIdx.x != 0) return;
+    const int i = first_point + (int)threadIdx.x;
+    const int mine = first_point / kCoordBlock;
+    const bool point = threadIdx.x < kFinalPoints && i < n;
+    // what does not depend on the prefix is requested beside it
+    const int in_block = (first_point / 64) & 3;
+    uint64_t w[4] = {0, 0, 0, 0};
+    int32_t slot = -1;
+    float x = 0.f, y = 0.f, z = 0.f, f = 0.f;
+    if (point) {
+        for (int q = 0; q <= in_block; ++q) w[q] = p.words[mine * 4 + q];
+        slot = p.pt_slot[i];
+        const float* pt = p.points + (size_t)i * p.pf;
+        x = pt[0];
+        y = pt[1];
+        z = pt[2];
+        f = pt[3];
+    }
+    uint32_t before = 0, total = 0;
+    for (int j = threadIdx.x; j < n_blocks; j += kCoordBlock) {
+        const uint32_t c = p.counts[j];
+        total += c;
+        if (j < mine) before += c;
+    }
+    uint64_t m = 0;
+    for (int q = 0; q < 4; ++q)
+        if (q == in_block) m = w[q];
+    const bool first = point && ((m >> threadIdx.x) & 1ull);
+    // the cell's further points: indices, then (below) the points, while the sums over the blocks are made
+    uint32_t* more = p.slots + (size_t)i * (p.max_pts - 1);
+    uint32_t idx[kAhead];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) idx[q] = first && q < p.max_pts - 1 ? more[q] : kEmpty;
+    before = block_sum(before, lds4);
+    total = block_sum(total, lds4);
+    const int rows = (int)(total > (uint32_t)p.max_voxels ? (uint32_t)p.max_voxels : total);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *p.voxel_num = rows;
+        p.status[0] = p.status[1] | (total > (uint32_t)p.max_voxels ? SESSD_STATUS_VOXEL_OVERFLOW : 0);
+        p.status[1] = 0;
+    }
+    for (int q = 0; q < 4; ++q)
+        if (q < in_block) before += __popcll(w[q]);
+    const uint32_t rank = rank_in_wave(m), vid = before + rank;
+    const bool kept = first && vid < (uint32_t)p.max_voxels;
+    float ahead[kAhead][4];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) {
+        const bool live = kept && idx[q] != kEmpty;
+        const float* pt = p.points + (size_t)(live ? idx[q] : 0) * p.pf;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ahead[q][e] = live ? pt[e] : 0.f;
+    }
+    if (threadIdx.x < 64) {
+        const int room = before >= (uint32_t)p.max_voxels ? 0 : (int)((uint32_t)p.max_voxels - before);
+        const int here = __popcll(m);
+        if (threadIdx.x == 0) s_m = here < room ? here : room;
+        if (kept) {
+            int ix, iy, iz;
+            (void)point_cell(p, x, y, z, ix, iy, iz);
+            reinterpret_cast<int4*>(p.coors)[vid] = make_int4(0, iz, iy, ix);  // voxelGenerator.cu:404-405
+            s_rows[rank] = make_int4((int)vid, iz, iy, ix);
+        }
+        // the table now maps cell -> voxel row; cells first seen beyond the cap are dropped
+        if (first) set_value(open_table(p.t, n), slot, kept ? vid : kEmpty);
+    }
+    if (has_next) {
+        __syncthreads();
+        sp_insert_rows(next, open_table(next.t, rows < next.max_voxels ? rows : next.max_voxels), s_rows, s_m, L);
+    }
+    // the places are left empty for the next frame
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q)
+        if (idx[q] != kEmpty) more[q] = kEmpty;
+    if (first && !kept)
+        for (int q = kAhead; q < p.max_pts - 1; ++q) more[q] = kEmpty;
+    if (!kept) return;
+    // voxelGenerator.cu:274-296: all S slots are summed left to right, unfilled slots count as 0
+    float sx = x, sy = y, sz = z, sw = f;
+    int cnt = 1;
+    for (int q = 0; q < p.max_pts - 1; ++q) {
+        float a[4] = {0.f, 0.f, 0.f, 0.f};
+        if (q < kAhead) {
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j)
+                if (j == q) {
+                    cnt += idx[j] != kEmpty ? 1 : 0;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) a[e] = ahead[j][e];
+                }
+        } else if (more[q] != kEmpty) {
+            const float* pt = p.points + (size_t)more[q] * p.pf;
+            for (int e = 0; e < 4; ++e) a[e] = pt[e];
+            ++cnt;
+            more[q] = kEmpty;
+        }
+        sx = sx + a[0];
+        sy = sy + a[1];
+        sz = sz + a[2];
+        sw = sw + a[3];
+    }
+    const float c = (float)cnt;
+    reinterpret_cast<float4*>(p.voxels)[vid] = make_float4(sx / c, sy / c, sz / c, sw / c);
+}
+
+// the tickets of a coors tensor (a strided layer on its own)
+__global__ void __launch_bounds__(kCoordBlock) sp_insert(SpPart P) {
+    __shared__ int4 s_rows[kTicketsAtOnce];
+    __shared__ InsertLds L;
+    const int n = clamp_rows(P.in_num, P.max_voxels);
+    const int per = kTicketsAtOnce / P.Kc > 0 ? kTicketsAtOnce / P.Kc : 1;  // rows a block takes at a time
+    const CellView t = open_table(P.t, n);
+    for (int r0 = blockIdx.x * per; r0 < n; r0 += gridDim.x * per) {
+        const int m = n - r0 < per ? n - r0 : per;
+        __syncthreads();
+        for (int r = threadIdx.x; r < m; r += kCoordBlock) {
+            const int4 c = reinterpret_cast<const int4*>(P.in_coors)[r0 + r];
+            s_rows[r] = make_int4(r0 + r, c.y, c.z, c.w);
+        }
+        __syncthreads();
+        sp_insert_rows(P, t, s_rows, m, L);
+    }
+}
+
+__device__ __forceinline__ void sp_flags_pass(const SpPart& P, int block, int blocks, uint32_t* lds4) {
+    const int n = clamp_rows(P.in_num, P.max_voxels);
+    const int64_t tickets = (int64_t)n * P.Kc;
+    const CellView t = open_table(P.t, n);
+    for (int c = block; (int64_t)c * kCoordBlock < tickets; c += blocks) {
+        const uint32_t tk = (uint32_t)c * kCoordBlock + threadIdx.x;
+        bool first = false;
+        if (tk < tickets) {
+            const uint32_t slot = P.cand[tk];
+            first = slot != kEmpty && value_at(t, slot & kSlotMask) == tk;
+        }
+        const uint64_t m = __ballot(first);
+        __syncthreads();
+        if ((threadIdx.x & 63) == 0) {
+            P.words[tk >> 6] = m;
+            lds4[threadIdx.x >> 6] = __popcll(m);
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) P.counts[c] = lds4[0] + lds4[1] + lds4[2] + lds4[3];
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// lookups
+// ---------------------------------------------------------------------------------------------
+// A wave takes 16 rows, four lanes per row with a quarter of the offsets each: the probes of a lane are independent
+// loads, all in flight at once, and its stores are runs of 16 rows.  With one (row, offset) per thread, two dependent
+// loads per probe and the upper half of the offsets written by symmetry this took 7-21 us at 16 000 - 75 000 rows.
+constexpr int kLookupRows = 64;                             // rows of a block
+constexpr int kLookupDepth = (kGemmMaxOffsets + 3) / 4;     // offsets of a lane
+
+__device__ __forceinline__ void lookup_pass(const LookupPart& P, int block, int32_t* lds4) {
+    const int n = clamp_rows(P.num, P.max_voxels);
+    if (P.meta && block == 0 && threadIdx.x == 0) {
+        P.meta[1] = n;
+    }
+    const CellView t = open_table(P.t, clamp_rows(P.t_num, P.t_max));
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i = lane & 15, q = lane >> 4;
+    const int per = (P.K + 3) >> 2;
+    const int k0 = q * per;
+    int kz0 = k0 / (P.k[1] * P.k[2]), ky0 = (k0 / P.k[2]) % P.k[1], kx0 = k0 % P.k[2];
+    for (int chunk = block; chunk * kLookupRows < n; chunk += P.blocks) {
+        const int row = chunk * kLookupRows + wave * 16 + i;
+        uint32_t key[kLookupDepth];
+        bool in_layer = false;
+        int4 c = make_int4(0, 0, 0, 0);
+        if (row < n) {
+            c = reinterpret_cast<const int4*>(P.coors)[row];
+            in_layer = c.y >= 0 && c.y < P.own[0] && c.z >= 0 && c.z < P.own[1] && c.w >= 0 && c.w < P.own[2];
+        }
+        const int z0 = c.y * P.s[0] - P.p[0], y0 = c.z * P.s[1] - P.p[1], x0 = c.w * P.s[2] - P.p[2];
+        int kz = kz0, ky = ky0, kx = kx0;
+#pragma unroll
+        for (int j = 0; j < kLookupDepth; ++j) {
+            const int z = z0 + kz, y = y0 + ky, x = x0 + kx;
+            const bool ok = in_layer && j < per && k0 + j < P.K && z >= 0 && z < P.t.gz && y >= 0 && y < P.t.gy && x >= 0 && x < P.t.gx;
+            key[j] = ok ? ((uint32_t)z * (uint32_t)P.t.gy + (uint32_t)y) * (uint32_t)P.t.gx + (uint32_t)x : kEmpty;
+            if (++kx == P.k[2]) {
+                kx = 0;
+                if (++ky == P.k[1]) {
+                    ky = 0;
+                    ++kz;
+                }
+            }
+        }
+        int cnt = 0;
+        if (t.d) {
+            uint32_t v[kLookupDepth];
+#pragma unroll
+            for (int j = 0; j < kLookupDepth; ++j) v[j] = key[j] != kEmpty ? t.d[key[j]] : kEmpty;
+#pragma unroll
+            for (int j = 0; j < kLookupDepth; ++j) {
+                cnt += v[j] != kEmpty ? 1 : 0;
+                if (row < n && j < per && k0 + j < P.K) P.nbr[(size_t)(k0 + j) * P.max_voxels + row] = (int32_t)v[j];
+            }
+        } else {
+            // All probe sequences advance together, a round of loads at a time, four entries per sequence and round: one
+            // after the other the collisions of seven sequences were seven times the latency (15 us for 2 000 rows).
+            uint32_t slot[kLookupDepth], val[kLookupDepth];
+            bool open[kLookupDepth], any = false;
+#pragma unroll
+            for (int j = 0; j < kLookupDepth; ++j) {
+                slot[j] = first_slot(t, key[j]);
+                val[j] = kEmpty;
+                open[j] = key[j] != kEmpty;
+                any |= open[j];
+            }
+            for (uint32_t round = 0; any && round <= t.mask; round += kGroup) {
+                EntryGroup g[kLookupDepth];
+#pragma unroll
+                for (int j = 0; j < kLookupDepth; ++j)
+                    if (open[j]) g[j] = load_group(t, slot[j]);
+                any = false;
+#pragma unroll
+                for (int j = 0; j < kLookupDepth; ++j) {
+                    if (open[j]) {
+#pragma unroll
+                        for (int e = 0; e < kGroup; ++e) {
+                            if (e < (int)(slot[j] & (kGroup - 1))) continue;
+                            if (entry_key(g[j].e[e]) == key[j]) {
+                                val[j] = entry_val(g[j].e[e]);
+                                open[j] = false;
+                            } else if (g[j].e[e] == kEmptyEntry) {
+                                open[j] = false;
+                            }
+                        }
+                        slot[j] = ((slot[j] | (kGroup - 1)) + 1) & t.mask;
+                    }
+                    any |= open[j];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < kLookupDepth; ++j) {
+                cnt += val[j] != kEmpty ? 1 : 0;
+                if (row < n && j < per && k0 + j < P.K) P.nbr[(size_t)(k0 + j) * P.max_voxels + row] = (int32_t)val[j];
+            }
+        }
+        if (P.w) {
+            cnt += __shfl_xor(cnt, 16, 64);
+            cnt += __shfl_xor(cnt, 32, 64);
+            int w = row < n ? cnt + P.row_weight : 0;
+            if (q == 0 && row < P.max_voxels) P.w[row] = w;
+#pragma unroll
+            for (int d = 8; d > 0; d >>= 1) w += __shfl_xor(w, d, 64);
+            __syncthreads();
+            if (lane == 0) lds4[wave] = w;
+            __syncthreads();
+            if (threadIdx.x == 0) P.wsum[chunk] = lds4[0] + lds4[1] + lds4[2] + lds4[3];
+        }
+    }
+}
+
+struct FlagsLookups {
+    SpPart flags;
+    int flag_blocks;
+    LookupPart look[kMaxLookups];
+    int n_look;
+};
+
+__global__ void __launch_bounds__(kCoordBlock) flags_lookups(FlagsLookups a) {
+    __shared__ uint32_t lds4[4];
+    int b = blockIdx.x;
+    if (b < a.flag_blocks) return sp_flags_pass(a.flags, b, a.flag_blocks, lds4);
+    b -= a.flag_blocks;
+    for (int l = 0; l < a.n_look; ++l) {
+        if (b < a.look[l].blocks) return lookup_pass(a.look[l], b, reinterpret_cast<int32_t*>(lds4));
+        b -= a.look[l].blocks;
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// numbering, tile cuts
+// ---------------------------------------------------------------------------------------------
+// A block takes the chunks block, block + blocks, ...  What its first chunk needs (words, cand, and with it the cell) is
+// requested before the row count and the sums over the chunks before it are known: the pass is a chain of round trips to
+// memory, and these are three of its seven otherwise.
+__device__ __forceinline__ void sp_number_pass(const SpPart& P, const SpPart& next, bool has_next, int block, int blocks,
+                                               uint32_t* lds4, int4* s_rows, InsertLds& L) {
+    uint64_t w[4];
+    uint32_t cand = 0;
+    auto request = [&](int c) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) w[q] = P.words[c * 4 + q];
+        cand = P.cand[(uint32_t)c * kCoordBlock + threadIdx.x];
+    };
+    request(block);  // (in bounds: at most n_chunks blocks; not used where the chunk is beyond the active ones)
+    // Only the chunks that hold tickets of active input rows carry anything.
+    const int n_in = clamp_rows(P.in_num, P.max_voxels);
+    const int active = (int)(((int64_t)n_in * P.Kc + kCoordBlock - 1) / kCoordBlock);
+    if (block >= active && block != 0) return;  // (no active input row at all: block 0 still owes the count)
+    const CellView t = open_table(P.t, n_in);
+    const int wave = threadIdx.x >> 6;
+    const uint32_t plane = (uint32_t)(P.os[1] * P.os[2]);
+    int n_out = 0;
+    for (int c = block; c < active || c == 0; c += blocks) {
+        if (c != block) request(c);
+        const bool first = c < active && ((w[wave] >> (threadIdx.x & 63)) & 1ull);
+        const uint32_t slot = cand & kSlotMask;
+        uint32_t key = 0;
+        if (first) key = key_at(t, slot);
+        uint32_t before = 0, total = 0;
+        for (int j = threadIdx.x; j < active; j += kCoordBlock) {
+            const uint32_t v = P.counts[j];
+            total += v;
+            if (j < c) before += v;
+        }
+        before = block_sum(before, lds4);
+        total = block_sum(total, lds4);
+        n_out = (int)(total > (uint32_t)P.max_voxels ? (uint32_t)P.max_voxels : total);
+        if (c == 0 && threadIdx.x == 0) {
+            *P.out_num = n_out;
+            P.meta[1] = n_out;
+            // (the reference overflows its buffers; here the site is dropped)
+            P.meta[0] = P.meta[2] | (total > (uint32_t)P.max_voxels ? SESSD_STATUS_VOXEL_OVERFLOW : 0);
+            P.meta[2] = 0;
+        }
+        if (active == 0) return;
+        uint32_t rank = rank_in_wave(w[wave]), here = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (q < wave) rank += __popcll(w[q]);
+            here += __popcll(w[q]);
+        }
+        if (first) {
+            const uint32_t id = before + rank;
+            if (id >= (uint32_t)P.max_voxels) {
+                set_value(t, slot, kEmpty);
+            } else {
+                set_value(t, slot, id);  // from here on the table maps cell -> output row
+                const int z = key / plane;
+                const int rem = key - z * plane;
+                const int y = rem / P.os[2], x = rem - y * P.os[2];
+                reinterpret_cast<int4*>(P.out_coors)[id] = make_int4(0, z, y, x);  // sparseConv3dlayer.cu:438-441
+                s_rows[rank] = make_int4((int)id, z, y, x);
+                // where sp_scatter fills the table in, the new row's entries start empty: clearing them here, row by
+                // row, touches only the rows that exist
+                if (P.nbr)
+                    for (int k = 0; k < P.K; ++k) P.nbr[(size_t)k * P.max_voxels + id] = -1;
+            }
+        }
+        if (has_next) {
+            const int room = before >= (uint32_t)P.max_voxels ? 0 : (int)((uint32_t)P.max_voxels - before);
+            __syncthreads();
+            sp_insert_rows(next, open_table(next.t, n_out), s_rows, (int)here < room ? (int)here : room, L);
+            __syncthreads();
+        }
+    }
+}
+
+// rows -> tile boundaries; 256 rows at a time
+__device__ __forceinline__ void cut_pass(const CutPart& P, int block, int32_t* lds) {
+    int32_t* s_wave = lds;
+    const int n = clamp_rows(P.num, P.max_voxels);
+    if (n == 0) {
+        if (block == 0 && threadIdx.x == 0) P.hdr[0] = 0;  // no cuts
+        return;
+    }
+    const int groups = (n + 63) / 64;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int tiles = tile_plan(n, P.wide ? P.num_cu >> wide_log2_split(n, P.K, P.num_cu) : P.num_cu, P.target).count;
+    uint32_t* lds4 = reinterpret_cast<uint32_t*>(lds) + 4;
+    for (int c = block; c * kCoordBlock < n; c += P.blocks) {
+        // weight before this chunk and in total
+        uint32_t before = 0, total = 0;
+        for (int g = threadIdx.x; g < groups; g += kCoordBlock) {
+            const uint32_t v = (uint32_t)P.wsum[g];
+            total += v;
+            if (g < c * 4) before += v;
+        }
+        const int row = c * kCoordBlock + threadIdx.x;
+        const int mine = row < n ? P.w[row] : 0;
+        const int prev_w = row < n && row > 0 ? P.w[row - 1] : 0;
+        before = block_sum(before, lds4);
+        total = block_sum(total, lds4);
+        // inclusive scan of the chunk's row weights
+        int inc = mine;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(inc, d, 64);
+            if (lane >= d) inc += o;
+        }
+        if (lane == 63) s_wave[wave] = inc;
+        __syncthreads();
+        int excl = (int)before + inc - mine;  // weight of all rows before this one
+        for (int v = 0; v < wave; ++v) excl += s_wave[v];
+        // W is kept above the heaviest possible row: a row then advances the tile id by at most one, so every id
+        // up to the last gets its start written (with few rows -- fewer than tiles -- total / tiles would fall
+        // below a row's weight, ids would skip, and the skipped entries of the table would be read unwritten)
+        int W = ((int)total + tiles - 1) / tiles;
+        W = W > kGemmMaxOffsets + P.row_weight ? W : kGemmMaxOffsets + P.row_weight + 1;
+        if (row < n) {
+            const int id = excl / W;
+            const int prev = row == 0 ? -1 : (excl - prev_w) / W;
+            int32_t* start = P.hdr + 4;
+            if (id != prev) start[id] = row;  // ids grow by at most one per row (W exceeds every row weight)
+            if (row == n - 1) {
+                start[id + 1] = n;
+                P.hdr[1] = W;
+                P.hdr[2] = (int)total;
+                P.hdr[0] = id + 1;
+            }
+        }
+        __syncthreads();
+    }
+}
+
+template <int N>
+struct NumberCuts {
+    SpPart number, next;
+    int number_blocks, has_next;
+    CutPart cut[kMaxCuts];
+    int n_cut;
+    CleanPart clean;
+    FillPlan<N> also;
+};
+
+template <int N>
+__global__ void __launch_bounds__(kCoordBlock) number_cuts(NumberCuts<N> a) {
+    __shared__ uint32_t lds[8];
+    __shared__ int4 s_rows[kCoordBlock];
+    __shared__ InsertLds L;
+    int b = blockIdx.x;
+    if (b < a.number_blocks) return sp_number_pass(a.number, a.next, a.has_next != 0, b, a.number_blocks, lds, s_rows, L);
+    b -= a.number_blocks;
+    for (int l = 0; l < a.n_cut; ++l) {
+        if (b < a.cut[l].blocks) return cut_pass(a.cut[l], b, reinterpret_cast<int32_t*>(lds));
+        b -= a.cut[l].blocks;
+    }
+    if (b < a.clean.blocks) return clean_pass(a.clean, b);
+    fill_pass(a.also, b - a.clean.blocks);
+}
+
+// rulebook of a strided layer on its own: one store per ticket into the rows sp_number has initialised
+__global__ void __launch_bounds__(kCoordBlock) sp_scatter(SpPart P) {
+    const int n = clamp_rows(P.in_num, P.max_voxels);
+    const CellView t = open_table(P.t, n);
+    const int64_t tickets = (int64_t)n * P.Kc;
+    for (int64_t tk = (int64_t)blockIdx.x * kCoordBlock + threadIdx.x; tk < tickets; tk += (int64_t)gridDim.x * kCoordBlock) {
+        const uint32_t c = P.cand[tk];
+        if (c == kEmpty) continue;
+        const uint32_t id = value_at(t, c & kSlotMask);
+        if (id == kEmpty) continue;
+        P.nbr[(size_t)(c >> kSlotBits) * P.max_voxels + id] = (int32_t)(tk / P.Kc);  // unique (offset, out row): plain store
+    }
+}
+
+// weights of the rows of a rulebook that was scattered: 256 rows per block, four threads per row (each sums every
+// fourth offset)
+constexpr int kSplit = 4;
+__global__ void __launch_bounds__(kCoordBlock * kSplit)
+tile_weights(const int32_t* __restrict__ nbr, const int32_t* __restrict__ num_out, int max_voxels, int K, int row_weight,
+             int32_t* __restrict__ w, int32_t* __restrict__ wsum) {
+    __shared__ int32_t s_cnt[kSplit][kCoordBlock];
+    const int n = clamp_rows(num_out, max_voxels);
+    if ((int)blockIdx.x * kCoordBlock >= n) return;
+    const int r = threadIdx.x % kCoordBlock, kg = threadIdx.x / kCoordBlock;
+    const int row = blockIdx.x * kCoordBlock + r;
+    int c = 0;
+    if (row < n) {
+        constexpr int kPer = (kGemmMaxOffsets + kSplit - 1) / kSplit;
+        int32_t e[kPer];  // all loads of the thread are requested before the first is used
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+            const int k = kg + j * kSplit;
+            e[j] = k < K ? nbr[(size_t)k * max_voxels + row] : -1;
+        }
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) c += e[j] >= 0 ? 1 : 0;
+    }
+    s_cnt[kg][r] = c;
+    __syncthreads();
+    if (kg != 0) return;
+    int v = 0;
+    if (row < n) {
+        v = row_weight;
+#pragma unroll
+        for (int g = 0; g < kSplit; ++g) v += s_cnt[g][r];
+    }
+    if (row < max_voxels) w[row] = v;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
+    if ((r & 63) == 0 && row < n) wsum[row >> 6] = v;
+}
+
+}  // namespace
+
+int sp_pass_blocks(const SpPart& s) { return s.n_chunks < kMaxPassBlocks ? s.n_chunks : kMaxPassBlocks; }
+int lookup_blocks(int max_voxels) {
+    const int b = ceil_div(max_voxels, kLookupRows);
+    return b < kMaxPassBlocks ? b : kMaxPassBlocks;
+}
+
+static int clean_blocks(int max_voxels) {
+    const int b = ceil_div(max_voxels, kCoordBlock);
+    return b < 128 ? b : 128;
+}
+
+template <int N>
+static int vg_insert_n(const VgPart& v, const Cleans& cleans, int n_clean_blocks, const FillArgs& also, hipStream_t stream) {
+    FillPlan<N> plan;
+    const int blocks = make_fill_plan(also, plan);
+    if (blocks < 0) return fail(SESSD_E_INVALID, "fill: a region is not 16-byte aligned");
+    hipLaunchKernelGGL(vg_insert<N>, dim3(v.n_blocks + n_clean_blocks + blocks), dim3(kCoordBlock), 0, stream, v, cleans, plan);
+    SESSD_HIP_TRY(hipGetLastError());
+    return SESSD_OK;
+}
+int launch_vg_insert(const VgPart& v, const CleanPart* cleans, int n_cleans, const FillArgs& also, hipStream_t stream) {
+    if (n_cleans < 0 || n_cleans > kMaxCleans) return fail(SESSD_E_INVALID, "vg_insert: at most %d tables are cleaned beside it", kMaxCleans);
+    Cleans c;
+    c.n = n_cleans;
+    int total = 0;
+    for (int i = 0; i < n_cleans; ++i) {
+        c.c[i] = cleans[i];
+        c.c[i].blocks = clean_blocks(cleans[i].max_voxels);
+        total += c.c[i].blocks;
+    }
+    return also.n <= kFewRegions ? vg_insert_n<kFewRegions>(v, c, total, also, stream)
+                                 : vg_insert_n<FillArgs::kMaxRegions>(v, c, total, also, stream);
+}
+
+template <int N>
+static int vg_flags_n(const VgPart& v, const FillArgs& also, hipStream_t stream) {
+    FillPlan<N> plan;
+    const int blocks = make_fill_plan(also, plan);
+    if (blocks < 0) return fail(SESSD_E_INVALID, "fill: a region is not 16-byte aligned");
+    hipLaunchKernelGGL(vg_flags<N>, dim3(v.n_blocks + blocks), dim3(kCoordBlock), 0, stream, v, plan);
+    SESSD_HIP_TRY(hipGetLastError());
+    return SESSD_OK;
+}
+int launch_vg_flags(const VgPart& v, const FillArgs& also, hipStream_t stream) {
+    return also.n <= kFewRegions ? vg_flags_n<kFewRegions>(v, also, stream) : vg_flags_n<FillArgs::kMaxRegions>(v, also, stream);
+}
+
+int launch_vg_finalize(const VgPart& v, const SpPart* next, hipStream_t stream) {
+    hipLaunchKernelGGL(vg_finalize, dim3(ceil_div(v.max_points, kFinalPoints)), dim3(kCoordBlock), 0, stream, v,
+                       next ? *next : SpPart(), next ? 1 : 0);
+    SESSD_HIP_TRY(hipGetLastError());
+    return SESSD_OK;
+}
+
+int launch_sp_insert(const SpPart& s, hipStream_t stream) {
+    const int per = kTicketsAtOnce / s.Kc > 0 ? kTicketsAtOnce / s.Kc : 1;
+    const int blocks = ceil_div(s.max_voxels, per);
+    hipLaunchKernelGGL(sp_insert, dim3(blocks < 2 * kMaxPassBlocks ? blocks : 2 * kMaxPassBlocks), dim3(kCoordBlock), 0, stream, s);
+    SESSD_HIP_TRY(hipGetLastError());
+    return SESSD_OK;
+}
+
+int launch_flags_lookups(const SpPart* flags, const LookupPart* lookups, int n, hipStream_t stream) {
+    if (n < 0 || n > kMaxLookups) return fail(SESSD_E_INVALID, "lookups: at most %d in one launch", kMaxLookups);
+    FlagsLookups a;
+    a.flag_blocks = 0;
+    if (flags) {
+        a.flags = *flags;
+        a.flag_blocks = sp_pass_blocks(*flags);
+    }
+    int blocks = a.flag_blocks;
+    a.n_look = n;
+    for (int l = 0; l < n; ++l) {
+        a.look[l] = lookups[l];
+        a.look[l].blocks = lookup_blocks(lookups[l].max_voxels);
+        blocks += a.look[l].blocks;
+    }
+    if (!blocks) return SESSD_OK;
+    hipLaunchKernelGGL(flags_lookups, dim3(blocks), dim3(kCoordBlock), 0, stream, a);
+    SESSD_HIP_TRY(hipGetLastError());
+    return SESSD_OK;
+}
+
+int launch_number(const SpPart* number, const SpPart* next, const CutPart* cuts, int n_cuts, const CleanPart* clean, const FillArgs* also,
+                  hipStream_t stream) {
+    if (n_cuts < 0 || n_cuts > kMaxCuts) return fail(SESSD_E_INVALID, "tile cuts: at most %d in one launch", kMaxCuts);
+    NumberCuts<1> a;
+    a.number_blocks = a.has_next = 0;
+    if (number) {
+        a.number = *number;
+        a.number_blocks = sp_pass_blocks(*number);
+        if (next) {
+            a.next = *next;
+            a.has_next = 1;
+        }
+    }
+    int blocks = a.number_blocks;
+    a.n_cut = n_cuts;
+    for (int l = 0; l < n_cuts; ++l) {
+        a.cut[l] = cuts[l];
+        blocks += a.cut[l].blocks;
+    }
+    if (clean) {
+        a.clean = *clean;
+        a.clean.blocks = clean_blocks(clean->max_voxels);
+        blocks += a.clean.blocks;
+    }
+    FillArgs none;
+    if (also && also->n > 1) return fail(SESSD_E_INVALID, "numbering: one region can be cleared beside it");
+    const int fill_blocks = make_fill_plan(also ? *also : none, a.also);
+    if (fill_blocks < 0) return fail(SESSD_E_INVALID, "fill: a region is not 16-byte aligned");
+    blocks += fill_blocks;
+    if (!blocks) return SESSD_OK;
+    hipLaunchKernelGGL(number_cuts<1>, dim3(blocks), dim3(kCoordBlock), 0, stream, a);
+    SESSD_HIP_TRY(hipGetLastError());
+    return SESSD_OK;
+}
+
+int launch_sp_scatter(const SpPart& s, hipStream_t stream) {
+    hipLaunchKernelGGL(sp_scatter, dim3(sp_pass_blocks(s)), dim3(kCoordBlock), 0, stream, s);
+    SESSD_HIP_TRY(hipGetLastError());
+    return SESSD_OK;
+}
+
+int launch_tile_weights(const int32_t* nbr, const int32_t* num_out, int K, int max_voxels, int row_weight, void* region, hipStream_t stream) {
+    hipLaunchKernelGGL(tile_weights, dim3(ceil_div(max_voxels, kCoordBlock)), dim3(kCoordBlock * kSplit), 0, stream, nbr, num_out,
+                       max_voxels, K, row_weight, tile_weight_array(region, max_voxels), tile_weight_sums(region, max_voxels));
+    SESSD_HIP_TRY(hipGetLastError());
+    return SESSD_OK;
+}
+
+}  // namespace sessd

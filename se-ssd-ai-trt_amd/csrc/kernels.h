@@ -21,7 +21,7 @@ struct GemmArgs {
     int relu;
     int write_pad_rows;      // rows >= *num_out get epilogue(0) (the reference zero-fills them)
     int force_valu;          // skip the MFMA kernels (cross-check)
-    const int32_t* tiles;    // tile cuts of this rulebook (launch_tile_cuts) or null: tiles of equal length
+    const int32_t* tiles;    // tile cuts of this rulebook (tile_cut.hip) or null: tiles of equal length
     DenseTarget dense;       // dense.dense != null: also scatter the rows there (MFMA kernel only)
 };
 
@@ -64,13 +64,9 @@ __host__ __device__ inline int wide_log2_split(int n, int K, int num_cu) {
 int gemm_tile_rows(int cin, int cout, int dtype);
 int gemm_compute_units();
 
-// equal-work tile cuts for the MFMA kernel, written into `region` (tile_cut_bytes() bytes of the layer's
-// workspace; its first word must be zero before the launch and stays zero when there are no active rows);
-// target_rows >= kGemmMinTileRows is the tile height aimed at; `wide`: for the
-// one-tile-per-unit kernel, whose workgroups may share a tile (wide_log2_split())
+// bytes of a layer's workspace for the equal-work tile cuts of its rulebook (tile_cut.hip, coord.h); the region's first
+// word is the tile count, 0 = none
 size_t tile_cut_bytes(int max_voxels);
-int launch_tile_cuts(const int32_t* nbr, const int32_t* num_out, int K, int max_voxels, int target_rows, int row_weight,
-                     bool wide, void* region, hipStream_t stream);
 
 // picks the kernel for the layer shape; returns SESSD_E_UNSUPPORTED for dtype pairs not covered, and when a
 // dense target is set but the layer does not run on the MFMA kernel (see gemm_runs_on_mfma)

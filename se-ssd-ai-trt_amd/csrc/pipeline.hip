@@ -44,6 +44,9 @@ struct ConvStage {
     std::unique_ptr<SubmConv3dLayerPlugin> subm;
     std::unique_ptr<SparseConv3dLayerPlugin> sparse;
     DeviceBuffer ws, feat, coors, num;  // coors/num only for sparse layers (they produce new ones)
+    // Sparse layers: output cell -> row, one word per cell of the output grid (47 MB for 21 x 800 x 704), kept from
+    // frame to frame and emptied row by row; empty where the grid is too large for that (the workspace's table then)
+    DeviceBuffer cells;
     int rulebook_from = -1;             // SubM layer whose workspace holds this layer's rulebook
     sessd_tensor_desc in_desc[3], out_desc[3];
     void* coors_ptr = nullptr;  // coordinates valid AFTER this layer
@@ -73,6 +76,7 @@ struct Pipeline {
     std::unique_ptr<Sparse2DensePlugin> s2d;
     std::vector<std::unique_ptr<ConvStage>> stages;
     DeviceBuffer vg_ws, vg_voxels, vg_coors, vg_num, s2d_ws;
+    DeviceBuffer vg_cells;  // the voxelizer's cell table, one word per cell (369 MB for 40 x 1600 x 1408), as ConvStage::cells
     sessd_tensor_desc vg_in[2], vg_out[3], s2d_in[3], s2d_out[1];
     int max_voxels = 0;
     size_t device_bytes = 0;
@@ -88,11 +92,16 @@ struct Pipeline {
     int64_t next_ticket = 0;
     int last_replica = 0;                       // replica of the last submitted frame (layer_io, status, stats)
 
-    // two-stream schedule: the frame's clears and the rulebook builds on `aux`; the voxelizer, the lookups on its
-    // voxels and the feature chain on the caller's stream; ev_build[l] = "rulebook of layer l is ready"
+    // two-stream schedule: the voxelizer, the lookups on its voxels and the feature chain on the caller's stream, the
+    // coordinate passes behind them on `aux`; ev_pass[i] = "coordinate pass i is done" (CoordPass)
     hipStream_t aux = nullptr;
-    hipEvent_t ev_start = nullptr, ev_vg = nullptr, ev_fill = nullptr;
-    std::vector<hipEvent_t> ev_build;
+    hipEvent_t ev_head = nullptr;
+    std::vector<hipEvent_t> ev_pass;
+    // The voxelizer's cell table is empty at the start of a frame: a pass behind its last reader empties it for the next
+    // one (a clear at the head of a frame was 4-6 us of every frame).  The strided layers' dense tables hold the rows
+    // of the frame before, as their coors tensors do.  False: clear them first (the first frame, one that did not get
+    // to its end, or one that has run plugin by plugin).
+    bool tables_ready = false;
 
     // profiling: one event per segment boundary (see sessd_pipeline_enqueue_timed)
     std::vector<hipEvent_t> events;
@@ -104,156 +113,252 @@ struct Pipeline {
             if (e) (void)hipEventDestroy(e);
         if (frame_stream) (void)hipStreamDestroy(frame_stream);
         for (hipEvent_t e : events) (void)hipEventDestroy(e);
-        for (hipEvent_t e : ev_build)
+        for (hipEvent_t e : ev_pass)
             if (e) (void)hipEventDestroy(e);
-        if (ev_start) (void)hipEventDestroy(ev_start);
-        if (ev_vg) (void)hipEventDestroy(ev_vg);
-        if (ev_fill) (void)hipEventDestroy(ev_fill);
+        if (ev_head) (void)hipEventDestroy(ev_head);
         if (aux) (void)hipStreamDestroy(aux);
     }
 
-    // The rulebooks depend only on coordinates, the GEMMs on rulebooks + features.  The coordinate chain
-    // (voxelizer, then every layer's rulebook build in order) runs on `aux`; the GEMM chain on `stream`
-    // waits per layer for the rulebook it needs, so the small build kernels of later layers overlap the
-    // GEMMs of earlier ones.  Under stream capture the fork/join becomes two branches of the graph.
-    // Whether the last layer's gather-GEMM scatters into the dense tensor itself (overlapped schedule, matrix-core
-    // kernel, same element type).  The tensor is then cleared on the fill branch, beside the GEMMs, and nothing
-    // follows the last GEMM; the plugin's own cell-major pass writes fewer bytes but puts two more launches at the
-    // end of the critical path (measured: frames 20-40 us longer).
+    // Whether the last layer's gather-GEMM scatters into the dense tensor itself (matrix-core kernel, same element
+    // type).  The tensor is then cleared beside the voxelizer's first pass and nothing follows the last GEMM; the
+    // plugin's own cell-major pass writes fewer bytes but puts two more launches at the end of the critical path
+    // (measured: frames 20-40 us longer).
     bool denseByEpilogue() const {
-        if (stages.empty() || !aux) return false;
+        if (stages.empty()) return false;
         const ConvStage& st = *stages.back();
         const ConvPluginBase* cp = st.subm ? static_cast<const ConvPluginBase*>(st.subm.get()) : st.sparse.get();
         return cp->out_type_ == s2d->out_type_ && cp->out_channel_ == s2d->feature_map_channel_ && cp->gemmOnMatrixCores();
     }
 
-    int enqueueOverlapped(const void* points, const void* points_size, void* dense, hipStream_t stream) {
-        SESSD_HIP_TRY(hipEventRecord(ev_start, stream));
-        SESSD_HIP_TRY(hipStreamWaitEvent(aux, ev_start, 0));
-        // The kernel that produced a coors tensor has left a cell -> row hash behind (the voxelizer's, or a
-        // strided layer's): a SubM layer on the same grid looks its neighbours up in that table and skips its
-        // own insert pass (and the clear of its own table).  Keys are (z*Y + y)*X + x: the same number in both
-        // grids when X and Y agree; cells of the layer's grid beyond the table's z extent are simply absent.
-        // (Beyond 2^20 slots -- 4 MB of keys, one XCD's L2 -- probing the upstream table costs more than the
-        // insert pass it saves.)  The first 3x3x3 SubM rulebook behind a producer is built with the symmetric
-        // lookup (13 probes per row instead of 27): the producer initialises the mirrored entries of the rows
-        // it creates (MirrorInit).
-        std::vector<char> probes_upstream(stages.size(), 0), mirrored(stages.size(), 0);
-        std::vector<MirrorInit> mirror_of(stages.size() + 1);  // [0]: the voxelizer, [l + 1]: strided stage l
-        {
-            uint32_t mask = vg->cellTable(vg_ws.p, desc.max_points).mask;
-            int cx = vg->grid_x_size_, cy = vg->grid_y_size_, cz = vg->grid_z_size_;
-            size_t producer = 0;
-            for (size_t l = 0; l < stages.size(); ++l) {
-                ConvStage& st = *stages[l];
-                if (st.subm) {
-                    probes_upstream[l] = st.rulebook_from < 0 && st.subm->out_shape_x_ == cx &&
-                                         st.subm->out_shape_y_ == cy && st.subm->out_shape_z_ >= cz && mask < (1u << 20);
-                    if (probes_upstream[l] && !mirror_of[producer].nbr) {
-                        const MirrorInit m = st.subm->mirrorInit(st.ws.p);
-                        if (m.nbr) {
-                            mirror_of[producer] = m;
-                            mirrored[l] = 1;
-                        }
-                    }
+    CellTable cellTable(const ConvStage& st) const {
+        CellTable t = st.sparse->cellTable(st.ws.p);
+        if (st.cells.p) {
+            t.base = st.cells.p;
+            t.cap = (uint32_t)(st.cells.bytes / sizeof(uint32_t));
+            t.dense = 1;
+        }
+        return t;
+    }
+    CellTable voxelTable() const {
+        CellTable t = vg->cellTable(vg_ws.p, desc.max_points);
+        if (vg_cells.p) {
+            t.base = vg_cells.p;
+            t.cap = (uint32_t)(vg_cells.bytes / sizeof(uint32_t));
+            t.dense = 1;
+        }
+        return t;
+    }
+    int clearTables(hipStream_t stream) {
+        FillArgs f;
+        vg->collectTableFill(vg_ws.p, desc.max_points, false, f);
+        if (vg_cells.p) f.add(vg_cells.p, vg_cells.bytes / sizeof(uint32_t), kEmpty);
+        for (auto& st : stages) {
+            if (!st->sparse || !st->cells.p) continue;
+            if (f.n + 2 > FillArgs::kMaxRegions) {
+                SESSD_TRY(launch_fill(f, stream));
+                f = FillArgs();
+            }
+            f.add(st->cells.p, st->cells.bytes / sizeof(uint32_t), kEmpty);
+            f.add(st->num.p, 4, 0);  // (no rows of a frame before)
+        }
+        SESSD_TRY(launch_fill(f, stream));
+        tables_ready = true;
+        return SESSD_OK;
+    }
+
+    // The rows of stage 0 are the voxels, those of stage i the output rows of the i-th strided layer.
+    struct Stage {
+        int layer = -1;            // the strided layer that makes the rows (-1: the voxelizer)
+        std::vector<int> lookups;  // layers whose rulebook is looked up once the rows are numbered
+        std::vector<int> builds;   // SubM layers on a grid of their own: the plugin's own build
+    };
+    std::vector<Stage> coordStages() const {
+        std::vector<Stage> v(1);
+        int gx = vg->grid_x_size_, gy = vg->grid_y_size_, gz = vg->grid_z_size_;
+        for (size_t l = 0; l < stages.size(); ++l) {
+            const ConvStage& st = *stages[l];
+            if (st.sparse) {
+                v.emplace_back();
+                v.back().layer = (int)l;
+                v.back().lookups.push_back((int)l);
+                gx = st.sparse->out_shape_x_;
+                gy = st.sparse->out_shape_y_;
+                gz = st.sparse->out_shape_z_;
+            } else if (st.rulebook_from < 0) {
+                // The pass that numbers a stage's rows leaves a cell -> row table behind.  Keys are (z*Y + y)*X + x: the
+                // same number in both grids when X and Y agree; cells of the layer's grid beyond the table's z extent
+                // are simply absent.
+                const bool same = st.subm->out_shape_x_ == gx && st.subm->out_shape_y_ == gy && st.subm->out_shape_z_ >= gz;
+                (same ? v.back().lookups : v.back().builds).push_back((int)l);
+            }
+        }
+        return v;
+    }
+
+    // One frame.  The rulebooks depend only on coordinates, the GEMMs on rulebooks + features.  The coordinate chain
+    // (coord.h) is  vg_insert | vg_flags | vg_finalize + insert 1 | then per stage i: flags i+1 + lookups on stage i |
+    // number i+1 + insert i+2 + tile cuts of those rulebooks.  With `aux`, everything behind the lookups on the voxels
+    // runs there and the GEMM chain waits per layer for the pass its rulebook comes from, so that the passes of later
+    // layers overlap the GEMMs of earlier ones; under stream capture that becomes two branches of the graph.
+    int enqueueFrame(const void* points, const void* points_size, void* dense, hipStream_t stream) {
+        tables_ready = false;  // (until the pass that cleans it is enqueued)
+        const std::vector<Stage> cs = coordStages();
+        const int m = (int)cs.size() - 1;  // strided layers
+        const int V = max_voxels;
+        // rows and table of every stage
+        struct Rows {
+            const int32_t *coors, *num;
+            CellTable table;
+            const int32_t* table_num;  // the row count the table was opened with
+            int table_max;
+        };
+        std::vector<Rows> rows(cs.size());
+        rows[0] = {static_cast<const int32_t*>(vg_coors.p), static_cast<const int32_t*>(vg_num.p), voxelTable(),
+                   static_cast<const int32_t*>(points_size), desc.max_points};
+        std::vector<SpPart> part(cs.size());
+        // cleared beside vg_insert: the cells of the last frame's rows, the dense tensor; beside vg_flags: coordinate
+        // rows beyond the active ones where the flags ask for them (the cells are found by them)
+        FillArgs clears, pads;
+        std::vector<CleanPart> cleans;
+        for (int i = 1; i <= m; ++i) {
+            ConvStage& st = *stages[(size_t)cs[(size_t)i].layer];
+            rows[(size_t)i] = {static_cast<const int32_t*>(st.coors.p), static_cast<const int32_t*>(st.num.p), cellTable(st),
+                               rows[(size_t)i - 1].num, V};
+            part[(size_t)i] = st.sparse->part(rows[(size_t)i - 1].coors, rows[(size_t)i - 1].num, static_cast<int32_t*>(st.coors.p),
+                                              static_cast<int32_t*>(st.num.p), st.ws.p, false);
+            part[(size_t)i].t = rows[(size_t)i].table;
+            if (clears.n + 6 > FillArgs::kMaxRegions || pads.n + 2 > FillArgs::kMaxRegions)
+                return fail(SESSD_E_UNSUPPORTED, "pipeline: more than %d strided layers", FillArgs::kMaxRegions - 6);
+            if (st.cells.p && cleans.size() < (size_t)kMaxCleans) {
+                CleanPart c;
+                c.coors = rows[(size_t)i].coors;
+                c.num = rows[(size_t)i].num;
+                c.max_voxels = V;
+                c.t = rows[(size_t)i].table;
+                cleans.push_back(c);
+            } else if (st.cells.p) {
+                clears.add(st.cells.p, st.cells.bytes / sizeof(uint32_t), kEmpty);
+            } else {
+                st.sparse->collectTableFill(st.ws.p, clears);
+            }
+            st.sparse->collectPadFill(static_cast<int32_t*>(st.coors.p), pads);
+        }
+        vg->collectPadFill(static_cast<float*>(vg_voxels.p), static_cast<int32_t*>(vg_coors.p), clears);
+        if (denseByEpilogue()) s2d->collectFill(dense, s2d_ws.p, clears);
+
+        VgPart v = vg->part(static_cast<const float*>(points), static_cast<const int32_t*>(points_size), desc.max_points,
+                                  desc.point_features, static_cast<float*>(vg_voxels.p), static_cast<int32_t*>(vg_coors.p),
+                                  static_cast<int32_t*>(vg_num.p), vg_ws.p);
+        v.t = rows[0].table;
+        SESSD_TRY(launch_vg_insert(v, cleans.data(), (int)cleans.size(), clears, stream));
+        SESSD_TRY(launch_vg_flags(v, pads, stream));
+        SESSD_TRY(launch_vg_finalize(v, m ? &part[1] : nullptr, stream));
+
+        // Coordinate passes are counted 2i (flags + lookups of stage i) and 2i + 1 (numbering, cuts).  ready[l] = the
+        // pass layer l's rulebook is complete after; pass 0 runs on the caller's stream.
+        std::vector<int> ready(stages.size(), 0);
+        for (int i = 0; i <= m; ++i) {
+            for (int l : cs[(size_t)i].lookups) {
+                const ConvStage& st = *stages[(size_t)l];
+                const bool cuts = st.subm ? st.subm->wantTileCuts() : st.sparse->wantTileCuts();
+                ready[(size_t)l] = 2 * i + (cuts ? 1 : 0);
+            }
+            for (int l : cs[(size_t)i].builds) ready[(size_t)l] = 2 * i + 1;
+        }
+        std::vector<char> awaited((size_t)(2 * m + 2), 0);
+        for (size_t l = 0; l < stages.size(); ++l) awaited[(size_t)ready[l]] = 1;
+        const bool fork = aux != nullptr && stages.size() > 0;
+        hipStream_t side = fork ? aux : stream;
+        int last_side = 0;  // last pass that did something on `side`
+        const int clean_at = m < 1 ? 0 : 1;  // stage 1's own rulebook is the last reader of the voxels' table
+        for (int i = 0; i <= m; ++i) {
+            const Stage& sg = cs[(size_t)i];
+            hipStream_t s = i == 0 ? stream : side;
+            // flags of the next strided layer and the lookups on this stage's rows
+            std::vector<LookupPart> looks;
+            std::vector<CutPart> cuts;
+            for (int l : sg.lookups) {
+                ConvStage& st = *stages[(size_t)l];
+                if (st.sparse) {
+                    const Rows& in = rows[(size_t)i - 1];
+                    looks.push_back(st.sparse->lookupPart(st.ws.p, rows[(size_t)i].coors, rows[(size_t)i].num, in.table, in.table_num, in.table_max));
+                    if (st.sparse->wantTileCuts()) cuts.push_back(st.sparse->cutPart(st.ws.p, rows[(size_t)i].num));
                 } else {
-                    mask = st.sparse->cellTable(st.ws.p).mask;
-                    cx = st.sparse->out_shape_x_;
-                    cy = st.sparse->out_shape_y_;
-                    cz = st.sparse->out_shape_z_;
-                    producer = l + 1;
+                    const Rows& r = rows[(size_t)i];
+                    looks.push_back(st.subm->lookupPart(st.ws.p, r.coors, r.num, r.table, r.table_num, r.table_max));
+                    if (st.subm->wantTileCuts()) cuts.push_back(st.subm->cutPart(st.ws.p, r.num));
                 }
             }
-        }
-        // The head of the frame -- the voxelizer and the lookups of the SubM layers on its voxels, which the first
-        // GEMMs wait for -- runs on the caller's stream itself, in front of those GEMMs: a kernel starts 1-2 us
-        // behind its producer on the same branch of the graph and 5-10 us behind one on another branch.  The
-        // status words of those SubM layers are cleared in the voxelizer's own clear launch.
-        const bool head_off = false;
-        std::vector<char> on_head(stages.size(), 0);
-        FillArgs head_clears;
-        for (size_t l = 0; l < stages.size() && !head_off; ++l) {
-            ConvStage& st = *stages[l];
-            if (!st.subm) break;
-            if (st.rulebook_from >= 0) continue;
-            if (!probes_upstream[l] || !st.ws.p) break;
-            on_head[l] = 1;
-            st.subm->collectFill(st.ws.p, head_clears, false);
-        }
-        hipStream_t head = head_off ? aux : stream;
-        const void* vin[2] = {points, points_size};
-        void* vout[3] = {vg_voxels.p, vg_coors.p, vg_num.p};
-        SESSD_TRY(vg->enqueue(vg_in, vg_out, vin, vout, vg_ws.p, head, mirror_of[0].nbr ? &mirror_of[0] : nullptr, &head_clears));
-        SESSD_HIP_TRY(hipEventRecord(ev_vg, head));
-        // every other clear of the frame (hash tables, neighbour tables, status words, the dense tensor) has no
-        // input: they run batched at the head of `aux`, which has nothing else to do while the voxelizer works (a
-        // stream of their own measured the same)
-        {
-            FillArgs f;
-            auto flush = [&]() -> int {
-                const int rc = launch_fill(f, aux);
-                f = FillArgs();
-                return rc;
-            };
-            for (size_t l = 0; l < stages.size(); ++l) {
-                auto& st = stages[l];
-                if (!st->ws.p || on_head[l]) continue;
-                if (f.n + 6 > FillArgs::kMaxRegions) SESSD_TRY(flush());
-                if (st->subm) st->subm->collectFill(st->ws.p, f, !probes_upstream[l]);
-                else st->sparse->collectFill(st->ws.p, static_cast<int32_t*>(st->coors.p), f);
+            const SpPart* next = i < m ? &part[(size_t)i + 1] : nullptr;
+            size_t at = 0;
+            do {
+                const size_t n = looks.size() - at < (size_t)kMaxLookups ? looks.size() - at : (size_t)kMaxLookups;
+                SESSD_TRY(launch_flags_lookups(at == 0 ? next : nullptr, looks.data() + at, (int)n, s));
+                at += n;
+            } while (at < looks.size());
+            if (i == 0 && fork) {
+                SESSD_HIP_TRY(hipEventRecord(ev_head, stream));
+                SESSD_HIP_TRY(hipStreamWaitEvent(side, ev_head, 0));
+            } else if (fork) {
+                if (awaited[(size_t)(2 * i)]) SESSD_HIP_TRY(hipEventRecord(ev_pass[(size_t)(2 * i)], side));
+                last_side = 2 * i;
             }
-            if (f.n + 2 > FillArgs::kMaxRegions) SESSD_TRY(flush());
-            if (denseByEpilogue()) s2d->collectFill(dense, s2d_ws.p, f);
-            SESSD_TRY(flush());
-            SESSD_HIP_TRY(hipEventRecord(ev_fill, aux));
+            // numbering of the next strided layer's rows (their tickets for the layer behind it), tile cuts
+            FillArgs clear;
+            CleanPart clean;
+            if (i == clean_at && vg_cells.p) {
+                clean.coors = rows[0].coors;
+                clean.num = rows[0].num;
+                clean.max_voxels = desc.voxelgen.max_voxels;
+                clean.t = rows[0].table;
+            } else if (i == clean_at) {
+                vg->collectTableFill(vg_ws.p, desc.max_points, true, clear);
+            }
+            const SpPart* after = i + 1 < m ? &part[(size_t)i + 2] : nullptr;
+            at = 0;
+            bool did = false;
+            while (at < cuts.size() || (!did && (next || i == clean_at))) {
+                const size_t n = cuts.size() - at < (size_t)kMaxCuts ? cuts.size() - at : (size_t)kMaxCuts;
+                SESSD_TRY(launch_number(did ? nullptr : next, did ? nullptr : after, cuts.data() + at, (int)n, did || !clean.coors ? nullptr : &clean,
+                                        did ? nullptr : &clear, side));
+                at += n;
+                did = true;
+            }
+            if (i == clean_at) tables_ready = true;
+            for (int l : sg.builds) {
+                ConvStage& st = *stages[(size_t)l];
+                SESSD_TRY(st.subm->enqueueBuild(rows[(size_t)i].coors, rows[(size_t)i].num, st.ws.p, side));
+                did = true;
+            }
+            if (fork && did) {
+                last_side = 2 * i + 1;
+                SESSD_HIP_TRY(hipEventRecord(ev_pass[(size_t)last_side], side));
+            }
         }
-        if (!head_off) SESSD_HIP_TRY(hipStreamWaitEvent(aux, ev_vg, 0));
+        if (fork && last_side > 0 && last_side % 2 == 0 && !awaited[(size_t)last_side]) SESSD_HIP_TRY(hipEventRecord(ev_pass[(size_t)last_side], side));
+
+        // the feature chain
+        const void* feat = vg_voxels.p;
         const int32_t* coors = static_cast<const int32_t*>(vg_coors.p);
         const int32_t* num = static_cast<const int32_t*>(vg_num.p);
-        HashTable cells = vg->cellTable(vg_ws.p, desc.max_points);  // the table upstream of the current layer
-        for (size_t l = 0; l < stages.size(); ++l) {
-            ConvStage& st = *stages[l];
-            if (st.subm) {
-                if (st.rulebook_from >= 0) continue;
-                SESSD_TRY(st.subm->enqueueBuild(coors, num, st.ws.p, on_head[l] ? stream : aux, true,
-                                                probes_upstream[l] ? &cells : nullptr, mirrored[l] != 0));
-                if (on_head[l]) continue;  // (its GEMM follows on the same stream: no event)
-            } else {
-                SESSD_TRY(st.sparse->enqueueBuild(coors, num, static_cast<int32_t*>(st.coors.p),
-                                                  static_cast<int32_t*>(st.num.p), st.ws.p, aux, true,
-                                                  mirror_of[l + 1].nbr ? &mirror_of[l + 1] : nullptr));
-                coors = static_cast<const int32_t*>(st.coors.p);
-                num = static_cast<const int32_t*>(st.num.p);
-                cells = st.sparse->cellTable(st.ws.p);
-            }
-            SESSD_HIP_TRY(hipEventRecord(ev_build[l], aux));
-        }
-        if (head_off) SESSD_HIP_TRY(hipStreamWaitEvent(stream, ev_vg, 0));
-        const void* feat = vg_voxels.p;
-        coors = static_cast<const int32_t*>(vg_coors.p);
-        num = static_cast<const int32_t*>(vg_num.p);
-        int last_waited = -1;
+        int last_waited = 0;
         bool scattered = false;
         for (size_t l = 0; l < stages.size(); ++l) {
             ConvStage& st = *stages[l];
             const int owner = st.rulebook_from >= 0 ? st.rulebook_from : (int)l;
-            if (owner > last_waited) {
-                if (!on_head[(size_t)owner]) SESSD_HIP_TRY(hipStreamWaitEvent(stream, ev_build[owner], 0));
-                last_waited = owner;
+            if (fork && ready[(size_t)owner] > last_waited) {
+                last_waited = ready[(size_t)owner];
+                SESSD_HIP_TRY(hipStreamWaitEvent(stream, ev_pass[(size_t)last_waited], 0));
             }
-            // the last layer's epilogue also writes the dense tensor when it runs on the matrix cores and its
-            // rows have the dense tensor's element type: the scatter kernel and its launch drop off the end
-            // of the critical path
             DenseTarget dt;
             const bool fuse = l + 1 == stages.size() && denseByEpilogue();
             if (fuse) {
-                SESSD_HIP_TRY(hipStreamWaitEvent(stream, ev_fill, 0));
                 const int32_t* oc = st.subm ? coors : static_cast<const int32_t*>(st.coors.p);
                 dt = s2d->denseTarget(dense, oc, s2d_ws.p);
                 scattered = true;
             }
             if (st.subm) {
-                SESSD_TRY(st.subm->enqueueGemm(feat, st.feat.p, num, stages[owner]->ws.p, stream, fuse ? &dt : nullptr));
+                SESSD_TRY(st.subm->enqueueGemm(feat, st.feat.p, num, stages[(size_t)owner]->ws.p, stream, fuse ? &dt : nullptr));
             } else {
                 SESSD_TRY(st.sparse->enqueueGemm(feat, st.feat.p, static_cast<const int32_t*>(st.num.p), st.ws.p, stream,
                                                  fuse ? &dt : nullptr));
@@ -262,22 +367,14 @@ struct Pipeline {
             }
             feat = st.feat.p;
         }
+        if (fork && last_side > last_waited) SESSD_HIP_TRY(hipStreamWaitEvent(stream, ev_pass[(size_t)last_side], 0));  // join
         if (scattered) return SESSD_OK;
-        // every event of `aux` has been waited on by now (the last build is the last aux operation)
-        if (stages.empty()) SESSD_HIP_TRY(hipStreamWaitEvent(stream, ev_vg, 0));
-        SESSD_HIP_TRY(hipStreamWaitEvent(stream, ev_fill, 0));
         const void* din[3] = {feat, coors, num};
         void* dout[1] = {dense};
         return s2d->enqueue(s2d_in, s2d_out, din, dout, s2d_ws.p, stream);
     }
 
-    int enqueueDirect(const void* points, const void* points_size, void* dense, hipStream_t stream) {
-        const void* vin[2] = {points, points_size};
-        void* vout[3] = {vg_voxels.p, vg_coors.p, vg_num.p};
-        SESSD_TRY(vg->enqueue(vg_in, vg_out, vin, vout, vg_ws.p, stream));
-        return enqueueAfterVoxelizer(dense, stream);
-    }
-
+    // plugin by plugin, each with its own clears and tables (enqueue_timed: what each of them costs alone)
     int enqueueAfterVoxelizer(void* dense, hipStream_t stream) {
         const void* feat = vg_voxels.p;
         const void* coors = vg_coors.p;
@@ -304,6 +401,11 @@ struct Pipeline {
         return s2d->enqueue(s2d_in, s2d_out, din, dout, s2d_ws.p, stream);
     }
 };
+
+// largest output grid that gets a dense table (a ticket keeps its cell in 26 bits)
+constexpr uint64_t kDenseCells = 1ull << 25;
+// ... and largest voxel grid
+constexpr uint64_t kDenseVoxelCells = 1ull << 27;
 
 static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
     if (d.n_layers < 0 || (d.n_layers && (!d.layers || !d.weights)))
@@ -335,7 +437,9 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
     SESSD_TRY(P->vg_voxels.alloc((size_t)V * 4 * sizeof(float)));
     SESSD_TRY(P->vg_coors.alloc((size_t)V * 4 * sizeof(int32_t)));
     SESSD_TRY(P->vg_num.alloc(256));
-    total += P->vg_ws.bytes + P->vg_voxels.bytes + P->vg_coors.bytes + 256;
+    const uint64_t cells = (uint64_t)vg->grid_x_size_ * (uint64_t)vg->grid_y_size_ * (uint64_t)vg->grid_z_size_;
+    if (cells <= kDenseVoxelCells) SESSD_TRY(P->vg_cells.alloc(cells * sizeof(uint32_t)));
+    total += P->vg_ws.bytes + P->vg_voxels.bytes + P->vg_coors.bytes + P->vg_cells.bytes + 256;
 
     int in_type = SESSD_FLOAT;  // the voxelizer's means are FP32
     int in_ch = 4;
@@ -403,6 +507,8 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
             SESSD_TRY(st->ws.alloc(p->getWorkspaceSize(st->in_desc, 3, st->out_desc, 3)));
             SESSD_TRY(st->coors.alloc((size_t)V * 4 * sizeof(int32_t)));
             SESSD_TRY(st->num.alloc(256));
+            const uint64_t volume = (uint64_t)s.out_shape[0] * (uint64_t)s.out_shape[1] * (uint64_t)s.out_shape[2];
+            if (volume <= kDenseCells) SESSD_TRY(st->cells.alloc(volume * sizeof(uint32_t)));
             last_subm_with_rulebook = -1;  // new coordinates: earlier rulebooks no longer apply
         } else {
             return fail(SESSD_E_INVALID, "pipeline: layer %d has unknown type %d", l, s.type);
@@ -410,7 +516,7 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
         base->flags_ = d.flags;
         SESSD_TRY(base->setEpilogue(d.scale ? d.scale[l] : nullptr, d.shift ? d.shift[l] : nullptr, d.relu));
         SESSD_TRY(st->feat.alloc((size_t)V * s.out_channel * dtype_size(ft)));
-        total += st->ws.bytes + st->feat.bytes + st->coors.bytes + st->num.bytes;
+        total += st->ws.bytes + st->feat.bytes + st->coors.bytes + st->num.bytes + st->cells.bytes;
         in_type = ft;
         in_ch = s.out_channel;
         P->stages.push_back(std::move(st));
@@ -434,11 +540,25 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
     P->device_bytes = total;
     if (d.overlap_streams) {
         SESSD_HIP_TRY(hipStreamCreateWithFlags(&P->aux, hipStreamNonBlocking));
-        SESSD_HIP_TRY(hipEventCreateWithFlags(&P->ev_fill, hipEventDisableTiming));
-        SESSD_HIP_TRY(hipEventCreateWithFlags(&P->ev_start, hipEventDisableTiming));
-        SESSD_HIP_TRY(hipEventCreateWithFlags(&P->ev_vg, hipEventDisableTiming));
-        P->ev_build.assign(P->stages.size(), nullptr);
-        for (auto& e : P->ev_build) SESSD_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        SESSD_HIP_TRY(hipEventCreateWithFlags(&P->ev_head, hipEventDisableTiming));
+        P->ev_pass.assign(2 * P->coordStages().size(), nullptr);
+        for (auto& e : P->ev_pass) SESSD_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    }
+    // what the passes leave as they need it for the next frame has to be right for the first
+    {
+        FillArgs f;
+        f.add(static_cast<uint8_t*>(P->vg_ws.p) + vg->statusOffset(d.max_points), 4, 0);
+        for (auto& st : P->stages) {
+            if (!st->ws.p) continue;
+            if (f.n + 2 > FillArgs::kMaxRegions) {
+                SESSD_TRY(launch_fill(f, nullptr));
+                f = FillArgs();
+            }
+            if (st->subm) st->subm->collectHeaderFill(st->ws.p, f);
+            else st->sparse->collectHeaderFill(st->ws.p, f);
+        }
+        SESSD_TRY(launch_fill(f, nullptr));
+        SESSD_HIP_TRY(hipStreamSynchronize(nullptr));
     }
     // the layer array of the caller need not outlive create()
     P->desc.layers = nullptr;
@@ -536,9 +656,8 @@ static Pipeline* current(sessd_pipeline* h) {
 // one frame on `stream`: a replay of the captured graph when the pipeline uses graphs (re-captured when a pointer
 // changed), direct launches otherwise
 static int run_frame(Pipeline* P, const void* points, const void* points_size, void* dense, hipStream_t stream) {
-    auto run = [&](hipStream_t st) {
-        return P->aux ? P->enqueueOverlapped(points, points_size, dense, st) : P->enqueueDirect(points, points_size, dense, st);
-    };
+    auto run = [&](hipStream_t st) { return P->enqueueFrame(points, points_size, dense, st); };
+    if (!P->tables_ready) SESSD_TRY(P->clearTables(stream));
     if (!P->desc.use_graph || stream == nullptr) return run(stream);
     CapturedGraph& g = P->captured;
     if (!g.exec || g.points != points || g.size != points_size || g.dense != dense) {
@@ -710,6 +829,7 @@ int sessd_pipeline_enqueue_timed(sessd_pipeline* h, const void* points, const vo
     SESSD_HIP_TRY(hipEventRecord(P->events[n_seg + 2], stream));
     SESSD_HIP_TRY(hipEventRecord(P->events[0], stream));
     int rc;
+    P->tables_ready = false;  // (the voxelizer alone leaves its table filled)
     {
         const void* vin[2] = {points, points_size};
         void* vout[3] = {P->vg_voxels.p, P->vg_coors.p, P->vg_num.p};

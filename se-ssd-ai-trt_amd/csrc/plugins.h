@@ -5,7 +5,7 @@
 
 #include <vector>
 
-#include "common.h"
+#include "coord.h"
 
 namespace sessd {
 
@@ -28,11 +28,8 @@ class VoxelGeneratorPlugin {
                         int nbOutputs);
     size_t getWorkspaceSize(const sessd_tensor_desc* inputs, int nbInputs,
                             const sessd_tensor_desc* outputs, int nbOutputs) const;
-    // `mirror`: the neighbour table of the SubM layer that will run its symmetric lookup on these voxels;
-    // `also_clear`: regions cleared in the same launch as the voxelizer's own tables
     int enqueue(const sessd_tensor_desc* inputDesc, const sessd_tensor_desc* outputDesc,
-                const void* const* inputs, void* const* outputs, void* workspace,
-                hipStream_t stream, const MirrorInit* mirror = nullptr, const FillArgs* also_clear = nullptr);
+                const void* const* inputs, void* const* outputs, void* workspace, hipStream_t stream);
     // enqueue() on the library's own static scratch array instead of a caller's workspace: allocates nothing;
     // rejects points tensors whose layout does not fit the array.  Calls that overlap on one GPU race.
     int enqueueStatic(const sessd_tensor_desc* inputDesc, const sessd_tensor_desc* outputDesc,
@@ -41,9 +38,15 @@ class VoxelGeneratorPlugin {
     void serialize(void* buffer) const;
     size_t statusOffset(int max_points) const;
     // After an enqueue the workspace's hash maps linear cell (z*Y + y)*X + x -> voxel row (kEmpty for cells
-    // dropped at the cap): a SubM layer on the same x/y grid can use it as its cell table
-    // (SubmConv3dLayerPlugin::enqueueBuild) instead of inserting every voxel into its own.
-    HashTable cellTable(void* workspace, int max_points) const;
+    // dropped at the cap): a SubM layer on the same x/y grid, and a strided layer, look their rulebooks up in it.
+    CellTable cellTable(void* workspace, int max_points) const;
+    // the passes of an enqueue (coord.h) and what has to be cleared before them: the table, and rows >= voxel_num
+    // where the flags ask for them.  status[1] must be 0 (every enqueue leaves it so).
+    VgPart part(const float* points, const int32_t* points_size, int max_points, int pf, float* voxels, int32_t* coors,
+                int32_t* voxel_num, void* workspace) const;
+    // (table_only: without the places of later points, which an enqueue leaves empty)
+    void collectTableFill(void* workspace, int max_points, bool table_only, FillArgs& f) const;
+    void collectPadFill(float* voxels, int32_t* coors, FillArgs& f) const;
 
     // serialized fields, in the reference's order (voxelGenerator.cu:584-599)
     int voxelNum_ = 0;      // max_voxels
@@ -67,7 +70,6 @@ class VoxelGeneratorPlugin {
 // ---------------------------------------------------------------------------------------------
 // Shared by both conv plugins: device weights (+ epilogue), dtype bookkeeping, GEMM dispatch
 // ---------------------------------------------------------------------------------------------
-bool gemm_runs_tall(int K, int cin, int cout, int in_type, int out_type);  // kernels.h
 // Cin * Cout (of the layer that builds it) from which a rulebook gets equal-work tile cuts.  At 32 x 32 the GEMM
 // measured the same with and without them, and the two launches lengthen the coordinate branch: frame 0.387 -> 0.377 ms.
 constexpr int kTileCutMinWork = 32 * 64;
@@ -107,11 +109,13 @@ class ConvPluginBase {
                 const int32_t* num_out, hipStream_t stream, const DenseTarget* dense = nullptr);
     // whether a rulebook built by this layer gets equal-work tile cuts: worth two small launches when the
     // GEMM runs on the matrix cores and is not tiny
+  public:
     bool wantTileCuts() const {
         return weights_packed_dev_ != nullptr && !(flags_ & SESSD_FLAG_FORCE_VALU) &&
                in_channel_ * out_channel_ >= kTileCutMinWork &&
                !gemm_runs_tall(kernel_volume_, in_channel_, out_channel_, in_type_, out_type_);
     }
+  protected:
     // tile height those cuts aim at: the capacity of this layer's own GEMM kernel
     int tileRows() const;
     // weight of a row beside its pairs in those cuts
@@ -144,15 +148,14 @@ class SubmConv3dLayerPlugin : public ConvPluginBase {
                       const void* const* inputs, void* const* outputs,
                       const void* rulebook_workspace, hipStream_t stream);
     // enqueue = enqueueBuild (coordinates -> rulebook) + enqueueGemm (features)
-    // `cells`: a cell -> row table over this layer's grid that some earlier kernel already built (the
-    // voxelizer's, or that of the strided layer that produced `coors`); the insert pass is skipped then
-    // `mirrored`: the producer of `coors` has initialised this layer's mirrored neighbour entries (mirrorInit()):
-    // the lookup then probes 13 offsets per row instead of 27 and writes both directions of every hit
-    int enqueueBuild(const int32_t* coors, const int32_t* voxel_num, void* workspace, hipStream_t stream,
-                     bool prefilled = false, const HashTable* cells = nullptr, bool mirrored = false);
-    // what the producer of this layer's coors tensor needs for that (nbr == nullptr: this layer cannot use it)
-    MirrorInit mirrorInit(void* workspace) const;
-    void collectFill(void* workspace, FillArgs& f, bool own_table = true) const;
+    int enqueueBuild(const int32_t* coors, const int32_t* voxel_num, void* workspace, hipStream_t stream);
+    // The rulebook from a table that some earlier pass has already built over this layer's grid (the voxelizer's, or
+    // that of the strided layer that produced `coors`), opened with cells_num (at most cells_max) rows.  The header
+    // words (collectHeaderFill) must have been cleared once.
+    LookupPart lookupPart(void* workspace, const int32_t* coors, const int32_t* voxel_num, const CellTable& cells,
+                          const int32_t* cells_num, int cells_max) const;
+    CutPart cutPart(void* workspace, const int32_t* voxel_num) const;
+    void collectHeaderFill(void* workspace, FillArgs& f) const;
     int enqueueGemm(const void* in_feat, void* out_feat, const int32_t* voxel_num,
                     const void* rulebook_workspace, hipStream_t stream, const DenseTarget* dense = nullptr);
     int exportRulebook(const void* workspace, int32_t* indice_pairs, uint32_t* indice_num,
@@ -167,6 +170,7 @@ class SubmConv3dLayerPlugin : public ConvPluginBase {
   private:
     struct Layout;
     Layout carve(void* workspace) const;
+    CellTable ownTable(void* workspace) const;
     int validate() const;
 };
 
@@ -190,10 +194,21 @@ class SparseConv3dLayerPlugin : public ConvPluginBase {
                        hipStream_t stream) const;
     int countPairs(const void* workspace, uint32_t* indice_num, hipStream_t stream) const;
     int enqueueBuild(const int32_t* coors, const int32_t* voxel_num, int32_t* out_coors, int32_t* out_num,
-                     void* workspace, hipStream_t stream, bool prefilled = false, const MirrorInit* mirror = nullptr);
-    // after enqueueBuild the workspace's hash maps output cell -> output row (see VoxelGeneratorPlugin::cellTable)
-    HashTable cellTable(void* workspace) const;
-    void collectFill(void* workspace, int32_t* out_coors, FillArgs& f) const;
+                     void* workspace, hipStream_t stream);
+    // after the numbering the workspace's table maps output cell -> output row (see VoxelGeneratorPlugin::cellTable)
+    CellTable cellTable(void* workspace) const;
+    // the passes of a build (coord.h); scattered: the rulebook is written by sp_scatter, else by the lookup of
+    // lookupPart() in the table of the input rows
+    SpPart part(const int32_t* coors, const int32_t* voxel_num, int32_t* out_coors, int32_t* out_num, void* workspace,
+                bool scattered) const;
+    LookupPart lookupPart(void* workspace, const int32_t* out_coors, const int32_t* out_num, const CellTable& cells,
+                          const int32_t* cells_num, int cells_max) const;
+    CutPart cutPart(void* workspace, const int32_t* out_num) const;
+    // cleared before every build: the table, and out_coors where the flags ask for its rows >= out_num; cleared once:
+    // the header words
+    void collectTableFill(void* workspace, FillArgs& f) const;
+    void collectHeaderFill(void* workspace, FillArgs& f) const;
+    void collectPadFill(int32_t* out_coors, FillArgs& f) const;
     int enqueueGemm(const void* in_feat, void* out_feat, const int32_t* out_num, const void* workspace,
                     hipStream_t stream, const DenseTarget* dense = nullptr);
     size_t getSerializationSize() const;

@@ -9,234 +9,33 @@
 //   sp_flags    one thread per ticket: "am I the first ticket of my cell" -> wave64 ballot words
 //   sp_number   exclusive prefix over the ballot words = output row in first-seen order (the order
 //               of a sequential walk, sparseConv3dlayer.cu:738-757); writes out coors + voxel_num
-//   sp_scatter  one thread per ticket: nbr[offset][out row] = input row
-//   gather-GEMM conv_gemm.hip
+//   sp_scatter  one thread per ticket: nbr[offset][out row] = input row  (in the pipeline, which has the table of the
+//               input rows at hand, the rulebook is looked up instead: LookupPart)
+//   gather-GEMM one launch for all offsets
+// (kernels: coord.hip)
 //
 // No pass touches anything larger than O(active sites); numbering is deterministic.
-#include "kernels.h"
+#include "coord.h"
 #include "plugins.h"
 
 namespace sessd {
 
-namespace {
-
-constexpr int kBlock = 256;
+// cand[] keeps a ticket's table slot in 26 bits
 constexpr uint32_t kSlotBits = 26;
-constexpr uint32_t kSlotMask = (1u << kSlotBits) - 1u;
-
-struct SpParams {
-    int k[3], s[3], p[3], os[3];  // z,y,x
-    int Kc;                       // enumeration slots per input row
-    int max_voxels;
-    int dilation;
-};
-
-__device__ __forceinline__ int clamp_count(const int32_t* p, int cap) {
-    int n = *p;
-    return n < 0 ? 0 : (n > cap ? cap : n);
-}
-
-// getValidOutPosKernel (sparseConv3dlayer.cu:310-386), one enumeration step: candidate `e` of the
-// input cell c.  Integer divisions truncate toward zero exactly as in the reference.
-// -> false when e is past the enumeration or the output cell is outside the grid
-__device__ __forceinline__ bool sp_candidate(const int c[3], const SpParams& P, int e, int o[3], int& offset) {
-    int lo[3], up[3], cs[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        lo[a] = (c[a] - (P.k[a] - 1) * P.dilation - 1 + P.s[a] + P.p[a]) / P.s[a];
-        up[a] = (c[a] + P.p[a]) / P.s[a];
-        cs[a] = (up[a] - lo[a]) / P.dilation + 1;
-    }
-    if (cs[0] <= 0 || cs[1] <= 0 || cs[2] <= 0 || e >= cs[0] * cs[1] * cs[2]) return false;
-    const int cnt[3] = {e / (cs[2] * cs[1]), (e / cs[2]) % cs[1], e % cs[2]};  // x fastest
-    bool valid = true;
-    int m = 1;
-    offset = 0;
-#pragma unroll
-    for (int a = 2; a >= 0; --a) {
-        o[a] = up[a] - cnt[a] * P.dilation;
-        if (o[a] < 0 || o[a] > P.os[a] - 1) valid = false;
-        offset += m * (c[a] - o[a] * P.s[a] + P.p[a]) / P.dilation;
-        m *= P.k[a];
-    }
-    return valid;
-}
-
-// Rows that follow each other name the same output cells again and again (eight input cells share an output cell
-// of a 3x3x3 stride-2 layer, and neighbours in space are mostly neighbours in the row order), and device-wide
-// atomics are what this pass is made of.  A block therefore gathers the cells its 256 tickets name in an LDS table
-// first (cell -> smallest ticket of the block), and one thread per distinct cell goes to the table in memory.
-constexpr int kLocalBits = 9, kLocalSlots = 1 << kLocalBits;  // twice the block's tickets
-
-__global__ void __launch_bounds__(kBlock)
-sp_insert(const int32_t* __restrict__ coors, const int32_t* __restrict__ voxel_num, SpParams P, HashTable t,
-          uint32_t* __restrict__ cand, int32_t* meta) {
-    __shared__ uint32_t s_key[kLocalSlots], s_val[kLocalSlots];
-    const uint32_t tk = blockIdx.x * kBlock + threadIdx.x;
-    const int v = tk / P.Kc, e = tk % P.Kc;
-    const int n = clamp_count(voxel_num, P.max_voxels);
-    if ((int64_t)blockIdx.x * kBlock >= (int64_t)n * P.Kc) return;  // (the whole block is beyond the active rows)
-    for (int i = threadIdx.x; i < kLocalSlots; i += kBlock) {
-        s_key[i] = kEmpty;
-        s_val[i] = kEmpty;
-    }
-    __syncthreads();
-    uint32_t key = kEmpty;
-    int offset = 0, local = -1;
-    bool owner = false;
-    if (v < n) {
-        const int4 cc = reinterpret_cast<const int4*>(coors)[v];
-        const int c[3] = {cc.y, cc.z, cc.w};
-        int o[3];
-        // A negative coordinate makes the truncating divisions of getValidOutPos yield kernel offsets outside [0, K)
-        // (c = -2, k = 3, s = 2, p = 1: o = 0, offset term -1), with which the reference indexes its rulebook.  Such a
-        // row contributes nothing here and raises BAD_COORD; the offset is checked as well, so that nothing a caller
-        // passes can make sp_scatter store outside the neighbour table.
-        const bool bad = c[0] < 0 || c[1] < 0 || c[2] < 0;
-        if (bad && e == 0) atomicOr(&meta[0], SESSD_STATUS_BAD_COORD);
-        if (!bad && sp_candidate(c, P, e, o, offset) && offset >= 0 && offset < P.k[0] * P.k[1] * P.k[2]) {
-            key = ((uint32_t)o[0] * (uint32_t)P.os[1] + (uint32_t)o[1]) * (uint32_t)P.os[2] + (uint32_t)o[2];
-            uint32_t ls = (key * 2654435769u) >> (32 - kLocalBits);
-            for (;;) {  // (at most kBlock keys in 2 * kBlock slots: room is always found)
-                const uint32_t prev = atomicCAS(&s_key[ls], kEmpty, key);
-                if (prev == kEmpty || prev == key) {
-                    owner = prev == kEmpty;
-                    break;
-                }
-                ls = (ls + 1) & (kLocalSlots - 1);
-            }
-            local = (int)ls;
-            atomicMin(&s_val[ls], tk);
-        }
-    }
-    __syncthreads();
-    if (owner) {  // this thread claimed the cell's LDS entry: it carries the block's smallest ticket to memory
-        const int32_t slot = hash_insert(t, key);
-        if (slot < 0) {
-            atomicOr(&meta[0], SESSD_STATUS_HASH_FULL);
-            s_key[local] = kEmpty;  // (read below as "no slot")
-        } else {
-            atomicMin(&t.vals[slot], s_val[local]);
-            s_val[local] = (uint32_t)slot;
-        }
-    }
-    __syncthreads();
-    if (v >= n) return;
-    cand[tk] = (local >= 0 && s_key[local] != kEmpty) ? (((uint32_t)offset << kSlotBits) | s_val[local]) : kEmpty;
-}
-
-__global__ void __launch_bounds__(kBlock)
-sp_flags(const int32_t* __restrict__ voxel_num, SpParams P, HashTable t, const uint32_t* __restrict__ cand,
-         uint64_t* __restrict__ first_words, uint32_t* __restrict__ block_counts) {
-    __shared__ uint32_t lds4[4];
-    const uint32_t tk = blockIdx.x * kBlock + threadIdx.x;
-    const int v = tk / P.Kc;
-    const int n = clamp_count(voxel_num, P.max_voxels);
-    // the grid covers the capacity; a block beyond the tickets of the active rows has nothing to say, and
-    // sp_number reads no word of it
-    if ((int64_t)blockIdx.x * kBlock >= (int64_t)n * P.Kc) return;
-    bool first = false;
-    if (v < n) {
-        const uint32_t c = cand[tk];
-        first = c != kEmpty && t.vals[c & kSlotMask] == tk;
-    }
-    const uint64_t m = __ballot(first);
-    if ((threadIdx.x & 63) == 0) {
-        first_words[tk >> 6] = m;
-        lds4[threadIdx.x >> 6] = __popcll(m);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) block_counts[blockIdx.x] = lds4[0] + lds4[1] + lds4[2] + lds4[3];
-}
-
-__global__ void __launch_bounds__(kBlock)
-sp_number(const int32_t* __restrict__ voxel_num, SpParams P, HashTable t, const uint32_t* __restrict__ cand,
-          const uint64_t* __restrict__ first_words, const uint32_t* __restrict__ block_counts, int n_blocks,
-          int32_t* __restrict__ out_coors, int32_t* __restrict__ out_num, int32_t* __restrict__ nbr, int K, int32_t* meta,
-          MirrorInit mi) {
-    __shared__ uint32_t lds4[4];
-    const int b = blockIdx.x;
-    // Only the blocks that hold tickets of active input rows carry anything (at a capacity of 100 000 rows and
-    // 26 000 active ones, three blocks in four would each add up thousands of counts to find nothing to number).
-    int active = (int)(((int64_t)clamp_count(voxel_num, P.max_voxels) * P.Kc + kBlock - 1) / kBlock);
-    active = active < n_blocks ? active : n_blocks;
-    if (b >= active) {
-        // (no active input row at all: block 0 still owes the count; the words sp_flags left unwritten are not read)
-        if (b == 0 && threadIdx.x == 0) {
-            *out_num = 0;
-            meta[1] = 0;
-        }
-        return;
-    }
-    const int upto = b == 0 ? active : b;  // block 0 computes the total
-    uint32_t part = 0;
-    for (int j = threadIdx.x; j < upto; j += kBlock) part += block_counts[j];
-    for (int off = 32; off > 0; off >>= 1) part += __shfl_down(part, off, 64);
-    if ((threadIdx.x & 63) == 0) lds4[threadIdx.x >> 6] = part;
-    __syncthreads();
-    const uint32_t sum = lds4[0] + lds4[1] + lds4[2] + lds4[3];
-    if (b == 0 && threadIdx.x == 0) {
-        const uint32_t m = sum > (uint32_t)P.max_voxels ? (uint32_t)P.max_voxels : sum;
-        *out_num = (int32_t)m;
-        meta[1] = (int32_t)m;
-        if (sum > (uint32_t)P.max_voxels) atomicOr(&meta[0], SESSD_STATUS_VOXEL_OVERFLOW);
-    }
-    uint32_t base = b == 0 ? 0u : sum;
-    const int wave = threadIdx.x >> 6;
-    for (int w = 0; w < wave; ++w) base += __popcll(first_words[b * 4 + w]);
-    const uint64_t m = first_words[b * 4 + wave];
-    if (!((m >> (threadIdx.x & 63)) & 1ull)) return;
-    const uint32_t id = base + rank_in_wave(m);
-    const uint32_t tk = b * kBlock + threadIdx.x;
-    const uint32_t slot = cand[tk] & kSlotMask;
-    if (id >= (uint32_t)P.max_voxels) {  // the reference overflows its buffers; the site is dropped
-        t.vals[slot] = kEmpty;
-        return;
-    }
-    t.vals[slot] = id;  // from here on the table maps cell -> output row
-    const uint32_t key = t.keys[slot];
-    const uint32_t plane = (uint32_t)(P.os[1] * P.os[2]);
-    const int z = key / plane;
-    const int rem = key - z * plane;
-    const int y = rem / P.os[2];
-    reinterpret_cast<int4*>(out_coors)[id] = make_int4(0, z, y, rem - y * P.os[2]);  // sparseConv3dlayer.cu:438-441
-    // the new row's neighbour entries start empty (sp_scatter fills in the pairs): clearing them here, row by
-    // row, instead of the whole K x max_voxels table before the frame touches only the rows that exist
-    for (int k = 0; k < K; ++k) nbr[(size_t)k * P.max_voxels + id] = -1;
-    // ... and so do the mirrored entries of this row in the table of the SubM layer that follows
-    if (mi.nbr && (int)id < mi.stride)
-        for (int k = mi.first_offset; k < mi.K; ++k) mi.nbr[(size_t)k * mi.stride + id] = -1;
-}
-
-__global__ void __launch_bounds__(kBlock)
-sp_scatter(const int32_t* __restrict__ voxel_num, SpParams P, HashTable t, const uint32_t* __restrict__ cand,
-           int32_t* __restrict__ nbr) {
-    const uint32_t tk = blockIdx.x * kBlock + threadIdx.x;
-    const int v = tk / P.Kc;
-    const int n = clamp_count(voxel_num, P.max_voxels);
-    if (v >= n) return;
-    const uint32_t c = cand[tk];
-    if (c == kEmpty) return;
-    const uint32_t id = t.vals[c & kSlotMask];
-    if (id == kEmpty) return;
-    nbr[(size_t)(c >> kSlotBits) * P.max_voxels + id] = v;  // unique (offset, out row): plain store
-}
-
-}  // namespace
 
 struct SparseConv3dLayerPlugin::Layout {
-    uint32_t* keys;
-    uint32_t* vals;
+    void* cells;  // table of output cells
     int32_t* nbr;
     uint32_t* cand;
-    uint64_t* first_words;
-    uint32_t* block_counts;
+    uint64_t* words;
+    uint32_t* counts;
     void* export_scratch;
     int32_t* tiles;  // equal-work tile cuts of the rulebook (tile_cut.hip); first word 0 = none
     int32_t* meta;
     uint32_t cap;
+    bool dense;
     int Kc;
-    int n_blocks;
+    int n_chunks;
     size_t meta_offset;
     size_t total;
 };
@@ -263,14 +62,17 @@ SparseConv3dLayerPlugin::Layout SparseConv3dLayerPlugin::carve(void* workspace) 
     // the worst case -- every input row with Kc candidates of its own -- of which a real frame uses a few per
     // cent, so the table is sized just above it rather than at twice it: half the bytes to clear per frame.
     L.cap = next_pow2(distinct + distinct / kHashSlack);
+    // One word per cell where that is at most twice the hash's bytes: an insert is then one atomic without an answer, a
+    // lookup one load without a probe sequence, and neighbours in x share lines.
+    L.dense = volume * 4 <= (uint64_t)L.cap * 8 * 2 && volume < (1ull << kSlotBits);
+    if (L.dense) L.cap = (uint32_t)volume;
     const int64_t tickets = (int64_t)L.Kc * max_voxels_;
-    L.n_blocks = ceil_div(tickets, kBlock);
-    L.keys = c.take<uint32_t>((size_t)L.cap * 2);
-    L.vals = L.keys ? L.keys + L.cap : nullptr;
+    L.n_chunks = ceil_div(tickets, 256);
+    L.cells = c.take<uint32_t>(L.dense ? (size_t)L.cap : (size_t)L.cap * 2);
     L.nbr = c.take<int32_t>((size_t)kernel_volume_ * max_voxels_);
-    L.cand = c.take<uint32_t>((size_t)L.n_blocks * kBlock);
-    L.first_words = c.take<uint64_t>((size_t)L.n_blocks * 4);
-    L.block_counts = c.take<uint32_t>((size_t)L.n_blocks);
+    L.cand = c.take<uint32_t>((size_t)L.n_chunks * 256);
+    L.words = c.take<uint64_t>((size_t)L.n_chunks * 4);
+    L.counts = c.take<uint32_t>((size_t)L.n_chunks);
     L.export_scratch = c.take<uint8_t>(export_scratch_bytes(kernel_volume_, max_voxels_));
     L.tiles = reinterpret_cast<int32_t*>(c.take<uint8_t>(tile_cut_bytes(max_voxels_)));
     L.meta_offset = c.offset;
@@ -409,53 +211,107 @@ size_t SparseConv3dLayerPlugin::getWorkspaceSize(const sessd_tensor_desc*, int, 
 
 size_t SparseConv3dLayerPlugin::statusOffset() const { return carve(nullptr).meta_offset; }
 
-// The two halves of enqueue (see SubmConv3dLayerPlugin::enqueueBuild): output sites + rulebook from the
-// coordinates, then the GEMM over the features.
-void SparseConv3dLayerPlugin::collectFill(void* workspace, int32_t* out_coors, FillArgs& f) const {
+CellTable SparseConv3dLayerPlugin::cellTable(void* workspace) const {
     const Layout L = carve(workspace);
-    f.add(L.keys, (uint64_t)L.cap * 2, kEmpty);
-    f.add(L.tiles, 4, 0);
-    f.add(L.meta, 4, 0);
-    if (!(flags_ & SESSD_FLAG_SKIP_PAD_ROWS)) f.add(out_coors, (uint64_t)max_voxels_ * 4, 0);  // :668
+    CellTable t;
+    t.base = L.cells;
+    t.cap = L.cap;
+    t.dense = L.dense ? 1 : 0;
+    t.per_row16 = L.Kc * (16 + 16 / (int)kHashSlack);
+    t.gx = out_shape_x_;
+    t.gy = out_shape_y_;
+    t.gz = out_shape_z_;
+    return t;
 }
 
-int SparseConv3dLayerPlugin::enqueueBuild(const int32_t* coors, const int32_t* voxel_num, int32_t* out_coors,
-                                          int32_t* out_num, void* workspace, hipStream_t stream, bool prefilled,
-                                          const MirrorInit* mirror) {
-    if (!coors || !voxel_num || !out_coors || !out_num || !workspace)
-        return fail(SESSD_E_INVALID, "sparseconv3d.build: null pointer");
-    if (reinterpret_cast<uintptr_t>(out_coors) & 15)
-        return fail(SESSD_E_INVALID, "sparseconv3d.build: output coors must be 16-byte aligned");
+SpPart SparseConv3dLayerPlugin::part(const int32_t* coors, const int32_t* voxel_num, int32_t* out_coors, int32_t* out_num,
+                                     void* workspace, bool scattered) const {
     const Layout L = carve(workspace);
-    const HashTable t = make_hash(L.keys, L.vals, L.cap);
-    SpParams P;
+    SpPart P;
     P.k[0] = ksize0_; P.k[1] = ksize1_; P.k[2] = ksize2_;
     P.s[0] = stride0_; P.s[1] = stride1_; P.s[2] = stride2_;
     P.p[0] = padding0_; P.p[1] = padding1_; P.p[2] = padding2_;
     P.os[0] = out_shape_z_; P.os[1] = out_shape_y_; P.os[2] = out_shape_x_;
     P.Kc = L.Kc;
     P.max_voxels = max_voxels_;
-    P.dilation = dilation_;
-
-    if (!prefilled) {
-        FillArgs f;
-        collectFill(workspace, out_coors, f);
-        SESSD_TRY(launch_fill(f, stream));
-    }
-    const dim3 grid(L.n_blocks), block(kBlock);
-    hipLaunchKernelGGL(sp_insert, grid, block, 0, stream, coors, voxel_num, P, t, L.cand, L.meta);
-    hipLaunchKernelGGL(sp_flags, grid, block, 0, stream, voxel_num, P, t, L.cand, L.first_words, L.block_counts);
-    hipLaunchKernelGGL(sp_number, grid, block, 0, stream, voxel_num, P, t, L.cand, L.first_words, L.block_counts,
-                       L.n_blocks, out_coors, out_num, L.nbr, kernel_volume_, L.meta, mirror ? *mirror : MirrorInit());
-    hipLaunchKernelGGL(sp_scatter, grid, block, 0, stream, voxel_num, P, t, L.cand, L.nbr);
-    SESSD_HIP_TRY(hipGetLastError());
-    if (wantTileCuts()) SESSD_TRY(launch_tile_cuts(L.nbr, out_num, kernel_volume_, max_voxels_, tileRows(), tileRowWeight(), tilesWide(), L.tiles, stream));
-    return SESSD_OK;
+    P.K = kernel_volume_;
+    P.t = cellTable(workspace);
+    P.cand = L.cand;
+    P.words = L.words;
+    P.counts = L.counts;
+    P.n_chunks = L.n_chunks;
+    P.in_coors = coors;
+    P.in_num = voxel_num;
+    P.out_coors = out_coors;
+    P.out_num = out_num;
+    P.nbr = scattered ? L.nbr : nullptr;
+    P.meta = L.meta;
+    return P;
 }
 
-HashTable SparseConv3dLayerPlugin::cellTable(void* workspace) const {
+LookupPart SparseConv3dLayerPlugin::lookupPart(void* workspace, const int32_t* out_coors, const int32_t* out_num, const CellTable& cells,
+                                               const int32_t* cells_num, int cells_max) const {
     const Layout L = carve(workspace);
-    return make_hash(L.keys, L.vals, L.cap);
+    LookupPart p;
+    p.coors = out_coors;
+    p.num = out_num;
+    p.max_voxels = max_voxels_;
+    p.k[0] = ksize0_; p.k[1] = ksize1_; p.k[2] = ksize2_;
+    p.s[0] = stride0_; p.s[1] = stride1_; p.s[2] = stride2_;
+    p.p[0] = padding0_; p.p[1] = padding1_; p.p[2] = padding2_;
+    p.K = kernel_volume_;
+    p.own[0] = out_shape_z_; p.own[1] = out_shape_y_; p.own[2] = out_shape_x_;
+    p.t = cells;
+    p.t_num = cells_num;
+    p.t_max = cells_max;
+    p.nbr = L.nbr;
+    if (wantTileCuts()) {
+        p.w = tile_weight_array(L.tiles, max_voxels_);
+        p.wsum = tile_weight_sums(L.tiles, max_voxels_);
+        p.row_weight = tileRowWeight();
+    }
+    return p;
+}
+
+CutPart SparseConv3dLayerPlugin::cutPart(void* workspace, const int32_t* out_num) const {
+    return make_cut_part(out_num, kernel_volume_, max_voxels_, tileRows(), tileRowWeight(), tilesWide(), carve(workspace).tiles);
+}
+
+void SparseConv3dLayerPlugin::collectTableFill(void* workspace, FillArgs& f) const {
+    f.add(carve(workspace).cells, cellTable(workspace).words(), kEmpty);
+}
+void SparseConv3dLayerPlugin::collectHeaderFill(void* workspace, FillArgs& f) const {
+    const Layout L = carve(workspace);
+    f.add(L.tiles, 4, 0);
+    f.add(L.meta, 4, 0);
+}
+void SparseConv3dLayerPlugin::collectPadFill(int32_t* out_coors, FillArgs& f) const {
+    if (!(flags_ & SESSD_FLAG_SKIP_PAD_ROWS)) f.add(out_coors, (uint64_t)max_voxels_ * 4, 0);  // :668
+}
+
+// The two halves of enqueue (see SubmConv3dLayerPlugin::enqueueBuild): output sites + rulebook from the
+// coordinates, then the GEMM over the features.
+int SparseConv3dLayerPlugin::enqueueBuild(const int32_t* coors, const int32_t* voxel_num, int32_t* out_coors,
+                                          int32_t* out_num, void* workspace, hipStream_t stream) {
+    if (!coors || !voxel_num || !out_coors || !out_num || !workspace)
+        return fail(SESSD_E_INVALID, "sparseconv3d.build: null pointer");
+    if (reinterpret_cast<uintptr_t>(out_coors) & 15)
+        return fail(SESSD_E_INVALID, "sparseconv3d.build: output coors must be 16-byte aligned");
+    const Layout L = carve(workspace);
+    const SpPart P = part(coors, voxel_num, out_coors, out_num, workspace, true);
+    FillArgs f;
+    collectTableFill(workspace, f);
+    collectHeaderFill(workspace, f);
+    collectPadFill(out_coors, f);
+    SESSD_TRY(launch_fill(f, stream));
+    SESSD_TRY(launch_sp_insert(P, stream));
+    SESSD_TRY(launch_flags_lookups(&P, nullptr, 0, stream));
+    SESSD_TRY(launch_number(&P, nullptr, nullptr, 0, nullptr, nullptr, stream));
+    SESSD_TRY(launch_sp_scatter(P, stream));
+    if (!wantTileCuts()) return SESSD_OK;
+    SESSD_TRY(launch_tile_weights(L.nbr, out_num, kernel_volume_, max_voxels_, tileRowWeight(), L.tiles, stream));
+    const CutPart cut = cutPart(workspace, out_num);
+    return launch_number(nullptr, nullptr, &cut, 1, nullptr, nullptr, stream);
 }
 
 int SparseConv3dLayerPlugin::enqueueGemm(const void* in_feat, void* out_feat, const int32_t* out_num,

@@ -5,13 +5,12 @@
 // with atomicAdd and then launches the GEMM kernel 27 times.  Here:
 //
 //   subm_insert      one thread per active voxel: cell key -> hash table (value = voxel row)
-//   subm_neighbours  one thread per (offset k, output row o): look up cell o - padding + k and
-//                    write nbr[k][o] (coalesced, one 4-byte store per thread)
-//   gather-GEMM      conv_gemm.hip, one launch for all offsets
+//   lookups          nbr[k][o] = the row in cell o - padding + k, all offsets of a row at once (coord.hip)
+//   gather-GEMM      one launch for all offsets
 //
 // nbr[k][o] is the rulebook: the pair (i, o) is in the reference's list of offset k exactly when
 // nbr[k][o] == i.  sessd_submconv3d_export_rulebook compacts it into the reference's layout.
-#include "kernels.h"
+#include "coord.h"
 #include "plugins.h"
 
 namespace sessd {
@@ -24,18 +23,12 @@ struct Grid3 {
     int X, Y, Z;
 };
 
-__device__ __forceinline__ int clamp_count(const int32_t* p, int cap) {
-    int n = *p;
-    return n < 0 ? 0 : (n > cap ? cap : n);
-}
-
 // submConv3dlayer.cu:441-459 (prepareSubMGridKernel) with the dense grid replaced by a hash
 __global__ void __launch_bounds__(kBlock)
 subm_insert(const int32_t* __restrict__ coors, const int32_t* __restrict__ voxel_num, int max_voxels,
-            Grid3 g, HashTable t, int32_t* meta) {
+            Grid3 g, CellTable table, int32_t* meta) {
     const int v = blockIdx.x * kBlock + threadIdx.x;
-    const int n = clamp_count(voxel_num, max_voxels);
-    if (v == 0) meta[1] = n;
+    const int n = clamp_rows(voxel_num, max_voxels);
     if (v >= n) return;
     const int4 c = reinterpret_cast<const int4*>(coors)[v];  // (b,z,y,x)
     if (c.y < 0 || c.y >= g.Z || c.z < 0 || c.z >= g.Y || c.w < 0 || c.w >= g.X) {
@@ -43,71 +36,13 @@ subm_insert(const int32_t* __restrict__ coors, const int32_t* __restrict__ voxel
         return;
     }
     const uint32_t key = ((uint32_t)c.y * (uint32_t)g.Y + (uint32_t)c.z) * (uint32_t)g.X + (uint32_t)c.w;
-    const int32_t slot = hash_insert(t, key);
-    if (slot < 0) {
-        atomicOr(&meta[0], SESSD_STATUS_HASH_FULL);
-        return;
-    }
-    atomicMin(&t.vals[slot], (uint32_t)v);
-}
-
-// submConv3dlayer.cu:271-358 + 376-424: the pair (i, o) exists at offset (kz,ky,kx) iff the active
-// cell i sits at o - padding + k on every axis (stride 1, dilation 1).
-__global__ void __launch_bounds__(kBlock)
-subm_neighbours(const int32_t* __restrict__ coors, const int32_t* __restrict__ voxel_num, int max_voxels,
-                Grid3 g, int ksize, int padding, HashTable t, int32_t* __restrict__ nbr, int32_t* meta) {
-    const int v = blockIdx.x * kBlock + threadIdx.x;
-    const int k = blockIdx.y;
-    const int n = clamp_count(voxel_num, max_voxels);
-    if (meta && v == 0 && k == 0) meta[1] = n;  // (subm_insert's job when that pass runs)
-    if (v >= n) return;
-    const int4 c = reinterpret_cast<const int4*>(coors)[v];
-    const int kz = k / (ksize * ksize), ky = (k / ksize) % ksize, kx = k % ksize;
-    const int z = c.y - padding + kz, y = c.z - padding + ky, x = c.w - padding + kx;
-    int32_t res = -1;
-    const bool self_ok = c.y >= 0 && c.y < g.Z && c.z >= 0 && c.z < g.Y && c.w >= 0 && c.w < g.X;
-    if (self_ok && z >= 0 && z < g.Z && y >= 0 && y < g.Y && x >= 0 && x < g.X) {
-        const uint32_t key = ((uint32_t)z * (uint32_t)g.Y + (uint32_t)y) * (uint32_t)g.X + (uint32_t)x;
-        const int32_t slot = hash_find(t, key);
-        if (slot >= 0) res = (int32_t)t.vals[slot];
-    }
-    nbr[(size_t)k * max_voxels + v] = res;
-}
-
-// The same lookup for a 3x3x3 kernel over a table whose rows are unique (coordinates made by the voxelizer or a
-// strided layer of this library): the pair (i, o) at offset k is the pair (o, i) at offset 26 - k, so a thread
-// probes only the 13 offsets below the centre and writes both directions of a hit; the centre is the row itself.
-// Entries 14..26 of the active rows must hold -1 before the launch (MirrorInit: the kernel that created the rows
-// wrote them), because only hits are written there.  Half the probes of subm_neighbours.
-__global__ void __launch_bounds__(kBlock)
-subm_neighbours_mirrored(const int32_t* __restrict__ coors, const int32_t* __restrict__ voxel_num, int max_voxels,
-                         Grid3 g, HashTable t, int32_t* __restrict__ nbr, int32_t* meta) {
-    const int v = blockIdx.x * kBlock + threadIdx.x;
-    const int k = blockIdx.y;  // 0 .. 13
-    const int n = clamp_count(voxel_num, max_voxels);
-    if (meta && v == 0 && k == 0) meta[1] = n;
-    if (v >= n) return;
-    if (k == 13) {
-        nbr[(size_t)13 * max_voxels + v] = v;
-        return;
-    }
-    const int4 c = reinterpret_cast<const int4*>(coors)[v];
-    const int z = c.y - 1 + k / 9, y = c.z - 1 + (k / 3) % 3, x = c.w - 1 + k % 3;
-    int32_t res = -1;
-    if (z >= 0 && z < g.Z && y >= 0 && y < g.Y && x >= 0 && x < g.X) {
-        const uint32_t key = ((uint32_t)z * (uint32_t)g.Y + (uint32_t)y) * (uint32_t)g.X + (uint32_t)x;
-        const int32_t slot = hash_find(t, key);
-        if (slot >= 0) res = (int32_t)t.vals[slot];  // (-1 for a cell that was dropped at the capacity)
-    }
-    nbr[(size_t)k * max_voxels + v] = res;
-    if (res >= 0 && res < max_voxels) nbr[(size_t)(26 - k) * max_voxels + res] = v;
+    if (insert_min(open_table(table, n), key, (uint32_t)v) < 0) atomicOr(&meta[0], SESSD_STATUS_HASH_FULL);
 }
 
 }  // namespace
 
 struct SubmConv3dLayerPlugin::Layout {
-    uint32_t* keys;
-    uint32_t* vals;
+    uint64_t* entries;  // cell table: cell -> row
     int32_t* nbr;
     void* export_scratch;
     int32_t* tiles;  // equal-work tile cuts of the rulebook (tile_cut.hip); first word 0 = none
@@ -121,8 +56,7 @@ SubmConv3dLayerPlugin::Layout SubmConv3dLayerPlugin::carve(void* workspace) cons
     Layout L;
     WorkspaceCarver c(workspace);
     L.cap = next_pow2((uint64_t)(max_voxels_ < 32 ? 32 : max_voxels_) * 2);
-    L.keys = c.take<uint32_t>((size_t)L.cap * 2);  // keys then vals: one fill region
-    L.vals = L.keys ? L.keys + L.cap : nullptr;
+    L.entries = c.take<uint64_t>(L.cap);
     L.nbr = c.take<int32_t>((size_t)kernel_volume_ * max_voxels_);
     L.export_scratch = c.take<uint8_t>(export_scratch_bytes(kernel_volume_, max_voxels_));
     L.tiles = reinterpret_cast<int32_t*>(c.take<uint8_t>(tile_cut_bytes(max_voxels_)));
@@ -251,52 +185,76 @@ size_t SubmConv3dLayerPlugin::getWorkspaceSize(const sessd_tensor_desc*, int, co
 
 size_t SubmConv3dLayerPlugin::statusOffset() const { return carve(nullptr).meta_offset; }
 
-// The two halves of enqueue.  The rulebook depends only on the coordinates, the GEMM only on the
-// rulebook and the features: a pipeline may run the halves of different layers on different streams.
-// what enqueueBuild clears before it launches anything: a caller that batches the clears of many layers
-// into one launch collects them with this and passes prefilled = true
-void SubmConv3dLayerPlugin::collectFill(void* workspace, FillArgs& f, bool own_table) const {
+CellTable SubmConv3dLayerPlugin::ownTable(void* workspace) const {
     const Layout L = carve(workspace);
-    if (own_table) f.add(L.keys, (uint64_t)L.cap * 2, kEmpty);  // (not when the build probes another table)
+    CellTable t;
+    t.base = L.entries;
+    t.cap = L.cap;
+    t.per_row16 = 32;  // at most half full
+    t.gx = out_shape_x_;
+    t.gy = out_shape_y_;
+    t.gz = out_shape_z_;
+    return t;
+}
+
+LookupPart SubmConv3dLayerPlugin::lookupPart(void* workspace, const int32_t* coors, const int32_t* voxel_num, const CellTable& cells,
+                                             const int32_t* cells_num, int cells_max) const {
+    const Layout L = carve(workspace);
+    LookupPart p;
+    p.coors = coors;
+    p.num = voxel_num;
+    p.max_voxels = max_voxels_;
+    for (int a = 0; a < 3; ++a) {
+        p.k[a] = ksize_;
+        p.s[a] = 1;
+        p.p[a] = padding_;
+    }
+    p.K = kernel_volume_;
+    p.own[0] = out_shape_z_;
+    p.own[1] = out_shape_y_;
+    p.own[2] = out_shape_x_;
+    p.t = cells;
+    p.t_num = cells_num;
+    p.t_max = cells_max;
+    p.nbr = L.nbr;
+    p.meta = L.meta;
+    if (wantTileCuts()) {
+        p.w = tile_weight_array(L.tiles, max_voxels_);
+        p.wsum = tile_weight_sums(L.tiles, max_voxels_);
+        p.row_weight = tileRowWeight();
+    }
+    return p;
+}
+
+CutPart SubmConv3dLayerPlugin::cutPart(void* workspace, const int32_t* voxel_num) const {
+    return make_cut_part(voxel_num, kernel_volume_, max_voxels_, tileRows(), tileRowWeight(), tilesWide(), carve(workspace).tiles);
+}
+
+void SubmConv3dLayerPlugin::collectHeaderFill(void* workspace, FillArgs& f) const {
+    const Layout L = carve(workspace);
     f.add(L.tiles, 4, 0);
     f.add(L.meta, 4, 0);
 }
 
-int SubmConv3dLayerPlugin::enqueueBuild(const int32_t* coors, const int32_t* voxel_num, void* workspace,
-                                        hipStream_t stream, bool prefilled, const HashTable* cells, bool mirrored) {
+// The two halves of enqueue.  The rulebook depends only on the coordinates, the GEMM only on the
+// rulebook and the features: a pipeline may run the halves of different layers on different streams.
+int SubmConv3dLayerPlugin::enqueueBuild(const int32_t* coors, const int32_t* voxel_num, void* workspace, hipStream_t stream) {
     if (!coors || !voxel_num || !workspace) return fail(SESSD_E_INVALID, "submconv3d.build: null pointer");
     const Layout L = carve(workspace);
-    const HashTable t = make_hash(L.keys, L.vals, L.cap);
     const Grid3 g{out_shape_x_, out_shape_y_, out_shape_z_};
-    if (!prefilled) {
-        FillArgs f;
-        collectFill(workspace, f);
-        SESSD_TRY(launch_fill(f, stream));
-    }
-    const int row_blocks = ceil_div(max_voxels_, kBlock);
-    if (!cells)
-        hipLaunchKernelGGL(subm_insert, dim3(row_blocks), dim3(kBlock), 0, stream, coors, voxel_num, max_voxels_,
-                           g, t, L.meta);
-    if (mirrored && cells && kernel_volume_ == 27)
-        hipLaunchKernelGGL(subm_neighbours_mirrored, dim3(row_blocks, 14), dim3(kBlock), 0, stream, coors, voxel_num,
-                           max_voxels_, g, *cells, L.nbr, L.meta);
-    else
-        hipLaunchKernelGGL(subm_neighbours, dim3(row_blocks, kernel_volume_), dim3(kBlock), 0, stream, coors,
-                           voxel_num, max_voxels_, g, ksize_, padding_, cells ? *cells : t, L.nbr,
-                           cells ? L.meta : nullptr);
+    const CellTable t = ownTable(workspace);
+    FillArgs f;
+    f.add(L.entries, t.words(), kEmpty);
+    collectHeaderFill(workspace, f);
+    SESSD_TRY(launch_fill(f, stream));
+    hipLaunchKernelGGL(subm_insert, dim3(ceil_div(max_voxels_, kBlock)), dim3(kBlock), 0, stream, coors, voxel_num, max_voxels_, g, t,
+                       L.meta);
     SESSD_HIP_TRY(hipGetLastError());
-    if (wantTileCuts()) SESSD_TRY(launch_tile_cuts(L.nbr, voxel_num, kernel_volume_, max_voxels_, tileRows(), tileRowWeight(), tilesWide(), L.tiles, stream));
-    return SESSD_OK;
-}
-
-MirrorInit SubmConv3dLayerPlugin::mirrorInit(void* workspace) const {
-    MirrorInit m;
-    if (kernel_volume_ != 27 || !workspace) return m;
-    m.nbr = carve(workspace).nbr;
-    m.stride = max_voxels_;
-    m.first_offset = 14;
-    m.K = 27;
-    return m;
+    const LookupPart look = lookupPart(workspace, coors, voxel_num, t, voxel_num, max_voxels_);
+    SESSD_TRY(launch_flags_lookups(nullptr, &look, 1, stream));
+    if (!wantTileCuts()) return SESSD_OK;
+    const CutPart cut = cutPart(workspace, voxel_num);
+    return launch_number(nullptr, nullptr, &cut, 1, nullptr, nullptr, stream);
 }
 
 int SubmConv3dLayerPlugin::enqueueGemm(const void* in_feat, void* out_feat, const int32_t* voxel_num,

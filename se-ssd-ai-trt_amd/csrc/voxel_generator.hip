@@ -4,20 +4,21 @@
 // [Z*Y*X][2] slot table (721 MB, memset every frame) and hands out voxel ids and point slots with
 // atomicAdd, so which points are kept and how voxels are numbered depends on scheduling.  Here:
 //
-//   vg_insert    one thread per point: cell key -> open-addressing hash (a few MB, L2 resident);
-//                each entry keeps the S smallest point indices of its cell, maintained with a
-//                chain of atomicMin "comparators" whose final state is independent of the order
-//                in which threads arrive
-//   vg_flags     one thread per point: "am I the lowest-index point of my cell" -> wave64 ballot
-//                words + per-block counts
+//   vg_insert    one thread per point: cell key -> open-addressing hash (a few MB, L2 resident), or a table with a word
+//                per cell where the pipeline keeps one; each cell keeps its smallest point index
+//   vg_flags     one thread per point: "am I the first point of my cell" -> wave64 ballot words + per-block counts;
+//                the later points of a cell go through a chain of atomicMin "comparators" behind its first one, whose
+//                final state is independent of the order in which threads arrive
 //   vg_finalize  exclusive prefix over the ballot words = voxel id in first-appearance order;
 //                that thread writes the coordinate and the mean of the (<= S) kept points
+// (kernels: coord.hip)
 //
 // The result equals a sequential walk over the points: ids in first-appearance order, the first S
 // points of a cell kept, cells first seen after max_voxels dropped.  All traffic is O(points):
 // 16 B/point read + 32 B/voxel written, plus the hash clear.
 #include <mutex>
 
+#include "coord.h"
 #include "plugins.h"
 
 namespace sessd {
@@ -25,145 +26,7 @@ namespace sessd {
 namespace {
 
 constexpr int kBlock = 256;
-
-struct VgParams {
-    float min_x, max_x, min_y, max_y, min_z, max_z;
-    float vx, vy, vz;
-    int gx, gy, gz;
-    int max_voxels;
-    int max_pts;  // S
-};
-
-__device__ __forceinline__ int clamp_count(const int32_t* p, int cap) {
-    int n = *p;
-    return n < 0 ? 0 : (n > cap ? cap : n);
-}
-
-// sum of v over the block (blockDim.x == kBlock), returned to every thread
-__device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t* lds4) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    const int wave = threadIdx.x >> 6;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) lds4[wave] = v;
-    __syncthreads();
-    return lds4[0] + lds4[1] + lds4[2] + lds4[3];
-}
-
-__global__ void __launch_bounds__(kBlock)
-vg_insert(const float* __restrict__ points, const int32_t* __restrict__ points_size, int max_points,
-          int pf, VgParams p, HashTable t, uint32_t* __restrict__ slots, int32_t* __restrict__ pt_slot,
-          int32_t* status) {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    const int n = clamp_count(points_size, max_points);
-    if (i >= n) return;
-    const float* pt = points + (size_t)i * pf;
-    const float x = pt[0], y = pt[1], z = pt[2];
-    int32_t slot = -1;
-    // voxelGenerator.cu:363-367: half-open range test
-    if (x >= p.min_x && x < p.max_x && y >= p.min_y && y < p.max_y && z >= p.min_z && z < p.max_z) {
-        // voxelGenerator.cu:369-371: IEEE FP32 division (never a reciprocal multiply)
-        const int ix = (int)floorf((x - p.min_x) / p.vx);
-        const int iy = (int)floorf((y - p.min_y) / p.vy);
-        const int iz = (int)floorf((z - p.min_z) / p.vz);
-        // voxelGenerator.cu:375: a value just below max can still land on the grid size
-        if (ix >= 0 && ix < p.gx && iy >= 0 && iy < p.gy && iz >= 0 && iz < p.gz) {
-            const uint32_t key = (uint32_t)iz * (uint32_t)(p.gy * p.gx) + (uint32_t)iy * (uint32_t)p.gx + (uint32_t)ix;
-            slot = hash_insert(t, key);
-            if (slot < 0) {
-                atomicOr(status, SESSD_STATUS_HASH_FULL);
-            } else {
-                // keep the S smallest point indices of the cell, ascending: slot q ends up with
-                // the minimum of everything offered to it and passes the rest on
-                uint32_t* s = slots + (size_t)slot * p.max_pts;
-                uint32_t cur = (uint32_t)i;
-                for (int q = 0; q < p.max_pts; ++q) {
-                    const uint32_t old = atomicMin(&s[q], cur);
-                    if (old == kEmpty) break;
-                    cur = old > cur ? old : cur;
-                }
-            }
-        }
-    }
-    pt_slot[i] = slot;
-}
-
-__global__ void __launch_bounds__(kBlock)
-vg_flags(const int32_t* __restrict__ points_size, int max_points, int max_pts,
-         const uint32_t* __restrict__ slots, const int32_t* __restrict__ pt_slot,
-         uint64_t* __restrict__ first_words, uint32_t* __restrict__ block_counts) {
-    __shared__ uint32_t lds4[4];
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    const int n = clamp_count(points_size, max_points);
-    bool first = false;
-    if (i < n) {
-        const int32_t slot = pt_slot[i];
-        first = slot >= 0 && slots[(size_t)slot * max_pts] == (uint32_t)i;
-    }
-    const uint64_t m = __ballot(first);
-    if ((threadIdx.x & 63) == 0) {
-        first_words[i >> 6] = m;
-        lds4[threadIdx.x >> 6] = __popcll(m);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) block_counts[blockIdx.x] = lds4[0] + lds4[1] + lds4[2] + lds4[3];
-}
-
-__global__ void __launch_bounds__(kBlock)
-vg_finalize(const float* __restrict__ points, int pf, VgParams p, HashTable t,
-            const uint32_t* __restrict__ slots, const int32_t* __restrict__ pt_slot,
-            const uint64_t* __restrict__ first_words, const uint32_t* __restrict__ block_counts,
-            int n_blocks, float* __restrict__ voxels, int32_t* __restrict__ coors,
-            int32_t* __restrict__ voxel_num, int32_t* status, MirrorInit mi) {
-    __shared__ uint32_t lds4[4];
-    const int b = blockIdx.x;
-    // block 0 sums every block's count (the total); the others sum the blocks before them
-    const int upto = b == 0 ? n_blocks : b;
-    uint32_t part = 0;
-    for (int j = threadIdx.x; j < upto; j += kBlock) part += block_counts[j];
-    const uint32_t sum = block_sum(part, lds4);
-    if (b == 0 && threadIdx.x == 0) {
-        *voxel_num = (int32_t)(sum > (uint32_t)p.max_voxels ? (uint32_t)p.max_voxels : sum);
-        if (sum > (uint32_t)p.max_voxels) atomicOr(status, SESSD_STATUS_VOXEL_OVERFLOW);
-    }
-    uint32_t base = b == 0 ? 0u : sum;
-    const int i = b * kBlock + threadIdx.x;
-    const int wave = threadIdx.x >> 6;
-    for (int w = 0; w < wave; ++w) base += __popcll(first_words[b * 4 + w]);
-    const uint64_t m = first_words[b * 4 + wave];
-    if (!((m >> (threadIdx.x & 63)) & 1ull)) return;
-    const uint32_t vid = base + rank_in_wave(m);
-    if (vid >= (uint32_t)p.max_voxels) return;  // cells first seen beyond the cap are dropped
-
-    const int32_t slot = pt_slot[i];
-    const uint32_t key = t.keys[slot];
-    const uint32_t plane = (uint32_t)(p.gy * p.gx);
-    const int iz = key / plane;
-    const int rem = key - iz * plane;
-    const int iy = rem / p.gx;
-    const int ix = rem - iy * p.gx;
-    reinterpret_cast<int4*>(coors)[vid] = make_int4(0, iz, iy, ix);  // voxelGenerator.cu:404-405
-    t.vals[slot] = vid;  // the table now maps cell -> voxel row (VoxelGeneratorPlugin::cellTable)
-    if (mi.nbr && (int)vid < mi.stride)  // the next SubM layer's mirrored neighbour entries of this row start empty
-        for (int k = mi.first_offset; k < mi.K; ++k) mi.nbr[(size_t)k * mi.stride + vid] = -1;
-
-    // voxelGenerator.cu:274-296: all S slots are summed left to right, unfilled slots count as 0
-    const uint32_t* s = slots + (size_t)slot * p.max_pts;
-    float sx = 0.f, sy = 0.f, sz = 0.f, sw = 0.f;
-    int cnt = 0;
-    for (int q = 0; q < p.max_pts; ++q) {
-        const uint32_t idx = s[q];
-        float ax = 0.f, ay = 0.f, az = 0.f, aw = 0.f;
-        if (idx != kEmpty) {
-            const float* pt = points + (size_t)idx * pf;
-            ax = pt[0]; ay = pt[1]; az = pt[2]; aw = pt[3];
-            ++cnt;
-        }
-        if (q == 0) { sx = ax; sy = ay; sz = az; sw = aw; }
-        else { sx = sx + ax; sy = sy + ay; sz = sz + az; sw = sw + aw; }
-    }
-    const float c = (float)cnt;
-    reinterpret_cast<float4*>(voxels)[vid] = make_float4(sx / c, sy / c, sz / c, sw / c);
-}
+constexpr int kSlotsPerPoint = 2;
 
 // np.round as in spconv's voxel generator (voxelGenerator.cu:61-68): half to even
 int np_round(float x) {
@@ -175,14 +38,14 @@ int np_round(float x) {
 }  // namespace
 
 struct VoxelGeneratorPlugin::Layout {
-    uint32_t* keys;
-    uint32_t* vals;  // voxel row of the cell (written by vg_finalize; kEmpty for dropped cells)
+    uint64_t* entries;  // cell table; its value is the voxel row after vg_finalize (kEmpty for dropped cells)
     uint32_t* slots;
     int32_t* pt_slot;
-    uint64_t* first_words;
-    uint32_t* block_counts;
+    uint64_t* words;
+    uint32_t* counts;
     int32_t* status;
     uint32_t cap;
+    uint64_t slot_words;
     int n_blocks;
     size_t status_offset;
     size_t total;
@@ -191,26 +54,76 @@ struct VoxelGeneratorPlugin::Layout {
 VoxelGeneratorPlugin::Layout VoxelGeneratorPlugin::carve(void* workspace, int max_points) const {
     Layout L;
     WorkspaceCarver c(workspace);
-    L.cap = next_pow2((uint64_t)(max_points < 32 ? 32 : max_points) * 2);
+    L.cap = next_pow2((uint64_t)(max_points < 32 ? 32 : max_points) * kSlotsPerPoint);
     L.n_blocks = ceil_div(max_points, kBlock);
-    // keys, vals and slots are adjacent so that one fill region clears all three
-    const size_t cap_words = align_up((size_t)L.cap * 4) / 4;
-    const size_t table_words = 2 * cap_words + (size_t)L.cap * pointNum_;
-    L.keys = c.take<uint32_t>(table_words);
-    L.vals = L.keys ? L.keys + cap_words : nullptr;
-    L.slots = L.keys ? L.keys + 2 * cap_words : nullptr;
+    // entries and slots are adjacent so that one fill region clears both
+    L.slot_words = (uint64_t)max_points * (pointNum_ - 1);
+    L.entries = reinterpret_cast<uint64_t*>(c.take<uint32_t>((uint64_t)L.cap * 2 + L.slot_words));
+    L.slots = L.entries ? reinterpret_cast<uint32_t*>(L.entries + L.cap) : nullptr;
     L.pt_slot = c.take<int32_t>((size_t)L.n_blocks * kBlock);
-    L.first_words = c.take<uint64_t>((size_t)L.n_blocks * 4);
-    L.block_counts = c.take<uint32_t>((size_t)L.n_blocks);
+    L.words = c.take<uint64_t>((size_t)L.n_blocks * 4);
+    L.counts = c.take<uint32_t>((size_t)L.n_blocks);
     L.status_offset = c.offset;
     L.status = c.take<int32_t>(4);
     L.total = c.total();
     return L;
 }
 
-HashTable VoxelGeneratorPlugin::cellTable(void* workspace, int max_points) const {
+CellTable VoxelGeneratorPlugin::cellTable(void* workspace, int max_points) const {
     const Layout L = carve(workspace, max_points);
-    return make_hash(L.keys, L.vals, L.cap);
+    CellTable t;
+    t.base = L.entries;
+    t.cap = L.cap;
+    t.per_row16 = 16 * kSlotsPerPoint;  // at most half full
+    t.gx = grid_x_size_;
+    t.gy = grid_y_size_;
+    t.gz = grid_z_size_;
+    return t;
+}
+
+VgPart VoxelGeneratorPlugin::part(const float* points, const int32_t* points_size, int max_points, int pf, float* voxels,
+                                  int32_t* coors, int32_t* voxel_num, void* workspace) const {
+    const Layout L = carve(workspace, max_points);
+    VgPart v;
+    v.points = points;
+    v.points_size = points_size;
+    v.max_points = max_points;
+    v.pf = pf;
+    v.min_x = min_x_range_;
+    v.max_x = max_x_range_;
+    v.min_y = min_y_range_;
+    v.max_y = max_y_range_;
+    v.min_z = min_z_range_;
+    v.max_z = max_z_range_;
+    v.vx = voxel_x_size_;
+    v.vy = voxel_y_size_;
+    v.vz = voxel_z_size_;
+    v.gx = grid_x_size_;
+    v.gy = grid_y_size_;
+    v.gz = grid_z_size_;
+    v.max_voxels = voxelNum_;
+    v.max_pts = pointNum_;
+    v.t = cellTable(workspace, max_points);
+    v.slots = L.slots;
+    v.pt_slot = L.pt_slot;
+    v.words = L.words;
+    v.counts = L.counts;
+    v.n_blocks = L.n_blocks;
+    v.voxels = voxels;
+    v.coors = coors;
+    v.voxel_num = voxel_num;
+    v.status = L.status;
+    return v;
+}
+
+void VoxelGeneratorPlugin::collectTableFill(void* workspace, int max_points, bool table_only, FillArgs& f) const {
+    const Layout L = carve(workspace, max_points);
+    f.add(L.entries, (uint64_t)L.cap * 2 + (table_only ? 0 : L.slot_words), kEmpty);
+}
+void VoxelGeneratorPlugin::collectPadFill(float* voxels, int32_t* coors, FillArgs& f) const {
+    if (flags_ & SESSD_FLAG_SKIP_PAD_ROWS) return;
+    f.add(voxels, (uint64_t)voxelNum_ * 4, 0);  // voxelGenerator.cu:524-525
+    f.add(coors, (uint64_t)voxelNum_ * 4, 0);
 }
 
 void VoxelGeneratorPlugin::deriveGrid() {
@@ -327,7 +240,7 @@ size_t VoxelGeneratorPlugin::statusOffset(int max_points) const {
 
 int VoxelGeneratorPlugin::enqueue(const sessd_tensor_desc* inputDesc, const sessd_tensor_desc*,
                                   const void* const* inputs, void* const* outputs, void* workspace,
-                                  hipStream_t stream, const MirrorInit* mirror, const FillArgs* also_clear) {
+                                  hipStream_t stream) {
     if (!inputDesc || !inputs || !outputs || !workspace)
         return fail(SESSD_E_INVALID, "voxelgen.enqueue: null argument");
     if (inputDesc[0].nbDims != 3 || inputDesc[0].d[0] != 1)
@@ -349,34 +262,16 @@ int VoxelGeneratorPlugin::enqueue(const sessd_tensor_desc* inputDesc, const sess
 
     lastMaxPoints_ = max_points;
     const Layout L = carve(workspace, max_points);
-    HashTable t = make_hash(L.keys, L.vals, L.cap);
-    VgParams p{min_x_range_, max_x_range_, min_y_range_, max_y_range_, min_z_range_, max_z_range_,
-               voxel_x_size_, voxel_y_size_, voxel_z_size_, grid_x_size_, grid_y_size_, grid_z_size_,
-               voxelNum_, pointNum_};
-
+    const VgPart v = part(points, points_size, max_points, pf, voxels, coors, voxel_num, workspace);
     FillArgs f;
-    f.add(L.keys, (uint64_t)(L.slots - L.keys) + (uint64_t)L.cap * pointNum_, kEmpty);
+    collectTableFill(workspace, max_points, false, f);
     f.add(L.status, 4, 0);
-    if (!(flags_ & SESSD_FLAG_SKIP_PAD_ROWS)) {  // voxelGenerator.cu:524-525
-        f.add(voxels, (uint64_t)voxelNum_ * 4, 0);
-        f.add(coors, (uint64_t)voxelNum_ * 4, 0);
-    }
-    if (also_clear) {  // a pipeline's small clears ride along in the launch that heads the frame anyway
-        if (f.n + also_clear->n > FillArgs::kMaxRegions) return fail(SESSD_E_INVALID, "voxelgen.enqueue: too many regions to clear");
-        for (int i = 0; i < also_clear->n; ++i) f.r[f.n++] = also_clear->r[i];
-    }
     SESSD_TRY(launch_fill(f, stream));
-
-    const dim3 grid(L.n_blocks), block(kBlock);
-    hipLaunchKernelGGL(vg_insert, grid, block, 0, stream, points, points_size, max_points, pf, p, t,
-                       L.slots, L.pt_slot, L.status);
-    hipLaunchKernelGGL(vg_flags, grid, block, 0, stream, points_size, max_points, pointNum_, L.slots,
-                       L.pt_slot, L.first_words, L.block_counts);
-    hipLaunchKernelGGL(vg_finalize, grid, block, 0, stream, points, pf, p, t, L.slots, L.pt_slot,
-                       L.first_words, L.block_counts, L.n_blocks, voxels, coors, voxel_num, L.status,
-                       mirror ? *mirror : MirrorInit());
-    SESSD_HIP_TRY(hipGetLastError());
-    return SESSD_OK;
+    FillArgs pads;
+    collectPadFill(voxels, coors, pads);
+    SESSD_TRY(launch_vg_insert(v, nullptr, 0, pads, stream));
+    SESSD_TRY(launch_vg_flags(v, FillArgs(), stream));
+    return launch_vg_finalize(v, nullptr, stream);
 }
 
 int read_status_word(const void* workspace, size_t offset, hipStream_t stream, int32_t* status) {
