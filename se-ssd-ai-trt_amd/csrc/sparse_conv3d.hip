@@ -62,9 +62,7 @@ SparseConv3dLayerPlugin::Layout SparseConv3dLayerPlugin::carve(void* workspace) 
     // the worst case -- every input row with Kc candidates of its own -- of which a real frame uses a few per
     // cent, so the table is sized just above it rather than at twice it: half the bytes to clear per frame.
     L.cap = next_pow2(distinct + distinct / kHashSlack);
-    // One word per cell where that is at most twice the hash's bytes: an insert is then one atomic without an answer, a
-    // lookup one load without a probe sequence, and neighbours in x share lines.
-    L.dense = volume * 4 <= (uint64_t)L.cap * 8 * 2 && volume < (1ull << kSlotBits);
+    L.dense = dense_pays(volume, (uint64_t)L.cap * 8) && volume < (1ull << kSlotBits);
     if (L.dense) L.cap = (uint32_t)volume;
     const int64_t tickets = (int64_t)L.Kc * max_voxels_;
     L.n_chunks = ceil_div(tickets, 256);

@@ -42,12 +42,13 @@ subm_insert(const int32_t* __restrict__ coors, const int32_t* __restrict__ voxel
 }  // namespace
 
 struct SubmConv3dLayerPlugin::Layout {
-    uint64_t* entries;  // cell table: cell -> row
+    void* cells;  // cell table: cell -> row
     int32_t* nbr;
     void* export_scratch;
     int32_t* tiles;  // equal-work tile cuts of the rulebook (tile_cut.hip); first word 0 = none
     int32_t* meta;  // [0] status word, [1] active rows of the last enqueue
     uint32_t cap;
+    bool dense;
     size_t meta_offset;
     size_t total;
 };
@@ -56,7 +57,10 @@ SubmConv3dLayerPlugin::Layout SubmConv3dLayerPlugin::carve(void* workspace) cons
     Layout L;
     WorkspaceCarver c(workspace);
     L.cap = next_pow2((uint64_t)(max_voxels_ < 32 ? 32 : max_voxels_) * 2);
-    L.entries = c.take<uint64_t>(L.cap);
+    const uint64_t volume = (uint64_t)out_shape_x_ * out_shape_y_ * out_shape_z_;
+    L.dense = dense_pays(volume, (uint64_t)L.cap * 8);
+    if (L.dense) L.cap = (uint32_t)volume;
+    L.cells = c.take<uint32_t>(L.dense ? (size_t)L.cap : (size_t)L.cap * 2);
     L.nbr = c.take<int32_t>((size_t)kernel_volume_ * max_voxels_);
     L.export_scratch = c.take<uint8_t>(export_scratch_bytes(kernel_volume_, max_voxels_));
     L.tiles = reinterpret_cast<int32_t*>(c.take<uint8_t>(tile_cut_bytes(max_voxels_)));
@@ -188,8 +192,9 @@ size_t SubmConv3dLayerPlugin::statusOffset() const { return carve(nullptr).meta_
 CellTable SubmConv3dLayerPlugin::ownTable(void* workspace) const {
     const Layout L = carve(workspace);
     CellTable t;
-    t.base = L.entries;
+    t.base = L.cells;
     t.cap = L.cap;
+    t.dense = L.dense ? 1 : 0;
     t.per_row16 = 32;  // at most half full
     t.gx = out_shape_x_;
     t.gy = out_shape_y_;
@@ -244,7 +249,7 @@ int SubmConv3dLayerPlugin::enqueueBuild(const int32_t* coors, const int32_t* vox
     const Grid3 g{out_shape_x_, out_shape_y_, out_shape_z_};
     const CellTable t = ownTable(workspace);
     FillArgs f;
-    f.add(L.entries, t.words(), kEmpty);
+    f.add(L.cells, t.words(), kEmpty);
     collectHeaderFill(workspace, f);
     SESSD_TRY(launch_fill(f, stream));
     hipLaunchKernelGGL(subm_insert, dim3(ceil_div(max_voxels_, kBlock)), dim3(kBlock), 0, stream, coors, voxel_num, max_voxels_, g, t,

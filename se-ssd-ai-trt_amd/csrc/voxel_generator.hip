@@ -26,7 +26,7 @@ namespace sessd {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kSlotsPerPoint = 2;
+constexpr int kSlotsPerPoint = 4;
 
 // np.round as in spconv's voxel generator (voxelGenerator.cu:61-68): half to even
 int np_round(float x) {
@@ -74,7 +74,7 @@ CellTable VoxelGeneratorPlugin::cellTable(void* workspace, int max_points) const
     CellTable t;
     t.base = L.entries;
     t.cap = L.cap;
-    t.per_row16 = 16 * kSlotsPerPoint;  // at most half full
+    t.per_row16 = 16 * kSlotsPerPoint;  // at most a quarter full: an insert mostly finds its first slot empty
     t.gx = grid_x_size_;
     t.gy = grid_y_size_;
     t.gz = grid_z_size_;

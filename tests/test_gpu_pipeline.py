@@ -406,3 +406,56 @@ def test_fp16_stack_ending_in_a_3x3x3_layer_scatters_from_the_tall_tile_kernel()
     assert np.array_equal(fused.read_layer(len(layers) - 1)[1], ref["coors"])
     assert_end_to_end_close(to_np(d_fused).astype(np.float32), want, True, "dense from the tall-tile kernel")
     assert torch.equal(d_fused, d_plain)
+
+
+@pytest.mark.parametrize("overlap", [True, False])
+@pytest.mark.parametrize("full_resolution", [False, True])
+def test_cell_tables_kept_between_frames_carry_nothing_over(full_resolution, overlap):
+    """The pipeline keeps its dense cell tables from frame to frame and empties them row by row.  Frames of different
+    sizes through one pipeline, an empty one and a plugin-by-plugin run (enqueue_timed, which overwrites the rows the
+    tables are emptied by) between them, each against the oracle.  full_resolution: a strided layer of stride 1 whose
+    output grid is too large for a dense table, so that its hash is cleared instead."""
+    layers = B.reference_layers()
+    if full_resolution:
+        at = next(i for i, l in enumerate(layers) if l.name == "sparse6")
+        wide = B.Layer("sparse5", D.SESSD_LAYER_SPARSE, 16, 16, layers[0].out_shape, (3, 3, 3), (1, 1, 1), (1, 1, 1))
+        layers = layers[:at] + [wide] + layers[at:]
+    W = B.random_weights(layers, seed=11, w_std=0.05)
+    mp, mv = 1024, 40000
+    pipe = api.Pipeline(layers, W, mp, mv, share_rulebooks=True, skip_pad_rows=overlap, use_graph=True, overlap_streams=overlap)
+    p, n = points_input(np.zeros((0, 4), np.float32), mp)
+    dense, stream = pipe.new_dense(), torch.cuda.Stream()
+    for step, npts in enumerate((400, 1000, 0, 250, 250)):
+        pts = F.lidar_frame(npts, 60 + step) if npts else np.zeros((0, 4), np.float32)
+        hp, hn = points_input(pts, mp)
+        with torch.cuda.stream(stream):
+            p.copy_(hp)
+            n.copy_(hn)
+            if step == 3:
+                pipe.enqueue_timed(p, n, dense, stream)
+            else:
+                pipe.enqueue(p, n, dense, stream)
+        stream.synchronize()
+        ref = O.frame(pts, B.voxelgen_desc(max_voxels=mv), layers, W, B.dense_desc())
+        assert pipe.status() == ref["status"] == 0
+        assert [pipe.layer_count(l) for l in range(-1, len(layers))] == list(ref["counts"]), npts
+        assert np.array_equal(pipe.read_layer(len(layers) - 1)[1], ref["coors"]), npts
+        assert_end_to_end_close(to_np(dense), ref["dense"], False, "dense, step %d" % step)
+
+
+@pytest.mark.parametrize("max_pts", [1, 2, 5, 6, 9])
+def test_voxelizer_keeps_the_first_points_of_crowded_cells(max_pts):
+    """More points per cell than are averaged, at point counts around a block: the later points of a cell go through a
+    chain of places behind its first one, of which four are read ahead."""
+    rng = np.random.default_rng(max_pts)
+    for npts in (1, 255, 257, 3000):
+        pts = np.zeros((npts, 4), np.float32)
+        pts[:, :3] = np.array([1.0, -2.0, -1.0]) + rng.uniform(0, 0.25, (npts, 3))
+        pts[:, 3] = rng.uniform(0, 1, npts)
+        vg = api.VoxelGenerator(max_voxels=4096, max_num_points_per_voxel=max_pts)
+        voxels, coors, num = vg(*points_input(pts, npts + 5))
+        torch.cuda.synchronize()
+        ref = O.voxelize(pts, B.POINT_CLOUD_RANGE, B.VOXEL_SIZE, max_pts, 4096)
+        assert int(num[0]) == ref[2]
+        assert np.array_equal(to_np(coors)[:ref[2]], ref[1][:ref[2]])
+        assert np.array_equal(to_np(voxels)[:ref[2]].view(np.uint32), ref[0][:ref[2]].view(np.uint32))
