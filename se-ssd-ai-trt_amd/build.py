@@ -20,6 +20,10 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-fast-math", "-Wall", "-Wno-unused-function",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
+# conv_tile.hip keeps its accumulators over a loop in which nothing else may wait; left to itself the compiler puts them
+# into accumulation registers and copies them back and forth once per kernel offset
+FILE_FLAGS = {"conv_tile.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+
 
 def sources():
     return sorted(glob.glob(os.path.join(SRC_DIR, "*.hip")))
@@ -39,7 +43,7 @@ def is_stale():
 
 def _compile(src):
     obj = os.path.join(OBJ_DIR, os.path.basename(src)[:-4] + ".o")
-    cmd = [HIPCC] + FLAGS + ["-c", src, "-o", obj]
+    cmd = [HIPCC] + FLAGS + FILE_FLAGS.get(os.path.basename(src), []) + ["-c", src, "-o", obj]
     r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     return src, obj, r.returncode, r.stdout
 

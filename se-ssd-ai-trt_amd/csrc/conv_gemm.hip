@@ -195,11 +195,13 @@ export_pairs(const int32_t* __restrict__ nbr, int max_voxels, int words_per_k,
 int launch_mfma(const GemmArgs& a, hipStream_t stream);  // conv_mfma.hip
 
 int launch_tall(const GemmArgs& a, hipStream_t stream);  // conv_tall.hip
+int launch_tile(const GemmArgs& a, hipStream_t stream);  // conv_tile.hip
 int launch_wide(const GemmArgs& a, hipStream_t stream);  // conv_wide.hip
 
 int launch_gather_gemm(const GemmArgs& a, hipStream_t stream) {
-    if (!a.force_valu) {  // FP16 3x3x3 layers from 32 channels up: the tall-tile kernel
-        const int rc = launch_tall(a, stream);
+    if (!a.force_valu) {  // FP16 layers from 32 channels up: one tile per compute unit, with Cin 32 tall tiles
+        int rc = launch_tile(a, stream);
+        if (rc == SESSD_E_UNSUPPORTED) rc = launch_tall(a, stream);
         if (rc != SESSD_E_UNSUPPORTED) return rc;
     }
     if (!a.force_valu) {  // FP32, 64 output columns: one tall tile per compute unit

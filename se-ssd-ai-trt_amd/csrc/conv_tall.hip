@@ -1,10 +1,10 @@
-// conv_tall.hip -- gather-GEMM for FP16 features with many active rows: tall tiles, weights through LDS.
+// conv_tall.hip -- gather-GEMM for FP16 layers with Cin 32: tall tiles, weights through LDS.
 //
 //     out[o][:] = epilogue( sum_k  in[nbr[k][o]][:] @ W[k] )
 //
 // The split-K kernel of conv_mfma.hip requests all of W once per 48..64-row tile; in FP16, where the matrix cores
-// are far from busy, those requests (and, at 128 columns, every row gathered twice) are what the compute units'
-// load path spends its time on.  Here a workgroup (4 wave64) owns 64 or 128 consecutive output rows:
+// are far from busy, those requests are what the compute units' load path spends its time on.  Here a workgroup (4
+// wave64) owns 64 or 128 consecutive output rows:
 //   * W[k] is copied once per workgroup and offset into LDS (two buffers; the host's MFMA operand order is also
 //     the LDS order): every wave requests its share a few offsets ahead into registers and stores it one offset
 //     before its use;
@@ -20,6 +20,8 @@
 // requests" did not reliably cover such a copy when ordinary loads were in flight behind it -- stale weights in a
 // few tiles per thousand launches -- and waiting for everything gives up the prefetch.)
 // Summation order per output element: offsets ascending, channels inside the MFMA: fixed, run-to-run identical.
+// (The ring of conv_tile.hip, faster from 64 channels up, has too little work per row here: 32 -> 32 at 60 000 rows
+// 15.6 us, this kernel 10.7; its slices would be half a cache line.)
 #include <type_traits>
 
 #include "kernels.h"
@@ -34,7 +36,6 @@ typedef unsigned int v4u32 __attribute__((__vector_size__(16)));
 
 constexpr int kWaves = 4;
 constexpr int kGroupsAhead = 3;  // groups of weight fragments a wave has requested from LDS ahead of the one it multiplies
-constexpr int kMaxK = kGemmMaxOffsets;
 constexpr unsigned kOutOfRange = 0x80000000u;
 constexpr int kRawBuffer = 0x00020000;
 
@@ -348,19 +349,10 @@ bool gemm_runs_tall(int K, int cin, int cout, int in_type, int out_type) {
     return (cin == 128 && cout == 128) || (cin == 64 && (cout == 128 || cout == 64)) || (cin == 32 && (cout == 64 || cout == 32));
 }
 
-// FP16 layers with 3x3x3 (or the reference's last 3x1x1) kernels whose inner dimension fills whole 32-channel chunks;
-// SESSD_E_UNSUPPORTED otherwise
 int launch_tall(const GemmArgs& a, hipStream_t stream) {
-    if (!a.w_packed || !gemm_runs_tall(a.K, a.cin, a.cout, a.in_type, a.out_type)) return SESSD_E_UNSUPPORTED;
+    if (!a.w_packed || a.K != 27 || a.in_type != SESSD_HALF || a.out_type != SESSD_HALF) return SESSD_E_UNSUPPORTED;
     if ((reinterpret_cast<uintptr_t>(a.in_feat) | reinterpret_cast<uintptr_t>(a.out_feat)) & 15) return SESSD_E_UNSUPPORTED;
     // <Cin, Cout, row blocks per wave in tall tiles, offsets the rows are requested ahead, weight register sets, K>
-    if (a.K == 3) {
-        if (a.cin == 128) return launch<128, 128, 2, 1, 1, 3>(a, stream);
-        return launch<64, 64, 2, 2, 2, 3>(a, stream);
-    }
-    if (a.cin == 128 && a.cout == 128) return launch<128, 128, 2, 1, 1, 27>(a, stream);
-    if (a.cin == 64 && a.cout == 128) return launch<64, 128, 2, 2, 1, 27>(a, stream);
-    if (a.cin == 64 && a.cout == 64) return launch<64, 64, 2, 3, 2, 27>(a, stream);
     if (a.cin == 32 && a.cout == 64) return launch<32, 64, 2, 3, 2, 27>(a, stream);
     if (a.cin == 32 && a.cout == 32) return launch<32, 32, 2, 3, 2, 27>(a, stream);
     return SESSD_E_UNSUPPORTED;

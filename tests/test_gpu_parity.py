@@ -755,6 +755,19 @@ def test_tall_fp16_kernel_with_two_row_blocks_per_wave(cin, cout, n):
         O.set_threads(1)
 
 
+@pytest.mark.parametrize("cin,cout,n", [(64, 64, 16384), (64, 64, 16385), (64, 64, 65537), (64, 64, 81920), (64, 64, 81921),
+                                        (64, 128, 8193), (128, 128, 8192), (128, 128, 8193), (128, 128, 32769), (128, 128, 49152),
+                                        (128, 128, 49153)])
+def test_fp16_ring_kernel_around_the_row_counts_of_its_tile_heights(cin, cout, n):
+    """On 256 compute units a tile of the LDS-ring kernel is 64 m rows high with 64 columns (m = 1 .. 5) and 32 m with 128
+    (m = 1 .. 6), the smallest that makes the launch one round of tiles; beyond the tallest there are two rounds."""
+    O.set_threads(16)
+    try:
+        _fp16_subm_against_oracle(cin, cout, n, n + 70, (21, 400, 352), 6000 + cin + cout)
+    finally:
+        O.set_threads(1)
+
+
 # ---------------------------------------------------------------------------------------------
 # the FP32 kernel with one tall tile per compute unit (conv_wide.hip: 64 -> 64 and 32 -> 64)
 # ---------------------------------------------------------------------------------------------
