@@ -99,8 +99,9 @@ struct Pipeline {
     std::vector<hipEvent_t> ev_pass;
     // The voxelizer's cell table is empty at the start of a frame: a pass behind its last reader empties it for the next
     // one (a clear at the head of a frame was 4-6 us of every frame).  The strided layers' dense tables hold the rows
-    // of the frame before, as their coors tensors do.  False: clear them first (the first frame, one that did not get
-    // to its end, or one that has run plugin by plugin).
+    // of the frame before, as their coors tensors do.  create() clears all of them, and so does a frame that has run
+    // plugin by plugin (behind its end): a frame that a caller has captured holds no clear of its own.  False: a frame
+    // did not get to its end, clear them first.
     bool tables_ready = false;
 
     // profiling: one event per segment boundary (see sessd_pipeline_enqueue_timed)
@@ -159,11 +160,8 @@ struct Pipeline {
                 f = FillArgs();
             }
             f.add(st->cells.p, st->cells.bytes / sizeof(uint32_t), kEmpty);
-            f.add(st->num.p, 4, 0);  // (no rows of a frame before)
         }
-        SESSD_TRY(launch_fill(f, stream));
-        tables_ready = true;
-        return SESSD_OK;
+        return launch_fill(f, stream);
     }
 
     // The rows of stage 0 are the voxels, those of stage i the output rows of the i-th strided layer.
@@ -219,6 +217,7 @@ struct Pipeline {
         // cleared beside vg_insert: the cells of the last frame's rows, the dense tensor; beside vg_flags: coordinate
         // rows beyond the active ones where the flags ask for them (the cells are found by them)
         FillArgs clears, pads;
+        std::vector<FillArgs> overflow;  // (of a backbone with dozens of strided layers)
         std::vector<CleanPart> cleans;
         for (int i = 1; i <= m; ++i) {
             ConvStage& st = *stages[(size_t)cs[(size_t)i].layer];
@@ -227,8 +226,11 @@ struct Pipeline {
             part[(size_t)i] = st.sparse->part(rows[(size_t)i - 1].coors, rows[(size_t)i - 1].num, static_cast<int32_t*>(st.coors.p),
                                               static_cast<int32_t*>(st.num.p), st.ws.p, false);
             part[(size_t)i].t = rows[(size_t)i].table;
-            if (clears.n + 6 > FillArgs::kMaxRegions || pads.n + 2 > FillArgs::kMaxRegions)
-                return fail(SESSD_E_UNSUPPORTED, "pipeline: more than %d strided layers", FillArgs::kMaxRegions - 6);
+            for (FillArgs* f : {&clears, &pads})
+                if (f->n + 6 > FillArgs::kMaxRegions) {
+                    overflow.push_back(*f);
+                    *f = FillArgs();
+                }
             if (st.cells.p && cleans.size() < (size_t)kMaxCleans) {
                 CleanPart c;
                 c.coors = rows[(size_t)i].coors;
@@ -251,6 +253,7 @@ struct Pipeline {
                                   static_cast<int32_t*>(vg_num.p), vg_ws.p);
         v.t = rows[0].table;
         SESSD_TRY(launch_vg_insert(v, cleans.data(), (int)cleans.size(), clears, stream));
+        for (const FillArgs& f : overflow) SESSD_TRY(launch_fill(f, stream));
         SESSD_TRY(launch_vg_flags(v, pads, stream));
         SESSD_TRY(launch_vg_finalize(v, m ? &part[1] : nullptr, stream));
 
@@ -549,8 +552,9 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
         FillArgs f;
         f.add(static_cast<uint8_t*>(P->vg_ws.p) + vg->statusOffset(d.max_points), 4, 0);
         for (auto& st : P->stages) {
+            if (st->num.p) f.add(st->num.p, 4, 0);  // (no rows of a frame before)
             if (!st->ws.p) continue;
-            if (f.n + 2 > FillArgs::kMaxRegions) {
+            if (f.n + 3 > FillArgs::kMaxRegions) {
                 SESSD_TRY(launch_fill(f, nullptr));
                 f = FillArgs();
             }
@@ -558,7 +562,9 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
             else st->sparse->collectHeaderFill(st->ws.p, f);
         }
         SESSD_TRY(launch_fill(f, nullptr));
+        SESSD_TRY(P->clearTables(nullptr));
         SESSD_HIP_TRY(hipStreamSynchronize(nullptr));
+        P->tables_ready = true;
     }
     // the layer array of the caller need not outlive create()
     P->desc.layers = nullptr;
@@ -657,7 +663,16 @@ static Pipeline* current(sessd_pipeline* h) {
 // changed), direct launches otherwise
 static int run_frame(Pipeline* P, const void* points, const void* points_size, void* dense, hipStream_t stream) {
     auto run = [&](hipStream_t st) { return P->enqueueFrame(points, points_size, dense, st); };
-    if (!P->tables_ready) SESSD_TRY(P->clearTables(stream));
+    if (!P->tables_ready) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        SESSD_HIP_TRY(hipStreamIsCapturing(stream, &capture));
+        SESSD_TRY(P->clearTables(stream));
+        if (capture != hipStreamCaptureStatusNone) {  // the caller's own graph: nothing is cleared until it is launched
+            const int rc = run(stream);
+            P->tables_ready = false;
+            return rc;
+        }
+    }
     if (!P->desc.use_graph || stream == nullptr) return run(stream);
     CapturedGraph& g = P->captured;
     if (!g.exec || g.points != points || g.size != points_size || g.dense != dense) {
@@ -829,7 +844,7 @@ int sessd_pipeline_enqueue_timed(sessd_pipeline* h, const void* points, const vo
     SESSD_HIP_TRY(hipEventRecord(P->events[n_seg + 2], stream));
     SESSD_HIP_TRY(hipEventRecord(P->events[0], stream));
     int rc;
-    P->tables_ready = false;  // (the voxelizer alone leaves its table filled)
+    P->tables_ready = false;  // (the plugins leave their tables filled)
     {
         const void* vin[2] = {points, points_size};
         void* vout[3] = {P->vg_voxels.p, P->vg_coors.p, P->vg_num.p};
@@ -844,6 +859,8 @@ int sessd_pipeline_enqueue_timed(sessd_pipeline* h, const void* points, const vo
         b->ev_gemm_begin_ = b->ev_gemm_end_ = nullptr;
     }
     SESSD_TRY(rc);
+    SESSD_TRY(P->clearTables(stream));
+    P->tables_ready = true;
     SESSD_HIP_TRY(hipStreamSynchronize(stream));
     for (int i = 0; i < n_seg; ++i)
         SESSD_HIP_TRY(hipEventElapsedTime(&segment_ms[i], P->events[i], P->events[i + 1]));

@@ -459,3 +459,59 @@ def test_voxelizer_keeps_the_first_points_of_crowded_cells(max_pts):
         assert int(num[0]) == ref[2]
         assert np.array_equal(to_np(coors)[:ref[2]], ref[1][:ref[2]])
         assert np.array_equal(to_np(voxels)[:ref[2]].view(np.uint32), ref[0][:ref[2]].view(np.uint32))
+
+
+@pytest.mark.parametrize("overlap", [True, False])
+def test_a_frame_in_the_callers_own_graph_finds_its_tables_empty(overlap):
+    """The first frame of a pipeline is captured by the caller and launched only after a frame of another size has run
+    directly; later replays follow direct frames and a plugin-by-plugin run.  No frame may depend on clears that another
+    one was meant to make."""
+    layers = B.reference_layers()
+    W = B.random_weights(layers, seed=12, w_std=0.05)
+    mp, mv = 1024, 20000
+    pipe = api.Pipeline(layers, W, mp, mv, share_rulebooks=True, skip_pad_rows=True, overlap_streams=overlap)
+    p, n = points_input(np.zeros((0, 4), np.float32), mp)
+    dense, stream = pipe.new_dense(), torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        pipe.enqueue(p, n, dense, stream)
+    for step, how in enumerate(("direct", "graph", "timed", "graph", "direct", "graph", "graph")):
+        npts = (700, 300, 1000, 500, 0, 900, 200)[step]
+        pts = F.lidar_frame(npts, 80 + step) if npts else np.zeros((0, 4), np.float32)
+        hp, hn = points_input(pts, mp)
+        with torch.cuda.stream(stream):
+            p.copy_(hp)
+            n.copy_(hn)
+            if how == "graph":
+                graph.replay()
+            elif how == "timed":
+                pipe.enqueue_timed(p, n, dense, stream)
+            else:
+                pipe.enqueue(p, n, dense, stream)
+        stream.synchronize()
+        ref = O.frame(pts, B.voxelgen_desc(max_voxels=mv), layers, W, B.dense_desc())
+        assert pipe.status() == ref["status"] == 0
+        assert [pipe.layer_count(l) for l in range(-1, len(layers))] == list(ref["counts"]), (step, how)
+        assert np.array_equal(pipe.read_layer(len(layers) - 1)[1], ref["coors"]), (step, how)
+        assert_end_to_end_close(to_np(dense), ref["dense"], False, "dense, step %d" % step)
+
+
+def test_dozens_of_strided_layers():
+    """More strided layers than the clears of one launch can hold; two frames, the second smaller."""
+    layers = B.reference_layers()
+    grid = layers[-2].out_shape
+    layers[-1:-1] = [B.Layer("s%d" % i, D.SESSD_LAYER_SPARSE, 64, 64, grid, (3, 1, 1), (1, 1, 1), (1, 0, 0)) for i in range(46)]
+    W = B.random_weights(layers, seed=13, w_std=0.05)
+    mp, mv = 512, 8000
+    pipe = api.Pipeline(layers, W, mp, mv, share_rulebooks=True)
+    dense, stream = pipe.new_dense(), torch.cuda.Stream()
+    for step, npts in enumerate((400, 250)):
+        pts = F.lidar_frame(npts, 90 + step)
+        p, n = points_input(pts, mp)
+        torch.cuda.synchronize()
+        pipe.enqueue(p, n, dense, stream)
+        stream.synchronize()
+        ref = O.frame(pts, B.voxelgen_desc(max_voxels=mv), layers, W, B.dense_desc())
+        assert pipe.status() == ref["status"] == 0
+        assert [pipe.layer_count(l) for l in range(-1, len(layers))] == list(ref["counts"])
+        assert np.array_equal(pipe.read_layer(len(layers) - 1)[1], ref["coors"])
