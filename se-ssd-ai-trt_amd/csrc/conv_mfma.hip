@@ -32,7 +32,9 @@
 //     output row is written once, coalesced.  No global atomics; results are bit-identical run to run.
 //     A caller may name a dense tensor (DenseTarget): the epilogue then also stores every row at its voxel's
 //     place there, which is the sparse2Dense step that follows the last layer.
-#include "kernels.h"
+#include <type_traits>
+
+#include "pad_rows.h"
 
 namespace sessd {
 
@@ -149,13 +151,14 @@ constexpr int min_waves_per_simd(int cin, int cout) {
 }
 
 // T = type of the input features and of the arithmetic's operands, TO = type the output rows are stored
-// in (differs only for the first layer of an FP16 pipeline: FP32 voxel means in, FP16 features out)
-template <typename T, int CIN, int COUT, typename TO = T>
+// in (differs only for the first layer of an FP16 pipeline: FP32 voxel means in, FP16 features out), PAD: the rows
+// beyond the active ones are written too
+template <typename T, int CIN, int COUT, typename TO, bool PAD>
 __global__ void __launch_bounds__(kWaves * 64, min_waves_per_simd(CIN, COUT))
 conv_mfma(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict__ Wp,
           const int32_t* __restrict__ nbr, const int32_t* __restrict__ num_out, int max_voxels, int K,
-          const float* __restrict__ scale, const float* __restrict__ shift, int relu, int write_pad,
-          int num_cu, const int32_t* __restrict__ tiles, DenseTarget dt) {
+          const float* __restrict__ scale, const float* __restrict__ shift, int relu, int num_cu,
+          const int32_t* __restrict__ tiles, DenseTarget dt) {
     using C = Chunk<T, CIN>;
     using Vec = typename C::Vec;
     constexpr int G = CIN / C::kChannels;  // K-chunks of the inner dimension
@@ -203,35 +206,19 @@ conv_mfma(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
     const int ec4 = (tid % kVecPerRow) * 4;  // this thread's epilogue columns, the same for every row it stores
     static_assert((kWaves * 64) % kVecPerRow == 0, "a thread must keep its columns from row to row");
 
-    // rows >= n: the reference zero-fills them (then BN+ReLU): epilogue(0), spread over all workgroups
-    if (write_pad) {
-        const int chunks = (max_voxels - n + kTileRows - 1) / kTileRows;
-        for (int c = blockIdx.x; c < chunks; c += gridDim.x)
-            for (int v = tid; v < kTileRows * kVecPerRow; v += kWaves * 64) {
-                const int row = n + c * kTileRows + v / kVecPerRow, c4 = (v % kVecPerRow) * 4;
-                if (row >= max_voxels) continue;
-                float o[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float s = 0.f;
-                    if (scale) s = s * scale[c4 + e];
-                    if (shift) s = s + shift[c4 + e];
-                    if (relu) s = s > 0.f ? s : 0.f;
-                    o[e] = s;
-                }
-                store4(out + (size_t)row * COUT + c4, o);
-            }
-    }
     // this workgroup's run of rows: from the rulebook's equal-work cuts, or equal lengths
     int run_begin, run_end;
     if (cut_count > 0) {
-        if ((int)blockIdx.x >= cut_count) return;
-        run_begin = cut_begin;
-        run_end = cut_end;
+        run_begin = (int)blockIdx.x < cut_count ? cut_begin : 0;
+        run_end = (int)blockIdx.x < cut_count ? cut_end : 0;
     } else {
         const int R = tile_plan(n, num_cu, kTileRows).height;
         run_begin = blockIdx.x * R;
         run_end = run_begin + R < n ? run_begin + R : n;
+    }
+    if (PAD && run_begin >= run_end && tid < COUT) {  // (no tile stages them)
+        s_epi[tid] = epi_scale;
+        s_epi[COUT + tid] = epi_shift;
     }
     const int i = lane & 15;  // pair inside a 16-pair block
     const int q = lane >> 4;  // channel group inside a K-chunk
@@ -461,6 +448,10 @@ conv_mfma(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
     }
     __syncthreads();  // the next piece reuses the lists and partial tiles
     }
+    if constexpr (PAD) {
+        __syncthreads();
+        write_pad_rows<TO, COUT, kWaves * 64>(out, n, max_voxels, s_epi, scale != nullptr, shift != nullptr, relu);
+    }
 }
 
 int compute_units() {
@@ -486,10 +477,12 @@ int launch(const GemmArgs& a, hipStream_t stream) {
     // enough workgroups for any cut of any n <= max_voxels rows: tile_plan() never makes more tiles for fewer
     // rows or a taller target (surplus workgroups return at once)
     const unsigned blocks = (unsigned)tile_plan(a.max_voxels, num_cu, kGemmMinTileRows).count;
-    hipLaunchKernelGGL((conv_mfma<T, CIN, COUT, TO>), dim3(blocks), dim3(kWaves * 64), 0, stream,
-                       static_cast<const T*>(a.in_feat), static_cast<TO*>(a.out_feat), a.w_packed, a.nbr,
-                       a.num_out, a.max_voxels, a.K, a.scale, a.shift, a.relu, a.write_pad_rows, num_cu, a.tiles,
-                       a.dense);
+    auto go = [&](auto pad) {
+        hipLaunchKernelGGL((conv_mfma<T, CIN, COUT, TO, decltype(pad)::value>), dim3(blocks), dim3(kWaves * 64), 0, stream,
+                           static_cast<const T*>(a.in_feat), static_cast<TO*>(a.out_feat), a.w_packed, a.nbr,
+                           a.num_out, a.max_voxels, a.K, a.scale, a.shift, a.relu, num_cu, a.tiles, a.dense);
+    };
+    a.write_pad_rows ? go(std::true_type{}) : go(std::false_type{});
     SESSD_HIP_TRY(hipGetLastError());
     return SESSD_OK;
 }

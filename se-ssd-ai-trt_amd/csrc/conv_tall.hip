@@ -24,7 +24,7 @@
 // 15.6 us, this kernel 10.7; its slices would be half a cache line.)
 #include <type_traits>
 
-#include "kernels.h"
+#include "pad_rows.h"
 
 namespace sessd {
 
@@ -277,27 +277,7 @@ conv_tall(const __half* __restrict__ in, __half* __restrict__ out, const void* _
     int n = *num_out;
     n = n < 0 ? 0 : (n > max_voxels ? max_voxels : n);
     const int tid = threadIdx.x;
-    constexpr int kVecPerRow = COUT / 4;
 
-    // rows >= n: epilogue(0), as the reference's zero fill followed by BN + ReLU
-    if (write_pad) {
-        const int chunks = (max_voxels - n + 63) / 64;
-        for (int c = blockIdx.x; c < chunks; c += gridDim.x)
-            for (int v = tid; v < 64 * kVecPerRow; v += kWaves * 64) {
-                const int row = n + c * 64 + v / kVecPerRow, c4 = (v % kVecPerRow) * 4;
-                if (row >= max_voxels) continue;
-                float o[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float s = 0.f;
-                    if (scale) s = s * scale[c4 + e];
-                    if (shift) s = s + shift[c4 + e];
-                    if (relu) s = s > 0.f ? s : 0.f;
-                    o[e] = s;
-                }
-                store4h(out + (size_t)row * COUT + c4, o);
-            }
-    }
     if (tid < COUT) {  // (published by the barrier behind the list staging)
         s_epi[tid] = scale ? scale[tid] : 1.f;
         s_epi[COUT + tid] = shift ? shift[tid] : 0.f;
@@ -317,6 +297,10 @@ conv_tall(const __half* __restrict__ in, __half* __restrict__ out, const void* _
         tall_tile<CIN, COUT, RB, D, DW, KC>(in, out, Wp, nbr, n, b * kTall, max_voxels, scale != nullptr, shift != nullptr, relu, dt, s_nbr, s_epi);
     else
         tall_tile<CIN, COUT, 1, D, DW, KC>(in, out, Wp, nbr, n, n_tall * kTall + (b - n_tall) * kShort, max_voxels, scale != nullptr, shift != nullptr, relu, dt, s_nbr, s_epi);
+    if (write_pad) {
+        __syncthreads();
+        write_pad_rows<__half, COUT, kWaves * 64>(out, n, max_voxels, s_epi, scale != nullptr, shift != nullptr, relu);
+    }
 }
 
 template <int CIN, int COUT, int RB, int D, int DW, int KC>

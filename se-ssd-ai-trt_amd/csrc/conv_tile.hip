@@ -31,7 +31,7 @@
 // 29.9 -> 24.4, at 26 247 rows 14.9 -> 11.7, at 3 060 rows 9.0 -> 8.5.  Beyond 40 960 rows (Cout 128) the loads bound it.
 #include <type_traits>
 
-#include "kernels.h"
+#include "pad_rows.h"
 
 namespace sessd {
 
@@ -301,27 +301,7 @@ conv_tile(const __half* __restrict__ in, __half* __restrict__ out, const void* _
     int n = *num_out;
     n = n < 0 ? 0 : (n > max_voxels ? max_voxels : n);
     const int tid = threadIdx.x;
-    constexpr int kVecPerRow = COUT / 4;
 
-    // rows >= n: epilogue(0), as the reference's zero fill followed by BN + ReLU
-    if (write_pad) {
-        const int chunks = (max_voxels - n + 63) / 64;
-        for (int c = blockIdx.x; c < chunks; c += gridDim.x)
-            for (int v = tid; v < 64 * kVecPerRow; v += kThreads) {
-                const int row = n + c * 64 + v / kVecPerRow, c4 = (v % kVecPerRow) * 4;
-                if (row >= max_voxels) continue;
-                float o[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float s = 0.f;
-                    if (scale) s = s * scale[c4 + e];
-                    if (shift) s = s + shift[c4 + e];
-                    if (relu) s = s > 0.f ? s : 0.f;
-                    o[e] = s;
-                }
-                store4h(out + (size_t)row * COUT + c4, o);
-            }
-    }
     if (tid < COUT) {  // (published by the barrier behind the list staging)
         s_epi[tid] = scale ? scale[tid] : 1.f;
         s_epi[COUT + tid] = shift ? shift[tid] : 0.f;
@@ -355,6 +335,10 @@ conv_tile(const __half* __restrict__ in, __half* __restrict__ out, const void* _
         case 5: tiles(std::integral_constant<int, 5>{}); break;
         case 6: tiles(std::integral_constant<int, 6>{}); break;
         default: break;  // no rows
+    }
+    if (write_pad) {
+        __syncthreads();
+        write_pad_rows<__half, COUT, kThreads>(out, n, max_voxels, s_epi, hs, hb, relu);
     }
 }
 

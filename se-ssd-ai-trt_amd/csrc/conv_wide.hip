@@ -21,7 +21,9 @@
 // Pair lists, operand order (the packed weights are conv_mfma.hip's), partial tiles in LDS (one per group and
 // column quarter, private to a wave, so the sum order is fixed), fixed-order reduction, fused scale/shift/ReLU and
 // the optional dense scatter are as in conv_mfma.hip; results are bit-identical run to run.
-#include "kernels.h"
+#include <type_traits>
+
+#include "pad_rows.h"
 
 namespace sessd {
 
@@ -51,12 +53,14 @@ __device__ __forceinline__ void mma16(const float4& w, const float4& x, v4f& acc
 
 // DENSE: the epilogue also scatters the rows into a dense tensor (the layer in front of sparse2Dense).  A variant of
 // its own because the scatter's addresses cost ten registers, and what this kernel leaves of the register file is
-// what the coordinate kernels of the frame's other branch run in beside it.
-template <int CIN, int COUT, bool DENSE>
+// what the coordinate kernels of the frame's other branch run in beside it.  PAD: the rows beyond the active ones are
+// written too; a variant for the same reason (with a run-time flag the scalar registers spill and the frame that asks for
+// no such rows is 9 us longer).
+template <int CIN, int COUT, bool DENSE, bool PAD>
 __global__ void __launch_bounds__(kWaves * 64)
 conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __restrict__ Wp,
           const int32_t* __restrict__ nbr, const int32_t* __restrict__ num_out, int max_voxels, int K,
-          const float* __restrict__ scale, const float* __restrict__ shift, int relu, int write_pad, int num_cu,
+          const float* __restrict__ scale, const float* __restrict__ shift, int relu, int num_cu,
           const int32_t* __restrict__ tiles, DenseTarget dt) {
     constexpr int G = CIN / 16;     // 16-channel chunks of the inner dimension
     constexpr int NBT = COUT / 16;  // 16-column blocks of the layer
@@ -114,25 +118,6 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
     const int pc4 = (tid & ((1 << lvec) - 1)) * 4, ec4 = part_id * (COUT >> lsplit) + pc4;
     static_assert(kVecPerRow == 16, "lvec");
 
-    // rows >= n: the reference zero-fills them (then BN+ReLU): epilogue(0), spread over all workgroups
-    if (write_pad) {
-        const int chunks = (max_voxels - n + kTileRows - 1) / kTileRows;
-        for (int c = blockIdx.x; c < chunks; c += gridDim.x)
-            for (int v = tid; v < kTileRows * kVecPerRow; v += kThreads) {
-                const int row = n + c * kTileRows + v / kVecPerRow, c4 = (v % kVecPerRow) * 4;
-                if (row >= max_voxels) continue;
-                float o[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float s = 0.f;
-                    if (scale) s = s * scale[c4 + e];
-                    if (shift) s = s + shift[c4 + e];
-                    if (relu) s = s > 0.f ? s : 0.f;
-                    o[e] = s;
-                }
-                *reinterpret_cast<float4*>(out + (size_t)row * COUT + c4) = make_float4(o[0], o[1], o[2], o[3]);
-            }
-    }
     // The grid is one workgroup per compute unit (a workgroup takes most of a unit's LDS, so workgroups with no
     // tile would queue behind the busy ones just to return); a workgroup walks tiles first_tile, first_tile +
     // row_groups, ...: runs of rows from the rulebook's equal-work cuts, or runs of equal length.
@@ -148,6 +133,7 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
     const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<void*>(Wp), 0, (int)((size_t)K * CIN * COUT * sizeof(float)), kRawBuffer);
 
+    bool idle = true;  // (no rows)
     for (int tile = first_tile; tile < tile_count; tile += row_groups) {
     int run_begin, run_end;
     if (cut_count > 0) {
@@ -177,6 +163,7 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
         s_epi[tid] = epi_scale;
         s_epi[COUT + tid] = epi_shift;
     }
+    idle = false;
     // zero this wave's partial tile (while the lists are on their way)
     float* part = s_part + wave * kTileRows * LDP;
     for (int t = lane; t < rows * LDP / 4; t += 64) reinterpret_cast<float4*>(part)[t] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -356,6 +343,14 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
     __syncthreads();  // the next piece reuses the lists and partial tiles
     }
     }
+    if constexpr (PAD) {
+        if (idle && tid < COUT) {  // (no tile has staged them)
+            s_epi[tid] = epi_scale;
+            s_epi[COUT + tid] = epi_shift;
+        }
+        __syncthreads();
+        write_pad_rows<float, COUT, kThreads>(out, n, max_voxels, s_epi, scale != nullptr, shift != nullptr, relu);
+    }
 }
 
 template <int CIN, int COUT>
@@ -365,16 +360,13 @@ int launch(const GemmArgs& a, hipStream_t stream) {
         return SESSD_E_UNSUPPORTED;
     const int num_cu = gemm_compute_units();
     const unsigned blocks = (unsigned)num_cu;
-    if (a.dense.dense)
-        hipLaunchKernelGGL((conv_wide<CIN, COUT, true>), dim3(blocks), dim3(kWaves * 64), 0, stream,
+    auto go = [&](auto dense, auto pad) {
+        hipLaunchKernelGGL((conv_wide<CIN, COUT, decltype(dense)::value, decltype(pad)::value>), dim3(blocks), dim3(kWaves * 64), 0, stream,
                            static_cast<const float*>(a.in_feat), static_cast<float*>(a.out_feat), a.w_packed, a.nbr,
-                           a.num_out, a.max_voxels, a.K, a.scale, a.shift, a.relu, a.write_pad_rows, num_cu, a.tiles,
-                           a.dense);
-    else
-        hipLaunchKernelGGL((conv_wide<CIN, COUT, false>), dim3(blocks), dim3(kWaves * 64), 0, stream,
-                           static_cast<const float*>(a.in_feat), static_cast<float*>(a.out_feat), a.w_packed, a.nbr,
-                           a.num_out, a.max_voxels, a.K, a.scale, a.shift, a.relu, a.write_pad_rows, num_cu, a.tiles,
-                           a.dense);
+                           a.num_out, a.max_voxels, a.K, a.scale, a.shift, a.relu, num_cu, a.tiles, a.dense);
+    };
+    if (a.dense.dense) a.write_pad_rows ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
+    else a.write_pad_rows ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
     SESSD_HIP_TRY(hipGetLastError());
     return SESSD_OK;
 }

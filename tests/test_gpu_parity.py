@@ -819,3 +819,21 @@ def test_wide_fp32_kernel_tall_tiles_and_two_tiles_per_workgroup(n, clustered, c
 def test_wide_fp32_kernel_around_the_row_counts_of_its_column_splits(n, cin):
     """On 256 compute units a tile's columns are dealt to four workgroups up to 3 072 rows, to two up to 10 240."""
     _fp32_subm_wide_against_oracle(n, n + 7, (11, 200, 176), 900 + n, threads=8, cin=cin)
+
+
+@pytest.mark.parametrize("cin,cout,half", [(16, 32, False), (64, 64, False), (32, 64, False), (128, 128, False), (16, 16, True),
+                                           (32, 64, True), (64, 64, True), (128, 128, True)])
+def test_every_row_is_a_pad_row(cin, cout, half):
+    """No active row: all workgroups of a gather-GEMM only write relu(shift), in each kernel, at row counts that do not
+    divide by anything the kernels count in."""
+    rng = np.random.default_rng(cin + cout)
+    sh = rng.uniform(-0.5, 0.5, cout).astype(np.float32)
+    for mv in (1, 257, 40003):
+        conv = api.SubmConv3d(cin, cout, (40, 40, 5), rng.normal(0, 0.1, (27, cin, cout)).astype(np.float32), mv)
+        conv.set_epilogue(np.ones(cout, np.float32), sh, relu=True)
+        feat = dev(np.ones((mv, cin), np.float16 if half else np.float32))
+        y = conv(feat, dev(np.zeros((mv, 4), np.int32)), dev(np.array([0], np.int32)))
+        torch.cuda.synchronize()
+        want = np.maximum(sh, 0).astype(np.float16 if half else np.float32)
+        assert np.array_equal(to_np(y), np.broadcast_to(want, (mv, cout))), mv
+        conv.close()
