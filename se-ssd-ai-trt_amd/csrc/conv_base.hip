@@ -101,8 +101,8 @@ bool ConvPluginBase::gemmOnMatrixCores() const {
 }
 
 int ConvPluginBase::tileRows() const { return gemm_tile_rows(in_channel_, out_channel_, out_type_); }
-bool ConvPluginBase::tilesWide() const {
-    return gemm_runs_wide(kernel_volume_, in_channel_, out_channel_, in_type_, out_type_);
+int ConvPluginBase::tilesWide() const {
+    return gemm_runs_wide(kernel_volume_, in_channel_, out_channel_, in_type_, out_type_) ? out_channel_ / 64 : 0;
 }
 int ConvPluginBase::tileRowWeight() const { return tilesWide() ? 4 : 20; }
 

@@ -571,7 +571,10 @@ int launch_mfma(const GemmArgs& a, hipStream_t stream) {
     SESSD_CASE(16, 16);
     SESSD_CASE(16, 32);
     SESSD_CASE(32, 32);
-    SESSD_CASE(32, 64);
+#undef SESSD_CASE
+#define SESSD_CASE(CI, CO) \
+    if (a.cin == CI && a.cout == CO && a.in_type == SESSD_HALF) return launch<__half, CI, CO>(a, stream)
+    SESSD_CASE(32, 64);  // (FP32: conv_wide.hip)
     SESSD_CASE(64, 64);
     SESSD_CASE(64, 128);
     SESSD_CASE(128, 128);

@@ -1,5 +1,5 @@
-// conv_wide.hip -- FP32 gather-GEMM for the layers with 64 output columns (Cin 32 or 64): one tall tile per compute
-// unit, sixteen waves.
+// conv_wide.hip -- FP32 gather-GEMM for the layers with 64 (Cin 32 or 64) or 128 output columns (Cin 64 or 128): one tall
+// tile per compute unit, sixteen waves.
 //
 //     out[o][:] = epilogue( sum_k  in[nbr[k][o]][:] @ W[k] )
 //
@@ -18,6 +18,10 @@
 //     tile, each taking a half or a quarter of the columns with 8 or 16 offset groups (wide_log2_split()).  Measured,
 //     launches back to back: 64 -> 64 at 2 259 rows 14.2 -> 9.9 us, at 3 476 rows 14.3 -> 11.4, at 8 615 rows 20.1 -> 19.1;
 //     at 16 914 rows unsplit tiles are the faster ones (29.5 us).
+//   * 128 columns: two workgroups take 64 each of every tile, as in such a split.  128 input channels: an offset's blocks
+//     are walked twice, with 64 channels each, so that the registers stay those of 64 (the split-K kernel spilled 297 of
+//     them).  128 -> 128, launches back to back: 3 877 rows 174 -> 41 us, 17 060 rows 270 -> 131 (floor by the matrix cores'
+//     rate 47); distance from the sums in 64 bits 1.7e-7 -> 1.4e-7 of their norm.
 // Pair lists, operand order (the packed weights are conv_mfma.hip's), partial tiles in LDS (one per group and
 // column quarter, private to a wave, so the sum order is fixed), fixed-order reduction, fused scale/shift/ReLU and
 // the optional dense scatter are as in conv_mfma.hip; results are bit-identical run to run.
@@ -60,20 +64,19 @@ template <int CIN, int COUT, bool DENSE, bool PAD>
 __global__ void __launch_bounds__(kWaves * 64)
 conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __restrict__ Wp,
           const int32_t* __restrict__ nbr, const int32_t* __restrict__ num_out, int max_voxels, int K,
-          const float* __restrict__ scale, const float* __restrict__ shift, int relu, int num_cu,
+          const float* __restrict__ scale, const float* __restrict__ shift, int relu, int units,
           const int32_t* __restrict__ tiles, DenseTarget dt) {
-    constexpr int G = CIN / 16;     // 16-channel chunks of the inner dimension
-    constexpr int NBT = COUT / 16;  // 16-column blocks of the layer
-    constexpr int kQ = 4;          // a wave takes a quarter of the layer's columns
-    constexpr int NB = NBT / kQ;   // column blocks of one wave
-    constexpr int CW = COUT / kQ;  // columns of one wave
+    constexpr int kParts = CIN > 64 ? CIN / 64 : 1;  // of the inner dimension, taken one after the other
+    constexpr int CP = CIN / kParts;  // channels of a part
+    constexpr int G = CP / 16;        // 16-channel chunks of a part
+    constexpr int NBT = COUT / 16;    // 16-column blocks of the layer
+    constexpr int NB = 1;             // column blocks of one wave
+    constexpr int CW = 16;            // columns of one wave
+    constexpr int kWgCols = 64;       // columns of a workgroup (before the split of short tiles)
     constexpr int LDP = CW + 4;     // padded row stride of a partial tile
     static_assert(kTileRows <= 128 && kTileRows % 16 == 0, "the lists are staged in two halves of 64 rows");
-    constexpr int kVecPerRow = COUT / 4;
     constexpr int kThreads = kWaves * 64;
-    static_assert(CIN % 16 == 0 && NBT % kQ == 0, "channel counts must fill whole MFMA chunks per wave");
-    static_assert(kThreads % kVecPerRow == 0, "a thread must keep its columns from row to row");
-    static_assert(COUT == 64, "the split below counts in quarters of 16 columns");
+    static_assert(CIN % 16 == 0 && CIN % kParts == 0 && COUT % kWgCols == 0, "whole MFMA chunks and column groups");
     __shared__ int32_t s_in[kMaxK * kTileRows];   // compacted pair lists: input row ...
     __shared__ uint8_t s_row[kMaxK * kTileRows];  // ... and local output row of pair j of offset k
     __shared__ int32_t s_cnt[kMaxK + 5];          // pairs per offset
@@ -82,32 +85,38 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
 
     int n = *num_out;
     const int cut_count = tiles ? tiles[0] : 0;
+    // Workgroups of `units` tiles for each 64 columns of the layer; what follows counts inside one such group.
+    int block = blockIdx.x, col0 = 0;
+    if constexpr (COUT > kWgCols) {
+        col0 = block / units * kWgCols;
+        block %= units;
+    }
     // the cuts of this workgroup's first tile under each split it may be part of: requested beside the row count
     int cut_begin[3], cut_end[3];
-    int tile_of[3] = {(int)blockIdx.x, (int)blockIdx.x, (int)blockIdx.x};
+    int tile_of[3] = {block, block, block};
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
 #pragma unroll
-        for (int part = 1; part < 1 << s; ++part) tile_of[s] -= (int)blockIdx.x >= part * (num_cu >> s) ? num_cu >> s : 0;
+        for (int part = 1; part < 1 << s; ++part) tile_of[s] -= block >= part * (units >> s) ? units >> s : 0;
         cut_begin[s] = tiles ? tiles[4 + tile_of[s]] : 0;
         cut_end[s] = tiles ? tiles[5 + tile_of[s]] : 0;
     }
     n = n < 0 ? 0 : (n > max_voxels ? max_voxels : n);
     // Column parts: 1 << lsplit workgroups share a tile.  The parts of a tile are row_groups apart in the grid, which
     // puts them on one XCD (workgroups are dealt round robin over eight): they read the same rows.
-    const int lsplit = wide_log2_split(n, K, num_cu);
-    const int row_groups = num_cu >> lsplit;  // workgroups of one column part
+    const int lsplit = wide_log2_split(n, K, units);
+    const int row_groups = units >> lsplit;  // workgroups of one column part
     const int first_tile = lsplit == 0 ? tile_of[0] : (lsplit == 1 ? tile_of[1] : tile_of[2]);
     int part_id = 0;
 #pragma unroll
-    for (int part = 1; part < 4; ++part) part_id += (int)blockIdx.x >= part * row_groups ? 1 : 0;
+    for (int part = 1; part < 4; ++part) part_id += block >= part * row_groups ? 1 : 0;
     const int lcs = 2 - lsplit, cs = 1 << lcs;                // waves of a group: the column quarters of this part
     const int lkg = 4 - lcs, kg = 1 << lkg;                   // groups the offsets are dealt to
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (tells the compiler that it is wave-uniform)
     const int kgrp = wave >> lcs;                                // offsets are dealt to this group ...
-    const int quarter = (part_id << lcs) + (wave & (cs - 1));  // ... and this wave computes these columns of them
+    const int quarter = col0 / CW + (part_id << lcs) + (wave & (cs - 1));  // ... and this wave computes these columns of them
     float epi_scale = 1.f, epi_shift = 0.f;
     if (tid < COUT) {
         if (scale) epi_scale = scale[tid];
@@ -115,8 +124,7 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
     }
     // this thread's epilogue columns (the same for every row it stores): within the part, and of the layer
     const int lvec = 4 - lsplit;  // log2 of the part's 4-column vectors
-    const int pc4 = (tid & ((1 << lvec) - 1)) * 4, ec4 = part_id * (COUT >> lsplit) + pc4;
-    static_assert(kVecPerRow == 16, "lvec");
+    const int pc4 = (tid & ((1 << lvec) - 1)) * 4, ec4 = col0 + part_id * (kWgCols >> lsplit) + pc4;
 
     // The grid is one workgroup per compute unit (a workgroup takes most of a unit's LDS, so workgroups with no
     // tile would queue behind the busy ones just to return); a workgroup walks tiles first_tile, first_tile +
@@ -212,11 +220,11 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
     // different rows and the same request takes four lookups: 18 instead of 48 bytes per cycle and compute unit,
     // measured.  The operand order is restored by a lane permutation (fetch()) before the MFMAs.
     // Padding lanes ask out of range (such a request returns zeros and touches no memory).
-    auto row_at = [&](int k, int cnt, int blk) -> unsigned {
+    auto row_at = [&](int k, int cnt, int blk, int part) -> unsigned {
         const int j = blk * 16 + (lane >> 2);
         const bool live = j < cnt;
         const int idx = s_in[k * kTileRows + (live ? j : 0)];
-        return live ? (unsigned)((idx * CIN + (lane & 3) * 4) * (int)sizeof(float)) : kOutOfRange;
+        return live ? (unsigned)((idx * CIN + part * CP + (lane & 3) * 4) * (int)sizeof(float)) : kOutOfRange;
     };
     const int from_lane4 = (4 * i + q) * 4;  // ds_bpermute address: this lane's operand sits in lane 4 * i + q
     auto fetch = [&](const float4& v) -> float4 {
@@ -232,8 +240,8 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
         for (int g = 0; g < G; ++g) a[g] = buffer_load16(rs_in, at + g * 16 * (unsigned)sizeof(float));
     };
     // chunk g of this wave's columns of W[k] -> operand registers (k < 0: nothing to fetch)
-    auto load_b = [&](int k, int g, float4 (&b)[NB]) {
-        const unsigned at = k >= 0 ? (unsigned)(((((k * G + g) * NBT + quarter * NB) * 64) + lane) * 16) : kOutOfRange;
+    auto load_b = [&](int k, int part, int g, float4 (&b)[NB]) {
+        const unsigned at = k >= 0 ? (unsigned)((((((k * kParts + part) * G + g) * NBT + quarter * NB) * 64) + lane) * 16) : kOutOfRange;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) b[nb] = buffer_load16(rs_w, at + nb * 64 * 16u);
     };
@@ -245,21 +253,29 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
     if (k_cur >= 0) {
         cnt_cur = __builtin_amdgcn_readfirstlane(s_cnt[k_cur]);
 #pragma unroll
-        for (int g = 0; g < G; ++g) load_b(k_cur, g, b[g]);
-        load_a(row_at(k_cur, cnt_cur, 0), a0);
+        for (int g = 0; g < G; ++g) load_b(k_cur, 0, g, b[g]);
+        load_a(row_at(k_cur, cnt_cur, 0, 0), a0);
     }
-    int k_nxt = -1, cnt_nxt = 0, nblk = 0, blk = 0;
+    // an offset's blocks are walked once for each part of the channels
+    int k_nxt = -1, cnt_nxt = 0, nblk = 0, blk = 0, part_cur = 0, part_nxt = 0;
     auto begin_offset = [&]() {
+        nblk = (cnt_cur + 15) >> 4;
+        blk = 0;
+        if (kParts > 1 && part_cur + 1 < kParts) {
+            k_nxt = k_cur;
+            cnt_nxt = cnt_cur;
+            part_nxt = part_cur + 1;
+            return;
+        }
+        part_nxt = 0;
         k_nxt = my_mask ? __ffs(my_mask) - 1 : -1;
         my_mask &= my_mask - 1;
         cnt_nxt = k_nxt >= 0 ? __builtin_amdgcn_readfirstlane(s_cnt[k_nxt]) : 0;  // wave-uniform
-        nblk = (cnt_cur + 15) >> 4;
-        blk = 0;
     };
     auto item = [&](float4 (&a_use)[G], float4 (&a_fill)[G]) {
         const bool last = blk + 1 == nblk;  // wave-uniform
         // the next block's rows: of this offset, or the first block of the next one (cnt_nxt = 0: none)
-        load_a(last ? row_at(k_nxt >= 0 ? k_nxt : 0, cnt_nxt, 0) : row_at(k_cur, cnt_cur, blk + 1), a_fill);
+        load_a(last ? row_at(k_nxt >= 0 ? k_nxt : 0, cnt_nxt, 0, part_nxt) : row_at(k_cur, cnt_cur, blk + 1, part_cur), a_fill);
         v4f acc[NB];
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) acc[nb] = (v4f){0.f, 0.f, 0.f, 0.f};
@@ -269,7 +285,7 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) mma16(b[g][nb], x, acc[nb]);
             // behind the offset's last block the next offset's chunk g replaces this one
-            if (last) load_b(k_nxt, g, b[g]);
+            if (last) load_b(k_nxt, part_nxt, g, b[g]);
         }
         const int j = blk * 16 + i;
         if (j < cnt_cur) {
@@ -287,6 +303,7 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
         if (last) {
             k_cur = k_nxt;
             cnt_cur = cnt_nxt;
+            part_cur = part_nxt;
             if (k_cur >= 0) begin_offset();
         } else {
             ++blk;
@@ -358,12 +375,12 @@ int launch(const GemmArgs& a, hipStream_t stream) {
     // operands are addressed with 32-bit byte offsets, 2^31 means "out of range"
     if ((size_t)a.max_voxels * CIN * sizeof(float) >= kOutOfRange || (size_t)a.K * CIN * COUT * sizeof(float) >= kOutOfRange)
         return SESSD_E_UNSUPPORTED;
-    const int num_cu = gemm_compute_units();
-    const unsigned blocks = (unsigned)num_cu;
+    const int units = gemm_compute_units() / (COUT / 64);
+    const unsigned blocks = (unsigned)(units * (COUT / 64));
     auto go = [&](auto dense, auto pad) {
         hipLaunchKernelGGL((conv_wide<CIN, COUT, decltype(dense)::value, decltype(pad)::value>), dim3(blocks), dim3(kWaves * 64), 0, stream,
                            static_cast<const float*>(a.in_feat), static_cast<float*>(a.out_feat), a.w_packed, a.nbr,
-                           a.num_out, a.max_voxels, a.K, a.scale, a.shift, a.relu, num_cu, a.tiles, a.dense);
+                           a.num_out, a.max_voxels, a.K, a.scale, a.shift, a.relu, units, a.tiles, a.dense);
     };
     if (a.dense.dense) a.write_pad_rows ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
     else a.write_pad_rows ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
@@ -375,7 +392,7 @@ int launch(const GemmArgs& a, hipStream_t stream) {
 
 bool gemm_runs_wide(int K, int cin, int cout, int in_type, int out_type) {
     if (in_type != SESSD_FLOAT || out_type != SESSD_FLOAT || K > kMaxK) return false;
-    return cout == 64 && (cin == 64 || cin == 32);
+    return cout == 64 ? cin == 64 || cin == 32 : cout == 128 && (cin == 64 || cin == 128);
 }
 
 int gemm_wide_tile_rows() { return kTileRows; }
@@ -385,6 +402,8 @@ int launch_wide(const GemmArgs& a, hipStream_t stream) {
     if ((reinterpret_cast<uintptr_t>(a.in_feat) | reinterpret_cast<uintptr_t>(a.out_feat)) & 15) return SESSD_E_UNSUPPORTED;
     if (a.cin == 64 && a.cout == 64) return launch<64, 64>(a, stream);
     if (a.cin == 32 && a.cout == 64) return launch<32, 64>(a, stream);
+    if (a.cin == 64 && a.cout == 128) return launch<64, 128>(a, stream);
+    if (a.cin == 128 && a.cout == 128) return launch<128, 128>(a, stream);
     return SESSD_E_UNSUPPORTED;
 }
 

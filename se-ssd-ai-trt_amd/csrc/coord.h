@@ -219,7 +219,7 @@ struct CutPart {
 // the weight arrays inside a rulebook's tile region (tile_cut_bytes())
 int32_t* tile_weight_array(void* region, int max_voxels);
 int32_t* tile_weight_sums(void* region, int max_voxels);
-CutPart make_cut_part(const int32_t* num_out, int K, int max_voxels, int target_rows, int row_weight, bool wide, void* region);
+CutPart make_cut_part(const int32_t* num_out, int K, int max_voxels, int target_rows, int row_weight, int wide, void* region);
 
 // A dense table that stays from frame to frame: emptied row by row instead of by a fill of its whole volume.
 struct CleanPart {

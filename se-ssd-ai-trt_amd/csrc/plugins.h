@@ -120,8 +120,9 @@ class ConvPluginBase {
     int tileRows() const;
     // weight of a row beside its pairs in those cuts
     int tileRowWeight() const;
-    // whether they are cut for the one-tile-per-unit kernel (wide_log2_split())
-    bool tilesWide() const;
+    // compute units that share a tile of the one-tile-per-unit kernel (conv_wide.hip), each 64 of the columns, where
+    // they are cut for that kernel; 0 = they are not
+    int tilesWide() const;
     int exportRulebook(const int32_t* nbr, const int32_t* num_out, void* scratch,
                        int32_t* indice_pairs, uint32_t* indice_num, hipStream_t stream) const;
     int freeDevice();

@@ -31,12 +31,12 @@ size_t tile_cut_bytes(int max_voxels) {
 int32_t* tile_weight_array(void* region, int max_voxels) { return static_cast<int32_t*>(region) + 4 + max_tiles(max_voxels) + 1; }
 int32_t* tile_weight_sums(void* region, int max_voxels) { return tile_weight_array(region, max_voxels) + max_voxels; }
 
-CutPart make_cut_part(const int32_t* num_out, int K, int max_voxels, int target_rows, int row_weight, bool wide, void* region) {
+CutPart make_cut_part(const int32_t* num_out, int K, int max_voxels, int target_rows, int row_weight, int wide, void* region) {
     CutPart c;
     c.num = num_out;
     c.max_voxels = max_voxels;
     c.K = K;
-    c.num_cu = gemm_compute_units();
+    c.num_cu = gemm_compute_units() / (wide ? wide : 1);
     c.target = target_rows;  // (>= kGemmMinTileRows: the cut table has room for the tiles of any row count)
     c.row_weight = row_weight;
     c.wide = wide ? 1 : 0;

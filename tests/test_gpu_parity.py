@@ -837,3 +837,28 @@ def test_every_row_is_a_pad_row(cin, cout, half):
         want = np.maximum(sh, 0).astype(np.float16 if half else np.float32)
         assert np.array_equal(to_np(y), np.broadcast_to(want, (mv, cout))), mv
         conv.close()
+
+
+@pytest.mark.parametrize("cin", [64, 128])
+@pytest.mark.parametrize("n", [1, 65, 97, 1536, 1537, 5120, 5121, 12289, 20000])
+def test_wide_fp32_kernel_with_128_columns(n, cin):
+    """128 output columns: two workgroups take 64 columns each of every tile (128 tiles a round on 256 compute units, of
+    up to 96 rows), up to 5 120 rows four, up to 1 536 rows eight; 128 input channels are walked in two parts.  Against
+    the oracle (pad rows included)."""
+    rng = np.random.default_rng(n + cin)
+    grid, mv = ((5, 40, 40) if n < 1000 else (21, 400, 352)), n + 39
+    coors = F.clustered_active_voxels(n, grid, n, n_blobs=max(4, n // 100))
+    feat = rng.uniform(-1, 1, (n, cin)).astype(np.float32)
+    w = rng.normal(0, 0.1, (27, cin, 128)).astype(np.float32)
+    sc, sh = rng.uniform(0.5, 1.5, 128).astype(np.float32), rng.uniform(-0.2, 0.2, 128).astype(np.float32)
+    conv, out, pairs, num, cbuf = run_subm(coors, n, feat, w, grid, mv, sc, sh, True)
+    O.set_threads(16)
+    try:
+        o_pairs, o_num, _ = O.subm_rulebook(coors, n, grid[::-1], mv)
+        o_out = O.scale_shift_relu(O.gather_gemm_scatter(feat, w, o_pairs, o_num, mv), mv, sc, sh, True)
+    finally:
+        O.set_threads(1)
+    assert np.array_equal(num, o_num)
+    assert_features_close(out, o_out, RTOL_FP32, "wide fp32 %d->128, %d rows" % (cin, n),
+                          abs_sum=abs_sum_of(feat, w, o_pairs, o_num, mv, mv, sc, sh))
+    conv.close()
