@@ -147,6 +147,13 @@ __device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t* lds4) {
 // ---------------------------------------------------------------------------------------------
 // what the passes work on (kernel arguments)
 // ---------------------------------------------------------------------------------------------
+// The cells that a frame's rows have taken in a table that is kept for the next frame: what empties the table goes by
+// this list.  The coors tensor names the same cells, but callers get pointers to it.
+struct CellList {
+    int32_t* num = nullptr;   // null: no list is kept
+    uint32_t* key = nullptr;  // [rows]
+};
+
 struct VgPart {
     const float* points = nullptr;
     const int32_t* points_size = nullptr;
@@ -165,6 +172,7 @@ struct VgPart {
     float* voxels = nullptr;
     int32_t* coors = nullptr;
     int32_t* voxel_num = nullptr;
+    CellList taken;
     int32_t* status = nullptr;  // [0] status, [1] what vg_insert has met (folded into [0] and cleared by vg_finalize)
 };
 
@@ -183,6 +191,7 @@ struct SpPart {
     const int32_t* in_num = nullptr;
     int32_t* out_coors = nullptr;
     int32_t* out_num = nullptr;
+    CellList taken;
     int32_t* nbr = nullptr;   // null: the rulebook is looked up (LookupPart), sp_number has nothing to initialise
     int32_t* meta = nullptr;  // [0] status, [1] output rows, [2] what sp_insert has met (folded into [0] by sp_number)
 };
@@ -221,10 +230,9 @@ int32_t* tile_weight_array(void* region, int max_voxels);
 int32_t* tile_weight_sums(void* region, int max_voxels);
 CutPart make_cut_part(const int32_t* num_out, int K, int max_voxels, int target_rows, int row_weight, int wide, void* region);
 
-// A dense table that stays from frame to frame: emptied row by row instead of by a fill of its whole volume.
+// A dense table that stays from frame to frame: emptied cell by cell instead of by a fill of its whole volume.
 struct CleanPart {
-    const int32_t* coors = nullptr;  // the rows of the frame before
-    const int32_t* num = nullptr;
+    CellList taken;
     int max_voxels = 0;
     CellTable t;
     int blocks = 0;

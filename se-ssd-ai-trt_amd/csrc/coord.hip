@@ -42,12 +42,12 @@ __device__ __forceinline__ uint32_t point_cell(const VgPart& p, float x, float y
     return ((uint32_t)iz * (uint32_t)p.gy + (uint32_t)iy) * (uint32_t)p.gx + (uint32_t)ix;
 }
 
-// cells of a stage's rows of the frame before -> empty
+// cells that rows have taken -> empty
 __device__ __forceinline__ void clean_pass(const CleanPart& P, int block) {
-    const int n = clamp_rows(P.num, P.max_voxels);
+    const int n = clamp_rows(P.taken.num, P.max_voxels);
     for (int row = block * kCoordBlock + (int)threadIdx.x; row < n; row += P.blocks * kCoordBlock) {
-        const int4 c = reinterpret_cast<const int4*>(P.coors)[row];
-        static_cast<uint32_t*>(P.t.base)[((uint32_t)c.y * (uint32_t)P.t.gy + (uint32_t)c.z) * (uint32_t)P.t.gx + (uint32_t)c.w] = kEmpty;
+        const uint32_t key = P.taken.key[row];
+        if (key < P.t.cap) static_cast<uint32_t*>(P.t.base)[key] = kEmpty;
     }
 }
 
@@ -308,6 +308,7 @@ __global__ void __launch_bounds__(kCoordBlock) vg_finalize(VgPart p, SpPart next
     const int rows = (int)(total > (uint32_t)p.max_voxels ? (uint32_t)p.max_voxels : total);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         *p.voxel_num = rows;
+        if (p.taken.num) *p.taken.num = rows;
         p.status[0] = p.status[1] | (total > (uint32_t)p.max_voxels ? SESSD_STATUS_VOXEL_OVERFLOW : 0);
         p.status[1] = 0;
     }
@@ -329,7 +330,8 @@ __global__ void __launch_bounds__(kCoordBlock) vg_finalize(VgPart p, SpPart next
         if (threadIdx.x == 0) s_m = here < room ? here : room;
         if (kept) {
             int ix, iy, iz;
-            (void)point_cell(p, x, y, z, ix, iy, iz);
+            const uint32_t key = point_cell(p, x, y, z, ix, iy, iz);
+            if (p.taken.num) p.taken.key[vid] = key;
             reinterpret_cast<int4*>(p.coors)[vid] = make_int4(0, iz, iy, ix);  // voxelGenerator.cu:404-405
             s_rows[rank] = make_int4((int)vid, iz, iy, ix);
         }
@@ -588,6 +590,7 @@ __device__ __forceinline__ void sp_number_pass(const SpPart& P, const SpPart& ne
         n_out = (int)(total > (uint32_t)P.max_voxels ? (uint32_t)P.max_voxels : total);
         if (c == 0 && threadIdx.x == 0) {
             *P.out_num = n_out;
+            if (P.taken.num) *P.taken.num = n_out;
             P.meta[1] = n_out;
             // (the reference overflows its buffers; here the site is dropped)
             P.meta[0] = P.meta[2] | (total > (uint32_t)P.max_voxels ? SESSD_STATUS_VOXEL_OVERFLOW : 0);
@@ -610,6 +613,7 @@ __device__ __forceinline__ void sp_number_pass(const SpPart& P, const SpPart& ne
                 const int rem = key - z * plane;
                 const int y = rem / P.os[2], x = rem - y * P.os[2];
                 reinterpret_cast<int4*>(P.out_coors)[id] = make_int4(0, z, y, x);  // sparseConv3dlayer.cu:438-441
+                if (P.taken.num) P.taken.key[id] = key;
                 s_rows[rank] = make_int4((int)id, z, y, x);
                 // where sp_scatter fills the table in, the new row's entries start empty: clearing them here, row by
                 // row, touches only the rows that exist

@@ -37,6 +37,45 @@ struct DeviceBuffer {
     }
 };
 
+// A cell table that stays from frame to frame: a word per cell of the grid and, behind it, the list of the cells that
+// the rows of the last frame have taken.  Nothing of it is handed out.
+struct KeptTable {
+    DeviceBuffer mem;
+    uint32_t cells = 0;  // 0: none
+    int alloc(uint64_t volume, int rows) {
+        SESSD_TRY(mem.alloc(listAt(volume) + kWorkspaceAlign + (size_t)rows * sizeof(uint32_t)));
+        cells = (uint32_t)volume;
+        return SESSD_OK;
+    }
+    static size_t listAt(uint64_t volume) { return align_up(volume * sizeof(uint32_t)); }
+    CellList taken() const {
+        CellList l;
+        if (!cells) return l;
+        uint8_t* p = static_cast<uint8_t*>(mem.p) + listAt(cells);
+        l.num = reinterpret_cast<int32_t*>(p);
+        l.key = reinterpret_cast<uint32_t*>(p + kWorkspaceAlign);
+        return l;
+    }
+    void replace(CellTable& t) const {  // t: the table of the workspace, for the same grid
+        if (!cells) return;
+        t.base = mem.p;
+        t.cap = cells;
+        t.dense = 1;
+    }
+    CleanPart clean(const CellTable& t, int max_rows) const {
+        CleanPart c;
+        c.taken = taken();
+        c.max_voxels = max_rows;
+        c.t = t;
+        return c;
+    }
+    void collectFill(FillArgs& f) const {
+        if (!cells) return;
+        f.add(mem.p, cells, kEmpty);
+        f.add(taken().num, 1, 0);
+    }
+};
+
 }  // namespace
 
 struct ConvStage {
@@ -44,9 +83,9 @@ struct ConvStage {
     std::unique_ptr<SubmConv3dLayerPlugin> subm;
     std::unique_ptr<SparseConv3dLayerPlugin> sparse;
     DeviceBuffer ws, feat, coors, num;  // coors/num only for sparse layers (they produce new ones)
-    // Sparse layers: output cell -> row, one word per cell of the output grid (47 MB for 21 x 800 x 704), kept from
-    // frame to frame and emptied row by row; empty where the grid is too large for that (the workspace's table then)
-    DeviceBuffer cells;
+    // Sparse layers: output cell -> row (47 MB for 21 x 800 x 704); none where the grid is too large for that (the
+    // workspace's table then)
+    KeptTable cells;
     int rulebook_from = -1;             // SubM layer whose workspace holds this layer's rulebook
     sessd_tensor_desc in_desc[3], out_desc[3];
     void* coors_ptr = nullptr;  // coordinates valid AFTER this layer
@@ -76,7 +115,7 @@ struct Pipeline {
     std::unique_ptr<Sparse2DensePlugin> s2d;
     std::vector<std::unique_ptr<ConvStage>> stages;
     DeviceBuffer vg_ws, vg_voxels, vg_coors, vg_num, s2d_ws;
-    DeviceBuffer vg_cells;  // the voxelizer's cell table, one word per cell (369 MB for 40 x 1600 x 1408), as ConvStage::cells
+    KeptTable vg_cells;  // the voxelizer's cell table (369 MB for 40 x 1600 x 1408), as ConvStage::cells
     sessd_tensor_desc vg_in[2], vg_out[3], s2d_in[3], s2d_out[1];
     int max_voxels = 0;
     size_t device_bytes = 0;
@@ -99,7 +138,7 @@ struct Pipeline {
     std::vector<hipEvent_t> ev_pass;
     // The voxelizer's cell table is empty at the start of a frame: a pass behind its last reader empties it for the next
     // one (a clear at the head of a frame was 4-6 us of every frame).  The strided layers' dense tables hold the rows
-    // of the frame before, as their coors tensors do.  create() clears all of them, and so does a frame that has run
+    // of the frame before, which their lists name.  create() clears all of them, and so does a frame that has run
     // plugin by plugin (behind its end): a frame that a caller has captured holds no clear of its own.  False: a frame
     // did not get to its end, clear them first.
     bool tables_ready = false;
@@ -133,33 +172,24 @@ struct Pipeline {
 
     CellTable cellTable(const ConvStage& st) const {
         CellTable t = st.sparse->cellTable(st.ws.p);
-        if (st.cells.p) {
-            t.base = st.cells.p;
-            t.cap = (uint32_t)(st.cells.bytes / sizeof(uint32_t));
-            t.dense = 1;
-        }
+        st.cells.replace(t);
         return t;
     }
     CellTable voxelTable() const {
         CellTable t = vg->cellTable(vg_ws.p, desc.max_points);
-        if (vg_cells.p) {
-            t.base = vg_cells.p;
-            t.cap = (uint32_t)(vg_cells.bytes / sizeof(uint32_t));
-            t.dense = 1;
-        }
+        vg_cells.replace(t);
         return t;
     }
     int clearTables(hipStream_t stream) {
         FillArgs f;
         vg->collectTableFill(vg_ws.p, desc.max_points, false, f);
-        if (vg_cells.p) f.add(vg_cells.p, vg_cells.bytes / sizeof(uint32_t), kEmpty);
+        vg_cells.collectFill(f);
         for (auto& st : stages) {
-            if (!st->sparse || !st->cells.p) continue;
             if (f.n + 2 > FillArgs::kMaxRegions) {
                 SESSD_TRY(launch_fill(f, stream));
                 f = FillArgs();
             }
-            f.add(st->cells.p, st->cells.bytes / sizeof(uint32_t), kEmpty);
+            st->cells.collectFill(f);
         }
         return launch_fill(f, stream);
     }
@@ -226,20 +256,16 @@ struct Pipeline {
             part[(size_t)i] = st.sparse->part(rows[(size_t)i - 1].coors, rows[(size_t)i - 1].num, static_cast<int32_t*>(st.coors.p),
                                               static_cast<int32_t*>(st.num.p), st.ws.p, false);
             part[(size_t)i].t = rows[(size_t)i].table;
+            part[(size_t)i].taken = st.cells.taken();
             for (FillArgs* f : {&clears, &pads})
                 if (f->n + 6 > FillArgs::kMaxRegions) {
                     overflow.push_back(*f);
                     *f = FillArgs();
                 }
-            if (st.cells.p && cleans.size() < (size_t)kMaxCleans) {
-                CleanPart c;
-                c.coors = rows[(size_t)i].coors;
-                c.num = rows[(size_t)i].num;
-                c.max_voxels = V;
-                c.t = rows[(size_t)i].table;
-                cleans.push_back(c);
-            } else if (st.cells.p) {
-                clears.add(st.cells.p, st.cells.bytes / sizeof(uint32_t), kEmpty);
+            if (st.cells.cells && cleans.size() < (size_t)kMaxCleans) {
+                cleans.push_back(st.cells.clean(rows[(size_t)i].table, V));
+            } else if (st.cells.cells) {
+                st.cells.collectFill(clears);
             } else {
                 st.sparse->collectTableFill(st.ws.p, clears);
             }
@@ -252,6 +278,7 @@ struct Pipeline {
                                   desc.point_features, static_cast<float*>(vg_voxels.p), static_cast<int32_t*>(vg_coors.p),
                                   static_cast<int32_t*>(vg_num.p), vg_ws.p);
         v.t = rows[0].table;
+        v.taken = vg_cells.taken();
         SESSD_TRY(launch_vg_insert(v, cleans.data(), (int)cleans.size(), clears, stream));
         for (const FillArgs& f : overflow) SESSD_TRY(launch_fill(f, stream));
         SESSD_TRY(launch_vg_flags(v, pads, stream));
@@ -309,11 +336,8 @@ struct Pipeline {
             // numbering of the next strided layer's rows (their tickets for the layer behind it), tile cuts
             FillArgs clear;
             CleanPart clean;
-            if (i == clean_at && vg_cells.p) {
-                clean.coors = rows[0].coors;
-                clean.num = rows[0].num;
-                clean.max_voxels = desc.voxelgen.max_voxels;
-                clean.t = rows[0].table;
+            if (i == clean_at && vg_cells.cells) {
+                clean = vg_cells.clean(rows[0].table, desc.voxelgen.max_voxels);
             } else if (i == clean_at) {
                 vg->collectTableFill(vg_ws.p, desc.max_points, true, clear);
             }
@@ -322,7 +346,7 @@ struct Pipeline {
             bool did = false;
             while (at < cuts.size() || (!did && (next || i == clean_at))) {
                 const size_t n = cuts.size() - at < (size_t)kMaxCuts ? cuts.size() - at : (size_t)kMaxCuts;
-                SESSD_TRY(launch_number(did ? nullptr : next, did ? nullptr : after, cuts.data() + at, (int)n, did || !clean.coors ? nullptr : &clean,
+                SESSD_TRY(launch_number(did ? nullptr : next, did ? nullptr : after, cuts.data() + at, (int)n, did || !clean.taken.num ? nullptr : &clean,
                                         did ? nullptr : &clear, side));
                 at += n;
                 did = true;
@@ -441,8 +465,8 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
     SESSD_TRY(P->vg_coors.alloc((size_t)V * 4 * sizeof(int32_t)));
     SESSD_TRY(P->vg_num.alloc(256));
     const uint64_t cells = (uint64_t)vg->grid_x_size_ * (uint64_t)vg->grid_y_size_ * (uint64_t)vg->grid_z_size_;
-    if (cells <= kDenseVoxelCells) SESSD_TRY(P->vg_cells.alloc(cells * sizeof(uint32_t)));
-    total += P->vg_ws.bytes + P->vg_voxels.bytes + P->vg_coors.bytes + P->vg_cells.bytes + 256;
+    if (cells <= kDenseVoxelCells) SESSD_TRY(P->vg_cells.alloc(cells, VG));
+    total += P->vg_ws.bytes + P->vg_voxels.bytes + P->vg_coors.bytes + P->vg_cells.mem.bytes + 256;
 
     int in_type = SESSD_FLOAT;  // the voxelizer's means are FP32
     int in_ch = 4;
@@ -511,7 +535,7 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
             SESSD_TRY(st->coors.alloc((size_t)V * 4 * sizeof(int32_t)));
             SESSD_TRY(st->num.alloc(256));
             const uint64_t volume = (uint64_t)s.out_shape[0] * (uint64_t)s.out_shape[1] * (uint64_t)s.out_shape[2];
-            if (volume <= kDenseCells) SESSD_TRY(st->cells.alloc(volume * sizeof(uint32_t)));
+            if (volume <= kDenseCells) SESSD_TRY(st->cells.alloc(volume, V));
             last_subm_with_rulebook = -1;  // new coordinates: earlier rulebooks no longer apply
         } else {
             return fail(SESSD_E_INVALID, "pipeline: layer %d has unknown type %d", l, s.type);
@@ -519,7 +543,7 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
         base->flags_ = d.flags;
         SESSD_TRY(base->setEpilogue(d.scale ? d.scale[l] : nullptr, d.shift ? d.shift[l] : nullptr, d.relu));
         SESSD_TRY(st->feat.alloc((size_t)V * s.out_channel * dtype_size(ft)));
-        total += st->ws.bytes + st->feat.bytes + st->coors.bytes + st->num.bytes + st->cells.bytes;
+        total += st->ws.bytes + st->feat.bytes + st->coors.bytes + st->num.bytes + st->cells.mem.bytes;
         in_type = ft;
         in_ch = s.out_channel;
         P->stages.push_back(std::move(st));
@@ -552,7 +576,7 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
         FillArgs f;
         f.add(static_cast<uint8_t*>(P->vg_ws.p) + vg->statusOffset(d.max_points), 4, 0);
         for (auto& st : P->stages) {
-            if (st->num.p) f.add(st->num.p, 4, 0);  // (no rows of a frame before)
+            if (st->num.p) f.add(st->num.p, 4, 0);  // (queries before the first frame find no rows)
             if (!st->ws.p) continue;
             if (f.n + 3 > FillArgs::kMaxRegions) {
                 SESSD_TRY(launch_fill(f, nullptr));

@@ -515,3 +515,42 @@ def test_dozens_of_strided_layers():
         assert pipe.status() == ref["status"] == 0
         assert [pipe.layer_count(l) for l in range(-1, len(layers))] == list(ref["counts"])
         assert np.array_equal(pipe.read_layer(len(layers) - 1)[1], ref["coors"])
+
+
+class _Words:
+    """`n` 32-bit words of device memory that the library owns, for torch.as_tensor."""
+
+    def __init__(self, ptr, n):
+        self.__cuda_array_interface__ = dict(shape=(n,), typestr="<i4", data=(ptr, False), version=2)
+
+
+@pytest.mark.parametrize("coordinate,count", [(0, None), (3, 0), (1 << 30, 1 << 30), (-1, -1)])
+def test_writing_to_a_layers_tensors_after_a_frame_leaves_the_next_one_alone(coordinate, count):
+    """sessd_pipeline_layer_io hands out the tensors of a finished frame.  What a caller does to them must not reach the
+    next frame: the cells that the kept tables are emptied by are listed in memory of the pipeline's own."""
+    layers = B.reference_layers()
+    W = B.random_weights(layers, seed=14, w_std=0.05)
+    mp, mv = 1024, 20000
+    overlap = coordinate >= 0
+    pipe = api.Pipeline(layers, W, mp, mv, share_rulebooks=True, skip_pad_rows=True, use_graph=overlap, overlap_streams=overlap)
+    p, n = points_input(np.zeros((0, 4), np.float32), mp)
+    dense, stream = pipe.new_dense(), torch.cuda.Stream()
+    for step, npts in enumerate((900, 1000, 300)):
+        pts = F.lidar_frame(npts, 110 + step)
+        hp, hn = points_input(pts, mp)
+        with torch.cuda.stream(stream):
+            p.copy_(hp)
+            n.copy_(hn)
+            pipe.enqueue(p, n, dense, stream)
+        stream.synchronize()
+        ref = O.frame(pts, B.voxelgen_desc(max_voxels=mv), layers, W, B.dense_desc())
+        assert pipe.status() == ref["status"] == 0
+        assert [pipe.layer_count(l) for l in range(-1, len(layers))] == list(ref["counts"]), step
+        assert np.array_equal(pipe.read_layer(len(layers) - 1)[1], ref["coors"]), step
+        assert_end_to_end_close(to_np(dense), ref["dense"], False, "dense, step %d" % step)
+        for l in range(-1, len(layers)):
+            _, coors, num, _, _ = pipe.layer_io(l)
+            torch.as_tensor(_Words(coors, mv * 4), device="cuda:0").fill_(coordinate)
+            if count is not None:
+                torch.as_tensor(_Words(num, 1), device="cuda:0").fill_(count)
+        torch.cuda.synchronize()
