@@ -445,7 +445,11 @@ int sessd_load_frame(const char* path, float* points, int32_t max_points, int32_
 int sessd_pipeline_create_from_wts(const sessd_pipeline_desc* desc, const sessd_wts* wts,
                                    const char* prefix, const int32_t* conv_index, float eps,
                                    sessd_pipeline** out);
-/* points f32[max_points,point_features], points_size i32[1], dense [C*D,H,W]: device pointers */
+/* points f32[max_points,point_features], points_size i32[1], dense [C*D,H,W]: device pointers.
+ * The pipeline keeps tables on the device from frame to frame.  A call that fails clears them on `stream`, behind what it
+ * has launched: order the next frame behind it as behind any other, also one in a graph of your own that was captured
+ * from an earlier enqueue.  Should that clear fail as well, the next enqueue begins with it; replay no such graph before
+ * an enqueue has succeeded. */
 int sessd_pipeline_enqueue(sessd_pipeline* h, const void* points, const void* points_size,
                            void* dense, sessd_stream_t stream);
 /* The two halves of sessd_pipeline_enqueue, for hosts that keep several frames in flight (frames_in_flight

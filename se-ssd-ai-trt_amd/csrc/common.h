@@ -26,9 +26,11 @@ int fail(int code, const char* fmt, ...);
 #define SESSD_HIP_TRY(expr)                                                                      \
     do {                                                                                         \
         hipError_t e__ = (expr);                                                                 \
-        if (e__ != hipSuccess)                                                                   \
+        if (e__ != hipSuccess) {                                                                 \
+            (void)hipGetLastError(); /* reported here, not once more by the next launch */       \
             return ::sessd::fail(SESSD_E_HIP, "%s:%d: %s -> %s", __FILE__, __LINE__, #expr,      \
                                  hipGetErrorString(e__));                                        \
+        }                                                                                        \
     } while (0)
 
 // The body of an extern "C" entry point that can allocate on the host (new, std::vector, std::string): no C++

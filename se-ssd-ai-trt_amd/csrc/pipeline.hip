@@ -139,8 +139,8 @@ struct Pipeline {
     // The voxelizer's cell table is empty at the start of a frame: a pass behind its last reader empties it for the next
     // one (a clear at the head of a frame was 4-6 us of every frame).  The strided layers' dense tables hold the rows
     // of the frame before, which their lists name.  create() clears all of them, and so does a frame that has run
-    // plugin by plugin (behind its end): a frame that a caller has captured holds no clear of its own.  False: a frame
-    // did not get to its end, clear them first.
+    // plugin by plugin (behind its end) and a call that has failed (recover()): a frame that a caller has captured holds
+    // no clear of its own.  False: that clear failed as well, the next frame begins with it.
     bool tables_ready = false;
 
     // profiling: one event per segment boundary (see sessd_pipeline_enqueue_timed)
@@ -194,6 +194,54 @@ struct Pipeline {
         return launch_fill(f, stream);
     }
 
+    // everything that a frame has to find as the one before leaves it, as for the first frame
+    int resetState(hipStream_t stream) {
+        FillArgs f;
+        f.add(static_cast<uint8_t*>(vg_ws.p) + vg->statusOffset(desc.max_points), 4, 0);
+        for (auto& st : stages) {
+            if (!st->ws.p) continue;
+            if (f.n + 2 > FillArgs::kMaxRegions) {
+                SESSD_TRY(launch_fill(f, stream));
+                f = FillArgs();
+            }
+            if (st->subm) st->subm->collectHeaderFill(st->ws.p, f);
+            else st->sparse->collectHeaderFill(st->ws.p, f);
+        }
+        SESSD_TRY(launch_fill(f, stream));
+        SESSD_TRY(clearTables(stream));
+        tables_ready = true;
+        return SESSD_OK;
+    }
+    static hipStreamCaptureStatus captureStatus(hipStream_t s) {
+        hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &c) == hipSuccess) return c;
+        (void)hipGetLastError();
+        return hipStreamCaptureStatusNone;
+    }
+    int joinAux(hipStream_t stream) {
+        if (!aux) return SESSD_OK;
+        SESSD_HIP_TRY(hipEventRecord(ev_head, aux));
+        SESSD_HIP_TRY(hipStreamWaitEvent(stream, ev_head, 0));
+        return SESSD_OK;
+    }
+    // Behind a call that failed with `rc`, which is returned.  Its launches may have left cells in the tables, and a graph
+    // that the caller captured from an earlier frame does not clear them: the clear goes to `stream` right here, behind
+    // what the call has launched on either stream.  Where `stream` is being captured nothing has run; only `aux` has to
+    // come back to it, so that the capture can be ended.
+    int recover(hipStream_t stream, int rc) {
+        char why[512];
+        snprintf(why, sizeof(why), "%s", sessd_last_error());
+        (void)hipGetLastError();  // (reported already; the launches below ask for theirs)
+        if (captureStatus(stream) != hipStreamCaptureStatusNone) {
+            if (aux && captureStatus(aux) == hipStreamCaptureStatusActive) (void)joinAux(stream);
+        } else {
+            tables_ready = false;
+            if (joinAux(stream) == SESSD_OK) (void)resetState(stream);
+        }
+        (void)hipGetLastError();
+        return fail(rc, "%s", why);
+    }
+
     // The rows of stage 0 are the voxels, those of stage i the output rows of the i-th strided layer.
     struct Stage {
         int layer = -1;            // the strided layer that makes the rows (-1: the voxelizer)
@@ -229,7 +277,6 @@ struct Pipeline {
     // runs there and the GEMM chain waits per layer for the pass its rulebook comes from, so that the passes of later
     // layers overlap the GEMMs of earlier ones; under stream capture that becomes two branches of the graph.
     int enqueueFrame(const void* points, const void* points_size, void* dense, hipStream_t stream) {
-        tables_ready = false;  // (until the pass that cleans it is enqueued)
         const std::vector<Stage> cs = coordStages();
         const int m = (int)cs.size() - 1;  // strided layers
         const int V = max_voxels;
@@ -351,7 +398,6 @@ struct Pipeline {
                 at += n;
                 did = true;
             }
-            if (i == clean_at) tables_ready = true;
             for (int l : sg.builds) {
                 ConvStage& st = *stages[(size_t)l];
                 SESSD_TRY(st.subm->enqueueBuild(rows[(size_t)i].coors, rows[(size_t)i].num, st.ws.p, side));
@@ -572,24 +618,18 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
         for (auto& e : P->ev_pass) SESSD_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
     // what the passes leave as they need it for the next frame has to be right for the first
-    {
-        FillArgs f;
-        f.add(static_cast<uint8_t*>(P->vg_ws.p) + vg->statusOffset(d.max_points), 4, 0);
-        for (auto& st : P->stages) {
-            if (st->num.p) f.add(st->num.p, 4, 0);  // (queries before the first frame find no rows)
-            if (!st->ws.p) continue;
-            if (f.n + 3 > FillArgs::kMaxRegions) {
-                SESSD_TRY(launch_fill(f, nullptr));
-                f = FillArgs();
-            }
-            if (st->subm) st->subm->collectHeaderFill(st->ws.p, f);
-            else st->sparse->collectHeaderFill(st->ws.p, f);
+    SESSD_TRY(P->resetState(nullptr));
+    FillArgs counts;  // queries before the first frame find no rows
+    counts.add(P->vg_num.p, 4, 0);
+    for (auto& st : P->stages) {
+        if (counts.full()) {
+            SESSD_TRY(launch_fill(counts, nullptr));
+            counts = FillArgs();
         }
-        SESSD_TRY(launch_fill(f, nullptr));
-        SESSD_TRY(P->clearTables(nullptr));
-        SESSD_HIP_TRY(hipStreamSynchronize(nullptr));
-        P->tables_ready = true;
+        counts.add(st->num.p, 4, 0);
     }
+    SESSD_TRY(launch_fill(counts, nullptr));
+    SESSD_HIP_TRY(hipStreamSynchronize(nullptr));
     // the layer array of the caller need not outlive create()
     P->desc.layers = nullptr;
     P->desc.weights = P->desc.scale = P->desc.shift = nullptr;
@@ -686,23 +726,25 @@ static Pipeline* current(sessd_pipeline* h) {
 // one frame on `stream`: a replay of the captured graph when the pipeline uses graphs (re-captured when a pointer
 // changed), direct launches otherwise
 static int run_frame(Pipeline* P, const void* points, const void* points_size, void* dense, hipStream_t stream) {
-    auto run = [&](hipStream_t st) { return P->enqueueFrame(points, points_size, dense, st); };
+    auto run = [&]() -> int {
+        const int rc = P->enqueueFrame(points, points_size, dense, stream);
+        return rc == SESSD_OK ? rc : P->recover(stream, rc);
+    };
     if (!P->tables_ready) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        SESSD_HIP_TRY(hipStreamIsCapturing(stream, &capture));
-        SESSD_TRY(P->clearTables(stream));
-        if (capture != hipStreamCaptureStatusNone) {  // the caller's own graph: nothing is cleared until it is launched
-            const int rc = run(stream);
+        const bool captured = P->captureStatus(stream) != hipStreamCaptureStatusNone;
+        if (!captured) SESSD_TRY(P->joinAux(stream));
+        SESSD_TRY(P->resetState(stream));
+        if (captured) {  // the caller's own graph: nothing is cleared until it is launched
             P->tables_ready = false;
-            return rc;
+            return run();
         }
     }
-    if (!P->desc.use_graph || stream == nullptr) return run(stream);
+    if (!P->desc.use_graph || stream == nullptr) return run();
     CapturedGraph& g = P->captured;
     if (!g.exec || g.points != points || g.size != points_size || g.dense != dense) {
         g.reset();
         SESSD_HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-        const int rc = run(stream);
+        const int rc = run();
         hipGraph_t captured = nullptr;
         const hipError_t e = hipStreamEndCapture(stream, &captured);
         if (rc != SESSD_OK) {
@@ -718,8 +760,9 @@ static int run_frame(Pipeline* P, const void* points, const void* points_size, v
         g.size = points_size;
         g.dense = dense;
     }
-    SESSD_HIP_TRY(hipGraphLaunch(g.exec, stream));
-    return SESSD_OK;
+    const hipError_t e = hipGraphLaunch(g.exec, stream);
+    if (e == hipSuccess) return SESSD_OK;
+    return P->recover(stream, fail(SESSD_E_HIP, "pipeline: launching the captured frame failed: %s", hipGetErrorString(e)));
 }
 
 int sessd_pipeline_submit(sessd_pipeline* h, const void* points, const void* points_size, void* dense,
@@ -868,7 +911,6 @@ int sessd_pipeline_enqueue_timed(sessd_pipeline* h, const void* points, const vo
     SESSD_HIP_TRY(hipEventRecord(P->events[n_seg + 2], stream));
     SESSD_HIP_TRY(hipEventRecord(P->events[0], stream));
     int rc;
-    P->tables_ready = false;  // (the plugins leave their tables filled)
     {
         const void* vin[2] = {points, points_size};
         void* vout[3] = {P->vg_voxels.p, P->vg_coors.p, P->vg_num.p};
@@ -882,9 +924,8 @@ int sessd_pipeline_enqueue_timed(sessd_pipeline* h, const void* points, const vo
                                                : static_cast<ConvPluginBase*>(P->stages[l]->sparse.get());
         b->ev_gemm_begin_ = b->ev_gemm_end_ = nullptr;
     }
-    SESSD_TRY(rc);
-    SESSD_TRY(P->clearTables(stream));
-    P->tables_ready = true;
+    if (rc == SESSD_OK) rc = P->clearTables(stream);  // (the plugins leave theirs filled)
+    if (rc != SESSD_OK) return P->recover(stream, rc);
     SESSD_HIP_TRY(hipStreamSynchronize(stream));
     for (int i = 0; i < n_seg; ++i)
         SESSD_HIP_TRY(hipEventElapsedTime(&segment_ms[i], P->events[i], P->events[i + 1]));

@@ -1,0 +1,187 @@
+"""The library on the stand-in runtime of fake_hip.cpp, without torch and without a GPU: run as a program of its own
+(tests/test_host_failures_cpu.py), because one process holds one HIP runtime.
+
+    python tests/host_pipeline.py <path of the stand-in library> <check>
+"""
+import ctypes as C
+import os
+import sys
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, os.path.join(ROOT, "se-ssd-ai-trt_amd"))
+sys.modules["torch"] = None  # (sessd3d.api binds the library to torch's runtime where it finds torch)
+
+import numpy as np  # noqa: E402
+from sessd3d import api, backbone as B, ctypes_defs as D  # noqa: E402
+
+FAKE = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+FAKE.fake_log.restype = C.c_char_p
+FAKE.fake_fail_launches.argtypes = [C.c_long, C.c_long]
+FAKE.fake_largest_allocation.argtypes = [C.c_ulonglong]
+FAKE.fake_fail_new.argtypes = [C.c_long]
+FAKE.fake_news_left.restype = C.c_long
+FAKE.fake_stream_number.argtypes = [C.c_void_p]
+FAKE.hipStreamBeginCapture.argtypes = [C.c_void_p, C.c_int]
+FAKE.hipStreamEndCapture.argtypes = [C.c_void_p, C.POINTER(C.c_void_p)]
+L = api.lib()
+
+POINTS, SIZE, DENSE = 4096, 8192, 12288  # device addresses that nothing reads
+
+
+def new_stream():
+    s = C.c_void_p()
+    assert FAKE.hipStreamCreateWithFlags(C.byref(s), 0) == 0
+    return s
+
+
+def create(layers=None, **options):
+    """-> (rc, handle) of a small pipeline over the reference backbone"""
+    layers = layers or B.reference_layers()
+    W = B.random_weights(layers, seed=1)
+    FP = C.POINTER(C.c_float)
+    arrays = (FP * len(layers))(*[w.ctypes.data_as(FP) for w in W.w])
+    d = D.PipelineDesc()
+    d.voxelgen = B.voxelgen_desc(600)
+    d.layer_max_voxels, d.max_points, d.point_features, d.n_layers = 600, 500, 4, len(layers)
+    d.layers, d.weights = B.layer_specs(layers), arrays
+    d.relu, d.feature_dtype, d.share_rulebooks = 1, D.SESSD_FLOAT, 1
+    d.dense = B.dense_desc(B.DENSE_SIZE_XYZ, layers[-1].cout)
+    for k, v in options.items():
+        setattr(d, k, v)
+    h = C.c_void_p()
+    return L.sessd_pipeline_create(C.byref(d), C.byref(h)), h
+
+
+def enqueue(h, stream):
+    return L.sessd_pipeline_enqueue(h, POINTS, SIZE, DENSE, stream)
+
+
+def timed(h, stream):
+    ms, n = (C.c_float * 64)(), C.c_int()
+    return L.sessd_pipeline_enqueue_timed(h, POINTS, SIZE, DENSE, stream, ms, 64, C.byref(n))
+
+
+def take_log():
+    lines = [l.split() for l in FAKE.fake_log().decode().splitlines()]
+    FAKE.fake_clear_log()
+    return lines
+
+
+def launches(log):
+    return [l for l in log if l[0] in ("launch", "graph")]
+
+
+def is_fill(line):
+    return line[0] == "launch" and "fill_kernel" in line[1]
+
+
+def unordered(log):
+    """Launches that the last launch of the log is not ordered behind."""
+    done, at = {}, {}  # stream -> launches before what comes next on it; event -> launches it stands for
+    last = set()
+    for i, l in enumerate(log):
+        if l[0] in ("launch", "graph"):
+            last = set(done.setdefault(l[-1], set()))
+            done[l[-1]].add(i)
+        elif l[0] == "record":
+            at[l[1]] = set(done.setdefault(l[2], set()))
+        elif l[0] == "wait":
+            done.setdefault(l[1], set()).update(at.get(l[2], ()))
+    every = [i for i, l in enumerate(log) if l[0] in ("launch", "graph")]
+    return [log[i] for i in every[:-1] if i not in last]
+
+
+def check_recovery(overlap, call):
+    """Every launch of a call is made to fail in turn: the call reports it, and its last launches are the clears, on the
+    caller's stream and ordered behind all others.  The next call does not clear again."""
+    rc, h = create(overlap_streams=overlap)
+    assert rc == 0, L.sessd_last_error()
+    stream = new_stream()
+    take_log()
+    assert call(h, stream) == 0
+    n = len(launches(take_log()))
+    assert n > 20
+    fill_ends = is_fill(launches_of(call, h, stream)[-1])
+    for i in range(n):
+        FAKE.fake_fail_launches(i, 1)
+        rc = call(h, stream)
+        log = take_log()
+        assert rc == D.SESSD_E_HIP and b"made to fail" in L.sessd_last_error(), i
+        made = launches(log)
+        assert len(made) > i + 1 and is_fill(made[-1]), (i, made[-1])
+        assert made[-1][-1] == str(FAKE.fake_stream_number(stream)), "the clear is on another stream than the caller's"
+        assert not unordered(log), (i, unordered(log))
+        FAKE.fake_fail_launches(-1, 0)
+        again = launches_of(call, h, stream)
+        assert len(again) == n and is_fill(again[-1]) == fill_ends, i
+
+
+def launches_of(call, h, stream):
+    take_log()
+    assert call(h, stream) == 0
+    return launches(take_log())
+
+
+def check_clear_that_failed_too(overlap):
+    """The clear behind a failed call fails as well: the next frame begins with it."""
+    rc, h = create(overlap_streams=overlap)
+    stream = new_stream()
+    plain = launches_of(enqueue, h, stream)
+    FAKE.fake_fail_launches(4, 1000)
+    assert enqueue(h, stream) != 0
+    FAKE.fake_fail_launches(-1, 0)
+    made = launches_of(enqueue, h, stream)
+    assert is_fill(made[0]) and len(made) > len(plain)
+    assert [l[1] for l in made[-len(plain):]] == [l[1] for l in plain]
+    assert len(launches_of(enqueue, h, stream)) == len(plain)
+
+
+def check_capture(overlap):
+    """A call that fails while the caller captures: nothing has run, so nothing is cleared, and the capture can be ended
+    (no branch of it is left open)."""
+    rc, h = create(overlap_streams=overlap)
+    stream = new_stream()
+    n = len(launches_of(enqueue, h, stream))
+    graph = C.c_void_p()
+    for i in range(n):
+        assert FAKE.hipStreamBeginCapture(stream, 0) == 0
+        FAKE.fake_fail_launches(i, 1)
+        assert enqueue(h, stream) == D.SESSD_E_HIP
+        FAKE.fake_fail_launches(-1, 0)
+        assert len(launches(take_log())) == i + 1, i
+        assert FAKE.hipStreamEndCapture(stream, C.byref(graph)) == 0, i
+        assert len(launches_of(enqueue, h, stream)) == n, i
+
+
+def check_own_graph():
+    """The pipeline's own graph: a capture that fails has run nothing; a graph launch that fails is followed by the clear."""
+    rc, h = create(overlap_streams=1, use_graph=1)
+    stream = new_stream()
+    FAKE.fake_fail_launches(5, 1)
+    assert enqueue(h, stream) == D.SESSD_E_HIP
+    FAKE.fake_fail_launches(-1, 0)
+    assert not any(l[0] == "graph" for l in take_log())
+    assert launches_of(enqueue, h, stream)[-1][0] == "graph"
+    assert [l[0] for l in launches_of(enqueue, h, stream)] == ["graph"]
+    FAKE.fake_fail_launches(0, 1)
+    assert enqueue(h, stream) == D.SESSD_E_HIP
+    FAKE.fake_fail_launches(-1, 0)
+    made = launches(take_log())
+    assert made[0][0] == "graph" and len(made) > 1 and all(is_fill(l) for l in made[1:])
+    assert [l[0] for l in launches_of(enqueue, h, stream)] == ["graph"]
+
+
+CHECKS = {
+    "recovery-direct": lambda: check_recovery(0, enqueue),
+    "recovery-overlap": lambda: check_recovery(1, enqueue),
+    "recovery-timed": lambda: check_recovery(1, timed),
+    "clear-failed-direct": lambda: check_clear_that_failed_too(0),
+    "clear-failed-overlap": lambda: check_clear_that_failed_too(1),
+    "capture-direct": lambda: check_capture(0),
+    "capture-overlap": lambda: check_capture(1),
+    "own-graph": check_own_graph,
+}
+
+if __name__ == "__main__":
+    CHECKS[sys.argv[2]]()
+    print("ok")

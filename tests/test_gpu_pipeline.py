@@ -1,5 +1,7 @@
 """GPU parity of the whole frame pipeline (voxelGenerator -> 14 conv layers with folded BN + ReLU ->
 sparse2Dense) against oracle_frame, plus size-independent properties at the full benchmark size."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -554,3 +556,49 @@ def test_writing_to_a_layers_tensors_after_a_frame_leaves_the_next_one_alone(coo
             if count is not None:
                 torch.as_tensor(_Words(num, 1), device="cuda:0").fill_(count)
         torch.cuda.synchronize()
+
+
+def _leave_an_error_pending():
+    """What a failed HIP call of the application's own leaves behind: the library's next launch check meets it, after the
+    launch itself has gone through."""
+    with open("/proc/self/maps") as f:
+        path = next(l.split()[-1] for l in f if "libamdhip64" in l)
+    assert ctypes.CDLL(path).hipSetDevice(12345) != 0
+
+
+@pytest.mark.parametrize("overlap", [True, False])
+def test_a_frame_in_the_callers_own_graph_survives_a_call_that_failed(overlap):
+    """An enqueue that fails after its first launch leaves the voxelizer's table filled.  The graph that the caller
+    captured before holds no clear; the failed call has to leave the tables as it found them."""
+    layers = B.reference_layers()
+    W = B.random_weights(layers, seed=15, w_std=0.05)
+    mp, mv = 1024, 20000
+    pipe = api.Pipeline(layers, W, mp, mv, share_rulebooks=True, skip_pad_rows=True, overlap_streams=overlap)
+    p, n = points_input(np.zeros((0, 4), np.float32), mp)
+    dense, stream = pipe.new_dense(), torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        pipe.enqueue(p, n, dense, stream)
+    for step, how in enumerate(("graph", "failed", "graph", "graph", "timed, failed", "graph", "direct", "graph")):
+        pts = F.lidar_frame((700, 900, 400, 1000, 800, 300, 600, 500)[step], 130 + step)
+        hp, hn = points_input(pts, mp)
+        with torch.cuda.stream(stream):
+            p.copy_(hp)
+            n.copy_(hn)
+            if "failed" in how:
+                stream.synchronize()
+                _leave_an_error_pending()
+                with pytest.raises(api.SessdError):
+                    (pipe.enqueue_timed if "timed" in how else pipe.enqueue)(p, n, dense, stream)
+            elif how == "graph":
+                graph.replay()
+            else:
+                pipe.enqueue(p, n, dense, stream)
+        stream.synchronize()
+        if "failed" in how:
+            continue
+        ref = O.frame(pts, B.voxelgen_desc(max_voxels=mv), layers, W, B.dense_desc())
+        assert pipe.status() == ref["status"] == 0
+        assert [pipe.layer_count(l) for l in range(-1, len(layers))] == list(ref["counts"]), (step, how)
+        assert np.array_equal(pipe.read_layer(len(layers) - 1)[1], ref["coors"]), (step, how)
+        assert_end_to_end_close(to_np(dense), ref["dense"], False, "dense, step %d" % step)

@@ -1,0 +1,33 @@
+"""What the host side of the library does when a runtime call or an allocation fails.  Nothing runs on a GPU: the library
+is loaded onto a stand-in for the HIP runtime (fake_hip.cpp) in a process of its own (host_pipeline.py)."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def fake_hip(tmp_path_factory):
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    if not shutil.which("g++"):
+        pytest.skip("no C++ compiler")
+    out = str(tmp_path_factory.mktemp("fake_hip") / "libfake_hip.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(rocm, "include"),
+                    os.path.join(HERE, "fake_hip.cpp"), "-o", out], check=True)
+    return out
+
+
+def run_check(fake_hip, check):
+    r = subprocess.run([sys.executable, os.path.join(HERE, "host_pipeline.py"), fake_hip, check], stdout=subprocess.PIPE,
+                       stderr=subprocess.STDOUT, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.rstrip().endswith("ok"), r.stdout[-4000:]
+
+
+@pytest.mark.parametrize("check", ["recovery-direct", "recovery-overlap", "recovery-timed", "clear-failed-direct", "clear-failed-overlap",
+                                   "capture-direct", "capture-overlap", "own-graph"])
+def test_failed_calls_leave_the_cell_tables_empty(fake_hip, check):
+    run_check(fake_hip, check)
