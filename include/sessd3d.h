@@ -129,9 +129,10 @@ int sessd_voxelgen_enqueue(sessd_voxelgen* h, const sessd_tensor_desc* inDesc,
 /* No counterpart in the reference.  For callers that cannot allocate device memory or hand over a
  * workspace (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc):
  * sessd_voxelgen_enqueue without the workspace argument.  The scratch memory is a static device array
- * inside the library, 8 MiB on every GPU the library runs on, held until the process ends; that is
- * enough for the reference's shape (80000-row points tensor, 5 points per voxel: 7.7 MB) and a request
- * that needs more is rejected with SESSD_E_INVALID before anything is launched.  The call allocates and
+ * inside the library, 8 MiB on every GPU the library runs on, held until the process ends.  That is
+ * enough for points tensors of 131072 rows with up to 7 points per voxel (the reference's 80000 rows with 5
+ * take 5.8 MB) and of 262144 rows with one; a request that needs more is rejected with SESSD_E_INVALID
+ * before anything is launched.  The call allocates and
  * frees nothing; its first use on a device looks the array's address up (make that call outside a
  * stream capture).  All calls on one GPU share the array: it is cleared by each call, and two calls that
  * overlap in time on one GPU (different streams, different handles) race.  Outputs are bit-identical

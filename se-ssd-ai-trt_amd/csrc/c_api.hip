@@ -86,14 +86,13 @@ int sessd_voxelgen_enqueue_static(sessd_voxelgen* h, const sessd_tensor_desc* in
 }
 int sessd_voxelgen_status(const sessd_voxelgen* h, const void* workspace, sessd_stream_t stream, int32_t* status) {
     NEED(h && status, "null argument");
-    NEED(CH_VG(h)->lastMaxPoints_ > 0, "configure or enqueue must run first (the layout depends on max_points)");
+    NEED(CH_VG(h)->lastMaxPoints_ > 0, "configure or enqueue must run first");
     void* own = nullptr;
     if (!workspace) {  // the static scratch of sessd_voxelgen_enqueue_static on the current device
         SESSD_TRY(voxelgen_static_scratch(&own));
         workspace = own;
     }
-    return read_status_word(workspace, CH_VG(h)->statusOffset(CH_VG(h)->lastMaxPoints_),
-                            static_cast<hipStream_t>(stream), status);
+    return read_status_word(workspace, CH_VG(h)->statusOffset(), static_cast<hipStream_t>(stream), status);
 }
 int sessd_voxelgen_set_flags(sessd_voxelgen* h, int32_t flags) {
     NEED(h, "null handle");

@@ -197,7 +197,7 @@ struct Pipeline {
     // everything that a frame has to find as the one before leaves it, as for the first frame
     int resetState(hipStream_t stream) {
         FillArgs f;
-        f.add(static_cast<uint8_t*>(vg_ws.p) + vg->statusOffset(desc.max_points), 4, 0);
+        f.add(static_cast<uint8_t*>(vg_ws.p) + vg->statusOffset(), 4, 0);
         for (auto& st : stages) {
             if (!st->ws.p) continue;
             if (f.n + 2 > FillArgs::kMaxRegions) {
@@ -869,7 +869,7 @@ int sessd_pipeline_status(sessd_pipeline* h, sessd_stream_t stream_, int32_t* st
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     SESSD_TRY(order_after_last_frame(h, stream));
     int32_t acc = 0, s = 0;
-    SESSD_TRY(read_status_word(P->vg_ws.p, P->vg->statusOffset(P->desc.max_points), stream, &s));
+    SESSD_TRY(read_status_word(P->vg_ws.p, P->vg->statusOffset(), stream, &s));
     acc |= s;
     for (auto& st : P->stages) {
         if (!st->ws.p) continue;

@@ -36,16 +36,20 @@ class VoxelGeneratorPlugin {
                       const void* const* inputs, void* const* outputs, hipStream_t stream);
     size_t getSerializationSize() const;
     void serialize(void* buffer) const;
-    size_t statusOffset(int max_points) const;
+    size_t statusOffset() const { return 0; }  // (whatever the layout behind it)
+    // Slots of the cell table's hash per point: at most a quarter full, an insert mostly finds its first slot empty.
+    static constexpr int kSlotsPerPoint = 4;
+    // ... in the static scratch array where only so many fit (enqueueStatic)
+    static constexpr int kSlotsPerPointDense = 2;
     // After an enqueue the workspace's hash maps linear cell (z*Y + y)*X + x -> voxel row (kEmpty for cells
     // dropped at the cap): a SubM layer on the same x/y grid, and a strided layer, look their rulebooks up in it.
-    CellTable cellTable(void* workspace, int max_points) const;
+    CellTable cellTable(void* workspace, int max_points, int slots_per_point = kSlotsPerPoint) const;
     // the passes of an enqueue (coord.h) and what has to be cleared before them: the table, and rows >= voxel_num
     // where the flags ask for them.  status[1] must be 0 (every enqueue leaves it so).
     VgPart part(const float* points, const int32_t* points_size, int max_points, int pf, float* voxels, int32_t* coors,
-                int32_t* voxel_num, void* workspace) const;
+                int32_t* voxel_num, void* workspace, int slots_per_point = kSlotsPerPoint) const;
     // (table_only: without the places of later points, which an enqueue leaves empty)
-    void collectTableFill(void* workspace, int max_points, bool table_only, FillArgs& f) const;
+    void collectTableFill(void* workspace, int max_points, bool table_only, FillArgs& f, int slots_per_point = kSlotsPerPoint) const;
     void collectPadFill(float* voxels, int32_t* coors, FillArgs& f) const;
 
     // serialized fields, in the reference's order (voxelGenerator.cu:584-599)
@@ -63,7 +67,9 @@ class VoxelGeneratorPlugin {
 
   private:
     struct Layout;
-    Layout carve(void* workspace, int max_points) const;
+    Layout carve(void* workspace, int max_points, int slots_per_point) const;
+    int enqueueOn(const sessd_tensor_desc* inputDesc, const void* const* inputs, void* const* outputs, void* workspace,
+                  int slots_per_point, hipStream_t stream);
     void deriveGrid();
 };
 

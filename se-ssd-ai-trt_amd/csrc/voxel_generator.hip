@@ -26,7 +26,6 @@ namespace sessd {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kSlotsPerPoint = 4;
 
 // np.round as in spconv's voxel generator (voxelGenerator.cu:61-68): half to even
 int np_round(float x) {
@@ -47,14 +46,14 @@ struct VoxelGeneratorPlugin::Layout {
     uint32_t cap;
     uint64_t slot_words;
     int n_blocks;
-    size_t status_offset;
     size_t total;
 };
 
-VoxelGeneratorPlugin::Layout VoxelGeneratorPlugin::carve(void* workspace, int max_points) const {
+VoxelGeneratorPlugin::Layout VoxelGeneratorPlugin::carve(void* workspace, int max_points, int slots_per_point) const {
     Layout L;
     WorkspaceCarver c(workspace);
-    L.cap = next_pow2((uint64_t)(max_points < 32 ? 32 : max_points) * kSlotsPerPoint);
+    L.status = c.take<int32_t>(4);
+    L.cap = next_pow2((uint64_t)(max_points < 32 ? 32 : max_points) * slots_per_point);
     L.n_blocks = ceil_div(max_points, kBlock);
     // entries and slots are adjacent so that one fill region clears both
     L.slot_words = (uint64_t)max_points * (pointNum_ - 1);
@@ -63,18 +62,16 @@ VoxelGeneratorPlugin::Layout VoxelGeneratorPlugin::carve(void* workspace, int ma
     L.pt_slot = c.take<int32_t>((size_t)L.n_blocks * kBlock);
     L.words = c.take<uint64_t>((size_t)L.n_blocks * 4);
     L.counts = c.take<uint32_t>((size_t)L.n_blocks);
-    L.status_offset = c.offset;
-    L.status = c.take<int32_t>(4);
     L.total = c.total();
     return L;
 }
 
-CellTable VoxelGeneratorPlugin::cellTable(void* workspace, int max_points) const {
-    const Layout L = carve(workspace, max_points);
+CellTable VoxelGeneratorPlugin::cellTable(void* workspace, int max_points, int slots_per_point) const {
+    const Layout L = carve(workspace, max_points, slots_per_point);
     CellTable t;
     t.base = L.entries;
     t.cap = L.cap;
-    t.per_row16 = 16 * kSlotsPerPoint;  // at most a quarter full: an insert mostly finds its first slot empty
+    t.per_row16 = 16 * slots_per_point;
     t.gx = grid_x_size_;
     t.gy = grid_y_size_;
     t.gz = grid_z_size_;
@@ -82,8 +79,8 @@ CellTable VoxelGeneratorPlugin::cellTable(void* workspace, int max_points) const
 }
 
 VgPart VoxelGeneratorPlugin::part(const float* points, const int32_t* points_size, int max_points, int pf, float* voxels,
-                                  int32_t* coors, int32_t* voxel_num, void* workspace) const {
-    const Layout L = carve(workspace, max_points);
+                                  int32_t* coors, int32_t* voxel_num, void* workspace, int slots_per_point) const {
+    const Layout L = carve(workspace, max_points, slots_per_point);
     VgPart v;
     v.points = points;
     v.points_size = points_size;
@@ -103,7 +100,7 @@ VgPart VoxelGeneratorPlugin::part(const float* points, const int32_t* points_siz
     v.gz = grid_z_size_;
     v.max_voxels = voxelNum_;
     v.max_pts = pointNum_;
-    v.t = cellTable(workspace, max_points);
+    v.t = cellTable(workspace, max_points, slots_per_point);
     v.slots = L.slots;
     v.pt_slot = L.pt_slot;
     v.words = L.words;
@@ -116,8 +113,8 @@ VgPart VoxelGeneratorPlugin::part(const float* points, const int32_t* points_siz
     return v;
 }
 
-void VoxelGeneratorPlugin::collectTableFill(void* workspace, int max_points, bool table_only, FillArgs& f) const {
-    const Layout L = carve(workspace, max_points);
+void VoxelGeneratorPlugin::collectTableFill(void* workspace, int max_points, bool table_only, FillArgs& f, int slots_per_point) const {
+    const Layout L = carve(workspace, max_points, slots_per_point);
     f.add(L.entries, (uint64_t)L.cap * 2 + (table_only ? 0 : L.slot_words), kEmpty);
 }
 void VoxelGeneratorPlugin::collectPadFill(float* voxels, int32_t* coors, FillArgs& f) const {
@@ -231,16 +228,17 @@ int VoxelGeneratorPlugin::configurePlugin(const sessd_tensor_desc* in, int nbInp
 size_t VoxelGeneratorPlugin::getWorkspaceSize(const sessd_tensor_desc* inputs, int nbInputs,
                                               const sessd_tensor_desc*, int) const {
     if (!inputs || nbInputs < 1 || inputs[0].nbDims != 3 || inputs[0].d[1] <= 0) return 0;
-    return carve(nullptr, inputs[0].d[1]).total;
-}
-
-size_t VoxelGeneratorPlugin::statusOffset(int max_points) const {
-    return carve(nullptr, max_points).status_offset;
+    return carve(nullptr, inputs[0].d[1], kSlotsPerPoint).total;
 }
 
 int VoxelGeneratorPlugin::enqueue(const sessd_tensor_desc* inputDesc, const sessd_tensor_desc*,
                                   const void* const* inputs, void* const* outputs, void* workspace,
                                   hipStream_t stream) {
+    return enqueueOn(inputDesc, inputs, outputs, workspace, kSlotsPerPoint, stream);
+}
+
+int VoxelGeneratorPlugin::enqueueOn(const sessd_tensor_desc* inputDesc, const void* const* inputs, void* const* outputs,
+                                    void* workspace, int slots_per_point, hipStream_t stream) {
     if (!inputDesc || !inputs || !outputs || !workspace)
         return fail(SESSD_E_INVALID, "voxelgen.enqueue: null argument");
     if (inputDesc[0].nbDims != 3 || inputDesc[0].d[0] != 1)
@@ -261,11 +259,10 @@ int VoxelGeneratorPlugin::enqueue(const sessd_tensor_desc* inputDesc, const sess
         return fail(SESSD_E_INVALID, "voxelgen.enqueue: outputs must be 16-byte aligned");
 
     lastMaxPoints_ = max_points;
-    const Layout L = carve(workspace, max_points);
-    const VgPart v = part(points, points_size, max_points, pf, voxels, coors, voxel_num, workspace);
+    const VgPart v = part(points, points_size, max_points, pf, voxels, coors, voxel_num, workspace, slots_per_point);
     FillArgs f;
-    collectTableFill(workspace, max_points, false, f);
-    f.add(L.status, 4, 0);
+    collectTableFill(workspace, max_points, false, f, slots_per_point);
+    f.add(v.status, 4, 0);
     SESSD_TRY(launch_fill(f, stream));
     FillArgs pads;
     collectPadFill(voxels, coors, pads);
@@ -288,7 +285,7 @@ int read_status_word(const void* workspace, size_t offset, hipStream_t stream, i
 // at its own address; `scratch` below is only the host-side name of the symbol, never a device pointer,
 // so host code asks the runtime for the address once per device and hands THAT to the kernels.
 // ---------------------------------------------------------------------------------------------
-constexpr size_t kStaticScratchBytes = 8u << 20;  // fits the reference's 80000-point tensor (7.7 MB)
+constexpr size_t kStaticScratchBytes = 8u << 20;  // fits the reference's 80000-point tensor (5.8 MB)
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
 namespace {
@@ -313,12 +310,16 @@ int voxelgen_static_scratch(void** out) {
     return SESSD_OK;
 }
 
-int VoxelGeneratorPlugin::enqueueStatic(const sessd_tensor_desc* inputDesc, const sessd_tensor_desc* outputDesc,
+int VoxelGeneratorPlugin::enqueueStatic(const sessd_tensor_desc* inputDesc, const sessd_tensor_desc*,
                                         const void* const* inputs, void* const* outputs, hipStream_t stream) {
     if (!inputDesc || inputDesc[0].nbDims != 3 || inputDesc[0].d[1] <= 0)
         return fail(SESSD_E_INVALID, "voxelgen.enqueue_static: points must be [1,max_points,F]");
     // the size check comes before any runtime call: a request that does not fit touches nothing
-    const size_t need = carve(nullptr, inputDesc[0].d[1]).total;
+    // With one point per voxel the hash is all that grows with the points: half as many slots double the rows that fit.
+    // (With more, the places of the later points grow too, and 131 072 rows remain the limit.)
+    int slots = kSlotsPerPoint;
+    if (pointNum_ == 1 && carve(nullptr, inputDesc[0].d[1], slots).total > kStaticScratchBytes) slots = kSlotsPerPointDense;
+    const size_t need = carve(nullptr, inputDesc[0].d[1], slots).total;
     if (need > kStaticScratchBytes)
         return fail(SESSD_E_INVALID,
                     "voxelgen.enqueue_static: a points tensor of %d rows with %d points per voxel needs %zu bytes of "
@@ -326,7 +327,7 @@ int VoxelGeneratorPlugin::enqueueStatic(const sessd_tensor_desc* inputDesc, cons
                     inputDesc[0].d[1], pointNum_, need, kStaticScratchBytes);
     void* ws = nullptr;
     SESSD_TRY(voxelgen_static_scratch(&ws));
-    return enqueue(inputDesc, outputDesc, inputs, outputs, ws, stream);
+    return enqueueOn(inputDesc, inputs, outputs, ws, slots, stream);
 }
 
 }  // namespace sessd

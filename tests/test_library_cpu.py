@@ -257,3 +257,21 @@ def test_pipeline_frames_in_flight_is_validated_before_anything_is_built():
     assert L.sessd_pipeline_create(C.byref(d), C.byref(h)) == D.SESSD_E_INVALID and b"overlap_streams" in L.sessd_last_error()
     assert L.sessd_pipeline_submit(None, None, None, None, None, None) == D.SESSD_E_INVALID
     assert L.sessd_pipeline_join(None, 0, None) == D.SESSD_E_INVALID
+
+
+@pytest.mark.parametrize("max_pts,rows", [(1, 131073), (1, 200000), (1, 262144), (2, 131072), (5, 131072), (7, 131072), (8, 65536), (64, 8192)])
+def test_voxelgen_static_enqueue_takes_every_size_it_is_documented_to_take(max_pts, rows):
+    """What fits the static array passes the size check: what the call then meets is a null output, not the check."""
+    vg = api.VoxelGenerator(max_voxels=60000, max_num_points_per_voxel=max_pts)
+    L = api.lib()
+    ind = (D.TensorDesc * 2)(D.TensorDesc.make([1, rows, 4], D.SESSD_FLOAT), D.TensorDesc.make([1], D.SESSD_INT32))
+    outd = (D.TensorDesc * 3)(D.TensorDesc.make([1, 60000, 4], D.SESSD_FLOAT),
+                              D.TensorDesc.make([1, 60000, 4], D.SESSD_INT32), D.TensorDesc.make([1], D.SESSD_INT32))
+    none = (C.c_void_p * 3)()
+    assert L.sessd_voxelgen_enqueue_static(vg.h, ind, outd, none, none, None) != D.SESSD_OK
+    assert b"static buffer holds" not in L.sessd_last_error(), L.sessd_last_error()
+    # one row more than the largest size is refused
+    if (max_pts, rows) in ((1, 262144), (5, 131072)):
+        ind[0] = D.TensorDesc.make([1, rows + 1, 4], D.SESSD_FLOAT)
+        assert L.sessd_voxelgen_enqueue_static(vg.h, ind, outd, none, none, None) == D.SESSD_E_INVALID
+        assert b"static buffer holds" in L.sessd_last_error()

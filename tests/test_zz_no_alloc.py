@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+import oracle_lib as O
 from gpu_util import dev, points_input, to_np
 from sessd3d import api, backbone as B, ctypes_defs as D, frames as F
 
@@ -70,3 +71,16 @@ def test_static_scratch_voxelizer_rejects_what_does_not_fit():
         vg.enqueue_static(ins, outs)
     torch.cuda.synchronize()
     assert int(to_np(outs[2])[0]) == 5                            # nothing was launched
+
+
+@pytest.mark.parametrize("rows", [131072, 131073, 262144])
+def test_static_scratch_voxelizer_with_one_point_per_voxel_at_its_largest_sizes(rows):
+    """Beyond 131 072 rows the static call works on a hash of half as many slots as the one with a workspace."""
+    pts = np.concatenate([F.lidar_frame(rows // 2, s, full_circle=True) for s in (8, 9)])
+    vg = api.VoxelGenerator(max_voxels=60000, max_num_points_per_voxel=1)
+    a, b, (st_a, st_b) = both_ways(vg, pts, rows, 60000)
+    ref = O.voxelize(pts, B.POINT_CLOUD_RANGE, B.VOXEL_SIZE, 1, 60000)
+    assert st_a == st_b == ref[4] and a[2][0] == b[2][0] == ref[2]
+    for got in (a, b):
+        assert np.array_equal(got[1][:ref[2]], ref[1][:ref[2]])
+        assert np.array_equal(got[0][:ref[2]].view(np.uint32), ref[0][:ref[2]].view(np.uint32))
