@@ -364,7 +364,13 @@ int sessd_sparse2dense_clone(const sessd_sparse2dense* h, sessd_sparse2dense** o
 /* ------------------------------------------------------------------------------------------ */
 /* The pipeline owns its plugins, intermediate tensors and workspaces (allocated at create);
  * enqueue allocates nothing.  It is what TensorRT's executor does for the reference: call each
- * plugin's enqueue in graph order on one stream. */
+ * plugin's enqueue in graph order on one stream.
+ *
+ * Memory: beside tensors and workspaces a pipeline keeps tables with 4 bytes per cell of the voxel grid (up to
+ * 2^27 cells) and of every strided layer's output grid (up to 2^25), 416 MB for the reference's grids, and once
+ * more for each of frames_in_flight replicas.  They are allocated last: where the device's memory is short, create
+ * succeeds without them and every frame clears hash tables in the workspaces instead (slower, same
+ * results).  sessd_pipeline_device_bytes says what a pipeline holds. */
 
 typedef struct sessd_pipeline sessd_pipeline;
 
@@ -493,6 +499,8 @@ int sessd_pipeline_layer_stats(sessd_pipeline* h, int layer, sessd_stream_t stre
                                int64_t* pairs);
 /* OR of every layer's status word (synchronises the stream) */
 int sessd_pipeline_status(sessd_pipeline* h, sessd_stream_t stream, int32_t* status);
+/* device memory that the pipeline holds: tensors, workspaces and the kept tables that could be allocated (the layers'
+ * weights come on top) */
 size_t sessd_pipeline_device_bytes(const sessd_pipeline* h);
 int sessd_pipeline_num_launches(const sessd_pipeline* h);
 void sessd_pipeline_destroy(sessd_pipeline* h);

@@ -28,8 +28,8 @@ struct DeviceBuffer {
     void* p = nullptr;
     size_t bytes = 0;
     int alloc(size_t n) {
-        bytes = n;
         SESSD_HIP_TRY(hipMalloc(&p, n ? n : 16));
+        bytes = n;
         return SESSD_OK;
     }
     ~DeviceBuffer() {
@@ -83,8 +83,8 @@ struct ConvStage {
     std::unique_ptr<SubmConv3dLayerPlugin> subm;
     std::unique_ptr<SparseConv3dLayerPlugin> sparse;
     DeviceBuffer ws, feat, coors, num;  // coors/num only for sparse layers (they produce new ones)
-    // Sparse layers: output cell -> row (47 MB for 21 x 800 x 704); none where the grid is too large for that (the
-    // workspace's table then)
+    // Sparse layers: output cell -> row (47 MB for 21 x 800 x 704); none where the grid or the device's memory does not
+    // allow it (the workspace's table then)
     KeptTable cells;
     int rulebook_from = -1;             // SubM layer whose workspace holds this layer's rulebook
     sessd_tensor_desc in_desc[3], out_desc[3];
@@ -115,7 +115,7 @@ struct Pipeline {
     std::unique_ptr<Sparse2DensePlugin> s2d;
     std::vector<std::unique_ptr<ConvStage>> stages;
     DeviceBuffer vg_ws, vg_voxels, vg_coors, vg_num, s2d_ws;
-    KeptTable vg_cells;  // the voxelizer's cell table (369 MB for 40 x 1600 x 1408), as ConvStage::cells
+    KeptTable vg_cells;  // the voxelizer's cell table (360 MB for 40 x 1600 x 1408), as ConvStage::cells
     sessd_tensor_desc vg_in[2], vg_out[3], s2d_in[3], s2d_out[1];
     int max_voxels = 0;
     size_t device_bytes = 0;
@@ -475,7 +475,7 @@ struct Pipeline {
     }
 };
 
-// largest output grid that gets a dense table (a ticket keeps its cell in 26 bits)
+// largest output grid that gets a kept table (a ticket keeps its cell in 26 bits)
 constexpr uint64_t kDenseCells = 1ull << 25;
 // ... and largest voxel grid
 constexpr uint64_t kDenseVoxelCells = 1ull << 27;
@@ -510,9 +510,7 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
     SESSD_TRY(P->vg_voxels.alloc((size_t)V * 4 * sizeof(float)));
     SESSD_TRY(P->vg_coors.alloc((size_t)V * 4 * sizeof(int32_t)));
     SESSD_TRY(P->vg_num.alloc(256));
-    const uint64_t cells = (uint64_t)vg->grid_x_size_ * (uint64_t)vg->grid_y_size_ * (uint64_t)vg->grid_z_size_;
-    if (cells <= kDenseVoxelCells) SESSD_TRY(P->vg_cells.alloc(cells, VG));
-    total += P->vg_ws.bytes + P->vg_voxels.bytes + P->vg_coors.bytes + P->vg_cells.mem.bytes + 256;
+    total += P->vg_ws.bytes + P->vg_voxels.bytes + P->vg_coors.bytes + 256;
 
     int in_type = SESSD_FLOAT;  // the voxelizer's means are FP32
     int in_ch = 4;
@@ -580,8 +578,6 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
             SESSD_TRY(st->ws.alloc(p->getWorkspaceSize(st->in_desc, 3, st->out_desc, 3)));
             SESSD_TRY(st->coors.alloc((size_t)V * 4 * sizeof(int32_t)));
             SESSD_TRY(st->num.alloc(256));
-            const uint64_t volume = (uint64_t)s.out_shape[0] * (uint64_t)s.out_shape[1] * (uint64_t)s.out_shape[2];
-            if (volume <= kDenseCells) SESSD_TRY(st->cells.alloc(volume, V));
             last_subm_with_rulebook = -1;  // new coordinates: earlier rulebooks no longer apply
         } else {
             return fail(SESSD_E_INVALID, "pipeline: layer %d has unknown type %d", l, s.type);
@@ -589,7 +585,7 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
         base->flags_ = d.flags;
         SESSD_TRY(base->setEpilogue(d.scale ? d.scale[l] : nullptr, d.shift ? d.shift[l] : nullptr, d.relu));
         SESSD_TRY(st->feat.alloc((size_t)V * s.out_channel * dtype_size(ft)));
-        total += st->ws.bytes + st->feat.bytes + st->coors.bytes + st->num.bytes + st->cells.mem.bytes;
+        total += st->ws.bytes + st->feat.bytes + st->coors.bytes + st->num.bytes;
         in_type = ft;
         in_ch = s.out_channel;
         P->stages.push_back(std::move(st));
@@ -617,6 +613,25 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
         P->ev_pass.assign(2 * P->coordStages().size(), nullptr);
         for (auto& e : P->ev_pass) SESSD_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
+    // the layer array of the caller need not outlive create()
+    P->desc.layers = nullptr;
+    P->desc.weights = P->desc.scale = P->desc.shift = nullptr;
+    return SESSD_OK;
+}
+
+// Behind everything that a pipeline (all its replicas) cannot do without: the tables it keeps.  Where memory for one is
+// short, the table in the workspace does, which every frame clears.
+static int finish_pipeline(Pipeline* P) {
+    const VoxelGeneratorPlugin& vg = *P->vg;
+    const uint64_t cells = (uint64_t)vg.grid_x_size_ * (uint64_t)vg.grid_y_size_ * (uint64_t)vg.grid_z_size_;
+    if (cells <= kDenseVoxelCells) (void)P->vg_cells.alloc(cells, P->desc.voxelgen.max_voxels);
+    P->device_bytes += P->vg_cells.mem.bytes;
+    for (auto& st : P->stages) {
+        if (!st->sparse) continue;
+        const uint64_t volume = (uint64_t)st->spec.out_shape[0] * (uint64_t)st->spec.out_shape[1] * (uint64_t)st->spec.out_shape[2];
+        if (volume <= kDenseCells) (void)st->cells.alloc(volume, P->max_voxels);
+        P->device_bytes += st->cells.mem.bytes;
+    }
     // what the passes leave as they need it for the next frame has to be right for the first
     SESSD_TRY(P->resetState(nullptr));
     FillArgs counts;  // queries before the first frame find no rows
@@ -630,9 +645,6 @@ static int build_pipeline(const sessd_pipeline_desc& d, Pipeline* P) {
     }
     SESSD_TRY(launch_fill(counts, nullptr));
     SESSD_HIP_TRY(hipStreamSynchronize(nullptr));
-    // the layer array of the caller need not outlive create()
-    P->desc.layers = nullptr;
-    P->desc.weights = P->desc.scale = P->desc.shift = nullptr;
     return SESSD_OK;
 }
 
@@ -698,15 +710,19 @@ static int pipeline_create_unguarded(const sessd_pipeline_desc* desc, sessd_pipe
             for (hipEvent_t* e : {&rep->ev_in, &rep->ev_frame_done})
                 SESSD_HIP_TRY(hipEventCreateWithFlags(e, hipEventDisableTiming));
             SESSD_HIP_TRY(hipStreamCreateWithFlags(&rep->frame_stream, hipStreamNonBlocking));
-            P->device_bytes += rep->device_bytes;
             P->max_voxels = rep->max_voxels;
             P->replicas.push_back(std::move(rep));
+        }
+        for (auto& rep : P->replicas) {
+            SESSD_TRY(finish_pipeline(rep.get()));
+            P->device_bytes += rep->device_bytes;
         }
         P->desc = *desc;
         P->desc.layers = nullptr;
         P->desc.weights = P->desc.scale = P->desc.shift = nullptr;
     } else {
         SESSD_TRY(build_pipeline(*desc, P.get()));
+        SESSD_TRY(finish_pipeline(P.get()));
     }
     *out = reinterpret_cast<sessd_pipeline*>(P.release());
     return SESSD_OK;

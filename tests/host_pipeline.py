@@ -171,6 +171,34 @@ def check_own_graph():
     assert [l[0] for l in launches_of(enqueue, h, stream)] == ["graph"]
 
 
+def check_short_memory():
+    """Device memory that holds everything but the kept cell tables: create succeeds, with fewer tables the fewer fit, and
+    frames run."""
+    L.sessd_pipeline_device_bytes.restype = C.c_size_t
+    bytes_of = lambda h: L.sessd_pipeline_device_bytes(h)  # noqa: E731
+    rc, h = create()
+    assert rc == 0
+    full = bytes_of(h)
+    kept = []
+    for limit in (300 << 20, 40 << 20):
+        FAKE.fake_largest_allocation(limit)
+        rc, h = create(overlap_streams=1)
+        assert rc == 0, L.sessd_last_error()
+        kept.append(full - bytes_of(h))
+        rc, two = create(overlap_streams=1, frames_in_flight=2)
+        assert rc == 0 and bytes_of(two) == 2 * bytes_of(h)
+        stream = new_stream()
+        take_log()
+        for _ in range(2):  # (an error left pending by the allocation would fail the first)
+            assert enqueue(h, stream) == 0, L.sessd_last_error()
+            assert not unordered(take_log())
+    voxels, strided = 40 * 1600 * 1408 * 4, 21 * 800 * 704 * 4
+    assert voxels < kept[0] < voxels + 4096 and voxels + strided < kept[1] < voxels + strided + 2 * 4096, kept
+    FAKE.fake_largest_allocation(1000)
+    rc, h = create()
+    assert rc == D.SESSD_E_HIP and not h.value
+
+
 CHECKS = {
     "recovery-direct": lambda: check_recovery(0, enqueue),
     "recovery-overlap": lambda: check_recovery(1, enqueue),
@@ -180,6 +208,7 @@ CHECKS = {
     "capture-direct": lambda: check_capture(0),
     "capture-overlap": lambda: check_capture(1),
     "own-graph": check_own_graph,
+    "short-memory": check_short_memory,
 }
 
 if __name__ == "__main__":

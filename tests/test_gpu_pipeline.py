@@ -602,3 +602,42 @@ def test_a_frame_in_the_callers_own_graph_survives_a_call_that_failed(overlap):
         assert [pipe.layer_count(l) for l in range(-1, len(layers))] == list(ref["counts"]), (step, how)
         assert np.array_equal(pipe.read_layer(len(layers) - 1)[1], ref["coors"]), (step, how)
         assert_end_to_end_close(to_np(dense), ref["dense"], False, "dense, step %d" % step)
+
+
+def test_a_voxel_grid_too_large_for_a_kept_table(monkeypatch):
+    """Voxels of half the size: neither the voxelizer's table nor the first strided layer's has room for a word per cell,
+    so every frame clears their hashes -- as it does where the memory for kept tables is short.  The frames shrink and
+    grow, so that what one leaves behind would reach the next."""
+    size = (0.025, 0.025, 0.1)
+    desc = lambda cap, pts=5: B.voxelgen_desc(cap, pts, B.POINT_CLOUD_RANGE, size)  # noqa: E731
+    S, P = D.SESSD_LAYER_SUBM, D.SESSD_LAYER_SPARSE
+    layers = [B.Layer("subm0", S, 4, 16, (2816, 3200, 41), (3, 3, 3), (1, 1, 1), (1, 1, 1)),
+              B.Layer("sparse1", P, 16, 32, (1408, 1600, 21), (3, 3, 3), (2, 2, 2), (1, 1, 1)),
+              B.Layer("subm2", S, 32, 32, (1408, 1600, 21), (3, 3, 3), (1, 1, 1), (1, 1, 1)),
+              B.Layer("sparse3", P, 32, 64, (704, 800, 11), (3, 3, 3), (2, 2, 2), (1, 1, 1)),
+              B.Layer("sparse4", P, 64, 64, (352, 400, 5), (3, 3, 3), (2, 2, 2), (0, 1, 1))]
+    W = B.random_weights(layers, seed=16, w_std=0.05)
+    mp, mv, dsize = 4096, 20000, (352, 400, 5)
+    with monkeypatch.context() as m:
+        original = B.voxelgen_desc
+        m.setattr(api.B, "voxelgen_desc", lambda cap, pts=5: original(cap, pts, B.POINT_CLOUD_RANGE, size))
+        pipes = [api.Pipeline(layers, W, mp, mv, dense_size_xyz=dsize, share_rulebooks=True, skip_pad_rows=True, use_graph=o,
+                              overlap_streams=o) for o in (True, False)]
+    p, n = points_input(np.zeros((0, 4), np.float32), mp)
+    stream = torch.cuda.Stream()
+    for step, npts in enumerate((3000, 600, 0, 4000, 1200)):
+        pts = F.lidar_frame(npts, 150 + step) if npts else np.zeros((0, 4), np.float32)
+        hp, hn = points_input(pts, mp)
+        p.copy_(hp)
+        n.copy_(hn)
+        torch.cuda.synchronize()
+        ref = O.frame(pts, desc(mv), layers, W, B.dense_desc(dsize, 64))
+        for pipe in pipes:
+            dense = pipe.new_dense()
+            torch.cuda.synchronize()
+            pipe.enqueue(p, n, dense, stream)
+            stream.synchronize()
+            assert pipe.status() == ref["status"] == 0
+            assert [pipe.layer_count(l) for l in range(-1, len(layers))] == list(ref["counts"]), step
+            assert np.array_equal(pipe.read_layer(len(layers) - 1)[1], ref["coors"]), step
+            assert_end_to_end_close(to_np(dense), ref["dense"], False, "dense, step %d" % step)

@@ -31,3 +31,7 @@ def run_check(fake_hip, check):
                                    "capture-direct", "capture-overlap", "own-graph"])
 def test_failed_calls_leave_the_cell_tables_empty(fake_hip, check):
     run_check(fake_hip, check)
+
+
+def test_a_pipeline_does_without_the_kept_tables_where_memory_is_short(fake_hip):
+    run_check(fake_hip, "short-memory")
