@@ -20,7 +20,6 @@ namespace sessd {
 // error reporting: no abort(), a thread-local message and an error code instead
 // (the reference's checkCudaErrors prints and aborts, voxelGenerator.cu:8-19)
 // ---------------------------------------------------------------------------------------------
-void set_last_error(const std::string& msg);
 int fail(int code, const char* fmt, ...);
 
 #define SESSD_HIP_TRY(expr)                                                                      \

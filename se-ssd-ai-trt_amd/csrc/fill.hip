@@ -6,22 +6,20 @@
 namespace sessd {
 
 namespace {
-thread_local std::string g_last_error;
+thread_local char g_last_error[1024] = "";  // (reporting that memory has run out takes none)
 }
 
-void set_last_error(const std::string& msg) { g_last_error = msg; }
-
 int fail(int code, const char* fmt, ...) {
-    char buf[1024];
+    char buf[sizeof(g_last_error)];  // (an argument may be the last message)
     va_list ap;
     va_start(ap, fmt);
     vsnprintf(buf, sizeof(buf), fmt, ap);
     va_end(ap);
-    g_last_error = buf;
+    std::memcpy(g_last_error, buf, sizeof(buf));
     return code;
 }
 
-const char* last_error_cstr() { return g_last_error.c_str(); }
+const char* last_error_cstr() { return g_last_error; }
 
 template <int N>
 __global__ void __launch_bounds__(256) fill_kernel(FillPlan<N> p) {

@@ -229,7 +229,7 @@ struct Pipeline {
     // what the call has launched on either stream.  Where `stream` is being captured nothing has run; only `aux` has to
     // come back to it, so that the capture can be ended.
     int recover(hipStream_t stream, int rc) {
-        char why[512];
+        char why[1024];
         snprintf(why, sizeof(why), "%s", sessd_last_error());
         (void)hipGetLastError();  // (reported already; the launches below ask for theirs)
         if (captureStatus(stream) != hipStreamCaptureStatusNone) {
@@ -742,8 +742,8 @@ static Pipeline* current(sessd_pipeline* h) {
 // one frame on `stream`: a replay of the captured graph when the pipeline uses graphs (re-captured when a pointer
 // changed), direct launches otherwise
 static int run_frame(Pipeline* P, const void* points, const void* points_size, void* dense, hipStream_t stream) {
-    auto run = [&]() -> int {
-        const int rc = P->enqueueFrame(points, points_size, dense, stream);
+    auto run = [&]() -> int {  // (building the passes of a frame allocates on the host)
+        const int rc = guarded("pipeline", [&]() -> int { return P->enqueueFrame(points, points_size, dense, stream); });
         return rc == SESSD_OK ? rc : P->recover(stream, rc);
     };
     if (!P->tables_ready) {
@@ -912,8 +912,15 @@ int sessd_pipeline_enqueue_timed(sessd_pipeline* h, const void* points, const vo
     const int n_seg = 2 * L + 2;  // voxelizer, {rulebook build, gather-GEMM} per layer, sparse2dense
     if (max_segments < n_seg) return fail(SESSD_E_INVALID, "pipeline_enqueue_timed: need room for %d segments", n_seg);
     if (P->events.empty()) {
-        P->events.resize(n_seg + 3);  // + two back-to-back events that bracket nothing (timer overhead)
-        for (auto& e : P->events) SESSD_HIP_TRY(hipEventCreate(&e));
+        SESSD_TRY(guarded(__func__, [&]() -> int {
+            P->events.reserve(n_seg + 3);  // + two back-to-back events that bracket nothing (timer overhead)
+            return SESSD_OK;
+        }));
+    }
+    while ((int)P->events.size() < n_seg + 3) {
+        hipEvent_t e = nullptr;
+        SESSD_HIP_TRY(hipEventCreate(&e));
+        P->events.push_back(e);
     }
     for (int l = 0; l < L; ++l) {
         ConvPluginBase* b = P->stages[l]->subm ? static_cast<ConvPluginBase*>(P->stages[l]->subm.get())

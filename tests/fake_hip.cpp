@@ -2,7 +2,7 @@
 // library can be tested without a GPU: the order of launches over streams and events, and what happens when a call fails.
 // Loaded before the library with its symbols global (tests/test_host_failures_cpu.py).
 //
-// Log lines:  launch <kernel> <stream> | record <event> <stream> | wait <stream> <event> | graph <stream>
+// Log lines:  launch <kernel> <stream> | record <event> <stream> | wait <stream> <event> | graph - <stream>
 // Streams and events are numbered; the default stream is 0.
 #include <hip/hip_runtime_api.h>
 
@@ -30,6 +30,12 @@ std::string& log_text() {
     static std::string s;
     return s;
 }
+long fail_new = -1;  // calls of operator new until they fail
+struct Own {  // what this file allocates itself does not count
+    const long keep = fail_new;
+    Own() { fail_new = -1; }
+    ~Own() { fail_new = keep; }
+};
 std::map<const void*, std::string>& kernels() {
     static std::map<const void*, std::string> m;
     return m;
@@ -44,12 +50,18 @@ std::map<Stream*, int>& streams() {
 }
 Stream* stream_of(hipStream_t s) { return s ? reinterpret_cast<Stream*>(s) : &default_stream(); }
 int number(Stream* s) { return s == &default_stream() ? 0 : streams()[s]; }
-void note(const std::string& line) { log_text() += line + "\n"; }
+void note(const char* what, const char* name, int number) {
+    Own own;
+    log_text() += std::string(what) + " " + name + " " + std::to_string(number) + "\n";
+}
+void note(const char* what, int a, int b) {
+    Own own;
+    note(what, std::to_string(a).c_str(), b);
+}
 
 hipError_t last_error = hipSuccess;
 long launches = 0, fail_from = -1, fail_to = -1;     // launches that report an error
 unsigned long long largest_allocation = ~0ull;
-long fail_new = -1;  // allocations of operator new until one fails
 int next_event = 0;
 
 hipError_t report(hipError_t e) {
@@ -61,7 +73,8 @@ hipError_t report(hipError_t e) {
 
 // every operator new of the library
 void* operator new(std::size_t n) {
-    if (fail_new >= 0 && fail_new-- == 0) throw std::bad_alloc();
+    if (fail_new == 0) throw std::bad_alloc();
+    if (fail_new > 0) --fail_new;
     void* p = std::malloc(n ? n : 1);
     if (!p) throw std::bad_alloc();
     return p;
@@ -78,7 +91,7 @@ void fake_fail_launches(long first, long count) {  // counted from the next one
     fail_to = fail_from + count;
 }
 void fake_largest_allocation(unsigned long long bytes) { largest_allocation = bytes; }
-void fake_fail_new(long after) { fail_new = after; }
+void fake_fail_new(long after) { fail_new = after; }  // (a negative number: never again)
 long fake_news_left() { return fail_new; }
 int fake_stream_number(hipStream_t s) { return number(stream_of(s)); }
 
@@ -109,7 +122,7 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipSt
 }
 hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void**, size_t, hipStream_t s) {
     if (grid.x == 0) return report(hipErrorInvalidConfiguration);
-    note("launch " + kernels()[f] + " " + std::to_string(number(stream_of(s))));
+    note("launch", kernels()[f].c_str(), number(stream_of(s)));
     const long i = launches++;
     if (fail_from >= 0 && i >= fail_from && i < fail_to) return report(hipErrorUnknown);
     return hipSuccess;
@@ -191,6 +204,7 @@ hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g) {
 }
 
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+    Own own;
     Event* ev = new Event();
     ev->id = next_event++;
     *e = reinterpret_cast<hipEvent_t>(ev);
@@ -205,10 +219,11 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
     Event* ev = reinterpret_cast<Event*>(e);
     ev->on = stream_of(s);
     ev->captured = ev->on->capturing;
-    note("record " + std::to_string(ev->id) + " " + std::to_string(number(ev->on)));
+    note("record", ev->id, number(ev->on));
     return hipSuccess;
 }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned int) {
+    Own own;
     Event* ev = reinterpret_cast<Event*>(e);
     Stream* st = stream_of(s);
     if (!ev->on) return hipSuccess;
@@ -222,7 +237,7 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned int) {
     } else if (st->capturing) {
         return report(hipErrorStreamCaptureIsolation);
     }
-    note("wait " + std::to_string(number(st)) + " " + std::to_string(ev->id));
+    note("wait", number(st), ev->id);
     return hipSuccess;
 }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
@@ -240,7 +255,7 @@ hipError_t hipGraphGetNodes(hipGraph_t, hipGraphNode_t*, size_t* n) {
     return hipSuccess;
 }
 hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t s) {
-    note("graph " + std::to_string(number(stream_of(s))));
+    note("graph", "-", number(stream_of(s)));
     const long i = launches++;
     if (fail_from >= 0 && i >= fail_from && i < fail_to) return report(hipErrorUnknown);
     return hipSuccess;

@@ -171,6 +171,32 @@ def check_own_graph():
     assert [l[0] for l in launches_of(enqueue, h, stream)] == ["graph"]
 
 
+def check_host_memory():
+    """Host memory runs out at every allocation of a frame in turn: an error code, no exception across the C boundary, and
+    the clears of a failed call."""
+    rc, h = create(overlap_streams=1)
+    stream = new_stream()
+    plain = launches_of(enqueue, h, stream)
+    failed = 0
+    while True:
+        FAKE.fake_fail_new(failed)
+        rc = enqueue(h, stream)
+        done = FAKE.fake_news_left()
+        FAKE.fake_fail_new(-1)
+        log = take_log()
+        if rc == 0:
+            break
+        assert rc == D.SESSD_E_NOMEM and done == 0 and b"out of host memory" in L.sessd_last_error(), (rc, done)
+        assert is_fill(launches(log)[-1]) and not unordered(log), failed
+        assert len(launches_of(enqueue, h, stream)) == len(plain)
+        failed += 1
+    assert failed > 5
+    FAKE.fake_fail_new(0)
+    rc = timed(h, stream)
+    FAKE.fake_fail_new(-1)
+    assert rc == D.SESSD_E_NOMEM and timed(h, stream) == 0
+
+
 def check_short_memory():
     """Device memory that holds everything but the kept cell tables: create succeeds, with fewer tables the fewer fit, and
     frames run."""
@@ -209,6 +235,7 @@ CHECKS = {
     "capture-overlap": lambda: check_capture(1),
     "own-graph": check_own_graph,
     "short-memory": check_short_memory,
+    "host-memory": check_host_memory,
 }
 
 if __name__ == "__main__":

@@ -35,3 +35,7 @@ def test_failed_calls_leave_the_cell_tables_empty(fake_hip, check):
 
 def test_a_pipeline_does_without_the_kept_tables_where_memory_is_short(fake_hip):
     run_check(fake_hip, "short-memory")
+
+
+def test_host_memory_that_runs_out_in_a_frame_is_an_error_code(fake_hip):
+    run_check(fake_hip, "host-memory")
