@@ -768,6 +768,35 @@ def test_fp16_ring_kernel_around_the_row_counts_of_its_tile_heights(cin, cout, n
         O.set_threads(1)
 
 
+@pytest.mark.parametrize("cin,cout,n", [(64, 64, 3060), (64, 64, 26247), (64, 64, 90000), (64, 128, 8193), (64, 128, 30000), (128, 128, 2833),
+                                        (128, 128, 19825), (128, 128, 40422), (128, 128, 60000)])
+def test_fp16_ring_kernel_gives_the_same_bits_launch_after_launch(cin, cout, n):
+    """The ring's waits are counted by hand over requests that go straight to LDS: a wait that covered one request too few
+    would show in a few tiles out of many launches.  1200 launches per shape, half of them while copies on another
+    stream load the memory; every output word against the first launch's."""
+    grid = (21, 400, 352)
+    coors = F.clustered_active_voxels(n, grid, 7100 + n, n_blobs=max(4, n // 100))
+    rng = np.random.default_rng(n)
+    cbuf = np.zeros((n, 4), np.int32)
+    cbuf[:, :] = coors
+    feat = dev(rng.uniform(-1, 1, (n, cin)).astype(np.float32), torch.float16)
+    args = (feat, dev(cbuf), dev(np.array([n], np.int32)))
+    w = rng.normal(0, 0.1, (27, cin, cout)).astype(np.float32)
+    conv = api.SubmConv3d(cin, cout, grid[::-1], w, n)
+    first = conv(*args).view(torch.int16)
+    op = api.SubmConv3d(cin, cout, grid[::-1], w, n)
+    bad = torch.zeros((), dtype=torch.int64, device="cuda:0")
+    other, (a, b) = torch.cuda.Stream(), torch.zeros((2, 32 << 20), dtype=torch.uint8, device="cuda:0")
+    torch.cuda.synchronize()
+    for i in range(1200):
+        if i >= 600 and i % 3 == 0:
+            with torch.cuda.stream(other):
+                b.copy_(a)
+        bad += (op(*args, rulebook_from=conv).view(torch.int16) != first).sum()
+    torch.cuda.synchronize()
+    assert int(bad) == 0
+
+
 # ---------------------------------------------------------------------------------------------
 # the FP32 kernel with one tall tile per compute unit (conv_wide.hip: 64 -> 64 and 32 -> 64)
 # ---------------------------------------------------------------------------------------------
