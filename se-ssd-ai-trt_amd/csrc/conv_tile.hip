@@ -84,13 +84,14 @@ __device__ __forceinline__ v4i make_rsrc(const void* p, unsigned bytes) {
 }
 
 // 16 bytes per lane from r[voff] to LDS bytes lds + 16 * lane.  (Written out: the compiler would wait for every such load
-// before any LDS read that it cannot tell apart from its destination.  It is told that m0 changes.)
+// before any LDS read that it cannot tell apart from its destination.  The compiler writes m0 itself; the nop is the wait
+// state that a load to LDS needs behind that.)
 __device__ __forceinline__ void load_to_lds(const v4i& r, unsigned voff, unsigned lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(voff), "s"(r) : "memory", "m0");
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r) : "memory");
 }
 // 4 bytes per lane to lds + 4 * lane
 __device__ __forceinline__ void load4_to_lds(const v4i& r, unsigned voff, unsigned lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds), "v"(voff), "s"(r) : "memory", "m0");
+    asm volatile("s_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r) : "memory");
 }
 template <int N>
 __device__ __forceinline__ void wait_loads() {  // all but the N youngest have arrived
