@@ -149,11 +149,16 @@ __device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t* lds4) {
 // ---------------------------------------------------------------------------------------------
 // The cells that a frame's rows have taken in a table that is kept for the next frame: what empties the table goes by
 // this list.  The coors tensor names the same cells, but callers get pointers to it.
-struct CellList {
-    int32_t* num = nullptr;   // null: no list is kept
-    uint32_t* key = nullptr;  // [rows]
-};
+// One pointer (kernels that pass two layers are short of scalar registers): [0] the number of cells, [kCellListHead ..]
+// their keys.  Null: no list is kept.
+typedef uint32_t* CellList;
+constexpr int kCellListHead = 64;
 
+// Every 64 points of vg_finalize need the counts of all 256-point blocks.  Beyond a million points the blocks read their
+// sums over 64 instead: reading them all grows with the square of the points (the plugin at
+// 2 400 000 points 452 -> 353 us, at 1 200 000 189 -> 176); below, the atomics that make the sums cost more than they
+// save (at 600 000 97 -> 101).
+constexpr int kCountsPerSum = 64, kSumsFromPoints = 1 << 20;
 struct VgPart {
     const float* points = nullptr;
     const int32_t* points_size = nullptr;
@@ -168,11 +173,12 @@ struct VgPart {
     int32_t* pt_slot = nullptr;
     uint64_t* words = nullptr;
     uint32_t* counts = nullptr;
+    uint32_t* sums = nullptr;  // null, or the sums of the counts of kCountsPerSum blocks
     int n_blocks = 0;
     float* voxels = nullptr;
     int32_t* coors = nullptr;
     int32_t* voxel_num = nullptr;
-    CellList taken;
+    CellList taken = nullptr;
     int32_t* status = nullptr;  // [0] status, [1] what vg_insert has met (folded into [0] and cleared by vg_finalize)
 };
 
@@ -191,7 +197,7 @@ struct SpPart {
     const int32_t* in_num = nullptr;
     int32_t* out_coors = nullptr;
     int32_t* out_num = nullptr;
-    CellList taken;
+    CellList taken = nullptr;
     int32_t* nbr = nullptr;   // null: the rulebook is looked up (LookupPart), sp_number has nothing to initialise
     int32_t* meta = nullptr;  // [0] status, [1] output rows, [2] what sp_insert has met (folded into [0] by sp_number)
 };
@@ -232,7 +238,7 @@ CutPart make_cut_part(const int32_t* num_out, int K, int max_voxels, int target_
 
 // A dense table that stays from frame to frame: emptied cell by cell instead of by a fill of its whole volume.
 struct CleanPart {
-    CellList taken;
+    CellList taken = nullptr;
     int max_voxels = 0;
     CellTable t;
     int blocks = 0;

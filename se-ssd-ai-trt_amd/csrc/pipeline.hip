@@ -43,18 +43,13 @@ struct KeptTable {
     DeviceBuffer mem;
     uint32_t cells = 0;  // 0: none
     int alloc(uint64_t volume, int rows) {
-        SESSD_TRY(mem.alloc(listAt(volume) + kWorkspaceAlign + (size_t)rows * sizeof(uint32_t)));
+        SESSD_TRY(mem.alloc(listAt(volume) + ((size_t)kCellListHead + rows) * sizeof(uint32_t)));
         cells = (uint32_t)volume;
         return SESSD_OK;
     }
     static size_t listAt(uint64_t volume) { return align_up(volume * sizeof(uint32_t)); }
     CellList taken() const {
-        CellList l;
-        if (!cells) return l;
-        uint8_t* p = static_cast<uint8_t*>(mem.p) + listAt(cells);
-        l.num = reinterpret_cast<int32_t*>(p);
-        l.key = reinterpret_cast<uint32_t*>(p + kWorkspaceAlign);
-        return l;
+        return cells ? reinterpret_cast<CellList>(static_cast<uint8_t*>(mem.p) + listAt(cells)) : nullptr;
     }
     void replace(CellTable& t) const {  // t: the table of the workspace, for the same grid
         if (!cells) return;
@@ -72,7 +67,7 @@ struct KeptTable {
     void collectFill(FillArgs& f) const {
         if (!cells) return;
         f.add(mem.p, cells, kEmpty);
-        f.add(taken().num, 1, 0);
+        f.add(taken(), 1, 0);
     }
 };
 
@@ -393,7 +388,7 @@ struct Pipeline {
             bool did = false;
             while (at < cuts.size() || (!did && (next || i == clean_at))) {
                 const size_t n = cuts.size() - at < (size_t)kMaxCuts ? cuts.size() - at : (size_t)kMaxCuts;
-                SESSD_TRY(launch_number(did ? nullptr : next, did ? nullptr : after, cuts.data() + at, (int)n, did || !clean.taken.num ? nullptr : &clean,
+                SESSD_TRY(launch_number(did ? nullptr : next, did ? nullptr : after, cuts.data() + at, (int)n, did || !clean.taken ? nullptr : &clean,
                                         did ? nullptr : &clear, side));
                 at += n;
                 did = true;

@@ -42,6 +42,7 @@ struct VoxelGeneratorPlugin::Layout {
     int32_t* pt_slot;
     uint64_t* words;
     uint32_t* counts;
+    uint32_t* sums;
     int32_t* status;
     uint32_t cap;
     uint64_t slot_words;
@@ -62,6 +63,7 @@ VoxelGeneratorPlugin::Layout VoxelGeneratorPlugin::carve(void* workspace, int ma
     L.pt_slot = c.take<int32_t>((size_t)L.n_blocks * kBlock);
     L.words = c.take<uint64_t>((size_t)L.n_blocks * 4);
     L.counts = c.take<uint32_t>((size_t)L.n_blocks);
+    L.sums = max_points > kSumsFromPoints ? c.take<uint32_t>((size_t)ceil_div(L.n_blocks, kCountsPerSum)) : nullptr;
     L.total = c.total();
     return L;
 }
@@ -105,6 +107,7 @@ VgPart VoxelGeneratorPlugin::part(const float* points, const int32_t* points_siz
     v.pt_slot = L.pt_slot;
     v.words = L.words;
     v.counts = L.counts;
+    v.sums = L.sums;
     v.n_blocks = L.n_blocks;
     v.voxels = voxels;
     v.coors = coors;

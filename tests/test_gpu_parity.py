@@ -59,6 +59,23 @@ def test_voxelgen_reference_shapes_and_padding():
     assert vg.status() == 0
 
 
+@pytest.mark.parametrize("npts", [1048476, 1048477, 1048576 + 16384, 1300001])
+def test_voxelgen_with_more_points_than_its_last_pass_reads_one_by_one(npts):
+    """Beyond 1 048 576 rows of points the pass that numbers voxels goes by sums over 64 blocks of 256 points.  A second call
+    on the same workspace with a third of the points, one that ends with a sum, and an empty one."""
+    pts = np.concatenate([F.lidar_frame(-(-npts // 3), s, full_circle=True) for s in (41, 42, 43)])[:npts]
+    vg = api.VoxelGenerator(max_voxels=npts)
+    p, size = points_input(pts, npts + 100)
+    for n in (npts, npts // 3, 4 * 16384, 4 * 16384 + 1, 0):
+        size.fill_(n)
+        voxels, coors, num = vg(p, size)
+        torch.cuda.synchronize()
+        ref = O.voxelize(pts[:n], RANGE, VSIZE, 5, npts)
+        assert int(num[0]) == ref[2] and vg.status() == ref[4]
+        assert np.array_equal(to_np(coors)[:ref[2]], ref[1][:ref[2]])
+        assert np.array_equal(to_np(voxels)[:ref[2]].view(np.uint32), ref[0][:ref[2]].view(np.uint32))
+
+
 def test_voxelgen_crowded_voxels_and_shuffled_order():
     rng = np.random.default_rng(3)
     pts = F.lidar_frame(12000, 3)
@@ -459,6 +476,37 @@ def test_sparse_layers_of_the_backbone(layer):
     a = canonical(oc, on, out)
     b = canonical(o_oc, o_on, o_out)
     assert_features_close(a[1], b[1], RTOL_FP32, layer.name + " (canonical order)", abs_sum=canonical(o_oc, o_on, terms)[1])
+
+
+@pytest.mark.parametrize("n", [32768, 32769, 66000, 150001])
+def test_strided_layer_with_more_chunks_than_blocks(n):
+    """A strided layer's passes have at most 1024 blocks of 256 tickets (32 768 rows of a stride-2 layer), the tile cuts 512 of
+    256 rows: beyond, a block walks several chunks and carries the count in front of it along."""
+    layer = SPARSE_LAYERS[1]                                    # 32 -> 64: the narrowest layer that gets tile cuts
+    ig = sparse_input_grid(layer)
+    rng = np.random.default_rng(n)
+    coors = F.clustered_active_voxels(n, ig, n, n_blobs=n // 50)
+    feat = rng.uniform(-1, 1, (n, layer.cin)).astype(np.float32)
+    w = rng.normal(0, 0.1, (layer.kvol, layer.cin, layer.cout)).astype(np.float32)
+    mv = n + 37
+    O.set_threads(16)
+    try:
+        conv, out, oc, on, pairs, num = run_sparse(layer, coors, n, feat, w, mv, ig)
+        o_pairs, o_num, o_oc, o_on, o_st = O.sparse_rulebook(coors, n, layer.out_shape, layer.ksize, layer.stride, layer.padding, mv)
+        assert on == o_on and conv.status() == o_st
+        assert np.array_equal(oc, o_oc) and np.array_equal(num, o_num)
+        o_out = O.gather_gemm_scatter(feat, w, o_pairs, o_num, mv)
+        assert_features_close(out, o_out, RTOL_FP32, layer.name, abs_sum=abs_sum_of(feat, w, o_pairs, o_num, mv))
+        # (tile cuts of as many output rows)
+        sub = api.SubmConv3d(32, 64, ig[::-1], w, n)
+        cbuf = np.zeros((n, 4), np.int32)
+        cbuf[:] = coors
+        got = to_np(sub(dev(feat), dev(cbuf), dev(np.array([n], np.int32))))
+        s_pairs, s_num, _ = O.subm_rulebook(coors, n, ig[::-1], n)
+        want = O.gather_gemm_scatter(feat, w, s_pairs, s_num, n)
+        assert_features_close(got, want, RTOL_FP32, "subm, %d rows" % n, abs_sum=abs_sum_of(feat, w, s_pairs, s_num, n, n))
+    finally:
+        O.set_threads(1)
 
 
 def test_sparse_cap_overflow_and_empty():

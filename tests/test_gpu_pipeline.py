@@ -641,3 +641,40 @@ def test_a_voxel_grid_too_large_for_a_kept_table(monkeypatch):
             assert [pipe.layer_count(l) for l in range(-1, len(layers))] == list(ref["counts"]), step
             assert np.array_equal(pipe.read_layer(len(layers) - 1)[1], ref["coors"]), step
             assert_end_to_end_close(to_np(dense), ref["dense"], False, "dense, step %d" % step)
+
+
+@pytest.mark.parametrize("overlap", [True, False])
+def test_more_points_than_the_numbering_reads_one_by_one(overlap):
+    """A points tensor of more than 1 048 576 rows: the pass that numbers voxels goes by sums over 64 blocks' counts.  Three
+    frames, the second small."""
+    S, P = D.SESSD_LAYER_SUBM, D.SESSD_LAYER_SPARSE
+    layers = [B.Layer("subm0", S, 4, 16, (1408, 1600, 41), (3, 3, 3), (1, 1, 1), (1, 1, 1)),
+              B.Layer("sparse1", P, 16, 16, (704, 800, 21), (3, 3, 3), (2, 2, 2), (1, 1, 1)),
+              B.Layer("sparse2", P, 16, 16, (352, 400, 11), (3, 3, 3), (2, 2, 2), (1, 1, 1)),
+              B.Layer("sparse3", P, 16, 16, (176, 200, 5), (3, 3, 3), (2, 2, 2), (0, 1, 1)),
+              B.Layer("sparse4", P, 16, 16, (176, 200, 2), (3, 1, 1), (2, 1, 1), (0, 0, 0))]
+    W = B.random_weights(layers, seed=17, w_std=0.1)
+    mp, mv = 1500000, 280000
+    pipe = api.Pipeline(layers, W, mp, mv, share_rulebooks=True, skip_pad_rows=True, use_graph=overlap, overlap_streams=overlap)
+    p, n = points_input(np.zeros((0, 4), np.float32), mp)
+    dense, stream = pipe.new_dense(), torch.cuda.Stream()
+    O.set_threads(16)
+    try:
+        for step, npts in enumerate((mp, 5000, 1048577)):
+            pts = np.concatenate([F.lidar_frame(-(-npts // 4), 170 + 4 * step + i, full_circle=i > 1) for i in range(4)])[:npts]
+            hp, hn = points_input(pts, mp)
+            with torch.cuda.stream(stream):
+                p.copy_(hp)
+                n.copy_(hn)
+                pipe.enqueue(p, n, dense, stream)
+            stream.synchronize()
+            ref = O.frame(pts, B.voxelgen_desc(max_voxels=mv), layers, W, B.dense_desc(B.DENSE_SIZE_XYZ, 16))
+            assert pipe.status() == ref["status"]
+            assert [pipe.layer_count(l) for l in range(-1, len(layers))] == list(ref["counts"]), step
+            vox = O.voxelize(pts, B.POINT_CLOUD_RANGE, B.VOXEL_SIZE, 5, mv)
+            feat, coors, cnt = pipe.read_layer(-1)
+            assert np.array_equal(coors, vox[1][:cnt]) and np.array_equal(feat.view(np.uint32), vox[0][:cnt].view(np.uint32))
+            assert np.array_equal(pipe.read_layer(len(layers) - 1)[1], ref["coors"]), step
+            assert_end_to_end_close(to_np(dense), ref["dense"], False, "dense, step %d" % step)
+    finally:
+        O.set_threads(1)
