@@ -137,8 +137,12 @@ def _stream_ptr(stream=None):
     of host time instead of 2)."""
     if stream is not None:
         return stream.cuda_stream
-    c = _torch()._C
-    return c._cuda_getCurrentRawStream(c._cuda_getDevice())
+    torch = _torch()
+    c = torch._C
+    try:
+        return c._cuda_getCurrentRawStream(c._cuda_getDevice())
+    except AttributeError:  # (private names: a torch without them)
+        return torch.cuda.current_stream().cuda_stream
 
 
 def _ptr(t):

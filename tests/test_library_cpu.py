@@ -275,3 +275,15 @@ def test_voxelgen_static_enqueue_takes_every_size_it_is_documented_to_take(max_p
         ind[0] = D.TensorDesc.make([1, rows + 1, 4], D.SESSD_FLOAT)
         assert L.sessd_voxelgen_enqueue_static(vg.h, ind, outd, none, none, None) == D.SESSD_E_INVALID
         assert b"static buffer holds" in L.sessd_last_error()
+
+
+def test_current_stream_with_and_without_torchs_private_functions(monkeypatch):
+    """The wrapper reads the current stream through private functions of torch; one that lacks either is asked by its
+    public interface."""
+    from types import SimpleNamespace as N
+    public = N(current_stream=lambda: N(cuda_stream=77))
+    fast = dict(_cuda_getCurrentRawStream=lambda device: 1000 + device, _cuda_getDevice=lambda: 3)
+    for names, want in ((list(fast), 1003), (["_cuda_getDevice"], 77), (["_cuda_getCurrentRawStream"], 77), ([], 77)):
+        monkeypatch.setattr(api, "_torch", lambda: N(_C=N(**{k: fast[k] for k in names}), cuda=public))
+        assert api._stream_ptr() == want
+    assert api._stream_ptr(N(cuda_stream=5)) == 5 and api._stream_ptr(api.STREAM_NONE) == -1
