@@ -195,8 +195,14 @@ export_pairs(const int32_t* __restrict__ nbr, int max_voxels, int words_per_k,
 int launch_mfma(const GemmArgs& a, hipStream_t stream);  // conv_mfma.hip
 
 int launch_tall(const GemmArgs& a, hipStream_t stream);  // conv_tall.hip
+bool gemm_runs_tall(int K, int cin, int cout);
 int launch_tile(const GemmArgs& a, hipStream_t stream);  // conv_tile.hip
+bool gemm_runs_tile(int K, int cin, int cout);
 int launch_wide(const GemmArgs& a, hipStream_t stream);  // conv_wide.hip
+
+bool gemm_cuts_own_tiles(int K, int cin, int cout, int in_type, int out_type) {
+    return in_type == SESSD_HALF && out_type == SESSD_HALF && (gemm_runs_tile(K, cin, cout) || gemm_runs_tall(K, cin, cout));
+}
 
 int launch_gather_gemm(const GemmArgs& a, hipStream_t stream) {
     if (!a.force_valu) {  // FP16 layers from 32 channels up: one tile per compute unit, with Cin 32 tall tiles
@@ -204,7 +210,7 @@ int launch_gather_gemm(const GemmArgs& a, hipStream_t stream) {
         if (rc == SESSD_E_UNSUPPORTED) rc = launch_tall(a, stream);
         if (rc != SESSD_E_UNSUPPORTED) return rc;
     }
-    if (!a.force_valu) {  // FP32, 64 output columns: one tall tile per compute unit
+    if (!a.force_valu) {  // FP32, 64 or 128 output columns from 32 input channels up: one tall tile per compute unit
         const int rc = launch_wide(a, stream);
         if (rc != SESSD_E_UNSUPPORTED) return rc;
     }

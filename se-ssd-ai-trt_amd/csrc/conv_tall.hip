@@ -35,6 +35,11 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef unsigned int v4u32 __attribute__((__vector_size__(16)));
 
 constexpr int kWaves = 4;
+constexpr int KC = 27;          // kernel offsets: the 3x3x3 layers
+constexpr int D = 3;            // offsets the rows are requested ahead
+constexpr int DW = 2;           // register sets for weights in flight
+constexpr int kTallBlocks = 2;  // 16-row blocks a wave owns in a tall tile (one in a short tile: the heights are chosen on
+                                // the device from the row count)
 constexpr int kGroupsAhead = 3;  // groups of weight fragments a wave has requested from LDS ahead of the one it multiplies
 constexpr unsigned kOutOfRange = 0x80000000u;
 constexpr int kRawBuffer = 0x00020000;
@@ -67,9 +72,8 @@ __device__ __forceinline__ float4* weight_slot() {
     return s_w;
 }
 
-// The tile of one workgroup.  RB = 16-row blocks per wave, D = offsets the rows are requested ahead, DW = register
-// sets for weights in flight.
-template <int CIN, int COUT, int RB, int D, int DW, int KC>
+// The tile of one workgroup.  RB = 16-row blocks per wave.
+template <int CIN, int COUT, int RB>
 __device__ __forceinline__ void tall_tile(const __half* __restrict__ in, __half* __restrict__ out,
                                           const void* __restrict__ Wp, const int32_t* __restrict__ nbr, int n,
                                           int row0, int max_voxels, bool has_scale, bool has_shift, int relu,
@@ -263,15 +267,14 @@ __device__ __forceinline__ void tall_tile(const __half* __restrict__ in, __half*
     }
 }
 
-// RB = 16-row blocks a wave owns in a tall tile (one in a short tile: the heights are chosen on the device from
-// the row count), D = offsets the rows are requested ahead, DW = register sets for weights in flight
-template <int CIN, int COUT, int RB, int D, int DW, int KC>
+template <int CIN, int COUT>
 __global__ void __launch_bounds__(kWaves * 64, 2)
 conv_tall(const __half* __restrict__ in, __half* __restrict__ out, const void* __restrict__ Wp,
           const int32_t* __restrict__ nbr, const int32_t* __restrict__ num_out, int max_voxels,
           const float* __restrict__ scale, const float* __restrict__ shift, int relu, int write_pad,
           int slots, DenseTarget dt) {
     static_assert(CIN % 32 == 0 && COUT % 16 == 0, "whole MFMA chunks");
+    constexpr int RB = kTallBlocks;
     __shared__ int32_t s_nbr[KC * kWaves * RB * 16];
     __shared__ float s_epi[2 * COUT];
     int n = *num_out;
@@ -288,22 +291,22 @@ conv_tall(const __half* __restrict__ in, __half* __restrict__ out, const void* _
     // whole tile's time; beyond 64 * RB * slots rows every tile is tall.
     constexpr int kShort = kWaves * 16, kTall = kShort * RB;
     int n_tall = 0;
-    if (RB > 1 && n > kShort * slots) {
+    if (n > kShort * slots) {
         n_tall = (n - kShort * slots + (kTall - kShort) - 1) / (kTall - kShort);
         if (n_tall > slots) n_tall = (n + kTall - 1) / kTall;
     }
     const int b = blockIdx.x;
     if (b < n_tall)
-        tall_tile<CIN, COUT, RB, D, DW, KC>(in, out, Wp, nbr, n, b * kTall, max_voxels, scale != nullptr, shift != nullptr, relu, dt, s_nbr, s_epi);
+        tall_tile<CIN, COUT, RB>(in, out, Wp, nbr, n, b * kTall, max_voxels, scale != nullptr, shift != nullptr, relu, dt, s_nbr, s_epi);
     else
-        tall_tile<CIN, COUT, 1, D, DW, KC>(in, out, Wp, nbr, n, n_tall * kTall + (b - n_tall) * kShort, max_voxels, scale != nullptr, shift != nullptr, relu, dt, s_nbr, s_epi);
+        tall_tile<CIN, COUT, 1>(in, out, Wp, nbr, n, n_tall * kTall + (b - n_tall) * kShort, max_voxels, scale != nullptr, shift != nullptr, relu, dt, s_nbr, s_epi);
     if (write_pad) {
         __syncthreads();
         write_pad_rows<__half, COUT, kWaves * 64>(out, n, max_voxels, s_epi, scale != nullptr, shift != nullptr, relu);
     }
 }
 
-template <int CIN, int COUT, int RB, int D, int DW, int KC>
+template <int CIN, int COUT>
 int launch(const GemmArgs& a, hipStream_t stream) {
     if ((size_t)a.max_voxels * CIN * sizeof(__half) >= kOutOfRange) return SESSD_E_UNSUPPORTED;
     const int num_cu = gemm_compute_units();
@@ -312,11 +315,11 @@ int launch(const GemmArgs& a, hipStream_t stream) {
     static int per_cu = 0;
     if (per_cu == 0) {
         int v = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, conv_tall<CIN, COUT, RB, D, DW, KC>, kWaves * 64, 0) != hipSuccess || v < 1)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, conv_tall<CIN, COUT>, kWaves * 64, 0) != hipSuccess || v < 1)
             v = 2;
         per_cu = v;
     }
-    hipLaunchKernelGGL((conv_tall<CIN, COUT, RB, D, DW, KC>), dim3(blocks), dim3(kWaves * 64), 0, stream,
+    hipLaunchKernelGGL((conv_tall<CIN, COUT>), dim3(blocks), dim3(kWaves * 64), 0, stream,
                        static_cast<const __half*>(a.in_feat), static_cast<__half*>(a.out_feat), a.w_packed, a.nbr,
                        a.num_out, a.max_voxels, a.scale, a.shift, a.relu, a.write_pad_rows,
                        per_cu * num_cu, a.dense);
@@ -326,19 +329,13 @@ int launch(const GemmArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-bool gemm_runs_tall(int K, int cin, int cout, int in_type, int out_type) {
-    if (in_type != SESSD_HALF || out_type != SESSD_HALF) return false;
-    if (K == 3) return cin == cout && (cin == 64 || cin == 128);  // the (3,1,1) layer that ends the backbone
-    if (K != 27) return false;
-    return (cin == 128 && cout == 128) || (cin == 64 && (cout == 128 || cout == 64)) || (cin == 32 && (cout == 64 || cout == 32));
-}
+bool gemm_runs_tall(int K, int cin, int cout) { return K == KC && cin == 32 && (cout == 64 || cout == 32); }
 
 int launch_tall(const GemmArgs& a, hipStream_t stream) {
-    if (!a.w_packed || a.K != 27 || a.in_type != SESSD_HALF || a.out_type != SESSD_HALF) return SESSD_E_UNSUPPORTED;
+    if (!a.w_packed || a.K != KC || a.in_type != SESSD_HALF || a.out_type != SESSD_HALF) return SESSD_E_UNSUPPORTED;
     if ((reinterpret_cast<uintptr_t>(a.in_feat) | reinterpret_cast<uintptr_t>(a.out_feat)) & 15) return SESSD_E_UNSUPPORTED;
-    // <Cin, Cout, row blocks per wave in tall tiles, offsets the rows are requested ahead, weight register sets, K>
-    if (a.cin == 32 && a.cout == 64) return launch<32, 64, 2, 3, 2, 27>(a, stream);
-    if (a.cin == 32 && a.cout == 32) return launch<32, 32, 2, 3, 2, 27>(a, stream);
+    if (a.cin == 32 && a.cout == 64) return launch<32, 64>(a, stream);
+    if (a.cin == 32 && a.cout == 32) return launch<32, 32>(a, stream);
     return SESSD_E_UNSUPPORTED;
 }
 

@@ -356,10 +356,15 @@ int launch(const GemmArgs& a, hipStream_t stream) {
 
 }  // namespace
 
+// (K 3: the (3,1,1) layer that ends the backbone)
+bool gemm_runs_tile(int K, int cin, int cout) {
+    return K == 3 ? cin == cout && (cin == 64 || cin == 128) : K == 27 && (cin == 64 || cin == 128) && (cout == 128 || cout == cin);
+}
+
 int launch_tile(const GemmArgs& a, hipStream_t stream) {
     if (!a.w_packed || a.in_type != SESSD_HALF || a.out_type != SESSD_HALF) return SESSD_E_UNSUPPORTED;
     if ((reinterpret_cast<uintptr_t>(a.in_feat) | reinterpret_cast<uintptr_t>(a.out_feat)) & 15) return SESSD_E_UNSUPPORTED;
-    if (a.K == 3) {  // the (3,1,1) layer that ends the backbone
+    if (a.K == 3) {
         if (a.cin == 128 && a.cout == 128) return launch<128, 128, 3>(a, stream);
         if (a.cin == 64 && a.cout == 64) return launch<64, 64, 3>(a, stream);
     } else if (a.K == 27) {

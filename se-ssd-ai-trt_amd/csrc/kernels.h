@@ -74,7 +74,7 @@ int launch_gather_gemm(const GemmArgs& a, hipStream_t stream);
 bool gemm_runs_on_mfma(int K, int cin, int cout, int in_type, int out_type);
 // whether the layer runs on one of the FP16 kernels (conv_tile.hip, conv_tall.hip) that cut their own tiles: a rulebook
 // whose owner does needs no equal-work cuts
-bool gemm_runs_tall(int K, int cin, int cout, int in_type, int out_type);
+bool gemm_cuts_own_tiles(int K, int cin, int cout, int in_type, int out_type);
 // whether the layer runs on the FP32 kernel with one tall tile per compute unit (conv_wide.hip), and that kernel's
 // tile capacity
 bool gemm_runs_wide(int K, int cin, int cout, int in_type, int out_type);

@@ -119,7 +119,7 @@ class ConvPluginBase {
     bool wantTileCuts() const {
         return weights_packed_dev_ != nullptr && !(flags_ & SESSD_FLAG_FORCE_VALU) &&
                in_channel_ * out_channel_ >= kTileCutMinWork &&
-               !gemm_runs_tall(kernel_volume_, in_channel_, out_channel_, in_type_, out_type_);
+               !gemm_cuts_own_tiles(kernel_volume_, in_channel_, out_channel_, in_type_, out_type_);
     }
   protected:
     // tile height those cuts aim at: the capacity of this layer's own GEMM kernel
