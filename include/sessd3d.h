@@ -482,7 +482,9 @@ int sessd_pipeline_join(sessd_pipeline* h, int64_t ticket, sessd_stream_t stream
  * coupling.  Only with frames_in_flight >= 2. */
 int sessd_pipeline_wait(sessd_pipeline* h, int64_t ticket);
 /* Device pointers to the tensors a layer produced in the last enqueue (layer = -1: voxelizer).
- * feat: [max_voxels, C]; coors: i32[max_voxels,4]; voxel_num: i32[1]; workspace of that layer. */
+ * feat: [max_voxels, C]; coors: i32[max_voxels,4]; voxel_num: i32[1]; workspace of that layer.  Between frames the
+ * tensors are the caller's to overwrite: the next frame writes them anew and reads nothing of what they held.  The
+ * workspace is for sessd_*_export_rulebook and must not be written. */
 int sessd_pipeline_layer_io(sessd_pipeline* h, int layer, void** feat, void** coors,
                             void** voxel_num, void** workspace, int32_t* channels);
 /* Profiling variant of enqueue: records HIP events on `stream` around the voxelizer, around each

@@ -794,7 +794,14 @@ int sessd_pipeline_submit(sessd_pipeline* h, const void* points, const void* poi
             SESSD_HIP_TRY(hipEventRecord(R->ev_in, stream));
             SESSD_HIP_TRY(hipStreamWaitEvent(R->frame_stream, R->ev_in, 0));
         }
-        SESSD_TRY(run_frame(R, points, points_size, dense, R->frame_stream));
+        const int rc = run_frame(R, points, points_size, dense, R->frame_stream);
+        if (rc != SESSD_OK) {
+            // no join follows: what the call has left on the replica's stream (the clears; while the caller captures, a
+            // branch of that capture) is put in front of what comes next on the caller's
+            if (stream_ != SESSD_STREAM_NONE && hipEventRecord(R->ev_frame_done, R->frame_stream) == hipSuccess)
+                (void)hipStreamWaitEvent(stream, R->ev_frame_done, 0);
+            return rc;
+        }
         SESSD_HIP_TRY(hipEventRecord(R->ev_frame_done, R->frame_stream));
         P->last_replica = r;
     }

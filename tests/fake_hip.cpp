@@ -18,12 +18,18 @@ namespace {
 struct Stream {
     bool capturing = false;
     Stream* origin = nullptr;   // of the capture it takes part in
-    std::set<Stream*> unjoined;  // (origin) streams that the capture has forked to and not come back from
+    std::set<Stream*> open;     // (origin) streams with captured work that no other stream has waited for
+    long ops = 0;               // launches and waits so far
+    void did() {
+        ++ops;
+        if (capturing && origin != this) origin->open.insert(this);
+    }
 };
 struct Event {
     int id;
     Stream* on = nullptr;
     bool captured = false;
+    long at = 0;  // of on->ops
 };
 
 std::string& log_text() {
@@ -123,6 +129,8 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipSt
 hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void**, size_t, hipStream_t s) {
     if (grid.x == 0) return report(hipErrorInvalidConfiguration);
     note("launch", kernels()[f].c_str(), number(stream_of(s)));
+    Own own;
+    stream_of(s)->did();
     const long i = launches++;
     if (fail_from >= 0 && i >= fail_from && i < fail_to) return report(hipErrorUnknown);
     return hipSuccess;
@@ -191,13 +199,13 @@ hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g) {
     Stream* st = stream_of(s);
     *g = nullptr;
     if (!st->capturing) return report(hipErrorIllegalState);
-    const bool open = !st->unjoined.empty();
+    const bool open = !st->open.empty();
     for (auto& other : streams())
         if (other.first->origin == st) {
             other.first->capturing = false;
             other.first->origin = nullptr;
         }
-    st->unjoined.clear();
+    st->open.clear();
     if (open) return report(hipErrorStreamCaptureUnjoined);
     *g = reinterpret_cast<hipGraph_t>(&default_stream());  // (only compared with null)
     return hipSuccess;
@@ -219,6 +227,7 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
     Event* ev = reinterpret_cast<Event*>(e);
     ev->on = stream_of(s);
     ev->captured = ev->on->capturing;
+    ev->at = ev->on->ops;
     note("record", ev->id, number(ev->on));
     return hipSuccess;
 }
@@ -232,8 +241,8 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned int) {
             st->capturing = true;
             st->origin = ev->on->origin;
         }
-        if (st == st->origin) st->unjoined.erase(ev->on);
-        else st->origin->unjoined.insert(st);
+        if (ev->at == ev->on->ops) st->origin->open.erase(ev->on);
+        st->did();
     } else if (st->capturing) {
         return report(hipErrorStreamCaptureIsolation);
     }

@@ -136,10 +136,10 @@ def check_clear_that_failed_too(overlap):
     assert len(launches_of(enqueue, h, stream)) == len(plain)
 
 
-def check_capture(overlap):
+def check_capture(overlap, replicas=0):
     """A call that fails while the caller captures: nothing has run, so nothing is cleared, and the capture can be ended
     (no branch of it is left open)."""
-    rc, h = create(overlap_streams=overlap)
+    rc, h = create(overlap_streams=overlap, frames_in_flight=replicas)
     stream = new_stream()
     n = len(launches_of(enqueue, h, stream))
     graph = C.c_void_p()
@@ -151,6 +151,22 @@ def check_capture(overlap):
         assert len(launches(take_log())) == i + 1, i
         assert FAKE.hipStreamEndCapture(stream, C.byref(graph)) == 0, i
         assert len(launches_of(enqueue, h, stream)) == n, i
+
+
+def check_in_flight():
+    """Frames in flight: the clears behind a failed frame are on the replica's stream, and the caller's waits for them."""
+    rc, h = create(overlap_streams=1, frames_in_flight=2)
+    stream = new_stream()
+    n = len(launches_of(enqueue, h, stream))
+    for i in range(n):
+        FAKE.fake_fail_launches(i, 1)
+        assert enqueue(h, stream) == D.SESSD_E_HIP
+        FAKE.fake_fail_launches(-1, 0)
+        log = take_log()
+        assert is_fill(launches(log)[-1])
+        # (a launch on the caller's stream would come behind all of it)
+        assert not unordered(log + [["launch", "next", str(FAKE.fake_stream_number(stream))]]), i
+        assert len(launches_of(enqueue, h, stream)) == n
 
 
 def check_own_graph():
@@ -233,6 +249,8 @@ CHECKS = {
     "clear-failed-overlap": lambda: check_clear_that_failed_too(1),
     "capture-direct": lambda: check_capture(0),
     "capture-overlap": lambda: check_capture(1),
+    "capture-in-flight": lambda: check_capture(1, 2),
+    "in-flight": check_in_flight,
     "own-graph": check_own_graph,
     "short-memory": check_short_memory,
     "host-memory": check_host_memory,

@@ -28,7 +28,7 @@ def run_check(fake_hip, check):
 
 
 @pytest.mark.parametrize("check", ["recovery-direct", "recovery-overlap", "recovery-timed", "clear-failed-direct", "clear-failed-overlap",
-                                   "capture-direct", "capture-overlap", "own-graph"])
+                                   "capture-direct", "capture-overlap", "capture-in-flight", "in-flight", "own-graph"])
 def test_failed_calls_leave_the_cell_tables_empty(fake_hip, check):
     run_check(fake_hip, check)
 
