@@ -12,7 +12,7 @@
 //
 // A pass that creates rows (vg_finalize, sp_number) holds their coordinates and numbers in registers: it inserts the
 // next strided layer's tickets right away, and what only needs finished tables (lookups, cuts) shares a launch with the
-// next step of the chain.  For the reference's backbone that is 12 launches a frame in place of 35.
+// next step of the chain.  For the reference's backbone that is 13 launches a frame in place of 35.
 // Measured (a graph of the coordinate passes alone, us): frames of 2 000 points 141 -> 79, 20 000 164 -> 97, 80 000 231 ->
 // 127, 60 000 (FP16 configuration) 162 -> 111, 150 000 221 -> 147.  A pass is bound by its chain of dependent trips to
 // memory (four to six of 0.7-1 us each) until some 40 000 rows, and by random accesses beyond.
