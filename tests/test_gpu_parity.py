@@ -755,7 +755,8 @@ def test_conv_plugins_by_name_and_their_clones():
 
 
 # ---------------------------------------------------------------------------------------------
-# the tall-tile FP16 kernel (3x3x3 layers from 32 channels up): tile edges and both tile heights
+# the FP16 kernels that cut their own tiles (3x3x3 layers from 32 channels up): with 32 input channels the tall-tile kernel
+# (conv_tall.hip), from 64 up the ring of LDS buffers (conv_tile.hip); tile edges and tile heights
 # ---------------------------------------------------------------------------------------------
 def _fp16_subm_against_oracle(cin, cout, n, mv, grid, seed, clustered=True, epilogue=True):
     rng = np.random.default_rng(seed)
@@ -786,19 +787,31 @@ def _fp16_subm_against_oracle(cin, cout, n, mv, grid, seed, clustered=True, epil
 @pytest.mark.parametrize("cin,cout", [(32, 32), (64, 64), (128, 128)])
 @pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 300])
 def test_tall_fp16_kernel_row_counts_around_its_tiles(cin, cout, n):
-    """A tile of the tall-tile kernel is 64 rows, 16 per wave: row counts on either side of a block, a wave's
-    share and a tile, down to a single row, against the oracle (pad rows included)."""
+    """A tile of the tall-tile kernel is 64 rows, 16 per wave (32 -> 32), one of the ring kernel 64 or 32 at these row counts:
+    row counts on either side of a block, a wave's share and a tile, down to a single row, against the oracle (pad rows
+    included)."""
     _fp16_subm_against_oracle(cin, cout, n, 512, (5, 40, 40), 900 + n, epilogue=(n % 2 == 1))
 
 
 @pytest.mark.parametrize("cin,cout,n", [(32, 32, 66000), (64, 64, 40000), (64, 128, 66000), (128, 128, 40000), (128, 128, 66000)])
 def test_tall_fp16_kernel_with_two_row_blocks_per_wave(cin, cout, n):
-    """Beyond 64 rows x the workgroups resident at a time, tiles at the head of the grid take two 16-row blocks per
-    wave (128 rows): a launch with short and tall tiles side by side (40 000 rows) and one with tall tiles only
-    (66 000 rows, the last tile partly filled), against the oracle on 16 threads."""
+    """Launches of many rows, the last tile partly filled, against the oracle on 16 threads: short tiles only on the
+    tall-tile kernel (32 -> 32; its tall tiles: the test below), tiles of several blocks a wave on the ring kernel."""
     O.set_threads(16)
     try:
         _fp16_subm_against_oracle(cin, cout, n, 66560, (21, 400, 352), 4000 + cin + cout)
+    finally:
+        O.set_threads(1)
+
+
+@pytest.mark.parametrize("cout,n", [(32, 81920), (32, 81921), (32, 120000), (32, 163841), (64, 65536), (64, 65537), (64, 100000), (64, 131073)])
+def test_tall_fp16_kernel_with_tall_tiles(cout, n):
+    """Beyond 64 rows x the workgroups resident at a time (1280 of the 32 -> 32 kernel, 1024 of 32 -> 64 by their registers on
+    256 compute units), tiles at the head of the grid take two 16-row blocks per wave (128 rows): the last launch of
+    short tiles, one with a single tall tile, short and tall ones side by side, and tall ones only."""
+    O.set_threads(16)
+    try:
+        _fp16_subm_against_oracle(32, cout, n, n + 70, (41, 400, 352), 8000 + cout)
     finally:
         O.set_threads(1)
 
@@ -843,6 +856,28 @@ def test_fp16_ring_kernel_gives_the_same_bits_launch_after_launch(cin, cout, n):
         bad += (op(*args, rulebook_from=conv).view(torch.int16) != first).sum()
     torch.cuda.synchronize()
     assert int(bad) == 0
+
+
+@pytest.mark.parametrize("channels,n", [(64, 5000), (64, 40000), (128, 20000)])
+def test_fp16_ring_kernel_of_the_last_layer_gives_the_same_bits_launch_after_launch(channels, n):
+    """The same for the 3x1x1 layer that ends the backbone, whose whole walk is three offsets: 400 calls, each with its
+    rulebook built anew."""
+    layer = SPARSE_LAYERS[3]
+    ig = sparse_input_grid(layer)
+    coors = F.clustered_active_voxels(n, ig, 7300 + n, n_blobs=n // 100)
+    rng = np.random.default_rng(n)
+    cbuf = np.zeros((n, 4), np.int32)
+    cbuf[:, :] = coors
+    args = (dev(rng.uniform(-1, 1, (n, channels)).astype(np.float32), torch.float16), dev(cbuf), dev(np.array([n], np.int32)))
+    w = rng.normal(0, 0.1, (3, channels, channels)).astype(np.float32)
+    op = api.SparseConv3d(channels, channels, layer.out_shape, ig[::-1], layer.ksize, layer.stride, layer.padding, w, n)
+    first, fc, fn = op(*args)
+    bad = torch.zeros((), dtype=torch.int64, device="cuda:0")
+    for _ in range(400):
+        out, oc, on = op(*args)
+        bad += (out.view(torch.int16) != first.view(torch.int16)).sum() + (oc != fc).sum() + (on != fn).sum()
+    torch.cuda.synchronize()
+    assert int(bad) == 0 and int(fn[0]) > 0
 
 
 # ---------------------------------------------------------------------------------------------

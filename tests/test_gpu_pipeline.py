@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import oracle_lib as O
-from gpu_util import (RTOL_FP16, RTOL_FP32, assert_end_to_end_close, assert_features_close, canonical, layer_abs_sum,
+from gpu_util import (RTOL_FP16, RTOL_FP32, assert_end_to_end_close, assert_features_close, canonical, dev, layer_abs_sum,
                       points_input, to_np)
 from sessd3d import api, backbone as B, ctypes_defs as D, frames as F
 
@@ -385,9 +385,9 @@ def test_frames_in_flight_give_the_bits_of_one_frame_at_a_time():
 
 
 def test_fp16_stack_ending_in_a_3x3x3_layer_scatters_from_the_tall_tile_kernel():
-    """A stack whose LAST layer is a 3x3x3 FP16 layer of 32+ channels: in the overlapped schedule that layer's
-    kernel (the tall-tile one) also writes the dense tensor.  Dense tensor, sites and status against the oracle,
-    and equal to the single-stream schedule's separate scatter bit for bit."""
+    """A stack whose LAST layer is a 3x3x3 FP16 layer of 32 channels: that layer's kernel (the tall-tile one) also writes
+    the dense tensor, in both schedules.  Dense tensor, sites and status against the oracle, and each schedule's tensor
+    equal to a scatter of its last layer's rows and to the plugin's cell-major pass over them bit for bit."""
     S, P = D.SESSD_LAYER_SUBM, D.SESSD_LAYER_SPARSE
     layers = [B.Layer("subm0", S, 4, 32, (1408, 1600, 41), (3, 3, 3), (1, 1, 1), (1, 1, 1)),
               B.Layer("sparse1", P, 32, 64, (704, 800, 21), (3, 3, 3), (2, 2, 2), (1, 1, 1)),
@@ -408,6 +408,15 @@ def test_fp16_stack_ending_in_a_3x3x3_layer_scatters_from_the_tall_tile_kernel()
     assert np.array_equal(fused.read_layer(len(layers) - 1)[1], ref["coors"])
     assert_end_to_end_close(to_np(d_fused).astype(np.float32), want, True, "dense from the tall-tile kernel")
     assert torch.equal(d_fused, d_plain)
+    for pipe, d in ((fused, d_fused), (plain, d_plain)):
+        feat, coors, m = pipe.read_layer(len(layers) - 1)
+        assert np.array_equal(to_np(d).astype(np.float32), O.zero_pad2d(O.sparse2dense(feat, coors, m, dsize), 1, 1, 1, 1))
+    rows, cbuf = np.zeros((mv, 32), np.float32), np.zeros((mv, 4), np.int32)
+    rows[:m], cbuf[:m] = feat, coors
+    s2d = api.Sparse2Dense(dsize, 32, padding=(1, 1, 1, 1))
+    as_plugin = s2d(dev(rows, torch.float16), dev(cbuf), dev(np.array([m], np.int32)))
+    torch.cuda.synchronize()
+    assert torch.equal(as_plugin.view(torch.int16).reshape(d_plain.shape), d_plain.view(torch.int16))
 
 
 @pytest.mark.parametrize("overlap", [True, False])

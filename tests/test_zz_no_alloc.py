@@ -64,7 +64,7 @@ def test_static_scratch_voxelizer_raises_the_same_flags_and_handles_a_second_han
 def test_static_scratch_voxelizer_rejects_what_does_not_fit():
     vg = api.VoxelGenerator(max_voxels=60000)
     pts = F.lidar_frame(1000, 1)
-    ins = list(points_input(pts, 150000))                         # 14.7 MB of scratch: beyond the 8 MiB array
+    ins = list(points_input(pts, 150000))                         # 11.4 MB of scratch: beyond the 8 MiB array
     outs = outputs(60000, 5)
     vg.configure(ins, outs)
     with pytest.raises(api.SessdError, match="static buffer holds"):
