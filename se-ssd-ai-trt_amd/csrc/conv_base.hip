@@ -28,8 +28,9 @@ int ConvPluginBase::uploadWeights(const float* w, size_t count) {
     weights_size_ = (int)count;
     SESSD_HIP_TRY(hipMalloc(reinterpret_cast<void**>(&weights_dev_), count * sizeof(float)));
     SESSD_HIP_TRY(hipMemcpy(weights_dev_, w, count * sizeof(float), hipMemcpyHostToDevice));
-    std::vector<__half> h(count);
-    for (size_t i = 0; i < count; ++i) h[i] = __float2half_rn(w[i]);
+    std::vector<uint16_t> h(count);
+    float value;
+    for (size_t i = 0; i < count; ++i) h[i] = nearest_half(w[i], &value);
     SESSD_HIP_TRY(hipMalloc(reinterpret_cast<void**>(&weights_half_dev_), count * sizeof(__half)));
     SESSD_HIP_TRY(hipMemcpy(weights_half_dev_, h.data(), count * sizeof(__half), hipMemcpyHostToDevice));
     packed_dtype_ = -1;
@@ -97,12 +98,13 @@ int ConvPluginBase::preparePacked() {
 
 bool ConvPluginBase::gemmOnMatrixCores() const {
     return weights_packed_dev_ != nullptr && !(flags_ & SESSD_FLAG_FORCE_VALU) &&
-           gemm_runs_on_mfma(kernel_volume_, in_channel_, out_channel_, in_type_, out_type_);
+           gemm_runs_on_mfma(kernel_volume_, in_channel_, out_channel_, in_type_, out_type_) &&
+           (in_type_ == SESSD_HALF || max_voxels_ < 1 << 24);  // (a pair of conv_wide.hip keeps its input row in 24 bits)
 }
 
 int ConvPluginBase::tileRows() const { return gemm_tile_rows(in_channel_, out_channel_, out_type_); }
 int ConvPluginBase::tilesWide() const {
-    return gemm_runs_wide(kernel_volume_, in_channel_, out_channel_, in_type_, out_type_) ? out_channel_ / 64 : 0;
+    return gemm_runs_wide(kernel_volume_, in_channel_, out_channel_, in_type_, out_type_) ? (out_channel_ > 64 ? out_channel_ / 64 : 1) : 0;
 }
 int ConvPluginBase::tileRowWeight() const { return tilesWide() ? 4 : 20; }
 

@@ -210,7 +210,7 @@ int launch_gather_gemm(const GemmArgs& a, hipStream_t stream) {
         if (rc == SESSD_E_UNSUPPORTED) rc = launch_tall(a, stream);
         if (rc != SESSD_E_UNSUPPORTED) return rc;
     }
-    if (!a.force_valu) {  // FP32, 64 or 128 output columns from 32 input channels up: one tall tile per compute unit
+    if (!a.force_valu) {  // FP32, and the first layer of an FP16 pipeline
         const int rc = launch_wide(a, stream);
         if (rc != SESSD_E_UNSUPPORTED) return rc;
     }

@@ -1,4 +1,5 @@
-// conv_mfma.hip -- gather-GEMM on the matrix cores (gfx950 MFMA), FP32 or FP16 features, FP32 accumulate.
+// conv_mfma.hip -- gather-GEMM of FP16 features on the matrix cores (gfx950 MFMA), FP32 accumulate: layers with fewer than 32 input
+// channels, and kernel volumes that conv_tall.hip and conv_tile.hip do not take.
 //
 //     out[o][:] = epilogue( sum_k  in[nbr[k][o]][:] @ W[k] )
 //
@@ -14,15 +15,12 @@
 //     16-pair blocks and dealt back and forth (0 1 2 3 3 2 1 0 ...): tiles x 4 waves is what fills 256 CUs
 //     with a ~17k-row problem.
 //   * A wave gathers 16 pairs per MFMA block straight into operand registers: lane (i = lane%16,
-//     q = lane/16) loads 16 bytes of pair i's input row per K-chunk (FP32: channels 16g+4q..+3, FP16:
-//     channels 32g+8q..+7), i.e. every row is read as 64-byte segments.  The weights were reordered on
-//     the host so that the other operand of the same MFMA steps is one 16-byte load per lane as well;
+//     q = lane/16) loads 16 bytes of pair i's input row per K-chunk (channels 32g+8q..+7).  The weights were reordered
+//     on the host so that the other operand of the same MFMA steps is one 16-byte load per lane as well;
 //     one pass over W[k] serves all blocks of the offset.  The next offset's rows are loaded at the top
 //     of the current one, and the weight registers of chunk g are refilled with the next offset's chunk g
-//     as soon as the MFMAs that read them have issued.  The FP32 kernels issue all of these as buffer loads
-//     outside any branch (a request with nothing to fetch points out of range), so that the waits the
-//     compiler inserts cover exactly the operands about to be used.
-//   * FP32: v_mfma_f32_16x16x4_f32; FP16: v_mfma_f32_16x16x32_f16 (16x16x16 for Cin = 16).  The weights
+//     as soon as the MFMAs that read them have issued.
+//   * v_mfma_f32_16x16x32_f16 (16x16x16 for Cin = 16).  The weights
 //     are the MFMA's A operand and the gathered rows its B operand, so a lane ends up with four
 //     consecutive output channels of one pair; the block is then added into the wave's private partial
 //     tile in LDS at the pairs' output rows with 16-byte read-modify-writes (only this wave touches its
@@ -46,50 +44,18 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr int kWaves = 4;           // wave64s per workgroup
 constexpr int kTileRowsBase = 48;   // tile capacity of most kernel instantiations
-constexpr int kTileRowsWideF16 = 64;  // ... and of the wide FP16 ones
+constexpr int kTileRowsWide = 64;   // ... and of the wide ones
 constexpr int kMaxK = kGemmMaxOffsets;
 
 // Tile capacity: most output rows a workgroup can own (<= 64: one wave stages a neighbour list).  The rows
-// of all blocks of two offsets live in registers, so the capacity is what the register file allows: 48 rows
-// for FP32 (64 spill in the 64-wide layers), 64 for the wide FP16 layers, whose rows take half the registers
-// and whose launches are short enough for one tile per CU less to show.  The narrow FP16 layers and
-// Cin = 128 measured slower with 64.
-constexpr int tile_rows(bool half_operands, int cin, int cout) {
-    return half_operands && cin <= 64 && cin * cout >= 32 * 64 ? kTileRowsWideF16 : kTileRowsBase;
-}
+// of all blocks of two offsets live in registers, so the capacity is what the register file allows: 64 rows in the wide
+// layers; the narrow ones and Cin = 128 measured slower with 64 than with 48.
+constexpr int tile_rows(int cin, int cout) { return cin <= 64 && cin * cout >= 32 * 64 ? kTileRowsWide : kTileRowsBase; }
 
-// Per-dtype shape of one K-chunk: how many channels it spans, what a lane holds of it, and the MFMA
-// sequence that consumes it (w = weights fragment -> A operand, x = gathered-row fragment -> B operand).
-template <typename T, int CIN>
-struct Chunk;
-
+// Shape of one K-chunk: how many channels it spans, what a lane holds of it, and the MFMA that consumes it (w = weights fragment
+// -> A operand, x = gathered-row fragment -> B operand).
 template <int CIN>
-struct Chunk<float, CIN> {
-    using Vec = float4;  // 4 channels
-    static constexpr int kChannels = 16, kLaneElems = 4;
-    static __device__ __forceinline__ Vec zero() { return make_float4(0.f, 0.f, 0.f, 0.f); }
-    static __device__ __forceinline__ void mma(const Vec& w, const Vec& x, v4f& acc) {
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x, x.x, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w.y, x.y, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w.z, x.z, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w.w, x.w, acc, 0, 0, 0);
-    }
-};
-
-// Cin = 4 (the voxel means entering the first layer): the whole inner dimension of an offset is one MFMA
-// K-step, a lane holds a single channel
-template <>
-struct Chunk<float, 4> {
-    using Vec = float;
-    static constexpr int kChannels = 4, kLaneElems = 1;
-    static __device__ __forceinline__ Vec zero() { return 0.f; }
-    static __device__ __forceinline__ void mma(const Vec& w, const Vec& x, v4f& acc) {
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w, x, acc, 0, 0, 0);
-    }
-};
-
-template <int CIN>
-struct Chunk<__half, CIN> {
+struct Chunk {
     using Vec = float4;  // 8 halfs = channels 32g+8q .. +7
     static constexpr int kChannels = 32, kLaneElems = 8;
     static __device__ __forceinline__ Vec zero() { return make_float4(0.f, 0.f, 0.f, 0.f); }
@@ -100,7 +66,7 @@ struct Chunk<__half, CIN> {
 };
 
 template <>
-struct Chunk<__half, 16> {
+struct Chunk<16> {
     using Vec = float2;  // 4 halfs = channels 4q .. +3
     static constexpr int kChannels = 16, kLaneElems = 4;
     static __device__ __forceinline__ Vec zero() { return make_float2(0.f, 0.f); }
@@ -110,30 +76,9 @@ struct Chunk<__half, 16> {
     }
 };
 
-// Buffer loads (FP32 kernels): a lane whose offset lies beyond the buffer gets zeros and no memory is touched,
-// so a request that has nothing to fetch needs no branch around it.
-typedef unsigned int v4u32 __attribute__((__vector_size__(16)));
-constexpr unsigned kOutOfRange = 0x80000000u;   // beyond any buffer the kernel is given (launch() checks)
-constexpr int kRawBuffer = 0x00020000;          // descriptor word 3: raw 32-bit data format, no swizzle
-template <typename Vec>
-__device__ __forceinline__ Vec buffer_load(__amdgpu_buffer_rsrc_t r, unsigned byte_offset) {
-    if constexpr (sizeof(Vec) == 16) {
-        v4u32 v = __builtin_amdgcn_raw_buffer_load_b128(r, byte_offset, 0, 0);
-        return *reinterpret_cast<Vec*>(&v);
-    } else {
-        static_assert(sizeof(Vec) == 4, "FP32 operands are 16 bytes per lane, or 4 when Cin = 4");
-        unsigned v = __builtin_amdgcn_raw_buffer_load_b32(r, byte_offset, 0, 0);
-        return *reinterpret_cast<Vec*>(&v);
-    }
-}
-
-__device__ __forceinline__ void store1(float* dst, float v) { *dst = v; }
 __device__ __forceinline__ void store1(__half* dst, float v) { *dst = __float2half_rn(v); }
 
 // four consecutive output channels -> memory
-__device__ __forceinline__ void store4(float* dst, const float (&o)[4]) {
-    *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
-}
 __device__ __forceinline__ void store4(__half* dst, const float (&o)[4]) {
     union {
         __half2 h[2];
@@ -150,16 +95,14 @@ constexpr int min_waves_per_simd(int cin, int cout) {
     return cin * cout >= 32 * 64 ? 2 : (cin * cout >= 32 * 32 ? 3 : 4);
 }
 
-// T = type of the input features and of the arithmetic's operands, TO = type the output rows are stored
-// in (differs only for the first layer of an FP16 pipeline: FP32 voxel means in, FP16 features out), PAD: the rows
-// beyond the active ones are written too
-template <typename T, int CIN, int COUT, typename TO, bool PAD>
+// PAD: the rows beyond the active ones are written too
+template <int CIN, int COUT, bool PAD>
 __global__ void __launch_bounds__(kWaves * 64, min_waves_per_simd(CIN, COUT))
-conv_mfma(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict__ Wp,
+conv_mfma(const __half* __restrict__ in, __half* __restrict__ out, const void* __restrict__ Wp,
           const int32_t* __restrict__ nbr, const int32_t* __restrict__ num_out, int max_voxels, int K,
           const float* __restrict__ scale, const float* __restrict__ shift, int relu, int num_cu,
           const int32_t* __restrict__ tiles, DenseTarget dt) {
-    using C = Chunk<T, CIN>;
+    using C = Chunk<CIN>;
     using Vec = typename C::Vec;
     constexpr int G = CIN / C::kChannels;  // K-chunks of the inner dimension
     constexpr int NBT = COUT / 16;         // 16-column blocks of the layer
@@ -173,7 +116,7 @@ conv_mfma(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
     constexpr int CW = COUT / CS;            // columns of one wave
     constexpr int LDP = CW + 4;              // padded row stride of the partial tiles in LDS
     static_assert(CIN % C::kChannels == 0 && COUT % 16 == 0, "channel counts must fill whole MFMA chunks");
-    constexpr int kTileRows = tile_rows(sizeof(T) == 2, CIN, COUT);
+    constexpr int kTileRows = tile_rows(CIN, COUT);
     constexpr int kMaxBlk = (kTileRows + 15) / 16;  // MFMA row blocks an offset can need
     static_assert(kGemmMinTileRows <= kTileRows && kTileRows <= 64, "capacity: at least the bound the grid is sized with, at most one wave");
     __shared__ int32_t s_in[kMaxK * kTileRows];   // compacted pair lists: input row ...
@@ -278,56 +221,29 @@ conv_mfma(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
         my_mask = (uint32_t)__ballot(b > 0 && w == kgrp);
     }
 
-    // FP32: every load of the main loop is a buffer load outside any branch -- padding lanes, absent blocks and
-    // the requests behind the last offset get an out-of-range offset.  Straight-line requests are what lets
-    // the compiler count the loads in flight exactly (s_waitcnt vmcnt counts in issue order; one load under a
-    // branch and every later wait becomes a wait for nearly everything, the operands just requested
-    // included).  64->64: 37 -> 33 us.  FP16 measured 1-2 % slower this way and keeps plain loads.
-    constexpr bool kBuf = sizeof(T) == 4;
-    __amdgpu_buffer_rsrc_t rs_in, rs_w;
-    if constexpr (kBuf) {
-        rs_in = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(in), 0, (int)((size_t)max_voxels * CIN * sizeof(T)),
-                                                  kRawBuffer);
-        rs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(Wp), 0,
-                                                 (int)((size_t)K * G * NBT * 64 * sizeof(Vec)), kRawBuffer);
-    }
     // gathered rows of all blocks of offset k -> operand registers (zeros for the padding pairs); cnt = 0:
     // nothing to fetch
     auto load_a_block = [&](int k, int cnt, int blk, Vec (&a)[kMaxBlk][G]) {
         const int j = blk * 16 + i;
         const bool live = j < cnt;
-        if constexpr (kBuf) {
-            const int idx = s_in[k * kTileRows + (live ? j : 0)];
-            const unsigned at = live ? (unsigned)((idx * CIN + q * C::kLaneElems) * (int)sizeof(T)) : kOutOfRange;
+        const int idx = live ? s_in[k * kTileRows + j] : 0;
+        const __half* src = in + (size_t)idx * CIN + q * C::kLaneElems;
 #pragma unroll
-            for (int g = 0; g < G; ++g) a[blk][g] = buffer_load<Vec>(rs_in, at + g * C::kChannels * (unsigned)sizeof(T));
-        } else {
-            const int idx = live ? s_in[k * kTileRows + j] : 0;
-            const T* src = in + (size_t)idx * CIN + q * C::kLaneElems;
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                Vec v = C::zero();
-                if (live) v = *reinterpret_cast<const Vec*>(src + g * C::kChannels);
-                a[blk][g] = v;
-            }
+        for (int g = 0; g < G; ++g) {
+            Vec v = C::zero();
+            if (live) v = *reinterpret_cast<const Vec*>(src + g * C::kChannels);
+            a[blk][g] = v;
         }
     };
     auto load_a = [&](int k, int cnt, Vec (&a)[kMaxBlk][G]) {
 #pragma unroll
         for (int blk = 0; blk < kMaxBlk; ++blk) load_a_block(k, cnt, blk, a);
     };
-    // chunk g of W[k] -> operand registers (buffer path: k < 0 = nothing to fetch)
+    // chunk g of W[k] -> operand registers
     auto load_b = [&](int k, int g, Vec (&b)[NB]) {
-        if constexpr (kBuf) {
-            const unsigned at = k >= 0 ? (unsigned)(((((k * G + g) * NBT + chalf * NB) * 64) + lane) * (int)sizeof(Vec))
-                                       : kOutOfRange;
+        const Vec* wk = wp + (((size_t)k * G + g) * NBT + chalf * NB) * 64;
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) b[nb] = buffer_load<Vec>(rs_w, at + nb * 64 * (unsigned)sizeof(Vec));
-        } else {
-            const Vec* wk = wp + (((size_t)k * G + g) * NBT + chalf * NB) * 64;
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) b[nb] = wk[nb * 64];
-        }
+        for (int nb = 0; nb < NB; ++nb) b[nb] = wk[nb * 64];
     };
 
     int k_cur = my_mask ? __ffs(my_mask) - 1 : -1;
@@ -343,19 +259,14 @@ conv_mfma(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
     while (k_cur >= 0) {
         const int k_nxt = my_mask ? __ffs(my_mask) - 1 : -1;
         my_mask &= my_mask - 1;
-        if constexpr (kBuf) {
-            // (the next offset's rows are requested block by block between the chunks below)
-            cnt_nxt = k_nxt >= 0 ? __builtin_amdgcn_readfirstlane(s_cnt[k_nxt]) : 0;  // wave-uniform: keep it scalar
-        } else {
-            // Everything requested during the previous offset is consumed by this one: wait for all of it here,
-            // before this offset's own requests go out.  Left to itself the compiler waits chunk by chunk, and
-            // because some requests sit under branches its count is inexact: the wait before the second chunk
-            // then also covers the rows and weights requested a moment ago for the NEXT offset.
-            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-            if (k_nxt >= 0) {
-                cnt_nxt = __builtin_amdgcn_readfirstlane(s_cnt[k_nxt]);
-                load_a(k_nxt, cnt_nxt, a_nxt);
-            }
+        // Everything requested during the previous offset is consumed by this one: wait for all of it here,
+        // before this offset's own requests go out.  Left to itself the compiler waits chunk by chunk, and
+        // because some requests sit under branches its count is inexact: the wait before the second chunk
+        // then also covers the rows and weights requested a moment ago for the NEXT offset.
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+        if (k_nxt >= 0) {
+            cnt_nxt = __builtin_amdgcn_readfirstlane(s_cnt[k_nxt]);  // wave-uniform: keep it scalar
+            load_a(k_nxt, cnt_nxt, a_nxt);
         }
         v4f acc[kMaxBlk][NB];
 #pragma unroll
@@ -370,16 +281,8 @@ conv_mfma(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) C::mma(b[g][nb], a_cur[blk][g], acc[blk][nb]);
             }
-            // The next offset's chunk g replaces this one, without a branch: FP32 asks out of range after the
-            // last offset, FP16 asks for the same chunk once more.
-            if constexpr (kBuf) load_b(k_nxt, g, b[g]);
-            else load_b(k_nxt >= 0 ? k_nxt : k_cur, g, b[g]);
-            // FP32: the next offset's rows follow, one block behind each chunk, instead of all at the top of the
-            // offset: the address unit sees the requests spread over the offset (frame 0.396 -> 0.390 ms)
-            if constexpr (kBuf) {
-#pragma unroll
-                for (int blk = g; blk < kMaxBlk; blk += G) load_a_block(k_nxt >= 0 ? k_nxt : 0, cnt_nxt, blk, a_nxt);
-            }
+            // the next offset's chunk g replaces this one, without a branch: behind the last offset the same chunk once more
+            load_b(k_nxt >= 0 ? k_nxt : k_cur, g, b[g]);
         }
         // block results -> partial tile.  D is the transposed block: lane (pair j = lane%16, q = lane/16)
         // holds output channels 16nb+4q .. +3 of pair j -- one 16-byte LDS read-modify-write per column
@@ -439,7 +342,7 @@ conv_mfma(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
             if (cc.x != 0 || cc.y < 0 || cc.y >= dt.D || cc.z < 0 || cc.z >= dt.H || cc.w < 0 || cc.w >= dt.W) {
                 if (dt.status && ec4 == 0) atomicOr(dt.status, SESSD_STATUS_BAD_COORD);
             } else {
-                TO* d = static_cast<TO*>(dt.dense) + ((size_t)cc.y * dt.Hp + cc.z + dt.pad_top) * dt.Wp + cc.w + dt.pad_left;
+                __half* d = static_cast<__half*>(dt.dense) + ((size_t)cc.y * dt.Hp + cc.z + dt.pad_top) * dt.Wp + cc.w + dt.pad_left;
                 const size_t plane = (size_t)dt.D * dt.Hp * dt.Wp;  // channel stride
 #pragma unroll
                 for (int e = 0; e < 4; ++e) store1(d + (size_t)(ec4 + e) * plane, o[e]);
@@ -450,7 +353,7 @@ conv_mfma(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
     }
     if constexpr (PAD) {
         __syncthreads();
-        write_pad_rows<TO, COUT, kWaves * 64>(out, n, max_voxels, s_epi, scale != nullptr, shift != nullptr, relu);
+        write_pad_rows<__half, COUT, kWaves * 64>(out, n, max_voxels, s_epi, scale != nullptr, shift != nullptr, relu);
     }
 }
 
@@ -467,19 +370,15 @@ int compute_units() {
     return cu;
 }
 
-template <typename T, int CIN, int COUT, typename TO = T>
+template <int CIN, int COUT>
 int launch(const GemmArgs& a, hipStream_t stream) {
-    // the FP32 kernels address their operands with 32-bit byte offsets and use 2^31 as "out of range"
-    if (sizeof(T) == 4 && ((size_t)a.max_voxels * CIN * sizeof(T) >= kOutOfRange ||
-                           (size_t)a.K * CIN * COUT * sizeof(T) >= kOutOfRange))
-        return SESSD_E_UNSUPPORTED;
     const int num_cu = compute_units();
     // enough workgroups for any cut of any n <= max_voxels rows: tile_plan() never makes more tiles for fewer
     // rows or a taller target (surplus workgroups return at once)
     const unsigned blocks = (unsigned)tile_plan(a.max_voxels, num_cu, kGemmMinTileRows).count;
     auto go = [&](auto pad) {
-        hipLaunchKernelGGL((conv_mfma<T, CIN, COUT, TO, decltype(pad)::value>), dim3(blocks), dim3(kWaves * 64), 0, stream,
-                           static_cast<const T*>(a.in_feat), static_cast<TO*>(a.out_feat), a.w_packed, a.nbr,
+        hipLaunchKernelGGL((conv_mfma<CIN, COUT, decltype(pad)::value>), dim3(blocks), dim3(kWaves * 64), 0, stream,
+                           static_cast<const __half*>(a.in_feat), static_cast<__half*>(a.out_feat), a.w_packed, a.nbr,
                            a.num_out, a.max_voxels, a.K, a.scale, a.shift, a.relu, num_cu, a.tiles, a.dense);
     };
     a.write_pad_rows ? go(std::true_type{}) : go(std::false_type{});
@@ -518,8 +417,8 @@ void chunk_shape(int dtype, int cin, int* channels, int* lane_elems) {
 int gemm_compute_units() { return compute_units(); }
 
 int gemm_tile_rows(int cin, int cout, int dtype) {
-    if (gemm_runs_wide(kMaxK, cin, cout, dtype, dtype)) return gemm_wide_tile_rows();
-    return tile_rows(dtype == SESSD_HALF && cin != 4, cin, cout);
+    if (gemm_runs_wide(kMaxK, cin, cout, dtype, dtype)) return gemm_wide_tile_rows(cout);
+    return tile_rows(cin, cout);
 }
 
 bool gemm_runs_on_mfma(int K, int cin, int cout, int in_type, int out_type) {
@@ -529,6 +428,7 @@ bool gemm_runs_on_mfma(int K, int cin, int cout, int in_type, int out_type) {
 
 size_t packed_weight_bytes(int K, int cin, int cout, int dtype) {
     if (!mfma_shape(K, cin, cout, dtype)) return 0;
+    if (wide_splits(cin) && gemm_runs_wide(K, cin, cout, dtype, dtype)) return wide_weight_bytes(K, cin, cout);
     return (size_t)K * cin * cout * (dtype == SESSD_HALF && cin != 4 ? sizeof(__half) : sizeof(float));
 }
 
@@ -537,6 +437,7 @@ size_t packed_weight_bytes(int K, int cin, int cout, int dtype) {
 // always takes FP32 operands (the voxel means are FP32); in an FP16 pipeline its weights are the
 // half-rounded values, as in every other layer of that pipeline.
 void pack_weights(const float* w, int K, int cin, int cout, int dtype, void* dst) {
+    if (wide_splits(cin) && gemm_runs_wide(K, cin, cout, dtype, dtype)) return pack_wide_weights(w, K, cin, cout, dst);
     int C, E;
     chunk_shape(dtype, cin, &C, &E);
     const int G = cin / C, NB = cout / 16;
@@ -547,34 +448,25 @@ void pack_weights(const float* w, int K, int cin, int cout, int dtype, void* dst
                     for (int e = 0; e < E; ++e) {
                         const size_t o = ((((size_t)k * G + g) * NB + nb) * 64 + lane) * E + e;
                         const float v = w[((size_t)k * cin + C * g + E * (lane / 16) + e) * cout + 16 * nb + lane % 16];
-                        if (dtype == SESSD_HALF && cin != 4) static_cast<__half*>(dst)[o] = __float2half_rn(v);
-                        else if (dtype == SESSD_HALF) static_cast<float*>(dst)[o] = __half2float(__float2half_rn(v));
-                        else static_cast<float*>(dst)[o] = v;
+                        float near = v;
+                        const uint16_t h = dtype == SESSD_HALF ? nearest_half(v, &near) : (uint16_t)0;
+                        if (dtype == SESSD_HALF && cin != 4) static_cast<uint16_t*>(dst)[o] = h;
+                        else static_cast<float*>(dst)[o] = near;
                     }
 }
 
 // -> SESSD_OK when an MFMA kernel was launched, SESSD_E_UNSUPPORTED when the shape/dtype is not covered
 int launch_mfma(const GemmArgs& a, hipStream_t stream) {
-    if (!a.w_packed || !mfma_shape(a.K, a.cin, a.cout, a.out_type)) return SESSD_E_UNSUPPORTED;
+    if (!a.w_packed || a.in_type != SESSD_HALF || a.out_type != SESSD_HALF || !mfma_shape(a.K, a.cin, a.cout, SESSD_HALF))
+        return SESSD_E_UNSUPPORTED;
     if ((reinterpret_cast<uintptr_t>(a.in_feat) | reinterpret_cast<uintptr_t>(a.out_feat)) & 15)
         return SESSD_E_UNSUPPORTED;
-    if (a.cin == 4 && a.in_type == SESSD_FLOAT && a.out_type == SESSD_HALF) {  // first layer of an FP16 pipeline
-        if (a.cout == 16) return launch<float, 4, 16, __half>(a, stream);
-        if (a.cout == 32) return launch<float, 4, 32, __half>(a, stream);
-    }
-    if (a.in_type != a.out_type) return SESSD_E_UNSUPPORTED;
-#define SESSD_CASE(CI, CO)                                                        \
-    if (a.cin == CI && a.cout == CO)                                              \
-    return a.in_type == SESSD_HALF ? launch<__half, CI, CO>(a, stream) : launch<float, CI, CO>(a, stream)
-    if (a.cin == 4 && a.cout == 16) return launch<float, 4, 16>(a, stream);  // (FP32 only: mfma_shape)
-    if (a.cin == 4 && a.cout == 32) return launch<float, 4, 32>(a, stream);
+#define SESSD_CASE(CI, CO) \
+    if (a.cin == CI && a.cout == CO) return launch<CI, CO>(a, stream)
     SESSD_CASE(16, 16);
     SESSD_CASE(16, 32);
     SESSD_CASE(32, 32);
-#undef SESSD_CASE
-#define SESSD_CASE(CI, CO) \
-    if (a.cin == CI && a.cout == CO && a.in_type == SESSD_HALF) return launch<__half, CI, CO>(a, stream)
-    SESSD_CASE(32, 64);  // (FP32: conv_wide.hip)
+    SESSD_CASE(32, 64);
     SESSD_CASE(64, 64);
     SESSD_CASE(64, 128);
     SESSD_CASE(128, 128);

@@ -1,31 +1,50 @@
-// conv_wide.hip -- FP32 gather-GEMM for the layers with 64 (Cin 32 or 64) or 128 output columns (Cin 64 or 128): one tall
-// tile per compute unit, sixteen waves.
+// conv_wide.hip -- FP32 gather-GEMM (all matrix-core shapes; with Cin 4 also the first layer of an FP16 pipeline).
 //
 //     out[o][:] = epilogue( sum_k  in[nbr[k][o]][:] @ W[k] )
 //
-// conv_mfma.hip gives a workgroup of four waves a tile of at most 48 rows; a wave there holds the rows of all
-// 16-pair blocks of two offsets and the whole W[k] in registers (247 of them in the 64 -> 64 layer), so a SIMD
-// holds two waves, and with ~17 000 rows a compute unit runs two 33-row tiles whose per-offset pair lists fill
-// 69 % of the 16-row MFMA blocks they occupy.  This kernel turns both knobs the other way:
-//   * one tile per compute unit, up to 96 rows: at 66 rows the pair lists fill 81 % of their blocks;
-//   * sixteen waves per tile: four groups share the tile's offsets (split-K), the four waves of a group take
-//     a quarter of the output columns each (more groups would need more partial tiles than LDS holds).  A wave
-//     works on ONE 16-pair block at a time -- the block's rows, its columns of W[k] and the next block's rows are
-//     all it holds -- so it stays far below 128 registers and a SIMD holds four waves: while one waits for rows
-//     or adds a block into its partial tile, the matrix core runs the others' blocks.
-//   * With few rows a tile per unit would be short (2 259 rows: 9), its pair lists mostly padding, and every unit would
-//     still read all 442 KB of W for it.  Up to 10 240 rows on 256 units two, up to 3 072 rows four workgroups share a
-//     tile, each taking a half or a quarter of the columns with 8 or 16 offset groups (wide_log2_split()).  Measured,
-//     launches back to back: 64 -> 64 at 2 259 rows 14.2 -> 9.9 us, at 3 476 rows 14.3 -> 11.4, at 8 615 rows 20.1 -> 19.1;
-//     at 16 914 rows unsplit tiles are the faster ones (29.5 us).
-//   * 128 columns: two workgroups take 64 each of every tile, as in such a split.  128 input channels: an offset's blocks
-//     are walked twice, with 64 channels each, so that the registers stay those of 64 (the split-K kernel spilled 297 of
-//     them).  128 -> 128, launches back to back: 3 877 rows 174 -> 41 us, 17 060 rows 270 -> 131 (floor by the matrix cores'
-//     rate 47); distance from the sums in 64 bits 1.7e-7 -> 1.4e-7 of their norm.
-// Pair lists, operand order (the packed weights are conv_mfma.hip's), partial tiles in LDS (one per group and
-// column quarter, private to a wave, so the sum order is fixed), fixed-order reduction, fused scale/shift/ReLU and
-// the optional dense scatter are as in conv_mfma.hip; results are bit-identical run to run.
+// A workgroup owns a tile of consecutive output rows (from the rulebook's equal-work cuts, tile_cut.hip, or of equal length)
+// and up to 64 columns.  The tile's neighbour lists are compacted per offset with wave64 ballots into pair lists in LDS; the
+// offsets are dealt to the waves; a wave multiplies 16 pairs at a time with all columns and adds the block into a partial
+// tile of its own in LDS (so the order of every sum is fixed); the partial tiles are summed in a fixed order, scale/shift/ReLU
+// follow, each row is stored once.  Results are bit-identical run to run.
+//
+// Products.  The FP32 matrix instruction does 32 multiply-adds a cycle and SIMD, the 16-bit ones 512, so operands are
+// split into 16-bit parts whose products are exact in FP32 and are accumulated in FP32:
+//   * Cin 64 and 128, halves: a row is scaled by a power of two that brings its largest element to [2^14, 2^15) (a column of W
+//     likewise, on the host) and x = hi + lo with 11 bits each; lo * hi, hi * lo and hi * hi on v_mfma_f32_16x16x32_f16.  What is
+//     left out is below 2^-23 of an operand and 2^-24 of a product; 3/16 of the FP32 instruction's time.
+//   * Cin 32, thirds: x = x0 + x1 + x2 with 8 bits each is exact, BF16 has FP32's range, and the six products down to 2^-24 of
+//     the largest are kept (v_mfma_f32_16x16x32_bf16; 6/16 of the time).  With halves these layers, whose sums are shorter, came
+//     out 11 % further from the sums in 64 bits than with the FP32 instruction; with thirds 30 % nearer.
+//   * Cin 4 and 16: the FP32 instruction (4 or 16 of them a block: it is not what they wait for).
+// Distance from the sums in 64 bits, 2-norm, FP32 instruction -> now: 64 -> 64 1.27e-7 -> 1.13e-7, 128 -> 128 1.31e-7 -> 1.20e-7,
+// 3x1x1 64 -> 64 1.13e-7 -> 1.00e-7, 32 -> 64 1.00e-7 -> 0.70e-7, 32 -> 32 0.93e-7 -> 0.66e-7, 16 -> 16 0.78e-7 -> 0.76e-7.  Infinities, NaN and
+// sums beyond the range come out of the parts as something that is not finite: such elements are summed again, plainly
+// (direct_sum()).
+//
+// What bounds it is instructions per wave and LDS, not the matrix cores: a block of 64 -> 64 takes a wave 1 650 cycles of
+// which 384 are MFMA; of the LDS's time a third is the lane permutation, half the partial tile.  Hence
+//   * a wave takes all 64 columns: rows are requested, split and permuted once (with 32 columns a wave 25 us at 17 262 rows,
+//     with 64 19 us);
+//   * six waves: as many partial tiles of 96 rows as LDS holds.  Eight with 72 rows are faster (17.7 against 18.5 us at 11 343
+//     rows) until a tile does not fit (25.9 against 21 us at 17 262 rows, whose cuts vary by a third);
+//   * the rows of the block after next are requested, and the next block's split, under a block's MFMAs; the next offset's
+//     weights are requested with the first block of an offset into a second set of registers;
+//   * a wave's blocks and offsets are listed once, a lane each, and read with readlane: the loop has no other bookkeeping.
+// Up to 16 (32) columns a tile is at most 112 (64) rows and a unit holds two workgroups, both used only where one tile for each
+// unit would be higher than that (32 -> 32, eight waves, 4 208 rows: one workgroup a unit 7.9 us, two 10.7).  What LDS they leave is what the
+// coordinate passes of a frame's other branch run in: 32 -> 32 with eight waves is the faster launch (15.9 us against 17.1 at
+// 28 043 rows) and makes the slower frame (20 000 points: 283 us against 274); 4 -> 32 likewise (487 against 475).
+//
+// Launches of SubM layers at the sites of scans, us, before (split-K on four waves, or sixteen waves of 16 columns, both with
+// the FP32 instruction) -> now: 64 -> 64 at 2 448 rows 10.4 -> 9.4, 8 662 20.7 -> 14.7, 17 262 31.7 -> 19.2 (99 TFLOP/s), 23 959 48.4
+// -> 30.7; 128 -> 128 at 3 594 rows 31.2 -> 19.3, 17 262 120 -> 57 (134 TFLOP/s); 64 -> 128 at 17 262 57 -> 35; 32 -> 64 at 28 043 32
+// -> 26; 32 -> 32 at 4 208 9.4 -> 8.9, 28 043 19.1 -> 16.9, 45 874 35.9 -> 27.9; 16 -> 16 at 17 132 8.3 -> 7.3; 4 -> 16 7.4 -> 6.5.  16 -> 32
+// 10.2 -> 9.0, but 14.9 -> 16.8 at 36 871 rows (a second round of tiles begins at 32 768).
+#include <cmath>
+#include <cstring>
 #include <type_traits>
+#include <vector>
 
 #include "pad_rows.h"
 
@@ -34,54 +53,362 @@ namespace sessd {
 namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef __bf16 v2b __attribute__((ext_vector_type(2)));
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef unsigned int v4u32 __attribute__((__vector_size__(16)));
 
-constexpr int kWaves = 16;          // wave64s per workgroup: four per SIMD
-constexpr int kTileRows = 96;       // tile capacity (rows): what the partial tiles leave of the 160 KB of LDS
-constexpr int kMaxBlk = kTileRows / 16;
 constexpr int kMaxK = kGemmMaxOffsets;
 constexpr unsigned kOutOfRange = 0x80000000u;  // beyond any buffer the kernel is given (launch() checks)
 constexpr int kRawBuffer = 0x00020000;         // descriptor word 3: raw 32-bit data format, no swizzle
 
-__device__ __forceinline__ float4 buffer_load16(__amdgpu_buffer_rsrc_t r, unsigned byte_offset) {
-    v4u32 v = __builtin_amdgcn_raw_buffer_load_b128(r, byte_offset, 0, 0);
-    return *reinterpret_cast<float4*>(&v);
+// how a layer's products are made: FP32 MFMA, or 16-bit MFMA on operands split into parts
+enum Arith { kPlain, kThirds, kHalves };
+constexpr Arith arith(int cin) { return cin >= 64 ? kHalves : (cin >= 32 ? kThirds : kPlain); }
+
+template <int CIN, int COUT>
+struct Shape {
+    static constexpr Arith kArith = arith(CIN);
+    static constexpr int kWeightBytes = CIN * COUT * (kArith == kThirds ? 6 : 4);  // of an offset
+    static constexpr int kWgCols = COUT < 64 ? COUT : 64;  // columns of a workgroup (before the split of short tiles)
+    static constexpr int kColGroups = COUT / kWgCols;      // workgroups beside each other
+    // (32 columns: four waves with 4 and 32 channels, whose launches are long enough for the frame's other branch to need the LDS)
+    static constexpr int kWaves = kWgCols == 64 ? 6 : (COUT == 32 && CIN != 16 ? 4 : 8);
+    static constexpr int kThreads = kWaves * 64;
+    static constexpr int kTileRows = kWgCols == 64 ? 96 : (kWgCols == 32 ? 64 : 112);  // tile capacity
+    static constexpr int kPerUnit = kWgCols == 64 ? 1 : 2;  // workgroups that can share a compute unit
+    static constexpr int kMaxBlk = kTileRows / 16;
+    static constexpr int kNone = kMaxK * kTileRows * 4;  // an item with no pairs
+    static constexpr int kParts = CIN > 64 ? CIN / 64 : 1;  // of the inner dimension, taken one after the other
+    static constexpr int CP = CIN / kParts;                 // channels of a part
+    static constexpr int G = CP < 16 ? 1 : CP / 16;         // pieces of a row that a lane requests: 4 channels each (Cin 4: 1)
+    static constexpr int kLaneBytes = CP < 16 ? 4 : 16;     // ... in bytes; of a weight operand as well
+    static constexpr int kMaxSplit = kWgCols == 64 ? 1 : 0;  // log2 of the column parts that short tiles are split into
+    static_assert(kTileRows <= 128 && kTileRows % 16 == 0, "the lists are staged in two halves of 64 rows");
+    static_assert((CP == 4 || CP % 16 == 0) && (kArith == kPlain || CP % 32 == 0) && COUT % kWgCols == 0, "whole MFMA steps and column groups");
+    static_assert((kMaxK + kWaves - 1) / kWaves * kMaxBlk * kParts + 2 <= 64, "an item a lane");
+};
+constexpr uint32_t kNoPair = 0xffffff00u;      // entry of a pair list that fills up its last block (no input row has that number)
+
+__device__ __forceinline__ void buffer_load(__amdgpu_buffer_rsrc_t r, unsigned byte_offset, int (&v)[4]) {
+    const v4u32 t = __builtin_amdgcn_raw_buffer_load_b128(r, byte_offset, 0, 0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (int)t[e];
+}
+__device__ __forceinline__ void buffer_load(__amdgpu_buffer_rsrc_t r, unsigned byte_offset, int (&v)[1]) {
+    v[0] = (int)__builtin_amdgcn_raw_buffer_load_b32(r, byte_offset, 0, 0);
+}
+__device__ __forceinline__ void store4(float* dst, const float (&o)[4]) { *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]); }
+__device__ __forceinline__ void store4(__half* dst, const float (&o)[4]) {
+    union {
+        __half2 h[2];
+        uint2 u;
+    } p;
+    p.h[0] = __floats2half2_rn(o[0], o[1]);
+    p.h[1] = __floats2half2_rn(o[2], o[3]);
+    *reinterpret_cast<uint2*>(dst) = p.u;
 }
 
-__device__ __forceinline__ void mma16(const float4& w, const float4& x, v4f& acc) {
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x, x.x, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w.y, x.y, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w.z, x.z, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w.w, x.w, acc, 0, 0, 0);
+template <int CTRL>
+__device__ __forceinline__ uint32_t quad_max(uint32_t v) {  // of this lane and the one of its quad that CTRL names
+    const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+    return v > o ? v : o;
 }
 
-// DENSE: the epilogue also scatters the rows into a dense tensor (the layer in front of sparse2Dense).  A variant of
-// its own because the scatter's addresses cost ten registers, and what this kernel leaves of the register file is
-// what the coordinate kernels of the frame's other branch run in beside it.  PAD: the rows beyond the active ones are
-// written too; a variant for the same reason (with a run-time flag the scalar registers spill and the frame that asks for
-// no such rows is 9 us longer).
-template <int CIN, int COUT, bool DENSE, bool PAD>
-__global__ void __launch_bounds__(kWaves * 64)
-conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __restrict__ Wp,
+// halves hi + lo = x * up, two of each in a word
+__device__ __forceinline__ void split_pair(float x0, float x1, float up, int& hi, int& lo) {
+    v2h h, l;
+    h.x = (_Float16)(x0 * up);
+    h.y = (_Float16)(x1 * up);
+    hi = __builtin_bit_cast(int, h);
+    asm("" : "+v"(hi));  // (or the compiler rounds each half a second time)
+    h = __builtin_bit_cast(v2h, hi);
+    l.x = (_Float16)fmaf(x0, up, -(float)h.x);
+    l.y = (_Float16)fmaf(x1, up, -(float)h.y);
+    lo = __builtin_bit_cast(int, l);
+}
+
+template <typename V>
+__device__ __forceinline__ V operand8(const int* w) {
+    const int4 v = make_int4(w[0], w[1], w[2], w[3]);
+    return __builtin_bit_cast(V, v);
+}
+
+// What a lane holds of a 16-pair block's rows (Rows, in the order of the request; words that a lane permutation brings to
+// the operands) and of an offset's weights, and the products of the two.
+template <int CIN, int COUT, int NB, Arith>
+struct Products;
+
+// FP32 MFMA
+template <int CIN, int COUT, int NB>
+struct Products<CIN, COUT, NB, kPlain> {
+    using S = Shape<CIN, COUT>;
+    static constexpr int G = S::G, E = S::kLaneBytes / 4, kWords = G * E, kPieces = G;  // (pieces: weight operands a column block)
+    static __device__ __forceinline__ void take(const int (&a)[G][E], int (&p)[kWords]) {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int e = 0; e < E; ++e) p[g * E + e] = a[g][e];
+    }
+    static __device__ __forceinline__ void multiply(const int (&w)[G][NB][E], const int (&x)[kWords], v4f (&acc)[NB]) {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(__int_as_float(w[g][nb][e]), __int_as_float(x[g * E + e]), acc[nb], 0, 0, 0);
+    }
+    static __device__ __forceinline__ float add(float p, const int (&)[kWords], float sum) { return sum + p; }
+};
+
+// BF16 MFMA on three parts of eight bits each: x = x0 + x1 + x2 exactly; the products down to 2^-24 of the largest, smallest first
+template <int CIN, int COUT, int NB>
+struct Products<CIN, COUT, NB, kThirds> {
+    using S = Shape<CIN, COUT>;
+    static constexpr int G = S::G, E = 4, C = S::CP / 32, kWords = G * 6, kPieces = 3 * C;  // (words: x0, x1, x2)
+    static __device__ __forceinline__ void take(const int (&a)[G][E], int (&p)[kWords]) {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                v2f r = {__int_as_float(a[g][2 * e]), __int_as_float(a[g][2 * e + 1])};
+#pragma unroll
+                for (int t = 0; t < 3; ++t) {
+                    int w = __builtin_bit_cast(int, __builtin_convertvector(r, v2b));
+                    asm("" : "+v"(w));
+                    p[2 * G * t + 2 * g + e] = w;
+                    r.x -= __int_as_float(w << 16);
+                    r.y -= __int_as_float(w & (int)0xffff0000);
+                }
+            }
+    }
+    static __device__ __forceinline__ void multiply(const int (&w)[3 * C][NB][E], const int (&x)[kWords], v4f (&acc)[NB]) {
+        constexpr int kPart[6][2] = {{0, 2}, {1, 1}, {2, 0}, {0, 1}, {1, 0}, {0, 0}};  // of w, of x
+#pragma unroll
+        for (int t = 0; t < 6; ++t)
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(operand8<v8b>(w[kPart[t][0] * C + c][nb]),
+                                                                      operand8<v8b>(x + 2 * G * kPart[t][1] + 4 * c), acc[nb], 0, 0, 0);
+    }
+    static __device__ __forceinline__ float add(float p, const int (&)[kWords], float sum) { return sum + p; }
+};
+
+// FP16 MFMA on the halves of both sides: low * high and high * low, then high * high, one accumulator
+template <int CIN, int COUT, int NB>
+struct Products<CIN, COUT, NB, kHalves> {
+    using S = Shape<CIN, COUT>;
+    static constexpr int G = S::G, E = 4, C = S::CP / 32, kWords = G * 4 + 1, kPieces = 2 * C;  // (words: high, low, power of two)
+    static __device__ __forceinline__ void take(const int (&a)[G][E], int (&p)[kWords]) {
+        // the row's largest magnitude -> power of two that brings it to [2^14, 2^15)
+        float big = 0.f;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            big = fmaxf(fmaxf(big, fabsf(__int_as_float(a[g][0]))), fabsf(__int_as_float(a[g][1])));
+            big = fmaxf(fmaxf(big, fabsf(__int_as_float(a[g][2]))), fabsf(__int_as_float(a[g][3])));
+        }
+        uint32_t expo = quad_max<0xB1>(__float_as_uint(big));  // (lanes 1 0 3 2; magnitudes order like their bits)
+        expo = quad_max<0x4E>(expo) & 0x7f800000u;             // (lanes 2 3 0 1)
+        expo = expo < (15u << 23) ? 15u << 23 : expo;
+        const float up = __uint_as_float((268u << 23) - expo);
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                split_pair(__int_as_float(a[g][2 * e]), __int_as_float(a[g][2 * e + 1]), up, p[2 * g + e], p[2 * G + 2 * g + e]);
+        p[4 * G] = (int)(expo - (14u << 23));
+    }
+    static __device__ __forceinline__ void multiply(const int (&w)[2 * C][NB][E], const int (&x)[kWords], v4f (&acc)[NB]) {
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(operand8<v8h>(w[C + c][nb]), operand8<v8h>(x + 4 * c), acc[nb], 0, 0, 0);
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(operand8<v8h>(w[c][nb]), operand8<v8h>(x + 2 * G + 4 * c), acc[nb], 0, 0, 0);
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(operand8<v8h>(w[c][nb]), operand8<v8h>(x + 4 * c), acc[nb], 0, 0, 0);
+    }
+    static __device__ __forceinline__ float add(float p, const int (&x)[kWords], float sum) { return fmaf(p, __int_as_float(x[4 * G]), sum); }
+};
+
+// One wave's share of a tile: the pairs of the offsets dealt to it, times its columns -- 16-column blocks nb0 .. nb0 + NB - 1
+// of the layer -- into its partial tile `part` (rows of 16 NB floats).
+template <int CIN, int COUT, int NB>
+__device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_buffer_rsrc_t rs_w, const uint32_t* s_pair,
+                                         const int32_t* s_blk, int K, int wave, int lane, int nb0, float* part) {
+    using S = Shape<CIN, COUT>;
+    using P = Products<CIN, COUT, NB, S::kArith>;
+    constexpr int kParts = S::kParts, G = S::G, E = S::kLaneBytes / 4, kWaves = S::kWaves, kTileRows = S::kTileRows;
+    constexpr int NBT = COUT / 16;                   // 16-column blocks of the layer
+    constexpr int kSlots = NB * 4;                   // 16-byte slots of a row of the partial tile
+    const int i = lane & 15;  // pair inside a 16-pair block
+    const int q = lane >> 4;  // channel group of a step
+
+    // offsets of this wave: ranked by their number of 16-pair blocks (ballots: lane k holds offset k)
+    // and dealt in that order back and forth over the waves (0 1 2 3 3 2 1 0 ...)
+    const int blocks_of = lane < K ? s_blk[lane] : 0;
+    uint32_t mask;
+    {
+        const uint64_t below = (1ull << lane) - 1ull;
+        int rank = 0, ahead = 0;
+#pragma unroll
+        for (int size = S::kMaxBlk; size >= 1; --size) {
+            const uint64_t m = __ballot(blocks_of == size);
+            if (blocks_of == size) rank = ahead + __popcll(m & below);
+            ahead += __popcll(m);
+        }
+        const int r2 = rank % (2 * kWaves);
+        const int w = r2 < kWaves ? r2 : 2 * kWaves - 1 - r2;
+        mask = (uint32_t)__ballot(blocks_of > 0 && w == wave);
+    }
+    if (!mask) return;
+    // An item is a 16-pair block of an offset (and of a part of the channels); a stage is an offset (and a part).  An offset's blocks
+    // are walked once for each part.  Lane t: where item t's pairs begin in s_pair, and its part; lane s: stage s.
+    int items = 0, stages = 0, item_at = S::kNone, stage_at = -1, stage_items = 0;
+    while (mask) {
+        const int k = __ffs(mask) - 1;
+        mask &= ~(1u << k);
+        const int n = __builtin_amdgcn_readlane(blocks_of, k);
+#pragma unroll
+        for (int part_no = 0; part_no < kParts; ++part_no) {
+            const int t = lane - items;
+            if (t >= 0 && t < n) item_at = ((k * kTileRows + t * 16) * 4) | part_no;
+            if (lane == stages) {
+                stage_at = k * kParts + part_no;
+                stage_items = n;
+            }
+            items += n;
+            ++stages;
+        }
+    }
+    // Rows are requested with four neighbouring lanes on the 64 contiguous bytes of one row (lane l: pair l / 4 of
+    // the block, bytes 16 * (l % 4) ..): the cache looks up one line per group of four lanes.  In the MFMA's
+    // operand order -- lane l: pair l % 16, bytes 16 * (l / 16) .. -- the four lanes of a group name four
+    // different rows and the same request takes four lookups: 18 instead of 48 bytes per cycle and compute unit,
+    // measured.  The operand order is restored by a lane permutation before the MFMAs.
+    // Filling pairs ask out of range (such a request returns zeros and touches no memory).
+    const char* pairs = reinterpret_cast<const char*>(s_pair);
+    auto entry_at = [&](int it, int j4) -> uint32_t { return *reinterpret_cast<const uint32_t*>(pairs + (kParts > 1 ? it & ~3 : it) + j4); };
+    auto load_a = [&](int it, uint32_t entry, int (&a)[G][E]) {
+        const unsigned row = (entry >> 8) * (unsigned)(CIN * sizeof(float)) + (kParts > 1 ? (unsigned)(it & 3) * (unsigned)(S::CP * sizeof(float)) : 0u);
+        const unsigned at = entry < kNoPair ? row + (lane & 3) * (unsigned)S::kLaneBytes : kOutOfRange;
+#pragma unroll
+        for (int g = 0; g < G; ++g) buffer_load(rs_in, at + g * 64u, a[g]);
+    };
+    auto load_b = [&](int stage, int (&b)[P::kPieces][NB][E]) {  // (stage < 0: nothing to fetch)
+        const unsigned at = stage >= 0 ? (unsigned)(((stage * P::kPieces * NBT + nb0) * 64 + lane) * S::kLaneBytes) : kOutOfRange;
+#pragma unroll
+        for (int c = 0; c < P::kPieces; ++c)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) buffer_load(rs_w, at + (c * NBT + nb) * (64u * S::kLaneBytes), b[c][nb]);
+    };
+    const int from_lane4 = (4 * i + q) * 4;  // ds_bpermute address: this lane's operand sits in lane 4 * i + q
+    const int request4 = lane & ~3, operand4 = i * 4;  // this lane's pair of a block in the request's and in the operands' order, times 4
+    int d0 = __builtin_amdgcn_readlane(item_at, 0), d1 = __builtin_amdgcn_readlane(item_at, 1), d2;
+    int a[G][E], p[P::kWords], b0[P::kPieces][NB][E], b1[P::kPieces][NB][E];
+    auto take = [&]() {
+        P::take(a, p);
+#pragma unroll
+        for (int w = 0; w < P::kWords; ++w) asm volatile("" : "+v"(p[w]));  // (here, not where they are used: `a` is free for the next request)
+    };
+    load_a(d0, entry_at(d0, request4), a);
+    load_b(__builtin_amdgcn_readlane(stage_at, 0), b0);
+    uint32_t next_entry = entry_at(d1, request4);
+    __builtin_amdgcn_sched_barrier(0);
+    take();
+    __builtin_amdgcn_sched_barrier(0);
+    load_a(d1, next_entry, a);
+    int t = 0, stage = 0;
+
+    // `use`: the weights of the item's stage; `fill`: those of the next one, requested behind its first block
+    auto item = [&](const int (&use)[P::kPieces][NB][E], int (&fill)[P::kPieces][NB][E], bool first) {
+        d2 = __builtin_amdgcn_readlane(item_at, t + 2);
+        ++t;
+        next_entry = entry_at(d2, request4);
+        const uint32_t mine = entry_at(d0, operand4);
+        int x[P::kWords];
+#pragma unroll
+        for (int w = 0; w < P::kWords; ++w) x[w] = __builtin_amdgcn_ds_bpermute(from_lane4, p[w]);
+        const int r = (int)(mine & 255u);
+        float4* const dst = reinterpret_cast<float4*>(part) + r * kSlots;
+        float4 sum[NB];
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) sum[nb] = dst[(nb * 4 + q) ^ (r & (kSlots - 1))];
+        v4f acc[NB];
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) acc[nb] = (v4f){0.f, 0.f, 0.f, 0.f};
+        P::multiply(use, x, acc);
+        take();  // (of d1's rows)
+        __builtin_amdgcn_sched_barrier(0);  // (or the requests below take other registers, which then have to arrive to be copied)
+        if (first) load_b(__builtin_amdgcn_readlane(stage_at, stage + 1), fill);
+        // (behind the weights in either case: what the waits count is then the same for every item)
+        load_a(d2, next_entry, a);
+        if (mine < kNoPair) {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                float4 v = sum[nb];
+                v.x = P::add(acc[nb][0], x, v.x);
+                v.y = P::add(acc[nb][1], x, v.y);
+                v.z = P::add(acc[nb][2], x, v.z);
+                v.w = P::add(acc[nb][3], x, v.w);
+                dst[(nb * 4 + q) ^ (r & (kSlots - 1))] = v;
+            }
+        }
+        d0 = d1;
+        d1 = d2;
+    };
+    auto run_stage = [&](const int (&use)[P::kPieces][NB][E], int (&fill)[P::kPieces][NB][E]) -> bool {
+        const int n = __builtin_amdgcn_readlane(stage_items, stage);
+        for (int j = 0; j < n; ++j) item(use, fill, j == 0);
+        return ++stage < stages;
+    };
+    while (run_stage(b0, b1) && run_stage(b1, b0)) {}
+}
+
+// four output elements of a row as plain FP32 sums (nbr: the row's neighbour at offset 0; the others follow max_voxels apart)
+template <int CIN, int COUT>
+__device__ __forceinline__ void direct_sum(const float* __restrict__ in, const float* __restrict__ w, const int32_t* __restrict__ nbr,
+                                           int max_voxels, int K, int col, float (&o)[4]) {
+    o[0] = o[1] = o[2] = o[3] = 0.f;
+    for (int k = 0; k < K; ++k) {
+        const int idx = nbr[(size_t)k * max_voxels];
+        if (idx < 0) continue;
+        for (int c = 0; c < CIN; ++c) {
+            const float x = in[(size_t)idx * CIN + c];
+            const float4 w4 = *reinterpret_cast<const float4*>(w + ((size_t)k * CIN + c) * COUT + col);
+            o[0] = fmaf(x, w4.x, o[0]);
+            o[1] = fmaf(x, w4.y, o[1]);
+            o[2] = fmaf(x, w4.z, o[2]);
+            o[3] = fmaf(x, w4.w, o[3]);
+        }
+        if (o[0] != o[0] && o[1] != o[1] && o[2] != o[2] && o[3] != o[3]) break;  // (NaN from here on)
+    }
+}
+
+// DENSE: the epilogue also scatters the rows into a dense tensor (the layer in front of sparse2Dense).  PAD: the rows beyond the
+// active ones are written too.  Variants of their own: what they need in registers is missing in the launches without.
+template <int CIN, int COUT, typename TO, bool DENSE, bool PAD>
+__global__ void __launch_bounds__((Shape<CIN, COUT>::kThreads), (Shape<CIN, COUT>::kWaves * Shape<CIN, COUT>::kPerUnit / 4))
+conv_wide(const float* __restrict__ in, TO* __restrict__ out, const void* __restrict__ Wp, const float* __restrict__ w_f32,
           const int32_t* __restrict__ nbr, const int32_t* __restrict__ num_out, int max_voxels, int K,
           const float* __restrict__ scale, const float* __restrict__ shift, int relu, int units,
           const int32_t* __restrict__ tiles, DenseTarget dt) {
-    constexpr int kParts = CIN > 64 ? CIN / 64 : 1;  // of the inner dimension, taken one after the other
-    constexpr int CP = CIN / kParts;  // channels of a part
-    constexpr int G = CP / 16;        // 16-channel chunks of a part
-    constexpr int NBT = COUT / 16;    // 16-column blocks of the layer
-    constexpr int NB = 1;             // column blocks of one wave
-    constexpr int CW = 16;            // columns of one wave
-    constexpr int kWgCols = 64;       // columns of a workgroup (before the split of short tiles)
-    constexpr int LDP = CW + 4;     // padded row stride of a partial tile
-    static_assert(kTileRows <= 128 && kTileRows % 16 == 0, "the lists are staged in two halves of 64 rows");
-    constexpr int kThreads = kWaves * 64;
-    static_assert(CIN % 16 == 0 && CIN % kParts == 0 && COUT % kWgCols == 0, "whole MFMA chunks and column groups");
-    __shared__ int32_t s_in[kMaxK * kTileRows];   // compacted pair lists: input row ...
-    __shared__ uint8_t s_row[kMaxK * kTileRows];  // ... and local output row of pair j of offset k
-    __shared__ int32_t s_cnt[kMaxK + 5];          // pairs per offset
-    __shared__ float s_epi[2 * COUT];
-    __shared__ float s_part[kWaves * kTileRows * LDP];
+    using S = Shape<CIN, COUT>;
+    constexpr int kWgCols = S::kWgCols, kMaxSplit = S::kMaxSplit, kTileRows = S::kTileRows, kWaves = S::kWaves, kThreads = S::kThreads;
+    // (one block more: all of it filling pairs)
+    __shared__ uint32_t s_pair[kMaxK * kTileRows + 16];  // compacted pair lists: pair j of offset k, input row << 8 | local output row
+    __shared__ int32_t s_blk[kMaxK + 5];            // 16-pair blocks per offset
+    __shared__ float s_epi[3 * COUT];
+    __shared__ __align__(16) float s_part[kWaves * kTileRows * kWgCols];
 
     int n = *num_out;
     const int cut_count = tiles ? tiles[0] : 0;
@@ -92,57 +419,50 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
         block %= units;
     }
     // the cuts of this workgroup's first tile under each split it may be part of: requested beside the row count
-    int cut_begin[3], cut_end[3];
-    int tile_of[3] = {block, block, block};
+    int cut_begin[kMaxSplit + 1], cut_end[kMaxSplit + 1], tile_of[kMaxSplit + 1];
 #pragma unroll
-    for (int s = 0; s < 3; ++s) {
-#pragma unroll
-        for (int part = 1; part < 1 << s; ++part) tile_of[s] -= block >= part * (units >> s) ? units >> s : 0;
+    for (int s = 0; s <= kMaxSplit; ++s) {
+        tile_of[s] = s && block >= units >> 1 ? block - (units >> 1) : block;
         cut_begin[s] = tiles ? tiles[4 + tile_of[s]] : 0;
         cut_end[s] = tiles ? tiles[5 + tile_of[s]] : 0;
     }
     n = n < 0 ? 0 : (n > max_voxels ? max_voxels : n);
     // Column parts: 1 << lsplit workgroups share a tile.  The parts of a tile are row_groups apart in the grid, which
     // puts them on one XCD (workgroups are dealt round robin over eight): they read the same rows.
-    const int lsplit = wide_log2_split(n, K, units);
+    const int lsplit = kMaxSplit ? wide_log2_split(n, K, units) : 0;
     const int row_groups = units >> lsplit;  // workgroups of one column part
-    const int first_tile = lsplit == 0 ? tile_of[0] : (lsplit == 1 ? tile_of[1] : tile_of[2]);
-    int part_id = 0;
-#pragma unroll
-    for (int part = 1; part < 4; ++part) part_id += block >= part * row_groups ? 1 : 0;
-    const int lcs = 2 - lsplit, cs = 1 << lcs;                // waves of a group: the column quarters of this part
-    const int lkg = 4 - lcs, kg = 1 << lkg;                   // groups the offsets are dealt to
+    const int first_tile = tile_of[kMaxSplit ? lsplit : 0];
+    const int part_id = lsplit && block >= row_groups ? 1 : 0;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (tells the compiler that it is wave-uniform)
-    const int kgrp = wave >> lcs;                                // offsets are dealt to this group ...
-    const int quarter = col0 / CW + (part_id << lcs) + (wave & (cs - 1));  // ... and this wave computes these columns of them
-    float epi_scale = 1.f, epi_shift = 0.f;
+    const int cols = kWgCols >> lsplit, col_first = col0 + part_id * cols;  // columns of this workgroup
+    float epi_scale = 1.f, epi_shift = 0.f, epi_col = 1.f;
     if (tid < COUT) {
         if (scale) epi_scale = scale[tid];
         if (shift) epi_shift = shift[tid];
+        if (S::kArith == kHalves) epi_col = reinterpret_cast<const float*>(static_cast<const char*>(Wp) + (size_t)K * S::kWeightBytes)[tid];
     }
     // this thread's epilogue columns (the same for every row it stores): within the part, and of the layer
-    const int lvec = 4 - lsplit;  // log2 of the part's 4-column vectors
-    const int pc4 = (tid & ((1 << lvec) - 1)) * 4, ec4 = col0 + part_id * (kWgCols >> lsplit) + pc4;
+    const int lvec = (kWgCols == 64 ? 4 : (kWgCols == 32 ? 3 : 2)) - lsplit;  // log2 of the part's 4-column vectors
+    const int vec = tid & ((1 << lvec) - 1), ec4 = col_first + vec * 4;
 
     // The grid is one workgroup per compute unit (a workgroup takes most of a unit's LDS, so workgroups with no
     // tile would queue behind the busy ones just to return); a workgroup walks tiles first_tile, first_tile +
     // row_groups, ...: runs of rows from the rulebook's equal-work cuts, or runs of equal length.
+    // (Two workgroups share a unit only where one tile for each unit would not do: a tile's weights are the same for any height.)
+    const int walkers = S::kPerUnit > 1 && cut_count == 0 && n <= units / S::kPerUnit * kTileRows ? units / S::kPerUnit : row_groups;
     TilePlan plan = {0, 0};
-    if (cut_count == 0) plan = tile_plan(n, row_groups, kTileRows);
+    if (cut_count == 0) plan = tile_plan(n, walkers, kTileRows);
     const int tile_count = cut_count > 0 ? cut_count : (n > 0 ? plan.count : 0);
-    const int first_begin = lsplit == 0 ? cut_begin[0] : (lsplit == 1 ? cut_begin[1] : cut_begin[2]);
-    const int first_end = lsplit == 0 ? cut_end[0] : (lsplit == 1 ? cut_end[1] : cut_end[2]);
-    const int i = lane & 15;  // pair inside a 16-pair block
-    const int q = lane >> 4;  // channel group inside a 16-channel chunk
+    const int first_begin = cut_begin[kMaxSplit ? lsplit : 0], first_end = cut_end[kMaxSplit ? lsplit : 0];
     const __amdgpu_buffer_rsrc_t rs_in = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(in), 0, (int)((size_t)max_voxels * CIN * sizeof(float)), kRawBuffer);
     const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<void*>(Wp), 0, (int)((size_t)K * CIN * COUT * sizeof(float)), kRawBuffer);
+        const_cast<void*>(Wp), 0, (int)((size_t)K * S::kWeightBytes), kRawBuffer);
 
     bool idle = true;  // (no rows)
-    for (int tile = first_tile; tile < tile_count; tile += row_groups) {
+    for (int tile = first_tile; tile < tile_count; tile += walkers) {
     int run_begin, run_end;
     if (cut_count > 0) {
         run_begin = tile == first_tile ? first_begin : tiles[4 + tile];
@@ -170,11 +490,13 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
     if (row0 == run_begin && tid < COUT) {
         s_epi[tid] = epi_scale;
         s_epi[COUT + tid] = epi_shift;
+        s_epi[2 * COUT + tid] = epi_col;
     }
     idle = false;
+    if (tid < 16) s_pair[kMaxK * kTileRows + tid] = kNoPair;
     // zero this wave's partial tile (while the lists are on their way)
-    float* part = s_part + wave * kTileRows * LDP;
-    for (int t = lane; t < rows * LDP / 4; t += 64) reinterpret_cast<float4*>(part)[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+    float* part = s_part + wave * kTileRows * cols;
+    for (int t = lane; t < rows << lvec; t += 64) reinterpret_cast<float4*>(part)[t] = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int s = 0; s < kListsPerWave; ++s) {
         const int k = wave + s * kWaves;
@@ -186,176 +508,87 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
             const uint64_t m = __ballot(v >= 0);
             if (v >= 0) {
                 const int j = base + __popcll(m & ((1ull << lane) - 1ull));
-                s_in[k * kTileRows + j] = v;
-                s_row[k * kTileRows + j] = (uint8_t)(h * 64 + lane);
+                s_pair[k * kTileRows + j] = ((uint32_t)v << 8) | (uint32_t)(h * 64 + lane);
             }
             base += __popcll(m);
         }
-        if (lane == 0) s_cnt[k] = base;
+        const int blocks = (base + 15) >> 4;
+        if (base + lane < blocks * 16) s_pair[k * kTileRows + base + lane] = kNoPair;
+        if (lane == 0) s_blk[k] = blocks;
     }
     __syncthreads();
+    if constexpr (kMaxSplit)
+        if (lsplit) multiply<CIN, COUT, kWgCols / 32>(rs_in, rs_w, s_pair, s_blk, K, wave, lane, col_first / 16, part);
+    if (!kMaxSplit || !lsplit) multiply<CIN, COUT, kWgCols / 16>(rs_in, rs_w, s_pair, s_blk, K, wave, lane, col_first / 16, part);
+    __syncthreads();
 
-    // offsets of this wave's group: ranked by their number of 16-pair blocks (ballots: lane k holds offset k)
-    // and dealt in that order back and forth over the groups (0 1 2 3 3 2 1 0 ...)
-    uint32_t my_mask;
-    {
-        const int c = lane < K ? s_cnt[lane] : 0;
-        const int b = (c + 15) >> 4;
-        const uint64_t below = (1ull << lane) - 1ull;
-        int rank = 0, ahead = 0;
+    // fixed-order sum of the waves' partial tiles, epilogue, coalesced stores; the sums of kAtOnce vectors are read together
+    constexpr int kAtOnce = 2;
+    float e_scale[4], e_shift[4], e_col[4];
 #pragma unroll
-        for (int size = kMaxBlk; size >= 1; --size) {
-            const uint64_t m = __ballot(b == size);
-            if (b == size) rank = ahead + __popcll(m & below);
-            ahead += __popcll(m);
-        }
-        const int r2 = rank & (2 * kg - 1);
-        const int w = r2 < kg ? r2 : 2 * kg - 1 - r2;
-        my_mask = (uint32_t)__ballot(b > 0 && w == kgrp);
+    for (int e = 0; e < 4; ++e) {
+        e_scale[e] = s_epi[ec4 + e];
+        e_shift[e] = s_epi[COUT + ec4 + e];
+        e_col[e] = s_epi[2 * COUT + ec4 + e];
     }
-
-    // Rows are requested with four neighbouring lanes on the 64 contiguous bytes of one row (lane l: pair l / 4 of
-    // the block, bytes 16 * (l % 4) ..): the cache looks up one line per group of four lanes.  In the MFMA's
-    // operand order -- lane l: pair l % 16, bytes 16 * (l / 16) .. -- the four lanes of a group name four
-    // different rows and the same request takes four lookups: 18 instead of 48 bytes per cycle and compute unit,
-    // measured.  The operand order is restored by a lane permutation (fetch()) before the MFMAs.
-    // Padding lanes ask out of range (such a request returns zeros and touches no memory).
-    auto row_at = [&](int k, int cnt, int blk, int part) -> unsigned {
-        const int j = blk * 16 + (lane >> 2);
-        const bool live = j < cnt;
-        const int idx = s_in[k * kTileRows + (live ? j : 0)];
-        return live ? (unsigned)((idx * CIN + part * CP + (lane & 3) * 4) * (int)sizeof(float)) : kOutOfRange;
-    };
-    const int from_lane4 = (4 * i + q) * 4;  // ds_bpermute address: this lane's operand sits in lane 4 * i + q
-    auto fetch = [&](const float4& v) -> float4 {
-        float4 r;
-        r.x = __int_as_float(__builtin_amdgcn_ds_bpermute(from_lane4, __float_as_int(v.x)));
-        r.y = __int_as_float(__builtin_amdgcn_ds_bpermute(from_lane4, __float_as_int(v.y)));
-        r.z = __int_as_float(__builtin_amdgcn_ds_bpermute(from_lane4, __float_as_int(v.z)));
-        r.w = __int_as_float(__builtin_amdgcn_ds_bpermute(from_lane4, __float_as_int(v.w)));
-        return r;
-    };
-    auto load_a = [&](unsigned at, float4 (&a)[G]) {
+    for (int v0 = tid; v0 < rows << lvec; v0 += kAtOnce * kThreads) {
+    float4 sums[kAtOnce];
 #pragma unroll
-        for (int g = 0; g < G; ++g) a[g] = buffer_load16(rs_in, at + g * 16 * (unsigned)sizeof(float));
-    };
-    // chunk g of this wave's columns of W[k] -> operand registers (k < 0: nothing to fetch)
-    auto load_b = [&](int k, int part, int g, float4 (&b)[NB]) {
-        const unsigned at = k >= 0 ? (unsigned)((((((k * kParts + part) * G + g) * NBT + quarter * NB) * 64) + lane) * 16) : kOutOfRange;
+    for (int u = 0; u < kAtOnce; ++u) {
+        const int r = (v0 + u * kThreads) >> lvec;
+        sums[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (r >= rows) break;
+        const float4* col = reinterpret_cast<const float4*>(s_part) + (r << lvec) + (vec ^ (r & ((1 << lvec) - 1)));
+        float4 p4[kWaves];
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) b[nb] = buffer_load16(rs_w, at + nb * 64 * 16u);
-    };
-
-    int k_cur = my_mask ? __ffs(my_mask) - 1 : -1;
-    my_mask &= my_mask - 1;
-    float4 a0[G], a1[G], b[G][NB];
-    int cnt_cur = 0;
-    if (k_cur >= 0) {
-        cnt_cur = __builtin_amdgcn_readfirstlane(s_cnt[k_cur]);
+        for (int w = 0; w < kWaves; ++w) p4[w] = col[w * (kTileRows << lvec)];
 #pragma unroll
-        for (int g = 0; g < G; ++g) load_b(k_cur, 0, g, b[g]);
-        load_a(row_at(k_cur, cnt_cur, 0, 0), a0);
+        for (int m = kWaves; m > 1; m = (m + 1) / 2)  // (folded: fewer roundings follow each other)
+#pragma unroll
+            for (int w = 0; w < m / 2; ++w) {
+                p4[w].x += p4[m - 1 - w].x;
+                p4[w].y += p4[m - 1 - w].y;
+                p4[w].z += p4[m - 1 - w].z;
+                p4[w].w += p4[m - 1 - w].w;
+            }
+        sums[u] = p4[0];
     }
-    // an offset's blocks are walked once for each part of the channels
-    int k_nxt = -1, cnt_nxt = 0, nblk = 0, blk = 0, part_cur = 0, part_nxt = 0;
-    auto begin_offset = [&]() {
-        nblk = (cnt_cur + 15) >> 4;
-        blk = 0;
-        if (kParts > 1 && part_cur + 1 < kParts) {
-            k_nxt = k_cur;
-            cnt_nxt = cnt_cur;
-            part_nxt = part_cur + 1;
-            return;
-        }
-        part_nxt = 0;
-        k_nxt = my_mask ? __ffs(my_mask) - 1 : -1;
-        my_mask &= my_mask - 1;
-        cnt_nxt = k_nxt >= 0 ? __builtin_amdgcn_readfirstlane(s_cnt[k_nxt]) : 0;  // wave-uniform
-    };
-    auto item = [&](float4 (&a_use)[G], float4 (&a_fill)[G]) {
-        const bool last = blk + 1 == nblk;  // wave-uniform
-        // the next block's rows: of this offset, or the first block of the next one (cnt_nxt = 0: none)
-        load_a(last ? row_at(k_nxt >= 0 ? k_nxt : 0, cnt_nxt, 0, part_nxt) : row_at(k_cur, cnt_cur, blk + 1, part_cur), a_fill);
-        v4f acc[NB];
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) acc[nb] = (v4f){0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < kAtOnce; ++u) {
+        const int r = (v0 + u * kThreads) >> lvec;
+        if (r >= rows) break;
+        float o[4] = {sums[u].x, sums[u].y, sums[u].z, sums[u].w};
+        bool finite = true;
+        if constexpr (S::kArith != kPlain) {
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const float4 x = fetch(a_use[g]);
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) mma16(b[g][nb], x, acc[nb]);
-            // behind the offset's last block the next offset's chunk g replaces this one
-            if (last) load_b(k_nxt, part_nxt, g, b[g]);
-        }
-        const int j = blk * 16 + i;
-        if (j < cnt_cur) {
-            float* dst = part + (int)s_row[k_cur * kTileRows + j] * LDP + q * 4;
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                float4 v = *reinterpret_cast<float4*>(dst + nb * 16);
-                v.x += acc[nb][0];
-                v.y += acc[nb][1];
-                v.z += acc[nb][2];
-                v.w += acc[nb][3];
-                *reinterpret_cast<float4*>(dst + nb * 16) = v;
+            for (int e = 0; e < 4; ++e) {
+                if (S::kArith == kHalves) o[e] *= e_col[e];
+                finite = finite && (__float_as_uint(o[e]) & 0x7f800000u) != 0x7f800000u;
             }
         }
-        if (last) {
-            k_cur = k_nxt;
-            cnt_cur = cnt_nxt;
-            part_cur = part_nxt;
-            if (k_cur >= 0) begin_offset();
-        } else {
-            ++blk;
-        }
-    };
-    if (k_cur >= 0) begin_offset();
-    while (k_cur >= 0) {
-        item(a0, a1);
-        if (k_cur < 0) break;
-        item(a1, a0);
-    }
-    __syncthreads();
-
-    // fixed-order sum of the groups' partial tiles, epilogue, coalesced stores
-    for (int v = tid; v < rows << lvec; v += kThreads) {
-        const int r = v >> lvec;
-        const float* col = s_part + ((pc4 / CW) * kTileRows + r) * LDP + pc4 % CW;
-        float4 acc4 = *reinterpret_cast<const float4*>(col);
-        auto add = [&](int w) {
-            const float4 p4 = *reinterpret_cast<const float4*>(col + (w << lcs) * kTileRows * LDP);
-            acc4.x += p4.x;
-            acc4.y += p4.y;
-            acc4.z += p4.z;
-            acc4.w += p4.w;
-        };
-#pragma unroll
-        for (int w = 1; w < 4; ++w) add(w);
-        for (int w0 = 4; w0 < kg; w0 += 4) {  // (8 or 16 groups under a column split)
-#pragma unroll
-            for (int w = 0; w < 4; ++w) add(w0 + w);
-        }
-        float o[4] = {acc4.x, acc4.y, acc4.z, acc4.w};
+        // the parts of an infinity, or a sum beyond their range, say nothing: the products themselves
+        if (S::kArith != kPlain && !finite) direct_sum<CIN, COUT>(in, w_f32, nbr + row0 + r, max_voxels, K, ec4, o);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             float s = o[e];
-            if (scale) s = s * s_epi[ec4 + e];
-            if (shift) s = s + s_epi[COUT + ec4 + e];
+            if (scale) s = s * e_scale[e];
+            if (shift) s = s + e_shift[e];
             if (relu) s = s > 0.f ? s : 0.f;
             o[e] = s;
         }
-        *reinterpret_cast<float4*>(out + (size_t)(row0 + r) * COUT + ec4) = make_float4(o[0], o[1], o[2], o[3]);
+        store4(out + (size_t)(row0 + r) * COUT + ec4, o);
         if (DENSE && dt.dense) {  // the sparse2Dense scatter of this row, fused (uniform branch)
             const int4 cc = reinterpret_cast<const int4*>(dt.coors)[row0 + r];  // (b,z,y,x)
             if (cc.x != 0 || cc.y < 0 || cc.y >= dt.D || cc.z < 0 || cc.z >= dt.H || cc.w < 0 || cc.w >= dt.W) {
                 if (dt.status && ec4 == 0) atomicOr(dt.status, SESSD_STATUS_BAD_COORD);
             } else {
-                float* d = static_cast<float*>(dt.dense) + ((size_t)cc.y * dt.Hp + cc.z + dt.pad_top) * dt.Wp + cc.w + dt.pad_left;
+                TO* d = static_cast<TO*>(dt.dense) + ((size_t)cc.y * dt.Hp + cc.z + dt.pad_top) * dt.Wp + cc.w + dt.pad_left;
                 const size_t plane = (size_t)dt.D * dt.Hp * dt.Wp;  // channel stride
 #pragma unroll
-                for (int e = 0; e < 4; ++e) d[(size_t)(ec4 + e) * plane] = o[e];
+                for (int e = 0; e < 4; ++e) d[(size_t)(ec4 + e) * plane] = (TO)o[e];
             }
         }
+    }
     }
     __syncthreads();  // the next piece reuses the lists and partial tiles
     }
@@ -366,21 +599,22 @@ conv_wide(const float* __restrict__ in, float* __restrict__ out, const void* __r
             s_epi[COUT + tid] = epi_shift;
         }
         __syncthreads();
-        write_pad_rows<float, COUT, kThreads>(out, n, max_voxels, s_epi, scale != nullptr, shift != nullptr, relu);
+        write_pad_rows<TO, COUT, kThreads>(out, n, max_voxels, s_epi, scale != nullptr, shift != nullptr, relu);
     }
 }
 
-template <int CIN, int COUT>
+template <int CIN, int COUT, typename TO = float>
 int launch(const GemmArgs& a, hipStream_t stream) {
-    // operands are addressed with 32-bit byte offsets, 2^31 means "out of range"
-    if ((size_t)a.max_voxels * CIN * sizeof(float) >= kOutOfRange || (size_t)a.K * CIN * COUT * sizeof(float) >= kOutOfRange)
+    // operands are addressed with 32-bit byte offsets, 2^31 means "out of range"; a pair keeps its input row in 24 bits
+    if ((size_t)a.max_voxels * CIN * sizeof(float) >= kOutOfRange || (size_t)a.K * Shape<CIN, COUT>::kWeightBytes >= kOutOfRange ||
+        a.max_voxels >= 1 << 24)
         return SESSD_E_UNSUPPORTED;
-    const int units = gemm_compute_units() / (COUT / 64);
-    const unsigned blocks = (unsigned)(units * (COUT / 64));
+    using S = Shape<CIN, COUT>;
+    const int units = gemm_compute_units() * S::kPerUnit / S::kColGroups;
     auto go = [&](auto dense, auto pad) {
-        hipLaunchKernelGGL((conv_wide<CIN, COUT, decltype(dense)::value, decltype(pad)::value>), dim3(blocks), dim3(kWaves * 64), 0, stream,
-                           static_cast<const float*>(a.in_feat), static_cast<float*>(a.out_feat), a.w_packed, a.nbr,
-                           a.num_out, a.max_voxels, a.K, a.scale, a.shift, a.relu, units, a.tiles, a.dense);
+        hipLaunchKernelGGL((conv_wide<CIN, COUT, TO, decltype(dense)::value, decltype(pad)::value>), dim3((unsigned)(units * S::kColGroups)),
+                           dim3(S::kThreads), 0, stream, static_cast<const float*>(a.in_feat), static_cast<TO*>(a.out_feat), a.w_packed,
+                           a.w_f32, a.nbr, a.num_out, a.max_voxels, a.K, a.scale, a.shift, a.relu, units, a.tiles, a.dense);
     };
     if (a.dense.dense) a.write_pad_rows ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
     else a.write_pad_rows ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
@@ -391,15 +625,77 @@ int launch(const GemmArgs& a, hipStream_t stream) {
 }  // namespace
 
 bool gemm_runs_wide(int K, int cin, int cout, int in_type, int out_type) {
-    if (in_type != SESSD_FLOAT || out_type != SESSD_FLOAT || K > kMaxK) return false;
-    return cout == 64 ? cin == 64 || cin == 32 : cout == 128 && (cin == 64 || cin == 128);
+    if (in_type != SESSD_FLOAT || K > kMaxK) return false;
+    if (cin == 4) return cout == 16 || cout == 32;  // (the first layer of an FP16 pipeline as well)
+    if (out_type != SESSD_FLOAT) return false;
+    const int shapes[][2] = {{16, 16}, {16, 32}, {32, 32}, {32, 64}, {64, 64}, {64, 128}, {128, 128}};
+    for (auto& s : shapes)
+        if (s[0] == cin && s[1] == cout) return true;
+    return false;
 }
 
-int gemm_wide_tile_rows() { return kTileRows; }
+int gemm_wide_tile_rows(int cout) { return cout >= 64 ? Shape<64, 64>::kTileRows : (cout >= 32 ? Shape<32, 32>::kTileRows : Shape<16, 16>::kTileRows); }
+
+bool wide_splits(int cin) { return arith(cin) != kPlain; }
+size_t wide_weight_bytes(int K, int cin, int cout) {
+    return arith(cin) == kThirds ? (size_t)K * cin * cout * 6 : ((size_t)K * cin + 1) * cout * sizeof(float);
+}
+
+// the nearest BF16, as nearest_half()
+static uint16_t nearest_bf16(float v, float* value) {
+    uint32_t u;
+    std::memcpy(&u, &v, 4);
+    u = (u & 0x7fffffffu) > 0x7f800000u ? u | 0x400000u : u + 0x7fffu + ((u >> 16) & 1u);
+    u &= 0xffff0000u;
+    std::memcpy(value, &u, 4);
+    return (uint16_t)(u >> 16);
+}
+
+// W in parts and in operand order: Wp[k][64 channels][part][step][16-column block][lane][8], element j of lane l being channel
+// 32 step + 16 (j / 4) + 4 (l / 16) + j % 4 (the channels that the lane permutation of the rows brings there), column
+// 16 block + l % 16.  Halves: of W * 2^e[column], and behind them 2^-e[column].
+void pack_wide_weights(const float* w, int K, int cin, int cout, void* dst) {
+    const bool halves = arith(cin) == kHalves;
+    std::vector<float> up(cout, 1.f);
+    if (halves) {
+        std::vector<float> big(cout, 0.f);
+        for (size_t t = 0; t < (size_t)K * cin; ++t)
+            for (int col = 0; col < cout; ++col) {
+                const float v = std::fabs(w[t * cout + col]);
+                if (v > big[col] && v <= 3.402823466e38f) big[col] = v;  // (finite)
+            }
+        float* down = reinterpret_cast<float*>(static_cast<char*>(dst) + (size_t)K * cin * cout * sizeof(float));
+        for (int col = 0; col < cout; ++col) {
+            int e = big[col] > 0.f ? 14 - std::ilogb(big[col]) : 0;
+            e = e > 126 ? 126 : e;
+            up[col] = std::ldexp(1.f, e);
+            down[col] = std::ldexp(1.f, -e);
+        }
+    }
+    const int cp = cin > 64 ? 64 : cin, steps = cp / 32, blocks = cout / 16, parts = halves ? 2 : 3;
+    uint16_t* o = static_cast<uint16_t*>(dst);
+    const size_t part_size = (size_t)steps * blocks * 512;
+    for (int k = 0; k < K; ++k)
+        for (int ch = 0; ch < cin; ++ch, w += cout) {
+            const int in_part = ch % cp, in_step = in_part % 32;
+            const int first_lane = in_step % 16 / 4 * 16, j = in_step / 16 * 4 + in_step % 4;
+            uint16_t* at = o + (size_t)(k * (cin / cp) + ch / cp) * parts * part_size + (size_t)(in_part / 32) * blocks * 512 + first_lane * 8 + j;
+            for (int col = 0; col < cout; ++col) {
+                uint16_t* to = at + (size_t)(col / 16) * 512 + col % 16 * 8;
+                float v = w[col] * up[col], near = 0.f;
+                for (int part = 0; part < parts; ++part, v -= near) to[part * part_size] = halves ? nearest_half(v, &near) : nearest_bf16(v, &near);
+            }
+        }
+}
 
 int launch_wide(const GemmArgs& a, hipStream_t stream) {
     if (!a.w_packed || !gemm_runs_wide(a.K, a.cin, a.cout, a.in_type, a.out_type)) return SESSD_E_UNSUPPORTED;
     if ((reinterpret_cast<uintptr_t>(a.in_feat) | reinterpret_cast<uintptr_t>(a.out_feat)) & 15) return SESSD_E_UNSUPPORTED;
+    if (a.cin == 4 && a.out_type == SESSD_HALF) return a.cout == 16 ? launch<4, 16, __half>(a, stream) : launch<4, 32, __half>(a, stream);
+    if (a.cin == 4) return a.cout == 16 ? launch<4, 16>(a, stream) : launch<4, 32>(a, stream);
+    if (a.cin == 16 && a.cout == 16) return launch<16, 16>(a, stream);
+    if (a.cin == 16 && a.cout == 32) return launch<16, 32>(a, stream);
+    if (a.cin == 32 && a.cout == 32) return launch<32, 32>(a, stream);
     if (a.cin == 64 && a.cout == 64) return launch<64, 64>(a, stream);
     if (a.cin == 32 && a.cout == 64) return launch<32, 64>(a, stream);
     if (a.cin == 64 && a.cout == 128) return launch<64, 128>(a, stream);

@@ -1,6 +1,8 @@
 // kernels.h -- launchers of the gather-GEMM kernels (conv_gemm.hip) used by both conv plugins.
 #pragma once
 
+#include <cstring>
+
 #include "common.h"
 
 namespace sessd {
@@ -50,15 +52,14 @@ __host__ __device__ inline TilePlan tile_plan(int n, int num_cu, int target) {
     p.height = (n + p.count - 1) / p.count;
     return p;
 }
-// The one-tile-per-unit FP32 kernel (conv_wide.hip) with few rows: the 64 output columns of a tile are dealt to `split`
-// workgroups, so that the tiles stay tall enough to fill their 16-pair blocks while every compute unit has work and
-// reads only its columns of the weights.  At the bounds a tile has 48 (split 4) and 80 rows (split 2): beyond them
-// the blocks of the unsplit tiles are full enough.  A kernel volume with fewer offsets than the groups of a split
-// tile could be dealt (the 3x1x1 layer) is not split.
-constexpr int kWideSplit4Rows = 48, kWideSplit2Rows = 80, kWideSplitMinOffsets = 16;
+// The FP32 kernel (conv_wide.hip) with few rows and 64 or more output columns: the 64 columns of a tile are dealt to two workgroups,
+// so that the tiles stay tall enough to fill their 16-pair blocks while every compute unit has work and reads only its
+// columns of the weights.  At the bound a tile has 80 rows: beyond it the blocks of the unsplit tiles are full enough.
+// A kernel volume with fewer offsets than could be dealt to the waves (the 3x1x1 layer) is not split.
+constexpr int kWideSplitRows = 80, kWideSplitMinOffsets = 16;
 __host__ __device__ inline int wide_log2_split(int n, int K, int num_cu) {
-    if (num_cu % 4 || K < kWideSplitMinOffsets) return 0;
-    return n <= num_cu / 4 * kWideSplit4Rows ? 2 : (n <= num_cu / 2 * kWideSplit2Rows ? 1 : 0);
+    if (num_cu % 2 || K < kWideSplitMinOffsets) return 0;
+    return n <= num_cu / 2 * kWideSplitRows ? 1 : 0;
 }
 // tile capacity (rows) of the MFMA kernel that serves this layer shape
 int gemm_tile_rows(int cin, int cout, int dtype);
@@ -75,16 +76,45 @@ bool gemm_runs_on_mfma(int K, int cin, int cout, int in_type, int out_type);
 // whether the layer runs on one of the FP16 kernels (conv_tile.hip, conv_tall.hip) that cut their own tiles: a rulebook
 // whose owner does needs no equal-work cuts
 bool gemm_cuts_own_tiles(int K, int cin, int cout, int in_type, int out_type);
-// whether the layer runs on the FP32 kernel with one tall tile per compute unit (conv_wide.hip), and that kernel's
-// tile capacity
+// whether the layer runs on the FP32 kernel (conv_wide.hip), that kernel's tile capacity, and whether it multiplies 16-bit
+// parts of the operands, which need weights of a form of their own
 bool gemm_runs_wide(int K, int cin, int cout, int in_type, int out_type);
-int gemm_wide_tile_rows();
+int gemm_wide_tile_rows(int cout);
+bool wide_splits(int cin);
+size_t wide_weight_bytes(int K, int cin, int cout);
+void pack_wide_weights(const float* w, int K, int cin, int cout, void* dst);
 
 // size in bytes of the packed weight copy for this shape/dtype (0 = shape runs on the VALU path)
 size_t packed_weight_bytes(int K, int cin, int cout, int dtype);
 // host-side packing into MFMA operand order; dst has packed_weight_bytes() bytes
 void pack_weights(const float* w, int K, int cin, int cout, int dtype, void* dst);
 
+// The nearest half, ties to even, as bits, and its value.  (Host code: the weights of a backbone are 500 000 and more, and the
+// compiler's conversion is a call.)
+inline uint16_t nearest_half(float v, float* value) {
+    uint32_t u;
+    std::memcpy(&u, &v, 4);
+    const uint32_t sign = u & 0x80000000u, mag = u ^ sign;
+    uint32_t h, back;
+    if (mag >= 0x477ff000u) {  // beyond the largest half, infinite or NaN
+        h = mag > 0x7f800000u ? 0x7e00u : 0x7c00u;
+        back = mag > 0x7f800000u ? 0x7fc00000u : 0x7f800000u;
+    } else if (mag >= 0x38800000u) {
+        back = (mag + 0xfffu + ((mag >> 13) & 1u)) & ~0x1fffu;
+        h = (back - 0x38000000u) >> 13;
+    } else {  // a multiple of 2^-24, the unit of the last place of 1/2
+        float f;
+        std::memcpy(&f, &mag, 4);
+        f += 0.5f;
+        std::memcpy(&h, &f, 4);
+        h -= 0x3f000000u;
+        f -= 0.5f;
+        std::memcpy(&back, &f, 4);
+    }
+    back |= sign;
+    std::memcpy(value, &back, 4);
+    return (uint16_t)(h | sign >> 16);
+}
 // rulebook export (reference layout indice_pairs[K][2][max_voxels], indice_num[K])
 size_t export_scratch_bytes(int K, int max_voxels);
 int launch_export_rulebook(const int32_t* nbr, const int32_t* num_out, int K, int max_voxels,

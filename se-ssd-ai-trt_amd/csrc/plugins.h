@@ -126,7 +126,7 @@ class ConvPluginBase {
     int tileRows() const;
     // weight of a row beside its pairs in those cuts
     int tileRowWeight() const;
-    // compute units that share a tile of the one-tile-per-unit kernel (conv_wide.hip), each 64 of the columns, where
+    // compute units that share a tile of the FP32 kernel (conv_wide.hip), each up to 64 of the columns, where
     // they are cut for that kernel; 0 = they are not
     int tilesWide() const;
     int exportRulebook(const int32_t* nbr, const int32_t* num_out, void* scratch,

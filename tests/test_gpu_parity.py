@@ -881,7 +881,7 @@ def test_fp16_ring_kernel_of_the_last_layer_gives_the_same_bits_launch_after_lau
 
 
 # ---------------------------------------------------------------------------------------------
-# the FP32 kernel with one tall tile per compute unit (conv_wide.hip: 64 -> 64 and 32 -> 64)
+# the FP32 kernel (conv_wide.hip)
 # ---------------------------------------------------------------------------------------------
 def _fp32_subm_wide_against_oracle(n, mv, grid, seed, clustered=True, epilogue=True, threads=1, cin=64):
     rng = np.random.default_rng(seed)
@@ -929,7 +929,7 @@ def test_wide_fp32_kernel_tall_tiles_and_two_tiles_per_workgroup(n, clustered, c
 @pytest.mark.parametrize("cin", [64, 32])
 @pytest.mark.parametrize("n", [3071, 3072, 3073, 10239, 10240, 10241])
 def test_wide_fp32_kernel_around_the_row_counts_of_its_column_splits(n, cin):
-    """On 256 compute units a tile's columns are dealt to four workgroups up to 3 072 rows, to two up to 10 240."""
+    """On 256 compute units the columns of a tile are dealt to two workgroups up to 10 240 rows."""
     _fp32_subm_wide_against_oracle(n, n + 7, (11, 200, 176), 900 + n, threads=8, cin=cin)
 
 
@@ -955,7 +955,7 @@ def test_every_row_is_a_pad_row(cin, cout, half):
 @pytest.mark.parametrize("n", [1, 65, 97, 1536, 1537, 5120, 5121, 12289, 20000])
 def test_wide_fp32_kernel_with_128_columns(n, cin):
     """128 output columns: two workgroups take 64 columns each of every tile (128 tiles a round on 256 compute units, of
-    up to 96 rows), up to 5 120 rows four, up to 1 536 rows eight; 128 input channels are walked in two parts.  Against
+    up to 96 rows), up to 5 120 rows four; 128 input channels are walked in two parts.  Against
     the oracle (pad rows included)."""
     rng = np.random.default_rng(n + cin)
     grid, mv = ((5, 40, 40) if n < 1000 else (21, 400, 352)), n + 39
@@ -973,4 +973,80 @@ def test_wide_fp32_kernel_with_128_columns(n, cin):
     assert np.array_equal(num, o_num)
     assert_features_close(out, o_out, RTOL_FP32, "wide fp32 %d->128, %d rows" % (cin, n),
                           abs_sum=abs_sum_of(feat, w, o_pairs, o_num, mv, mv, sc, sh))
+    conv.close()
+
+
+@pytest.mark.parametrize("cin,cout", [(4, 16), (4, 32), (16, 16), (16, 32), (32, 32)])
+@pytest.mark.parametrize("n", [1, 16, 63, 65, 129, 32767, 32769, 40000])
+def test_wide_fp32_kernel_with_few_columns(n, cin, cout):
+    """16 and 32 output columns: tiles of up to 128 (64) rows, one workgroup per compute unit up to 256 full tiles (32 768
+    rows with 16 columns, 16 384 with 32), two beyond.  Against the oracle (pad rows included)."""
+    rng = np.random.default_rng(n + cin)
+    grid, mv = ((5, 40, 40) if n < 1000 else (21, 400, 352)), n + 39
+    coors = F.clustered_active_voxels(n, grid, n, n_blobs=max(4, n // 100))
+    feat = rng.uniform(-1, 1, (n, cin)).astype(np.float32)
+    w = rng.normal(0, 0.1, (27, cin, cout)).astype(np.float32)
+    sc, sh = rng.uniform(0.5, 1.5, cout).astype(np.float32), rng.uniform(-0.2, 0.2, cout).astype(np.float32)
+    conv, out, pairs, num, cbuf = run_subm(coors, n, feat, w, grid, mv, sc, sh, True)
+    O.set_threads(16)
+    try:
+        o_pairs, o_num, _ = O.subm_rulebook(coors, n, grid[::-1], mv)
+        o_out = O.scale_shift_relu(O.gather_gemm_scatter(feat, w, o_pairs, o_num, mv), mv, sc, sh, True)
+    finally:
+        O.set_threads(1)
+    assert np.array_equal(num, o_num)
+    assert_features_close(out, o_out, RTOL_FP32, "fp32 %d->%d, %d rows" % (cin, cout, n),
+                          abs_sum=abs_sum_of(feat, w, o_pairs, o_num, mv, mv, sc, sh))
+    conv.close()
+
+
+def _sums_in_64_bits(feat, w, pairs, num, n):
+    with np.errstate(all="ignore"):
+        out = np.zeros((n, w.shape[2]))
+        for k in range(w.shape[0]):
+            i, o = pairs[k, 0, :num[k]], pairs[k, 1, :num[k]]
+            out[o] += (feat[i].astype(np.float64)[:, :, None] * w[k].astype(np.float64)[None]).sum(1)
+    return out
+
+
+@pytest.mark.parametrize("cin,cout", [(16, 32), (32, 32), (32, 64), (64, 64), (128, 128)])
+@pytest.mark.parametrize("lo,hi", [(-60, 60), (-110, -90), (60, 90)])
+def test_wide_fp32_kernel_keeps_32_bits_whatever_the_magnitude(cin, cout, lo, hi):
+    """Rows and columns of W of very different magnitude: the kernel multiplies 16-bit parts of the operands, whose range is
+    smaller than FP32's.  Bound: 27 * Cin terms of which each side is off by at most one unit in the last place of its
+    operands (2^-23 each) and of its sum: SUM_TOL times the sum of the terms' magnitudes, as everywhere in these tests."""
+    rng = np.random.default_rng([cin, lo + 200])
+    n, grid = 300, (5, 20, 20)
+    coors = F.clustered_active_voxels(n, grid, 3, n_blobs=4)
+    feat = (rng.uniform(-1, 1, (n, cin)) * 2.0 ** rng.integers(lo, hi, (n, 1))).astype(np.float32)
+    w = (rng.normal(0, 0.1, (27, cin, cout)) * 2.0 ** rng.integers(-20, 20, (1, 1, cout))).astype(np.float32)
+    conv, out, pairs, num, cbuf = run_subm(coors, n, feat, w, grid, n, None, None, False)
+    o_pairs, o_num, _ = O.subm_rulebook(coors, n, grid[::-1], n)
+    want = _sums_in_64_bits(feat, w, o_pairs, o_num, n)
+    A = _sums_in_64_bits(np.abs(feat), np.abs(w), o_pairs, o_num, n)
+    assert np.all(np.abs(out[:n] - want) <= 2e-6 * A + 2.0 ** -126)
+    conv.close()
+
+
+@pytest.mark.parametrize("cin,cout", [(4, 16), (16, 32), (32, 32), (32, 64), (64, 64), (64, 128), (128, 128)])
+def test_wide_fp32_kernel_infinities_and_nan(cin, cout):
+    """An infinity, a NaN and finite values whose products overflow reach the outputs that plain FP32 sums would make of them,
+    and no others."""
+    rng = np.random.default_rng(cin * cout)
+    n, grid = 400, (5, 30, 30)
+    coors = F.clustered_active_voxels(n, grid, 5, n_blobs=8)
+    feat = rng.uniform(0.5, 1, (n, cin)).astype(np.float32)
+    w = rng.uniform(0.5, 1, (27, cin, cout)).astype(np.float32) * rng.choice([-1, 1], (27, 1, cout)).astype(np.float32)
+    feat[10, 1], feat[60, 3], feat[150, 0] = np.inf, -np.inf, np.nan
+    feat[250] = np.finfo(np.float32).max  # (times a weight of half and more, Cin times: beyond the range, of one sign per offset)
+    conv, out, pairs, num, cbuf = run_subm(coors, n, feat, w, grid, n, None, None, False)
+    o_pairs, o_num, _ = O.subm_rulebook(coors, n, grid[::-1], n)
+    want = _sums_in_64_bits(feat, w, o_pairs, o_num, n)
+    out = out[:n]
+    assert np.array_equal(np.isnan(out), np.isnan(want))
+    big = ~np.isnan(want) & (np.abs(want) > 3.5e38)  # (infinities and sums beyond the range)
+    assert big.sum() > cout and np.array_equal(out[big], np.where(want[big] > 0, np.inf, -np.inf))
+    rest = ~np.isnan(want) & (np.abs(want) < 1e30)
+    A = _sums_in_64_bits(np.abs(feat), np.abs(w), o_pairs, o_num, n)
+    assert rest.sum() > n and np.all(np.abs(out[rest] - want[rest]) <= 2e-6 * A[rest])
     conv.close()
