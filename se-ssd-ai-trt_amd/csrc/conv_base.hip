@@ -99,10 +99,10 @@ int ConvPluginBase::preparePacked() {
 bool ConvPluginBase::gemmOnMatrixCores() const {
     return weights_packed_dev_ != nullptr && !(flags_ & SESSD_FLAG_FORCE_VALU) &&
            gemm_runs_on_mfma(kernel_volume_, in_channel_, out_channel_, in_type_, out_type_) &&
-           (in_type_ == SESSD_HALF || max_voxels_ < 1 << 24);  // (a pair of conv_wide.hip keeps its input row in 24 bits)
+           gemm_wide_takes_rows(max_voxels_, in_channel_, in_type_);
 }
 
-int ConvPluginBase::tileRows() const { return gemm_tile_rows(in_channel_, out_channel_, out_type_); }
+int ConvPluginBase::tileRows() const { return gemm_wide_tile_rows(out_channel_, out_type_); }
 int ConvPluginBase::tilesWide() const {
     return gemm_runs_wide(kernel_volume_, in_channel_, out_channel_, in_type_, out_type_) ? (out_channel_ > 64 ? out_channel_ / 64 : 1) : 0;
 }

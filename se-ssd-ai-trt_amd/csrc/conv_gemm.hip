@@ -192,8 +192,6 @@ export_pairs(const int32_t* __restrict__ nbr, int max_voxels, int words_per_k,
 
 }  // namespace
 
-int launch_mfma(const GemmArgs& a, hipStream_t stream);  // conv_mfma.hip
-
 int launch_tall(const GemmArgs& a, hipStream_t stream);  // conv_tall.hip
 bool gemm_runs_tall(int K, int cin, int cout);
 int launch_tile(const GemmArgs& a, hipStream_t stream);  // conv_tile.hip
@@ -210,12 +208,8 @@ int launch_gather_gemm(const GemmArgs& a, hipStream_t stream) {
         if (rc == SESSD_E_UNSUPPORTED) rc = launch_tall(a, stream);
         if (rc != SESSD_E_UNSUPPORTED) return rc;
     }
-    if (!a.force_valu) {  // FP32, and the first layer of an FP16 pipeline
+    if (!a.force_valu) {  // FP32, FP16 below 32 input channels, kernel volumes that the two above do not take
         const int rc = launch_wide(a, stream);
-        if (rc != SESSD_E_UNSUPPORTED) return rc;
-    }
-    if (!a.force_valu) {
-        const int rc = launch_mfma(a, stream);
         if (rc != SESSD_E_UNSUPPORTED) return rc;  // launched (or failed for good)
     }
     if (a.dense.dense) return fail(SESSD_E_UNSUPPORTED, "gather-GEMM: the fused dense scatter needs the MFMA kernel");

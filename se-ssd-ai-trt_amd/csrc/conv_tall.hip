@@ -2,7 +2,7 @@
 //
 //     out[o][:] = epilogue( sum_k  in[nbr[k][o]][:] @ W[k] )
 //
-// The split-K kernel of conv_mfma.hip requests all of W once per 48..64-row tile; in FP16, where the matrix cores
+// A kernel with short tiles requests all of W once per 48 or 64 rows; in FP16, where the matrix cores
 // are far from busy, those requests are what the compute units' load path spends its time on.  Here a workgroup (4
 // wave64) owns 64 or 128 consecutive output rows:
 //   * W[k] is copied once per workgroup and offset into LDS (two buffers; the host's MFMA operand order is also

@@ -1,4 +1,5 @@
-// conv_wide.hip -- FP32 gather-GEMM (all matrix-core shapes; with Cin 4 also the first layer of an FP16 pipeline).
+// conv_wide.hip -- gather-GEMM of the FP32 layers, of the FP16 layers that conv_tile.hip and conv_tall.hip do not take (Cin 16, kernel
+// volumes other than theirs) and of an FP16 pipeline's first layer.
 //
 //     out[o][:] = epilogue( sum_k  in[nbr[k][o]][:] @ W[k] )
 //
@@ -35,12 +36,15 @@
 // unit would be higher than that (32 -> 32, eight waves, 4 208 rows: one workgroup a unit 7.9 us, two 10.7).  What LDS they leave is what the
 // coordinate passes of a frame's other branch run in: 32 -> 32 with eight waves is the faster launch (15.9 us against 17.1 at
 // 28 043 rows) and makes the slower frame (20 000 points: 283 us against 274); 4 -> 32 likewise (487 against 475).
+// FP16 features (Cin 16) have so little in each block that four waves and 64 rows do: four workgroups share a unit, with 40 KB of LDS
+// each.  From 32 channels up FP16 is faster without pair lists (32 -> 32 at 45 874 rows 10.6 us on conv_tall.hip, 18 here).
 //
 // Launches of SubM layers at the sites of scans, us, before (split-K on four waves, or sixteen waves of 16 columns, both with
 // the FP32 instruction) -> now: 64 -> 64 at 2 448 rows 10.4 -> 9.4, 8 662 20.7 -> 14.7, 17 262 31.7 -> 19.2 (99 TFLOP/s), 23 959 48.4
 // -> 30.7; 128 -> 128 at 3 594 rows 31.2 -> 19.3, 17 262 120 -> 57 (134 TFLOP/s); 64 -> 128 at 17 262 57 -> 35; 32 -> 64 at 28 043 32
 // -> 26; 32 -> 32 at 4 208 9.4 -> 8.9, 28 043 19.1 -> 16.9, 45 874 35.9 -> 27.9; 16 -> 16 at 17 132 8.3 -> 7.3; 4 -> 16 7.4 -> 6.5.  16 -> 32
-// 10.2 -> 9.0, but 14.9 -> 16.8 at 36 871 rows (a second round of tiles begins at 32 768).
+// 10.2 -> 9.0, but 14.9 -> 16.8 at 36 871 rows (a second round of tiles begins at 32 768).  FP16 16 -> 16 at 1 901 rows 6.3 -> 5.9, 60 000
+// 14.2 -> 10.8; 16 -> 32 6.7 -> 6.2, 16.6 -> 12.9.
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -58,6 +62,8 @@ typedef float v2f __attribute__((ext_vector_type(2)));
 typedef __bf16 v2b __attribute__((ext_vector_type(2)));
 typedef __bf16 v8b __attribute__((ext_vector_type(8)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef unsigned int v2u32 __attribute__((__vector_size__(8)));
 typedef unsigned int v4u32 __attribute__((__vector_size__(16)));
 
 constexpr int kMaxK = kGemmMaxOffsets;
@@ -65,29 +71,30 @@ constexpr unsigned kOutOfRange = 0x80000000u;  // beyond any buffer the kernel i
 constexpr int kRawBuffer = 0x00020000;         // descriptor word 3: raw 32-bit data format, no swizzle
 
 // how a layer's products are made: FP32 MFMA, or 16-bit MFMA on operands split into parts
-enum Arith { kPlain, kThirds, kHalves };
-constexpr Arith arith(int cin) { return cin >= 64 ? kHalves : (cin >= 32 ? kThirds : kPlain); }
+enum Arith { kPlain, kThirds, kHalves, kFp16 };
+constexpr Arith arith(int cin) { return cin >= 64 ? kHalves : (cin >= 32 ? kThirds : kPlain); }  // (of FP32 features)
 
-template <int CIN, int COUT>
+template <typename T, int CIN, int COUT>  // T: the input features' type
 struct Shape {
-    static constexpr Arith kArith = arith(CIN);
-    static constexpr int kWeightBytes = CIN * COUT * (kArith == kThirds ? 6 : 4);  // of an offset
+    static constexpr Arith kArith = sizeof(T) == 2 ? kFp16 : arith(CIN);
+    static constexpr int kWeightBytes = CIN * COUT * (kArith == kFp16 ? 2 : (kArith == kThirds ? 6 : 4));  // of an offset
     static constexpr int kWgCols = COUT < 64 ? COUT : 64;  // columns of a workgroup (before the split of short tiles)
     static constexpr int kColGroups = COUT / kWgCols;      // workgroups beside each other
     // (32 columns: four waves with 4 and 32 channels, whose launches are long enough for the frame's other branch to need the LDS)
-    static constexpr int kWaves = kWgCols == 64 ? 6 : (COUT == 32 && CIN != 16 ? 4 : 8);
+    static constexpr int kWaves = kWgCols == 64 ? 6 : (sizeof(T) == 2 || (COUT == 32 && CIN != 16) ? 4 : 8);
     static constexpr int kThreads = kWaves * 64;
-    static constexpr int kTileRows = kWgCols == 64 ? 96 : (kWgCols == 32 ? 64 : 112);  // tile capacity
-    static constexpr int kPerUnit = kWgCols == 64 ? 1 : 2;  // workgroups that can share a compute unit
+    static constexpr int kTileRows = kWgCols == 64 ? 96 : (sizeof(T) == 2 || kWgCols == 32 ? 64 : 112);  // tile capacity
+    static constexpr int kPerUnit = kWgCols == 64 ? 1 : (sizeof(T) == 2 ? 4 : 2);  // workgroups that can share a compute unit
     static constexpr int kMaxBlk = kTileRows / 16;
     static constexpr int kNone = kMaxK * kTileRows * 4;  // an item with no pairs
     static constexpr int kParts = CIN > 64 ? CIN / 64 : 1;  // of the inner dimension, taken one after the other
     static constexpr int CP = CIN / kParts;                 // channels of a part
-    static constexpr int G = CP < 16 ? 1 : CP / 16;         // pieces of a row that a lane requests: 4 channels each (Cin 4: 1)
-    static constexpr int kLaneBytes = CP < 16 ? 4 : 16;     // ... in bytes; of a weight operand as well
+    static constexpr int kRowBytes = CIN * (int)sizeof(T), kPartBytes = CP * (int)sizeof(T);
+    static constexpr int kLaneBytes = kPartBytes < 64 ? kPartBytes / 4 : 16;  // of a row that a lane requests at a time; of a weight operand as well
+    static constexpr int G = kPartBytes / (4 * kLaneBytes);  // requests for a part
     static constexpr int kMaxSplit = kWgCols == 64 ? 1 : 0;  // log2 of the column parts that short tiles are split into
     static_assert(kTileRows <= 128 && kTileRows % 16 == 0, "the lists are staged in two halves of 64 rows");
-    static_assert((CP == 4 || CP % 16 == 0) && (kArith == kPlain || CP % 32 == 0) && COUT % kWgCols == 0, "whole MFMA steps and column groups");
+    static_assert((CP == 4 || CP % 16 == 0) && (kArith == kPlain || kArith == kFp16 || CP % 32 == 0) && COUT % kWgCols == 0, "whole MFMA steps and column groups");
     static_assert((kMaxK + kWaves - 1) / kWaves * kMaxBlk * kParts + 2 <= 64, "an item a lane");
 };
 constexpr uint32_t kNoPair = 0xffffff00u;      // entry of a pair list that fills up its last block (no input row has that number)
@@ -96,6 +103,11 @@ __device__ __forceinline__ void buffer_load(__amdgpu_buffer_rsrc_t r, unsigned b
     const v4u32 t = __builtin_amdgcn_raw_buffer_load_b128(r, byte_offset, 0, 0);
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = (int)t[e];
+}
+__device__ __forceinline__ void buffer_load(__amdgpu_buffer_rsrc_t r, unsigned byte_offset, int (&v)[2]) {
+    const v2u32 t = __builtin_amdgcn_raw_buffer_load_b64(r, byte_offset, 0, 0);
+    v[0] = (int)t[0];
+    v[1] = (int)t[1];
 }
 __device__ __forceinline__ void buffer_load(__amdgpu_buffer_rsrc_t r, unsigned byte_offset, int (&v)[1]) {
     v[0] = (int)__builtin_amdgcn_raw_buffer_load_b32(r, byte_offset, 0, 0);
@@ -138,13 +150,38 @@ __device__ __forceinline__ V operand8(const int* w) {
 
 // What a lane holds of a 16-pair block's rows (Rows, in the order of the request; words that a lane permutation brings to
 // the operands) and of an offset's weights, and the products of the two.
-template <int CIN, int COUT, int NB, Arith>
+template <typename S, int NB, Arith>
 struct Products;
 
+// FP16 features: their own MFMA
+template <typename S, int NB>
+struct Products<S, NB, kFp16> {
+    static constexpr int G = S::G, E = S::kLaneBytes / 4, kWords = G * E, kPieces = G;
+    static __device__ __forceinline__ void take(const int (&a)[G][E], int (&p)[kWords]) {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int e = 0; e < E; ++e) p[g * E + e] = a[g][e];
+    }
+    static __device__ __forceinline__ void multiply(const int (&w)[G][NB][E], const int (&x)[kWords], v4f (&acc)[NB]) {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                if constexpr (E == 4) {
+                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(operand8<v8h>(w[g][nb]), operand8<v8h>(x + g * E), acc[nb], 0, 0, 0);
+                } else {
+                    const int2 a = make_int2(w[g][nb][0], w[g][nb][1]), b = make_int2(x[g * E], x[g * E + 1]);
+                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(v4h, a), __builtin_bit_cast(v4h, b), acc[nb], 0, 0, 0);
+                }
+            }
+    }
+    static __device__ __forceinline__ float add(float p, const int (&)[kWords], float sum) { return sum + p; }
+};
+
 // FP32 MFMA
-template <int CIN, int COUT, int NB>
-struct Products<CIN, COUT, NB, kPlain> {
-    using S = Shape<CIN, COUT>;
+template <typename S, int NB>
+struct Products<S, NB, kPlain> {
     static constexpr int G = S::G, E = S::kLaneBytes / 4, kWords = G * E, kPieces = G;  // (pieces: weight operands a column block)
     static __device__ __forceinline__ void take(const int (&a)[G][E], int (&p)[kWords]) {
 #pragma unroll
@@ -165,9 +202,8 @@ struct Products<CIN, COUT, NB, kPlain> {
 };
 
 // BF16 MFMA on three parts of eight bits each: x = x0 + x1 + x2 exactly; the products down to 2^-24 of the largest, smallest first
-template <int CIN, int COUT, int NB>
-struct Products<CIN, COUT, NB, kThirds> {
-    using S = Shape<CIN, COUT>;
+template <typename S, int NB>
+struct Products<S, NB, kThirds> {
     static constexpr int G = S::G, E = 4, C = S::CP / 32, kWords = G * 6, kPieces = 3 * C;  // (words: x0, x1, x2)
     static __device__ __forceinline__ void take(const int (&a)[G][E], int (&p)[kWords]) {
 #pragma unroll
@@ -200,9 +236,8 @@ struct Products<CIN, COUT, NB, kThirds> {
 };
 
 // FP16 MFMA on the halves of both sides: low * high and high * low, then high * high, one accumulator
-template <int CIN, int COUT, int NB>
-struct Products<CIN, COUT, NB, kHalves> {
-    using S = Shape<CIN, COUT>;
+template <typename S, int NB>
+struct Products<S, NB, kHalves> {
     static constexpr int G = S::G, E = 4, C = S::CP / 32, kWords = G * 4 + 1, kPieces = 2 * C;  // (words: high, low, power of two)
     static __device__ __forceinline__ void take(const int (&a)[G][E], int (&p)[kWords]) {
         // the row's largest magnitude -> power of two that brings it to [2^14, 2^15)
@@ -242,11 +277,10 @@ struct Products<CIN, COUT, NB, kHalves> {
 
 // One wave's share of a tile: the pairs of the offsets dealt to it, times its columns -- 16-column blocks nb0 .. nb0 + NB - 1
 // of the layer -- into its partial tile `part` (rows of 16 NB floats).
-template <int CIN, int COUT, int NB>
+template <typename S, int COUT, int NB>
 __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_buffer_rsrc_t rs_w, const uint32_t* s_pair,
                                          const int32_t* s_blk, int K, int wave, int lane, int nb0, float* part) {
-    using S = Shape<CIN, COUT>;
-    using P = Products<CIN, COUT, NB, S::kArith>;
+    using P = Products<S, NB, S::kArith>;
     constexpr int kParts = S::kParts, G = S::G, E = S::kLaneBytes / 4, kWaves = S::kWaves, kTileRows = S::kTileRows;
     constexpr int NBT = COUT / 16;                   // 16-column blocks of the layer
     constexpr int kSlots = NB * 4;                   // 16-byte slots of a row of the partial tile
@@ -299,7 +333,7 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
     const char* pairs = reinterpret_cast<const char*>(s_pair);
     auto entry_at = [&](int it, int j4) -> uint32_t { return *reinterpret_cast<const uint32_t*>(pairs + (kParts > 1 ? it & ~3 : it) + j4); };
     auto load_a = [&](int it, uint32_t entry, int (&a)[G][E]) {
-        const unsigned row = (entry >> 8) * (unsigned)(CIN * sizeof(float)) + (kParts > 1 ? (unsigned)(it & 3) * (unsigned)(S::CP * sizeof(float)) : 0u);
+        const unsigned row = (entry >> 8) * (unsigned)S::kRowBytes + (kParts > 1 ? (unsigned)(it & 3) * (unsigned)S::kPartBytes : 0u);
         const unsigned at = entry < kNoPair ? row + (lane & 3) * (unsigned)S::kLaneBytes : kOutOfRange;
 #pragma unroll
         for (int g = 0; g < G; ++g) buffer_load(rs_in, at + g * 64u, a[g]);
@@ -396,13 +430,13 @@ __device__ __forceinline__ void direct_sum(const float* __restrict__ in, const f
 
 // DENSE: the epilogue also scatters the rows into a dense tensor (the layer in front of sparse2Dense).  PAD: the rows beyond the
 // active ones are written too.  Variants of their own: what they need in registers is missing in the launches without.
-template <int CIN, int COUT, typename TO, bool DENSE, bool PAD>
-__global__ void __launch_bounds__((Shape<CIN, COUT>::kThreads), (Shape<CIN, COUT>::kWaves * Shape<CIN, COUT>::kPerUnit / 4))
-conv_wide(const float* __restrict__ in, TO* __restrict__ out, const void* __restrict__ Wp, const float* __restrict__ w_f32,
+template <int CIN, int COUT, typename T, typename TO, bool DENSE, bool PAD>
+__global__ void __launch_bounds__((Shape<T, CIN, COUT>::kThreads), (Shape<T, CIN, COUT>::kWaves * Shape<T, CIN, COUT>::kPerUnit / 4))
+conv_wide(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict__ Wp, const float* __restrict__ w_f32,
           const int32_t* __restrict__ nbr, const int32_t* __restrict__ num_out, int max_voxels, int K,
           const float* __restrict__ scale, const float* __restrict__ shift, int relu, int units,
           const int32_t* __restrict__ tiles, DenseTarget dt) {
-    using S = Shape<CIN, COUT>;
+    using S = Shape<T, CIN, COUT>;
     constexpr int kWgCols = S::kWgCols, kMaxSplit = S::kMaxSplit, kTileRows = S::kTileRows, kWaves = S::kWaves, kThreads = S::kThreads;
     // (one block more: all of it filling pairs)
     __shared__ uint32_t s_pair[kMaxK * kTileRows + 16];  // compacted pair lists: pair j of offset k, input row << 8 | local output row
@@ -450,14 +484,18 @@ conv_wide(const float* __restrict__ in, TO* __restrict__ out, const void* __rest
     // The grid is one workgroup per compute unit (a workgroup takes most of a unit's LDS, so workgroups with no
     // tile would queue behind the busy ones just to return); a workgroup walks tiles first_tile, first_tile +
     // row_groups, ...: runs of rows from the rulebook's equal-work cuts, or runs of equal length.
-    // (Two workgroups share a unit only where one tile for each unit would not do: a tile's weights are the same for any height.)
-    const int walkers = S::kPerUnit > 1 && cut_count == 0 && n <= units / S::kPerUnit * kTileRows ? units / S::kPerUnit : row_groups;
+    // (Workgroups share a unit only where one tile for each unit would be higher than they are: a tile's weights are the same for any height.)
+    int walkers = row_groups;
+    if (S::kPerUnit > 1 && cut_count == 0) {
+        const int per_unit = (n + units / S::kPerUnit * kTileRows - 1) / (units / S::kPerUnit * kTileRows);
+        walkers = units / S::kPerUnit * (per_unit < 1 ? 1 : (per_unit > S::kPerUnit ? S::kPerUnit : per_unit));
+    }
     TilePlan plan = {0, 0};
     if (cut_count == 0) plan = tile_plan(n, walkers, kTileRows);
     const int tile_count = cut_count > 0 ? cut_count : (n > 0 ? plan.count : 0);
     const int first_begin = cut_begin[kMaxSplit ? lsplit : 0], first_end = cut_end[kMaxSplit ? lsplit : 0];
     const __amdgpu_buffer_rsrc_t rs_in = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(in), 0, (int)((size_t)max_voxels * CIN * sizeof(float)), kRawBuffer);
+        const_cast<T*>(in), 0, (int)((size_t)max_voxels * S::kRowBytes), kRawBuffer);
     const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<void*>(Wp), 0, (int)((size_t)K * S::kWeightBytes), kRawBuffer);
 
@@ -518,8 +556,8 @@ conv_wide(const float* __restrict__ in, TO* __restrict__ out, const void* __rest
     }
     __syncthreads();
     if constexpr (kMaxSplit)
-        if (lsplit) multiply<CIN, COUT, kWgCols / 32>(rs_in, rs_w, s_pair, s_blk, K, wave, lane, col_first / 16, part);
-    if (!kMaxSplit || !lsplit) multiply<CIN, COUT, kWgCols / 16>(rs_in, rs_w, s_pair, s_blk, K, wave, lane, col_first / 16, part);
+        if (lsplit) multiply<S, COUT, kWgCols / 32>(rs_in, rs_w, s_pair, s_blk, K, wave, lane, col_first / 16, part);
+    if (!kMaxSplit || !lsplit) multiply<S, COUT, kWgCols / 16>(rs_in, rs_w, s_pair, s_blk, K, wave, lane, col_first / 16, part);
     __syncthreads();
 
     // fixed-order sum of the waves' partial tiles, epilogue, coalesced stores; the sums of kAtOnce vectors are read together
@@ -559,7 +597,8 @@ conv_wide(const float* __restrict__ in, TO* __restrict__ out, const void* __rest
         if (r >= rows) break;
         float o[4] = {sums[u].x, sums[u].y, sums[u].z, sums[u].w};
         bool finite = true;
-        if constexpr (S::kArith != kPlain) {
+        constexpr bool kParted = S::kArith == kThirds || S::kArith == kHalves;
+        if constexpr (kParted) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 if (S::kArith == kHalves) o[e] *= e_col[e];
@@ -567,7 +606,8 @@ conv_wide(const float* __restrict__ in, TO* __restrict__ out, const void* __rest
             }
         }
         // the parts of an infinity, or a sum beyond their range, say nothing: the products themselves
-        if (S::kArith != kPlain && !finite) direct_sum<CIN, COUT>(in, w_f32, nbr + row0 + r, max_voxels, K, ec4, o);
+        if constexpr (kParted)
+            if (!finite) direct_sum<CIN, COUT>(in, w_f32, nbr + row0 + r, max_voxels, K, ec4, o);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             float s = o[e];
@@ -603,17 +643,16 @@ conv_wide(const float* __restrict__ in, TO* __restrict__ out, const void* __rest
     }
 }
 
-template <int CIN, int COUT, typename TO = float>
+template <int CIN, int COUT, typename T = float, typename TO = T>
 int launch(const GemmArgs& a, hipStream_t stream) {
     // operands are addressed with 32-bit byte offsets, 2^31 means "out of range"; a pair keeps its input row in 24 bits
-    if ((size_t)a.max_voxels * CIN * sizeof(float) >= kOutOfRange || (size_t)a.K * Shape<CIN, COUT>::kWeightBytes >= kOutOfRange ||
-        a.max_voxels >= 1 << 24)
+    if (!gemm_wide_takes_rows(a.max_voxels, CIN, a.in_type) || (size_t)a.K * Shape<T, CIN, COUT>::kWeightBytes >= kOutOfRange)
         return SESSD_E_UNSUPPORTED;
-    using S = Shape<CIN, COUT>;
+    using S = Shape<T, CIN, COUT>;
     const int units = gemm_compute_units() * S::kPerUnit / S::kColGroups;
     auto go = [&](auto dense, auto pad) {
-        hipLaunchKernelGGL((conv_wide<CIN, COUT, TO, decltype(dense)::value, decltype(pad)::value>), dim3((unsigned)(units * S::kColGroups)),
-                           dim3(S::kThreads), 0, stream, static_cast<const float*>(a.in_feat), static_cast<TO*>(a.out_feat), a.w_packed,
+        hipLaunchKernelGGL((conv_wide<CIN, COUT, T, TO, decltype(dense)::value, decltype(pad)::value>), dim3((unsigned)(units * S::kColGroups)),
+                           dim3(S::kThreads), 0, stream, static_cast<const T*>(a.in_feat), static_cast<TO*>(a.out_feat), a.w_packed,
                            a.w_f32, a.nbr, a.num_out, a.max_voxels, a.K, a.scale, a.shift, a.relu, units, a.tiles, a.dense);
     };
     if (a.dense.dense) a.write_pad_rows ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
@@ -625,16 +664,24 @@ int launch(const GemmArgs& a, hipStream_t stream) {
 }  // namespace
 
 bool gemm_runs_wide(int K, int cin, int cout, int in_type, int out_type) {
-    if (in_type != SESSD_FLOAT || K > kMaxK) return false;
-    if (cin == 4) return cout == 16 || cout == 32;  // (the first layer of an FP16 pipeline as well)
-    if (out_type != SESSD_FLOAT) return false;
+    if (K > kMaxK) return false;
+    if (cin == 4) return in_type == SESSD_FLOAT && (cout == 16 || cout == 32);  // (the first layer of an FP16 pipeline as well)
+    if (in_type != out_type) return false;
     const int shapes[][2] = {{16, 16}, {16, 32}, {32, 32}, {32, 64}, {64, 64}, {64, 128}, {128, 128}};
     for (auto& s : shapes)
         if (s[0] == cin && s[1] == cout) return true;
     return false;
 }
 
-int gemm_wide_tile_rows(int cout) { return cout >= 64 ? Shape<64, 64>::kTileRows : (cout >= 32 ? Shape<32, 32>::kTileRows : Shape<16, 16>::kTileRows); }
+// (a kernel that has a shape to itself takes more; the pipeline asks before it relies on the fused scatter)
+bool gemm_wide_takes_rows(int max_voxels, int cin, int in_type) {
+    return max_voxels < 1 << 24 && (size_t)max_voxels * cin * (in_type == SESSD_HALF ? 2 : 4) < kOutOfRange;
+}
+
+int gemm_wide_tile_rows(int cout, int type) {
+    if (cout >= 64) return Shape<float, 64, 64>::kTileRows;
+    return type == SESSD_HALF || cout >= 32 ? Shape<float, 32, 32>::kTileRows : Shape<float, 16, 16>::kTileRows;
+}
 
 bool wide_splits(int cin) { return arith(cin) != kPlain; }
 size_t wide_weight_bytes(int K, int cin, int cout) {
@@ -691,15 +738,18 @@ void pack_wide_weights(const float* w, int K, int cin, int cout, void* dst) {
 int launch_wide(const GemmArgs& a, hipStream_t stream) {
     if (!a.w_packed || !gemm_runs_wide(a.K, a.cin, a.cout, a.in_type, a.out_type)) return SESSD_E_UNSUPPORTED;
     if ((reinterpret_cast<uintptr_t>(a.in_feat) | reinterpret_cast<uintptr_t>(a.out_feat)) & 15) return SESSD_E_UNSUPPORTED;
-    if (a.cin == 4 && a.out_type == SESSD_HALF) return a.cout == 16 ? launch<4, 16, __half>(a, stream) : launch<4, 32, __half>(a, stream);
+    if (a.cin == 4 && a.out_type == SESSD_HALF) return a.cout == 16 ? launch<4, 16, float, __half>(a, stream) : launch<4, 32, float, __half>(a, stream);
     if (a.cin == 4) return a.cout == 16 ? launch<4, 16>(a, stream) : launch<4, 32>(a, stream);
-    if (a.cin == 16 && a.cout == 16) return launch<16, 16>(a, stream);
-    if (a.cin == 16 && a.cout == 32) return launch<16, 32>(a, stream);
-    if (a.cin == 32 && a.cout == 32) return launch<32, 32>(a, stream);
-    if (a.cin == 64 && a.cout == 64) return launch<64, 64>(a, stream);
-    if (a.cin == 32 && a.cout == 64) return launch<32, 64>(a, stream);
-    if (a.cin == 64 && a.cout == 128) return launch<64, 128>(a, stream);
-    if (a.cin == 128 && a.cout == 128) return launch<128, 128>(a, stream);
+#define SESSD_CASE(CI, CO) \
+    if (a.cin == CI && a.cout == CO) return a.in_type == SESSD_HALF ? launch<CI, CO, __half>(a, stream) : launch<CI, CO>(a, stream)
+    SESSD_CASE(16, 16);
+    SESSD_CASE(16, 32);
+    SESSD_CASE(32, 32);
+    SESSD_CASE(32, 64);
+    SESSD_CASE(64, 64);
+    SESSD_CASE(64, 128);
+    SESSD_CASE(128, 128);
+#undef SESSD_CASE
     return SESSD_E_UNSUPPORTED;
 }
 

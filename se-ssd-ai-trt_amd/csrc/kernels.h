@@ -31,7 +31,7 @@ struct GemmArgs {
 // r = the smallest tiles-per-CU count that keeps the mean tile at or below the target height, so that every
 // CU gets the same number of tiles (a fixed 32-row tiling leaves e.g. 529 tiles for 256 CUs: some CUs run
 // three tiles, most two, and the kernel lasts as long as the three).
-// The target is the tile capacity of the kernel the rulebook's owner runs (gemm_tile_rows()): the tallest
+// The target is the tile capacity of the kernel the rulebook's owner runs (gemm_wide_tile_rows()): the tallest
 // tiles the quantisation to whole tiles per CU allows.  Any cut is correct for any kernel: runs longer than
 // a kernel's capacity are walked in pieces.
 constexpr int kGemmMinTileRows = 48;  // smallest capacity of any kernel: bounds the tile count
@@ -61,8 +61,6 @@ __host__ __device__ inline int wide_log2_split(int n, int K, int num_cu) {
     if (num_cu % 2 || K < kWideSplitMinOffsets) return 0;
     return n <= num_cu / 2 * kWideSplitRows ? 1 : 0;
 }
-// tile capacity (rows) of the MFMA kernel that serves this layer shape
-int gemm_tile_rows(int cin, int cout, int dtype);
 int gemm_compute_units();
 
 // bytes of a layer's workspace for the equal-work tile cuts of its rulebook (tile_cut.hip, coord.h); the region's first
@@ -76,10 +74,11 @@ bool gemm_runs_on_mfma(int K, int cin, int cout, int in_type, int out_type);
 // whether the layer runs on one of the FP16 kernels (conv_tile.hip, conv_tall.hip) that cut their own tiles: a rulebook
 // whose owner does needs no equal-work cuts
 bool gemm_cuts_own_tiles(int K, int cin, int cout, int in_type, int out_type);
-// whether the layer runs on the FP32 kernel (conv_wide.hip), that kernel's tile capacity, and whether it multiplies 16-bit
-// parts of the operands, which need weights of a form of their own
+// whether the layer runs on conv_wide.hip's kernel (where the two above leave it), that kernel's tile capacity, how many rows it
+// takes, and whether it multiplies 16-bit parts of FP32 operands, which need weights of a form of their own
 bool gemm_runs_wide(int K, int cin, int cout, int in_type, int out_type);
-int gemm_wide_tile_rows(int cout);
+int gemm_wide_tile_rows(int cout, int type);
+bool gemm_wide_takes_rows(int max_voxels, int cin, int in_type);
 bool wide_splits(int cin);
 size_t wide_weight_bytes(int K, int cin, int cout);
 void pack_wide_weights(const float* w, int K, int cin, int cout, void* dst);

@@ -977,9 +977,9 @@ def test_wide_fp32_kernel_with_128_columns(n, cin):
 
 
 @pytest.mark.parametrize("cin,cout", [(4, 16), (4, 32), (16, 16), (16, 32), (32, 32)])
-@pytest.mark.parametrize("n", [1, 16, 63, 65, 129, 32767, 32769, 40000])
+@pytest.mark.parametrize("n", [1, 16, 63, 65, 113, 129, 16385, 28672, 28673, 40000])
 def test_wide_fp32_kernel_with_few_columns(n, cin, cout):
-    """16 and 32 output columns: tiles of up to 128 (64) rows, one workgroup per compute unit up to 256 full tiles (32 768
+    """16 and 32 output columns: tiles of up to 112 (64) rows, one workgroup per compute unit up to 256 full tiles (28 672
     rows with 16 columns, 16 384 with 32), two beyond.  Against the oracle (pad rows included)."""
     rng = np.random.default_rng(n + cin)
     grid, mv = ((5, 40, 40) if n < 1000 else (21, 400, 352)), n + 39
@@ -997,6 +997,32 @@ def test_wide_fp32_kernel_with_few_columns(n, cin, cout):
     assert np.array_equal(num, o_num)
     assert_features_close(out, o_out, RTOL_FP32, "fp32 %d->%d, %d rows" % (cin, cout, n),
                           abs_sum=abs_sum_of(feat, w, o_pairs, o_num, mv, mv, sc, sh))
+    conv.close()
+
+
+@pytest.mark.parametrize("cout", [16, 32])
+@pytest.mark.parametrize("n", [1, 63, 65, 16383, 16385, 40000, 65537])
+def test_fp16_kernel_with_16_channels(n, cout):
+    """FP16, 16 input channels: tiles of up to 64 rows, one to four workgroups per compute unit (16 384 rows each on 256 units),
+    a second round of tiles beyond 65 536 rows.  Against the oracle (pad rows included), one rounding to half apart."""
+    rng = np.random.default_rng(n + cout)
+    grid, mv = ((5, 40, 40) if n < 1000 else (21, 400, 352)), n + 39
+    coors = F.clustered_active_voxels(n, grid, n, n_blobs=max(4, n // 100))
+    feat = O.round_to_half(rng.uniform(-1, 1, (n, 16)).astype(np.float32))
+    w = O.round_to_half(rng.normal(0, 0.1, (27, 16, cout)).astype(np.float32))
+    cbuf, fbuf = np.zeros((mv, 4), np.int32), np.zeros((mv, 16), np.float32)
+    cbuf[:n], fbuf[:n] = coors, feat
+    conv = api.SubmConv3d(16, cout, grid[::-1], w, mv)
+    out = conv(dev(fbuf, torch.float16), dev(cbuf), dev(np.array([n], np.int32)), out_dtype=torch.float16)
+    torch.cuda.synchronize()
+    O.set_threads(16)
+    try:
+        o_pairs, o_num, _ = O.subm_rulebook(coors, n, grid[::-1], mv)
+        o_out = O.gather_gemm_scatter(feat, w, o_pairs, o_num, mv)
+    finally:
+        O.set_threads(1)
+    assert_features_close(to_np(out.float()), O.round_to_half(o_out), RTOL_FP16, "fp16 16->%d, %d rows" % (cout, n), half=True,
+                          abs_sum=abs_sum_of(feat, w, o_pairs, o_num, mv, mv))
     conv.close()
 
 
