@@ -39,6 +39,107 @@ subm_insert(const int32_t* __restrict__ coors, const int32_t* __restrict__ voxel
     if (insert_min(open_table(table, n), key, (uint32_t)v) < 0) atomicOr(&meta[0], SESSD_STATUS_HASH_FULL);
 }
 
+// The whole rulebook of a layer of few rows in one launch: every workgroup keeps the cells of all rows in a hash table of its own,
+// in LDS, and looks up the neighbours of 64 rows.  Clearing, filling and reading a table in memory are three launches, which is what
+// a small layer spends its time on.  The table is lists of rows, one for each hash value: a row enters with one exchange, where the
+// probes of an open table, each waiting for the one before, took 8 us for 2 000 rows.  What bounds it are two trips to memory and the
+// launch.  Layer 4 -> 16, three launches before and this: 300 rows 19.0 -> 11.4 us, 2 000 18.6 -> 11.5, 8 000 19.5 -> 12.2; 64 -> 64 with 8 000
+// rows 26.4 -> 20.8.  The line lies where the table still fits LDS: lists of 8 192 rows, 128 KB.
+constexpr int kSmallRows = 8192;
+constexpr int kSmallHeads = 16384;
+constexpr int kSmallBlock = 1024;
+constexpr int kSmallWaves = kSmallBlock / 64;
+constexpr int kSmallOwn = kSmallRows / kSmallBlock;                                 // rows that a thread enters
+constexpr int kSmallDepth = (kGemmMaxOffsets + kSmallWaves - 1) / kSmallWaves;  // offsets that it looks up
+static_assert(kSmallRows < 0xffff, "rows in 16 bits beside kNoRow");
+
+__global__ void __launch_bounds__(kSmallBlock)
+subm_small_rulebook(LookupPart P, int32_t* __restrict__ tiles) {
+    constexpr uint32_t kNoRow = 0xffffu;
+    __shared__ __align__(16) uint32_t s_head[kSmallHeads];  // first row of a list
+    __shared__ uint2 s_cell[kSmallRows];                    // a row's cell, the next row of its list
+    __shared__ int32_t s_pairs[64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int4* coors = reinterpret_cast<const int4*>(P.coors);  // (b,z,y,x)
+    const int heads_lg = P.max_voxels <= kSmallHeads / 8 ? 32 - __clz(P.max_voxels * 4) : 14;  // (four and more a row, up to the room there is)
+    const int shift = 32 - (heads_lg < 6 ? 6 : heads_lg);
+    // (all of it requested before the row count is known)
+    int4 c[kSmallOwn];
+#pragma unroll
+    for (int j = 0; j < kSmallOwn; ++j) {
+        const int v = j * kSmallBlock + tid;
+        c[j] = make_int4(0, 0, 0, 0);
+        if (v < P.max_voxels) c[j] = coors[v];
+    }
+    const int row = blockIdx.x * 64 + lane;  // whose neighbours this lane looks up, at offsets wave, wave + kSmallWaves, ...
+    const int4 own = coors[row < P.max_voxels ? row : 0];
+    for (int t = tid; t < (1 << (32 - shift)) / 4; t += kSmallBlock) reinterpret_cast<uint4*>(s_head)[t] = make_uint4(kNoRow, kNoRow, kNoRow, kNoRow);
+    if (tid < 64) s_pairs[tid] = 0;
+    const int n = clamp_rows(P.num, P.max_voxels);
+    if ((int)blockIdx.x * 64 >= n && blockIdx.x) return;
+    __syncthreads();
+    auto cell = [&](int z, int y, int x) { return ((uint32_t)z * (uint32_t)P.t.gy + (uint32_t)y) * (uint32_t)P.t.gx + (uint32_t)x; };
+    auto list = [&](uint32_t key) { return (key * 2654435769u) >> shift; };
+    bool bad = false;
+#pragma unroll
+    for (int j = 0; j < kSmallOwn; ++j) {
+        const int v = j * kSmallBlock + tid;
+        if (v < n) {
+            if (c[j].y < 0 || c[j].y >= P.t.gz || c[j].z < 0 || c[j].z >= P.t.gy || c[j].w < 0 || c[j].w >= P.t.gx) {
+                bad = true;  // the reference would write outside its grid
+            } else {
+                const uint32_t key = cell(c[j].y, c[j].z, c[j].w);
+                s_cell[v] = make_uint2(key, atomicExch(&s_head[list(key)], (uint32_t)v));
+            }
+        }
+    }
+    const bool any_bad = __syncthreads_or(bad);
+    if (blockIdx.x == 0 && tid < 4) {
+        P.meta[tid] = tid == 0 ? (any_bad ? SESSD_STATUS_BAD_COORD : 0) : (tid == 1 ? n : 0);
+        tiles[tid] = 0;
+    }
+    const bool in_layer = row < n && own.y >= 0 && own.y < P.t.gz && own.z >= 0 && own.z < P.t.gy && own.w >= 0 && own.w < P.t.gx;
+    uint32_t key[kSmallDepth], at[kSmallDepth], found[kSmallDepth];
+    int open = 0;
+#pragma unroll
+    for (int j = 0; j < kSmallDepth; ++j) {
+        const int k = wave + j * kSmallWaves;
+        const int z = own.y - P.p[0] + k / (P.k[1] * P.k[2]), y = own.z - P.p[1] + k / P.k[2] % P.k[1], x = own.w - P.p[2] + k % P.k[2];
+        const bool ok = in_layer && k < P.K && z >= 0 && z < P.t.gz && y >= 0 && y < P.t.gy && x >= 0 && x < P.t.gx;
+        key[j] = cell(z, y, x);
+        at[j] = ok ? s_head[list(key[j])] : kNoRow;
+        found[j] = kEmpty;
+    }
+    do {  // (lists end: a row is in one of them, in front of the rows that were in it before)
+        open = 0;
+#pragma unroll
+        for (int j = 0; j < kSmallDepth; ++j) {
+            if (at[j] == kNoRow) continue;
+            const uint2 e = s_cell[at[j]];
+            if (e.x == key[j]) found[j] = found[j] < at[j] ? found[j] : at[j];  // (a cell that two rows name belongs to the first)
+            at[j] = e.y;
+            open |= e.y != kNoRow ? 1 : 0;
+        }
+    } while (open);
+    int pairs = 0;
+#pragma unroll
+    for (int j = 0; j < kSmallDepth; ++j) {
+        const int k = wave + j * kSmallWaves;
+        pairs += found[j] != kEmpty ? 1 : 0;
+        if (k < P.K && row < n) P.nbr[(size_t)k * P.max_voxels + row] = (int32_t)found[j];
+    }
+    if (!P.w) return;  // (uniform)
+    atomicAdd(&s_pairs[lane], pairs);
+    __syncthreads();
+    if (wave == 0) {  // as lookup_pass() leaves them
+        int w = row < n ? s_pairs[lane] + P.row_weight : 0;
+        if (row < P.max_voxels) P.w[row] = w;
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) w += __shfl_xor(w, d, 64);
+        if (lane == 0 && (int)blockIdx.x * 64 < n) P.wsum[blockIdx.x] = w;
+    }
+}
+
 }  // namespace
 
 struct SubmConv3dLayerPlugin::Layout {
@@ -248,15 +349,20 @@ int SubmConv3dLayerPlugin::enqueueBuild(const int32_t* coors, const int32_t* vox
     const Layout L = carve(workspace);
     const Grid3 g{out_shape_x_, out_shape_y_, out_shape_z_};
     const CellTable t = ownTable(workspace);
-    FillArgs f;
-    f.add(L.cells, t.words(), kEmpty);
-    collectHeaderFill(workspace, f);
-    SESSD_TRY(launch_fill(f, stream));
-    hipLaunchKernelGGL(subm_insert, dim3(ceil_div(max_voxels_, kBlock)), dim3(kBlock), 0, stream, coors, voxel_num, max_voxels_, g, t,
-                       L.meta);
-    SESSD_HIP_TRY(hipGetLastError());
     const LookupPart look = lookupPart(workspace, coors, voxel_num, t, voxel_num, max_voxels_);
-    SESSD_TRY(launch_flags_lookups(nullptr, &look, 1, stream));
+    if (max_voxels_ <= kSmallRows) {
+        hipLaunchKernelGGL(subm_small_rulebook, dim3(ceil_div(max_voxels_, 64)), dim3(kSmallBlock), 0, stream, look, L.tiles);
+        SESSD_HIP_TRY(hipGetLastError());
+    } else {
+        FillArgs f;
+        f.add(L.cells, t.words(), kEmpty);
+        collectHeaderFill(workspace, f);
+        SESSD_TRY(launch_fill(f, stream));
+        hipLaunchKernelGGL(subm_insert, dim3(ceil_div(max_voxels_, kBlock)), dim3(kBlock), 0, stream, coors, voxel_num, max_voxels_, g, t,
+                           L.meta);
+        SESSD_HIP_TRY(hipGetLastError());
+        SESSD_TRY(launch_flags_lookups(nullptr, &look, 1, stream));
+    }
     if (!wantTileCuts()) return SESSD_OK;
     const CutPart cut = cutPart(workspace, voxel_num);
     return launch_number(nullptr, nullptr, &cut, 1, nullptr, nullptr, stream);

@@ -141,6 +141,34 @@ def test_subm_config1_rulebook_and_features():
     assert conv.status() == 0
 
 
+@pytest.mark.parametrize("n,mv,ksize,cin,cout", [(0, 1, 3, 4, 16), (1, 1, 3, 4, 16), (64, 64, 3, 4, 16), (65, 70, 3, 64, 64), (1024, 1025, 3, 4, 16),
+                                                 (2047, 2048, 3, 64, 64), (2049, 2049, 1, 5, 7), (5000, 8191, 3, 64, 64), (8192, 8192, 3, 4, 16)])
+def test_subm_rulebook_of_a_small_layer_equals_the_general_one(n, mv, ksize, cin, cout):
+    """A layer of at most 8 192 rows builds its rulebook in one launch; with one row more it takes the passes over a table in memory.
+    Same pairs, status and outputs, also where two rows name one cell and where rows lie outside the grid."""
+    rng = np.random.default_rng(n + mv)
+    grid, most = (41, 300, 200), 8193
+    coors = np.zeros((most, 4), np.int32)
+    coors[:n] = F.clustered_active_voxels(n, grid, 7, n_blobs=12)[:n] if n else 0
+    if n >= 64:
+        coors[n - 5:n] = coors[3:8]  # (the first row of a cell has it)
+        coors[10, 1], coors[20, 2], coors[30, 3] = -1, grid[1], grid[2] + 7
+    feat = np.zeros((most, cin), np.float32)
+    feat[:n] = rng.uniform(-1, 1, (n, cin))
+    w = rng.normal(0, 0.1, (ksize ** 3, cin, cout)).astype(np.float32)
+    got = []
+    for rows in (mv, most):
+        conv = api.SubmConv3d(cin, cout, grid[::-1], w, rows, ksize=ksize, padding=ksize // 2)
+        out = conv(dev(feat[:rows]), dev(coors[:rows]), dev(np.array([n], np.int32)))
+        pairs, num = conv.export_rulebook()
+        got.append((to_np(pairs)[:, :, :n], to_np(num), to_np(out)[:n], conv.status()))
+        conv.close()
+    assert got[0][3] == got[1][3] == (D.SESSD_STATUS_BAD_COORD if n >= 64 else 0)
+    assert np.array_equal(got[0][1], got[1][1]) and np.array_equal(got[0][0], got[1][0])
+    # (the general path's workgroups may hold other tiles: sums in another order, 2^-24 a term and fewer than 27 Cin terms of 0.5 |x w|)
+    assert np.allclose(got[0][2], got[1][2], rtol=0, atol=ksize ** 3 * cin * 2.0 ** -24)
+
+
 @pytest.mark.parametrize("cin,cout", [(4, 16), (16, 16), (16, 32), (32, 32), (32, 64), (64, 64), (64, 128), (128, 128),
                                       (5, 7), (8, 32)])
 def test_subm_clustered_with_epilogue_and_pad_rows(cin, cout):
