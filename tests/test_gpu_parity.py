@@ -661,6 +661,27 @@ def test_sparse2dense_long_lines_and_odd_shapes(size_xyz, channel, pad):
         assert s2d.status() == 0
 
 
+@pytest.mark.parametrize("size_xyz,channel,pad", [((178, 20, 2), 33, (0, 0, 0, 0)), ((176, 20, 1), 64, (1, 1, 1, 1)), ((450, 7, 2), 40, (0, 0, 0, 0)),
+                                                  ((2, 5, 1), 3, (0, 0, 0, 0)), ((5, 6, 1), 8, (0, 0, 1, 0))])
+@pytest.mark.parametrize("tin", [torch.float32, torch.float16])
+@pytest.mark.parametrize("tout", [torch.float32, torch.float16])
+def test_sparse2dense_lines_of_an_even_width(size_xyz, channel, pad, tin, tout):
+    """Lines that no 16-byte run divides but pairs of elements do, also in two segments and with two cells only: a copy, bit for bit."""
+    rng = np.random.default_rng(9)
+    W, H, Dz = size_xyz
+    n, mv = min(1500, W * H * Dz // 2), 1600
+    coors = F.random_active_voxels(n, (Dz, H, W), 8)
+    cbuf = np.zeros((mv, 4), np.int32)
+    cbuf[:n] = coors
+    f = dev(rng.uniform(0.1, 1, (mv, channel)).astype(np.float32)).to(tin)
+    s2d = api.Sparse2Dense(size_xyz, channel, padding=pad)
+    dense = s2d(f, dev(cbuf), dev(np.array([n], np.int32)), out_dtype=tout)
+    torch.cuda.synchronize()
+    want = O.zero_pad2d(O.sparse2dense(to_np(f[:n].to(tout).float()), coors, n, size_xyz), *pad)
+    assert dense.dtype == tout and np.array_equal(to_np(dense.float()), want)
+    assert s2d.status() == 0
+
+
 def test_sparse2dense():
     rng = np.random.default_rng(2)
     n, mv, c = 2739, 60000, 64
