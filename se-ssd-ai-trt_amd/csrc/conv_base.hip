@@ -106,7 +106,7 @@ int ConvPluginBase::tileRows() const { return gemm_wide_tile_rows(out_channel_, 
 int ConvPluginBase::tilesWide() const {
     return gemm_runs_wide(kernel_volume_, in_channel_, out_channel_, in_type_, out_type_) ? (out_channel_ > 64 ? out_channel_ / 64 : 1) : 0;
 }
-int ConvPluginBase::tileRowWeight() const { return tilesWide() ? 4 : 20; }
+int ConvPluginBase::tileRowWeight() const { return 4; }  // (only conv_wide.hip takes cuts)
 
 int ConvPluginBase::runGemm(const void* in_feat, void* out_feat, const int32_t* nbr, const int32_t* tiles,
                             const int32_t* num_out, hipStream_t stream, const DenseTarget* dense) {

@@ -7,8 +7,7 @@
 // busiest unit.  Here every row gets the weight  pairs(row) + row_weight  and the rows are cut where the
 // running sum crosses multiples of W = ceil(total / T), T = the tile count the equal-length rule would
 // use (tile_plan() with the target height the caller names).  The per-row constant is the caller's: what a row
-// costs its GEMM kernel beside its pairs (20 pairs' worth on the split-K kernel, 4 on the one-tile-per-unit kernel,
-// whose tile time measured 732 cycles per 16-pair block + 22 per row); it also keeps sparse runs from growing far
+// costs its GEMM kernel beside its pairs (4 pairs' worth on conv_wide.hip); it also keeps sparse runs from growing far
 // beyond the kernel's tile capacity.  Runs that still do are walked in capacity-sized pieces by the kernel, so any
 // cut is correct.
 //
