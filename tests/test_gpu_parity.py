@@ -976,9 +976,9 @@ def test_wide_fp32_kernel_tall_tiles_and_two_tiles_per_workgroup(n, clustered, c
 
 
 @pytest.mark.parametrize("cin", [64, 32])
-@pytest.mark.parametrize("n", [3071, 3072, 3073, 10239, 10240, 10241])
+@pytest.mark.parametrize("n", [3071, 3072, 3073, 7679, 7680, 7681, 10239, 10240, 10241])
 def test_wide_fp32_kernel_around_the_row_counts_of_its_column_splits(n, cin):
-    """On 256 compute units the columns of a tile are dealt to two workgroups up to 10 240 rows."""
+    """On 256 compute units the columns of a tile are dealt to two workgroups up to 7 680 rows."""
     _fp32_subm_wide_against_oracle(n, n + 7, (11, 200, 176), 900 + n, threads=8, cin=cin)
 
 
