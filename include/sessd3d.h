@@ -153,7 +153,9 @@ void sessd_voxelgen_destroy(sessd_voxelgen* h);
 /* inputs : 0 feat [1,max_voxels,Cin] f32|f16   1 coors i32[1,max_voxels,4]   2 voxel_num i32[1]
  * outputs: 0 feat [1,max_voxels,Cout] f32|f16
  * out[o] = sum_k W[k]^T in[nbr(o,k)], weights FP32 [K][Cin][Cout] (K = ksize^3, offset index
- * kz*9+ky*3+kx), no bias; optional fused y = max(0, x*scale[c]+shift[c]) epilogue. */
+ * kz*9+ky*3+kx), no bias; optional fused y = max(0, x*scale[c]+shift[c]) epilogue.
+ * FP32 features: both operands count with all of their bits whatever their magnitude and that of their neighbours, a product
+ * is within 2^-23 of itself, sums are FP32 (here and in the strided layers). */
 
 typedef struct sessd_submconv3d sessd_submconv3d;
 

@@ -9,28 +9,25 @@
 // tile of its own in LDS (so the order of every sum is fixed); the partial tiles are summed in a fixed order, scale/shift/ReLU
 // follow, each row is stored once.  Results are bit-identical run to run.
 //
-// Products.  The FP32 matrix instruction does 32 multiply-adds a cycle and SIMD, the 16-bit ones 512, so operands are
-// split into 16-bit parts whose products are exact in FP32 and are accumulated in FP32:
-//   * Cin 64 and 128, halves: a row is scaled by a power of two that brings its largest element to [2^14, 2^15) (a column of W
-//     likewise, on the host) and x = hi + lo with 11 bits each; lo * hi, hi * lo and hi * hi on v_mfma_f32_16x16x32_f16.  What is
-//     left out is below 2^-23 of an operand and 2^-24 of a product; 3/16 of the FP32 instruction's time.
-//   * Cin 32, thirds: x = x0 + x1 + x2 with 8 bits each is exact, BF16 has FP32's range, and the six products down to 2^-24 of
-//     the largest are kept (v_mfma_f32_16x16x32_bf16; 6/16 of the time).  With halves these layers, whose sums are shorter, came
-//     out 11 % further from the sums in 64 bits than with the FP32 instruction; with thirds 30 % nearer.
-//   * Cin 4 and 16: the FP32 instruction (4 or 16 of them a block: it is not what they wait for).
-// Distance from the sums in 64 bits, 2-norm, FP32 instruction -> now: 64 -> 64 1.27e-7 -> 1.13e-7, 128 -> 128 1.31e-7 -> 1.20e-7,
-// 3x1x1 64 -> 64 1.13e-7 -> 1.00e-7, 32 -> 64 1.00e-7 -> 0.70e-7, 32 -> 32 0.93e-7 -> 0.66e-7, 16 -> 16 0.78e-7 -> 0.76e-7.  Infinities, NaN and
-// sums beyond the range come out of the parts as something that is not finite: such elements are summed again, plainly
-// (direct_sum()).
+// Products.  The FP32 matrix instruction does 32 multiply-adds a cycle and SIMD, the 16-bit ones 512.  From 32 channels up both
+// operands are split into three BF16 parts of eight bits, x = x0 + x1 + x2 exactly, and the six largest products of
+// parts are added in FP32, smallest first (v_mfma_f32_16x16x32_bf16; 6/16 of the FP32 instruction's time).  What is left out is
+// below 2^-23 of a product, and BF16 has FP32's range, so that this holds for every element by itself, whatever the others of its row or column are.  What does not fit --
+// numbers below 2^-110 whose last bits lie under BF16's smallest number, infinities and NaN, sums that overflow on the
+// way -- comes out as something that is not finite, and such elements are summed again, plainly (direct_sum()).  Two FP16
+// parts of operands scaled by row and column are three products instead of six (64 -> 64 at 17 262 rows 19.1 us, 24.9 so) but
+// hold an element to 2^-24 of its row's largest and not of itself: a channel at 1e8 beside others at 1 cost these 5e-5 of
+// their sums.  Cin 4 and 16: the FP32 instruction (4 or 16 of them a block: it is not what they wait for).
+// Distance from the sums in 64 bits, 2-norm, FP32 instruction and parts: 64 -> 64 1.27e-7, 0.72e-7; 128 -> 128 1.31e-7, 0.81e-7; 64 -> 128
+// 1.24e-7, 0.72e-7; 32 -> 64 1.00e-7, 0.70e-7; 32 -> 32 0.93e-7, 0.67e-7.
 //
-// What bounds it is instructions per wave and LDS, not the matrix cores: a block of 64 -> 64 takes a wave 1 650 cycles of
-// which 384 are MFMA; of the LDS's time a third is the lane permutation, half the partial tile.  Hence
-//   * a wave takes all 64 columns: rows are requested, split and permuted once (with 32 columns a wave 25 us at 17 262 rows,
-//     with 64 19 us);
-//   * six waves: as many partial tiles of 96 rows as LDS holds.  Eight with 72 rows are faster (17.7 against 18.5 us at 11 343
-//     rows) until a tile does not fit (25.9 against 21 us at 17 262 rows, whose cuts vary by a third);
+// What bounds it: a block of 64 -> 64 is 768 cycles of MFMA (with half of them left out the launch above takes 20.0 us), the rest a wave's
+// instructions and LDS.  Hence
+//   * a wave takes all 64 columns: rows are requested, permuted and split once;
+//   * six waves: as many partial tiles of 96 rows as LDS holds.  Eight with 72 rows are faster until a tile does not fit;
 //   * the rows of the block after next are requested, and the next block's split, under a block's MFMAs; the next offset's
-//     weights are requested with the first block of an offset into a second set of registers;
+//     weights are requested with the first block of an offset into a second set of registers, or, where these do not hold two
+//     sets (64 x 64), behind the MFMAs of its last into the only one;
 //   * a wave's blocks and offsets are listed once, a lane each, and read with readlane: the loop has no other bookkeeping.
 // Up to 16 (32) columns a tile is at most 112 (64) rows and a unit holds two workgroups, both used only where one tile for each
 // unit would be higher than that (32 -> 32, eight waves, 4 208 rows: one workgroup a unit 7.9 us, two 10.7).  What LDS they leave is what the
@@ -39,12 +36,11 @@
 // FP16 features (Cin 16) have so little in each block that four waves and 64 rows do: four workgroups share a unit, with 40 KB of LDS
 // each.  From 32 channels up FP16 is faster without pair lists (32 -> 32 at 45 874 rows 10.6 us on conv_tall.hip, 18 here).
 //
-// Launches of SubM layers at the sites of scans, us, before (split-K on four waves, or sixteen waves of 16 columns, both with
-// the FP32 instruction) -> now: 64 -> 64 at 2 448 rows 10.4 -> 9.4, 8 662 20.7 -> 14.7, 17 262 31.7 -> 19.2 (99 TFLOP/s), 23 959 48.4
-// -> 30.7; 128 -> 128 at 3 594 rows 31.2 -> 19.3, 17 262 120 -> 57 (134 TFLOP/s); 64 -> 128 at 17 262 57 -> 35; 32 -> 64 at 28 043 32
-// -> 26; 32 -> 32 at 4 208 9.4 -> 8.9, 28 043 19.1 -> 16.9, 45 874 35.9 -> 27.9; 16 -> 16 at 17 132 8.3 -> 7.3; 4 -> 16 7.4 -> 6.5.  16 -> 32
-// 10.2 -> 9.0, but 14.9 -> 16.8 at 36 871 rows (a second round of tiles begins at 32 768).  FP16 16 -> 16 at 1 901 rows 6.3 -> 5.9, 60 000
-// 14.2 -> 10.8; 16 -> 32 6.7 -> 6.2, 16.6 -> 12.9.
+// Launches of SubM layers at the sites of scans, us, with the FP32 instruction (sixteen waves, or split-K) and now: 64 -> 64 at 3 051 rows
+// 10.7, 11.9; 7 120 18.3, 16.3; 17 262 32.2, 24.9; 23 959 48.7, 39.4; 128 -> 128 at 3 815 rows 33.9, 24.8; 17 262 121, 76; 64 -> 128 at 17 262 58, 46;
+// 32 -> 64 at 28 043 32, 26; 32 -> 32 at 28 043 19.3, 16.7; 45 874 36.1, 27.8; 16 -> 16 at 17 132 8.3, 7.3; 4 -> 16 7.4, 6.5; 16 -> 32 10.2, 9.0, but
+// 14.9, 16.8 at 36 871 rows (a second round of tiles begins at 32 768).  FP16 16 -> 16 at 60 000 rows 14.2, 10.8; 16 -> 32 16.6, 12.9.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -57,7 +53,6 @@ namespace sessd {
 namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef __bf16 v2b __attribute__((ext_vector_type(2)));
 typedef __bf16 v8b __attribute__((ext_vector_type(8)));
@@ -71,8 +66,8 @@ constexpr unsigned kOutOfRange = 0x80000000u;  // beyond any buffer the kernel i
 constexpr int kRawBuffer = 0x00020000;         // descriptor word 3: raw 32-bit data format, no swizzle
 
 // how a layer's products are made: FP32 MFMA, or 16-bit MFMA on operands split into parts
-enum Arith { kPlain, kThirds, kHalves, kFp16 };
-constexpr Arith arith(int cin) { return cin >= 64 ? kHalves : (cin >= 32 ? kThirds : kPlain); }  // (of FP32 features)
+enum Arith { kPlain, kThirds, kFp16 };
+constexpr Arith arith(int cin) { return cin >= 32 ? kThirds : kPlain; }  // (of FP32 features)
 
 template <typename T, int CIN, int COUT>  // T: the input features' type
 struct Shape {
@@ -123,24 +118,7 @@ __device__ __forceinline__ void store4(__half* dst, const float (&o)[4]) {
     *reinterpret_cast<uint2*>(dst) = p.u;
 }
 
-template <int CTRL>
-__device__ __forceinline__ uint32_t quad_max(uint32_t v) {  // of this lane and the one of its quad that CTRL names
-    const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
-    return v > o ? v : o;
-}
-
-// halves hi + lo = x * up, two of each in a word
-__device__ __forceinline__ void split_pair(float x0, float x1, float up, int& hi, int& lo) {
-    v2h h, l;
-    h.x = (_Float16)(x0 * up);
-    h.y = (_Float16)(x1 * up);
-    hi = __builtin_bit_cast(int, h);
-    asm("" : "+v"(hi));  // (or the compiler rounds each half a second time)
-    h = __builtin_bit_cast(v2h, hi);
-    l.x = (_Float16)fmaf(x0, up, -(float)h.x);
-    l.y = (_Float16)fmaf(x1, up, -(float)h.y);
-    lo = __builtin_bit_cast(int, l);
-}
+constexpr unsigned kUpperHalves = 0x07060302u;  // v_perm_b32: the upper half of the second word, then that of the first
 
 template <typename V>
 __device__ __forceinline__ V operand8(const int* w) {
@@ -148,8 +126,7 @@ __device__ __forceinline__ V operand8(const int* w) {
     return __builtin_bit_cast(V, v);
 }
 
-// What a lane holds of a 16-pair block's rows (Rows, in the order of the request; words that a lane permutation brings to
-// the operands) and of an offset's weights, and the products of the two.
+// What a lane holds of a 16-pair block's rows (take(): in operand order) and of an offset's weights, and the products of the two.
 template <typename S, int NB, Arith>
 struct Products;
 
@@ -176,7 +153,6 @@ struct Products<S, NB, kFp16> {
                 }
             }
     }
-    static __device__ __forceinline__ float add(float p, const int (&)[kWords], float sum) { return sum + p; }
 };
 
 // FP32 MFMA
@@ -198,28 +174,32 @@ struct Products<S, NB, kPlain> {
                 for (int nb = 0; nb < NB; ++nb)
                     acc[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(__int_as_float(w[g][nb][e]), __int_as_float(x[g * E + e]), acc[nb], 0, 0, 0);
     }
-    static __device__ __forceinline__ float add(float p, const int (&)[kWords], float sum) { return sum + p; }
 };
 
-// BF16 MFMA on three parts of eight bits each: x = x0 + x1 + x2 exactly; the products down to 2^-24 of the largest, smallest first
+// BF16 MFMA on three parts of eight bits each, x = x0 + x1 + x2: x0 cut off (rounded, the largest numbers would become
+// infinite), x1 rounded, x2 what is left, which eight bits hold unless it reaches below BF16's smallest number; such a row becomes
+// NaN.  The six largest products of parts, smallest first.
 template <typename S, int NB>
 struct Products<S, NB, kThirds> {
     static constexpr int G = S::G, E = 4, C = S::CP / 32, kWords = G * 6, kPieces = 3 * C;  // (words: x0, x1, x2)
     static __device__ __forceinline__ void take(const int (&a)[G][E], int (&p)[kWords]) {
+        uint32_t left = 0;  // (of any element beyond the three parts: the low half of a word)
 #pragma unroll
         for (int g = 0; g < G; ++g)
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-                v2f r = {__int_as_float(a[g][2 * e]), __int_as_float(a[g][2 * e + 1])};
-#pragma unroll
-                for (int t = 0; t < 3; ++t) {
-                    int w = __builtin_bit_cast(int, __builtin_convertvector(r, v2b));
-                    asm("" : "+v"(w));
-                    p[2 * G * t + 2 * g + e] = w;
-                    r.x -= __int_as_float(w << 16);
-                    r.y -= __int_as_float(w & (int)0xffff0000);
-                }
+                const uint32_t u0 = (uint32_t)a[g][2 * e], u1 = (uint32_t)a[g][2 * e + 1];
+                const int at = 2 * g + e;
+                p[at] = (int)__builtin_amdgcn_perm(u1, u0, kUpperHalves);
+                v2f r = {__uint_as_float(u0) - __uint_as_float(u0 & 0xffff0000u), __uint_as_float(u1) - __uint_as_float(u1 & 0xffff0000u)};
+                int w = __builtin_bit_cast(int, __builtin_convertvector(r, v2b));
+                asm("" : "+v"(w));
+                p[2 * G + at] = w;
+                const uint32_t r0 = __float_as_uint(r.x - __int_as_float(w << 16)), r1 = __float_as_uint(r.y - __int_as_float(w & (int)0xffff0000));
+                p[4 * G + at] = (int)__builtin_amdgcn_perm(r1, r0, kUpperHalves);
+                left |= r0 | r1;
             }
+        p[kWords - 1] |= left & 0xffffu ? 0x7fff : 0;  // (the last word: what waits for all of them is last)
     }
     static __device__ __forceinline__ void multiply(const int (&w)[3 * C][NB][E], const int (&x)[kWords], v4f (&acc)[NB]) {
         constexpr int kPart[6][2] = {{0, 2}, {1, 1}, {2, 0}, {0, 1}, {1, 0}, {0, 0}};  // of w, of x
@@ -232,47 +212,6 @@ struct Products<S, NB, kThirds> {
                     acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(operand8<v8b>(w[kPart[t][0] * C + c][nb]),
                                                                       operand8<v8b>(x + 2 * G * kPart[t][1] + 4 * c), acc[nb], 0, 0, 0);
     }
-    static __device__ __forceinline__ float add(float p, const int (&)[kWords], float sum) { return sum + p; }
-};
-
-// FP16 MFMA on the halves of both sides: low * high and high * low, then high * high, one accumulator
-template <typename S, int NB>
-struct Products<S, NB, kHalves> {
-    static constexpr int G = S::G, E = 4, C = S::CP / 32, kWords = G * 4 + 1, kPieces = 2 * C;  // (words: high, low, power of two)
-    static __device__ __forceinline__ void take(const int (&a)[G][E], int (&p)[kWords]) {
-        // the row's largest magnitude -> power of two that brings it to [2^14, 2^15)
-        float big = 0.f;
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            big = fmaxf(fmaxf(big, fabsf(__int_as_float(a[g][0]))), fabsf(__int_as_float(a[g][1])));
-            big = fmaxf(fmaxf(big, fabsf(__int_as_float(a[g][2]))), fabsf(__int_as_float(a[g][3])));
-        }
-        uint32_t expo = quad_max<0xB1>(__float_as_uint(big));  // (lanes 1 0 3 2; magnitudes order like their bits)
-        expo = quad_max<0x4E>(expo) & 0x7f800000u;             // (lanes 2 3 0 1)
-        expo = expo < (15u << 23) ? 15u << 23 : expo;
-        const float up = __uint_as_float((268u << 23) - expo);
-#pragma unroll
-        for (int g = 0; g < G; ++g)
-#pragma unroll
-            for (int e = 0; e < 2; ++e)
-                split_pair(__int_as_float(a[g][2 * e]), __int_as_float(a[g][2 * e + 1]), up, p[2 * g + e], p[2 * G + 2 * g + e]);
-        p[4 * G] = (int)(expo - (14u << 23));
-    }
-    static __device__ __forceinline__ void multiply(const int (&w)[2 * C][NB][E], const int (&x)[kWords], v4f (&acc)[NB]) {
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(operand8<v8h>(w[C + c][nb]), operand8<v8h>(x + 4 * c), acc[nb], 0, 0, 0);
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(operand8<v8h>(w[c][nb]), operand8<v8h>(x + 2 * G + 4 * c), acc[nb], 0, 0, 0);
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(operand8<v8h>(w[c][nb]), operand8<v8h>(x + 4 * c), acc[nb], 0, 0, 0);
-    }
-    static __device__ __forceinline__ float add(float p, const int (&x)[kWords], float sum) { return fmaf(p, __int_as_float(x[4 * G]), sum); }
 };
 
 // One wave's share of a tile: the pairs of the offsets dealt to it, times its columns -- 16-column blocks nb0 .. nb0 + NB - 1
@@ -282,6 +221,7 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
                                          const int32_t* s_blk, int K, int wave, int lane, int nb0, float* part) {
     using P = Products<S, NB, S::kArith>;
     constexpr int kParts = S::kParts, G = S::G, E = S::kLaneBytes / 4, kWaves = S::kWaves, kTileRows = S::kTileRows;
+    constexpr int kSets = P::kPieces * NB * E > 64 ? 1 : 2;  // of weights: the registers do not hold two of the largest
     constexpr int NBT = COUT / 16;                   // 16-column blocks of the layer
     constexpr int kSlots = NB * 4;                   // 16-byte slots of a row of the partial tile
     const int i = lane & 15;  // pair inside a 16-pair block
@@ -328,7 +268,7 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
     // the block, bytes 16 * (l % 4) ..): the cache looks up one line per group of four lanes.  In the MFMA's
     // operand order -- lane l: pair l % 16, bytes 16 * (l / 16) .. -- the four lanes of a group name four
     // different rows and the same request takes four lookups: 18 instead of 48 bytes per cycle and compute unit,
-    // measured.  The operand order is restored by a lane permutation before the MFMAs.
+    // measured.  The operand order is restored by a lane permutation when the rows have arrived.
     // Filling pairs ask out of range (such a request returns zeros and touches no memory).
     const char* pairs = reinterpret_cast<const char*>(s_pair);
     auto entry_at = [&](int it, int j4) -> uint32_t { return *reinterpret_cast<const uint32_t*>(pairs + (kParts > 1 ? it & ~3 : it) + j4); };
@@ -348,9 +288,14 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
     const int from_lane4 = (4 * i + q) * 4;  // ds_bpermute address: this lane's operand sits in lane 4 * i + q
     const int request4 = lane & ~3, operand4 = i * 4;  // this lane's pair of a block in the request's and in the operands' order, times 4
     int d0 = __builtin_amdgcn_readlane(item_at, 0), d1 = __builtin_amdgcn_readlane(item_at, 1), d2;
-    int a[G][E], p[P::kWords], b0[P::kPieces][NB][E], b1[P::kPieces][NB][E];
-    auto take = [&]() {
-        P::take(a, p);
+    int a[G][E], p[P::kWords], b0[P::kPieces][NB][E], b1[kSets == 2 ? P::kPieces : 1][NB][E];
+    auto take = [&]() {  // (permuted before they are split: two words instead of three)
+        int row[G][E];
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int e = 0; e < E; ++e) row[g][e] = __builtin_amdgcn_ds_bpermute(from_lane4, a[g][e]);
+        P::take(row, p);
 #pragma unroll
         for (int w = 0; w < P::kWords; ++w) asm volatile("" : "+v"(p[w]));  // (here, not where they are used: `a` is free for the next request)
     };
@@ -363,15 +308,13 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
     load_a(d1, next_entry, a);
     int t = 0, stage = 0;
 
-    // `use`: the weights of the item's stage; `fill`: those of the next one, requested behind its first block
-    auto item = [&](const int (&use)[P::kPieces][NB][E], int (&fill)[P::kPieces][NB][E], bool first) {
+    // `use`: the weights of the item's stage; `fill`: those of the next one, requested behind its first block, or, where there is one
+    // set, behind its last
+    auto item = [&](const int (&use)[P::kPieces][NB][E], int (&fill)[P::kPieces][NB][E], bool request) {
         d2 = __builtin_amdgcn_readlane(item_at, t + 2);
         ++t;
         next_entry = entry_at(d2, request4);
         const uint32_t mine = entry_at(d0, operand4);
-        int x[P::kWords];
-#pragma unroll
-        for (int w = 0; w < P::kWords; ++w) x[w] = __builtin_amdgcn_ds_bpermute(from_lane4, p[w]);
         const int r = (int)(mine & 255u);
         float4* const dst = reinterpret_cast<float4*>(part) + r * kSlots;
         float4 sum[NB];
@@ -380,20 +323,20 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
         v4f acc[NB];
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) acc[nb] = (v4f){0.f, 0.f, 0.f, 0.f};
-        P::multiply(use, x, acc);
+        P::multiply(use, p, acc);
         take();  // (of d1's rows)
         __builtin_amdgcn_sched_barrier(0);  // (or the requests below take other registers, which then have to arrive to be copied)
-        if (first) load_b(__builtin_amdgcn_readlane(stage_at, stage + 1), fill);
+        if (request) load_b(__builtin_amdgcn_readlane(stage_at, stage + 1), fill);
         // (behind the weights in either case: what the waits count is then the same for every item)
         load_a(d2, next_entry, a);
         if (mine < kNoPair) {
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
                 float4 v = sum[nb];
-                v.x = P::add(acc[nb][0], x, v.x);
-                v.y = P::add(acc[nb][1], x, v.y);
-                v.z = P::add(acc[nb][2], x, v.z);
-                v.w = P::add(acc[nb][3], x, v.w);
+                v.x += acc[nb][0];
+                v.y += acc[nb][1];
+                v.z += acc[nb][2];
+                v.w += acc[nb][3];
                 dst[(nb * 4 + q) ^ (r & (kSlots - 1))] = v;
             }
         }
@@ -402,10 +345,13 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
     };
     auto run_stage = [&](const int (&use)[P::kPieces][NB][E], int (&fill)[P::kPieces][NB][E]) -> bool {
         const int n = __builtin_amdgcn_readlane(stage_items, stage);
-        for (int j = 0; j < n; ++j) item(use, fill, j == 0);
+        for (int j = 0; j < n; ++j) item(use, fill, j == (kSets == 2 ? 0 : n - 1));
         return ++stage < stages;
     };
-    while (run_stage(b0, b1) && run_stage(b1, b0)) {}
+    if constexpr (kSets == 2)
+        while (run_stage(b0, b1) && run_stage(b1, b0)) {}
+    else
+        while (run_stage(b0, b0)) {}
 }
 
 // four output elements of a row as plain FP32 sums (nbr: the row's neighbour at offset 0; the others follow max_voxels apart)
@@ -466,6 +412,7 @@ conv_wide(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
     const int lsplit = kMaxSplit ? wide_log2_split(n, K, units) : 0;
     const int row_groups = units >> lsplit;  // workgroups of one column part
     const int first_tile = tile_of[kMaxSplit ? lsplit : 0];
+    const int first_begin = cut_begin[kMaxSplit ? lsplit : 0], first_end = cut_end[kMaxSplit ? lsplit : 0];
     const int part_id = lsplit && block >= row_groups ? 1 : 0;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -475,7 +422,7 @@ conv_wide(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
     if (tid < COUT) {
         if (scale) epi_scale = scale[tid];
         if (shift) epi_shift = shift[tid];
-        if (S::kArith == kHalves) epi_col = reinterpret_cast<const float*>(static_cast<const char*>(Wp) + (size_t)K * S::kWeightBytes)[tid];
+        if (S::kArith == kThirds) epi_col = reinterpret_cast<const float*>(static_cast<const char*>(Wp) + (size_t)K * S::kWeightBytes)[tid];
     }
     // this thread's epilogue columns (the same for every row it stores): within the part, and of the layer
     const int lvec = (kWgCols == 64 ? 4 : (kWgCols == 32 ? 3 : 2)) - lsplit;  // log2 of the part's 4-column vectors
@@ -493,7 +440,6 @@ conv_wide(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
     TilePlan plan = {0, 0};
     if (cut_count == 0) plan = tile_plan(n, walkers, kTileRows);
     const int tile_count = cut_count > 0 ? cut_count : (n > 0 ? plan.count : 0);
-    const int first_begin = cut_begin[kMaxSplit ? lsplit : 0], first_end = cut_end[kMaxSplit ? lsplit : 0];
     const __amdgpu_buffer_rsrc_t rs_in = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<T*>(in), 0, (int)((size_t)max_voxels * S::kRowBytes), kRawBuffer);
     const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
@@ -597,16 +543,15 @@ conv_wide(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
         if (r >= rows) break;
         float o[4] = {sums[u].x, sums[u].y, sums[u].z, sums[u].w};
         bool finite = true;
-        constexpr bool kParted = S::kArith == kThirds || S::kArith == kHalves;
-        if constexpr (kParted) {
+        if constexpr (S::kArith == kThirds) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                if (S::kArith == kHalves) o[e] *= e_col[e];
+                o[e] *= e_col[e];
                 finite = finite && (__float_as_uint(o[e]) & 0x7f800000u) != 0x7f800000u;
             }
         }
-        // the parts of an infinity, or a sum beyond their range, say nothing: the products themselves
-        if constexpr (kParted)
+        // (parts of an infinity, of a row that is not all in its parts, or a sum beyond the range on the way: the products themselves)
+        if constexpr (S::kArith == kThirds)
             if (!finite) direct_sum<CIN, COUT>(in, w_f32, nbr + row0 + r, max_voxels, K, ec4, o);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -684,15 +629,14 @@ int gemm_wide_tile_rows(int cout, int type) {
 }
 
 bool wide_splits(int cin) { return arith(cin) != kPlain; }
-size_t wide_weight_bytes(int K, int cin, int cout) {
-    return arith(cin) == kThirds ? (size_t)K * cin * cout * 6 : ((size_t)K * cin + 1) * cout * sizeof(float);
-}
+size_t wide_weight_bytes(int K, int cin, int cout) { return (size_t)K * cin * cout * 6 + cout * sizeof(float); }
 
-// the nearest BF16, as nearest_half()
-static uint16_t nearest_bf16(float v, float* value) {
+// the nearest BF16, as nearest_half(); cut: the next one towards zero
+static uint16_t nearest_bf16(float v, float* value, bool cut) {
     uint32_t u;
     std::memcpy(&u, &v, 4);
-    u = (u & 0x7fffffffu) > 0x7f800000u ? u | 0x400000u : u + 0x7fffu + ((u >> 16) & 1u);
+    if ((u & 0x7fffffffu) > 0x7f800000u) u |= 0x400000u;  // (NaN)
+    else if (!cut) u += 0x7fffu + ((u >> 16) & 1u);
     u &= 0xffff0000u;
     std::memcpy(value, &u, 4);
     return (uint16_t)(u >> 16);
@@ -700,37 +644,38 @@ static uint16_t nearest_bf16(float v, float* value) {
 
 // W in parts and in operand order: Wp[k][64 channels][part][step][16-column block][lane][8], element j of lane l being channel
 // 32 step + 16 (j / 4) + 4 (l / 16) + j % 4 (the channels that the lane permutation of the rows brings there), column
-// 16 block + l % 16.  Halves: of W * 2^e[column], and behind them 2^-e[column].
+// 16 block + l % 16; behind them a factor for each column.  Three parts hold a number from 2^-110 up.  A column with smaller
+// ones is multiplied by a power of two (its largest to 2^30), and divided by it where the sums are; what is too small even then
+// becomes NaN, and the column's sums are made plainly.
 void pack_wide_weights(const float* w, int K, int cin, int cout, void* dst) {
-    const bool halves = arith(cin) == kHalves;
-    std::vector<float> up(cout, 1.f);
-    if (halves) {
-        std::vector<float> big(cout, 0.f);
-        for (size_t t = 0; t < (size_t)K * cin; ++t)
-            for (int col = 0; col < cout; ++col) {
-                const float v = std::fabs(w[t * cout + col]);
-                if (v > big[col] && v <= 3.402823466e38f) big[col] = v;  // (finite)
-            }
-        float* down = reinterpret_cast<float*>(static_cast<char*>(dst) + (size_t)K * cin * cout * sizeof(float));
+    std::vector<float> up(cout, 1.f), big(cout, 0.f), small(cout, 1.f);
+    for (size_t t = 0; t < (size_t)K * cin; ++t)
         for (int col = 0; col < cout; ++col) {
-            int e = big[col] > 0.f ? 14 - std::ilogb(big[col]) : 0;
-            e = e > 126 ? 126 : e;
-            up[col] = std::ldexp(1.f, e);
-            down[col] = std::ldexp(1.f, -e);
+            const float v = std::fabs(w[t * cout + col]);
+            if (v > big[col] && v <= 3.402823466e38f) big[col] = v;  // (finite)
+            if (v < small[col] && v > 0.f) small[col] = v;
         }
+    float* down = reinterpret_cast<float*>(static_cast<char*>(dst) + (size_t)K * cin * cout * 6);
+    for (int col = 0; col < cout; ++col) {
+        int e = 0;
+        if (small[col] < std::ldexp(1.f, -110)) e = std::min(std::max(30 - std::ilogb(big[col]), 0), 126);
+        up[col] = std::ldexp(1.f, e);
+        down[col] = std::ldexp(1.f, -e);
     }
-    const int cp = cin > 64 ? 64 : cin, steps = cp / 32, blocks = cout / 16, parts = halves ? 2 : 3;
+    const int cp = cin > 64 ? 64 : cin, steps = cp / 32, blocks = cout / 16;
     uint16_t* o = static_cast<uint16_t*>(dst);
     const size_t part_size = (size_t)steps * blocks * 512;
     for (int k = 0; k < K; ++k)
         for (int ch = 0; ch < cin; ++ch, w += cout) {
             const int in_part = ch % cp, in_step = in_part % 32;
             const int first_lane = in_step % 16 / 4 * 16, j = in_step / 16 * 4 + in_step % 4;
-            uint16_t* at = o + (size_t)(k * (cin / cp) + ch / cp) * parts * part_size + (size_t)(in_part / 32) * blocks * 512 + first_lane * 8 + j;
+            uint16_t* at = o + (size_t)(k * (cin / cp) + ch / cp) * 3 * part_size + (size_t)(in_part / 32) * blocks * 512 + first_lane * 8 + j;
             for (int col = 0; col < cout; ++col) {
                 uint16_t* to = at + (size_t)(col / 16) * 512 + col % 16 * 8;
                 float v = w[col] * up[col], near = 0.f;
-                for (int part = 0; part < parts; ++part, v -= near) to[part * part_size] = halves ? nearest_half(v, &near) : nearest_bf16(v, &near);
+                const bool cut = std::fabs(v) > 3.38953139e38f;  // (beyond the largest BF16: infinite, if rounded)
+                for (int part = 0; part < 3; ++part, v -= near) to[part * part_size] = nearest_bf16(v, &near, cut && part == 0);
+                if (v != 0.f) to[0] = 0x7fc0;
             }
         }
 }

@@ -1087,8 +1087,8 @@ def _sums_in_64_bits(feat, w, pairs, num, n):
 @pytest.mark.parametrize("cin,cout", [(16, 32), (32, 32), (32, 64), (64, 64), (128, 128)])
 @pytest.mark.parametrize("lo,hi", [(-60, 60), (-110, -90), (60, 90)])
 def test_wide_fp32_kernel_keeps_32_bits_whatever_the_magnitude(cin, cout, lo, hi):
-    """Rows and columns of W of very different magnitude: the kernel multiplies 16-bit parts of the operands, whose range is
-    smaller than FP32's.  Bound: 27 * Cin terms of which each side is off by at most one unit in the last place of its
+    """Whole rows and whole columns of W of very different magnitude (channels: the test below): the kernel multiplies 16-bit
+    parts of the operands.  Bound: 27 * Cin terms of which each side is off by at most one unit in the last place of its
     operands (2^-23 each) and of its sum: SUM_TOL times the sum of the terms' magnitudes, as everywhere in these tests."""
     rng = np.random.default_rng([cin, lo + 200])
     n, grid = 300, (5, 20, 20)
@@ -1100,6 +1100,48 @@ def test_wide_fp32_kernel_keeps_32_bits_whatever_the_magnitude(cin, cout, lo, hi
     want = _sums_in_64_bits(feat, w, o_pairs, o_num, n)
     A = _sums_in_64_bits(np.abs(feat), np.abs(w), o_pairs, o_num, n)
     assert np.all(np.abs(out[:n] - want) <= 2e-6 * A + 2.0 ** -126)
+    conv.close()
+
+
+def _magnitudes_along_channels(kind, n, cin, cout, rng):
+    feat = rng.uniform(0.5, 1, (n, cin)) * rng.choice([-1, 1], (n, cin))
+    w = rng.uniform(0.5, 1, (27, cin, cout)) * rng.choice([-1, 1], (27, cin, cout))
+    if kind[0] == "opposed":  # products all alike
+        s = rng.integers(-kind[1], kind[1] + 1, cin)
+        s[:2] = kind[1], -kind[1]
+        feat *= 2.0 ** s
+        w *= 2.0 ** -s[:, None]
+    elif kind[0] == "unused":  # a channel without weights
+        feat[:, cin // 2], w[:, cin // 2] = kind[1], 0.0
+        feat[::2, 1], w[:, 1] = kind[1], 0.0
+    elif kind[0] == "small rows":  # features of 2^-100 down to the smallest subnormal numbers
+        feat *= 2.0 ** rng.integers(-148, -100, (n, cin))
+        feat[:, 0] *= 2.0 ** 30
+        w *= 2.0 ** 60
+    else:  # small weights, in columns with larger ones beside them and without
+        feat *= 2.0 ** 70
+        w *= 2.0 ** rng.integers(-148, -100, (27, cin, cout))
+        w[:, 0, ::2] *= 2.0 ** 90
+        feat[::3, 0] = 0.0
+    return feat.astype(np.float32), w.astype(np.float32)
+
+
+@pytest.mark.parametrize("cin,cout", [(32, 32), (32, 64), (64, 64), (64, 128), (128, 128)])
+@pytest.mark.parametrize("kind", [("opposed", 12), ("opposed", 20), ("opposed", 40), ("unused", 1e8), ("unused", 1e12),
+                                  ("unused", float(np.finfo(np.float32).min)), ("small rows", 0), ("small weights", 0)], ids=str)
+def test_wide_fp32_kernel_keeps_every_channel_whatever_the_magnitude_of_others(cin, cout, kind):
+    """Channels of a row, and elements of a column of W, of very different magnitude: an element keeps its bits beside larger
+    ones.  The bound is that of the rows and columns of different magnitude above."""
+    rng = np.random.default_rng([cin, cout, len(kind[0])])
+    n, grid = 300, (5, 20, 20)
+    coors = F.clustered_active_voxels(n, grid, 3, n_blobs=4)
+    feat, w = _magnitudes_along_channels(kind, n, cin, cout, rng)
+    conv, out, pairs, num, cbuf = run_subm(coors, n, feat, w, grid, n, None, None, False)
+    o_pairs, o_num, _ = O.subm_rulebook(coors, n, grid[::-1], n)
+    want = _sums_in_64_bits(feat, w, o_pairs, o_num, n)
+    A = _sums_in_64_bits(np.abs(feat), np.abs(w), o_pairs, o_num, n)
+    worst = float((np.abs(out[:n] - want) / np.maximum(A, 2.0 ** -100)).max())
+    assert np.all(np.abs(out[:n] - want) <= 2e-6 * A + 2.0 ** -126), "worst difference %.3g of the sum of |terms|" % worst
     conv.close()
 
 
