@@ -99,7 +99,7 @@ int ConvPluginBase::preparePacked() {
 bool ConvPluginBase::gemmOnMatrixCores() const {
     return weights_packed_dev_ != nullptr && !(flags_ & SESSD_FLAG_FORCE_VALU) &&
            gemm_runs_on_mfma(kernel_volume_, in_channel_, out_channel_, in_type_, out_type_) &&
-           gemm_wide_takes_rows(max_voxels_, in_channel_, in_type_);
+           gemm_wide_takes_rows(max_voxels_, in_channel_, out_channel_, in_type_);
 }
 
 int ConvPluginBase::tileRows() const { return gemm_wide_tile_rows(out_channel_, out_type_); }

@@ -69,6 +69,10 @@ constexpr int kRawBuffer = 0x00020000;         // descriptor word 3: raw 32-bit 
 enum Arith { kPlain, kThirds, kFp16 };
 constexpr Arith arith(int cin) { return cin >= 32 ? kThirds : kPlain; }  // (of FP32 features)
 
+// an entry of a pair list: input row << bits | row in the tile
+constexpr uint32_t kNoPair = 0xffffff00u;  // fills up a list's last block (no input row has that number: gemm_wide_takes_rows())
+constexpr int pair_row_bits(int tile_rows) { return tile_rows <= 64 ? 6 : 7; }
+
 template <typename T, int CIN, int COUT>  // T: the input features' type
 struct Shape {
     static constexpr Arith kArith = sizeof(T) == 2 ? kFp16 : arith(CIN);
@@ -81,6 +85,7 @@ struct Shape {
     static constexpr int kTileRows = kWgCols == 64 ? 96 : (sizeof(T) == 2 || kWgCols == 32 ? 64 : 112);  // tile capacity
     static constexpr int kPerUnit = kWgCols == 64 ? 1 : (sizeof(T) == 2 ? 4 : 2);  // workgroups that can share a compute unit
     static constexpr int kMaxBlk = kTileRows / 16;
+    static constexpr int kRowBits = pair_row_bits(kTileRows);
     static constexpr int kNone = kMaxK * kTileRows * 4;  // an item with no pairs
     static constexpr int kParts = CIN > 64 ? CIN / 64 : 1;  // of the inner dimension, taken one after the other
     static constexpr int CP = CIN / kParts;                 // channels of a part
@@ -90,9 +95,9 @@ struct Shape {
     static constexpr int kMaxSplit = kWgCols == 64 ? 1 : 0;  // log2 of the column parts that short tiles are split into
     static_assert(kTileRows <= 128 && kTileRows % 16 == 0, "the lists are staged in two halves of 64 rows");
     static_assert((CP == 4 || CP % 16 == 0) && (kArith == kPlain || kArith == kFp16 || CP % 32 == 0) && COUT % kWgCols == 0, "whole MFMA steps and column groups");
+    static_assert(kTileRows <= 1 << kRowBits, "a pair holds its row in the tile");
     static_assert((kMaxK + kWaves - 1) / kWaves * kMaxBlk * kParts + 2 <= 64, "an item a lane");
 };
-constexpr uint32_t kNoPair = 0xffffff00u;      // entry of a pair list that fills up its last block (no input row has that number)
 
 __device__ __forceinline__ void buffer_load(__amdgpu_buffer_rsrc_t r, unsigned byte_offset, int (&v)[4]) {
     const v4u32 t = __builtin_amdgcn_raw_buffer_load_b128(r, byte_offset, 0, 0);
@@ -273,7 +278,7 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
     const char* pairs = reinterpret_cast<const char*>(s_pair);
     auto entry_at = [&](int it, int j4) -> uint32_t { return *reinterpret_cast<const uint32_t*>(pairs + (kParts > 1 ? it & ~3 : it) + j4); };
     auto load_a = [&](int it, uint32_t entry, int (&a)[G][E]) {
-        const unsigned row = (entry >> 8) * (unsigned)S::kRowBytes + (kParts > 1 ? (unsigned)(it & 3) * (unsigned)S::kPartBytes : 0u);
+        const unsigned row = (entry >> S::kRowBits) * (unsigned)S::kRowBytes + (kParts > 1 ? (unsigned)(it & 3) * (unsigned)S::kPartBytes : 0u);
         const unsigned at = entry < kNoPair ? row + (lane & 3) * (unsigned)S::kLaneBytes : kOutOfRange;
 #pragma unroll
         for (int g = 0; g < G; ++g) buffer_load(rs_in, at + g * 64u, a[g]);
@@ -315,7 +320,7 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
         ++t;
         next_entry = entry_at(d2, request4);
         const uint32_t mine = entry_at(d0, operand4);
-        const int r = (int)(mine & 255u);
+        const int r = (int)(mine & ((1u << S::kRowBits) - 1u));
         float4* const dst = reinterpret_cast<float4*>(part) + r * kSlots;
         float4 sum[NB];
 #pragma unroll
@@ -406,7 +411,7 @@ conv_wide(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
     using S = Shape<T, CIN, COUT>;
     constexpr int kWgCols = S::kWgCols, kMaxSplit = S::kMaxSplit, kTileRows = S::kTileRows, kWaves = S::kWaves, kThreads = S::kThreads;
     // (one block more: all of it filling pairs)
-    __shared__ uint32_t s_pair[kMaxK * kTileRows + 16];  // compacted pair lists: pair j of offset k, input row << 8 | local output row
+    __shared__ uint32_t s_pair[kMaxK * kTileRows + 16];  // compacted pair lists: pair j of offset k
     __shared__ int32_t s_blk[kMaxK + 5];            // 16-pair blocks per offset
     __shared__ float s_epi[3 * COUT];
     __shared__ __align__(16) float s_part[kWaves * kTileRows * kWgCols];
@@ -513,7 +518,7 @@ conv_wide(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
             const uint64_t m = __ballot(v >= 0);
             if (v >= 0) {
                 const int j = base + __popcll(m & ((1ull << lane) - 1ull));
-                s_pair[k * kTileRows + j] = ((uint32_t)v << 8) | (uint32_t)(h * 64 + lane);
+                s_pair[k * kTileRows + j] = ((uint32_t)v << S::kRowBits) | (uint32_t)(h * 64 + lane);
             }
             base += __popcll(m);
         }
@@ -630,8 +635,8 @@ conv_wide(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
 
 template <int CIN, int COUT, typename T = float, typename TO = T>
 int launch(const GemmArgs& a, hipStream_t stream) {
-    // operands are addressed with 32-bit byte offsets, 2^31 means "out of range"; a pair keeps its input row in 24 bits
-    if (!gemm_wide_takes_rows(a.max_voxels, CIN, a.in_type) || (size_t)a.K * Shape<T, CIN, COUT>::kWeightBytes >= kOutOfRange)
+    // operands are addressed with 32-bit byte offsets, 2^31 means "out of range"
+    if (!gemm_wide_takes_rows(a.max_voxels, CIN, COUT, a.in_type) || (size_t)a.K * Shape<T, CIN, COUT>::kWeightBytes >= kOutOfRange)
         return SESSD_E_UNSUPPORTED;
     using S = Shape<T, CIN, COUT>;
     const int units = gemm_compute_units() * S::kPerUnit / S::kColGroups;
@@ -659,8 +664,9 @@ bool gemm_runs_wide(int K, int cin, int cout, int in_type, int out_type) {
 }
 
 // (a kernel that has a shape to itself takes more; the pipeline asks before it relies on the fused scatter)
-bool gemm_wide_takes_rows(int max_voxels, int cin, int in_type) {
-    return max_voxels < 1 << 24 && (size_t)max_voxels * cin * (in_type == SESSD_HALF ? 2 : 4) < kOutOfRange;
+bool gemm_wide_takes_rows(int max_voxels, int cin, int cout, int in_type) {
+    return (uint32_t)max_voxels <= kNoPair >> pair_row_bits(gemm_wide_tile_rows(cout, in_type)) &&
+           (size_t)max_voxels * cin * (in_type == SESSD_HALF ? 2 : 4) < kOutOfRange;
 }
 
 int gemm_wide_tile_rows(int cout, int type) {

@@ -80,7 +80,7 @@ bool gemm_cuts_own_tiles(int K, int cin, int cout, int in_type, int out_type);
 // takes, and whether it multiplies 16-bit parts of FP32 operands, which need weights of a form of their own
 bool gemm_runs_wide(int K, int cin, int cout, int in_type, int out_type);
 int gemm_wide_tile_rows(int cout, int type);
-bool gemm_wide_takes_rows(int max_voxels, int cin, int in_type);
+bool gemm_wide_takes_rows(int max_voxels, int cin, int cout, int in_type);
 bool wide_splits(int cin);
 size_t wide_weight_bytes(int K, int cin, int cout);
 void pack_wide_weights(const float* w, int K, int cin, int cout, void* dst);

@@ -241,7 +241,38 @@ def check_short_memory():
     assert rc == D.SESSD_E_HIP and not h.value
 
 
+def gemm_kernel(cin, cout, rows, dtype):
+    """The kernel that multiplies in a SubM layer of so many rows (nothing runs: the addresses are read by nobody)."""
+    d = D.SubmConv3dDesc()
+    d.in_channel, d.out_channel, d.max_voxels, d.feature_num, d.ksize, d.stride, d.padding, d.dilation = cin, cout, rows, cin, 3, 1, 1, 1
+    for a in range(3):
+        d.out_shape[a] = d.spatial_shape[a] = 1000
+    w, h = np.zeros((27, cin, cout), np.float32), C.c_void_p()
+    assert L.sessd_submconv3d_create(C.byref(d), w.ctypes.data, C.byref(h)) == 0, L.sessd_last_error()
+    ins = (D.TensorDesc * 3)(D.TensorDesc.make((1, rows, cin), dtype), D.TensorDesc.make((1, rows, 4), D.SESSD_INT32),
+                             D.TensorDesc.make((1,), D.SESSD_INT32))
+    outs = (D.TensorDesc * 1)(D.TensorDesc.make((1, rows, cout), dtype))
+    assert L.sessd_submconv3d_configure(h, ins, 3, outs, 1) == 0, L.sessd_last_error()
+    take_log()
+    assert L.sessd_submconv3d_enqueue_shared(h, ins, outs, (C.c_void_p * 3)(4096, 8192, 12288), (C.c_void_p * 1)(16384), 20480, None) == 0
+    log = take_log()
+    L.sessd_submconv3d_destroy(h)
+    assert len(log) == 1
+    return log[0][1]
+
+
+def check_row_limits():
+    """Layers with few channels run on the matrix cores in tensors of 2^24 rows and more: a pair holds an input row in 25 or 26
+    bits.  (From 32 FP32 channels up 2^24 rows are 2 GB, which operands are not addressed in.)"""
+    f32, f16 = D.SESSD_FLOAT, D.SESSD_HALF
+    for cin, cout, dtype, most in ((4, 16, f32, 2 ** 25 - 2), (4, 32, f32, 2 ** 26 - 4), (16, 16, f32, 2 ** 25 - 2), (16, 32, f32, 2 ** 25 - 1),
+                                   (16, 16, f16, 2 ** 26 - 4), (16, 32, f16, 2 ** 26 - 4), (32, 32, f32, 2 ** 24 - 1), (64, 64, f32, 2 ** 23 - 1)):
+        assert "conv_wide" in gemm_kernel(cin, cout, most, dtype), (cin, cout, dtype)
+        assert "conv_wide" not in gemm_kernel(cin, cout, most + 1, dtype), (cin, cout, dtype)
+
+
 CHECKS = {
+    "row-limits": check_row_limits,
     "recovery-direct": lambda: check_recovery(0, enqueue),
     "recovery-overlap": lambda: check_recovery(1, enqueue),
     "recovery-timed": lambda: check_recovery(1, timed),

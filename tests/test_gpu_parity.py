@@ -1075,6 +1075,33 @@ def test_fp16_kernel_with_16_channels(n, cout):
     conv.close()
 
 
+@pytest.mark.parametrize("cin,cout,half", [(4, 16, False), (16, 16, False), (16, 32, True)])
+def test_kernel_with_few_channels_in_a_tensor_of_more_than_2_to_the_24_rows(cin, cout, half):
+    """Every cell of a grid of 16 785 408, in the order of its cells: the last two lines in y, whose rows and neighbours lie beyond
+    row 2^24, against the dense convolution in 64 bits."""
+    grid = (4, 2049, 2048)
+    n = grid[0] * grid[1] * grid[2]
+    dt = torch.float16 if half else torch.float32
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(cin + cout)
+    feat = (torch.rand((n, cin), generator=gen, device="cuda:0") - 0.5).to(dt)
+    cell = torch.arange(n, dtype=torch.int32, device="cuda:0")
+    coors = torch.stack([torch.zeros_like(cell), cell // (grid[1] * grid[2]), cell // grid[2] % grid[1], cell % grid[2]], 1).contiguous()
+    rng = np.random.default_rng(cout)
+    w = rng.normal(0, 0.1, (27, cin, cout)).astype(np.float32)
+    if half:
+        w = O.round_to_half(w)
+    conv = api.SubmConv3d(cin, cout, grid[::-1], w, n)
+    out = conv(feat, coors, dev(np.array([n], np.int32)), out_dtype=dt)
+    assert conv.status() == 0
+    got = out.view(*grid, cout)[3, -2:].cpu().double()
+    x = feat.view(*grid, cin)[2:, -3:].cpu().double().permute(3, 0, 1, 2)[None]
+    k = torch.as_tensor(w).double().view(3, 3, 3, cin, cout).permute(4, 3, 0, 1, 2)
+    want, A = (torch.nn.functional.conv3d(f(x), f(k), padding=1)[0, :, 1, 1:].permute(1, 2, 0) for f in (lambda t: t, torch.abs))
+    assert torch.all((got - want).abs() <= 2e-6 * A + (2.0 ** -10 * want.abs() + 2.0 ** -24 if half else 0.0))
+    conv.close()
+
+
 def _sums_in_64_bits(feat, w, pairs, num, n):
     with np.errstate(all="ignore"):
         out = np.zeros((n, w.shape[2]))

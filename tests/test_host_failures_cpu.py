@@ -37,5 +37,9 @@ def test_a_pipeline_does_without_the_kept_tables_where_memory_is_short(fake_hip)
     run_check(fake_hip, "short-memory")
 
 
+def test_layers_with_few_channels_run_on_the_matrix_cores_in_large_tensors(fake_hip):
+    run_check(fake_hip, "row-limits")
+
+
 def test_host_memory_that_runs_out_in_a_frame_is_an_error_code(fake_hip):
     run_check(fake_hip, "host-memory")
