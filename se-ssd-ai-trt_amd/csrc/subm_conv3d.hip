@@ -41,10 +41,12 @@ subm_insert(const int32_t* __restrict__ coors, const int32_t* __restrict__ voxel
 
 // The whole rulebook of a layer of few rows in one launch: every workgroup keeps the cells of all rows in a hash table of its own,
 // in LDS, and looks up the neighbours of 64 rows.  Clearing, filling and reading a table in memory are three launches, which is what
-// a small layer spends its time on.  The table is lists of rows, one for each hash value: a row enters with one exchange, where the
-// probes of an open table, each waiting for the one before, took 8 us for 2 000 rows.  What bounds it are two trips to memory and the
-// launch.  Layer 4 -> 16, three launches before and this: 300 rows 19.0 -> 11.4 us, 2 000 18.6 -> 11.5, 8 000 19.5 -> 12.2; 64 -> 64 with 8 000
-// rows 26.4 -> 20.8.  The line lies where the table still fits LDS: lists of 8 192 rows, 128 KB.
+// a small layer spends its time on.  For each hash value the table holds the first row that has it and a list of the rows of other
+// cells: a row enters with one minimum and, where cells collide, one exchange (the probes of an open table, each waiting for the one
+// before, took 8 us for 2 000 rows).  Rows that name one cell are in no list: as one, which each of them walked, 8 192 of them were
+// a layer of 882 us, 17 now.  What bounds it are two trips to memory and the launch.  Layer 4 -> 16, three launches before and this: 300 rows 19.0 -> 11.4
+// us, 2 000 18.6 -> 11.5, 8 000 19.5 -> 13.0; 64 -> 64 with 8 000 rows 26.4 -> 22.  The line lies where the table still fits LDS: 8 192 rows and
+// their lists, 128 KB.  It is drawn at the tensors' capacity, which is what the host knows when it launches.
 constexpr int kSmallRows = 8192;
 constexpr int kSmallHeads = 16384;
 constexpr int kSmallBlock = 1024;
@@ -56,7 +58,7 @@ static_assert(kSmallRows < 0xffff, "rows in 16 bits beside kNoRow");
 __global__ void __launch_bounds__(kSmallBlock)
 subm_small_rulebook(LookupPart P, int32_t* __restrict__ tiles) {
     constexpr uint32_t kNoRow = 0xffffu;
-    __shared__ __align__(16) uint32_t s_head[kSmallHeads];  // first row of a list
+    __shared__ __align__(16) uint32_t s_head[kSmallHeads];  // of a hash value: first row << 16 | first row of the list of others
     __shared__ uint2 s_cell[kSmallRows];                    // a row's cell, the next row of its list
     __shared__ int32_t s_pairs[64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -73,7 +75,7 @@ subm_small_rulebook(LookupPart P, int32_t* __restrict__ tiles) {
     }
     const int row = blockIdx.x * 64 + lane;  // whose neighbours this lane looks up, at offsets wave, wave + kSmallWaves, ...
     const int4 own = coors[row < P.max_voxels ? row : 0];
-    for (int t = tid; t < (1 << (32 - shift)) / 4; t += kSmallBlock) reinterpret_cast<uint4*>(s_head)[t] = make_uint4(kNoRow, kNoRow, kNoRow, kNoRow);
+    for (int t = tid; t < (1 << (32 - shift)) / 4; t += kSmallBlock) reinterpret_cast<uint4*>(s_head)[t] = make_uint4(~0u, ~0u, ~0u, ~0u);
     if (tid < 64) s_pairs[tid] = 0;
     const int n = clamp_rows(P.num, P.max_voxels);
     if ((int)blockIdx.x * 64 >= n && blockIdx.x) return;
@@ -81,19 +83,31 @@ subm_small_rulebook(LookupPart P, int32_t* __restrict__ tiles) {
     auto cell = [&](int z, int y, int x) { return ((uint32_t)z * (uint32_t)P.t.gy + (uint32_t)y) * (uint32_t)P.t.gx + (uint32_t)x; };
     auto list = [&](uint32_t key) { return (key * 2654435769u) >> shift; };
     bool bad = false;
+    uint32_t mine[kSmallOwn], hash[kSmallOwn];  // (of rows that are in the layer)
 #pragma unroll
     for (int j = 0; j < kSmallOwn; ++j) {
         const int v = j * kSmallBlock + tid;
+        hash[j] = ~0u;
         if (v < n) {
             if (c[j].y < 0 || c[j].y >= P.t.gz || c[j].z < 0 || c[j].z >= P.t.gy || c[j].w < 0 || c[j].w >= P.t.gx) {
                 bad = true;  // the reference would write outside its grid
             } else {
-                const uint32_t key = cell(c[j].y, c[j].z, c[j].w);
-                s_cell[v] = make_uint2(key, atomicExch(&s_head[list(key)], (uint32_t)v));
+                mine[j] = cell(c[j].y, c[j].z, c[j].w);
+                hash[j] = list(mine[j]);
+                s_cell[v].x = mine[j];
+                atomicMin(&s_head[hash[j]], (uint32_t)v << 16 | kNoRow);
             }
         }
     }
     const bool any_bad = __syncthreads_or(bad);
+#pragma unroll
+    for (int j = 0; j < kSmallOwn; ++j) {
+        const int v = j * kSmallBlock + tid;
+        if (hash[j] == ~0u) continue;
+        const uint32_t first = s_head[hash[j]] >> 16;
+        if (s_cell[first].x != mine[j]) s_cell[v].y = atomicExch(&s_head[hash[j]], first << 16 | (uint32_t)v) & 0xffffu;
+    }
+    __syncthreads();
     if (blockIdx.x == 0 && tid < 4) {
         P.meta[tid] = tid == 0 ? (any_bad ? SESSD_STATUS_BAD_COORD : 0) : (tid == 1 ? n : 0);
         tiles[tid] = 0;
@@ -107,10 +121,14 @@ subm_small_rulebook(LookupPart P, int32_t* __restrict__ tiles) {
         const int z = own.y - P.p[0] + k / (P.k[1] * P.k[2]), y = own.z - P.p[1] + k / P.k[2] % P.k[1], x = own.w - P.p[2] + k % P.k[2];
         const bool ok = in_layer && k < P.K && z >= 0 && z < P.t.gz && y >= 0 && y < P.t.gy && x >= 0 && x < P.t.gx;
         key[j] = cell(z, y, x);
-        at[j] = ok ? s_head[list(key[j])] : kNoRow;
-        found[j] = kEmpty;
+        const uint32_t head = ok ? s_head[list(key[j])] : ~0u;
+        const uint32_t first = head >> 16;
+        const bool here = first != kNoRow && s_cell[first != kNoRow ? first : 0].x == key[j];
+        found[j] = here ? first : kEmpty;
+        at[j] = here ? kNoRow : head & 0xffffu;
+        open |= at[j] != kNoRow ? 1 : 0;
     }
-    do {  // (lists end: a row is in one of them, in front of the rows that were in it before)
+    while (open) {  // (lists end: a row is in one of them, in front of the rows that were in it before)
         open = 0;
 #pragma unroll
         for (int j = 0; j < kSmallDepth; ++j) {
@@ -120,7 +138,7 @@ subm_small_rulebook(LookupPart P, int32_t* __restrict__ tiles) {
             at[j] = e.y;
             open |= e.y != kNoRow ? 1 : 0;
         }
-    } while (open);
+    }
     int pairs = 0;
 #pragma unroll
     for (int j = 0; j < kSmallDepth; ++j) {
