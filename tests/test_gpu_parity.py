@@ -1104,6 +1104,35 @@ def test_fp16_kernel_with_16_channels(n, cout):
     conv.close()
 
 
+@pytest.mark.parametrize("cin,cout", [(16, 16), (16, 32), (32, 32), (32, 64), (64, 64), (64, 128), (128, 128)])
+@pytest.mark.parametrize("k", [(1, 1, 1), (1, 1, 2), (3, 2, 1), (1, 3, 3), (2, 3, 3)])
+@pytest.mark.parametrize("n", [1, 97, 6000, 17000])
+def test_fp16_kernel_with_pair_lists_whatever_the_kernel_volume(n, k, cin, cout):
+    """FP16 layers whose kernel volume is neither 27 nor 3 run on the kernel with pair lists: fewer offsets than waves, more than it
+    splits columns from (18), one row, more than a tile, tiles split and not."""
+    rng = np.random.default_rng([n, cin, cout, k[0] * 9 + k[1] * 3 + k[2]])
+    ig, st, p = (9, 70, 60), (1, 1, 1), tuple(v // 2 for v in k)
+    og = tuple(B.conv_out_size(ig[a], k[a], st[a], p[a]) for a in range(3))
+    coors = F.random_active_voxels(n, ig, n)
+    mv = min(n * k[0] * k[1] * k[2], og[0] * og[1] * og[2]) + 50
+    feat = O.round_to_half(rng.uniform(-1, 1, (n, cin)).astype(np.float32))
+    w = O.round_to_half(rng.normal(0, 0.1, (k[0] * k[1] * k[2], cin, cout)).astype(np.float32))
+    cbuf, fbuf = np.zeros((mv, 4), np.int32), np.zeros((mv, cin), np.float32)
+    cbuf[:n], fbuf[:n] = coors, feat
+    conv = api.SparseConv3d(cin, cout, og[::-1], ig[::-1], k, st, p, w, mv)
+    out, oc, on = conv(dev(fbuf, torch.float16), dev(cbuf), dev(np.array([n], np.int32)))
+    O.set_threads(16)
+    try:
+        pairs, num, o_oc, o_on, status = O.sparse_rulebook(coors, n, og[::-1], k, st, p, mv)
+        want, A = O.gather_gemm_scatter(feat, w, pairs, num, mv), abs_sum_of(feat, w, pairs, num, mv)
+    finally:
+        O.set_threads(1)
+    assert int(to_np(on)[0]) == o_on and np.array_equal(to_np(oc), o_oc) and conv.status() == status
+    assert_features_close(to_np(out.float()), O.round_to_half(want), RTOL_FP16, "fp16 %s %d->%d, %d rows" % (k, cin, cout, n), half=True,
+                          abs_sum=A)
+    conv.close()
+
+
 @pytest.mark.parametrize("cin,cout,half", [(4, 16, False), (16, 16, False), (16, 32, True)])
 def test_kernel_with_few_channels_in_a_tensor_of_more_than_2_to_the_24_rows(cin, cout, half):
     """Every cell of a grid of 16 785 408, in the order of its cells: the last two lines in y, whose rows and neighbours lie beyond
