@@ -677,29 +677,18 @@ int gemm_wide_tile_rows(int cout, int type) {
 bool wide_splits(int cin) { return arith(cin) != kPlain; }
 size_t wide_weight_bytes(int K, int cin, int cout) { return (size_t)K * cin * cout * 6 + cout * sizeof(float); }
 
-// the nearest BF16, as nearest_half(); cut: the next one towards zero
-static uint16_t nearest_bf16(float v, float* value, bool cut) {
-    uint32_t u;
-    std::memcpy(&u, &v, 4);
-    if ((u & 0x7fffffffu) > 0x7f800000u) u |= 0x400000u;  // (NaN)
-    else if (!cut) u += 0x7fffu + ((u >> 16) & 1u);
-    u &= 0xffff0000u;
-    std::memcpy(value, &u, 4);
-    return (uint16_t)(u >> 16);
-}
-
 // W in parts and in operand order: Wp[k][64 channels][part][step][16-column block][lane][8], element j of lane l being channel
 // 32 step + 16 (j / 4) + 4 (l / 16) + j % 4 (the channels that the lane permutation of the rows brings there), column
 // 16 block + l % 16; behind them a factor for each column.  Three parts hold a number from 2^-110 up.  A column with smaller
 // ones is multiplied by a power of two (its largest to 2^30), and divided by it where the sums are; what is too small even then
 // becomes NaN, and the column's sums are made plainly.
 void pack_wide_weights(const float* w, int K, int cin, int cout, void* dst) {
-    std::vector<float> up(cout, 1.f), big(cout, 0.f), small(cout, 1.f);
+    std::vector<float> up(cout, 1.f), big(cout, 0.f), small(cout, 1.f);  // (the columns' largest finite and smallest magnitudes)
     for (size_t t = 0; t < (size_t)K * cin; ++t)
         for (int col = 0; col < cout; ++col) {
-            const float v = std::fabs(w[t * cout + col]);
-            if (v > big[col] && v <= 3.402823466e38f) big[col] = v;  // (finite)
-            if (v < small[col] && v > 0.f) small[col] = v;
+            const float v = std::fabs(w[t * cout + col]), finite = v <= 3.402823466e38f ? v : 0.f, some = v > 0.f ? v : 1.f;
+            big[col] = finite > big[col] ? finite : big[col];
+            small[col] = some < small[col] ? some : small[col];
         }
     float* down = reinterpret_cast<float*>(static_cast<char*>(dst) + (size_t)K * cin * cout * 6);
     for (int col = 0; col < cout; ++col) {
@@ -711,17 +700,36 @@ void pack_wide_weights(const float* w, int K, int cin, int cout, void* dst) {
     const int cp = cin > 64 ? 64 : cin, steps = cp / 32, blocks = cout / 16;
     uint16_t* o = static_cast<uint16_t*>(dst);
     const size_t part_size = (size_t)steps * blocks * 512;
+    auto nearest = [](uint32_t u) { return (u + 0x7fffu + ((u >> 16) & 1u)) & 0xffff0000u; };  // BF16 in the upper half
+    std::vector<uint32_t> parts(3 * (size_t)cout);
+    uint32_t *p0 = parts.data(), *p1 = p0 + cout, *p2 = p1 + cout;
     for (int k = 0; k < K; ++k)
         for (int ch = 0; ch < cin; ++ch, w += cout) {
+            // (without branches: the weights of a backbone are 500 000 and more)
+            for (int col = 0; col < cout; ++col) {
+                float v = w[col] * up[col], part;
+                uint32_t u, rest;
+                std::memcpy(&u, &v, 4);
+                const uint32_t mag = u & 0x7fffffffu;
+                const uint32_t first = mag < 0x7f7f8000u ? nearest(u) : u & 0xffff0000u;  // (rounded, the largest would be infinite)
+                std::memcpy(&part, &first, 4);
+                v -= part;
+                std::memcpy(&u, &v, 4);
+                p1[col] = nearest(u);
+                std::memcpy(&part, &p1[col], 4);
+                v -= part;
+                std::memcpy(&rest, &v, 4);
+                p2[col] = rest;
+                p0[col] = mag >= 0x7f800000u || (rest & 0xffffu) ? 0x7fc00000u : first;
+            }
             const int in_part = ch % cp, in_step = in_part % 32;
             const int first_lane = in_step % 16 / 4 * 16, j = in_step / 16 * 4 + in_step % 4;
             uint16_t* at = o + (size_t)(k * (cin / cp) + ch / cp) * 3 * part_size + (size_t)(in_part / 32) * blocks * 512 + first_lane * 8 + j;
             for (int col = 0; col < cout; ++col) {
                 uint16_t* to = at + (size_t)(col / 16) * 512 + col % 16 * 8;
-                float v = w[col] * up[col], near = 0.f;
-                const bool cut = std::fabs(v) > 3.38953139e38f;  // (beyond the largest BF16: infinite, if rounded)
-                for (int part = 0; part < 3; ++part, v -= near) to[part * part_size] = nearest_bf16(v, &near, cut && part == 0);
-                if (v != 0.f) to[0] = 0x7fc0;
+                to[0] = (uint16_t)(p0[col] >> 16);
+                to[part_size] = (uint16_t)(p1[col] >> 16);
+                to[2 * part_size] = (uint16_t)(p2[col] >> 16);
             }
         }
 }
