@@ -20,8 +20,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-fast-math", "-Wall", "-Wno-unused-function",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          # A kernel's first arguments are in registers when it starts: they were a trip to memory of their own, 300-500 cycles, in
-         # front of everything else.  20 launches in a row pay it one after the other: frames of 2 000 points 196.1 -> 193.9 us, of
-         # 20 000 273.3 -> 269.1, a SubM layer 64 -> 64 with its rulebook 35.0 -> 34.5.  (16 arguments measured the same.)
+         # front of everything else.  A SubM layer 64 -> 64 with its rulebook 39.7 -> 39.3 us; frames, whose launches overlap, 208.8 and
+         # 298 us with it, 209.0 and 298.5 without (two runs differ by 0.6 and 1.2).
          "-mllvm", "-amdgpu-kernarg-preload-count=8"]
 
 # conv_tile.hip keeps its accumulators over a loop in which nothing else may wait; left to itself the compiler puts them

@@ -10,21 +10,21 @@
 // follow, each row is stored once.  Results are bit-identical run to run.
 //
 // Products.  The FP32 matrix instruction does 32 multiply-adds a cycle and SIMD, the 16-bit ones 512.  From 32 channels up both
-// operands are split into three BF16 parts of eight bits, x = x0 + x1 + x2 exactly, and the six largest products of
+// operands are split into three BF16 parts of eight bits each, x = x0 + x1 + x2 exactly, and the six largest products of
 // parts are added in FP32, smallest first (v_mfma_f32_16x16x32_bf16; 6/16 of the FP32 instruction's time).  What is left out is
-// below 2^-23 of a product, and BF16 has FP32's range, so that this holds for every element by itself, whatever the others of its row or column are.  What does not fit --
-// numbers below 2^-110 whose last bits lie under BF16's smallest number, infinities and NaN, sums that overflow on the
-// way -- comes out as something that is not finite, and such elements are summed again, plainly (direct_sum()).  Two FP16
-// parts of operands scaled by row and column are three products instead of six (64 -> 64 at 17 262 rows 19.1 us, 24.9 so) but
-// hold an element to 2^-24 of its row's largest and not of itself: a channel at 1e8 beside others at 1 cost these 5e-5 of
-// their sums.  Cin 4 and 16: the FP32 instruction (4 or 16 of them a block: it is not what they wait for).
-// Distance from the sums in 64 bits, 2-norm, FP32 instruction and parts: 64 -> 64 1.27e-7, 0.72e-7; 128 -> 128 1.31e-7, 0.81e-7; 64 -> 128
-// 1.24e-7, 0.72e-7; 32 -> 64 1.00e-7, 0.70e-7; 32 -> 32 0.93e-7, 0.67e-7.
+// below 2^-23 of a product, and BF16 has FP32's range, so that this holds for every element by itself, whatever the others
+// of its row or column are.  What does not fit -- numbers below 2^-110 whose last bits lie under BF16's smallest number,
+// infinities and NaN, sums that overflow on the way -- comes out as something that is not finite, and such elements are
+// summed again, plainly (direct_sum()).  Two FP16 parts of operands scaled by row and column are three products (64 -> 64 at 17 262
+// rows 19.1 us, 24.9 so; the FP32 instruction 32.2) but hold an element to 2^-24 of its row's largest and not of itself: one channel
+// at 1e8 beside others at 1 cost these 5e-5 of their sums.  Cin 4 and 16: the FP32 instruction (it is not what they wait for).
+// Distance from the sums in 64 bits, 2-norm, FP32 instruction and parts: 64 -> 64 1.27e-7, 0.72e-7; 128 -> 128 1.31e-7, 0.81e-7; 32 -> 32
+// 0.93e-7, 0.67e-7.
 //
 // What bounds it: a block of 64 -> 64 is 768 cycles of MFMA (with half of them left out the launch above takes 20.0 us), the rest a wave's
 // instructions and LDS.  Hence
 //   * a wave takes all 64 columns: rows are requested, permuted and split once;
-//   * six waves: as many partial tiles of 96 rows as LDS holds.  Eight with 72 rows are faster until a tile does not fit;
+//   * six waves: as many partial tiles of 96 rows as LDS holds;
 //   * the rows of the block after next are requested, and the next block's split, under a block's MFMAs; the next offset's
 //     weights are requested with the first block of an offset into a second set of registers, or, where these do not hold two
 //     sets (64 x 64), behind the MFMAs of its last into the only one;
@@ -35,11 +35,6 @@
 // 28 043 rows) and makes the slower frame (20 000 points: 283 us against 274); 4 -> 32 likewise (487 against 475).
 // FP16 features (Cin 16) have so little in each block that four waves and 64 rows do: four workgroups share a unit, with 40 KB of LDS
 // each.  From 32 channels up FP16 is faster without pair lists (32 -> 32 at 45 874 rows 10.6 us on conv_tall.hip, 18 here).
-//
-// Launches of SubM layers at the sites of scans, us, with the FP32 instruction (sixteen waves, or split-K) and now: 64 -> 64 at 3 051 rows
-// 10.7, 11.9; 7 120 18.3, 16.3; 17 262 32.2, 24.9; 23 959 48.7, 39.4; 128 -> 128 at 3 815 rows 33.9, 24.8; 17 262 121, 76; 64 -> 128 at 17 262 58, 46;
-// 32 -> 64 at 28 043 32, 26; 32 -> 32 at 28 043 19.3, 16.7; 45 874 36.1, 27.8; 16 -> 16 at 17 132 8.3, 7.3; 4 -> 16 7.4, 6.5; 16 -> 32 10.2, 9.0, but
-// 14.9, 16.8 at 36 871 rows (a second round of tiles begins at 32 768).  FP16 16 -> 16 at 60 000 rows 14.2, 10.8; 16 -> 32 16.6, 12.9.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
