@@ -687,3 +687,24 @@ def test_more_points_than_the_numbering_reads_one_by_one(overlap):
             assert_end_to_end_close(to_np(dense), ref["dense"], False, "dense, step %d" % step)
     finally:
         O.set_threads(1)
+
+
+@pytest.mark.parametrize("width", [1, 2])
+@pytest.mark.parametrize("schedule", [{}, dict(overlap_streams=True, use_graph=True, skip_pad_rows=True)], ids=["direct", "graph"])
+def test_frame_of_very_small_features_through_the_split_products(width, schedule):
+    """The first layer scales its features to 2^-108 and below, the last one back: rows whose elements do not fit their BF16 parts
+    in every layer from 32 channels up, the last one with its scatter into the dense tensor among them.  Against the VALU kernels,
+    within the whole-frame bound."""
+    pts = F.lidar_frame(3000, 5)
+    layers = B.reference_layers(width_mult=width)
+    W = B.random_weights(layers, seed=9, w_std=0.05, bn=False)
+    W.scale[0] *= np.float32(2.0 ** -108)
+    W.scale[-1] *= np.float32(2.0 ** 108)
+    kw = dict(share_rulebooks=True, **schedule)
+    fast, a, _ = run_pipeline(pts, layers, W, 3000, 20000, **kw)
+    slow, b, _ = run_pipeline(pts, layers, W, 3000, 20000, force_valu=True, **kw)
+    inside = fast.read_layer(len(layers) - 3)[0]
+    assert 0 < np.abs(inside).max() < 2.0 ** -90 and (np.abs(inside[inside != 0]) < 2.0 ** -110).mean() > 0.05
+    a, b = to_np(a), to_np(b)
+    assert np.isfinite(a).all() and a.any()
+    assert_end_to_end_close(a, b, False, "very small features, MFMA vs VALU")
