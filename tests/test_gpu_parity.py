@@ -1030,10 +1030,10 @@ def test_every_row_is_a_pad_row(cin, cout, half):
 
 
 @pytest.mark.parametrize("cin", [64, 128])
-@pytest.mark.parametrize("n", [1, 65, 97, 1536, 1537, 5120, 5121, 12289, 20000])
+@pytest.mark.parametrize("n", [1, 65, 97, 1536, 1537, 3840, 3841, 5120, 5121, 12289, 20000])
 def test_wide_fp32_kernel_with_128_columns(n, cin):
     """128 output columns: two workgroups take 64 columns each of every tile (128 tiles a round on 256 compute units, of
-    up to 96 rows), up to 5 120 rows four; 128 input channels are walked in two parts.  Against
+    up to 96 rows), up to 3 840 rows four; 128 input channels are walked in two parts.  Against
     the oracle (pad rows included)."""
     rng = np.random.default_rng(n + cin)
     grid, mv = ((5, 40, 40) if n < 1000 else (21, 400, 352)), n + 39
