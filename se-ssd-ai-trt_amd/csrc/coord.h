@@ -210,6 +210,7 @@ struct LookupPart {
     int max_voxels = 0;
     int k[3], s[3], p[3];  // z,y,x
     int K = 0;
+    int first[4];  // first offset of each quarter: z << 16 | y << 8 | x (launch_flags_lookups())
     int own[3];  // the layer's grid (z,y,x): a row outside it has no neighbours
     CellTable t;
     const int32_t* t_num = nullptr;  // rows the table was opened with

@@ -406,16 +406,22 @@ __global__ void __launch_bounds__(kCoordBlock) sp_insert(SpPart P) {
     }
 }
 
-__device__ __forceinline__ void sp_flags_pass(const SpPart& P, int block, int blocks, uint32_t* lds4) {
-    const int n = clamp_rows(P.in_num, P.max_voxels);
-    const int64_t tickets = (int64_t)n * P.Kc;
-    const CellView t = open_table(P.t, n);
+// A launch passes its arguments by value, and the compiler reads each of them where it is used: one trip to memory of 400-1 100
+// cycles after the other, nine in a row in front of the first probe of a lookup.  The passes name all that they need in one place
+// (an asm without instructions), so that it arrives together.
+__device__ __forceinline__ void sp_flags_pass(const SpPart& a, int block, int blocks, uint32_t* lds4) {
+    SpPart P = a;
+    asm volatile("" :: "s"(P.in_num), "s"(P.max_voxels), "s"(P.Kc), "s"(P.t.base), "s"(P.t.dense), "s"(P.cand), "s"(P.words), "s"(P.counts));
+    // (the first chunk's tickets beside the row count: in bounds, there are at most n_chunks blocks)
+    uint32_t slot = P.cand[(uint32_t)block * kCoordBlock + threadIdx.x];
+    const int64_t tickets = (int64_t)clamp_rows(P.in_num, P.max_voxels) * P.Kc;
     for (int c = block; (int64_t)c * kCoordBlock < tickets; c += blocks) {
         const uint32_t tk = (uint32_t)c * kCoordBlock + threadIdx.x;
+        if (c != block) slot = P.cand[tk];
         bool first = false;
-        if (tk < tickets) {
-            const uint32_t slot = P.cand[tk];
-            first = slot != kEmpty && value_at(t, slot & kSlotMask) == tk;
+        if (tk < tickets && slot != kEmpty) {
+            const uint32_t at = slot & kSlotMask;
+            first = (P.t.dense ? static_cast<const uint32_t*>(P.t.base)[at] : static_cast<const uint32_t*>(P.t.base)[2 * (size_t)at]) == tk;
         }
         const uint64_t m = __ballot(first);
         __syncthreads();
@@ -431,132 +437,174 @@ __device__ __forceinline__ void sp_flags_pass(const SpPart& P, int block, int bl
 // ---------------------------------------------------------------------------------------------
 // lookups
 // ---------------------------------------------------------------------------------------------
-// A wave takes 16 rows, four lanes per row with a quarter of the offsets each: the probes of a lane are independent
-// loads, all in flight at once, and its stores are runs of 16 rows.  With one (row, offset) per thread, two dependent
-// loads per probe and the upper half of the offsets written by symmetry this took 7-21 us at 16 000 - 75 000 rows (kernel
-// trace, where an empty launch reads 4.6); now 5.9 at 2 000, 6.2 at 27 000 and 10.5 at 75 000 rows of a dense table, 12-26
-// of a hash, whose 27 probes per row land on 27 lines.
+// A block takes 64 rows, a lane each; each of its four waves takes a quarter of the offsets, so that an offset's place in the kernel
+// is the same for the whole wave, all probes of a lane are in flight at once, and stores are runs of 64 rows.
+// A block of 64 rows at 17 262 rows: 11 900 cycles with four lanes a row (each lane a quarter of the offsets, their places found per
+// lane: 2 000 for seven keys) and the arguments read as they came, 6 100 now; the SubM plugin 64 -> 64 40.3 -> 37.9 us, frames of 2 000
+// points 205.5 -> 200.8, 20 000 306.9 -> 300.6, 60 000 (FP16) 250.7 -> 246.4.
 constexpr int kLookupRows = 64;                             // rows of a block
-constexpr int kLookupDepth = (kGemmMaxOffsets + 3) / 4;     // offsets of a lane
+constexpr int kLookupDepth = (kGemmMaxOffsets + 3) / 4;     // offsets of a wave
+struct LookupLds {
+    int32_t found[kCoordBlock];  // by each wave for each row
+    int32_t sum[4];              // ... for all of its rows
+};
 
-__device__ __forceinline__ void lookup_pass(const LookupPart& P, int block, int32_t* lds4) {
-    const int n = clamp_rows(P.num, P.max_voxels);
-    if (P.meta && block == 0 && threadIdx.x == 0) {
-        P.meta[1] = n;
-    }
-    const CellView t = open_table(P.t, clamp_rows(P.t_num, P.t_max));
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int i = lane & 15, q = lane >> 4;
-    const int per = (P.K + 3) >> 2;
-    const int k0 = q * per;
-    int kz0 = k0 / (P.k[1] * P.k[2]), ky0 = (k0 / P.k[2]) % P.k[1], kx0 = k0 % P.k[2];
-    for (int chunk = block; chunk * kLookupRows < n; chunk += P.blocks) {
-        const int row = chunk * kLookupRows + wave * 16 + i;
-        uint32_t key[kLookupDepth];
-        bool in_layer = false;
-        int4 c = make_int4(0, 0, 0, 0);
-        if (row < n) {
-            c = reinterpret_cast<const int4*>(P.coors)[row];
-            in_layer = c.y >= 0 && c.y < P.own[0] && c.z >= 0 && c.z < P.own[1] && c.w >= 0 && c.w < P.own[2];
-        }
-        const int z0 = c.y * P.s[0] - P.p[0], y0 = c.z * P.s[1] - P.p[1], x0 = c.w * P.s[2] - P.p[2];
-        int kz = kz0, ky = ky0, kx = kx0;
+// What a wave finds for a row: val[j] = the row at the wave's j-th offset.  QUARTER 0 .. 3: of a 3x3x3 kernel on a dense table, where
+// the offsets are constants; -1: any (`start`: the first offset, z << 16 | y << 8 | x, `mine`: how many).
+template <int QUARTER>
+__device__ __forceinline__ void look_up(const LookupPart& P, const int4& c, bool in_layer, int start, int mine, uint32_t (&val)[kLookupDepth]) {
+    const int z0 = c.y * P.s[0] - P.p[0], y0 = c.z * P.s[1] - P.p[1], x0 = c.w * P.s[2] - P.p[2];
+    const uint32_t origin = ((uint32_t)z0 * (uint32_t)P.t.gy + (uint32_t)y0) * (uint32_t)P.t.gx + (uint32_t)x0;
+    uint32_t key[kLookupDepth];
+    bool ok[kLookupDepth];
+    auto probe = [&](int j, int kz, int ky, int kx) {
+        ok[j] = in_layer && (uint32_t)(z0 + kz) < (uint32_t)P.t.gz && (uint32_t)(y0 + ky) < (uint32_t)P.t.gy && (uint32_t)(x0 + kx) < (uint32_t)P.t.gx;
+        key[j] = origin + ((uint32_t)(kz * P.t.gy + ky) * (uint32_t)P.t.gx + (uint32_t)kx);
+    };
+    if constexpr (QUARTER >= 0) {
+        const uint32_t* d = static_cast<const uint32_t*>(P.t.base);
 #pragma unroll
         for (int j = 0; j < kLookupDepth; ++j) {
-            const int z = z0 + kz, y = y0 + ky, x = x0 + kx;
-            const bool ok = in_layer && j < per && k0 + j < P.K && z >= 0 && z < P.t.gz && y >= 0 && y < P.t.gy && x >= 0 && x < P.t.gx;
-            key[j] = ok ? ((uint32_t)z * (uint32_t)P.t.gy + (uint32_t)y) * (uint32_t)P.t.gx + (uint32_t)x : kEmpty;
-            if (++kx == P.k[2]) {
-                kx = 0;
-                if (++ky == P.k[1]) {
-                    ky = 0;
-                    ++kz;
-                }
-            }
-        }
-        int cnt = 0;
-        if (t.d) {
-            uint32_t v[kLookupDepth];
-#pragma unroll
-            for (int j = 0; j < kLookupDepth; ++j) v[j] = key[j] != kEmpty ? t.d[key[j]] : kEmpty;
-#pragma unroll
-            for (int j = 0; j < kLookupDepth; ++j) {
-                cnt += v[j] != kEmpty ? 1 : 0;
-                if (row < n && j < per && k0 + j < P.K) P.nbr[(size_t)(k0 + j) * P.max_voxels + row] = (int32_t)v[j];
-            }
-        } else {
-            // All probe sequences advance together, a round of loads at a time, four entries per sequence and round: one
-            // after the other the collisions of seven sequences were seven times the latency (15 us for 2 000 rows).
-            uint32_t slot[kLookupDepth], val[kLookupDepth];
-            bool open[kLookupDepth], any = false;
-#pragma unroll
-            for (int j = 0; j < kLookupDepth; ++j) {
-                slot[j] = first_slot(t, key[j]);
+            constexpr int kFirst = QUARTER * kLookupDepth;
+            const int k = kFirst + j;
+            if (k >= 27) {
                 val[j] = kEmpty;
-                open[j] = key[j] != kEmpty;
-                any |= open[j];
+                continue;
             }
-            for (uint32_t round = 0; any && round <= t.mask; round += kGroup) {
-                EntryGroup g[kLookupDepth];
+            probe(j, k / 9, k / 3 % 3, k % 3);
+            val[j] = d[ok[j] ? key[j] : 0];
+        }
 #pragma unroll
-                for (int j = 0; j < kLookupDepth; ++j)
-                    if (open[j]) g[j] = load_group(t, slot[j]);
-                any = false;
+        for (int j = 0; j < kLookupDepth; ++j)
+            if (QUARTER * kLookupDepth + j < 27) val[j] = ok[j] ? val[j] : kEmpty;
+        return;
+    }
+    int kz = start >> 16, ky = (start >> 8) & 255, kx = start & 255;
 #pragma unroll
-                for (int j = 0; j < kLookupDepth; ++j) {
-                    if (open[j]) {
-#pragma unroll
-                        for (int e = 0; e < kGroup; ++e) {
-                            if (e < (int)(slot[j] & (kGroup - 1))) continue;
-                            if (entry_key(g[j].e[e]) == key[j]) {
-                                val[j] = entry_val(g[j].e[e]);
-                                open[j] = false;
-                            } else if (g[j].e[e] == kEmptyEntry) {
-                                open[j] = false;
-                            }
-                        }
-                        slot[j] = ((slot[j] | (kGroup - 1)) + 1) & t.mask;
-                    }
-                    any |= open[j];
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < kLookupDepth; ++j) {
-                cnt += val[j] != kEmpty ? 1 : 0;
-                if (row < n && j < per && k0 + j < P.K) P.nbr[(size_t)(k0 + j) * P.max_voxels + row] = (int32_t)val[j];
+    for (int j = 0; j < kLookupDepth; ++j) {
+        probe(j, kz, ky, kx);
+        ok[j] = ok[j] && j < mine;
+        if (++kx == P.k[2]) {
+            kx = 0;
+            if (++ky == P.k[1]) {
+                ky = 0;
+                ++kz;
             }
         }
-        if (P.w) {
-            cnt += __shfl_xor(cnt, 16, 64);
-            cnt += __shfl_xor(cnt, 32, 64);
-            int w = row < n ? cnt + P.row_weight : 0;
-            if (q == 0 && row < P.max_voxels) P.w[row] = w;
+    }
+    if (P.t.dense) {
+        const uint32_t* d = static_cast<const uint32_t*>(P.t.base);
 #pragma unroll
-            for (int d = 8; d > 0; d >>= 1) w += __shfl_xor(w, d, 64);
-            __syncthreads();
-            if (lane == 0) lds4[wave] = w;
-            __syncthreads();
-            if (threadIdx.x == 0) P.wsum[chunk] = lds4[0] + lds4[1] + lds4[2] + lds4[3];
+        for (int j = 0; j < kLookupDepth; ++j) val[j] = d[ok[j] ? key[j] : 0];
+#pragma unroll
+        for (int j = 0; j < kLookupDepth; ++j) val[j] = ok[j] ? val[j] : kEmpty;
+        return;
+    }
+    // All probe sequences advance together, a round of loads at a time, four entries per sequence and round: one
+    // after the other the collisions of seven sequences were seven times the latency (15 us for 2 000 rows).
+    const CellView t = open_table(P.t, clamp_rows(P.t_num, P.t_max));
+    uint32_t slot[kLookupDepth];
+    bool any = false;
+#pragma unroll
+    for (int j = 0; j < kLookupDepth; ++j) {
+        slot[j] = first_slot(t, key[j]);
+        val[j] = kEmpty;
+        any |= ok[j];
+    }
+    for (uint32_t round = 0; any && round <= t.mask; round += kGroup) {
+        EntryGroup g[kLookupDepth];
+#pragma unroll
+        for (int j = 0; j < kLookupDepth; ++j)
+            if (ok[j]) g[j] = load_group(t, slot[j]);
+        any = false;
+#pragma unroll
+        for (int j = 0; j < kLookupDepth; ++j) {
+            if (ok[j]) {
+#pragma unroll
+                for (int e = 0; e < kGroup; ++e) {
+                    if (e < (int)(slot[j] & (kGroup - 1))) continue;
+                    if (entry_key(g[j].e[e]) == key[j]) {
+                        val[j] = entry_val(g[j].e[e]);
+                        ok[j] = false;
+                    } else if (g[j].e[e] == kEmptyEntry) {
+                        ok[j] = false;
+                    }
+                }
+                slot[j] = ((slot[j] | (kGroup - 1)) + 1) & t.mask;
+            }
+            any |= ok[j];
         }
     }
 }
 
+// CUBE: a 3x3x3 kernel on a dense table
+template <bool CUBE>
+__device__ __forceinline__ void lookup_rows(const LookupPart& P, int block, int n, int start, int4 c, LookupLds& L) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int K = CUBE ? 27 : P.K, per = (K + 3) >> 2, k0 = wave * per, mine = K - k0 < per ? K - k0 : per;  // (mine may be negative: none)
+    int row = block * kLookupRows + lane;
+    for (int chunk = block; chunk * kLookupRows < n; chunk += P.blocks, row += P.blocks * kLookupRows) {
+        if (chunk != block) c = reinterpret_cast<const int4*>(P.coors)[row < n ? row : n - 1];
+        const bool in_layer = row < n && (uint32_t)c.y < (uint32_t)P.own[0] && (uint32_t)c.z < (uint32_t)P.own[1] && (uint32_t)c.w < (uint32_t)P.own[2];
+        uint32_t val[kLookupDepth];
+        if (!CUBE) look_up<-1>(P, c, in_layer, start, mine, val);
+        else if (wave == 0) look_up<0>(P, c, in_layer, 0, 0, val);
+        else if (wave == 1) look_up<1>(P, c, in_layer, 0, 0, val);
+        else if (wave == 2) look_up<2>(P, c, in_layer, 0, 0, val);
+        else look_up<3>(P, c, in_layer, 0, 0, val);
+        int cnt = 0, sum = 0;
+        int32_t* to = P.nbr + (size_t)k0 * P.max_voxels + row;
+#pragma unroll
+        for (int j = 0; j < kLookupDepth; ++j, to += P.max_voxels) {
+            if (j >= (CUBE ? 27 - 3 * kLookupDepth : 0) && j >= mine) break;
+            const bool hit = val[j] != kEmpty;
+            cnt += hit ? 1 : 0;
+            sum += __popcll(__ballot(hit));
+            if (row < n) *to = (int32_t)val[j];
+        }
+        if (P.w) {
+            __syncthreads();
+            L.found[threadIdx.x] = cnt;
+            if (lane == 0) L.sum[wave] = sum;
+            __syncthreads();
+            if (wave == 0) {
+                const int w = cnt + L.found[64 + lane] + L.found[128 + lane] + L.found[192 + lane] + P.row_weight;
+                if (row < P.max_voxels) P.w[row] = row < n ? w : 0;
+                const int rows = n - chunk * kLookupRows < kLookupRows ? n - chunk * kLookupRows : kLookupRows;
+                if (lane == 0) P.wsum[chunk] = L.sum[0] + L.sum[1] + L.sum[2] + L.sum[3] + rows * P.row_weight;
+            }
+        }
+    }
+}
+
+__device__ __forceinline__ void lookup_pass(const LookupPart& a, int block, LookupLds& L) {
+    const LookupPart P = a;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), start = a.first[wave];
+    asm volatile("" :: "s"(P.coors), "s"(P.num), "s"(P.max_voxels), "s"(P.t.base), "s"(P.nbr), "s"(P.meta), "s"(P.w), "s"(P.K), "s"(start));
+    const int row = block * kLookupRows + (threadIdx.x & 63);
+    // (the first rows' coordinates beside the row count: in bounds, not used beyond the active ones)
+    const int4 c = reinterpret_cast<const int4*>(P.coors)[row < P.max_voxels ? row : P.max_voxels - 1];
+    const int n = __builtin_amdgcn_readfirstlane(clamp_rows(P.num, P.max_voxels));
+    if (P.meta && block == 0 && threadIdx.x == 0) P.meta[1] = n;
+    if (block * kLookupRows >= n) return;
+    if (P.t.dense && P.k[0] == 3 && P.k[1] == 3 && P.k[2] == 3) lookup_rows<true>(P, block, n, start, c, L);
+    else lookup_rows<false>(P, block, n, start, c, L);
+}
+
 struct FlagsLookups {
     SpPart flags;
-    int flag_blocks;
     LookupPart look[kMaxLookups];
-    int n_look;
 };
 
-__global__ void __launch_bounds__(kCoordBlock) flags_lookups(FlagsLookups a) {
-    __shared__ uint32_t lds4[4];
-    int b = blockIdx.x;
-    if (b < a.flag_blocks) return sp_flags_pass(a.flags, b, a.flag_blocks, lds4);
-    b -= a.flag_blocks;
-    for (int l = 0; l < a.n_look; ++l) {
-        if (b < a.look[l].blocks) return lookup_pass(a.look[l], b, reinterpret_cast<int32_t*>(lds4));
-        b -= a.look[l].blocks;
-    }
+// end1 .. end3: where the blocks of the lookups behind the first begin.  (Arguments of their own: those are in registers when the
+// kernel starts.)
+__global__ void __launch_bounds__(kCoordBlock) flags_lookups(int flag_blocks, int end1, int end2, int end3, FlagsLookups a) {
+    __shared__ LookupLds L;
+    const int b = blockIdx.x;
+    if (b < flag_blocks) return sp_flags_pass(a.flags, b, flag_blocks, reinterpret_cast<uint32_t*>(L.sum));
+    const int l = __builtin_amdgcn_readfirstlane((b >= end1 ? 1 : 0) + (b >= end2 ? 1 : 0) + (b >= end3 ? 1 : 0));
+    static_assert(kMaxLookups == 4, "one argument for each lookup but the first");
+    lookup_pass(a.look[l], b - (l == 0 ? flag_blocks : (l == 1 ? end1 : (l == 2 ? end2 : end3))), L);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -850,20 +898,28 @@ int launch_sp_insert(const SpPart& s, hipStream_t stream) {
 int launch_flags_lookups(const SpPart* flags, const LookupPart* lookups, int n, hipStream_t stream) {
     if (n < 0 || n > kMaxLookups) return fail(SESSD_E_INVALID, "lookups: at most %d in one launch", kMaxLookups);
     FlagsLookups a;
-    a.flag_blocks = 0;
+    int flag_blocks = 0;
     if (flags) {
         a.flags = *flags;
-        a.flag_blocks = sp_pass_blocks(*flags);
+        flag_blocks = sp_pass_blocks(*flags);
     }
-    int blocks = a.flag_blocks;
-    a.n_look = n;
-    for (int l = 0; l < n; ++l) {
-        a.look[l] = lookups[l];
-        a.look[l].blocks = lookup_blocks(lookups[l].max_voxels);
-        blocks += a.look[l].blocks;
+    int blocks = flag_blocks, end[kMaxLookups];
+    for (int l = 0; l < kMaxLookups; ++l) {
+        if (l < n) {
+            LookupPart& p = a.look[l];
+            p = lookups[l];
+            p.blocks = lookup_blocks(p.max_voxels);
+            const int per = (p.K + 3) >> 2;  // (offsets of a wave)
+            for (int w = 0; w < 4; ++w) {
+                const int k = w * per;
+                p.first[w] = (k / (p.k[1] * p.k[2])) << 16 | (k / p.k[2] % p.k[1]) << 8 | k % p.k[2];
+            }
+            blocks += p.blocks;
+        }
+        end[l] = blocks;
     }
     if (!blocks) return SESSD_OK;
-    hipLaunchKernelGGL(flags_lookups, dim3(blocks), dim3(kCoordBlock), 0, stream, a);
+    hipLaunchKernelGGL(flags_lookups, dim3(blocks), dim3(kCoordBlock), 0, stream, flag_blocks, end[0], end[1], end[2], a);
     SESSD_HIP_TRY(hipGetLastError());
     return SESSD_OK;
 }
