@@ -133,14 +133,40 @@ __device__ __forceinline__ int clamp_rows(const int32_t* p, int cap) {
     const int n = *p;
     return n < 0 ? 0 : (n > cap ? cap : n);
 }
-// sum of v over the block, returned to every thread
-__device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t* lds4) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+// Sum over the lanes up to and with this one.  (Data-parallel moves between lanes: six additions, where a sum by __shfl is six trips
+// through LDS, some 700 cycles.)
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr:1, 2, 4, 8: sums in rows of 16
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15: the row before, into rows 1 and 3
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31: both rows before, into rows 2 and 3
+    return v;
+}
+// sums of a and b over the block, returned to every thread; lds: eight words
+__device__ __forceinline__ void block_sums(uint32_t& a, uint32_t& b, uint32_t* lds) {
+    a = wave_scan(a);
+    b = wave_scan(b);
     __syncthreads();
-    if ((threadIdx.x & 63) == 0) lds4[threadIdx.x >> 6] = v;
+    if ((threadIdx.x & 63) == 63) {
+        lds[threadIdx.x >> 6] = a;
+        lds[4 + (threadIdx.x >> 6)] = b;
+    }
     __syncthreads();
-    return lds4[0] + lds4[1] + lds4[2] + lds4[3];
+    a = lds[0] + lds[1] + lds[2] + lds[3];
+    b = lds[4] + lds[5] + lds[6] + lds[7];
+}
+// n / d for inv = reciprocal(d): off by one at most before the correction, as d * inv is within d of 2^32
+__host__ __device__ inline uint32_t reciprocal(uint32_t d) { return 0xffffffffu / d; }
+__device__ __forceinline__ uint32_t divide(uint32_t n, uint32_t d, uint32_t inv, uint32_t& rest) {
+    uint32_t q = __umulhi(n, inv);
+    rest = n - q * d;
+    if (rest >= d) {
+        rest -= d;
+        ++q;
+    }
+    return q;
 }
 #endif
 
@@ -186,6 +212,7 @@ struct VgPart {
 struct SpPart {
     int k[3], s[3], p[3], os[3];  // z,y,x
     int Kc = 0;                   // enumeration slots per input row
+    int halving = 0;              // kernels of 3 and strides of 2 on every axis (Kc = 8)
     int max_voxels = 0;           // rows of the input and of the output tensors
     int K = 0;
     CellTable t;  // output cell -> smallest ticket, then output row
@@ -193,6 +220,7 @@ struct SpPart {
     uint64_t* words = nullptr;
     uint32_t* counts = nullptr;
     int n_chunks = 0;  // 256-ticket chunks at capacity
+    uint32_t per_plane = 0, per_line = 0;  // reciprocal() of the output grid's cells a plane and a line (launch_number())
     const int32_t* in_coors = nullptr;
     const int32_t* in_num = nullptr;
     int32_t* out_coors = nullptr;

@@ -66,13 +66,16 @@ __global__ void __launch_bounds__(kCoordBlock) vg_insert(VgPart p, Cleans cleans
         }
         return fill_pass(also, b);
     }
-    if (p.sums && threadIdx.x == 0 && blockIdx.x % kCountsPerSum == 0) p.sums[blockIdx.x / kCountsPerSum] = 0;
+    asm volatile("" :: "s"(p.points), "s"(p.points_size), "s"(p.max_points), "s"(p.pf), "s"(p.min_x), "s"(p.vz), "s"(p.gx), "s"(p.t.base), "s"(p.t.dense),
+                 "s"(p.pt_slot), "s"(p.sums), "s"(p.status));
     const int i = blockIdx.x * kCoordBlock + threadIdx.x;
-    const int n = clamp_rows(p.points_size, p.max_points);
+    const float* pt = p.points + (size_t)(i < p.max_points ? i : p.max_points - 1) * p.pf;  // (beside the number of points)
+    const float x = pt[0], y = pt[1], z = pt[2];
+    const int n = __builtin_amdgcn_readfirstlane(clamp_rows(p.points_size, p.max_points));
+    if (p.sums && threadIdx.x == 0 && blockIdx.x % kCountsPerSum == 0) p.sums[blockIdx.x / kCountsPerSum] = 0;
     if (i >= n) return;
-    const float* pt = p.points + (size_t)i * p.pf;
     int ix, iy, iz;
-    const uint32_t key = point_cell(p, pt[0], pt[1], pt[2], ix, iy, iz);
+    const uint32_t key = point_cell(p, x, y, z, ix, iy, iz);
     int32_t slot = -1;
     if (key != kEmpty) {
         slot = insert_min(open_table(p.t, n), key, (uint32_t)i);
@@ -88,11 +91,13 @@ template <int N>
 __global__ void __launch_bounds__(kCoordBlock) vg_flags(VgPart p, FillPlan<N> also) {
     if ((int)blockIdx.x >= p.n_blocks) return fill_pass(also, blockIdx.x - p.n_blocks);
     __shared__ uint32_t lds4[4];
+    asm volatile("" :: "s"(p.points_size), "s"(p.max_points), "s"(p.max_pts), "s"(p.t.base), "s"(p.t.dense), "s"(p.slots), "s"(p.pt_slot), "s"(p.words),
+                 "s"(p.counts), "s"(p.sums));
     const int i = blockIdx.x * kCoordBlock + threadIdx.x;
-    const int n = clamp_rows(p.points_size, p.max_points);
+    const int32_t slot = p.pt_slot[i < p.max_points ? i : p.max_points - 1];  // (beside the number of points)
+    const int n = __builtin_amdgcn_readfirstlane(clamp_rows(p.points_size, p.max_points));
     bool first = false;
     if (i < n) {
-        const int32_t slot = p.pt_slot[i];
         if (slot >= 0) {
             const uint32_t f = value_at(open_table(p.t, n), slot);
             first = f == (uint32_t)i;
@@ -127,6 +132,7 @@ __global__ void __launch_bounds__(kCoordBlock) vg_flags(VgPart p, FillPlan<N> al
 __device__ __forceinline__ int div_trunc(int x, int s) {
     if (s == 1) return x;
     if (s == 2) return (x - (x >> 31)) >> 1;
+    asm volatile("" : "+s"(s));  // (or the division's preparations are made in front of everything, whatever s is)
     return x / s;
 }
 // e / c for the short candidate lists (e < 27)
@@ -168,18 +174,35 @@ __device__ __forceinline__ bool sp_candidate(const int c[3], const SpPart& P, in
 constexpr int kPerThread = 2;
 constexpr int kTicketsAtOnce = kPerThread * kCoordBlock;
 constexpr int kLocalBits = 10, kLocalSlots = 1 << kLocalBits;  // twice the tickets
-struct InsertLds {
+struct alignas(16) InsertLds {
     uint32_t key[kLocalSlots], val[kLocalSlots];
 };
 
+// The same for kernels of 3 and strides of 2 on every axis, where an axis has one or two candidates; c >= 0.
+__device__ __forceinline__ bool sp_candidate_halving(const int c[3], const SpPart& P, int e, int o[3], int& offset) {
+    offset = 0;
+    int m = 1;
+    bool valid = true;
+#pragma unroll
+    for (int a = 2; a >= 0; --a) {
+        const int at = c[a] + P.p[a], two = !(at & 1) && at > 0 ? 1 : 0, second = e & two;
+        e >>= two;
+        o[a] = (at >> 1) - second;
+        valid = valid && (uint32_t)o[a] < (uint32_t)P.os[a];
+        offset += m * ((at & 1) + 2 * second);
+        m *= 3;
+    }
+    return valid && e == 0;
+}
+
 // the tickets of m rows (row, z, y, x) in LDS; the whole block takes part
+template <bool HALVING>
 __device__ __forceinline__ void sp_insert_rows(const SpPart& P, const CellView& t, const int4* rows, int m, InsertLds& L) {
     const int total = m * P.Kc;
     for (int base = 0; base < total; base += kTicketsAtOnce) {
-        for (int i = threadIdx.x; i < kLocalSlots; i += kCoordBlock) {
-            L.key[i] = kEmpty;
-            L.val[i] = kEmpty;
-        }
+        static_assert(kLocalSlots == 4 * kCoordBlock, "a store for each thread");
+        reinterpret_cast<uint4*>(L.key)[threadIdx.x] = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
+        reinterpret_cast<uint4*>(L.val)[threadIdx.x] = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
         __syncthreads();
         uint32_t key[kPerThread], tk[kPerThread];
         int local[kPerThread], offset[kPerThread];
@@ -193,7 +216,13 @@ __device__ __forceinline__ void sp_insert_rows(const SpPart& P, const CellView& 
             offset[j] = 0;
             key[j] = tk[j] = kEmpty;
             if (!live[j]) continue;
-            const int r = P.Kc == 8 ? item >> 3 : item / P.Kc, e = item - r * P.Kc;
+            int r = item >> 3, e = item & 7;
+            if (!HALVING && P.Kc != 8) {
+                int per = P.Kc;
+                asm volatile("" : "+s"(per));
+                r = item / per;
+                e = item - r * per;
+            }
             const int4 row = rows[r];
             const int c[3] = {row.y, row.z, row.w};
             tk[j] = (uint32_t)row.x * (uint32_t)P.Kc + (uint32_t)e;
@@ -202,9 +231,11 @@ __device__ __forceinline__ void sp_insert_rows(const SpPart& P, const CellView& 
             // [0, K) (c = -2, k = 3, s = 2, p = 1: o = 0, offset term -1), with which the reference indexes its
             // rulebook.  Such a row contributes nothing here and raises BAD_COORD; the offset is checked as well, so
             // that nothing a caller passes can make sp_scatter store outside the neighbour table.
-            const bool bad = c[0] < 0 || c[1] < 0 || c[2] < 0;
+            const bool bad = (c[0] | c[1] | c[2]) < 0;
             if (bad && e == 0) atomicOr(&P.meta[2], SESSD_STATUS_BAD_COORD);
-            if (bad || !sp_candidate(c, P, e, o, offset[j]) || offset[j] < 0 || offset[j] >= P.K) continue;
+            if (bad || !(HALVING ? sp_candidate_halving(c, P, e, o, offset[j]) : sp_candidate(c, P, e, o, offset[j])) || offset[j] < 0 ||
+                offset[j] >= P.K)
+                continue;
             key[j] = ((uint32_t)o[0] * (uint32_t)P.os[1] + (uint32_t)o[1]) * (uint32_t)P.os[2] + (uint32_t)o[2];
             uint32_t ls = (key[j] * 2654435769u) >> (32 - kLocalBits);
             for (;;) {  // (at most kTicketsAtOnce keys in twice as many slots: room is always found)
@@ -261,60 +292,99 @@ __device__ __forceinline__ void sp_insert_rows(const SpPart& P, const CellView& 
         if (base + kTicketsAtOnce < total) __syncthreads();
     }
 }
+__device__ __forceinline__ void sp_insert_rows(const SpPart& P, const CellView& t, const int4* rows, int m, InsertLds& L) {
+    if (P.halving) sp_insert_rows<true>(P, t, rows, m, L);
+    else sp_insert_rows<false>(P, t, rows, m, L);
+}
 
 // Points per block of vg_finalize: with a strided layer behind it, a wave of points gives the block's four waves about
 // one round of tickets.
 constexpr int kFinalPoints = 64;
+constexpr int kBlocksAhead = 3;  // counts of 256-point blocks that a thread asks for at once (196 608 points)
 constexpr int kAhead = 4;  // further points of a cell that are requested ahead (the reference averages five)
 
 __global__ void __launch_bounds__(kCoordBlock) vg_finalize(VgPart p, SpPart next, int has_next) {
-    __shared__ uint32_t lds4[4];
+    __shared__ uint32_t lds[8];
     __shared__ int4 s_rows[kFinalPoints];
     __shared__ int s_m;
     __shared__ InsertLds L;
-    const int n = clamp_rows(p.points_size, p.max_points);
-    const int n_blocks = (n + kCoordBlock - 1) / kCoordBlock;  // 256-point blocks that hold points
+    asm volatile("" :: "s"(p.points), "s"(p.points_size), "s"(p.max_points), "s"(p.pf), "s"(p.max_voxels), "s"(p.max_pts), "s"(p.slots), "s"(p.pt_slot),
+                 "s"(p.words), "s"(p.counts), "s"(p.sums), "s"(p.n_blocks), "s"(p.voxels), "s"(p.coors), "s"(p.taken), "s"(next.halving), "s"(next.t.base),
+                 "s"(next.meta));
+    // What the block's points need is requested beside the number of points, which says how much of it counts: their words, cells and
+    // coordinates, the counts of the blocks in front of them and, for any that turns out to be its cell's first, the cell's further
+    // points.
     const int first_point = blockIdx.x * kFinalPoints;
-    if (first_point >= n && blockIdx.x != 0) return;
     const int i = first_point + (int)threadIdx.x;
-    const int mine = first_point / kCoordBlock;
-    const bool point = threadIdx.x < kFinalPoints && i < n;
-    // what does not depend on the prefix is requested beside it
-    const int in_block = (first_point / 64) & 3;
-    uint64_t w[4] = {0, 0, 0, 0};
+    const int mine = first_point / kCoordBlock, in_block = (first_point / 64) & 3;
+    uint64_t w[4];
     int32_t slot = -1;
     float x = 0.f, y = 0.f, z = 0.f, f = 0.f;
-    if (point) {
-        for (int q = 0; q <= in_block; ++q) w[q] = p.words[mine * 4 + q];
+    uint32_t* more = p.slots + (size_t)i * (p.max_pts - 1);
+    uint32_t idx[kAhead];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) idx[q] = kEmpty;
+    for (int q = 0; q < 4; ++q) w[q] = p.words[mine * 4 + q];
+    if (threadIdx.x < kFinalPoints && i < p.max_points) {
         slot = p.pt_slot[i];
         const float* pt = p.points + (size_t)i * p.pf;
         x = pt[0];
         y = pt[1];
         z = pt[2];
         f = pt[3];
+#pragma unroll
+        for (int q = 0; q < kAhead; ++q)
+            if (q < p.max_pts - 1) idx[q] = more[q];
     }
-    // the counts in front of the block's points and of all: each of them, or the sums over 64 and the own 64's
-    const int own = p.sums ? mine / kCountsPerSum : mine, parts = p.sums ? (n_blocks + kCountsPerSum - 1) / kCountsPerSum : n_blocks;
-    const uint32_t* part = p.sums ? p.sums : p.counts;
-    uint32_t before = 0, total = 0;
-    static_assert(kCountsPerSum <= kCoordBlock, "one count a thread");
-    if (p.sums && (int)threadIdx.x < mine - own * kCountsPerSum) before = p.counts[own * kCountsPerSum + (int)threadIdx.x];
-    for (int j = threadIdx.x; j < parts; j += kCoordBlock) {
-        const uint32_t c = part[j];
-        total += c;
-        if (j < own) before += c;
+    uint32_t count[kBlocksAhead];
+    if (!p.sums) {
+#pragma unroll
+        for (int q = 0; q < kBlocksAhead; ++q) {
+            const int b = q * kCoordBlock + (int)threadIdx.x;
+            count[q] = p.counts[b < p.n_blocks ? b : p.n_blocks - 1];
+        }
     }
+    const int n = __builtin_amdgcn_readfirstlane(clamp_rows(p.points_size, p.max_points));
+    const int n_blocks = (n + kCoordBlock - 1) / kCoordBlock;  // 256-point blocks that hold points
+    if (first_point >= n && blockIdx.x != 0) return;
+    const bool point = threadIdx.x < kFinalPoints && i < n;
     uint64_t m = 0;
     for (int q = 0; q < 4; ++q)
-        if (q == in_block) m = w[q];
+        if (q == in_block) m = first_point < n ? w[q] : 0;
     const bool first = point && ((m >> threadIdx.x) & 1ull);
-    // the cell's further points: indices, then (below) the points, while the sums over the blocks are made
-    uint32_t* more = p.slots + (size_t)i * (p.max_pts - 1);
-    uint32_t idx[kAhead];
+    float ahead[kAhead][4];
 #pragma unroll
-    for (int q = 0; q < kAhead; ++q) idx[q] = first && q < p.max_pts - 1 ? more[q] : kEmpty;
-    before = block_sum(before, lds4);
-    total = block_sum(total, lds4);
+    for (int q = 0; q < kAhead; ++q) {
+        if (!first) idx[q] = kEmpty;
+        const float* pt = p.points + (size_t)(idx[q] != kEmpty ? idx[q] : 0) * p.pf;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ahead[q][e] = idx[q] != kEmpty ? pt[e] : 0.f;
+    }
+    // the counts in front of the block's points and of all: each of them, or the sums over 64 and the own 64's
+    uint32_t before = 0, total = 0;
+    static_assert(kCountsPerSum <= kCoordBlock, "one count a thread");
+    if (p.sums) {
+        const int own = mine / kCountsPerSum, parts = (n_blocks + kCountsPerSum - 1) / kCountsPerSum;
+        if ((int)threadIdx.x < mine - own * kCountsPerSum) before = p.counts[own * kCountsPerSum + (int)threadIdx.x];
+        for (int j = threadIdx.x; j < parts; j += kCoordBlock) {
+            const uint32_t c = p.sums[j];
+            total += c;
+            if (j < own) before += c;
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < kBlocksAhead; ++q) {
+            const int b = q * kCoordBlock + (int)threadIdx.x;
+            total += b < n_blocks ? count[q] : 0;
+            before += b < mine && b < n_blocks ? count[q] : 0;
+        }
+        for (int b = kBlocksAhead * kCoordBlock + (int)threadIdx.x; b < n_blocks; b += kCoordBlock) {
+            const uint32_t c = p.counts[b];
+            total += c;
+            if (b < mine) before += c;
+        }
+    }
+    block_sums(before, total, lds);
     const int rows = (int)(total > (uint32_t)p.max_voxels ? (uint32_t)p.max_voxels : total);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         *p.voxel_num = rows;
@@ -326,14 +396,6 @@ __global__ void __launch_bounds__(kCoordBlock) vg_finalize(VgPart p, SpPart next
         if (q < in_block) before += __popcll(w[q]);
     const uint32_t rank = rank_in_wave(m), vid = before + rank;
     const bool kept = first && vid < (uint32_t)p.max_voxels;
-    float ahead[kAhead][4];
-#pragma unroll
-    for (int q = 0; q < kAhead; ++q) {
-        const bool live = kept && idx[q] != kEmpty;
-        const float* pt = p.points + (size_t)(live ? idx[q] : 0) * p.pf;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) ahead[q][e] = live ? pt[e] : 0.f;
-    }
     if (threadIdx.x < 64) {
         const int room = before >= (uint32_t)p.max_voxels ? 0 : (int)((uint32_t)p.max_voxels - before);
         const int here = __popcll(m);
@@ -610,26 +672,40 @@ __global__ void __launch_bounds__(kCoordBlock) flags_lookups(int flag_blocks, in
 // ---------------------------------------------------------------------------------------------
 // numbering, tile cuts
 // ---------------------------------------------------------------------------------------------
-// A block takes the chunks block, block + blocks, ...  What its first chunk needs (words, cand, and with it the cell) is
-// requested before the row count and the sums over the chunks before it are known: the pass is a chain of round trips to
-// memory, and these are three of its seven otherwise.
-__device__ __forceinline__ void sp_number_pass(const SpPart& P, const SpPart& next, bool has_next, int block, int blocks,
-                                               uint32_t* lds4, int4* s_rows, InsertLds& L) {
+// A block takes the chunks block, block + blocks, ...  All that its first chunk needs (words, cand, and the counts of the chunks in
+// front of it) is requested before the row count is known, which says how many of the counts count: the pass is a chain of
+// round trips to memory.  (A block at 45 874 input rows 15 000 -> 8 600 cycles: counts asked for one by one, two sums through LDS
+// permutations, the divisions of a general stride prepared whatever the stride is.  The strided plugin 40.8 -> 36.9 us, frames of
+// 60 000 points (FP16) 246 -> 240, 150 000 476 -> 461.)
+constexpr int kCountsAhead = 8;  // counts that a thread asks for at a time: 2 048 chunks, 65 536 input rows of a 3x3x3 layer
+__device__ __forceinline__ void sp_number_pass(const SpPart& a, const SpPart& next, bool has_next, int block, int blocks,
+                                               uint32_t* lds, int4* s_rows, InsertLds& L) {
+    const SpPart P = a;
+    asm volatile("" :: "s"(P.words), "s"(P.cand), "s"(P.counts), "s"(P.in_num), "s"(P.max_voxels), "s"(P.Kc), "s"(P.t.base), "s"(P.t.dense), "s"(P.n_chunks),
+                 "s"(P.out_coors), "s"(P.taken), "s"(P.nbr), "s"(next.halving), "s"(next.t.base), "s"(next.meta));
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     uint64_t w[4];
-    uint32_t cand = 0;
+    uint32_t cand = 0, count[kCountsAhead];
     auto request = [&](int c) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) w[q] = P.words[c * 4 + q];
         cand = P.cand[(uint32_t)c * kCoordBlock + threadIdx.x];
     };
+    auto request_counts = [&](int from, int end) {
+#pragma unroll
+        for (int q = 0; q < kCountsAhead; ++q) {
+            const uint32_t j = (uint32_t)(from + q * kCoordBlock) + threadIdx.x;
+            count[q] = P.counts[j < (uint32_t)end ? j : (uint32_t)end - 1];
+        }
+    };
     request(block);  // (in bounds: at most n_chunks blocks; not used where the chunk is beyond the active ones)
+    request_counts(0, P.n_chunks);
     // Only the chunks that hold tickets of active input rows carry anything.
-    const int n_in = clamp_rows(P.in_num, P.max_voxels);
+    const int n_in = __builtin_amdgcn_readfirstlane(clamp_rows(P.in_num, P.max_voxels));
     const int active = (int)(((int64_t)n_in * P.Kc + kCoordBlock - 1) / kCoordBlock);
     if (block >= active && block != 0) return;  // (no active input row at all: block 0 still owes the count)
     const CellView t = open_table(P.t, n_in);
-    const int wave = threadIdx.x >> 6;
-    const uint32_t plane = (uint32_t)(P.os[1] * P.os[2]);
+    const uint32_t line = (uint32_t)P.os[2], plane = (uint32_t)P.os[1] * line;
     // the counts in front of the block's chunk: all of them for the first, then those it has stepped over (read anew for
     // every chunk they grew with the square of the rows: the strided plugin at 200 000 rows 146 -> 133 us, at 1 000 000
     // 800 -> 452)
@@ -642,15 +718,20 @@ __device__ __forceinline__ void sp_number_pass(const SpPart& P, const SpPart& ne
         uint32_t key = 0;
         if (first) key = key_at(t, slot);
         uint32_t passed = 0, total = 0;
-        for (int j = from + (int)threadIdx.x; j < to; j += kCoordBlock) {
-            const uint32_t v = P.counts[j];
-            total += v;
-            if (j < c) passed += v;
+        for (int at = from; at < to; at += kCountsAhead * kCoordBlock) {
+            if (c != block || at != 0) request_counts(at, to);
+#pragma unroll
+            for (int q = 0; q < kCountsAhead; ++q) {
+                const int j = at + q * kCoordBlock + (int)threadIdx.x;
+                const uint32_t v = j < to ? count[q] : 0;
+                total += v;
+                passed += j < c ? v : 0;
+            }
         }
         from = c;
         to = c + blocks;
-        before += block_sum(passed, lds4);
-        total = block_sum(total, lds4);
+        block_sums(passed, total, lds);
+        before += passed;
         if (c == block) n_out = (int)(total > (uint32_t)P.max_voxels ? (uint32_t)P.max_voxels : total);
         if (c == 0 && threadIdx.x == 0) {
             *P.out_num = n_out;
@@ -673,12 +754,11 @@ __device__ __forceinline__ void sp_number_pass(const SpPart& P, const SpPart& ne
                 set_value(t, slot, kEmpty);
             } else {
                 set_value(t, slot, id);  // from here on the table maps cell -> output row
-                const int z = key / plane;
-                const int rem = key - z * plane;
-                const int y = rem / P.os[2], x = rem - y * P.os[2];
-                reinterpret_cast<int4*>(P.out_coors)[id] = make_int4(0, z, y, x);  // sparseConv3dlayer.cu:438-441
+                uint32_t rem, x;
+                const uint32_t z = divide(key, plane, P.per_plane, rem), y = divide(rem, line, P.per_line, x);
+                reinterpret_cast<int4*>(P.out_coors)[id] = make_int4(0, (int)z, (int)y, (int)x);  // sparseConv3dlayer.cu:438-441
                 if (P.taken) P.taken[kCellListHead + id] = key;
-                s_rows[rank] = make_int4((int)id, z, y, x);
+                s_rows[rank] = make_int4((int)id, (int)z, (int)y, (int)x);
                 // where sp_scatter fills the table in, the new row's entries start empty: clearing them here, row by
                 // row, touches only the rows that exist
                 if (P.nbr)
@@ -695,17 +775,18 @@ __device__ __forceinline__ void sp_number_pass(const SpPart& P, const SpPart& ne
 }
 
 // rows -> tile boundaries; 256 rows at a time
-__device__ __forceinline__ void cut_pass(const CutPart& P, int block, int32_t* lds) {
-    int32_t* s_wave = lds;
-    const int n = clamp_rows(P.num, P.max_voxels);
+__device__ __forceinline__ void cut_pass(const CutPart& a, int block, uint32_t* lds) {
+    const CutPart P = a;
+    asm volatile("" :: "s"(P.num), "s"(P.max_voxels), "s"(P.w), "s"(P.wsum), "s"(P.hdr), "s"(P.num_cu), "s"(P.target), "s"(P.blocks));
+    const int n = __builtin_amdgcn_readfirstlane(clamp_rows(P.num, P.max_voxels));
     if (n == 0) {
         if (block == 0 && threadIdx.x == 0) P.hdr[0] = 0;  // no cuts
         return;
     }
     const int groups = (n + 63) / 64;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int tiles = tile_plan(n, P.wide ? P.num_cu >> wide_log2_split(n, P.K, P.num_cu) : P.num_cu, P.target).count;
-    uint32_t* lds4 = reinterpret_cast<uint32_t*>(lds) + 4;
+    uint32_t* const s_wave = lds + 8;
     constexpr int kGroups = kCoordBlock / 64;  // sums of a chunk
     uint32_t before = 0, total = 0;  // weight before the chunk and of all rows
     for (int c = block; c * kCoordBlock < n; c += P.blocks) {
@@ -719,32 +800,29 @@ __device__ __forceinline__ void cut_pass(const CutPart& P, int block, int32_t* l
         const int row = c * kCoordBlock + threadIdx.x;
         const int mine = row < n ? P.w[row] : 0;
         const int prev_w = row < n && row > 0 ? P.w[row - 1] : 0;
-        before += block_sum(passed, lds4);
-        if (begin) total = block_sum(all, lds4);
-        // inclusive scan of the chunk's row weights
-        int inc = mine;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int o = __shfl_up(inc, d, 64);
-            if (lane >= d) inc += o;
-        }
+        block_sums(passed, all, lds);
+        before += passed;
+        if (begin) total = all;
+        const uint32_t inc = wave_scan((uint32_t)mine);  // of the chunk's row weights, up to and with this one
         if (lane == 63) s_wave[wave] = inc;
         __syncthreads();
-        int excl = (int)before + inc - mine;  // weight of all rows before this one
+        uint32_t excl = before + inc - (uint32_t)mine;  // weight of all rows before this one
         for (int v = 0; v < wave; ++v) excl += s_wave[v];
         // W is kept above the heaviest possible row: a row then advances the tile id by at most one, so every id
         // up to the last gets its start written (with few rows -- fewer than tiles -- total / tiles would fall
         // below a row's weight, ids would skip, and the skipped entries of the table would be read unwritten)
-        int W = ((int)total + tiles - 1) / tiles;
-        W = W > kGemmMaxOffsets + P.row_weight ? W : kGemmMaxOffsets + P.row_weight + 1;
+        uint32_t W = (total + (uint32_t)tiles - 1) / (uint32_t)tiles;
+        W = W > (uint32_t)(kGemmMaxOffsets + P.row_weight) ? W : (uint32_t)(kGemmMaxOffsets + P.row_weight) + 1;
         if (row < n) {
-            const int id = excl / W;
-            const int prev = row == 0 ? -1 : (excl - prev_w) / W;
+            uint32_t rest;
+            const int id = (int)divide(excl, W, reciprocal(W), rest);
+            // the row before began in the tile before where its weight reaches back beyond this tile's first unit
+            const int prev = row == 0 ? -1 : (rest >= (uint32_t)prev_w ? id : id - 1);
             int32_t* start = P.hdr + 4;
             if (id != prev) start[id] = row;  // ids grow by at most one per row (W exceeds every row weight)
             if (row == n - 1) {
                 start[id + 1] = n;
-                P.hdr[1] = W;
+                P.hdr[1] = (int)W;
                 P.hdr[2] = (int)total;
                 P.hdr[0] = id + 1;
             }
@@ -756,27 +834,27 @@ __device__ __forceinline__ void cut_pass(const CutPart& P, int block, int32_t* l
 template <int N>
 struct NumberCuts {
     SpPart number, next;
-    int number_blocks, has_next;
     CutPart cut[kMaxCuts];
-    int n_cut;
     CleanPart clean;
     FillPlan<N> also;
 };
 
+// end0 .. end3: where the blocks of the cuts end, clean_end: those of the cleaning.
 template <int N>
-__global__ void __launch_bounds__(kCoordBlock) number_cuts(NumberCuts<N> a) {
-    __shared__ uint32_t lds[8];
+__global__ void __launch_bounds__(kCoordBlock) number_cuts(int number_blocks, int has_next, int end0, int end1, int end2, int end3, int clean_end,
+                                                           NumberCuts<N> a) {
+    __shared__ uint32_t lds[12];
     __shared__ int4 s_rows[kCoordBlock];
     __shared__ InsertLds L;
-    int b = blockIdx.x;
-    if (b < a.number_blocks) return sp_number_pass(a.number, a.next, a.has_next != 0, b, a.number_blocks, lds, s_rows, L);
-    b -= a.number_blocks;
-    for (int l = 0; l < a.n_cut; ++l) {
-        if (b < a.cut[l].blocks) return cut_pass(a.cut[l], b, reinterpret_cast<int32_t*>(lds));
-        b -= a.cut[l].blocks;
+    const int b = blockIdx.x;
+    if (b < number_blocks) return sp_number_pass(a.number, a.next, has_next != 0, b, number_blocks, lds, s_rows, L);
+    static_assert(kMaxCuts == 4, "an argument for each");
+    if (b < end3) {
+        const int l = __builtin_amdgcn_readfirstlane((b >= end0 ? 1 : 0) + (b >= end1 ? 1 : 0) + (b >= end2 ? 1 : 0));
+        return cut_pass(a.cut[l], b - (l == 0 ? number_blocks : (l == 1 ? end0 : (l == 2 ? end1 : end2))), lds);
     }
-    if (b < a.clean.blocks) return clean_pass(a.clean, b);
-    fill_pass(a.also, b - a.clean.blocks);
+    if (b < clean_end) return clean_pass(a.clean, b - end3);
+    fill_pass(a.also, b - clean_end);
 }
 
 // rulebook of a strided layer on its own: one store per ticket into the rows sp_number has initialised
@@ -928,33 +1006,38 @@ int launch_number(const SpPart* number, const SpPart* next, const CutPart* cuts,
                   hipStream_t stream) {
     if (n_cuts < 0 || n_cuts > kMaxCuts) return fail(SESSD_E_INVALID, "tile cuts: at most %d in one launch", kMaxCuts);
     NumberCuts<1> a;
-    a.number_blocks = a.has_next = 0;
+    int number_blocks = 0, has_next = 0;
     if (number) {
         a.number = *number;
-        a.number_blocks = sp_pass_blocks(*number);
+        a.number.per_line = reciprocal((uint32_t)number->os[2]);
+        a.number.per_plane = reciprocal((uint32_t)number->os[1] * (uint32_t)number->os[2]);
+        number_blocks = sp_pass_blocks(*number);
         if (next) {
             a.next = *next;
-            a.has_next = 1;
+            has_next = 1;
         }
     }
-    int blocks = a.number_blocks;
-    a.n_cut = n_cuts;
-    for (int l = 0; l < n_cuts; ++l) {
-        a.cut[l] = cuts[l];
-        blocks += a.cut[l].blocks;
+    int blocks = number_blocks, end[kMaxCuts];
+    for (int l = 0; l < kMaxCuts; ++l) {
+        if (l < n_cuts) {
+            a.cut[l] = cuts[l];
+            blocks += a.cut[l].blocks;
+        }
+        end[l] = blocks;
     }
     if (clean) {
         a.clean = *clean;
         a.clean.blocks = clean_blocks(clean->max_voxels);
         blocks += a.clean.blocks;
     }
+    const int clean_end = blocks;
     FillArgs none;
     if (also && also->n > 1) return fail(SESSD_E_INVALID, "numbering: one region can be cleared beside it");
     const int fill_blocks = make_fill_plan(also ? *also : none, a.also);
     if (fill_blocks < 0) return fail(SESSD_E_INVALID, "fill: a region is not 16-byte aligned");
     blocks += fill_blocks;
     if (!blocks) return SESSD_OK;
-    hipLaunchKernelGGL(number_cuts<1>, dim3(blocks), dim3(kCoordBlock), 0, stream, a);
+    hipLaunchKernelGGL(number_cuts<1>, dim3(blocks), dim3(kCoordBlock), 0, stream, number_blocks, has_next, end[0], end[1], end[2], end[3], clean_end, a);
     SESSD_HIP_TRY(hipGetLastError());
     return SESSD_OK;
 }

@@ -231,6 +231,8 @@ SpPart SparseConv3dLayerPlugin::part(const int32_t* coors, const int32_t* voxel_
     P.p[0] = padding0_; P.p[1] = padding1_; P.p[2] = padding2_;
     P.os[0] = out_shape_z_; P.os[1] = out_shape_y_; P.os[2] = out_shape_x_;
     P.Kc = L.Kc;
+    P.halving = L.Kc == 8;
+    for (int x = 0; x < 3; ++x) P.halving = P.halving && P.k[x] == 3 && P.s[x] == 2;
     P.max_voxels = max_voxels_;
     P.K = kernel_volume_;
     P.t = cellTable(workspace);
