@@ -342,6 +342,50 @@ struct Pipeline {
         const bool fork = aux != nullptr && stages.size() > 0;
         hipStream_t side = fork ? aux : stream;
         int last_side = 0;  // last pass that did something on `side`
+        // The feature chain, as far as the passes up to `last_pass` allow.  A wait for the other branch costs the chain 4-5 us in a graph,
+        // however long the pass has been done; behind the second strided layer the branch is far ahead of the chain, and the layers from
+        // there on wait once, for its end (frames of 2 000 points 200 -> 193.5 us, 20 000 301 -> 295, 60 000 (FP16) 240 -> 234).
+        const void* feat = vg_voxels.p;
+        const int32_t* coors = static_cast<const int32_t*>(vg_coors.p);
+        const int32_t* num = static_cast<const int32_t*>(vg_num.p);
+        size_t next_layer = 0;
+        int last_waited = 0;
+        bool scattered = false;
+        constexpr int kOwnWaits = 4;  // passes that are waited for one by one: to the lookups on the second strided layer's rows
+        auto layers = [&](int last_pass) -> int {
+            for (; next_layer < stages.size(); ++next_layer) {
+                ConvStage& st = *stages[next_layer];
+                const int owner = st.rulebook_from >= 0 ? st.rulebook_from : (int)next_layer;
+                const int pass = ready[(size_t)owner];
+                if (pass > last_pass) return SESSD_OK;
+                if (fork && pass > last_waited) {
+                    last_waited = pass > kOwnWaits ? last_side : pass;
+                    SESSD_HIP_TRY(hipStreamWaitEvent(stream, ev_pass[(size_t)last_waited], 0));
+                }
+                DenseTarget dt;
+                const bool fuse = next_layer + 1 == stages.size() && denseByEpilogue();
+                if (fuse) {
+                    const int32_t* oc = st.subm ? coors : static_cast<const int32_t*>(st.coors.p);
+                    dt = s2d->denseTarget(dense, oc, s2d_ws.p);
+                    scattered = true;
+                }
+                if (st.subm) {
+                    SESSD_TRY(st.subm->enqueueGemm(feat, st.feat.p, num, stages[(size_t)owner]->ws.p, stream, fuse ? &dt : nullptr));
+                } else {
+                    SESSD_TRY(st.sparse->enqueueGemm(feat, st.feat.p, static_cast<const int32_t*>(st.num.p), st.ws.p, stream,
+                                                     fuse ? &dt : nullptr));
+                    coors = static_cast<const int32_t*>(st.coors.p);
+                    num = static_cast<const int32_t*>(st.num.p);
+                }
+                feat = st.feat.p;
+            }
+            return SESSD_OK;
+        };
+        // Of the two branches that begin here the one that is launched first follows at once in a graph, the other 6 us later.  That is
+        // the chain, except in FP32 frames of few points, whose layers are short beside the passes until the second strided layer:
+        // 2 000 points 199.2 us with the chain first, 192.6 with the passes, 4 000 213.6 and 212.6, 10 000 253.5 and 252.9, 80 000 444
+        // and 460; FP16 2 000 points 172.9 and 173.7, 10 000 181.6 and 184.1, 60 000 223.1 and 225.2.
+        const bool chain_first = desc.feature_dtype != SESSD_FLOAT || desc.max_points > 4096;
         const int clean_at = m < 1 ? 0 : 1;  // stage 1's own rulebook is the last reader of the voxels' table
         for (int i = 0; i <= m; ++i) {
             const Stage& sg = cs[(size_t)i];
@@ -371,6 +415,7 @@ struct Pipeline {
             if (i == 0 && fork) {
                 SESSD_HIP_TRY(hipEventRecord(ev_head, stream));
                 SESSD_HIP_TRY(hipStreamWaitEvent(side, ev_head, 0));
+                if (chain_first) SESSD_TRY(layers(0));
             } else if (fork) {
                 if (awaited[(size_t)(2 * i)]) SESSD_HIP_TRY(hipEventRecord(ev_pass[(size_t)(2 * i)], side));
                 last_side = 2 * i;
@@ -405,36 +450,7 @@ struct Pipeline {
         }
         if (fork && last_side > 0 && last_side % 2 == 0 && !awaited[(size_t)last_side]) SESSD_HIP_TRY(hipEventRecord(ev_pass[(size_t)last_side], side));
 
-        // the feature chain
-        const void* feat = vg_voxels.p;
-        const int32_t* coors = static_cast<const int32_t*>(vg_coors.p);
-        const int32_t* num = static_cast<const int32_t*>(vg_num.p);
-        int last_waited = 0;
-        bool scattered = false;
-        for (size_t l = 0; l < stages.size(); ++l) {
-            ConvStage& st = *stages[l];
-            const int owner = st.rulebook_from >= 0 ? st.rulebook_from : (int)l;
-            if (fork && ready[(size_t)owner] > last_waited) {
-                last_waited = ready[(size_t)owner];
-                SESSD_HIP_TRY(hipStreamWaitEvent(stream, ev_pass[(size_t)last_waited], 0));
-            }
-            DenseTarget dt;
-            const bool fuse = l + 1 == stages.size() && denseByEpilogue();
-            if (fuse) {
-                const int32_t* oc = st.subm ? coors : static_cast<const int32_t*>(st.coors.p);
-                dt = s2d->denseTarget(dense, oc, s2d_ws.p);
-                scattered = true;
-            }
-            if (st.subm) {
-                SESSD_TRY(st.subm->enqueueGemm(feat, st.feat.p, num, stages[(size_t)owner]->ws.p, stream, fuse ? &dt : nullptr));
-            } else {
-                SESSD_TRY(st.sparse->enqueueGemm(feat, st.feat.p, static_cast<const int32_t*>(st.num.p), st.ws.p, stream,
-                                                 fuse ? &dt : nullptr));
-                coors = static_cast<const int32_t*>(st.coors.p);
-                num = static_cast<const int32_t*>(st.num.p);
-            }
-            feat = st.feat.p;
-        }
+        SESSD_TRY(layers(2 * m + 1));
         if (fork && last_side > last_waited) SESSD_HIP_TRY(hipStreamWaitEvent(stream, ev_pass[(size_t)last_side], 0));  // join
         if (scattered) return SESSD_OK;
         const void* din[3] = {feat, coors, num};
