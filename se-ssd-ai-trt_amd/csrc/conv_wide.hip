@@ -215,10 +215,10 @@ struct Products<S, NB, kThirds> {
 };
 
 // One wave's share of a tile: the pairs of the offsets dealt to it, times its columns -- 16-column blocks nb0 .. nb0 + NB - 1
-// of the layer -- into its partial tile `part` (rows of 16 NB floats).
+// of the layer -- into its partial tile `part` (rows of 16 NB floats).  most: blocks that an offset can have in this tile.
 template <typename S, int COUT, int NB>
 __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_buffer_rsrc_t rs_w, const uint32_t* s_pair,
-                                         const int32_t* s_blk, int K, int wave, int lane, int nb0, float* part) {
+                                         const int32_t* s_blk, int K, int wave, int lane, int nb0, int most, float* part) {
     using P = Products<S, NB, S::kArith>;
     constexpr int kParts = S::kParts, G = S::G, E = S::kLaneBytes / 4, kWaves = S::kWaves, kTileRows = S::kTileRows;
     constexpr int kSets = P::kPieces * NB * E > 64 ? 1 : 2;  // of weights: the registers do not hold two of the largest
@@ -232,12 +232,11 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
     const int blocks_of = lane < K ? s_blk[lane] : 0;
     uint32_t mask;
     {
-        const uint64_t below = (1ull << lane) - 1ull;
         int rank = 0, ahead = 0;
-#pragma unroll
-        for (int size = S::kMaxBlk; size >= 1; --size) {
+        for (int size = most; size >= 1; --size) {
             const uint64_t m = __ballot(blocks_of == size);
-            if (blocks_of == size) rank = ahead + __popcll(m & below);
+            const int before = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, ahead));
+            if (blocks_of == size) rank = before;
             ahead += __popcll(m);
         }
         const int r2 = rank % (2 * kWaves);
@@ -399,10 +398,9 @@ __device__ __forceinline__ void direct_sum(const float* __restrict__ in, const f
 // active ones are written too.  Variants of their own: what they need in registers is missing in the launches without.
 template <int CIN, int COUT, typename T, typename TO, bool DENSE, bool PAD>
 __global__ void __launch_bounds__((Shape<T, CIN, COUT>::kThreads), (Shape<T, CIN, COUT>::kWaves * Shape<T, CIN, COUT>::kPerUnit / 4))
-conv_wide(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict__ Wp, const float* __restrict__ w_f32,
-          const int32_t* __restrict__ nbr, const int32_t* __restrict__ num_out, int max_voxels, int K,
-          const float* __restrict__ scale, const float* __restrict__ shift, int relu, int units,
-          const int32_t* __restrict__ tiles, DenseTarget dt) {
+conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles, const int32_t* __restrict__ nbr,
+          const void* __restrict__ Wp, const T* __restrict__ in, int max_voxels, int K, int units, TO* __restrict__ out,
+          const float* __restrict__ w_f32, const float* __restrict__ scale, const float* __restrict__ shift, int relu, DenseTarget dt) {
     using S = Shape<T, CIN, COUT>;
     constexpr int kWgCols = S::kWgCols, kMaxSplit = S::kMaxSplit, kTileRows = S::kTileRows, kWaves = S::kWaves, kThreads = S::kThreads;
     // (one block more: all of it filling pairs)
@@ -411,22 +409,30 @@ conv_wide(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
     __shared__ float s_epi[3 * COUT];
     __shared__ __align__(16) float s_part[kWaves * kTileRows * kWgCols];
 
+    // The row count, the number of cuts and the cuts of this workgroup's first tile under each split it may be part of are one
+    // trip to memory: without a branch around any of them (no cuts: the row count's word in their place; with branches they and the
+    // arguments that do not fit in registers were six trips, 2 700 cycles).
+    const int32_t* const cuts = tiles ? tiles : num_out;
+    const unsigned has_cuts = tiles ? 1 : 0;
     int n = *num_out;
-    const int cut_count = tiles ? tiles[0] : 0;
+    int cut_count = cuts[0];
     // Workgroups of `units` tiles for each 64 columns of the layer; what follows counts inside one such group.
     int block = blockIdx.x, col0 = 0;
     if constexpr (COUT > kWgCols) {
         col0 = block / units * kWgCols;
         block %= units;
     }
-    // the cuts of this workgroup's first tile under each split it may be part of: requested beside the row count
     int cut_begin[kMaxSplit + 1], cut_end[kMaxSplit + 1], tile_of[kMaxSplit + 1];
 #pragma unroll
     for (int s = 0; s <= kMaxSplit; ++s) {
         tile_of[s] = s && block >= units >> 1 ? block - (units >> 1) : block;
-        cut_begin[s] = tiles ? tiles[4 + tile_of[s]] : 0;
-        cut_end[s] = tiles ? tiles[5 + tile_of[s]] : 0;
+        const unsigned at = tiles ? 4u + (unsigned)tile_of[s] : 0u;
+        cut_begin[s] = cuts[at];
+        cut_end[s] = cuts[at + has_cuts];
     }
+#pragma unroll
+    for (int s = 0; s <= kMaxSplit; ++s) asm volatile("" : "+s"(n), "+s"(cut_count), "+s"(cut_begin[s]), "+s"(cut_end[s]));
+    cut_count = tiles ? cut_count : 0;
     n = n < 0 ? 0 : (n > max_voxels ? max_voxels : n);
     // Column parts: 1 << lsplit workgroups share a tile.  The parts of a tile are row_groups apart in the grid, which
     // puts them on one XCD (workgroups are dealt round robin over eight): they read the same rows.
@@ -435,19 +441,7 @@ conv_wide(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
     const int first_tile = tile_of[kMaxSplit ? lsplit : 0];
     const int first_begin = cut_begin[kMaxSplit ? lsplit : 0], first_end = cut_end[kMaxSplit ? lsplit : 0];
     const int part_id = lsplit && block >= row_groups ? 1 : 0;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (tells the compiler that it is wave-uniform)
-    const int cols = kWgCols >> lsplit, col_first = col0 + part_id * cols;  // columns of this workgroup
-    float epi_scale = 1.f, epi_shift = 0.f, epi_col = 1.f;
-    if (tid < COUT) {
-        if (scale) epi_scale = scale[tid];
-        if (shift) epi_shift = shift[tid];
-        if (S::kArith == kThirds) epi_col = reinterpret_cast<const float*>(static_cast<const char*>(Wp) + (size_t)K * S::kWeightBytes)[tid];
-    }
-    // this thread's epilogue columns (the same for every row it stores): within the part, and of the layer
-    const int lvec = (kWgCols == 64 ? 4 : (kWgCols == 32 ? 3 : 2)) - lsplit;  // log2 of the part's 4-column vectors
-    const int vec = tid & ((1 << lvec) - 1), ec4 = col_first + vec * 4;
+    const int thread = threadIdx.x, own_wave = __builtin_amdgcn_readfirstlane(thread >> 6);  // (tells the compiler that it is wave-uniform)
 
     // The grid is one workgroup per compute unit (a workgroup takes most of a unit's LDS, so workgroups with no
     // tile would queue behind the busy ones just to return); a workgroup walks tiles first_tile, first_tile +
@@ -461,11 +455,6 @@ conv_wide(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
     TilePlan plan = {0, 0};
     if (cut_count == 0) plan = tile_plan(n, walkers, kTileRows);
     const int tile_count = cut_count > 0 ? cut_count : (n > 0 ? plan.count : 0);
-    const __amdgpu_buffer_rsrc_t rs_in = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<T*>(in), 0, (int)((size_t)max_voxels * S::kRowBytes), kRawBuffer);
-    const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<void*>(Wp), 0, (int)((size_t)K * S::kWeightBytes), kRawBuffer);
-
     bool idle = true;  // (no rows)
     for (int tile = first_tile; tile < tile_count; tile += walkers) {
     int run_begin, run_end;
@@ -483,48 +472,81 @@ conv_wide(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
     // ---- stage + compact: a wave turns an offset's neighbour list (two halves of 64 rows) into a pair list ----
     constexpr int kListsPerWave = (kMaxK + kWaves - 1) / kWaves;
     int staged[kListsPerWave][2];
+    auto ask = [&](int h) {
+        uint64_t at = reinterpret_cast<uint64_t>(nbr) + 4 * ((uint64_t)(uint32_t)own_wave * (uint32_t)max_voxels + (uint32_t)(row0 + 64 * h));
 #pragma unroll
-    for (int s = 0; s < kListsPerWave; ++s) {
-        const int k = wave + s * kWaves;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int r = h * 64 + lane;
-            staged[s][h] = (k < K && r < rows) ? nbr[(size_t)k * max_voxels + row0 + r] : -1;
+        for (int s = 0; s < kListsPerWave; ++s) {
+            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+                reinterpret_cast<void*>(at), 0, own_wave + s * kWaves < K ? (rows - 64 * h) * 4 : 0, kRawBuffer);
+            staged[s][h] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, (thread & 63) * 4, 0, 0);
+            at += 4 * (uint64_t)kWaves * (uint32_t)max_voxels;
         }
-    }
-    if (row0 == run_begin && tid < COUT) {
-        s_epi[tid] = epi_scale;
-        s_epi[COUT + tid] = epi_shift;
-        s_epi[2 * COUT + tid] = epi_col;
-    }
+    };
+    const bool tall = kTileRows > 64 && rows > 64;  // (more than one half)
+    ask(0);
+    if (tall) ask(1);
+    // What everything else is computed from is hidden from the compiler until these requests are out: it would compute it in front of
+    // the loops, 200 instructions and the trip to memory of the arguments that are not in registers.  (64 -> 64 at 2 448 rows 10.9 ->
+    // 10.2 us, 8 662 18.8 -> 18.0, 17 262 25.0 -> 24.5; frames of 2 000 points 193.2 -> 187.9, 20 000 279.9 -> 273.8.  One asm for each: an
+    // asm that also has a vector operand makes the scalar ones divergent.)
+    __builtin_amdgcn_sched_barrier(0);
+    int tid = thread, wave = own_wave, volume = K, split = __builtin_amdgcn_readfirstlane(lsplit), part_of = __builtin_amdgcn_readfirstlane(part_id);
+    asm volatile("" : "+v"(tid));
+    asm volatile("" : "+s"(wave));
+    asm volatile("" : "+s"(volume));
+    asm volatile("" : "+s"(split));
+    asm volatile("" : "+s"(part_of));
+    if constexpr (!kMaxSplit) split = part_of = 0;
+    const int lane = tid & 63;
+    const int cols = kWgCols >> split, col_first = col0 + part_of * cols;  // columns of this workgroup
+    // this thread's epilogue columns (the same for every row it stores): within the part, and of the layer
+    const int lvec = (kWgCols == 64 ? 4 : (kWgCols == 32 ? 3 : 2)) - split;  // log2 of the part's 4-column vectors
+    const int vec = tid & ((1 << lvec) - 1), ec4 = col_first + vec * 4;
+    const __amdgpu_buffer_rsrc_t rs_in = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<T*>(in), 0, (int)((size_t)max_voxels * S::kRowBytes), kRawBuffer);
+    const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<void*>(Wp), 0, (int)((size_t)volume * S::kWeightBytes), kRawBuffer);
     idle = false;
     if (tid < 16) s_pair[kMaxK * kTileRows + tid] = kNoPair;
     // zero this wave's partial tile (while the lists are on their way)
     float* part = s_part + wave * kTileRows * cols;
     for (int t = lane; t < rows << lvec; t += 64) reinterpret_cast<float4*>(part)[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+    float epi_scale = 1.f, epi_shift = 0.f, epi_col = 1.f;
+    if (row0 == run_begin && tid < COUT) {
+        if (scale) epi_scale = scale[tid];
+        if (shift) epi_shift = shift[tid];
+        if (S::kArith == kThirds) epi_col = reinterpret_cast<const float*>(static_cast<const char*>(Wp) + (size_t)volume * S::kWeightBytes)[tid];
+    }
+    auto compact = [&](auto halves) {
 #pragma unroll
-    for (int s = 0; s < kListsPerWave; ++s) {
-        const int k = wave + s * kWaves;
-        if (k >= K) break;
-        int base = 0;
+        for (int s = 0; s < kListsPerWave; ++s) {
+            const int k = wave + s * kWaves;
+            if (k >= volume) break;
+            int base = 0;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int v = staged[s][h];
-            const uint64_t m = __ballot(v >= 0);
-            if (v >= 0) {
-                const int j = base + __popcll(m & ((1ull << lane) - 1ull));
-                s_pair[k * kTileRows + j] = ((uint32_t)v << S::kRowBits) | (uint32_t)(h * 64 + lane);
+            for (int h = 0; h < decltype(halves)::value; ++h) {
+                const int v = h * 64 + lane < rows ? staged[s][h] : -1;
+                const uint64_t m = __ballot(v >= 0);
+                const int j = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, base));
+                if (v >= 0) s_pair[k * kTileRows + j] = ((uint32_t)v << S::kRowBits) | (uint32_t)(h * 64 + lane);
+                base += __popcll(m);
             }
-            base += __popcll(m);
+            const int blocks = (base + 15) >> 4;
+            if (base + lane < blocks * 16) s_pair[k * kTileRows + base + lane] = kNoPair;
+            if (lane == 0) s_blk[k] = blocks;
         }
-        const int blocks = (base + 15) >> 4;
-        if (base + lane < blocks * 16) s_pair[k * kTileRows + base + lane] = kNoPair;
-        if (lane == 0) s_blk[k] = blocks;
+    };
+    if (tall) compact(std::integral_constant<int, 2>{});
+    else compact(std::integral_constant<int, 1>{});
+    if (row0 == run_begin && tid < COUT) {
+        s_epi[tid] = epi_scale;
+        s_epi[COUT + tid] = epi_shift;
+        s_epi[2 * COUT + tid] = epi_col;
     }
     __syncthreads();
     if constexpr (kMaxSplit)
-        if (lsplit) multiply<S, COUT, kWgCols / 32>(rs_in, rs_w, s_pair, s_blk, K, wave, lane, col_first / 16, part);
-    if (!kMaxSplit || !lsplit) multiply<S, COUT, kWgCols / 16>(rs_in, rs_w, s_pair, s_blk, K, wave, lane, col_first / 16, part);
+        if (split) multiply<S, COUT, kWgCols / 32>(rs_in, rs_w, s_pair, s_blk, volume, wave, lane, col_first / 16, (rows + 15) >> 4, part);
+    if (!kMaxSplit || !split) multiply<S, COUT, kWgCols / 16>(rs_in, rs_w, s_pair, s_blk, volume, wave, lane, col_first / 16, (rows + 15) >> 4, part);
     __syncthreads();
 
     // fixed-order sum of the waves' partial tiles, epilogue, coalesced stores; the sums of kAtOnce vectors are read together
@@ -611,7 +633,7 @@ conv_wide(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
                 const float4 sum = sums_of(r);
                 float o[4] = {sum.x, sum.y, sum.z, sum.w};
                 if (finite(o)) continue;
-                direct_sum<CIN, COUT>(in, w_f32, nbr + row0 + r, max_voxels, K, ec4, o);
+                direct_sum<CIN, COUT>(in, w_f32, nbr + row0 + r, max_voxels, volume, ec4, o);
                 put(r, o);
             }
     }
@@ -619,9 +641,9 @@ conv_wide(const T* __restrict__ in, TO* __restrict__ out, const void* __restrict
     }
     }
     if constexpr (PAD) {
-        if (idle && tid < COUT) {  // (no tile has staged them)
-            s_epi[tid] = epi_scale;
-            s_epi[COUT + tid] = epi_shift;
+        if (idle && thread < COUT) {  // (no tile has staged them)
+            s_epi[thread] = scale ? scale[thread] : 1.f;
+            s_epi[COUT + thread] = shift ? shift[thread] : 0.f;
         }
         __syncthreads();
         write_pad_rows<TO, COUT, kThreads>(out, n, max_voxels, s_epi, scale != nullptr, shift != nullptr, relu);
@@ -637,8 +659,8 @@ int launch(const GemmArgs& a, hipStream_t stream) {
     const int units = gemm_compute_units() * S::kPerUnit / S::kColGroups;
     auto go = [&](auto dense, auto pad) {
         hipLaunchKernelGGL((conv_wide<CIN, COUT, T, TO, decltype(dense)::value, decltype(pad)::value>), dim3((unsigned)(units * S::kColGroups)),
-                           dim3(S::kThreads), 0, stream, static_cast<const T*>(a.in_feat), static_cast<TO*>(a.out_feat), a.w_packed,
-                           a.w_f32, a.nbr, a.num_out, a.max_voxels, a.K, a.scale, a.shift, a.relu, units, a.tiles, a.dense);
+                           dim3(S::kThreads), 0, stream, a.num_out, a.tiles, a.nbr, a.w_packed, static_cast<const T*>(a.in_feat),
+                           a.max_voxels, a.K, units, static_cast<TO*>(a.out_feat), a.w_f32, a.scale, a.shift, a.relu, a.dense);
     };
     if (a.dense.dense) a.write_pad_rows ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
     else a.write_pad_rows ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
