@@ -102,7 +102,7 @@ bool ConvPluginBase::gemmOnMatrixCores() const {
            gemm_wide_takes_rows(max_voxels_, in_channel_, out_channel_, in_type_);
 }
 
-int ConvPluginBase::tileRows() const { return gemm_wide_tile_rows(out_channel_, out_type_); }
+int ConvPluginBase::tileRows() const { return gemm_wide_tile_rows(in_channel_, out_channel_, out_type_); }
 int ConvPluginBase::tilesWide() const {
     return gemm_runs_wide(kernel_volume_, in_channel_, out_channel_, in_type_, out_type_) ? (out_channel_ > 64 ? out_channel_ / 64 : 1) : 0;
 }

@@ -29,10 +29,15 @@
 //     weights are requested with the first block of an offset into a second set of registers, or, where these do not hold two
 //     sets (64 x 64), behind the MFMAs of its last into the only one;
 //   * a wave's blocks and offsets are listed once, a lane each, and read with readlane: the loop has no other bookkeeping.
-// Up to 16 (32) columns a tile is at most 112 (64) rows and a unit holds two workgroups, both used only where one tile for each
-// unit would be higher than that (32 -> 32, eight waves, 4 208 rows: one workgroup a unit 7.9 us, two 10.7).  What LDS they leave is what the
+// Up to 32 columns two to four workgroups share a unit, as many as the rows need: only where one tile for each unit would be higher than a
+// tile can be does a second one begin (32 -> 32, eight waves, 4 208 rows: one workgroup a unit 7.9 us, two 10.7).  Beyond what they hold
+// together a launch is two rounds of tiles, of which the second costs its lists and sums again; the tiles are therefore as high, or the
+// workgroups as many, as the LDS takes: 16 columns 2 x 128 rows (60 000 rows, 4 -> 16 12.7 -> 10.3 us, 16 -> 16 15.2 -> 12.4 against 2 x 112),
+// 4 -> 32 4 x 64 (54 613 rows 16.2 -> 12.7 against 2 x 64), 32 -> 32 3 x 80 (40 088 rows 26.1 -> 21.5, 60 727 33.3 -> 28.4 against 2 x 64; frames of
+// 40 000 points 363 -> 351, of 80 000, whose coordinate passes miss the LDS, 428 -> 431).  What LDS they leave is what the
 // coordinate passes of a frame's other branch run in: 32 -> 32 with eight waves is the faster launch (15.9 us against 17.1 at
-// 28 043 rows) and makes the slower frame (20 000 points: 283 us against 274); 4 -> 32 likewise (487 against 475).
+// 28 043 rows) and makes the slower frame (20 000 points: 283 us against 274); 4 -> 32 likewise (487 against 475).  16 -> 32 with four waves and
+// 3 x 80 rows: 54 613 rows 18.4 -> 17.4 us, but 17 132 rows 9.0 -> 11.4.
 // FP16 features (Cin 16) have so little in each block that four waves and 64 rows do: four workgroups share a unit, with 40 KB of LDS
 // each.  From 32 channels up FP16 is faster without pair lists (32 -> 32 at 45 874 rows 10.6 us on conv_tall.hip, 18 here).
 #include <algorithm>
@@ -77,8 +82,9 @@ struct Shape {
     // (32 columns: four waves with 4 and 32 channels, whose launches are long enough for the frame's other branch to need the LDS)
     static constexpr int kWaves = kWgCols == 64 ? 6 : (sizeof(T) == 2 || (COUT == 32 && CIN != 16) ? 4 : 8);
     static constexpr int kThreads = kWaves * 64;
-    static constexpr int kTileRows = kWgCols == 64 ? 96 : (sizeof(T) == 2 || kWgCols == 32 ? 64 : 112);  // tile capacity
-    static constexpr int kPerUnit = kWgCols == 64 ? 1 : (sizeof(T) == 2 ? 4 : 2);  // workgroups that can share a compute unit
+    // rows of a tile at most, and workgroups that can share a compute unit
+    static constexpr int kTileRows = kWgCols == 64 ? 96 : (sizeof(T) == 2 ? 64 : (kWgCols == 16 ? 128 : (CIN == 32 ? 80 : 64)));
+    static constexpr int kPerUnit = kWgCols == 64 ? 1 : (sizeof(T) == 2 || (CIN == 4 && COUT == 32) ? 4 : (CIN == 32 ? 3 : 2));
     static constexpr int kMaxBlk = kTileRows / 16;
     static constexpr int kRowBits = pair_row_bits(kTileRows);
     static constexpr int kNone = kMaxK * kTileRows * 4;  // an item with no pairs
@@ -682,13 +688,15 @@ bool gemm_runs_wide(int K, int cin, int cout, int in_type, int out_type) {
 
 // (a kernel that has a shape to itself takes more; the pipeline asks before it relies on the fused scatter)
 bool gemm_wide_takes_rows(int max_voxels, int cin, int cout, int in_type) {
-    return (uint32_t)max_voxels <= kNoPair >> pair_row_bits(gemm_wide_tile_rows(cout, in_type)) &&
+    return (uint32_t)max_voxels <= kNoPair >> pair_row_bits(gemm_wide_tile_rows(cin, cout, in_type)) &&
            (size_t)max_voxels * cin * (in_type == SESSD_HALF ? 2 : 4) < kOutOfRange;
 }
 
-int gemm_wide_tile_rows(int cout, int type) {
+int gemm_wide_tile_rows(int cin, int cout, int type) {
     if (cout >= 64) return Shape<float, 64, 64>::kTileRows;
-    return type == SESSD_HALF || cout >= 32 ? Shape<float, 32, 32>::kTileRows : Shape<float, 16, 16>::kTileRows;
+    if (type == SESSD_HALF) return Shape<__half, 16, 16>::kTileRows;
+    if (cout == 16) return Shape<float, 16, 16>::kTileRows;
+    return cin == 32 ? Shape<float, 32, 32>::kTileRows : Shape<float, 16, 32>::kTileRows;
 }
 
 bool wide_splits(int cin) { return arith(cin) != kPlain; }

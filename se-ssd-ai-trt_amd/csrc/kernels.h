@@ -79,7 +79,7 @@ bool gemm_cuts_own_tiles(int K, int cin, int cout, int in_type, int out_type);
 // whether the layer runs on conv_wide.hip's kernel (where the two above leave it), that kernel's tile capacity, how many rows it
 // takes, and whether it multiplies 16-bit parts of FP32 operands, which need weights of a form of their own
 bool gemm_runs_wide(int K, int cin, int cout, int in_type, int out_type);
-int gemm_wide_tile_rows(int cout, int type);
+int gemm_wide_tile_rows(int cin, int cout, int type);
 bool gemm_wide_takes_rows(int max_voxels, int cin, int cout, int in_type);
 bool wide_splits(int cin);
 size_t wide_weight_bytes(int K, int cin, int cout);
