@@ -76,8 +76,8 @@ __device__ __forceinline__ float4* weight_slot() {
 template <int CIN, int COUT, int RB>
 __device__ __forceinline__ void tall_tile(const __half* __restrict__ in, __half* __restrict__ out,
                                           const void* __restrict__ Wp, const int32_t* __restrict__ nbr, int n,
-                                          int row0, int max_voxels, bool has_scale, bool has_shift, int relu,
-                                          DenseTarget dt, int32_t* s_nbr, const float* s_epi) {
+                                          int row0, int max_voxels, const float* __restrict__ scale, const float* __restrict__ shift,
+                                          int relu, DenseTarget dt, int32_t* s_nbr, float* s_epi) {
     constexpr int G = CIN / 32;        // K-chunks (32 channels) of the inner dimension
     constexpr int NBT = COUT / 16;     // 16-column blocks
     constexpr int U = G * NBT;         // 1 KB units (64 lanes x 16 bytes) of one offset's weights
@@ -89,12 +89,37 @@ __device__ __forceinline__ void tall_tile(const __half* __restrict__ in, __half*
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (row0 >= n) return;
 
-    // the tile's neighbour lists (rows beyond n: none) -> LDS
-    for (int e = tid; e < KC * TR; e += kWaves * 64) {
-        const int k = e / TR, r = e - k * TR;
-        s_nbr[e] = row0 + r < n ? nbr[(size_t)k * max_voxels + row0 + r] : -1;
+    // The tile's neighbour lists (rows beyond n: none) -> LDS.  A wave takes 64 rows of one offset at a time, all of them requested before
+    // the first is stored.  (In a loop over the entries each was a trip to memory of its own, behind those for scale, shift and the row
+    // count: 32 -> 32 at 4 208 rows 5.9 -> 5.4 us, 45 874 10.5 -> 9.9, 72 487 16.1 -> 14.8; 32 -> 64 at 45 874 12.3 -> 11.8.)
+    constexpr int kRuns = TR / 64, kLists = (KC * kRuns + kWaves - 1) / kWaves;  // runs of 64 rows an offset, runs a wave
+    static_assert(kWaves % kRuns == 0, "a wave's runs are all of the same rows");
+    const int run = wave % kRuns, here = n - row0 - run * 64;  // (rows of the run; may be none)
+    int32_t list[kLists];
+    {
+        uint64_t at = reinterpret_cast<uint64_t>(nbr) + 4 * ((uint64_t)(uint32_t)(wave / kRuns) * (uint32_t)max_voxels + (uint32_t)(row0 + run * 64));
+#pragma unroll
+        for (int t = 0; t < kLists; ++t) {
+            const int k = wave / kRuns + t * (kWaves / kRuns);
+            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(at), 0, k < KC && here > 0 ? here * 4 : 0, kRawBuffer);
+            list[t] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, lane * 4, 0, 0);
+            at += 4 * (uint64_t)(kWaves / kRuns) * (uint32_t)max_voxels;
+        }
+    }
+    if (tid < COUT) {
+        float by = 1.f, plus = 0.f;
+        if (scale) by = scale[tid];
+        if (shift) plus = shift[tid];
+        s_epi[tid] = by;
+        s_epi[COUT + tid] = plus;
+    }
+#pragma unroll
+    for (int t = 0; t < kLists; ++t) {
+        const int k = wave / kRuns + t * (kWaves / kRuns);
+        if (k < KC) s_nbr[k * TR + run * 64 + lane] = lane < here ? list[t] : -1;
     }
     __syncthreads();
+    const bool has_scale = scale != nullptr, has_shift = shift != nullptr;
 
     const int i = lane & 15;  // row inside a 16-row block
     const int q = lane >> 4;  // 8-channel group inside a K-chunk
@@ -269,22 +294,17 @@ __device__ __forceinline__ void tall_tile(const __half* __restrict__ in, __half*
 
 template <int CIN, int COUT>
 __global__ void __launch_bounds__(kWaves * 64, 2)
-conv_tall(const __half* __restrict__ in, __half* __restrict__ out, const void* __restrict__ Wp,
-          const int32_t* __restrict__ nbr, const int32_t* __restrict__ num_out, int max_voxels,
-          const float* __restrict__ scale, const float* __restrict__ shift, int relu, int write_pad,
-          int slots, DenseTarget dt) {
+conv_tall(const int32_t* __restrict__ num_out, const int32_t* __restrict__ nbr, const __half* __restrict__ in,
+          const void* __restrict__ Wp, int max_voxels, int slots, int relu, int write_pad, __half* __restrict__ out,
+          const float* __restrict__ scale, const float* __restrict__ shift, DenseTarget dt) {
     static_assert(CIN % 32 == 0 && COUT % 16 == 0, "whole MFMA chunks");
     constexpr int RB = kTallBlocks;
     __shared__ int32_t s_nbr[KC * kWaves * RB * 16];
     __shared__ float s_epi[2 * COUT];
+    // (the lists wait for nothing else: the arguments in front of `out` are in registers)
     int n = *num_out;
+    asm volatile("" : "+s"(n));
     n = n < 0 ? 0 : (n > max_voxels ? max_voxels : n);
-    const int tid = threadIdx.x;
-
-    if (tid < COUT) {  // (published by the barrier behind the list staging)
-        s_epi[tid] = scale ? scale[tid] : 1.f;
-        s_epi[COUT + tid] = shift ? shift[tid] : 0.f;
-    }
     // Tile heights.  `slots` workgroups are resident at a time.  Up to 64 * slots rows every
     // tile is 64 rows (one block per wave); beyond that just enough tiles at the head of the grid take RB blocks
     // per wave for the launch to stay one round of resident workgroups -- a second, mostly empty round costs a
@@ -297,10 +317,14 @@ conv_tall(const __half* __restrict__ in, __half* __restrict__ out, const void* _
     }
     const int b = blockIdx.x;
     if (b < n_tall)
-        tall_tile<CIN, COUT, RB>(in, out, Wp, nbr, n, b * kTall, max_voxels, scale != nullptr, shift != nullptr, relu, dt, s_nbr, s_epi);
+        tall_tile<CIN, COUT, RB>(in, out, Wp, nbr, n, b * kTall, max_voxels, scale, shift, relu, dt, s_nbr, s_epi);
     else
-        tall_tile<CIN, COUT, 1>(in, out, Wp, nbr, n, n_tall * kTall + (b - n_tall) * kShort, max_voxels, scale != nullptr, shift != nullptr, relu, dt, s_nbr, s_epi);
+        tall_tile<CIN, COUT, 1>(in, out, Wp, nbr, n, n_tall * kTall + (b - n_tall) * kShort, max_voxels, scale, shift, relu, dt, s_nbr, s_epi);
     if (write_pad) {
+        if (threadIdx.x < COUT) {  // (a workgroup may have had no tile)
+            s_epi[threadIdx.x] = scale ? scale[threadIdx.x] : 1.f;
+            s_epi[COUT + threadIdx.x] = shift ? shift[threadIdx.x] : 0.f;
+        }
         __syncthreads();
         write_pad_rows<__half, COUT, kWaves * 64>(out, n, max_voxels, s_epi, scale != nullptr, shift != nullptr, relu);
     }
@@ -320,9 +344,8 @@ int launch(const GemmArgs& a, hipStream_t stream) {
         per_cu = v;
     }
     hipLaunchKernelGGL((conv_tall<CIN, COUT>), dim3(blocks), dim3(kWaves * 64), 0, stream,
-                       static_cast<const __half*>(a.in_feat), static_cast<__half*>(a.out_feat), a.w_packed, a.nbr,
-                       a.num_out, a.max_voxels, a.scale, a.shift, a.relu, a.write_pad_rows,
-                       per_cu * num_cu, a.dense);
+                       a.num_out, a.nbr, static_cast<const __half*>(a.in_feat), a.w_packed, a.max_voxels, per_cu * num_cu, a.relu,
+                       a.write_pad_rows, static_cast<__half*>(a.out_feat), a.scale, a.shift, a.dense);
     SESSD_HIP_TRY(hipGetLastError());
     return SESSD_OK;
 }
