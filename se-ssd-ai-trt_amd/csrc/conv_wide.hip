@@ -21,13 +21,18 @@
 // Distance from the sums in 64 bits, 2-norm, FP32 instruction and parts: 64 -> 64 1.27e-7, 0.72e-7; 128 -> 128 1.31e-7, 0.81e-7; 32 -> 32
 // 0.93e-7, 0.67e-7.
 //
-// What bounds it: a block of 64 -> 64 is 768 cycles of MFMA (with half of them left out the launch above takes 20.0 us), the rest a wave's
+// What bounds it: a block of 64 -> 64 is 768 cycles of MFMA (with half of them left out the launch above took 20.0 us of 24.9), the rest a wave's
 // instructions and LDS.  Hence
 //   * a wave takes all 64 columns: rows are requested, permuted and split once;
-//   * six waves: as many partial tiles of 96 rows as LDS holds;
+//   * as many waves as LDS holds partial tiles of: eight up to 72 rows and where two workgroups share the columns, seven up to 82, six up
+//     to the 96 that a tile of all columns can have (with six on four SIMDs, two of these work alone and slower.  64 -> 64 at 11 252 rows
+//     19.6 -> 18.8 us, 14 629 22.9 -> 21.9; 128 -> 128 at 14 629 69.7 -> 66.1; frames of 20 000 points 271 -> 266; up to 4 200 rows the
+//     call with its pad rows 13.9 -> 14.2, frames of 2 000 points the same).  Longer runs are walked in two halves rather than in 96
+//     rows and the rest (64 -> 64 at 21 591 rows 38.6 -> 34.4);
 //   * the rows of the block after next are requested, and the next block's split, under a block's MFMAs; the next offset's
 //     weights are requested with the first block of an offset into a second set of registers, or, where these do not hold two
-//     sets (64 x 64), behind the MFMAs of its last into the only one;
+//     sets (64 x 64), in its last block into the only one, each 16 columns as soon as the block's products with them are made (behind all
+//     products: part of the figures above; by itself 0.5-1 %);
 //   * a wave's blocks and offsets are listed once, a lane each, and read with readlane: the loop has no other bookkeeping.
 // Up to 32 columns two to four workgroups share a unit, as many as the rows need: only where one tile for each unit would be higher than a
 // tile can be does a second one begin (32 -> 32, eight waves, 4 208 rows: one workgroup a unit 7.9 us, two 10.7).  Beyond what they hold
@@ -80,16 +85,20 @@ struct Shape {
     static constexpr int kWgCols = COUT < 64 ? COUT : 64;  // columns of a workgroup (before the split of short tiles)
     static constexpr int kColGroups = COUT / kWgCols;      // workgroups beside each other
     // (32 columns: four waves with 4 and 32 channels, whose launches are long enough for the frame's other branch to need the LDS)
-    static constexpr int kWaves = kWgCols == 64 ? 6 : (sizeof(T) == 2 || (COUT == 32 && CIN != 16) ? 4 : 8);
+    static constexpr int kWaves = kWgCols == 64 ? 8 : (sizeof(T) == 2 || (COUT == 32 && CIN != 16) ? 4 : 8);
     static constexpr int kThreads = kWaves * 64;
-    // rows of a tile at most, and workgroups that can share a compute unit
-    static constexpr int kTileRows = kWgCols == 64 ? 96 : (sizeof(T) == 2 ? 64 : (kWgCols == 16 ? 128 : (CIN == 32 ? 80 : 64)));
+    static constexpr int kParts = CIN > 64 ? CIN / 64 : 1;  // of the inner dimension, taken one after the other
+    static constexpr int CP = CIN / kParts;                 // channels of a part
+    // Rows of a tile at most, and workgroups that can share a compute unit.  64 columns: as many waves multiply as the LDS holds partial
+    // tiles of the tile's rows, eight up to 72 rows and kFewestWaves with kWholeRows; with half of the columns always all.
+    static constexpr int kTileRows = kWgCols == 64 ? (kParts > 1 ? 112 : 128) : (sizeof(T) == 2 ? 64 : (kWgCols == 16 ? 128 : (CIN == 32 ? 80 : 64)));
+    static constexpr int kWholeRows = kWgCols == 64 ? 96 : kTileRows;
+    static constexpr int kFewestWaves = kWgCols == 64 ? 6 : kWaves;
+    static constexpr int kPartRows = kFewestWaves * kWholeRows;  // of all partial tiles together
     static constexpr int kPerUnit = kWgCols == 64 ? 1 : (sizeof(T) == 2 || (CIN == 4 && COUT == 32) ? 4 : (CIN == 32 ? 3 : 2));
     static constexpr int kMaxBlk = kTileRows / 16;
     static constexpr int kRowBits = pair_row_bits(kTileRows);
     static constexpr int kNone = kMaxK * kTileRows * 4;  // an item with no pairs
-    static constexpr int kParts = CIN > 64 ? CIN / 64 : 1;  // of the inner dimension, taken one after the other
-    static constexpr int CP = CIN / kParts;                 // channels of a part
     static constexpr int kRowBytes = CIN * (int)sizeof(T), kPartBytes = CP * (int)sizeof(T);
     static constexpr int kLaneBytes = kPartBytes < 64 ? kPartBytes / 4 : 16;  // of a row that a lane requests at a time; of a weight operand as well
     static constexpr int G = kPartBytes / (4 * kLaneBytes);  // requests for a part
@@ -97,7 +106,9 @@ struct Shape {
     static_assert(kTileRows <= 128 && kTileRows % 16 == 0, "the lists are staged in two halves of 64 rows");
     static_assert((CP == 4 || CP % 16 == 0) && (kArith == kPlain || kArith == kFp16 || CP % 32 == 0) && COUT % kWgCols == 0, "whole MFMA steps and column groups");
     static_assert(kTileRows <= 1 << kRowBits, "a pair holds its row in the tile");
-    static_assert((kMaxK + kWaves - 1) / kWaves * kMaxBlk * kParts + 2 <= 64, "an item a lane");
+    static_assert((kMaxK + kWaves - 1) / kWaves * kMaxBlk * kParts + 2 <= 64 &&
+                  (kMaxK + kFewestWaves - 1) / kFewestWaves * (kWholeRows / 16) * kParts + 2 <= 64, "an item a lane");
+    static_assert(kMaxSplit == 0 || kWaves * kTileRows <= 2 * kPartRows, "partial tiles of half of the columns");
 };
 
 __device__ __forceinline__ void buffer_load(__amdgpu_buffer_rsrc_t r, unsigned byte_offset, int (&v)[4]) {
@@ -207,26 +218,36 @@ struct Products<S, NB, kThirds> {
             }
         p[kWords - 1] |= left & 0xffffu ? 0x7fff : 0;  // (the last word: what waits for all of them is last)
     }
-    static __device__ __forceinline__ void multiply(const int (&w)[3 * C][NB][E], const int (&x)[kWords], v4f (&acc)[NB]) {
+    static __device__ __forceinline__ void step(const int (&w)[3 * C][NB][E], const int (&x)[kWords], v4f (&acc)[NB], int t, int c, int nb) {
         constexpr int kPart[6][2] = {{0, 2}, {1, 1}, {2, 0}, {0, 1}, {1, 0}, {0, 0}};  // of w, of x
+        acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(operand8<v8b>(w[kPart[t][0] * C + c][nb]),
+                                                          operand8<v8b>(x + 2 * G * kPart[t][1] + 4 * c), acc[nb], 0, 0, 0);
+    }
+    static __device__ __forceinline__ void multiply(const int (&w)[3 * C][NB][E], const int (&x)[kWords], v4f (&acc)[NB]) {
 #pragma unroll
         for (int t = 0; t < 6; ++t)
 #pragma unroll
             for (int c = 0; c < C; ++c)
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
-                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(operand8<v8b>(w[kPart[t][0] * C + c][nb]),
-                                                                      operand8<v8b>(x + 2 * G * kPart[t][1] + 4 * c), acc[nb], 0, 0, 0);
+                for (int nb = 0; nb < NB; ++nb) step(w, x, acc, t, c, nb);
+    }
+    // one column block; its weights are free behind it
+    static __device__ __forceinline__ void multiply_block(const int (&w)[3 * C][NB][E], const int (&x)[kWords], v4f (&acc)[NB], int nb) {
+#pragma unroll
+        for (int t = 0; t < 6; ++t)
+#pragma unroll
+            for (int c = 0; c < C; ++c) step(w, x, acc, t, c, nb);
     }
 };
 
 // One wave's share of a tile: the pairs of the offsets dealt to it, times its columns -- 16-column blocks nb0 .. nb0 + NB - 1
-// of the layer -- into its partial tile `part` (rows of 16 NB floats).  most: blocks that an offset can have in this tile.
+// of the layer -- into its partial tile `part` (rows of 16 NB floats).  waves: among which the offsets are dealt; most: blocks that an
+// offset can have in this tile.
 template <typename S, int COUT, int NB>
 __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_buffer_rsrc_t rs_w, const uint32_t* s_pair,
-                                         const int32_t* s_blk, int K, int wave, int lane, int nb0, int most, float* part) {
+                                         const int32_t* s_blk, int K, int wave, int waves, int lane, int nb0, int most, float* part) {
     using P = Products<S, NB, S::kArith>;
-    constexpr int kParts = S::kParts, G = S::G, E = S::kLaneBytes / 4, kWaves = S::kWaves, kTileRows = S::kTileRows;
+    constexpr int kParts = S::kParts, G = S::G, E = S::kLaneBytes / 4, kTileRows = S::kTileRows;
     constexpr int kSets = P::kPieces * NB * E > 64 ? 1 : 2;  // of weights: the registers do not hold two of the largest
     constexpr int NBT = COUT / 16;                   // 16-column blocks of the layer
     constexpr int kSlots = NB * 4;                   // 16-byte slots of a row of the partial tile
@@ -245,8 +266,15 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
             if (blocks_of == size) rank = before;
             ahead += __popcll(m);
         }
-        const int r2 = rank % (2 * kWaves);
-        const int w = r2 < kWaves ? r2 : 2 * kWaves - 1 - r2;
+        int r2 = rank;
+        if constexpr (S::kFewestWaves == S::kWaves) {
+            r2 = rank % (2 * waves);
+        } else {  // (without a division: fewer than three rounds)
+            static_assert(kMaxK <= 6 * S::kFewestWaves, "rounds");
+            r2 -= r2 >= 4 * waves ? 4 * waves : 0;
+            r2 -= r2 >= 2 * waves ? 2 * waves : 0;
+        }
+        const int w = r2 < waves ? r2 : 2 * waves - 1 - r2;
         mask = (uint32_t)__ballot(blocks_of > 0 && w == wave);
     }
     if (!mask) return;
@@ -283,8 +311,15 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
 #pragma unroll
         for (int g = 0; g < G; ++g) buffer_load(rs_in, at + g * 64u, a[g]);
     };
-    auto load_b = [&](int stage, int (&b)[P::kPieces][NB][E]) {  // (stage < 0: nothing to fetch)
-        const unsigned at = stage >= 0 ? (unsigned)(((stage * P::kPieces * NBT + nb0) * 64 + lane) * S::kLaneBytes) : kOutOfRange;
+    auto stage_weights = [&](int stage) -> unsigned {  // (stage < 0: nothing to fetch)
+        return stage >= 0 ? (unsigned)(((stage * P::kPieces * NBT + nb0) * 64 + lane) * S::kLaneBytes) : kOutOfRange;
+    };
+    auto load_b1 = [&](unsigned at, int (&b)[P::kPieces][NB][E], int nb) {
+#pragma unroll
+        for (int c = 0; c < P::kPieces; ++c) buffer_load(rs_w, at + (c * NBT + nb) * (64u * S::kLaneBytes), b[c][nb]);
+    };
+    auto load_b = [&](int stage, int (&b)[P::kPieces][NB][E]) {
+        const unsigned at = stage_weights(stage);
 #pragma unroll
         for (int c = 0; c < P::kPieces; ++c)
 #pragma unroll
@@ -328,10 +363,27 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
         v4f acc[NB];
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) acc[nb] = (v4f){0.f, 0.f, 0.f, 0.f};
-        P::multiply(use, p, acc);
+        if constexpr (kSets == 1 && S::kArith == kThirds) {
+            // one column block after the other: in an offset's last item the next offset's weights of a block are requested as soon
+            // as its own are used, under the products of the blocks behind it
+            const unsigned next = request ? stage_weights(__builtin_amdgcn_readlane(stage_at, stage + 1)) : 0u;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                P::multiply_block(use, p, acc, nb);
+                if (request) {
+                    __builtin_amdgcn_sched_barrier(0);  // (or they take other registers, which then have to arrive to be copied)
+                    load_b1(next, fill, nb);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        } else {
+            P::multiply(use, p, acc);
+        }
         take();  // (of d1's rows)
-        __builtin_amdgcn_sched_barrier(0);  // (or the requests below take other registers, which then have to arrive to be copied)
-        if (request) load_b(__builtin_amdgcn_readlane(stage_at, stage + 1), fill);
+        __builtin_amdgcn_sched_barrier(0);  // (or the requests below take other registers)
+        if constexpr (kSets == 2 || S::kArith != kThirds) {
+            if (request) load_b(__builtin_amdgcn_readlane(stage_at, stage + 1), fill);
+        }
         // (behind the weights in either case: what the waits count is then the same for every item)
         load_a(d2, next_entry, a);
         if (mine < kNoPair) {
@@ -413,7 +465,7 @@ conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles
     __shared__ uint32_t s_pair[kMaxK * kTileRows + 16];  // compacted pair lists: pair j of offset k
     __shared__ int32_t s_blk[kMaxK + 5];            // 16-pair blocks per offset
     __shared__ float s_epi[3 * COUT];
-    __shared__ __align__(16) float s_part[kWaves * kTileRows * kWgCols];
+    __shared__ __align__(16) float s_part[S::kPartRows * kWgCols];
 
     // The row count, the number of cuts and the cuts of this workgroup's first tile under each split it may be part of are one
     // trip to memory: without a branch around any of them (no cuts: the row count's word in their place; with branches they and the
@@ -459,7 +511,7 @@ conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles
         walkers = units / S::kPerUnit * (per_unit < 1 ? 1 : (per_unit > S::kPerUnit ? S::kPerUnit : per_unit));
     }
     TilePlan plan = {0, 0};
-    if (cut_count == 0) plan = tile_plan(n, walkers, kTileRows);
+    if (cut_count == 0) plan = tile_plan(n, walkers, kMaxSplit && lsplit ? kTileRows : S::kWholeRows);
     const int tile_count = cut_count > 0 ? cut_count : (n > 0 ? plan.count : 0);
     bool idle = true;  // (no rows)
     for (int tile = first_tile; tile < tile_count; tile += walkers) {
@@ -471,9 +523,11 @@ conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles
         run_begin = tile * plan.height;
         run_end = run_begin + plan.height < n ? run_begin + plan.height : n;
     }
-    // a run longer than the tile capacity (sparse stretches under equal-work cuts) is walked in pieces
-    for (int row0 = run_begin; row0 < run_end; row0 += kTileRows) {
-    const int rows = run_end - row0 < kTileRows ? run_end - row0 : kTileRows;
+    // a run longer than the tile capacity (sparse stretches under equal-work cuts) is walked in pieces, of equal length if two do
+    const int capacity = kMaxSplit && lsplit ? kTileRows : S::kWholeRows, length = run_end - run_begin;
+    const int piece = length <= capacity ? capacity : (length <= 2 * capacity ? (length + 1) >> 1 : capacity);
+    for (int row0 = run_begin; row0 < run_end; row0 += piece) {
+    const int rows = run_end - row0 < piece ? run_end - row0 : piece;
 
     // ---- stage + compact: a wave turns an offset's neighbour list (two halves of 64 rows) into a pair list ----
     constexpr int kListsPerWave = (kMaxK + kWaves - 1) / kWaves;
@@ -515,8 +569,14 @@ conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles
     idle = false;
     if (tid < 16) s_pair[kMaxK * kTileRows + tid] = kNoPair;
     // zero this wave's partial tile (while the lists are on their way)
-    float* part = s_part + wave * kTileRows * cols;
-    for (int t = lane; t < rows << lvec; t += 64) reinterpret_cast<float4*>(part)[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+    int waves = kWaves, part_rows = kTileRows;
+    if constexpr (kMaxSplit) {
+        part_rows = rows;
+        waves = split || rows * 8 <= S::kPartRows ? 8 : (rows * 7 <= S::kPartRows ? 7 : 6);
+        static_assert(kWaves == 8 && S::kFewestWaves == 6, "waves");
+    }
+    float* part = s_part + wave * part_rows * cols;
+    for (int t = lane; t < (wave < waves ? rows << lvec : 0); t += 64) reinterpret_cast<float4*>(part)[t] = make_float4(0.f, 0.f, 0.f, 0.f);
     float epi_scale = 1.f, epi_shift = 0.f, epi_col = 1.f;
     if (row0 == run_begin && tid < COUT) {
         if (scale) epi_scale = scale[tid];
@@ -551,8 +611,8 @@ conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles
     }
     __syncthreads();
     if constexpr (kMaxSplit)
-        if (split) multiply<S, COUT, kWgCols / 32>(rs_in, rs_w, s_pair, s_blk, volume, wave, lane, col_first / 16, (rows + 15) >> 4, part);
-    if (!kMaxSplit || !split) multiply<S, COUT, kWgCols / 16>(rs_in, rs_w, s_pair, s_blk, volume, wave, lane, col_first / 16, (rows + 15) >> 4, part);
+        if (split) multiply<S, COUT, kWgCols / 32>(rs_in, rs_w, s_pair, s_blk, volume, wave, waves, lane, col_first / 16, (rows + 15) >> 4, part);
+    if (!kMaxSplit || !split) multiply<S, COUT, kWgCols / 16>(rs_in, rs_w, s_pair, s_blk, volume, wave, waves, lane, col_first / 16, (rows + 15) >> 4, part);
     __syncthreads();
 
     // fixed-order sum of the waves' partial tiles, epilogue, coalesced stores; the sums of kAtOnce vectors are read together
@@ -568,7 +628,7 @@ conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles
         const float4* col = reinterpret_cast<const float4*>(s_part) + (r << lvec) + (vec ^ (r & ((1 << lvec) - 1)));
         float4 p4[kWaves];
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) p4[w] = col[w * (kTileRows << lvec)];
+        for (int w = 0; w < kWaves; ++w) p4[w] = w < S::kFewestWaves || w < waves ? col[w * (part_rows << lvec)] : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int m = kWaves; m > 1; m = (m + 1) / 2)  // (folded: fewer roundings follow each other)
 #pragma unroll
@@ -693,7 +753,7 @@ bool gemm_wide_takes_rows(int max_voxels, int cin, int cout, int in_type) {
 }
 
 int gemm_wide_tile_rows(int cin, int cout, int type) {
-    if (cout >= 64) return Shape<float, 64, 64>::kTileRows;
+    if (cout >= 64) return Shape<float, 64, 64>::kWholeRows;
     if (type == SESSD_HALF) return Shape<__half, 16, 16>::kTileRows;
     if (cout == 16) return Shape<float, 16, 16>::kTileRows;
     return cin == 32 ? Shape<float, 32, 32>::kTileRows : Shape<float, 16, 32>::kTileRows;

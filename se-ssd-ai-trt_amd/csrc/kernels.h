@@ -54,11 +54,11 @@ __host__ __device__ inline TilePlan tile_plan(int n, int num_cu, int target) {
 }
 // The FP32 kernel (conv_wide.hip) with few rows and 64 or more output columns: the 64 columns of a tile are dealt to two workgroups,
 // so that the tiles stay tall enough to fill their 16-pair blocks while every compute unit has work and reads only its
-// columns of the weights.  At the bound a tile has 60 rows: beyond it the blocks of the unsplit tiles are full enough, and taller
-// ones reach beyond the kernel's 96 rows where the pairs are few (64 -> 64 at 3 815 rows 12.2 us split, 14.8 not;
-// at 7 120 16.4, 17.2; at 9 106 22.8, 18.8; 32 -> 64 at 4 593 9.6, 10.5; at 7 218 10.8, 11.2; at 10 139 16.8, 12.8).
+// columns of the weights.  At the bound a tile has 75 rows (the kernel holds 128 with half of the columns, 112 with 128 channels): beyond
+// it the blocks of the unsplit tiles are full enough (64 -> 64 at 3 815 rows 12.2 us split, 14.8 not; at 8 330 16.8, 17.6; at 9 145
+// 17.0, 17.6; at 10 070 18.3, 18.0).
 // A kernel volume with fewer offsets than could be dealt to the waves (the 3x1x1 layer) is not split.
-constexpr int kWideSplitRows = 60, kWideSplitMinOffsets = 16;
+constexpr int kWideSplitRows = 75, kWideSplitMinOffsets = 16;
 __host__ __device__ inline int wide_log2_split(int n, int K, int num_cu) {
     if (num_cu % 2 || K < kWideSplitMinOffsets) return 0;
     return n <= num_cu / 2 * kWideSplitRows ? 1 : 0;

@@ -1011,6 +1011,40 @@ def test_wide_fp32_kernel_around_the_row_counts_of_its_column_splits(n, cin):
     _fp32_subm_wide_against_oracle(n, n + 7, (11, 200, 176), 900 + n, threads=8, cin=cin)
 
 
+@pytest.mark.parametrize("cin,cout", [(64, 64), (128, 128)])
+@pytest.mark.parametrize("per_unit", [37, 38, 72, 73, 82, 83, 96, 97])
+def test_wide_fp32_kernel_around_its_numbers_of_waves(per_unit, cin, cout):
+    """64 columns: eight waves multiply a tile of up to 72 rows, seven one of up to 82, six one of up to 96; up to 75 rows for two units
+    (37 a unit) these share a tile.  A solid block of voxels (equal tiles) of that many rows for each of 256 units, and half of it
+    solid with the rest scattered, whose tiles are several times as long as the others and walked in pieces, against the oracle (pad
+    rows included)."""
+    n = 256 * per_unit * 64 // cout
+    rng = np.random.default_rng(n + cout)
+    grid, mv = (21, 400, 352), n + 5
+    side = int(np.ceil((n / 16) ** 0.5))
+    z, y, x = (a.ravel() for a in np.meshgrid(np.arange(16), np.arange(side), np.arange(side), indexing="ij"))
+    solid = np.stack([np.zeros_like(z), z, y, x], 1)[:n].astype(np.int32)
+    z, y, x = (a.ravel() for a in np.meshgrid(np.arange(1, 21, 2), np.arange(200, 400, 2), np.arange(1, 352, 2), indexing="ij"))
+    far = np.stack([np.zeros_like(z), z, y, x], 1).astype(np.int32)
+    mixed = np.concatenate([solid[:n // 2], far[rng.permutation(len(far))[:n - n // 2]]])
+    feat = rng.uniform(-1, 1, (n, cin)).astype(np.float32)
+    w = rng.normal(0, 0.1, (27, cin, cout)).astype(np.float32)
+    sc, sh = rng.uniform(0.5, 1.5, cout).astype(np.float32), rng.uniform(-0.2, 0.2, cout).astype(np.float32)
+    for coors in (solid, mixed):
+        conv, out, pairs, num, cbuf = run_subm(coors, n, feat, w, grid, mv, sc, sh, True)
+        O.set_threads(16)
+        try:
+            o_pairs, o_num, _ = O.subm_rulebook(coors, n, grid[::-1], mv)
+            o_out = O.scale_shift_relu(O.gather_gemm_scatter(feat, w, o_pairs, o_num, mv), mv, sc, sh, True)
+        finally:
+            O.set_threads(1)
+        assert np.array_equal(num, o_num)
+        assert_features_close(out, o_out, RTOL_FP32, "wide fp32 %d->%d, %d rows" % (cin, cout, n),
+                              abs_sum=abs_sum_of(feat, w, o_pairs, o_num, mv, mv, sc, sh))
+        assert conv.status() == 0
+        conv.close()
+
+
 @pytest.mark.parametrize("cin,cout,half", [(16, 32, False), (64, 64, False), (32, 64, False), (128, 128, False), (16, 16, True),
                                            (32, 64, True), (64, 64, True), (128, 128, True)])
 def test_every_row_is_a_pad_row(cin, cout, half):
