@@ -29,10 +29,14 @@
 //     19.6 -> 18.8 us, 14 629 22.9 -> 21.9; 128 -> 128 at 14 629 69.7 -> 66.1; frames of 20 000 points 271 -> 266; up to 4 200 rows the
 //     call with its pad rows 13.9 -> 14.2, frames of 2 000 points the same).  Longer runs are walked in two halves rather than in 96
 //     rows and the rest (64 -> 64 at 21 591 rows 38.6 -> 34.4);
-//   * the rows of the block after next are requested, and the next block's split, under a block's MFMAs; the next offset's
-//     weights are requested with the first block of an offset into a second set of registers, or, where these do not hold two
-//     sets (64 x 64), in its last block into the only one, each 16 columns as soon as the block's products with them are made (behind all
-//     products: part of the figures above; by itself 0.5-1 %);
+//   * a block's MFMAs are one column block after the other.  Under those of the next one a column block's sums are added to the partial
+//     tile (filling pairs add to a row of their own, so that no branch is in the way) and, where the registers do not hold two
+//     sets of weights (64 x 64), the next offset's weights of its columns requested if this is the offset's last block; else these
+//     are requested with the offset's first into a second set.  The next block's rows are permuted and those of the block after it
+//     requested under the last MFMAs, and split behind them (32 -> 32 at 62 674 rows 32.4 -> 30.6 us, 64 -> 64 at 21 591 34.3 -> 32.9, frames of
+//     80 000 points 424 -> 410.  Split between the MFMAs instead: the same, the SIMD's other wave has filled those slots already);
+//   * the last, incomplete round of the offsets goes to the waves 0, 1, ..: a SIMD serves its older wave first (64 -> 64 at 4 217 rows 14.3 ->
+//     13.6 us, 7 236 17.2 -> 16.7; frames of 2 000 points 190.7 -> 186.7);
 //   * a wave's blocks and offsets are listed once, a lane each, and read with readlane: the loop has no other bookkeeping.
 // Up to 32 columns two to four workgroups share a unit, as many as the rows need: only where one tile for each unit would be higher than a
 // tile can be does a second one begin (32 -> 32, eight waves, 4 208 rows: one workgroup a unit 7.9 us, two 10.7).  Beyond what they hold
@@ -49,6 +53,7 @@
 #include <cmath>
 #include <cstring>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "pad_rows.h"
@@ -218,34 +223,28 @@ struct Products<S, NB, kThirds> {
             }
         p[kWords - 1] |= left & 0xffffu ? 0x7fff : 0;  // (the last word: what waits for all of them is last)
     }
-    static __device__ __forceinline__ void step(const int (&w)[3 * C][NB][E], const int (&x)[kWords], v4f (&acc)[NB], int t, int c, int nb) {
+    // the MFMAs of a block in their order: one column block after the other, whose weights are free behind it
+    static constexpr int kSteps = 6 * C * NB;
+    static __device__ __forceinline__ void step(int n, const int (&w)[3 * C][NB][E], const int (&x)[kWords], v4f (&acc)[NB]) {
         constexpr int kPart[6][2] = {{0, 2}, {1, 1}, {2, 0}, {0, 1}, {1, 0}, {0, 0}};  // of w, of x
+        const int nb = n / (6 * C), t = n / C % 6, c = n % C;
         acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(operand8<v8b>(w[kPart[t][0] * C + c][nb]),
                                                           operand8<v8b>(x + 2 * G * kPart[t][1] + 4 * c), acc[nb], 0, 0, 0);
     }
-    static __device__ __forceinline__ void multiply(const int (&w)[3 * C][NB][E], const int (&x)[kWords], v4f (&acc)[NB]) {
-#pragma unroll
-        for (int t = 0; t < 6; ++t)
-#pragma unroll
-            for (int c = 0; c < C; ++c)
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb) step(w, x, acc, t, c, nb);
-    }
-    // one column block; its weights are free behind it
-    static __device__ __forceinline__ void multiply_block(const int (&w)[3 * C][NB][E], const int (&x)[kWords], v4f (&acc)[NB], int nb) {
-#pragma unroll
-        for (int t = 0; t < 6; ++t)
-#pragma unroll
-            for (int c = 0; c < C; ++c) step(w, x, acc, t, c, nb);
-    }
 };
+
+// f(0), f(1) .. f(N - 1), the numbers as types
+template <typename F, int... N>
+__device__ __forceinline__ void unrolled(F f, std::integer_sequence<int, N...>) {
+    (f(std::integral_constant<int, N>{}), ...);
+}
 
 // One wave's share of a tile: the pairs of the offsets dealt to it, times its columns -- 16-column blocks nb0 .. nb0 + NB - 1
 // of the layer -- into its partial tile `part` (rows of 16 NB floats).  waves: among which the offsets are dealt; most: blocks that an
-// offset can have in this tile.
+// offset can have in this tile; spare: a row for what filling pairs add.
 template <typename S, int COUT, int NB>
 __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_buffer_rsrc_t rs_w, const uint32_t* s_pair,
-                                         const int32_t* s_blk, int K, int wave, int waves, int lane, int nb0, int most, float* part) {
+                                         const int32_t* s_blk, int K, int wave, int waves, int lane, int nb0, int most, float* part, float* spare) {
     using P = Products<S, NB, S::kArith>;
     constexpr int kParts = S::kParts, G = S::G, E = S::kLaneBytes / 4, kTileRows = S::kTileRows;
     constexpr int kSets = P::kPieces * NB * E > 64 ? 1 : 2;  // of weights: the registers do not hold two of the largest
@@ -255,7 +254,7 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
     const int q = lane >> 4;  // channel group of a step
 
     // offsets of this wave: ranked by their number of 16-pair blocks (ballots: lane k holds offset k)
-    // and dealt in that order back and forth over the waves (0 1 2 3 3 2 1 0 ...)
+    // and dealt in that order back and forth over the waves (0 1 2 3 3 2 1 0 ...; or 3 2 1 0 0 1 2 3 ...)
     const int blocks_of = lane < K ? s_blk[lane] : 0;
     uint32_t mask;
     {
@@ -274,7 +273,14 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
             r2 -= r2 >= 4 * waves ? 4 * waves : 0;
             r2 -= r2 >= 2 * waves ? 2 * waves : 0;
         }
-        const int w = r2 < waves ? r2 : 2 * waves - 1 - r2;
+        // (the last round, of few offsets, begins with the first wave: the older waves of a SIMD are served first and end earlier)
+        const int lists = __popcll(__ballot(blocks_of > 0));
+        int rounds = 0;
+#pragma unroll
+        for (int n = 0; n * S::kFewestWaves < kMaxK; ++n) rounds += lists > n * waves;
+        const bool back = (r2 >= waves) != (rounds % 2 == 0);
+        const int in_round = r2 < waves ? r2 : r2 - waves;
+        const int w = back ? waves - 1 - in_round : in_round;
         mask = (uint32_t)__ballot(blocks_of > 0 && w == wave);
     }
     if (!mask) return;
@@ -350,59 +356,103 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
 
     // `use`: the weights of the item's stage; `fill`: those of the next one, requested behind its first block, or, where there is one
     // set, behind its last
-    auto item = [&](const int (&use)[P::kPieces][NB][E], int (&fill)[P::kPieces][NB][E], bool request) {
-        d2 = __builtin_amdgcn_readlane(item_at, t + 2);
-        ++t;
-        next_entry = entry_at(d2, request4);
-        const uint32_t mine = entry_at(d0, operand4);
-        const int r = (int)(mine & ((1u << S::kRowBits) - 1u));
-        float4* const dst = reinterpret_cast<float4*>(part) + r * kSlots;
-        float4 sum[NB];
+    auto plain_item = [&](const int (&use)[P::kPieces][NB][E], int (&fill)[P::kPieces][NB][E], bool request) {
+        if constexpr (S::kArith != kThirds) {
+            d2 = __builtin_amdgcn_readlane(item_at, t + 2);
+            ++t;
+            next_entry = entry_at(d2, request4);
+            const uint32_t mine = entry_at(d0, operand4);
+            const int r = (int)(mine & ((1u << S::kRowBits) - 1u));
+            float4* const dst = reinterpret_cast<float4*>(part) + r * kSlots;
+            float4 sum[NB];
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) sum[nb] = dst[(nb * 4 + q) ^ (r & (kSlots - 1))];
-        v4f acc[NB];
+            for (int nb = 0; nb < NB; ++nb) sum[nb] = dst[(nb * 4 + q) ^ (r & (kSlots - 1))];
+            v4f acc[NB];
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) acc[nb] = (v4f){0.f, 0.f, 0.f, 0.f};
-        if constexpr (kSets == 1 && S::kArith == kThirds) {
-            // one column block after the other: in an offset's last item the next offset's weights of a block are requested as soon
-            // as its own are used, under the products of the blocks behind it
-            const unsigned next = request ? stage_weights(__builtin_amdgcn_readlane(stage_at, stage + 1)) : 0u;
+            for (int nb = 0; nb < NB; ++nb) acc[nb] = (v4f){0.f, 0.f, 0.f, 0.f};
+            P::multiply(use, p, acc);
+            take();  // (of d1's rows)
+            __builtin_amdgcn_sched_barrier(0);  // (or the requests below take other registers)
+            if (request) load_b(__builtin_amdgcn_readlane(stage_at, stage + 1), fill);
+            // (behind the weights in either case: what the waits count is then the same for every item)
+            load_a(d2, next_entry, a);
+            if (mine < kNoPair) {
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                P::multiply_block(use, p, acc, nb);
-                if (request) {
-                    __builtin_amdgcn_sched_barrier(0);  // (or they take other registers, which then have to arrive to be copied)
-                    load_b1(next, fill, nb);
-                    __builtin_amdgcn_sched_barrier(0);
+                for (int nb = 0; nb < NB; ++nb) {
+                    float4 v = sum[nb];
+                    v.x += acc[nb][0];
+                    v.y += acc[nb][1];
+                    v.z += acc[nb][2];
+                    v.w += acc[nb][3];
+                    dst[(nb * 4 + q) ^ (r & (kSlots - 1))] = v;
                 }
             }
-        } else {
-            P::multiply(use, p, acc);
+            d0 = d1;
+            d1 = d2;
         }
-        take();  // (of d1's rows)
-        __builtin_amdgcn_sched_barrier(0);  // (or the requests below take other registers)
-        if constexpr (kSets == 2 || S::kArith != kThirds) {
-            if (request) load_b(__builtin_amdgcn_readlane(stage_at, stage + 1), fill);
-        }
-        // (behind the weights in either case: what the waits count is then the same for every item)
-        load_a(d2, next_entry, a);
-        if (mine < kNoPair) {
+    };
+    // The same with what there is to do between the MFMAs in its place: a column block's sums are added under the products of the
+    // next, the rows permuted and requested under the last.
+    auto dense_item = [&](const int (&use)[P::kPieces][NB][E], int (&fill)[P::kPieces][NB][E], auto request) {
+        if constexpr (S::kArith == kThirds) {
+            constexpr int kBlockSteps = P::kSteps / NB, kAddAt = kBlockSteps / 3, kRowsAt = P::kSteps - P::kSteps / 12;
+            d2 = __builtin_amdgcn_readlane(item_at, t + 2);
+            ++t;
+            next_entry = entry_at(d2, request4);
+            const uint32_t mine = entry_at(d0, operand4);
+            const unsigned next = stage_weights(request.value ? __builtin_amdgcn_readlane(stage_at, stage + 1) : -1);
+            const int r = (int)(mine & ((1u << S::kRowBits) - 1u));
+            float4* const dst = mine < kNoPair ? reinterpret_cast<float4*>(part) + r * kSlots : reinterpret_cast<float4*>(spare);
+            float4 sum[NB];
+            v4f acc[NB];
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
+            for (int nb = 0; nb < NB; ++nb) acc[nb] = (v4f){0.f, 0.f, 0.f, 0.f};
+            auto add = [&](int nb) {
                 float4 v = sum[nb];
                 v.x += acc[nb][0];
                 v.y += acc[nb][1];
                 v.z += acc[nb][2];
                 v.w += acc[nb][3];
                 dst[(nb * 4 + q) ^ (r & (kSlots - 1))] = v;
-            }
+            };
+            int row[G][E];
+            __builtin_amdgcn_sched_barrier(0);
+            unrolled([&](auto n_c) {
+                constexpr int n = decltype(n_c)::value;
+                P::step(n, use, p, acc);
+                if constexpr (n == 1) {
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb) sum[nb] = dst[(nb * 4 + q) ^ (r & (kSlots - 1))];
+                }
+                if constexpr (request.value && kSets == 1 && n % kBlockSteps == kBlockSteps - 1) load_b1(next, fill, n / kBlockSteps);
+                if constexpr (n >= kBlockSteps && n % kBlockSteps == kAddAt) add(n / kBlockSteps - 1);
+                if constexpr (n == kRowsAt) {
+#pragma unroll
+                    for (int g = 0; g < G; ++g)
+#pragma unroll
+                        for (int e = 0; e < E; ++e) row[g][e] = __builtin_amdgcn_ds_bpermute(from_lane4, a[g][e]);
+                    if constexpr (request.value && kSets == 2) load_b(__builtin_amdgcn_readlane(stage_at, stage + 1), fill);
+                    load_a(d2, next_entry, a);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }, std::make_integer_sequence<int, P::kSteps>{});
+            add(NB - 1);
+            P::take(row, p);
+#pragma unroll
+            for (int w = 0; w < P::kWords; ++w) asm volatile("" : "+v"(p[w]));
+            d0 = d1;
+            d1 = d2;
         }
-        d0 = d1;
-        d1 = d2;
     };
     auto run_stage = [&](const int (&use)[P::kPieces][NB][E], int (&fill)[P::kPieces][NB][E]) -> bool {
         const int n = __builtin_amdgcn_readlane(stage_items, stage);
-        for (int j = 0; j < n; ++j) item(use, fill, j == (kSets == 2 ? 0 : n - 1));
+        if constexpr (S::kArith == kThirds) {
+            if constexpr (kSets == 2) dense_item(use, fill, std::true_type{});
+            for (int j = 1; j < n; ++j) dense_item(use, fill, std::false_type{});
+            if constexpr (kSets == 1) dense_item(use, fill, std::true_type{});
+        } else {
+            for (int j = 0; j < n; ++j) plain_item(use, fill, j == (kSets == 2 ? 0 : n - 1));
+        }
         return ++stage < stages;
     };
     if constexpr (kSets == 2)
@@ -465,7 +515,7 @@ conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles
     __shared__ uint32_t s_pair[kMaxK * kTileRows + 16];  // compacted pair lists: pair j of offset k
     __shared__ int32_t s_blk[kMaxK + 5];            // 16-pair blocks per offset
     __shared__ float s_epi[3 * COUT];
-    __shared__ __align__(16) float s_part[S::kPartRows * kWgCols];
+    __shared__ __align__(16) float s_part[S::kPartRows * kWgCols + (S::kArith == kThirds ? kWgCols : 0)];  // (and the spare row)
 
     // The row count, the number of cuts and the cuts of this workgroup's first tile under each split it may be part of are one
     // trip to memory: without a branch around any of them (no cuts: the row count's word in their place; with branches they and the
@@ -611,8 +661,8 @@ conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles
     }
     __syncthreads();
     if constexpr (kMaxSplit)
-        if (split) multiply<S, COUT, kWgCols / 32>(rs_in, rs_w, s_pair, s_blk, volume, wave, waves, lane, col_first / 16, (rows + 15) >> 4, part);
-    if (!kMaxSplit || !split) multiply<S, COUT, kWgCols / 16>(rs_in, rs_w, s_pair, s_blk, volume, wave, waves, lane, col_first / 16, (rows + 15) >> 4, part);
+        if (split) multiply<S, COUT, kWgCols / 32>(rs_in, rs_w, s_pair, s_blk, volume, wave, waves, lane, col_first / 16, (rows + 15) >> 4, part, s_part + S::kPartRows * kWgCols);
+    if (!kMaxSplit || !split) multiply<S, COUT, kWgCols / 16>(rs_in, rs_w, s_pair, s_blk, volume, wave, waves, lane, col_first / 16, (rows + 15) >> 4, part, s_part + S::kPartRows * kWgCols);
     __syncthreads();
 
     // fixed-order sum of the waves' partial tiles, epilogue, coalesced stores; the sums of kAtOnce vectors are read together
