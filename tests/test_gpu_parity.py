@@ -1005,9 +1005,9 @@ def test_wide_fp32_kernel_tall_tiles_and_two_tiles_per_workgroup(n, clustered, c
 
 
 @pytest.mark.parametrize("cin", [64, 32])
-@pytest.mark.parametrize("n", [3071, 3072, 3073, 7679, 7680, 7681, 10239, 10240, 10241])
+@pytest.mark.parametrize("n", [3071, 3072, 3073, 7679, 7680, 7681, 9599, 9600, 9601, 10239, 10240, 10241])
 def test_wide_fp32_kernel_around_the_row_counts_of_its_column_splits(n, cin):
-    """On 256 compute units the columns of a tile are dealt to two workgroups up to 7 680 rows."""
+    """On 256 compute units the columns of a tile are dealt to two workgroups up to 9 600 rows."""
     _fp32_subm_wide_against_oracle(n, n + 7, (11, 200, 176), 900 + n, threads=8, cin=cin)
 
 
@@ -1067,7 +1067,7 @@ def test_every_row_is_a_pad_row(cin, cout, half):
 @pytest.mark.parametrize("n", [1, 65, 97, 1536, 1537, 3840, 3841, 5120, 5121, 12289, 20000])
 def test_wide_fp32_kernel_with_128_columns(n, cin):
     """128 output columns: two workgroups take 64 columns each of every tile (128 tiles a round on 256 compute units, of
-    up to 96 rows), up to 3 840 rows four; 128 input channels are walked in two parts.  Against
+    up to 96 rows), up to 4 800 rows four; 128 input channels are walked in two parts.  Against
     the oracle (pad rows included)."""
     rng = np.random.default_rng(n + cin)
     grid, mv = ((5, 40, 40) if n < 1000 else (21, 400, 352)), n + 39
@@ -1091,8 +1091,8 @@ def test_wide_fp32_kernel_with_128_columns(n, cin):
 @pytest.mark.parametrize("cin,cout", [(4, 16), (4, 32), (16, 16), (16, 32), (32, 32)])
 @pytest.mark.parametrize("n", [1, 16, 63, 65, 113, 129, 16385, 28672, 28673, 40000])
 def test_wide_fp32_kernel_with_few_columns(n, cin, cout):
-    """16 and 32 output columns: tiles of up to 112 (64) rows, one workgroup per compute unit up to 256 full tiles (28 672
-    rows with 16 columns, 16 384 with 32), two beyond.  Against the oracle (pad rows included)."""
+    """16 and 32 output columns: tiles of up to 128 (64, from 32 channels 80) rows, one workgroup per compute unit up to 256 full tiles,
+    two, three or four beyond.  Against the oracle (pad rows included)."""
     rng = np.random.default_rng(n + cin)
     grid, mv = ((5, 40, 40) if n < 1000 else (21, 400, 352)), n + 39
     coors = F.clustered_active_voxels(n, grid, n, n_blobs=max(4, n // 100))
