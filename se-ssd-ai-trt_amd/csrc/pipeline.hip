@@ -269,8 +269,9 @@ struct Pipeline {
     // One frame.  The rulebooks depend only on coordinates, the GEMMs on rulebooks + features.  The coordinate chain
     // (coord.h) is  vg_insert | vg_flags | vg_finalize + insert 1 | then per stage i: flags i+1 + lookups on stage i |
     // number i+1 + insert i+2 + tile cuts of those rulebooks.  With `aux`, everything behind the lookups on the voxels
-    // runs there and the GEMM chain waits per layer for the pass its rulebook comes from, so that the passes of later
-    // layers overlap the GEMMs of earlier ones; under stream capture that becomes two branches of the graph.
+    // runs there, and the GEMM chain waits for the passes its layers' rulebooks come from (one by one at first, then for the
+    // branch's end: kOwnWaits), so that the passes of later layers overlap the GEMMs of earlier ones; under stream capture
+    // that becomes two branches of the graph.
     int enqueueFrame(const void* points, const void* points_size, void* dense, hipStream_t stream) {
         const std::vector<Stage> cs = coordStages();
         const int m = (int)cs.size() - 1;  // strided layers
@@ -326,42 +327,59 @@ struct Pipeline {
         SESSD_TRY(launch_vg_flags(v, pads, stream));
         SESSD_TRY(launch_vg_finalize(v, m ? &part[1] : nullptr, stream));
 
-        // Coordinate passes are counted 2i (flags + lookups of stage i) and 2i + 1 (numbering, cuts).  ready[l] = the
-        // pass layer l's rulebook is complete after; pass 0 runs on the caller's stream.
+        // Coordinate passes are counted 2i (flags + lookups of stage i) and 2i + 1 (numbering, cuts, builds).  ready[l] = the
+        // pass layer l's rulebook is complete after; pass 0 runs on the caller's stream.  works[p]: it does something on the other.
+        const int clean_at = m < 1 ? 0 : 1;  // stage 1's own rulebook is the last reader of the voxels' table
         std::vector<int> ready(stages.size(), 0);
+        std::vector<char> works((size_t)(2 * m + 2), 0);
         for (int i = 0; i <= m; ++i) {
-            for (int l : cs[(size_t)i].lookups) {
+            const Stage& sg = cs[(size_t)i];
+            works[(size_t)(2 * i)] = i > 0;
+            works[(size_t)(2 * i + 1)] = i < m || i == clean_at || !sg.builds.empty();
+            for (int l : sg.lookups) {
                 const ConvStage& st = *stages[(size_t)l];
                 const bool cuts = st.subm ? st.subm->wantTileCuts() : st.sparse->wantTileCuts();
                 ready[(size_t)l] = 2 * i + (cuts ? 1 : 0);
+                if (cuts) works[(size_t)(2 * i + 1)] = 1;
             }
-            for (int l : cs[(size_t)i].builds) ready[(size_t)l] = 2 * i + 1;
+            for (int l : sg.builds) ready[(size_t)l] = 2 * i + 1;
         }
-        std::vector<char> awaited((size_t)(2 * m + 2), 0);
-        for (size_t l = 0; l < stages.size(); ++l) awaited[(size_t)ready[l]] = 1;
+        int last_side = 2 * m + 1;
+        while (last_side > 0 && !works[(size_t)last_side]) --last_side;
+        // wait_for[l]: the pass that layer l has the chain wait for (0: none); an event stands for each of them and for the join, for no
+        // other pass.  A wait for the other branch costs the chain 4-5 us in a graph, however long the pass has been done; behind the
+        // second strided layer the branch is far ahead of the chain, and the layers from there on wait once, for its end (frames of
+        // 2 000 points 200 -> 193.5 us, 20 000 301 -> 295, 60 000 (FP16) 240 -> 234).
+        constexpr int kOwnWaits = 4;  // passes that are waited for one by one: to the lookups on the second strided layer's rows
         const bool fork = aux != nullptr && stages.size() > 0;
         hipStream_t side = fork ? aux : stream;
-        int last_side = 0;  // last pass that did something on `side`
-        // The feature chain, as far as the passes up to `last_pass` allow.  A wait for the other branch costs the chain 4-5 us in a graph,
-        // however long the pass has been done; behind the second strided layer the branch is far ahead of the chain, and the layers from
-        // there on wait once, for its end (frames of 2 000 points 200 -> 193.5 us, 20 000 301 -> 295, 60 000 (FP16) 240 -> 234).
+        std::vector<int> wait_for(stages.size(), 0);
+        std::vector<char> awaited((size_t)(2 * m + 2), 0);
+        bool join = false;  // at the end, for what no layer has waited for
+        if (fork) {
+            int waited = 0;
+            for (size_t l = 0; l < stages.size(); ++l) {
+                const int pass = ready[(size_t)(stages[l]->rulebook_from >= 0 ? stages[l]->rulebook_from : (int)l)];
+                if (pass <= waited) continue;
+                waited = pass > kOwnWaits ? last_side : pass;
+                wait_for[l] = waited;
+                awaited[(size_t)waited] = 1;
+            }
+            join = last_side > waited;
+            if (join) awaited[(size_t)last_side] = 1;
+        }
+        // The feature chain, as far as the passes up to `last_pass` allow.
         const void* feat = vg_voxels.p;
         const int32_t* coors = static_cast<const int32_t*>(vg_coors.p);
         const int32_t* num = static_cast<const int32_t*>(vg_num.p);
         size_t next_layer = 0;
-        int last_waited = 0;
         bool scattered = false;
-        constexpr int kOwnWaits = 4;  // passes that are waited for one by one: to the lookups on the second strided layer's rows
         auto layers = [&](int last_pass) -> int {
             for (; next_layer < stages.size(); ++next_layer) {
                 ConvStage& st = *stages[next_layer];
                 const int owner = st.rulebook_from >= 0 ? st.rulebook_from : (int)next_layer;
-                const int pass = ready[(size_t)owner];
-                if (pass > last_pass) return SESSD_OK;
-                if (fork && pass > last_waited) {
-                    last_waited = pass > kOwnWaits ? last_side : pass;
-                    SESSD_HIP_TRY(hipStreamWaitEvent(stream, ev_pass[(size_t)last_waited], 0));
-                }
+                if (ready[(size_t)owner] > last_pass) return SESSD_OK;
+                if (wait_for[next_layer]) SESSD_HIP_TRY(hipStreamWaitEvent(stream, ev_pass[(size_t)wait_for[next_layer]], 0));
                 DenseTarget dt;
                 const bool fuse = next_layer + 1 == stages.size() && denseByEpilogue();
                 if (fuse) {
@@ -386,7 +404,6 @@ struct Pipeline {
         // 2 000 points 199.2 us with the chain first, 192.6 with the passes, 4 000 213.6 and 212.6, 10 000 253.5 and 252.9, 80 000 444
         // and 460; FP16 2 000 points 172.9 and 173.7, 10 000 181.6 and 184.1, 60 000 223.1 and 225.2.
         const bool chain_first = desc.feature_dtype != SESSD_FLOAT || desc.max_points > 4096;
-        const int clean_at = m < 1 ? 0 : 1;  // stage 1's own rulebook is the last reader of the voxels' table
         for (int i = 0; i <= m; ++i) {
             const Stage& sg = cs[(size_t)i];
             hipStream_t s = i == 0 ? stream : side;
@@ -416,9 +433,8 @@ struct Pipeline {
                 SESSD_HIP_TRY(hipEventRecord(ev_head, stream));
                 SESSD_HIP_TRY(hipStreamWaitEvent(side, ev_head, 0));
                 if (chain_first) SESSD_TRY(layers(0));
-            } else if (fork) {
-                if (awaited[(size_t)(2 * i)]) SESSD_HIP_TRY(hipEventRecord(ev_pass[(size_t)(2 * i)], side));
-                last_side = 2 * i;
+            } else if (awaited[(size_t)(2 * i)]) {
+                SESSD_HIP_TRY(hipEventRecord(ev_pass[(size_t)(2 * i)], side));
             }
             // numbering of the next strided layer's rows (their tickets for the layer behind it), tile cuts
             FillArgs clear;
@@ -441,17 +457,12 @@ struct Pipeline {
             for (int l : sg.builds) {
                 ConvStage& st = *stages[(size_t)l];
                 SESSD_TRY(st.subm->enqueueBuild(rows[(size_t)i].coors, rows[(size_t)i].num, st.ws.p, side));
-                did = true;
             }
-            if (fork && did) {
-                last_side = 2 * i + 1;
-                SESSD_HIP_TRY(hipEventRecord(ev_pass[(size_t)last_side], side));
-            }
+            if (awaited[(size_t)(2 * i + 1)]) SESSD_HIP_TRY(hipEventRecord(ev_pass[(size_t)(2 * i + 1)], side));
         }
-        if (fork && last_side > 0 && last_side % 2 == 0 && !awaited[(size_t)last_side]) SESSD_HIP_TRY(hipEventRecord(ev_pass[(size_t)last_side], side));
 
         SESSD_TRY(layers(2 * m + 1));
-        if (fork && last_side > last_waited) SESSD_HIP_TRY(hipStreamWaitEvent(stream, ev_pass[(size_t)last_side], 0));  // join
+        if (join) SESSD_HIP_TRY(hipStreamWaitEvent(stream, ev_pass[(size_t)last_side], 0));
         if (scattered) return SESSD_OK;
         const void* din[3] = {feat, coors, num};
         void* dout[1] = {dense};

@@ -241,6 +241,43 @@ def check_short_memory():
     assert rc == D.SESSD_E_HIP and not h.value
 
 
+def deeper(stages):
+    """The reference backbone with so many strided layers more, two SubM layers behind each."""
+    layers = B.reference_layers()
+    grid = layers[-2].out_shape
+    for i in range(stages):
+        layers[-1:-1] = [B.Layer("p%d" % i, D.SESSD_LAYER_SPARSE, 64, 64, grid, (3, 1, 1), (1, 1, 1), (1, 0, 0))]
+        layers[-1:-1] = [B.Layer("s%d%d" % (i, j), D.SESSD_LAYER_SUBM, 64, 64, grid) for j in range(2)]
+    return layers
+
+
+def overlapped_frame(layers, dtype, **options):
+    """The log of a frame on two streams."""
+    rc, h = create(layers, overlap_streams=1, feature_dtype=dtype, **options)
+    assert rc == 0, L.sessd_last_error()
+    stream = new_stream()
+    assert enqueue(h, stream) == 0
+    take_log()
+    assert enqueue(h, stream) == 0
+    log = take_log()
+    L.sessd_pipeline_destroy(h)
+    return log
+
+
+def check_events():
+    """Every event that a frame on two streams records is waited for, on the other stream, before it is recorded again; what comes
+    next on the caller's stream is behind all of the frame."""
+    for layers in (B.reference_layers(), B.reference_layers()[:2], deeper(4)):
+        for dtype in (D.SESSD_FLOAT, D.SESSD_HALF):
+            log = overlapped_frame(layers, dtype)
+            assert not unordered(log + [["launch", "next", log[0][-1]]])
+            for i, l in enumerate(log):
+                if l[0] != "record":
+                    continue
+                after = [k for k in log[i + 1:] if (k[0] == "record" and k[1] == l[1]) or (k[0] == "wait" and k[2] == l[1])]
+                assert after and after[0][0] == "wait" and after[0][1] != l[2], (len(layers), dtype, l, log)
+
+
 def gemm_kernel(cin, cout, rows, dtype):
     """The kernel that multiplies in a SubM layer of so many rows (nothing runs: the addresses are read by nobody)."""
     d = D.SubmConv3dDesc()
@@ -272,6 +309,7 @@ def check_row_limits():
 
 
 CHECKS = {
+    "events": check_events,
     "row-limits": check_row_limits,
     "recovery-direct": lambda: check_recovery(0, enqueue),
     "recovery-overlap": lambda: check_recovery(1, enqueue),

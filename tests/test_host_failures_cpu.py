@@ -1,5 +1,6 @@
-"""What the host side of the library does when a runtime call or an allocation fails.  Nothing runs on a GPU: the library
-is loaded onto a stand-in for the HIP runtime (fake_hip.cpp) in a process of its own (host_pipeline.py)."""
+"""The host side of the library: its launches over streams and events, and what it does when a runtime call or an allocation
+fails.  Nothing runs on a GPU: the library is loaded onto a stand-in for the HIP runtime (fake_hip.cpp) in a process of its
+own (host_pipeline.py)."""
 import os
 import shutil
 import subprocess
@@ -43,3 +44,7 @@ def test_layers_with_few_channels_run_on_the_matrix_cores_in_large_tensors(fake_
 
 def test_host_memory_that_runs_out_in_a_frame_is_an_error_code(fake_hip):
     run_check(fake_hip, "host-memory")
+
+
+def test_every_event_of_an_overlapped_frame_is_waited_for(fake_hip):
+    run_check(fake_hip, "events")
