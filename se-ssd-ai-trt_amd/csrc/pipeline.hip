@@ -269,8 +269,8 @@ struct Pipeline {
     // One frame.  The rulebooks depend only on coordinates, the GEMMs on rulebooks + features.  The coordinate chain
     // (coord.h) is  vg_insert | vg_flags | vg_finalize + insert 1 | then per stage i: flags i+1 + lookups on stage i |
     // number i+1 + insert i+2 + tile cuts of those rulebooks.  With `aux`, everything behind the lookups on the voxels
-    // runs there, and the GEMM chain waits for the passes its layers' rulebooks come from (one by one at first, then for the
-    // branch's end: kOwnWaits), so that the passes of later layers overlap the GEMMs of earlier ones; under stream capture
+    // runs there, and the GEMM chain waits for the passes its layers' rulebooks come from (one by one at first, further on for
+    // some at once: wait_for), so that the passes of later layers overlap the GEMMs of earlier ones; under stream capture
     // that becomes two branches of the graph.
     int enqueueFrame(const void* points, const void* points_size, void* dense, hipStream_t stream) {
         const std::vector<Stage> cs = coordStages();
@@ -347,10 +347,14 @@ struct Pipeline {
         int last_side = 2 * m + 1;
         while (last_side > 0 && !works[(size_t)last_side]) --last_side;
         // wait_for[l]: the pass that layer l has the chain wait for (0: none); an event stands for each of them and for the join, for no
-        // other pass.  A wait for the other branch costs the chain 4-5 us in a graph, however long the pass has been done; behind the
-        // second strided layer the branch is far ahead of the chain, and the layers from there on wait once, for its end (frames of
-        // 2 000 points 200 -> 193.5 us, 20 000 301 -> 295, 60 000 (FP16) 240 -> 234).
+        // other pass.  A wait for the other branch costs the chain 4-5 us in a graph, however long the pass has been done.  Behind the
+        // second strided layer the branch is ahead of the chain: a layer that waits there waits for the next stage's passes as well, and
+        // for all that are left where these are two stages', but for no rulebook that a later layer builds on a grid of its own.
+        // Each pass by itself / for the branch's end / so, us: the reference's backbone, FP32 2 000 points 183, 178, 178, 20 000 252, 247, 247,
+        // FP16 60 000 222, 219, 219 (so is its end); four strided layers more, each with two SubM layers, FP32 2 000 points 343, 371, 330,
+        // 20 000 487, 517, 474, FP16 20 000 319, 328, 311; twelve more, FP32 2 000 675, 770, 645.
         constexpr int kOwnWaits = 4;  // passes that are waited for one by one: to the lookups on the second strided layer's rows
+        constexpr int kAhead = 2, kRest = 4;
         const bool fork = aux != nullptr && stages.size() > 0;
         hipStream_t side = fork ? aux : stream;
         std::vector<int> wait_for(stages.size(), 0);
@@ -361,7 +365,12 @@ struct Pipeline {
             for (size_t l = 0; l < stages.size(); ++l) {
                 const int pass = ready[(size_t)(stages[l]->rulebook_from >= 0 ? stages[l]->rulebook_from : (int)l)];
                 if (pass <= waited) continue;
-                waited = pass > kOwnWaits ? last_side : pass;
+                waited = pass;
+                const int end = pass <= kOwnWaits ? pass : (last_side - pass <= kRest ? last_side : pass + kAhead);
+                for (int p = pass + 1; p <= end; ++p) {
+                    if (p % 2 && !cs[(size_t)(p / 2)].builds.empty()) break;
+                    if (works[(size_t)p]) waited = p;
+                }
                 wait_for[l] = waited;
                 awaited[(size_t)waited] = 1;
             }

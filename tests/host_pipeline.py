@@ -278,6 +278,45 @@ def check_events():
                 assert after and after[0][0] == "wait" and after[0][1] != l[2], (len(layers), dtype, l, log)
 
 
+def passes_before_gemms(log):
+    """For each gather-GEMM of a frame, in the order of the layers: how many lookup passes it is ordered behind."""
+    done, at, counts = {}, {}, []
+    for i, l in enumerate(log):
+        if l[0] == "launch":
+            if "conv_" in l[1]:
+                counts.append(sum("flags_lookups" in log[j][1] for j in done.get(l[2], ())))
+            done.setdefault(l[2], set()).add(i)
+        elif l[0] == "record":
+            at[l[1]] = set(done.get(l[2], ()))
+        elif l[0] == "wait":
+            done.setdefault(l[1], set()).update(at.get(l[2], ()))
+    return counts
+
+
+def check_waits():
+    """A layer of an overlapped frame runs behind the lookups on its own stage's rows, and however deep the backbone is, behind those
+    on the rows of at most two later stages."""
+    for more in (0, 1, 2, 4, 12):
+        layers = deeper(more)
+        for dtype in (D.SESSD_FLOAT, D.SESSD_HALF):
+            stage, counts = 0, passes_before_gemms(overlapped_frame(layers, dtype))
+            assert len(counts) == len(layers)
+            for l, n in zip(layers, counts):
+                stage += l.type == D.SESSD_LAYER_SPARSE
+                assert stage + 1 <= n <= stage + 3, (more, dtype, l.name, n, counts)
+    # a SubM layer on a grid of its own builds its rulebook behind the stage's lookups: the strided layer in front of it, which has
+    # its rulebook then (FP16 layers need no tile cuts), does not wait for that
+    layers = deeper(4)
+    at = [l.name for l in layers].index("s30")
+    x, y, z = layers[at].out_shape
+    layers[at].out_shape = (x + 1, y, z)
+    log = overlapped_frame(layers, D.SESSD_HALF)
+    assert len(passes_before_gemms(log)) == len(layers)
+    names = [l[1] if l[0] == "launch" else l[0] for l in log]
+    waits = [sum(n == "wait" for n in names[:i]) for i, n in enumerate(names) if "conv_" in n]
+    assert waits[at] == waits[at - 1] + 1, waits
+
+
 def gemm_kernel(cin, cout, rows, dtype):
     """The kernel that multiplies in a SubM layer of so many rows (nothing runs: the addresses are read by nobody)."""
     d = D.SubmConv3dDesc()
@@ -310,6 +349,7 @@ def check_row_limits():
 
 CHECKS = {
     "events": check_events,
+    "waits": check_waits,
     "row-limits": check_row_limits,
     "recovery-direct": lambda: check_recovery(0, enqueue),
     "recovery-overlap": lambda: check_recovery(1, enqueue),

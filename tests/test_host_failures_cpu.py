@@ -48,3 +48,7 @@ def test_host_memory_that_runs_out_in_a_frame_is_an_error_code(fake_hip):
 
 def test_every_event_of_an_overlapped_frame_is_waited_for(fake_hip):
     run_check(fake_hip, "events")
+
+
+def test_layers_of_a_deep_backbone_do_not_wait_for_the_whole_coordinate_branch(fake_hip):
+    run_check(fake_hip, "waits")
