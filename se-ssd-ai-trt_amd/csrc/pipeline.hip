@@ -360,12 +360,14 @@ struct Pipeline {
         std::vector<int> wait_for(stages.size(), 0);
         std::vector<char> awaited((size_t)(2 * m + 2), 0);
         bool join = false;  // at the end, for what no layer has waited for
+        int longer = -1;    // passes less layers in front of the last layer that waits by itself for what it needs
         if (fork) {
             int waited = 0;
             for (size_t l = 0; l < stages.size(); ++l) {
                 const int pass = ready[(size_t)(stages[l]->rulebook_from >= 0 ? stages[l]->rulebook_from : (int)l)];
                 if (pass <= waited) continue;
                 waited = pass;
+                if (pass <= kOwnWaits + 1) longer = pass - (int)l;
                 const int end = pass <= kOwnWaits ? pass : (last_side - pass <= kRest ? last_side : pass + kAhead);
                 for (int p = pass + 1; p <= end; ++p) {
                     if (p % 2 && !cs[(size_t)(p / 2)].builds.empty()) break;
@@ -408,11 +410,16 @@ struct Pipeline {
             }
             return SESSD_OK;
         };
-        // Of the two branches that begin here the one that is launched first follows at once in a graph, the other 6 us later.  That is
-        // the chain, except in FP32 frames of few points, whose layers are short beside the passes until the second strided layer:
-        // 2 000 points 199.2 us with the chain first, 192.6 with the passes, 4 000 213.6 and 212.6, 10 000 253.5 and 252.9, 80 000 444
-        // and 460; FP16 2 000 points 172.9 and 173.7, 10 000 181.6 and 184.1, 60 000 223.1 and 225.2.
-        const bool chain_first = desc.feature_dtype != SESSD_FLOAT || desc.max_points > 4096;
+        // Of the two branches that begin here the one that is launched first follows at once in a graph, the other 6 us later.  With few
+        // points a layer takes about as long as a pass, so that the longer one until the second strided layer's rulebook is the one with more
+        // launches: the passes in the reference's backbone in FP32 (five for five layers; in FP16, without tile cuts, four), the
+        // chain with four SubM layers in front of the first strided one.  Layers grow with the points and passes hardly.  Passes first /
+        // chain first, us, FP32 and FP16: 2 000 points 177.5 / 184.0, 164.2 / 166.1, 5 000 204.3 / 208.2, 170.3 / 168.7, 8 500 218.9 / 221.7,
+        // 172.8 / 171.0, 12 000 242.5 / 240.8, 177.8 / 174.4, 40 000 331.6 / 320.9, 206.5 / 205.3; one SubM layer in front 5 000 203.9 / 207.8,
+        // 165.9 / 169.1, 20 000 244.0 / 245.6, 177.3 / 177.7; four 2 000 189.8 / 182.8, 176.6 / 167.3, 10 000 256.3 / 252.5, 194.3 / 185.8; doubled
+        // widths, FP32 5 000 332.6 / 341.4, 20 000 478.4 / 476.3.  The points are those that the tensor holds, which is what the host
+        // knows: a frame of 2 000 points in a tensor for 20 000 takes 184.7, passes first it would be 177.7.
+        const bool chain_first = longer < 0 || desc.max_points > 10000;
         for (int i = 0; i <= m; ++i) {
             const Stage& sg = cs[(size_t)i];
             hipStream_t s = i == 0 ? stream : side;

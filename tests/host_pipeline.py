@@ -317,6 +317,21 @@ def check_waits():
     assert waits[at] == waits[at - 1] + 1, waits
 
 
+def check_order():
+    """Which of an overlapped frame's branches is launched first: with few points the one with more launches until the second strided
+    layer's rulebook, else the chain of layers."""
+    ref = B.reference_layers()
+    one = [B.Layer("subm0", D.SESSD_LAYER_SUBM, 4, 16, ref[0].out_shape)] + ref[2:]
+    four = ref[:2] + [ref[1]] * 2 + ref[2:]
+    f32, f16 = D.SESSD_FLOAT, D.SESSD_HALF
+    for layers, dtype, points, chain in ((ref, f32, 500, False), (ref, f32, 10000, False), (ref, f32, 10001, True), (ref, f16, 500, True),
+                                         (one, f32, 500, False), (one, f16, 500, False), (one, f16, 20000, True), (four, f32, 500, True),
+                                         (four, f16, 500, True), (deeper(2), f32, 500, False), (ref[:2], f32, 500, True)):
+        names = [l[1] for l in launches(overlapped_frame(layers, dtype, max_points=points))]
+        first = [i for i, n in enumerate(names) if "conv_" in n][0], [i for i, n in enumerate(names) if "number_cuts" in n][0]
+        assert (first[0] < first[1]) == chain, (len(layers), dtype, points, first)
+
+
 def gemm_kernel(cin, cout, rows, dtype):
     """The kernel that multiplies in a SubM layer of so many rows (nothing runs: the addresses are read by nobody)."""
     d = D.SubmConv3dDesc()
@@ -350,6 +365,7 @@ def check_row_limits():
 CHECKS = {
     "events": check_events,
     "waits": check_waits,
+    "order": check_order,
     "row-limits": check_row_limits,
     "recovery-direct": lambda: check_recovery(0, enqueue),
     "recovery-overlap": lambda: check_recovery(1, enqueue),

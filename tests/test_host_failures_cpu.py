@@ -52,3 +52,7 @@ def test_every_event_of_an_overlapped_frame_is_waited_for(fake_hip):
 
 def test_layers_of_a_deep_backbone_do_not_wait_for_the_whole_coordinate_branch(fake_hip):
     run_check(fake_hip, "waits")
+
+
+def test_the_longer_branch_of_a_small_frame_is_launched_first(fake_hip):
+    run_check(fake_hip, "order")
