@@ -504,16 +504,20 @@ __device__ __forceinline__ void sp_flags_pass(const SpPart& a, int block, int bl
 // A block of 64 rows at 17 262 rows: 11 900 cycles with four lanes a row (each lane a quarter of the offsets, their places found per
 // lane: 2 000 for seven keys) and the arguments read as they came, 6 100 now; the SubM plugin 64 -> 64 40.3 -> 37.9 us, frames of 2 000
 // points 205.5 -> 200.8, 20 000 306.9 -> 300.6, 60 000 (FP16) 250.7 -> 246.4.
+// HASH: some of the launch's tables are hashes.  The probes of a hash take 106 registers, which leaves the blocks no room beside three
+// workgroups of conv_wide<32,32> (3 x 144 of 512) or one of the 64-column kernels (2 x 216); dense tables alone take 48 and, with a row's
+// counts in bytes, 272 B of LDS of the 576 or more that those leave.  Frames, one launch for both / so: FP32 5 000 points 211.5 -> 209.2 us,
+// 40 000 332 -> 323, 80 000 418 -> 410, whose 61 440 rows and more in the second stage are two rounds of tiles; FP16 20 000 184.8 -> 181.0.
 constexpr int kLookupRows = 64;                             // rows of a block
 constexpr int kLookupDepth = (kGemmMaxOffsets + 3) / 4;     // offsets of a wave
 struct LookupLds {
-    int32_t found[kCoordBlock];  // by each wave for each row
+    uint8_t found[kCoordBlock];  // by each wave for each row (kLookupDepth at most)
     int32_t sum[4];              // ... for all of its rows
 };
 
 // What a wave finds for a row: val[j] = the row at the wave's j-th offset.  QUARTER 0 .. 3: of a 3x3x3 kernel on a dense table, where
 // the offsets are constants; -1: any (`start`: the first offset, z << 16 | y << 8 | x, `mine`: how many).
-template <int QUARTER>
+template <int QUARTER, bool HASH>
 __device__ __forceinline__ void look_up(const LookupPart& P, const int4& c, bool in_layer, int start, int mine, uint32_t (&val)[kLookupDepth]) {
     const int z0 = c.y * P.s[0] - P.p[0], y0 = c.z * P.s[1] - P.p[1], x0 = c.w * P.s[2] - P.p[2];
     const uint32_t origin = ((uint32_t)z0 * (uint32_t)P.t.gy + (uint32_t)y0) * (uint32_t)P.t.gx + (uint32_t)x0;
@@ -554,7 +558,7 @@ __device__ __forceinline__ void look_up(const LookupPart& P, const int4& c, bool
             }
         }
     }
-    if (P.t.dense) {
+    if (!HASH || P.t.dense) {
         const uint32_t* d = static_cast<const uint32_t*>(P.t.base);
 #pragma unroll
         for (int j = 0; j < kLookupDepth; ++j) val[j] = d[ok[j] ? key[j] : 0];
@@ -600,7 +604,7 @@ __device__ __forceinline__ void look_up(const LookupPart& P, const int4& c, bool
 }
 
 // CUBE: a 3x3x3 kernel on a dense table
-template <bool CUBE>
+template <bool CUBE, bool HASH>
 __device__ __forceinline__ void lookup_rows(const LookupPart& P, int block, int n, int start, int4 c, LookupLds& L) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int K = CUBE ? 27 : P.K, per = (K + 3) >> 2, k0 = wave * per, mine = K - k0 < per ? K - k0 : per;  // (mine may be negative: none)
@@ -609,11 +613,11 @@ __device__ __forceinline__ void lookup_rows(const LookupPart& P, int block, int 
         if (chunk != block) c = reinterpret_cast<const int4*>(P.coors)[row < n ? row : n - 1];
         const bool in_layer = row < n && (uint32_t)c.y < (uint32_t)P.own[0] && (uint32_t)c.z < (uint32_t)P.own[1] && (uint32_t)c.w < (uint32_t)P.own[2];
         uint32_t val[kLookupDepth];
-        if (!CUBE) look_up<-1>(P, c, in_layer, start, mine, val);
-        else if (wave == 0) look_up<0>(P, c, in_layer, 0, 0, val);
-        else if (wave == 1) look_up<1>(P, c, in_layer, 0, 0, val);
-        else if (wave == 2) look_up<2>(P, c, in_layer, 0, 0, val);
-        else look_up<3>(P, c, in_layer, 0, 0, val);
+        if (!CUBE) look_up<-1, HASH>(P, c, in_layer, start, mine, val);
+        else if (wave == 0) look_up<0, HASH>(P, c, in_layer, 0, 0, val);
+        else if (wave == 1) look_up<1, HASH>(P, c, in_layer, 0, 0, val);
+        else if (wave == 2) look_up<2, HASH>(P, c, in_layer, 0, 0, val);
+        else look_up<3, HASH>(P, c, in_layer, 0, 0, val);
         int cnt = 0, sum = 0;
         int32_t* to = P.nbr + (size_t)k0 * P.max_voxels + row;
 #pragma unroll
@@ -626,7 +630,7 @@ __device__ __forceinline__ void lookup_rows(const LookupPart& P, int block, int 
         }
         if (P.w) {
             __syncthreads();
-            L.found[threadIdx.x] = cnt;
+            L.found[threadIdx.x] = (uint8_t)cnt;
             if (lane == 0) L.sum[wave] = sum;
             __syncthreads();
             if (wave == 0) {
@@ -639,6 +643,7 @@ __device__ __forceinline__ void lookup_rows(const LookupPart& P, int block, int 
     }
 }
 
+template <bool HASH>
 __device__ __forceinline__ void lookup_pass(const LookupPart& a, int block, LookupLds& L) {
     const LookupPart P = a;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), start = a.first[wave];
@@ -649,8 +654,8 @@ __device__ __forceinline__ void lookup_pass(const LookupPart& a, int block, Look
     const int n = __builtin_amdgcn_readfirstlane(clamp_rows(P.num, P.max_voxels));
     if (P.meta && block == 0 && threadIdx.x == 0) P.meta[1] = n;
     if (block * kLookupRows >= n) return;
-    if (P.t.dense && P.k[0] == 3 && P.k[1] == 3 && P.k[2] == 3) lookup_rows<true>(P, block, n, start, c, L);
-    else lookup_rows<false>(P, block, n, start, c, L);
+    if (P.t.dense && P.k[0] == 3 && P.k[1] == 3 && P.k[2] == 3) lookup_rows<true, HASH>(P, block, n, start, c, L);
+    else lookup_rows<false, HASH>(P, block, n, start, c, L);
 }
 
 struct FlagsLookups {
@@ -660,13 +665,14 @@ struct FlagsLookups {
 
 // end1 .. end3: where the blocks of the lookups behind the first begin.  (Arguments of their own: those are in registers when the
 // kernel starts.)
+template <bool HASH>
 __global__ void __launch_bounds__(kCoordBlock) flags_lookups(int flag_blocks, int end1, int end2, int end3, FlagsLookups a) {
     __shared__ LookupLds L;
     const int b = blockIdx.x;
     if (b < flag_blocks) return sp_flags_pass(a.flags, b, flag_blocks, reinterpret_cast<uint32_t*>(L.sum));
     const int l = __builtin_amdgcn_readfirstlane((b >= end1 ? 1 : 0) + (b >= end2 ? 1 : 0) + (b >= end3 ? 1 : 0));
     static_assert(kMaxLookups == 4, "one argument for each lookup but the first");
-    lookup_pass(a.look[l], b - (l == 0 ? flag_blocks : (l == 1 ? end1 : (l == 2 ? end2 : end3))), L);
+    lookup_pass<HASH>(a.look[l], b - (l == 0 ? flag_blocks : (l == 1 ? end1 : (l == 2 ? end2 : end3))), L);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -997,7 +1003,10 @@ int launch_flags_lookups(const SpPart* flags, const LookupPart* lookups, int n, 
         end[l] = blocks;
     }
     if (!blocks) return SESSD_OK;
-    hipLaunchKernelGGL(flags_lookups, dim3(blocks), dim3(kCoordBlock), 0, stream, flag_blocks, end[0], end[1], end[2], a);
+    bool hash = false;  // (the flags read either kind of table)
+    for (int l = 0; l < n; ++l) hash = hash || !lookups[l].t.dense;
+    if (hash) hipLaunchKernelGGL(flags_lookups<true>, dim3(blocks), dim3(kCoordBlock), 0, stream, flag_blocks, end[0], end[1], end[2], a);
+    else hipLaunchKernelGGL(flags_lookups<false>, dim3(blocks), dim3(kCoordBlock), 0, stream, flag_blocks, end[0], end[1], end[2], a);
     SESSD_HIP_TRY(hipGetLastError());
     return SESSD_OK;
 }

@@ -5,6 +5,7 @@
 """
 import ctypes as C
 import os
+import re
 import sys
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -220,6 +221,7 @@ def check_short_memory():
     bytes_of = lambda h: L.sessd_pipeline_device_bytes(h)  # noqa: E731
     rc, h = create()
     assert rc == 0
+    assert not any("flags_lookupsILb1" in l[1] for l in launches_of(enqueue, h, new_stream()))
     full = bytes_of(h)
     kept = []
     for limit in (300 << 20, 40 << 20):
@@ -233,7 +235,11 @@ def check_short_memory():
         take_log()
         for _ in range(2):  # (an error left pending by the allocation would fail the first)
             assert enqueue(h, stream) == 0, L.sessd_last_error()
-            assert not unordered(take_log())
+            log = take_log()
+            assert not unordered(log)
+        # lookups that need a hash run on the kernel that knows it, the others on the one that leaves room beside the GEMMs
+        hashes = [bool(int(re.search(r"flags_lookupsILb(\d)", l[1]).group(1))) for l in log if "flags_lookups" in l[1]]
+        assert hashes == [True, True, len(kept) == 2, False, False], hashes
     voxels, strided = 40 * 1600 * 1408 * 4, 21 * 800 * 704 * 4
     assert voxels < kept[0] < voxels + 4096 and voxels + strided < kept[1] < voxels + strided + 2 * 4096, kept
     FAKE.fake_largest_allocation(1000)
