@@ -638,6 +638,26 @@ def test_sparse_generic_stride1_and_corner_truncation():
         assert_features_close(out, O.gather_gemm_scatter(feat, w, o_pairs, o_num, mv), RTOL_FP32, str((k, s, p)))
 
 
+@pytest.mark.parametrize("less", [0, 1])
+@pytest.mark.parametrize("padding", [(2, 2, 2), (2, 0, 1), (0, 2, 1), (1, 1, 2)])
+def test_sparse_kernels_of_3_with_strides_of_2(padding, less):
+    """Candidates that are found without a division, for every padding up to 2, grids of even and odd size, and an output grid that the
+    last candidates lie outside of."""
+    k, s, rng = (3, 3, 3), (2, 2, 2), np.random.default_rng(7)
+    for ig in ((6, 9, 8), (7, 12, 11)):
+        og = tuple(B.conv_out_size(ig[a], k[a], s[a], padding[a]) - less for a in range(3))
+        layer = B.Layer("t", D.SESSD_LAYER_SPARSE, 8, 16, og[::-1], k, s, padding)
+        n, mv = ig[0] * ig[1] * ig[2] // 2, 1024
+        coors = F.random_active_voxels(n, ig, 6)
+        feat = rng.uniform(-1, 1, (n, 8)).astype(np.float32)
+        w = rng.normal(0, 0.1, (27, 8, 16)).astype(np.float32)
+        conv, out, oc, on, pairs, num = run_sparse(layer, coors, n, feat, w, mv, ig)
+        o_pairs, o_num, o_oc, o_on, o_st = O.sparse_rulebook(coors, n, og[::-1], k, s, padding, mv)
+        assert conv.status() == o_st
+        assert on == o_on and np.array_equal(oc, o_oc) and np.array_equal(num, o_num), ig
+        assert_features_close(out, O.gather_gemm_scatter(feat, w, o_pairs, o_num, mv), RTOL_FP32, str((ig, padding)))
+
+
 def test_sparse2dense_with_folded_zero_pad():
     # sparse2Dense followed by ZeroPad2dPlugin (se-ssd-ai-trt.cpp:1253) in one scatter; a copy: bit-exact
     rng = np.random.default_rng(12)
@@ -989,9 +1009,9 @@ def _fp32_subm_wide_against_oracle(n, mv, grid, seed, clustered=True, epilogue=T
 @pytest.mark.parametrize("cin", [64, 32])
 @pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 95, 96, 97, 255, 256, 257, 1000])
 def test_wide_fp32_kernel_row_counts_around_its_tiles(n, cin):
-    """One workgroup per compute unit walks tiles of up to 96 rows whose neighbour lists are staged in two halves
-    of 64 rows: row counts on either side of a 16-pair block, the staging halves, the tile capacity and the number
-    of compute units (256 rows: one row per tile), against the oracle (pad rows included)."""
+    """Few rows: tiles of one row to eight on 256 compute units, fewer rows than tiles, as many, and one more; two workgroups share
+    the columns of each.  (Tiles whose lists fill their two halves of 64 rows are in the tests below.)  Against the oracle (pad rows
+    included)."""
     _fp32_subm_wide_against_oracle(n, n + 200, (5, 40, 40), 700 + n, epilogue=(n % 2 == 1), cin=cin)
 
 
@@ -1088,11 +1108,7 @@ def test_wide_fp32_kernel_with_128_columns(n, cin):
     conv.close()
 
 
-@pytest.mark.parametrize("cin,cout", [(4, 16), (4, 32), (16, 16), (16, 32), (32, 32)])
-@pytest.mark.parametrize("n", [1, 16, 63, 65, 113, 129, 16385, 28672, 28673, 40000])
-def test_wide_fp32_kernel_with_few_columns(n, cin, cout):
-    """16 and 32 output columns: tiles of up to 128 (64, from 32 channels 80) rows, one workgroup per compute unit up to 256 full tiles,
-    two, three or four beyond.  Against the oracle (pad rows included)."""
+def _fp32_subm_with_few_columns_against_oracle(n, cin, cout):
     rng = np.random.default_rng(n + cin)
     grid, mv = ((5, 40, 40) if n < 1000 else (21, 400, 352)), n + 39
     coors = F.clustered_active_voxels(n, grid, n, n_blobs=max(4, n // 100))
@@ -1110,6 +1126,23 @@ def test_wide_fp32_kernel_with_few_columns(n, cin, cout):
     assert_features_close(out, o_out, RTOL_FP32, "fp32 %d->%d, %d rows" % (cin, cout, n),
                           abs_sum=abs_sum_of(feat, w, o_pairs, o_num, mv, mv, sc, sh))
     conv.close()
+
+
+@pytest.mark.parametrize("cin,cout", [(4, 16), (4, 32), (16, 16), (16, 32), (32, 32)])
+@pytest.mark.parametrize("n", [1, 16, 63, 65, 113, 129, 16385, 28672, 28673, 40000])
+def test_wide_fp32_kernel_with_few_columns(n, cin, cout):
+    """16 and 32 output columns: few rows, row counts around a tile's, and some thousands.  Against the oracle (pad rows included)."""
+    _fp32_subm_with_few_columns_against_oracle(n, cin, cout)
+
+
+@pytest.mark.parametrize("cin,cout,rows,groups", [(4, 16, 128, 2), (16, 16, 128, 2), (4, 32, 64, 4), (16, 32, 64, 2), (32, 32, 80, 3)])
+def test_wide_fp32_kernel_around_its_workgroups_per_compute_unit(cin, cout, rows, groups):
+    """16 and 32 output columns: one workgroup per compute unit while tiles of `rows` rows hold the layer, up to `groups` beyond, then a
+    second round of tiles: the row counts on both sides of each of these lines.  Against the oracle (pad rows included)."""
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    for held in range(1, groups + 1):
+        for n in (units * rows * held, units * rows * held + 1):
+            _fp32_subm_with_few_columns_against_oracle(n, cin, cout)
 
 
 @pytest.mark.parametrize("cout", [16, 32])

@@ -507,14 +507,16 @@ def test_a_frame_in_the_callers_own_graph_finds_its_tables_empty(overlap):
         assert_end_to_end_close(to_np(dense), ref["dense"], False, "dense, step %d" % step)
 
 
-def test_dozens_of_strided_layers():
-    """More strided layers than the clears of one launch can hold; two frames, the second smaller."""
+@pytest.mark.parametrize("schedule", [{}, dict(overlap_streams=True), dict(overlap_streams=True, use_graph=True)], ids=["one", "two", "graph"])
+def test_dozens_of_strided_layers(schedule):
+    """More strided layers than the clears of one launch can hold, on one stream and with the coordinate branch on another; two frames,
+    the second smaller."""
     layers = B.reference_layers()
     grid = layers[-2].out_shape
     layers[-1:-1] = [B.Layer("s%d" % i, D.SESSD_LAYER_SPARSE, 64, 64, grid, (3, 1, 1), (1, 1, 1), (1, 0, 0)) for i in range(46)]
     W = B.random_weights(layers, seed=13, w_std=0.05)
     mp, mv = 512, 8000
-    pipe = api.Pipeline(layers, W, mp, mv, share_rulebooks=True)
+    pipe = api.Pipeline(layers, W, mp, mv, share_rulebooks=True, **schedule)
     dense, stream = pipe.new_dense(), torch.cuda.Stream()
     for step, npts in enumerate((400, 250)):
         pts = F.lidar_frame(npts, 90 + step)
