@@ -14,9 +14,10 @@
  *
  * Tensor contract (same as the reference): every tensor is linear, batch dimension 1, device
  * memory owned by the caller; `voxel_num` / `points_size` are int32 scalars in DEVICE memory and
- * are only read inside kernels.  enqueue only enqueues work on `stream` (a hipStream_t); it never
- * synchronises, allocates or frees.  Outputs and workspace are (re)initialised inside every
- * enqueue.  Return value 0 = success, anything else is a SESSD_E_* code (the reference aborts).
+ * are only read inside kernels.  A tensor has all the rows that its descriptor names: those beyond the active ones (or
+ * beyond points_size) may hold anything, may be read and do not count.  enqueue only enqueues work on `stream` (a
+ * hipStream_t); it never synchronises, allocates or frees.  Outputs and workspace are (re)initialised inside every enqueue.
+ * Return value 0 = success, anything else is a SESSD_E_* code (the reference aborts).
  *
  * All plain C: no HIP, torch or C++ types appear in any signature.
  */

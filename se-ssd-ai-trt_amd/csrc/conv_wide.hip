@@ -43,8 +43,8 @@
 // together a launch is two rounds of tiles, of which the second costs its lists and sums again; the tiles are therefore as high, or the
 // workgroups as many, as the LDS takes: 16 columns 2 x 128 rows (60 000 rows, 4 -> 16 12.7 -> 10.3 us, 16 -> 16 15.2 -> 12.4 against 2 x 112),
 // 4 -> 32 4 x 64 (54 613 rows 16.2 -> 12.7 against 2 x 64), 32 -> 32 3 x 80 (40 088 rows 26.1 -> 21.5, 60 727 33.3 -> 28.4 against 2 x 64; frames of
-// 40 000 points 363 -> 351, of 80 000, whose coordinate passes miss the LDS, 428 -> 431).  What LDS they leave is what the
-// coordinate passes of a frame's other branch run in: 32 -> 32 with eight waves is the faster launch (15.9 us against 17.1 at
+// 40 000 points 331 -> 324; of 80 000 398 and 405 where the rows are more than the 61 440 that three workgroups a unit hold, the same where
+// they are fewer).  What LDS and registers they leave is what the coordinate passes of a frame's other branch run in: 32 -> 32 with eight waves is the faster launch (15.9 us against 17.1 at
 // 28 043 rows) and makes the slower frame (20 000 points: 283 us against 274); 4 -> 32 likewise (487 against 475).  16 -> 32 with four waves and
 // 3 x 80 rows: 54 613 rows 18.4 -> 17.4 us, but 17 132 rows 9.0 -> 11.4.
 // FP16 features (Cin 16) have so little in each block that four waves and 64 rows do: four workgroups share a unit, with 40 KB of LDS

@@ -13,8 +13,8 @@
 // A pass that creates rows (vg_finalize, sp_number) holds their coordinates and numbers in registers: it inserts the
 // next strided layer's tickets right away, and what only needs finished tables (lookups, cuts) shares a launch with the
 // next step of the chain.  For the reference's backbone that is 13 launches a frame in place of 35.
-// Measured (a graph of the coordinate passes alone, us): frames of 2 000 points 141 -> 79, 20 000 164 -> 97, 80 000 231 ->
-// 127, 60 000 (FP16 configuration) 162 -> 111, 150 000 221 -> 147.  A pass is bound by its chain of dependent trips to
+// Measured (frames without their GEMMs, us; 35 launches, 13, 13 as they are now): 2 000 points 141, 79, 62, 20 000 164, 97, 72, 80 000
+// 231, 127, 95, 60 000 (FP16 configuration) 162, 111, 84, 150 000 221, 147, 111.  A pass is bound by its chain of dependent trips to
 // memory (four to six of 0.7-1 us each) until some 40 000 rows, and by random accesses beyond.
 #include "coord.h"
 #include "fill.h"
