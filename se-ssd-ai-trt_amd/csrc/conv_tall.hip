@@ -320,13 +320,19 @@ conv_tall(const int32_t* __restrict__ num_out, const int32_t* __restrict__ nbr, 
         tall_tile<CIN, COUT, RB>(in, out, Wp, nbr, n, b * kTall, max_voxels, scale, shift, relu, dt, s_nbr, s_epi);
     else
         tall_tile<CIN, COUT, 1>(in, out, Wp, nbr, n, n_tall * kTall + (b - n_tall) * kShort, max_voxels, scale, shift, relu, dt, s_nbr, s_epi);
-    if (write_pad) {
-        if (threadIdx.x < COUT) {  // (a workgroup may have had no tile)
+    // The rows beyond the active ones are the business of the workgroups without a tile: the grid has one for every 64 rows.
+    const int tiles = n_tall + (n > n_tall * kTall ? (n - n_tall * kTall + kShort - 1) / kShort : 0);
+    const int idle = (int)gridDim.x - tiles;
+    if (write_pad && (b >= tiles || idle == 0)) {
+        if (threadIdx.x < COUT) {
             s_epi[threadIdx.x] = scale ? scale[threadIdx.x] : 1.f;
             s_epi[COUT + threadIdx.x] = shift ? shift[threadIdx.x] : 0.f;
         }
         __syncthreads();
-        write_pad_rows<__half, COUT, kWaves * 64>(out, n, max_voxels, s_epi, scale != nullptr, shift != nullptr, relu);
+        const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+        PadRows<__half, COUT> pads(out, n, max_voxels, (unsigned)((idle ? b - tiles : b) * kWaves + wave), (unsigned)((idle ? idle : (int)gridDim.x) * kWaves));
+        pads.layer(s_epi, scale != nullptr, shift != nullptr, relu);
+        pads.rest();
     }
 }
 

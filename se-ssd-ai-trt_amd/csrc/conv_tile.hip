@@ -113,10 +113,10 @@ __device__ __forceinline__ void store4h(__half* dst, const float (&o)[4]) {
     *reinterpret_cast<uint2*>(dst) = p.u;
 }
 
-template <int CIN, int COUT, int KC, int MF>
+template <int CIN, int COUT, int KC, int MF, typename Pads>
 __device__ __forceinline__ void run_tile(const v4i& rs_in, const v4i& rs_w, const v4i& rs_nbr, unsigned nbr_stride,
                                          __half* __restrict__ out, int row0, int row_end, bool has_scale, bool has_shift, int relu,
-                                         const DenseTarget& dt, unsigned char* pool, const float* s_epi) {
+                                         const DenseTarget& dt, unsigned char* pool, const float* s_epi, Pads& pads) {
     using C = Shape<CIN, COUT, KC>;
     constexpr int H = C::U * MF;
     constexpr int R = C::ring(MF);
@@ -242,8 +242,12 @@ __device__ __forceinline__ void run_tile(const v4i& rs_in, const v4i& rs_w, cons
     int at = 0;  // the stage in use
     stage_barrier();
     read(0, 0, f0);
+    constexpr bool kPads = KC > 3;  // (three offsets are unrolled, and the registers full)
+    if constexpr (kPads) pads.layer(s_epi, has_scale, has_shift, relu);
     for (int s = 0; s < C::S; ++s) {
         step(f0, f1, at, 1);
+        if constexpr (kPads)
+            if (pads.left()) pads.step();  // (these waves wait for no other request in the loop)
         stage_barrier();  // the stage in use is read, the next one complete
         at += C::stage_bytes(MF);
         at = at == R * C::stage_bytes(MF) ? 0 : at;
@@ -290,11 +294,13 @@ __device__ __forceinline__ void run_tile(const v4i& rs_in, const v4i& rs_w, cons
     __syncthreads();
 }
 
-template <int CIN, int COUT, int KC>
+// PAD: the rows beyond the active ones are written too.  A variant of its own: in the launches of a frame without, its registers are what
+// the coordinate passes beside them run in (frames of 60 000 points 231 us, with one kernel for both 235).
+template <int CIN, int COUT, int KC, bool PAD>
 __global__ void __launch_bounds__(kThreads, 2)
 conv_tile(const __half* __restrict__ in, __half* __restrict__ out, const void* __restrict__ Wp,
           const int32_t* __restrict__ nbr, const int32_t* __restrict__ num_out, int max_voxels,
-          const float* __restrict__ scale, const float* __restrict__ shift, int relu, int write_pad, DenseTarget dt) {
+          const float* __restrict__ scale, const float* __restrict__ shift, int relu, DenseTarget dt) {
     using C = Shape<CIN, COUT, KC>;
     static_assert(CIN % 64 == 0 && COUT % 16 == 0, "whole MFMA chunks");
     __shared__ __align__(1024) unsigned char pool[kPool];
@@ -316,6 +322,11 @@ conv_tile(const __half* __restrict__ in, __half* __restrict__ out, const void* _
     const v4i rs_w = make_rsrc(Wp, (unsigned)(C::S * C::kWeightBytes));
     const v4i rs_nbr = make_rsrc(nbr, (unsigned)((size_t)KC * max_voxels * sizeof(int32_t)));
     const bool hs = scale != nullptr, hb = shift != nullptr;
+    const unsigned wave = __builtin_amdgcn_readfirstlane((unsigned)tid >> 6);
+    auto pads = [&]() {
+        if constexpr (PAD) return PadRows<__half, COUT>(out, n, max_voxels, blockIdx.x * kWaves + wave, gridDim.x * kWaves);  // (by the waves that multiply)
+        else return NoPadRows();
+    }();
     // the first tile's row: up to one round, tile t goes to workgroup t / each + 8 * (t % each)
     auto first = [&](int h) {
         const int t = (n + h - 1) / h, each = (t + 7) / 8, x = blockIdx.x & 7, j = blockIdx.x >> 3;
@@ -326,7 +337,7 @@ conv_tile(const __half* __restrict__ in, __half* __restrict__ out, const void* _
         if constexpr (MF <= C::kMaxMf)
             for (int row0 = first(C::U * MF); row0 < n; row0 += slots * (C::U * MF))
                 run_tile<CIN, COUT, KC, MF>(rs_in, rs_w, rs_nbr, (unsigned)max_voxels * 4u, out, row0,
-                                            row0 + C::U * MF < n ? row0 + C::U * MF : n, hs, hb, relu, dt, pool, s_epi);
+                                            row0 + C::U * MF < n ? row0 + C::U * MF : n, hs, hb, relu, dt, pool, s_epi, pads);
     };
     switch (mf) {
         case 1: tiles(std::integral_constant<int, 1>{}); break;
@@ -337,9 +348,12 @@ conv_tile(const __half* __restrict__ in, __half* __restrict__ out, const void* _
         case 6: tiles(std::integral_constant<int, 6>{}); break;
         default: break;  // no rows
     }
-    if (write_pad) {
-        __syncthreads();
-        write_pad_rows<__half, COUT, kThreads>(out, n, max_voxels, s_epi, hs, hb, relu);
+    if constexpr (PAD) {
+        __syncthreads();  // (a workgroup may have had no tile)
+        if (wave < kWaves) {
+            pads.layer(s_epi, hs, hb, relu);
+            pads.rest();
+        }
     }
 }
 
@@ -347,9 +361,12 @@ template <int CIN, int COUT, int KC>
 int launch(const GemmArgs& a, hipStream_t stream) {
     if ((size_t)a.max_voxels * (CIN * sizeof(__half)) >= kOutOfRange) return SESSD_E_UNSUPPORTED;
     if ((size_t)a.max_voxels * (KC * sizeof(int32_t)) >= kOutOfRange) return SESSD_E_UNSUPPORTED;
-    hipLaunchKernelGGL((conv_tile<CIN, COUT, KC>), dim3(gemm_compute_units()), dim3(kThreads), 0, stream,
-                       static_cast<const __half*>(a.in_feat), static_cast<__half*>(a.out_feat), a.w_packed, a.nbr,
-                       a.num_out, a.max_voxels, a.scale, a.shift, a.relu, a.write_pad_rows, a.dense);
+    auto go = [&](auto pad) {
+        hipLaunchKernelGGL((conv_tile<CIN, COUT, KC, decltype(pad)::value>), dim3(gemm_compute_units()), dim3(kThreads), 0, stream,
+                           static_cast<const __half*>(a.in_feat), static_cast<__half*>(a.out_feat), a.w_packed, a.nbr, a.num_out,
+                           a.max_voxels, a.scale, a.shift, a.relu, a.dense);
+    };
+    a.write_pad_rows ? go(std::true_type{}) : go(std::false_type{});
     SESSD_HIP_TRY(hipGetLastError());
     return SESSD_OK;
 }

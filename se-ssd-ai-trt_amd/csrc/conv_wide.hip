@@ -242,9 +242,9 @@ __device__ __forceinline__ void unrolled(F f, std::integer_sequence<int, N...>) 
 // One wave's share of a tile: the pairs of the offsets dealt to it, times its columns -- 16-column blocks nb0 .. nb0 + NB - 1
 // of the layer -- into its partial tile `part` (rows of 16 NB floats).  waves: among which the offsets are dealt; most: blocks that an
 // offset can have in this tile; spare: a row for what filling pairs add.
-template <typename S, int COUT, int NB>
+template <typename S, int COUT, int NB, typename Pads>
 __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_buffer_rsrc_t rs_w, const uint32_t* s_pair,
-                                         const int32_t* s_blk, int K, int wave, int waves, int lane, int nb0, int most, float* part, float* spare) {
+                                         const int32_t* s_blk, int K, int wave, int waves, int lane, int nb0, int most, float* part, float* spare, Pads& pads) {
     using P = Products<S, NB, S::kArith>;
     constexpr int kParts = S::kParts, G = S::G, E = S::kLaneBytes / 4, kTileRows = S::kTileRows;
     constexpr int kSets = P::kPieces * NB * E > 64 ? 1 : 2;  // of weights: the registers do not hold two of the largest
@@ -376,6 +376,7 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
             if (request) load_b(__builtin_amdgcn_readlane(stage_at, stage + 1), fill);
             // (behind the weights in either case: what the waits count is then the same for every item)
             load_a(d2, next_entry, a);
+            pads.step();  // (behind what the next item waits for)
             if (mine < kNoPair) {
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) {
@@ -433,6 +434,7 @@ __device__ __forceinline__ void multiply(__amdgpu_buffer_rsrc_t rs_in, __amdgpu_
                         for (int e = 0; e < E; ++e) row[g][e] = __builtin_amdgcn_ds_bpermute(from_lane4, a[g][e]);
                     if constexpr (request.value && kSets == 2) load_b(__builtin_amdgcn_readlane(stage_at, stage + 1), fill);
                     load_a(d2, next_entry, a);
+                    pads.step();  // (behind what the next item waits for)
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }, std::make_integer_sequence<int, P::kSteps>{});
@@ -564,6 +566,10 @@ conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles
     if (cut_count == 0) plan = tile_plan(n, walkers, kMaxSplit && lsplit ? kTileRows : S::kWholeRows);
     const int tile_count = cut_count > 0 ? cut_count : (n > 0 ? plan.count : 0);
     bool idle = true;  // (no rows)
+    auto pads = [&]() {
+        if constexpr (PAD) return PadRows<TO, COUT>(out, n, max_voxels, blockIdx.x * kWaves + own_wave, gridDim.x * kWaves);
+        else return NoPadRows();
+    }();
     for (int tile = first_tile; tile < tile_count; tile += walkers) {
     int run_begin, run_end;
     if (cut_count > 0) {
@@ -660,9 +666,11 @@ conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles
         s_epi[2 * COUT + tid] = epi_col;
     }
     __syncthreads();
+    pads.layer(s_epi, scale != nullptr, shift != nullptr, relu);
     if constexpr (kMaxSplit)
-        if (split) multiply<S, COUT, kWgCols / 32>(rs_in, rs_w, s_pair, s_blk, volume, wave, waves, lane, col_first / 16, (rows + 15) >> 4, part, s_part + S::kPartRows * kWgCols);
-    if (!kMaxSplit || !split) multiply<S, COUT, kWgCols / 16>(rs_in, rs_w, s_pair, s_blk, volume, wave, waves, lane, col_first / 16, (rows + 15) >> 4, part, s_part + S::kPartRows * kWgCols);
+        if (split) multiply<S, COUT, kWgCols / 32>(rs_in, rs_w, s_pair, s_blk, volume, wave, waves, lane, col_first / 16, (rows + 15) >> 4, part, s_part + S::kPartRows * kWgCols, pads);
+    if (!kMaxSplit || !split) multiply<S, COUT, kWgCols / 16>(rs_in, rs_w, s_pair, s_blk, volume, wave, waves, lane, col_first / 16, (rows + 15) >> 4, part, s_part + S::kPartRows * kWgCols, pads);
+    pads.rest();
     __syncthreads();
 
     // fixed-order sum of the waves' partial tiles, epilogue, coalesced stores; the sums of kAtOnce vectors are read together
@@ -756,13 +764,14 @@ conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles
     __syncthreads();  // the next piece reuses the lists and partial tiles
     }
     }
-    if constexpr (PAD) {
-        if (idle && thread < COUT) {  // (no tile has staged them)
+    if (PAD && idle) {  // (no tile has staged scale and shift)
+        if (thread < COUT) {
             s_epi[thread] = scale ? scale[thread] : 1.f;
             s_epi[COUT + thread] = shift ? shift[thread] : 0.f;
         }
         __syncthreads();
-        write_pad_rows<TO, COUT, kThreads>(out, n, max_voxels, s_epi, scale != nullptr, shift != nullptr, relu);
+        pads.layer(s_epi, scale != nullptr, shift != nullptr, relu);
+        pads.rest();
     }
 }
 

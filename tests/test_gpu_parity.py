@@ -1083,6 +1083,35 @@ def test_every_row_is_a_pad_row(cin, cout, half):
         conv.close()
 
 
+@pytest.mark.parametrize("cin,cout,half", [(4, 16, False), (16, 32, False), (32, 32, False), (64, 64, False), (128, 128, False), (16, 16, True),
+                                           (32, 32, True), (32, 64, True), (64, 64, True), (128, 128, True)])
+def test_pad_rows_beside_the_products(cin, cout, half):
+    """Rows beyond the active ones are written while a launch multiplies: one of them, fewer than the launch has waves, more than it has
+    steps for, and none left for the workgroups without a tile.  The active rows come out as in a tensor with none or few, bit for bit."""
+    rng = np.random.default_rng(cin + cout)
+    grid = (11, 200, 176)
+    coors = F.clustered_active_voxels(12000, grid, 1, n_blobs=60)
+    w = rng.normal(0, 0.1, (27, cin, cout)).astype(np.float32)
+    sc, sh = rng.uniform(0.5, 1.5, cout).astype(np.float32), rng.uniform(-0.5, 0.5, cout).astype(np.float32)
+    dtype = np.float16 if half else np.float32
+    feat = rng.uniform(0, 1, (12000, cin)).astype(dtype)
+
+    def rows(n, mv):
+        conv = api.SubmConv3d(cin, cout, grid[::-1], w, mv)
+        conv.set_epilogue(sc, sh, relu=True)
+        f, c = np.zeros((mv, cin), dtype), np.zeros((mv, 4), np.int32)
+        f[:n], c[:n] = feat[:n], coors[:n]
+        y = to_np(conv(dev(f), dev(c), dev(np.array([n], np.int32))))
+        conv.close()
+        return y
+
+    for n, more in ((1, 1), (639, 1), (640, 3), (640, 131), (12000, 1), (12000, 9000), (300, 150000)):
+        y = rows(n, n + more)
+        few = n if n + more <= 8192 else max(n, 8193)  # (beyond 8 192 rows a rulebook has cuts, by which sums are ordered)
+        assert np.array_equal(y[:n], rows(n, few)[:n]), (n, more)
+        assert np.array_equal(y[n:], np.broadcast_to(np.maximum(sh, 0).astype(dtype), (more, cout))), (n, more)
+
+
 @pytest.mark.parametrize("cin", [64, 128])
 @pytest.mark.parametrize("n", [1, 65, 97, 1536, 1537, 3840, 3841, 5120, 5121, 12289, 20000])
 def test_wide_fp32_kernel_with_128_columns(n, cin):
