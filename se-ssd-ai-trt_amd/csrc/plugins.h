@@ -156,6 +156,8 @@ class SubmConv3dLayerPlugin : public ConvPluginBase {
                       const void* rulebook_workspace, hipStream_t stream);
     // enqueue = enqueueBuild (coordinates -> rulebook) + enqueueGemm (features)
     int enqueueBuild(const int32_t* coors, const int32_t* voxel_num, void* workspace, hipStream_t stream);
+    bool runsInOne() const;
+    int enqueueInOne(const void* in_feat, const int32_t* coors, const int32_t* voxel_num, void* out_feat, void* workspace, hipStream_t stream);
     // The rulebook from a table that some earlier pass has already built over this layer's grid (the voxelizer's, or
     // that of the strided layer that produced `coors`), opened with cells_num (at most cells_max) rows.  The header
     // words (collectHeaderFill) must have been cleared once.

@@ -45,7 +45,7 @@ subm_insert(const int32_t* __restrict__ coors, const int32_t* __restrict__ voxel
 // cells: a row enters with one minimum and, where cells collide, one exchange (the probes of an open table, each waiting for the one
 // before, took 8 us for 2 000 rows).  Rows that name one cell are in no list: as one, which each of them walked, 8 192 of them were
 // a layer of 882 us, 17 now.  What bounds it are two trips to memory and the launch.  Layer 4 -> 16, three launches before and this: 300 rows 19.0 -> 11.4
-// us, 2 000 18.6 -> 11.5, 8 000 19.5 -> 13.0; 64 -> 64 with 8 000 rows 26.4 -> 22.  The line lies where the table still fits LDS: 8 192 rows and
+// us, 2 000 18.6 -> 11.5, 8 000 19.5 -> 13.0 (then with a launch for the products); 64 -> 64 with 8 000 rows 26.4 -> 22.  The line lies where the table still fits LDS: 8 192 rows and
 // their lists, 128 KB.  It is drawn at the tensors' capacity, which is what the host knows when it launches.
 constexpr int kSmallRows = 8192;
 constexpr int kSmallHeads = 16384;
@@ -55,12 +55,59 @@ constexpr int kSmallOwn = kSmallRows / kSmallBlock;                             
 constexpr int kSmallDepth = (kGemmMaxOffsets + kSmallWaves - 1) / kSmallWaves;  // offsets that it looks up
 static_assert(kSmallRows < 0xffff, "rows in 16 bits beside kNoRow");
 
+// The layer behind such a rulebook where its products are plain FP32 and few: the workgroup that has looked up the neighbours of its 64
+// rows multiplies them as well.  What bounds a call of two launches is the host, which takes 3.4 us for each, from 2 000 rows up the
+// GPU, where the second one's trips to memory (row count, lists, rows) are gone but for the rows.  A wave takes 16 of the rows and a
+// quarter of the offsets, whose weights it has asked for in front of everything else; an absent neighbour's product is left out behind
+// the MFMA (0 x infinity).  An offset's products are summed by themselves, the sums of offsets and of the four quarters two by two.
+// Two launches / one, a call: 4 -> 16 at 300 rows 10.9 / 8.1 us, 2 000 10.9 / 7.8, 8 000 13.9 / 11.0; 4 -> 32 10.8 / 7.7, 11.9 / 8.5,
+// 15.9 / 11.6; 16 -> 16 11.0 / 8.2, 11.0 / 9.1, 14.7 / 12.0.  Not 16 -> 32, 10.9 / 11.7, 11.5 / 12.8, 15.9 / 16.2: every 64 rows wait for 54 KB
+// of weights, and the registers spill.  Distance from 64-bit sums at 2 000 rows 3.58e-8 / 3.58e-8, 3.53e-8 / 3.53e-8, 6.04e-8 / 6.04e-8.
+struct SmallGemm {
+    const float* in = nullptr;
+    float* out = nullptr;
+    const float* w = nullptr;  // operand order (pack_weights())
+    const float* scale = nullptr;
+    const float* shift = nullptr;
+    int relu = 0, write_pad = 0;
+};
+constexpr int kSmallQuarters = 4, kSmallQuarter = (kGemmMaxOffsets + kSmallQuarters - 1) / kSmallQuarters;  // offsets of a quarter
+static_assert(kSmallWaves == 4 * kSmallQuarters, "a wave for each 16 rows and quarter");
+
+__device__ __forceinline__ void small_operand(const float* from, float (&v)[1]) { v[0] = from[0]; }
+__device__ __forceinline__ void small_operand(const float* from, float (&v)[4]) {
+    const float4 t = *reinterpret_cast<const float4*>(from);
+    v[0] = t.x;
+    v[1] = t.y;
+    v[2] = t.z;
+    v[3] = t.w;
+}
+
+// four output elements of a row
+__device__ __forceinline__ float4 small_epilogue(const SmallGemm& g, float4 v, const float4& scale, const float4& shift) {
+    float o[4] = {v.x, v.y, v.z, v.w};
+    const float sc[4] = {scale.x, scale.y, scale.z, scale.w}, sh[4] = {shift.x, shift.y, shift.z, shift.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (g.scale) o[e] = o[e] * sc[e];
+        if (g.shift) o[e] = o[e] + sh[e];
+        if (g.relu) o[e] = o[e] > 0.f ? o[e] : 0.f;
+    }
+    return make_float4(o[0], o[1], o[2], o[3]);
+}
+
+// CIN 0: the rulebook alone
+template <int CIN, int COUT>
 __global__ void __launch_bounds__(kSmallBlock)
-subm_small_rulebook(LookupPart P, int32_t* __restrict__ tiles) {
+subm_small(LookupPart P, int32_t* __restrict__ tiles, SmallGemm G) {
     constexpr uint32_t kNoRow = 0xffffu;
+    constexpr bool kGemm = CIN > 0;
+    constexpr int E = kGemm ? CIN / 4 : 1, NB = kGemm ? COUT / 16 : 1, kVecs = kGemm ? COUT / 4 : 1;
     __shared__ __align__(16) uint32_t s_head[kSmallHeads];  // of a hash value: first row << 16 | first row of the list of others
     __shared__ uint2 s_cell[kSmallRows];                    // a row's cell, the next row of its list
     __shared__ int32_t s_pairs[64];
+    __shared__ int32_t s_found[kGemm ? kSmallQuarters * kSmallQuarter * 64 : 1];  // [offset][row]
+    static_assert(kSmallQuarters * 64 * 32 <= kSmallHeads, "the quarters' sums take the heads' place");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int4* coors = reinterpret_cast<const int4*>(P.coors);  // (b,z,y,x)
     const int heads_lg = P.max_voxels <= kSmallHeads / 8 ? 32 - __clz(P.max_voxels * 4) : 14;  // (four and more a row, up to the room there is)
@@ -75,10 +122,29 @@ subm_small_rulebook(LookupPart P, int32_t* __restrict__ tiles) {
     }
     const int row = blockIdx.x * 64 + lane;  // whose neighbours this lane looks up, at offsets wave, wave + kSmallWaves, ...
     const int4 own = coors[row < P.max_voxels ? row : 0];
+    const int quarter = wave >> 2, rows16 = (wave & 3) * 16 + (lane & 15);  // of the products: the wave's offsets, the lane's row
+    const int vec = (tid % kVecs) * 4;                                      // of the epilogue: the thread's columns
+    float w[kSmallQuarter][NB][E];
+    float4 epi_scale = make_float4(1.f, 1.f, 1.f, 1.f), epi_shift = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (kGemm) {
+#pragma unroll
+        for (int j = 0; j < kSmallQuarter; ++j) {
+            const int k = quarter * kSmallQuarter + j;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) small_operand(G.w + (((k < P.K ? k : 0) * NB + nb) * 64 + lane) * E, w[j][nb]);
+        }
+        if (G.scale) epi_scale = *reinterpret_cast<const float4*>(G.scale + vec);
+        if (G.shift) epi_shift = *reinterpret_cast<const float4*>(G.shift + vec);
+    }
     for (int t = tid; t < (1 << (32 - shift)) / 4; t += kSmallBlock) reinterpret_cast<uint4*>(s_head)[t] = make_uint4(~0u, ~0u, ~0u, ~0u);
     if (tid < 64) s_pairs[tid] = 0;
     const int n = clamp_rows(P.num, P.max_voxels);
-    if ((int)blockIdx.x * 64 >= n && blockIdx.x) return;
+    if ((int)blockIdx.x * 64 >= n && blockIdx.x) {
+        const int r = blockIdx.x * 64 + tid / kVecs;
+        if (kGemm && G.write_pad && tid < 64 * kVecs && r < P.max_voxels)
+            *reinterpret_cast<float4*>(G.out + (size_t)r * COUT + vec) = small_epilogue(G, make_float4(0.f, 0.f, 0.f, 0.f), epi_scale, epi_shift);
+        return;
+    }
     __syncthreads();
     auto cell = [&](int z, int y, int x) { return ((uint32_t)z * (uint32_t)P.t.gy + (uint32_t)y) * (uint32_t)P.t.gx + (uint32_t)x; };
     auto list = [&](uint32_t key) { return (key * 2654435769u) >> shift; };
@@ -145,6 +211,56 @@ subm_small_rulebook(LookupPart P, int32_t* __restrict__ tiles) {
         const int k = wave + j * kSmallWaves;
         pairs += found[j] != kEmpty ? 1 : 0;
         if (k < P.K && row < n) P.nbr[(size_t)k * P.max_voxels + row] = (int32_t)found[j];
+        if (kGemm && k < kSmallQuarters * kSmallQuarter) s_found[k * 64 + lane] = k < P.K ? (int32_t)found[j] : -1;
+    }
+    if constexpr (kGemm) {
+        typedef float v4f __attribute__((ext_vector_type(4)));
+        static_assert(kSmallDepth * kSmallWaves >= kSmallQuarters * kSmallQuarter, "an entry for each offset");
+        const int q = lane >> 4;  // channels of an MFMA's operands, columns of its results
+        __syncthreads();
+        float x[kSmallQuarter][E];
+        int idx[kSmallQuarter];
+#pragma unroll
+        for (int j = 0; j < kSmallQuarter; ++j) idx[j] = s_found[(quarter * kSmallQuarter + j) * 64 + rows16];
+#pragma unroll
+        for (int j = 0; j < kSmallQuarter; ++j)
+            small_operand(G.in + (idx[j] >= 0 ? idx[j] : 0) * CIN + q * E, x[j]);
+        v4f sum[kSmallQuarter][NB];
+#pragma unroll
+        for (int j = 0; j < kSmallQuarter; ++j)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                v4f acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int e = 0; e < E; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][nb][e], x[j][e], acc, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sum[j][nb][r] = idx[j] >= 0 ? acc[r] : 0.f;
+            }
+#pragma unroll
+        for (int m = kSmallQuarter; m > 1; m = (m + 1) / 2)
+#pragma unroll
+            for (int j = 0; j < m / 2; ++j)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sum[j][nb][r] += sum[m - 1 - j][nb][r];
+        float4* const part = reinterpret_cast<float4*>(s_head);  // [quarter][row][column / 4]
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+            part[(quarter * 64 + rows16) * kVecs + nb * 4 + q] = make_float4(sum[0][nb][0], sum[0][nb][1], sum[0][nb][2], sum[0][nb][3]);
+        __syncthreads();
+        const int r = blockIdx.x * 64 + tid / kVecs;
+        if (tid < 64 * kVecs && r < (G.write_pad ? P.max_voxels : n)) {
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (r < n) {
+                float4 p[kSmallQuarters];
+#pragma unroll
+                for (int g = 0; g < kSmallQuarters; ++g) p[g] = part[g * 64 * kVecs + tid];
+                v = make_float4((p[0].x + p[3].x) + (p[1].x + p[2].x), (p[0].y + p[3].y) + (p[1].y + p[2].y),
+                                (p[0].z + p[3].z) + (p[1].z + p[2].z), (p[0].w + p[3].w) + (p[1].w + p[2].w));
+            }
+            *reinterpret_cast<float4*>(G.out + (size_t)r * COUT + vec) = small_epilogue(G, v, epi_scale, epi_shift);
+        }
     }
     if (!P.w) return;  // (uniform)
     atomicAdd(&s_pairs[lane], pairs);
@@ -369,7 +485,7 @@ int SubmConv3dLayerPlugin::enqueueBuild(const int32_t* coors, const int32_t* vox
     const CellTable t = ownTable(workspace);
     const LookupPart look = lookupPart(workspace, coors, voxel_num, t, voxel_num, max_voxels_);
     if (max_voxels_ <= kSmallRows) {
-        hipLaunchKernelGGL(subm_small_rulebook, dim3(ceil_div(max_voxels_, 64)), dim3(kSmallBlock), 0, stream, look, L.tiles);
+        hipLaunchKernelGGL((subm_small<0, 0>), dim3(ceil_div(max_voxels_, 64)), dim3(kSmallBlock), 0, stream, look, L.tiles, SmallGemm());
         SESSD_HIP_TRY(hipGetLastError());
     } else {
         FillArgs f;
@@ -384,6 +500,33 @@ int SubmConv3dLayerPlugin::enqueueBuild(const int32_t* coors, const int32_t* vox
     if (!wantTileCuts()) return SESSD_OK;
     const CutPart cut = cutPart(workspace, voxel_num);
     return launch_number(nullptr, nullptr, &cut, 1, nullptr, nullptr, stream);
+}
+
+// Rulebook and products in one launch (subm_small): layers of few rows on plain FP32 products.  Where a caller times the products
+// they are a launch of their own.
+bool SubmConv3dLayerPlugin::runsInOne() const {
+    const bool shape = out_channel_ == 16 ? in_channel_ == 4 || in_channel_ == 16 : out_channel_ == 32 && in_channel_ == 4;
+    return max_voxels_ <= kSmallRows && shape && in_type_ == SESSD_FLOAT && out_type_ == SESSD_FLOAT && gemmOnMatrixCores() && !wantTileCuts() &&
+           !ev_gemm_begin_ && !ev_gemm_end_;
+}
+
+int SubmConv3dLayerPlugin::enqueueInOne(const void* in_feat, const int32_t* coors, const int32_t* voxel_num, void* out_feat, void* workspace,
+                                        hipStream_t stream) {
+    const Layout L = carve(workspace);
+    const LookupPart look = lookupPart(workspace, coors, voxel_num, ownTable(workspace), voxel_num, max_voxels_);
+    SmallGemm g;
+    g.in = static_cast<const float*>(in_feat);
+    g.out = static_cast<float*>(out_feat);
+    g.w = static_cast<const float*>(weights_packed_dev_);
+    g.scale = epi_.scale_dev;
+    g.shift = epi_.shift_dev;
+    g.relu = epi_.relu;
+    g.write_pad = (flags_ & SESSD_FLAG_SKIP_PAD_ROWS) ? 0 : 1;
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(ceil_div(max_voxels_, 64)), dim3(kSmallBlock), 0, stream, look, L.tiles, g); };
+    if (in_channel_ == 16) go(subm_small<16, 16>);
+    else out_channel_ == 16 ? go(subm_small<4, 16>) : go(subm_small<4, 32>);
+    SESSD_HIP_TRY(hipGetLastError());
+    return SESSD_OK;
 }
 
 int SubmConv3dLayerPlugin::enqueueGemm(const void* in_feat, void* out_feat, const int32_t* voxel_num,
@@ -401,8 +544,9 @@ int SubmConv3dLayerPlugin::enqueue(const sessd_tensor_desc* inputDesc, const ses
     SESSD_TRY(conv_check_io(inputDesc, outputDesc, inputs, outputs, in_type_, out_type_, max_voxels_,
                             in_channel_, out_channel_, "submconv3d.enqueue"));
     if (!workspace) return fail(SESSD_E_INVALID, "submconv3d.enqueue: workspace is null");
-    const int32_t* voxel_num = static_cast<const int32_t*>(inputs[2]);
-    SESSD_TRY(enqueueBuild(static_cast<const int32_t*>(inputs[1]), voxel_num, workspace, stream));
+    const int32_t *coors = static_cast<const int32_t*>(inputs[1]), *voxel_num = static_cast<const int32_t*>(inputs[2]);
+    if (runsInOne()) return enqueueInOne(inputs[0], coors, voxel_num, outputs[0], workspace, stream);
+    SESSD_TRY(enqueueBuild(coors, voxel_num, workspace, stream));
     return enqueueGemm(inputs[0], outputs[0], voxel_num, workspace, stream);
 }
 

@@ -198,6 +198,45 @@ def test_small_layer_whose_rows_name_few_cells(side):
     assert np.allclose(got[0][2], got[1][2], rtol=0, atol=27 * 4 * 2.0 ** -24)
 
 
+@pytest.mark.parametrize("ksize", [1, 3])
+@pytest.mark.parametrize("cin,cout", [(4, 16), (4, 32), (16, 16)])
+def test_small_layer_with_its_products_in_the_same_launch(cin, cout, ksize):
+    """FP32 layers of at most 8 192 rows and few channels multiply in the launch that builds their rulebook: the outputs of the
+    two launches (the layer on its own rulebook as a sharer), and all rows beyond the active ones.  An infinite weight reaches the
+    rows that have the neighbour, and no other."""
+    rng = np.random.default_rng(cin + cout + ksize)
+    grid, K = (41, 300, 200), ksize ** 3
+    sc, sh = rng.uniform(0.5, 1.5, cout).astype(np.float32), rng.uniform(-0.5, 0.5, cout).astype(np.float32)
+    for n, mv, infinite in ((0, 1, False), (1, 1, False), (0, 130, False), (63, 64, False), (64, 65, False), (65, 400, True), (2000, 2000, False),
+                            (4097, 5000, True), (8192, 8192, False)):
+        coors = np.zeros((mv, 4), np.int32)
+        coors[:n] = F.clustered_active_voxels(n, grid, 7, n_blobs=12)[:n] if n else 0
+        if n >= 64:
+            coors[n - 5:n] = coors[3:8]
+            coors[10, 1], coors[20, 2], coors[30, 3] = -1, grid[1], grid[2] + 7
+        feat = rng.uniform(-1, 1, (mv, cin)).astype(np.float32)
+        w = rng.normal(0, 0.1, (K, cin, cout)).astype(np.float32)
+        if infinite:
+            w[K // 3, 1, 2] = np.inf
+        conv = api.SubmConv3d(cin, cout, grid[::-1], w, mv, ksize=ksize, padding=ksize // 2)
+        args = dev(feat), dev(coors), dev(np.array([n], np.int32))
+        for epilogue in (False, True):
+            if epilogue:
+                conv.set_epilogue(sc, sh, relu=True)
+            one = to_np(conv(*args))
+            two = to_np(conv(*args, rulebook_from=conv))
+            assert np.array_equal(np.isnan(one), np.isnan(two)) and np.array_equal(np.isinf(one), np.isinf(two)), (n, mv)
+            assert np.array_equal(one[n:], np.broadcast_to(np.maximum(sh, 0) if epilogue else np.float32(0), (mv - n, cout))), (n, mv)
+            # (sums in another order: 2^-24 a term of at most 0.5, times a scale of 1.5)
+            some = np.isfinite(two)
+            assert np.allclose(one[some], two[some], rtol=0, atol=1.5 * K * cin * 2.0 ** -24), (n, mv)
+        conv.set_flags(D.SESSD_FLAG_SKIP_PAD_ROWS)
+        out = torch.full((mv, cout), 7.0, device="cuda:0")
+        conv.enqueue(list(args), [out])
+        assert np.array_equal(to_np(out)[:n], one[:n], equal_nan=True) and (to_np(out)[n:] == 7).all(), (n, mv)
+        conv.close()
+
+
 @pytest.mark.parametrize("cin,cout", [(4, 16), (16, 16), (16, 32), (32, 32), (32, 64), (64, 64), (64, 128), (128, 128),
                                       (5, 7), (8, 32)])
 def test_subm_clustered_with_epilogue_and_pad_rows(cin, cout):
