@@ -7,6 +7,7 @@ declared in include/sessd3d.h.  There is no fallback: if the library is missing 
 import ctypes as C
 import os
 import re
+import struct
 
 import numpy as np
 
@@ -58,7 +59,7 @@ def lib():
         getattr(L, "sessd_%s_configure" % name).argtypes = [vp, TD, C.c_int, TD, C.c_int]
         getattr(L, "sessd_%s_workspace_size" % name).restype = sz
         getattr(L, "sessd_%s_workspace_size" % name).argtypes = [vp, TD, C.c_int, TD, C.c_int]
-        getattr(L, "sessd_%s_enqueue" % name).argtypes = [vp, TD, TD, VPP, VPP, vp, vp]
+        getattr(L, "sessd_%s_enqueue" % name).argtypes = [vp, TD, TD, vp, vp, vp, vp]  # (pointer arrays: _pointers())
         getattr(L, "sessd_%s_destroy" % name).argtypes = [vp]
         getattr(L, "sessd_%s_destroy" % name).restype = None
     for name in ("voxelgen", "submconv3d", "sparseconv3d"):
@@ -69,9 +70,9 @@ def lib():
         getattr(L, "sessd_%s_export_rulebook" % name).argtypes = [vp, vp, vp, vp, vp]
     L.sessd_voxelgen_create.argtypes = [C.POINTER(D.VoxelGenDesc), VPP]
     L.sessd_voxelgen_grid_size.argtypes = [vp, C.POINTER(i32)]
-    L.sessd_voxelgen_enqueue_static.argtypes = [vp, TD, TD, VPP, VPP, vp]
+    L.sessd_voxelgen_enqueue_static.argtypes = [vp, TD, TD, vp, vp, vp]
     L.sessd_submconv3d_create.argtypes = [C.POINTER(D.SubmConv3dDesc), vp, VPP]
-    L.sessd_submconv3d_enqueue_shared.argtypes = [vp, TD, TD, VPP, VPP, vp, vp]
+    L.sessd_submconv3d_enqueue_shared.argtypes = [vp, TD, TD, vp, vp, vp, vp]
     L.sessd_sparseconv3d_create.argtypes = [C.POINTER(D.SparseConv3dDesc), vp, VPP]
     L.sessd_sparse2dense_create.argtypes = [C.POINTER(D.Sparse2DenseDesc), VPP]
     L.sessd_sparse2dense_set_padding.argtypes = [C.c_void_p] + [C.c_int32] * 4
@@ -166,15 +167,31 @@ def _descs(tensors):
     return arr
 
 
-_VP = [C.c_void_p * n for n in range(17)]
+_PACK = [struct.Struct("%dP" % n).pack for n in range(17)]
 
 
-def _voidpp(tensors):
-    return _VP[len(tensors)](*[t.data_ptr() for t in tensors])
+def _pointers(tensors):
+    """The tensors' addresses as an array of pointers, for a call that reads it (bytes: half of what a ctypes array takes to make)."""
+    if len(tensors) == 3:
+        a, b, c = tensors
+        return _PACK[3](a.data_ptr(), b.data_ptr(), c.data_ptr())
+    if len(tensors) == 1:
+        return _PACK[1](tensors[0].data_ptr())
+    if len(tensors) == 2:
+        return _PACK[2](tensors[0].data_ptr(), tensors[1].data_ptr())
+    return _PACK[len(tensors)](*[t.data_ptr() for t in tensors])
 
 
 def _signature(tensors):
-    return tuple([(t.shape, t.dtype) for t in tensors])
+    if len(tensors) == 3:
+        a, b, c = tensors
+        return a.shape, a.dtype, b.shape, b.dtype, c.shape, c.dtype
+    if len(tensors) == 1:
+        return tensors[0].shape, tensors[0].dtype
+    if len(tensors) == 2:
+        a, b = tensors
+        return a.shape, a.dtype, b.shape, b.dtype
+    return tuple([v for t in tensors for v in (t.shape, t.dtype)])
 
 
 class _Bound:
@@ -261,9 +278,12 @@ class _Plugin:
         return self._enqueue_bound(self._bound(inputs, outputs), inputs, outputs, stream, workspace)
 
     def _enqueue_bound(self, bound, inputs, outputs, stream, workspace=None):
-        ws = workspace if workspace is not None else self._workspace(bound, inputs[0].device)
-        check(self._enqueue(self.h, bound.ins, bound.outs, _voidpp(inputs), _voidpp(outputs), ws.data_ptr(),
-                            _stream_ptr(stream)))
+        ws = workspace if workspace is not None else self.ws
+        if ws is None or (workspace is None and ws.numel() < bound.ws_bytes):
+            ws = self._workspace(bound, inputs[0].device)
+        rc = self._enqueue(self.h, bound.ins, bound.outs, _pointers(inputs), _pointers(outputs), ws.data_ptr(), _stream_ptr(stream))
+        if rc:
+            check(rc)
         return ws
 
     def status(self, stream=None) -> int:
@@ -304,8 +324,8 @@ class VoxelGenerator(_Plugin):
 
     def enqueue_static(self, inputs, outputs, stream=None):
         """enqueue() on the library's static scratch array: no workspace, no allocation (sessd_voxelgen_enqueue_static)."""
-        check(lib().sessd_voxelgen_enqueue_static(self.h, _descs(inputs), _descs(outputs), _voidpp(inputs),
-                                                  _voidpp(outputs), _stream_ptr(stream)))
+        check(lib().sessd_voxelgen_enqueue_static(self.h, _descs(inputs), _descs(outputs), _pointers(inputs),
+                                                  _pointers(outputs), _stream_ptr(stream)))
 
     def status_static(self, stream=None) -> int:
         s = C.c_int32(0)
@@ -364,7 +384,7 @@ class SubmConv3d(_Conv):
         if rulebook_from is None:
             self._enqueue_bound(bound, ins, outs, stream)
         else:
-            check(lib().sessd_submconv3d_enqueue_shared(self.h, bound.ins, bound.outs, _voidpp(ins), _voidpp(outs),
+            check(lib().sessd_submconv3d_enqueue_shared(self.h, bound.ins, bound.outs, _pointers(ins), _pointers(outs),
                                                         _ptr(rulebook_from.ws), _stream_ptr(stream)))
         return out
 
