@@ -1,27 +1,28 @@
-// conv_tall.hip -- gather-GEMM for FP16 layers with Cin 32: tall tiles, weights through LDS.
+// conv_tall.hip -- gather-GEMM for FP16 3x3x3 layers with Cin 32: all of W in LDS, no barrier between the offsets.
 //
 //     out[o][:] = epilogue( sum_k  in[nbr[k][o]][:] @ W[k] )
 //
-// A kernel with short tiles requests all of W once per 48 or 64 rows; in FP16, where the matrix cores
-// are far from busy, those requests are what the compute units' load path spends its time on.  Here a workgroup (4
-// wave64) owns 64 or 128 consecutive output rows:
-//   * W[k] is copied once per workgroup and offset into LDS (two buffers; the host's MFMA operand order is also
-//     the LDS order): every wave requests its share a few offsets ahead into registers and stores it one offset
-//     before its use;
-//   * a wave owns 16 or 32 of the rows and ALL columns, and keeps their accumulators in registers over all K
-//     offsets: no compaction, no partial tiles.  A row without a neighbour at offset k contributes a zero operand
-//     (a buffer load that points out of range: zeros, no memory touched), so the matrix cores multiply about twice
-//     the useful pairs -- in FP16 they have the headroom;
-//   * every gathered row is requested once, D offsets ahead, by the wave that uses it;
-//   * all requests of the offset loop are unconditional and in a fixed order, so the compiler's waits cover exactly
-//     the operands about to be used; one barrier per offset publishes the next offset's weights and frees the buffer
-//     they overwrite.
-// (Copying the weights with direct-to-LDS loads needs no registers, but a wait for "all but the N youngest
-// requests" did not reliably cover such a copy when ordinary loads were in flight behind it -- stale weights in a
-// few tiles per thousand launches -- and waiting for everything gives up the prefetch.)
-// Summation order per output element: offsets ascending, channels inside the MFMA: fixed, run-to-run identical.
-// (The ring of conv_tile.hip, faster from 64 channels up, has too little work per row here: 32 -> 32 at 60 000 rows
-// 15.6 us, this kernel 10.7; its slices would be half a cache line.)
+// W is 55 or 110 KB and one workgroup a compute unit keeps all of it, so that its waves meet only once, in front of the first product.
+//   * A workgroup owns a run of output rows, 16 at a time (a block) for each of its eight waves, and all columns; the accumulators stay
+//     in registers over all offsets: no compaction, no partial tiles.  A row without a neighbour contributes a zero operand (a buffer
+//     load that points out of range: zeros, no memory touched), so the matrix cores multiply about twice the useful pairs -- in FP16
+//     they have the headroom.
+//   * A step is four offsets.  Lane (i, q) of a wave requests all 64 bytes of the neighbour of row i at offset 4 step + q, and the inner
+//     dimension of an MFMA is eight channels of each of the four offsets: the lane's own list entries are all that it needs, no other
+//     lane's, and W is in LDS as the host has packed it (lane (i, q) reads the operand that holds these channels of W[4 step + q]).
+//     Rows are requested two steps (eight offsets) ahead, all of them by straight-line code: the compiler's waits are exact.
+//   * With few rows two or four waves share a block and take every second or fourth step; their sums are added in LDS.
+//   * W, the row count and, behind that, the lists are on their way together; the first rows are requested in front of the barrier.
+//   * The rows beyond the active ones are written by four waves of their own.
+// What bounds it from some 40 000 rows up are the requests for rows in four cache lookups a row (coalesced ones, with a 4 x 4
+// transposition in registers, took longer: 49 874 rows 8.4 -> 9.5 us) and the reads of W from LDS (two blocks a wave: 8.4 -> 8.7), below
+// the trips to memory: row count, lists, rows.
+// Measured against the kernel with a barrier and 2 or 4 KB of W an offset that these layers ran on, launches back to back, 32 -> 32 and
+// 32 -> 64: 801 rows 5.05 -> 3.5 us and 5.9 -> 4.8, 13 907 rows 5.3 -> 4.7 and 6.2 -> 6.25, 26 575 rows 7.1 -> 5.7 and 7.9 -> 7.3,
+// 49 874 rows 11.2 -> 8.4 and 13.1 -> 10.9, 74 606 rows 13.9 -> 10.9 and 16.1 -> 13.4; frames of 60 000 points 230.6 -> 226.6.
+// The waves are eight because the coordinate passes beside them need registers (12: the same times, and 504 of 512 taken).
+// Summation order per output element: steps ascending, in a step the channels eight at a time: fixed, run-to-run identical.
+// (The ring of conv_tile.hip, faster from 64 channels up, has too little work per row here.)
 #include <type_traits>
 
 #include "pad_rows.h"
@@ -34,15 +35,14 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef unsigned int v4u32 __attribute__((__vector_size__(16)));
 
-constexpr int kWaves = 4;
-constexpr int KC = 27;          // kernel offsets: the 3x3x3 layers
-constexpr int D = 3;            // offsets the rows are requested ahead
-constexpr int DW = 2;           // register sets for weights in flight
-constexpr int kTallBlocks = 2;  // 16-row blocks a wave owns in a tall tile (one in a short tile: the heights are chosen on
-                                // the device from the row count)
-constexpr int kGroupsAhead = 3;  // groups of weight fragments a wave has requested from LDS ahead of the one it multiplies
+constexpr int kWaves = 8;     // that multiply
+constexpr int kPadWaves = 4;  // that write the rows beyond the active ones
+constexpr int KC = 27;                  // kernel offsets: the 3x3x3 layers
+constexpr int kSteps = (KC + 3) / 4;    // of four offsets
+constexpr int CIN = 32, kPieces = 4;    // 16-byte pieces of a row
 constexpr unsigned kOutOfRange = 0x80000000u;
 constexpr int kRawBuffer = 0x00020000;
+constexpr int kDepth = 2;  // steps whose rows are on their way (3: the same times, 16 registers more)
 
 __device__ __forceinline__ void store4h(__half* dst, const float (&o)[4]) {
     union {
@@ -54,304 +54,243 @@ __device__ __forceinline__ void store4h(__half* dst, const float (&o)[4]) {
     *reinterpret_cast<uint2*>(dst) = p.u;
 }
 
-// The barrier of the offset loop.  __syncthreads() would add workgroup-scope fences, for which the compiler drains
-// every request in flight -- the rows and weights just requested for later offsets included.  What the loop needs
-// published are this wave's LDS stores (waited for explicitly); the compiler must only keep its LDS accesses on
-// their side of the barrier.
-__device__ __forceinline__ void ring_barrier() {
+// This wave's LDS accesses are done, and everybody else's.  (__syncthreads() would wait for the rows on their way as well.)
+__device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): vmcnt and expcnt fields at their maximum = no wait
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
 
-// One of the two weight buffers in LDS
-template <int U, int slot>
-__device__ __forceinline__ float4* weight_slot() {
-    __shared__ float4 s_w[U * 64];
-    return s_w;
+struct Tensors {
+    __amdgpu_buffer_rsrc_t in, nbr;
+    __half* out;
+    unsigned stride4;  // bytes from offset to offset of the rulebook
+    int n, relu;
+    bool has_scale, has_shift;
+};
+
+// Where the neighbours of the lane's row are, at the lane's offset of steps first, first + BY, ... (-1: none)
+template <int BY>
+__device__ __forceinline__ void ask_lists(const Tensors& t, int lane, int row0, int first, int (&idx)[kSteps]) {
+    const int row = row0 + (lane & 15), q = lane >> 4;
+#pragma unroll
+    for (int m = 0; m < (kSteps + BY - 1) / BY; ++m) {
+        const int k = 4 * (first + m * BY) + q;
+        const bool some = k < KC && row < t.n;
+        idx[m] = (int)__builtin_amdgcn_raw_buffer_load_b32(t.nbr, some ? (unsigned)k * t.stride4 + (unsigned)row * 4u : kOutOfRange, 0, 0);
+        idx[m] = some ? idx[m] : -1;
+    }
 }
 
-// The tile of one workgroup.  RB = 16-row blocks per wave.
-template <int CIN, int COUT, int RB>
-__device__ __forceinline__ void tall_tile(const __half* __restrict__ in, __half* __restrict__ out,
-                                          const void* __restrict__ Wp, const int32_t* __restrict__ nbr, int n,
-                                          int row0, int max_voxels, const float* __restrict__ scale, const float* __restrict__ shift,
-                                          int relu, DenseTarget dt, int32_t* s_nbr, float* s_epi) {
-    constexpr int G = CIN / 32;        // K-chunks (32 channels) of the inner dimension
-    constexpr int NBT = COUT / 16;     // 16-column blocks
-    constexpr int U = G * NBT;         // 1 KB units (64 lanes x 16 bytes) of one offset's weights
-    constexpr int NBUF = D + 1;        // row register sets
-    constexpr int TR = kWaves * RB * 16;
-    constexpr int UW = (U + kWaves - 1) / kWaves;  // weight units a wave copies per offset
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    if (row0 >= n) return;
-
-    // The tile's neighbour lists (rows beyond n: none) -> LDS.  A wave takes 64 rows of one offset at a time, all of them requested before
-    // the first is stored.  (In a loop over the entries each was a trip to memory of its own, behind those for scale, shift and the row
-    // count: 32 -> 32 at 4 208 rows 5.9 -> 5.4 us, 45 874 10.5 -> 9.9, 72 487 16.1 -> 14.8; 32 -> 64 at 45 874 12.3 -> 11.8.)
-    constexpr int kRuns = TR / 64, kLists = (KC * kRuns + kWaves - 1) / kWaves;  // runs of 64 rows an offset, runs a wave
-    static_assert(kWaves % kRuns == 0, "a wave's runs are all of the same rows");
-    const int run = wave % kRuns, here = n - row0 - run * 64;  // (rows of the run; may be none)
-    int32_t list[kLists];
-    {
-        uint64_t at = reinterpret_cast<uint64_t>(nbr) + 4 * ((uint64_t)(uint32_t)(wave / kRuns) * (uint32_t)max_voxels + (uint32_t)(row0 + run * 64));
+// Steps first, first + BY, ... of the block
+template <int COUT, int BY>
+__device__ __forceinline__ void multiply(const Tensors& t, int lane, const int (&idx)[kSteps], int first, const unsigned char* s_w, bool wait_for_w,
+                                         v4f (&acc)[COUT / 16]) {
+    constexpr int NB = COUT / 16, N = (kSteps + BY - 1) / BY;
+    const int i = lane & 15, q = lane >> 4;
+    v4u32 x[kDepth][kPieces];
+    auto request = [&](int m) {  // (m < N)
+        const unsigned at = idx[m] >= 0 ? (unsigned)idx[m] * (unsigned)(CIN * sizeof(__half)) : kOutOfRange;
 #pragma unroll
-        for (int t = 0; t < kLists; ++t) {
-            const int k = wave / kRuns + t * (kWaves / kRuns);
-            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(at), 0, k < KC && here > 0 ? here * 4 : 0, kRawBuffer);
-            list[t] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, lane * 4, 0, 0);
-            at += 4 * (uint64_t)(kWaves / kRuns) * (uint32_t)max_voxels;
+        for (int p = 0; p < kPieces; ++p) x[m % kDepth][p] = __builtin_amdgcn_raw_buffer_load_b128(t.in, at + p * 16u, 0, 0);
+    };
+    static_assert(N >= kDepth, "steps");
+#pragma unroll
+    for (int m = 0; m < kDepth; ++m) request(m);
+    if (wait_for_w) lds_barrier();
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[nb] = (v4f){0.f, 0.f, 0.f, 0.f};
+    const unsigned char* w_at = s_w + (first * 4 + q) * (NB * 1024) + i * 16;
+#pragma unroll
+    for (int m = 0; m < N; ++m, w_at += BY * 4 * NB * 1024) {
+        if (BY > 1 && first + m * BY >= kSteps) break;  // (uniform)
+        // (the weights of a piece or two at a time: registers)
+        constexpr int kAtOnce = NB > 2 ? 1 : 2;
+        v8h w[2][kAtOnce][NB];
+        auto weights = [&](int p, v8h (&to)[kAtOnce][NB]) {
+#pragma unroll
+            for (int a = 0; a < kAtOnce; ++a)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) to[a][nb] = *reinterpret_cast<const v8h*>(w_at + nb * 1024 + (p + a) * 256);
+        };
+        weights(0, w[0]);
+#pragma unroll
+        for (int p = 0; p < kPieces; p += kAtOnce) {
+            if (p + kAtOnce < kPieces) weights(p + kAtOnce, w[p / kAtOnce % 2 ^ 1]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int a = 0; a < kAtOnce; ++a)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[p / kAtOnce % 2][a][nb], __builtin_bit_cast(v8h, x[m % kDepth][p + a]), acc[nb], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (m + kDepth < N) request(m + kDepth);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// lane (i, q) holds output channels 16nb+4q .. +3 of row i
+template <int COUT>
+__device__ __forceinline__ void put(const Tensors& t, int lane, int row0, const v4f (&acc)[COUT / 16], const float* s_epi, const DenseTarget& dt) {
+    constexpr int NB = COUT / 16;
+    const int i = lane & 15, q = lane >> 4;
+    const int row = row0 + i;
+    if (row >= t.n) return;
+    bool to_dense = false;
+    __half* d = nullptr;
+    size_t plane = 0;
+    if (dt.dense) {  // the sparse2Dense scatter of this row, fused (uniform branch)
+        const int4 cc = reinterpret_cast<const int4*>(dt.coors)[row];  // (b,z,y,x)
+        if (cc.x != 0 || cc.y < 0 || cc.y >= dt.D || cc.z < 0 || cc.z >= dt.H || cc.w < 0 || cc.w >= dt.W) {
+            if (dt.status && q == 0) atomicOr(dt.status, SESSD_STATUS_BAD_COORD);
+        } else {
+            to_dense = true;
+            d = static_cast<__half*>(dt.dense) + ((size_t)cc.y * dt.Hp + cc.z + dt.pad_top) * dt.Wp + cc.w + dt.pad_left;
+            plane = (size_t)dt.D * dt.Hp * dt.Wp;
         }
     }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+        const int c4 = nb * 16 + q * 4;
+        float o[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float s = acc[nb][e];
+            if (t.has_scale) s = s * s_epi[c4 + e];
+            if (t.has_shift) s = s + s_epi[COUT + c4 + e];
+            if (t.relu) s = s > 0.f ? s : 0.f;
+            o[e] = s;
+        }
+        store4h(t.out + (size_t)row * COUT + c4, o);
+        if (to_dense) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) d[(size_t)(c4 + e) * plane] = __float2half_rn(o[e]);
+        }
+    }
+}
+
+template <int COUT, bool PAD>
+__global__ void __launch_bounds__((kWaves + (PAD ? kPadWaves : 0)) * 64)
+conv_tall(const int32_t* __restrict__ num_out, const int32_t* __restrict__ nbr, const __half* __restrict__ in,
+          const void* __restrict__ Wp, int max_voxels, int relu, __half* __restrict__ out,
+          const float* __restrict__ scale, const float* __restrict__ shift, DenseTarget dt) {
+    constexpr int NB = COUT / 16, kThreads = (kWaves + (PAD ? kPadWaves : 0)) * 64;
+    constexpr int kOffsetBytes = NB * 1024, kVectors = KC * kOffsetBytes / 16, kCopies = (kVectors + kThreads - 1) / kThreads;
+    // (one offset more than there are, of zeros)
+    __shared__ __align__(16) unsigned char s_w[kSteps * 4 * kOffsetBytes];
+    __shared__ float s_epi[2 * COUT];
+    static_assert(kSteps * 4 == KC + 1, "steps");
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    v4f copy[kCopies];
+#pragma unroll
+    for (int c = 0; c < kCopies; ++c) {
+        const int v = c * kThreads + tid;
+        copy[c] = reinterpret_cast<const v4f*>(Wp)[v < kVectors ? v : 0];
+    }
+    int n = *num_out;
+    n = n < 0 ? 0 : (n > max_voxels ? max_voxels : n);
+    float by = 1.f, plus = 0.f;
     if (tid < COUT) {
-        float by = 1.f, plus = 0.f;
         if (scale) by = scale[tid];
         if (shift) plus = shift[tid];
-        s_epi[tid] = by;
-        s_epi[COUT + tid] = plus;
     }
+    // a workgroup's share: `per` blocks of 16 rows; the workgroups of an XCD (dealt round robin over eight) take neighbouring ones
+    const int blocks = (n + 15) >> 4, groups = gridDim.x, per = (blocks + groups - 1) / groups;
+    const int share = groups % 8 ? (int)blockIdx.x : (int)(blockIdx.x & 7) * (groups >> 3) + (int)(blockIdx.x >> 3);
+    const int begin = share * per < blocks ? share * per : blocks, end = begin + per < blocks ? begin + per : blocks;
+    Tensors t;
+    t.in = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half*>(in), 0, (int)((size_t)max_voxels * CIN * sizeof(__half)), kRawBuffer);
+    t.nbr = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(nbr), 0, (int)((size_t)KC * max_voxels * sizeof(int32_t)), kRawBuffer);
+    t.out = out;
+    t.stride4 = (unsigned)max_voxels * 4u;
+    t.n = n;
+    t.relu = relu;
+    t.has_scale = scale != nullptr;
+    t.has_shift = shift != nullptr;
+    auto publish = [&]() {  // the weights and the epilogue's factors; the barrier that makes them visible follows
 #pragma unroll
-    for (int t = 0; t < kLists; ++t) {
-        const int k = wave / kRuns + t * (kWaves / kRuns);
-        if (k < KC) s_nbr[k * TR + run * 64 + lane] = lane < here ? list[t] : -1;
-    }
-    __syncthreads();
-    const bool has_scale = scale != nullptr, has_shift = shift != nullptr;
-
-    const int i = lane & 15;  // row inside a 16-row block
-    const int q = lane >> 4;  // 8-channel group inside a K-chunk
-    const __amdgpu_buffer_rsrc_t rs_in = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<__half*>(in), 0, (int)((size_t)max_voxels * CIN * sizeof(__half)), kRawBuffer);
-    const float4* wsrc = reinterpret_cast<const float4*>(Wp) + lane;
-
-    float4 a[NBUF][RB][G];
-    v4f wreg[DW][UW];  // (a native vector type: as an array of structs these registers ended up on the stack)
-    v4f acc[RB][NBT];
-#pragma unroll
-    for (int blk = 0; blk < RB; ++blk)
-#pragma unroll
-        for (int nb = 0; nb < NBT; ++nb) acc[blk][nb] = (v4f){0.f, 0.f, 0.f, 0.f};
-
-    // The offset loop runs in periods of P offsets (P = a common multiple of the row register sets, the two weight
-    // buffers and the weight register sets), the period unrolled, so that every register set and buffer has a
-    // compile-time name: s = position inside the period, k = k0 + s the offset.
-    constexpr int P = NBUF % 2 == 0 ? NBUF : 2 * NBUF;
-    static_assert(P % NBUF == 0 && P % 2 == 0 && P % DW == 0, "period");
-    // unit j of this wave's share of W[k] -> registers (beyond the last offset: the last one again, never used)
-    auto load_w1 = [&](int k, auto s_c, int j) {
-        constexpr int set = decltype(s_c)::value % DW;
-        const int kw = k < KC ? k : KC - 1;
-        // (fewer units than waves: some are copied twice, same bytes to the same place)
-        const int u = U % kWaves == 0 ? wave + j * kWaves : (wave + j * kWaves) % U;
-        wreg[set][j] = *reinterpret_cast<const v4f*>(wsrc + ((size_t)kw * U + u) * 64);
-    };
-    // ... -> LDS (beyond the last offset: into the buffer nobody reads any more)
-    auto store_w1 = [&](auto s_c, int j) {
-        constexpr int s = decltype(s_c)::value;
-        const int u = U % kWaves == 0 ? wave + j * kWaves : (wave + j * kWaves) % U;
-        *reinterpret_cast<v4f*>(weight_slot<U, s % 2>() + u * 64 + lane) = wreg[s % DW][j];
-    };
-    // block blk of this wave's rows of offset k -> registers (beyond the last offset: requests that fetch nothing)
-    auto load_rows1 = [&](int k, auto s_c, int blk) {
-        constexpr int set = decltype(s_c)::value % NBUF;
-        const int kr = k < KC ? k : KC - 1;
-        int idx = s_nbr[kr * TR + (wave * RB + blk) * 16 + i];
-        idx = k < KC ? idx : -1;
-        const unsigned at = idx >= 0 ? (unsigned)((idx * CIN + q * 8) * (int)sizeof(__half)) : kOutOfRange;
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            v4u32 v = __builtin_amdgcn_raw_buffer_load_b128(rs_in, at + g * 64u, 0, 0);
-            a[set][blk][g] = *reinterpret_cast<float4*>(&v);
+        for (int c = 0; c < kCopies; ++c) {
+            const int v = c * kThreads + tid;
+            if (v < kVectors) reinterpret_cast<v4f*>(s_w)[v] = copy[c];
+        }
+        if (tid < kOffsetBytes / 16) reinterpret_cast<v4f*>(s_w)[kVectors + tid] = (v4f){0.f, 0.f, 0.f, 0.f};
+        if (tid < COUT) {
+            s_epi[tid] = by;
+            s_epi[COUT + tid] = plus;
         }
     };
-    // Offset k at position s of the period.  Its weight fragments (one per K-chunk and column block, 16 bytes per
-    // lane) come from LDS in groups of BG, requested kGroupsAhead groups before they multiply.  The offset's other
-    // work -- the rows of offset k+D requested, W[k+1] stored to its buffer, W[k+1+DW] requested -- is dealt over
-    // the groups, so that those instructions issue while the matrix cores work on the group before (issued in one
-    // piece ahead of the first MFMA they took as long as the MFMAs themselves).
-    auto offset_step = [&](int k, auto s_c) {
-        constexpr int s = decltype(s_c)::value;
-        const v4f* const s_w = reinterpret_cast<const v4f*>(weight_slot<U, s % 2>()) + lane;
-        constexpr int BG = U < 4 ? U : 4;
-        constexpr int NG = U / BG;
-        static_assert(U % BG == 0, "whole groups");
-        constexpr int NI = RB + UW;                  // side items: RB row blocks, then UW weight units
-        constexpr int IPG = (NI + NG - 1) / NG;      // ... per group
-        constexpr int PD = NG >= 3 ? kGroupsAhead : 1;  // groups requested ahead
-        v4f b[PD + 1][BG];
-#pragma unroll
-        for (int g0 = 0; g0 < PD; ++g0)
-#pragma unroll
-            for (int j = 0; j < BG; ++j) b[g0][j] = s_w[(g0 * BG + j) * 64];
-#pragma unroll
-        for (int grp = 0; grp < NG; ++grp) {
-            if (grp + PD < NG) {
-#pragma unroll
-                for (int j = 0; j < BG; ++j) b[(grp + PD) % (PD + 1)][j] = s_w[((grp + PD) * BG + j) * 64];
+    // BY waves a block
+    auto walk = [&](auto by_c) {
+        constexpr int BY = decltype(by_c)::value;
+        if (PAD && wave >= kWaves) {
+            publish();
+            lds_barrier();
+            PadRows<__half, COUT> pads(out, n, max_voxels, blockIdx.x * kPadWaves + (wave - kWaves), gridDim.x * kPadWaves);
+            pads.layer(s_epi, t.has_scale, t.has_shift, relu);
+            pads.rest();
+            if (BY > 1) {  // (the barriers below)
+                lds_barrier();
+                lds_barrier();
             }
-#pragma unroll
-            for (int it = grp * IPG; it < (grp + 1) * IPG && it < NI; ++it) {
-                if (it < RB) {
-                    load_rows1(k + D, std::integral_constant<int, s + D>{}, it);
-                } else {
-                    store_w1(std::integral_constant<int, s + 1>{}, it - RB);
-                    load_w1(k + 1 + DW, std::integral_constant<int, s + 1 + DW>{}, it - RB);
-                }
+            return;
+        }
+        const int part = wave % BY;
+        bool first = true;
+        for (int at = begin; first || at < end; at += kWaves / BY) {
+            const int block = at + wave / BY, row0 = block * 16;
+            const bool work = block < end;  // (uniform)
+            int lane = tid & 63;
+            asm volatile("" : "+v"(lane));  // (or what a round reads from LDS is read in front of the rounds, into registers)
+            int idx[kSteps];
+            v4f acc[NB];
+            if (work) ask_lists<BY>(t, lane, row0, part, idx);
+            if (first) {
+                publish();
+                if (!work) lds_barrier();
             }
-            __builtin_amdgcn_sched_barrier(0);
+            if (work) multiply<COUT, BY>(t, lane, idx, part, s_w, first, acc);
+            if constexpr (BY > 1) {  // (there is one round: a workgroup has at most kWaves / BY blocks)
+                float4* const sums = reinterpret_cast<float4*>(s_w);
+                lds_barrier();
+                if (work && part)
 #pragma unroll
-            for (int j = 0; j < BG; ++j) {
-                const int f = grp * BG + j, g = f / NBT, nb = f % NBT;
+                    for (int nb = 0; nb < NB; ++nb) sums[(wave * NB + nb) * 64 + lane] = make_float4(acc[nb][0], acc[nb][1], acc[nb][2], acc[nb][3]);
+                lds_barrier();
+                if (work && part == 0)
 #pragma unroll
-                for (int blk = 0; blk < RB; ++blk)
-                    acc[blk][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const v8h*>(&b[grp % (PD + 1)][j]),
-                                                                         *reinterpret_cast<const v8h*>(&a[s % NBUF][blk][g]),
-                                                                         acc[blk][nb], 0, 0, 0);
+                    for (int o = BY - 1; o > 0; --o)
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb) {
+                            const float4 v = sums[((wave + o) * NB + nb) * 64 + lane];
+                            acc[nb][0] += v.x;
+                            acc[nb][1] += v.y;
+                            acc[nb][2] += v.z;
+                            acc[nb][3] += v.w;
+                        }
             }
-            __builtin_amdgcn_sched_barrier(0);
+            if (work && part == 0) put<COUT>(t, lane, row0, acc, s_epi, dt);
+            first = false;
         }
     };
-    // prologue: W[0] into its buffer, W[1 .. DW] and the rows of offsets 0 .. D-1 requested
-#pragma unroll
-    for (int j = 0; j < UW; ++j) load_w1(0, std::integral_constant<int, 0>{}, j);
-#pragma unroll
-    for (int j = 0; j < UW; ++j) store_w1(std::integral_constant<int, 0>{}, j);
-    auto ahead = [&](auto self, auto k_c) -> void {
-        constexpr int k = decltype(k_c)::value;
-        if constexpr (k <= DW) {
-#pragma unroll
-            for (int j = 0; j < UW; ++j) load_w1(k, k_c, j);
-            self(self, std::integral_constant<int, k + 1>{});
-        }
-    };
-    ahead(ahead, std::integral_constant<int, 1>{});
-    auto rows_ahead = [&](auto self, auto k_c) -> void {
-        constexpr int k = decltype(k_c)::value;
-        if constexpr (k < D) {
-#pragma unroll
-            for (int blk = 0; blk < RB; ++blk) load_rows1(k, k_c, blk);
-            self(self, std::integral_constant<int, k + 1>{});
-        }
-    };
-    rows_ahead(rows_ahead, std::integral_constant<int, 0>{});
-
-    // positions s .. `last` - 1 of the period that starts at offset k0
-    auto steps = [&](auto self, int k0, auto s_c, auto last_c) -> void {
-        constexpr int s = decltype(s_c)::value;
-        if constexpr (s < decltype(last_c)::value) {
-            // behind this barrier W[k] is in its buffer (every wave stored its share during the previous offset)
-            // and every wave is done with offset k-1, whose buffer W[k+1] now overwrites
-            ring_barrier();
-            offset_step(k0 + s, s_c);
-            self(self, k0, std::integral_constant<int, s + 1>{}, last_c);
-        }
-    };
-    int k0 = 0;
-    for (; k0 + P <= KC; k0 += P) steps(steps, k0, std::integral_constant<int, 0>{}, std::integral_constant<int, P>{});
-    steps(steps, k0, std::integral_constant<int, 0>{}, std::integral_constant<int, KC % P>{});
-
-    // epilogue: lane (i, q) holds output channels 16nb+4q .. +3 of row i of each of its blocks
-#pragma unroll
-    for (int blk = 0; blk < RB; ++blk) {
-        const int row = row0 + (wave * RB + blk) * 16 + i;
-        if (row >= n) continue;
-        bool to_dense = false;
-        __half* d = nullptr;
-        size_t plane = 0;
-        if (dt.dense) {  // the sparse2Dense scatter of this row, fused (uniform branch)
-            const int4 cc = reinterpret_cast<const int4*>(dt.coors)[row];  // (b,z,y,x)
-            if (cc.x != 0 || cc.y < 0 || cc.y >= dt.D || cc.z < 0 || cc.z >= dt.H || cc.w < 0 || cc.w >= dt.W) {
-                if (dt.status && q == 0) atomicOr(dt.status, SESSD_STATUS_BAD_COORD);
-            } else {
-                to_dense = true;
-                d = static_cast<__half*>(dt.dense) + ((size_t)cc.y * dt.Hp + cc.z + dt.pad_top) * dt.Wp + cc.w + dt.pad_left;
-                plane = (size_t)dt.D * dt.Hp * dt.Wp;
-            }
-        }
-#pragma unroll
-        for (int nb = 0; nb < NBT; ++nb) {
-            const int c4 = nb * 16 + q * 4;
-            float o[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                float s = acc[blk][nb][e];
-                if (has_scale) s = s * s_epi[c4 + e];
-                if (has_shift) s = s + s_epi[COUT + c4 + e];
-                if (relu) s = s > 0.f ? s : 0.f;
-                o[e] = s;
-            }
-            store4h(out + (size_t)row * COUT + c4, o);
-            if (to_dense) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) d[(size_t)(c4 + e) * plane] = __float2half_rn(o[e]);
-            }
-        }
-    }
+    if (per <= kWaves / 4) walk(std::integral_constant<int, 4>{});
+    else if (per <= kWaves / 2) walk(std::integral_constant<int, 2>{});
+    else walk(std::integral_constant<int, 1>{});
 }
 
-template <int CIN, int COUT>
-__global__ void __launch_bounds__(kWaves * 64, 2)
-conv_tall(const int32_t* __restrict__ num_out, const int32_t* __restrict__ nbr, const __half* __restrict__ in,
-          const void* __restrict__ Wp, int max_voxels, int slots, int relu, int write_pad, __half* __restrict__ out,
-          const float* __restrict__ scale, const float* __restrict__ shift, DenseTarget dt) {
-    static_assert(CIN % 32 == 0 && COUT % 16 == 0, "whole MFMA chunks");
-    constexpr int RB = kTallBlocks;
-    __shared__ int32_t s_nbr[KC * kWaves * RB * 16];
-    __shared__ float s_epi[2 * COUT];
-    // (the lists wait for nothing else: the arguments in front of `out` are in registers)
-    int n = *num_out;
-    asm volatile("" : "+s"(n));
-    n = n < 0 ? 0 : (n > max_voxels ? max_voxels : n);
-    // Tile heights.  `slots` workgroups are resident at a time.  Up to 64 * slots rows every
-    // tile is 64 rows (one block per wave); beyond that just enough tiles at the head of the grid take RB blocks
-    // per wave for the launch to stay one round of resident workgroups -- a second, mostly empty round costs a
-    // whole tile's time; beyond 64 * RB * slots rows every tile is tall.
-    constexpr int kShort = kWaves * 16, kTall = kShort * RB;
-    int n_tall = 0;
-    if (n > kShort * slots) {
-        n_tall = (n - kShort * slots + (kTall - kShort) - 1) / (kTall - kShort);
-        if (n_tall > slots) n_tall = (n + kTall - 1) / kTall;
-    }
-    const int b = blockIdx.x;
-    if (b < n_tall)
-        tall_tile<CIN, COUT, RB>(in, out, Wp, nbr, n, b * kTall, max_voxels, scale, shift, relu, dt, s_nbr, s_epi);
-    else
-        tall_tile<CIN, COUT, 1>(in, out, Wp, nbr, n, n_tall * kTall + (b - n_tall) * kShort, max_voxels, scale, shift, relu, dt, s_nbr, s_epi);
-    // The rows beyond the active ones are the business of the workgroups without a tile: the grid has one for every 64 rows.
-    const int tiles = n_tall + (n > n_tall * kTall ? (n - n_tall * kTall + kShort - 1) / kShort : 0);
-    const int idle = (int)gridDim.x - tiles;
-    if (write_pad && (b >= tiles || idle == 0)) {
-        if (threadIdx.x < COUT) {
-            s_epi[threadIdx.x] = scale ? scale[threadIdx.x] : 1.f;
-            s_epi[COUT + threadIdx.x] = shift ? shift[threadIdx.x] : 0.f;
-        }
-        __syncthreads();
-        const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-        PadRows<__half, COUT> pads(out, n, max_voxels, (unsigned)((idle ? b - tiles : b) * kWaves + wave), (unsigned)((idle ? idle : (int)gridDim.x) * kWaves));
-        pads.layer(s_epi, scale != nullptr, shift != nullptr, relu);
-        pads.rest();
-    }
-}
-
-template <int CIN, int COUT>
+template <int COUT>
 int launch(const GemmArgs& a, hipStream_t stream) {
     if ((size_t)a.max_voxels * CIN * sizeof(__half) >= kOutOfRange) return SESSD_E_UNSUPPORTED;
-    const int num_cu = gemm_compute_units();
-    const unsigned blocks = (unsigned)((a.max_voxels + 63) / 64);
-    // workgroups of this instantiation a compute unit holds at a time (registers and LDS decide; asked once)
-    static int per_cu = 0;
-    if (per_cu == 0) {
-        int v = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, conv_tall<CIN, COUT>, kWaves * 64, 0) != hipSuccess || v < 1)
-            v = 2;
-        per_cu = v;
-    }
-    hipLaunchKernelGGL((conv_tall<CIN, COUT>), dim3(blocks), dim3(kWaves * 64), 0, stream,
-                       a.num_out, a.nbr, static_cast<const __half*>(a.in_feat), a.w_packed, a.max_voxels, per_cu * num_cu, a.relu,
-                       a.write_pad_rows, static_cast<__half*>(a.out_feat), a.scale, a.shift, a.dense);
+    if ((size_t)a.max_voxels * (KC * sizeof(int32_t)) >= kOutOfRange) return SESSD_E_UNSUPPORTED;
+    auto go = [&](auto pad) {
+        hipLaunchKernelGGL((conv_tall<COUT, decltype(pad)::value>), dim3(gemm_compute_units()),
+                           dim3((kWaves + (decltype(pad)::value ? kPadWaves : 0)) * 64), 0, stream, a.num_out, a.nbr,
+                           static_cast<const __half*>(a.in_feat), a.w_packed, a.max_voxels, a.relu, static_cast<__half*>(a.out_feat), a.scale,
+                           a.shift, a.dense);
+    };
+    a.write_pad_rows ? go(std::true_type{}) : go(std::false_type{});
     SESSD_HIP_TRY(hipGetLastError());
     return SESSD_OK;
 }
@@ -363,8 +302,8 @@ bool gemm_runs_tall(int K, int cin, int cout) { return K == KC && cin == 32 && (
 int launch_tall(const GemmArgs& a, hipStream_t stream) {
     if (!a.w_packed || a.K != KC || a.in_type != SESSD_HALF || a.out_type != SESSD_HALF) return SESSD_E_UNSUPPORTED;
     if ((reinterpret_cast<uintptr_t>(a.in_feat) | reinterpret_cast<uintptr_t>(a.out_feat)) & 15) return SESSD_E_UNSUPPORTED;
-    if (a.cin == 32 && a.cout == 64) return launch<32, 64>(a, stream);
-    if (a.cin == 32 && a.cout == 32) return launch<32, 32>(a, stream);
+    if (a.cin == 32 && a.cout == 64) return launch<64>(a, stream);
+    if (a.cin == 32 && a.cout == 32) return launch<32>(a, stream);
     return SESSD_E_UNSUPPORTED;
 }
 
