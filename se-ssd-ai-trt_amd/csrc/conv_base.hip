@@ -1,5 +1,7 @@
 // conv_base.hip -- what SubmConv3dLayerPlugin and SparseConv3dLayerPlugin share: the device copies
 // of the weights, the fused scale/shift/ReLU epilogue, dtype bookkeeping and the GEMM dispatch.
+#include <cmath>
+
 #include "kernels.h"
 #include "plugins.h"
 
@@ -92,6 +94,11 @@ int ConvPluginBase::preparePacked() {
         SESSD_HIP_TRY(hipMalloc(&weights_packed_dev_, bytes));
         SESSD_HIP_TRY(hipMemcpy(weights_packed_dev_, host.data(), bytes, hipMemcpyHostToDevice));
     }
+    packed_finite_ = true;
+    for (float w : weights_data_) {
+        if (compute_type == SESSD_HALF) (void)nearest_half(w, &w);
+        packed_finite_ = packed_finite_ && std::isfinite(w);
+    }
     packed_dtype_ = compute_type;
     return SESSD_OK;
 }
@@ -125,6 +132,7 @@ int ConvPluginBase::runGemm(const void* in_feat, void* out_feat, const int32_t* 
     a.w_f32 = weights_dev_;
     a.w_f16 = weights_half_dev_;
     a.w_packed = weights_packed_dev_;
+    a.w_finite = packed_finite_;
     a.scale = epi_.scale_dev;
     a.shift = epi_.shift_dev;
     a.relu = epi_.relu;

@@ -1,13 +1,13 @@
-// conv_tall.hip -- gather-GEMM for FP16 3x3x3 layers with Cin 32: all of W in LDS, no barrier between the offsets.
+// conv_tall.hip -- gather-GEMM for FP16 3x3x3 layers with Cin 16 or 32: all of W in LDS, no barrier between the offsets.
 //
 //     out[o][:] = epilogue( sum_k  in[nbr[k][o]][:] @ W[k] )
 //
-// W is 55 or 110 KB and one workgroup a compute unit keeps all of it, so that its waves meet only once, in front of the first product.
+// W is 14 to 110 KB and one workgroup a compute unit keeps all of it, so that its waves meet only once, in front of the first product.
 //   * A workgroup owns a run of output rows, 16 at a time (a block) for each of its eight waves, and all columns; the accumulators stay
 //     in registers over all offsets: no compaction, no partial tiles.  A row without a neighbour contributes a zero operand (a buffer
 //     load that points out of range: zeros, no memory touched), so the matrix cores multiply about twice the useful pairs -- in FP16
 //     they have the headroom.
-//   * A step is four offsets.  Lane (i, q) of a wave requests all 64 bytes of the neighbour of row i at offset 4 step + q, and the inner
+//   * A step is four offsets.  Lane (i, q) of a wave requests all 32 or 64 bytes of the neighbour of row i at offset 4 step + q, and the inner
 //     dimension of an MFMA is eight channels of each of the four offsets: the lane's own list entries are all that it needs, no other
 //     lane's, and W is in LDS as the host has packed it (lane (i, q) reads the operand that holds these channels of W[4 step + q]).
 //     Rows are requested two steps (eight offsets) ahead, all of them by straight-line code: the compiler's waits are exact.
@@ -19,7 +19,9 @@
 // the trips to memory: row count, lists, rows.
 // Measured against the kernel with a barrier and 2 or 4 KB of W an offset that these layers ran on, launches back to back, 32 -> 32 and
 // 32 -> 64: 801 rows 5.05 -> 3.5 us and 5.9 -> 4.8, 13 907 rows 5.3 -> 4.7 and 6.2 -> 6.25, 26 575 rows 7.1 -> 5.7 and 7.9 -> 7.3,
-// 49 874 rows 11.2 -> 8.4 and 13.1 -> 10.9, 74 606 rows 13.9 -> 10.9 and 16.1 -> 13.4; frames of 60 000 points 230.6 -> 226.6.
+// 49 874 rows 11.2 -> 8.4 and 13.1 -> 10.9, 74 606 rows 13.9 -> 10.9 and 16.1 -> 13.4; frames of 60 000 points 229.6 -> 224.9.
+// 16 -> 16 and 16 -> 32 against conv_wide.hip's pair lists (a quarter of the neighbours is there): 1 947 rows 5.0 -> 2.9 us and 5.2 -> 3.2,
+// 16 198 rows 7.2 -> 3.3 and 8.1 -> 3.7, 60 000 rows 10.4 -> 4.9 and 11.9 -> 5.8; frames of 60 000 points 225.9 -> 215.7.
 // The waves are eight because the coordinate passes beside them need registers (12: the same times, and 504 of 512 taken).
 // Summation order per output element: steps ascending, in a step the channels eight at a time: fixed, run-to-run identical.
 // (The ring of conv_tile.hip, faster from 64 channels up, has too little work per row here.)
@@ -31,6 +33,7 @@ namespace sessd {
 
 namespace {
 
+typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef unsigned int v4u32 __attribute__((__vector_size__(16)));
@@ -39,10 +42,10 @@ constexpr int kWaves = 8;     // that multiply
 constexpr int kPadWaves = 4;  // that write the rows beyond the active ones
 constexpr int KC = 27;                  // kernel offsets: the 3x3x3 layers
 constexpr int kSteps = (KC + 3) / 4;    // of four offsets
-constexpr int CIN = 32, kPieces = 4;    // 16-byte pieces of a row
 constexpr unsigned kOutOfRange = 0x80000000u;
 constexpr int kRawBuffer = 0x00020000;
-constexpr int kDepth = 2;  // steps whose rows are on their way (3: the same times, 16 registers more)
+// steps whose rows are on their way (with 32 channels 3: the same times, 16 registers more)
+constexpr int depth(int cin) { return cin == 32 ? 2 : 3; }
 
 __device__ __forceinline__ void store4h(__half* dst, const float (&o)[4]) {
     union {
@@ -84,10 +87,11 @@ __device__ __forceinline__ void ask_lists(const Tensors& t, int lane, int row0, 
 }
 
 // Steps first, first + BY, ... of the block
-template <int COUT, int BY>
+template <int CIN, int COUT, int BY>
 __device__ __forceinline__ void multiply(const Tensors& t, int lane, const int (&idx)[kSteps], int first, const unsigned char* s_w, bool wait_for_w,
                                          v4f (&acc)[COUT / 16]) {
-    constexpr int NB = COUT / 16, N = (kSteps + BY - 1) / BY;
+    constexpr int NB = COUT / 16, N = (kSteps + BY - 1) / BY, kPieces = CIN / 8;  // (16 bytes of a row each)
+    constexpr int kDepth = depth(CIN) < N ? depth(CIN) : N;
     const int i = lane & 15, q = lane >> 4;
     v4u32 x[kDepth][kPieces];
     auto request = [&](int m) {  // (m < N)
@@ -95,15 +99,14 @@ __device__ __forceinline__ void multiply(const Tensors& t, int lane, const int (
 #pragma unroll
         for (int p = 0; p < kPieces; ++p) x[m % kDepth][p] = __builtin_amdgcn_raw_buffer_load_b128(t.in, at + p * 16u, 0, 0);
     };
-    static_assert(N >= kDepth, "steps");
 #pragma unroll
     for (int m = 0; m < kDepth; ++m) request(m);
     if (wait_for_w) lds_barrier();
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[nb] = (v4f){0.f, 0.f, 0.f, 0.f};
-    const unsigned char* w_at = s_w + (first * 4 + q) * (NB * 1024) + i * 16;
+    const unsigned char* w_at = s_w + (first * 4 + q) * (NB * kPieces * 256) + i * 16;
 #pragma unroll
-    for (int m = 0; m < N; ++m, w_at += BY * 4 * NB * 1024) {
+    for (int m = 0; m < N; ++m, w_at += BY * 4 * NB * kPieces * 256) {
         if (BY > 1 && first + m * BY >= kSteps) break;  // (uniform)
         // (the weights of a piece or two at a time: registers)
         constexpr int kAtOnce = NB > 2 ? 1 : 2;
@@ -112,7 +115,7 @@ __device__ __forceinline__ void multiply(const Tensors& t, int lane, const int (
 #pragma unroll
             for (int a = 0; a < kAtOnce; ++a)
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb) to[a][nb] = *reinterpret_cast<const v8h*>(w_at + nb * 1024 + (p + a) * 256);
+                for (int nb = 0; nb < NB; ++nb) to[a][nb] = *reinterpret_cast<const v8h*>(w_at + (nb * kPieces + p + a) * 256);
         };
         weights(0, w[0]);
 #pragma unroll
@@ -171,17 +174,17 @@ __device__ __forceinline__ void put(const Tensors& t, int lane, int row0, const 
     }
 }
 
-template <int COUT, bool PAD>
+template <int CIN, int COUT, bool PAD>
 __global__ void __launch_bounds__((kWaves + (PAD ? kPadWaves : 0)) * 64)
 conv_tall(const int32_t* __restrict__ num_out, const int32_t* __restrict__ nbr, const __half* __restrict__ in,
           const void* __restrict__ Wp, int max_voxels, int relu, __half* __restrict__ out,
           const float* __restrict__ scale, const float* __restrict__ shift, DenseTarget dt) {
     constexpr int NB = COUT / 16, kThreads = (kWaves + (PAD ? kPadWaves : 0)) * 64;
-    constexpr int kOffsetBytes = NB * 1024, kVectors = KC * kOffsetBytes / 16, kCopies = (kVectors + kThreads - 1) / kThreads;
+    constexpr int kOffsetBytes = CIN * COUT * 2, kVectors = KC * kOffsetBytes / 16, kCopies = (kVectors + kThreads - 1) / kThreads;
     // (one offset more than there are, of zeros)
     __shared__ __align__(16) unsigned char s_w[kSteps * 4 * kOffsetBytes];
     __shared__ float s_epi[2 * COUT];
-    static_assert(kSteps * 4 == KC + 1, "steps");
+    static_assert(kSteps * 4 == KC + 1 && sizeof(s_w) >= kWaves * NB * 1024, "steps; the sums of waves that share a block");
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     v4f copy[kCopies];
@@ -214,7 +217,15 @@ conv_tall(const int32_t* __restrict__ num_out, const int32_t* __restrict__ nbr, 
 #pragma unroll
         for (int c = 0; c < kCopies; ++c) {
             const int v = c * kThreads + tid;
-            if (v < kVectors) reinterpret_cast<v4f*>(s_w)[v] = copy[c];
+            if (v >= kVectors) continue;
+            if constexpr (CIN == 32) {
+                reinterpret_cast<v4f*>(s_w)[v] = copy[c];
+            } else {  // (packed four channels of a column at a time: here eight)
+                const int in_block = v & 31, g = in_block >> 3, i = (in_block & 7) * 2;  // of a column block: channels 4g .., columns i, i + 1
+                unsigned char* to = s_w + (v >> 5) * 512 + (g >> 1) * 256 + i * 16 + (g & 1) * 8;
+                *reinterpret_cast<v2f*>(to) = (v2f){copy[c][0], copy[c][1]};
+                *reinterpret_cast<v2f*>(to + 16) = (v2f){copy[c][2], copy[c][3]};
+            }
         }
         if (tid < kOffsetBytes / 16) reinterpret_cast<v4f*>(s_w)[kVectors + tid] = (v4f){0.f, 0.f, 0.f, 0.f};
         if (tid < COUT) {
@@ -251,7 +262,7 @@ conv_tall(const int32_t* __restrict__ num_out, const int32_t* __restrict__ nbr, 
                 publish();
                 if (!work) lds_barrier();
             }
-            if (work) multiply<COUT, BY>(t, lane, idx, part, s_w, first, acc);
+            if (work) multiply<CIN, COUT, BY>(t, lane, idx, part, s_w, first, acc);
             if constexpr (BY > 1) {  // (there is one round: a workgroup has at most kWaves / BY blocks)
                 float4* const sums = reinterpret_cast<float4*>(s_w);
                 lds_barrier();
@@ -280,12 +291,12 @@ conv_tall(const int32_t* __restrict__ num_out, const int32_t* __restrict__ nbr, 
     else walk(std::integral_constant<int, 1>{});
 }
 
-template <int COUT>
+template <int CIN, int COUT>
 int launch(const GemmArgs& a, hipStream_t stream) {
     if ((size_t)a.max_voxels * CIN * sizeof(__half) >= kOutOfRange) return SESSD_E_UNSUPPORTED;
     if ((size_t)a.max_voxels * (KC * sizeof(int32_t)) >= kOutOfRange) return SESSD_E_UNSUPPORTED;
     auto go = [&](auto pad) {
-        hipLaunchKernelGGL((conv_tall<COUT, decltype(pad)::value>), dim3(gemm_compute_units()),
+        hipLaunchKernelGGL((conv_tall<CIN, COUT, decltype(pad)::value>), dim3(gemm_compute_units()),
                            dim3((kWaves + (decltype(pad)::value ? kPadWaves : 0)) * 64), 0, stream, a.num_out, a.nbr,
                            static_cast<const __half*>(a.in_feat), a.w_packed, a.max_voxels, a.relu, static_cast<__half*>(a.out_feat), a.scale,
                            a.shift, a.dense);
@@ -297,13 +308,16 @@ int launch(const GemmArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-bool gemm_runs_tall(int K, int cin, int cout) { return K == KC && cin == 32 && (cout == 64 || cout == 32); }
+bool gemm_runs_tall(int K, int cin, int cout) { return K == KC && ((cin == 32 && (cout == 64 || cout == 32)) || (cin == 16 && (cout == 16 || cout == 32))); }
 
 int launch_tall(const GemmArgs& a, hipStream_t stream) {
-    if (!a.w_packed || a.K != KC || a.in_type != SESSD_HALF || a.out_type != SESSD_HALF) return SESSD_E_UNSUPPORTED;
+    // (0 x infinity: with weights that are not finite an absent neighbour may not be a row of zeros)
+    if (!a.w_packed || !a.w_finite || a.K != KC || a.in_type != SESSD_HALF || a.out_type != SESSD_HALF) return SESSD_E_UNSUPPORTED;
     if ((reinterpret_cast<uintptr_t>(a.in_feat) | reinterpret_cast<uintptr_t>(a.out_feat)) & 15) return SESSD_E_UNSUPPORTED;
-    if (a.cin == 32 && a.cout == 64) return launch<64>(a, stream);
-    if (a.cin == 32 && a.cout == 32) return launch<32>(a, stream);
+    if (a.cin == 32 && a.cout == 64) return launch<32, 64>(a, stream);
+    if (a.cin == 32 && a.cout == 32) return launch<32, 32>(a, stream);
+    if (a.cin == 16 && a.cout == 16) return launch<16, 16>(a, stream);
+    if (a.cin == 16 && a.cout == 32) return launch<16, 32>(a, stream);
     return SESSD_E_UNSUPPORTED;
 }
 

@@ -1,5 +1,5 @@
-// conv_wide.hip -- gather-GEMM of the FP32 layers, of the FP16 layers that conv_tile.hip and conv_tall.hip do not take (Cin 16, kernel
-// volumes other than theirs) and of an FP16 pipeline's first layer.
+// conv_wide.hip -- gather-GEMM of the FP32 layers, of the FP16 layers that conv_tile.hip and conv_tall.hip do not take (kernel
+// volumes other than theirs, weights that are not finite) and of an FP16 pipeline's first layer.
 //
 //     out[o][:] = epilogue( sum_k  in[nbr[k][o]][:] @ W[k] )
 //

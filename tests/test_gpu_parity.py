@@ -953,6 +953,37 @@ def test_tall_fp16_kernel_with_tall_tiles(cout, n):
         O.set_threads(1)
 
 
+@pytest.mark.parametrize("cin,cout", [(16, 16), (16, 32), (32, 32), (32, 64)])
+@pytest.mark.parametrize("n", [1, 17, 4095, 8192, 8193, 16385, 32768, 32769, 33000, 66000])
+def test_fp16_kernel_with_all_weights_in_lds(cin, cout, n):
+    """On 256 compute units four waves share 16 rows up to 8 192 rows, two up to 16 384; from 32 769 on waves take a second block."""
+    O.set_threads(16)
+    try:
+        _fp16_subm_against_oracle(cin, cout, n, n + 70 if n % 2 else n, (41, 400, 352), n + cout)
+    finally:
+        O.set_threads(1)
+
+
+@pytest.mark.parametrize("cin,cout,half", [(16, 16, True), (16, 32, True), (32, 32, True), (32, 64, True), (4, 16, False), (16, 16, False)])
+def test_an_infinite_weight_reaches_the_rows_that_have_the_neighbour(cin, cout, half):
+    """... and makes no NaN of the others, whose absent neighbours are multiplied as rows of zeros where all weights are finite."""
+    rng = np.random.default_rng(cin + cout)
+    grid, n, mv = (11, 200, 176), 9000, 9100
+    coors = np.zeros((mv, 4), np.int32)
+    coors[:n] = F.clustered_active_voxels(n, grid, 3, n_blobs=60)
+    feat = rng.uniform(0.5, 1, (mv, cin)).astype(np.float32)
+    w = O.round_to_half(rng.normal(0, 0.1, (27, cin, cout)).astype(np.float32))
+    w[5, 1, 2] = 1e6 if half else np.inf  # (infinite as a half)
+    conv = api.SubmConv3d(cin, cout, grid[::-1], w, mv)
+    out = to_np(conv(dev(feat, torch.float16 if half else None), dev(coors), dev(np.array([n], np.int32))).float())
+    pairs, num = (to_np(t) for t in conv.export_rulebook())
+    want = np.zeros(n, bool)
+    want[pairs[5, 1, :num[5]]] = True
+    assert want.any() and not want.all()
+    assert np.array_equal(np.isinf(out[:n, 2]), want) and np.isfinite(np.delete(out[:n], 2, 1)).all() and not np.isnan(out).any()
+    conv.close()
+
+
 @pytest.mark.parametrize("cin,cout,n", [(64, 64, 16384), (64, 64, 16385), (64, 64, 65537), (64, 64, 81920), (64, 64, 81921),
                                         (64, 128, 8193), (128, 128, 8192), (128, 128, 8193), (128, 128, 32769), (128, 128, 49152),
                                         (128, 128, 49153)])
