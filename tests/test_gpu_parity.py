@@ -430,7 +430,7 @@ def test_subm_shared_rulebook_skip_pad_and_empty():
 
 @pytest.mark.parametrize("owner_cout,sharer_cout", [(64, 32), (32, 64)])
 def test_shared_rulebook_between_layers_of_different_tile_capacity(owner_cout, sharer_cout):
-    """Two FP16 3x3x3 layers of different widths on one rulebook.  Both run on the tall-tile kernel, which cuts
+    """Two FP16 3x3x3 layers of different widths on one rulebook.  Both run on the kernel of conv_tall.hip, which cuts
     its own tiles (a rulebook built by such a layer carries no equal-work cuts) and sums a row's offsets in
     ascending order whatever tile the row falls in: the sharer's output on the owner's rulebook must equal its
     output on its own bit for bit."""
@@ -892,8 +892,8 @@ def test_conv_plugins_by_name_and_their_clones():
 
 
 # ---------------------------------------------------------------------------------------------
-# the FP16 kernels that cut their own tiles (3x3x3 layers from 32 channels up): with 32 input channels the tall-tile kernel
-# (conv_tall.hip), from 64 up the ring of LDS buffers (conv_tile.hip); tile edges and tile heights
+# the FP16 kernels that cut their own tiles (3x3x3 layers from 16 channels up): with 16 and 32 input channels the one that keeps all
+# weights in LDS (conv_tall.hip), from 64 up the ring of LDS buffers (conv_tile.hip); tile edges and tile heights
 # ---------------------------------------------------------------------------------------------
 def _fp16_subm_against_oracle(cin, cout, n, mv, grid, seed, clustered=True, epilogue=True):
     rng = np.random.default_rng(seed)
@@ -924,16 +924,16 @@ def _fp16_subm_against_oracle(cin, cout, n, mv, grid, seed, clustered=True, epil
 @pytest.mark.parametrize("cin,cout", [(32, 32), (64, 64), (128, 128)])
 @pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 300])
 def test_tall_fp16_kernel_row_counts_around_its_tiles(cin, cout, n):
-    """A tile of the tall-tile kernel is 64 rows, 16 per wave (32 -> 32), one of the ring kernel 64 or 32 at these row counts:
-    row counts on either side of a block, a wave's share and a tile, down to a single row, against the oracle (pad rows
+    """A wave of the kernel with all weights in LDS has 16 rows (32 -> 32), a tile of the ring kernel 64 or 32 at these row counts:
+    row counts on either side of a block and a tile, down to a single row, against the oracle (pad rows
     included)."""
     _fp16_subm_against_oracle(cin, cout, n, 512, (5, 40, 40), 900 + n, epilogue=(n % 2 == 1))
 
 
 @pytest.mark.parametrize("cin,cout,n", [(32, 32, 66000), (64, 64, 40000), (64, 128, 66000), (128, 128, 40000), (128, 128, 66000)])
 def test_tall_fp16_kernel_with_two_row_blocks_per_wave(cin, cout, n):
-    """Launches of many rows, the last tile partly filled, against the oracle on 16 threads: short tiles only on the
-    tall-tile kernel (32 -> 32; its tall tiles: the test below), tiles of several blocks a wave on the ring kernel."""
+    """Launches of many rows, the last tile partly filled, against the oracle on 16 threads: two or three blocks for a wave, one
+    after the other with 32 channels, in one tile on the ring kernel."""
     O.set_threads(16)
     try:
         _fp16_subm_against_oracle(cin, cout, n, 66560, (21, 400, 352), 4000 + cin + cout)
@@ -943,9 +943,7 @@ def test_tall_fp16_kernel_with_two_row_blocks_per_wave(cin, cout, n):
 
 @pytest.mark.parametrize("cout,n", [(32, 81920), (32, 81921), (32, 120000), (32, 163841), (64, 65536), (64, 65537), (64, 100000), (64, 131073)])
 def test_tall_fp16_kernel_with_tall_tiles(cout, n):
-    """Beyond 64 rows x the workgroups resident at a time (1280 of the 32 -> 32 kernel, 1024 of 32 -> 64 by their registers on
-    256 compute units), tiles at the head of the grid take two 16-row blocks per wave (128 rows): the last launch of
-    short tiles, one with a single tall tile, short and tall ones side by side, and tall ones only."""
+    """Launches of so many rows that every wave walks two to five blocks of 16, some a block more than others."""
     O.set_threads(16)
     try:
         _fp16_subm_against_oracle(32, cout, n, n + 70, (41, 400, 352), 8000 + cout)
