@@ -338,13 +338,15 @@ def check_order():
         assert (first[0] < first[1]) == chain, (len(layers), dtype, points, first)
 
 
-def gemm_kernel(cin, cout, rows, dtype):
-    """The kernel that multiplies in a SubM layer of so many rows (nothing runs: the addresses are read by nobody)."""
+def gemm_kernel(cin, cout, rows, dtype, weight=0.0):
+    """The kernel that multiplies in a SubM layer of so many rows, `weight` being one of its weights and the others 0 (nothing runs: the
+    addresses are read by nobody)."""
     d = D.SubmConv3dDesc()
     d.in_channel, d.out_channel, d.max_voxels, d.feature_num, d.ksize, d.stride, d.padding, d.dilation = cin, cout, rows, cin, 3, 1, 1, 1
     for a in range(3):
         d.out_shape[a] = d.spatial_shape[a] = 1000
     w, h = np.zeros((27, cin, cout), np.float32), C.c_void_p()
+    w[5, 1, 2] = weight
     assert L.sessd_submconv3d_create(C.byref(d), w.ctypes.data, C.byref(h)) == 0, L.sessd_last_error()
     ins = (D.TensorDesc * 3)(D.TensorDesc.make((1, rows, cin), dtype), D.TensorDesc.make((1, rows, 4), D.SESSD_INT32),
                              D.TensorDesc.make((1,), D.SESSD_INT32))
@@ -368,7 +370,20 @@ def check_row_limits():
         assert "conv_wide" not in gemm_kernel(cin, cout, most + 1, dtype), (cin, cout, dtype)
 
 
+def check_weights_not_finite():
+    """FP16 layers run on the kernels that multiply an absent neighbour as a row of zeros only where all weights are finite as halves."""
+    f32, f16 = D.SESSD_FLOAT, D.SESSD_HALF
+    for cin, cout in ((16, 16), (16, 32), (32, 32), (32, 64), (64, 64), (64, 128), (128, 128)):
+        own = "conv_tile" if cin >= 64 else "conv_tall"
+        for weight in (0.0, 65504.0, -65519.0, 1e-30):
+            assert own in gemm_kernel(cin, cout, 9000, f16, weight), (cin, cout, weight)
+        for weight in (65520.0, -1e6, np.inf, -np.inf, np.nan):
+            assert "conv_wide" in gemm_kernel(cin, cout, 9000, f16, weight), (cin, cout, weight)
+            assert "conv_wide" in gemm_kernel(cin, cout, 9000, f32, weight), (cin, cout, weight)
+
+
 CHECKS = {
+    "weights-not-finite": check_weights_not_finite,
     "events": check_events,
     "waits": check_waits,
     "order": check_order,

@@ -962,24 +962,65 @@ def test_fp16_kernel_with_all_weights_in_lds(cin, cout, n):
         O.set_threads(1)
 
 
-@pytest.mark.parametrize("cin,cout,half", [(16, 16, True), (16, 32, True), (32, 32, True), (32, 64, True), (4, 16, False), (16, 16, False)])
+def _check_infinite_weight(conv, out, n_out, feat, w):
+    """Column 2 of the rows with a neighbour at the weight's offset is infinite; everything else is what the oracle makes of the other
+    weights and the layer's own rulebook."""
+    pairs, num = (to_np(t) for t in conv.export_rulebook())
+    (k,), mv = np.unique(np.nonzero(~np.isfinite(O.round_to_half(w)))[0]), len(feat)
+    has = np.zeros(n_out, bool)
+    has[pairs[k, 1, :num[k]]] = True
+    assert has.any() and not has.all()
+    assert not np.isnan(out).any() and np.array_equal(np.isinf(out[:n_out, 2]), has)
+    finite = np.where(np.isfinite(O.round_to_half(w)), w, np.float32(0))
+    O.set_threads(16)
+    try:
+        want = O.gather_gemm_scatter(feat, finite, pairs, num, mv)
+        terms = O.gather_gemm_scatter(np.abs(feat), np.abs(finite), pairs, num, mv)
+    finally:
+        O.set_threads(1)
+    got = out.copy()
+    for v in (got, want, terms):
+        v[:n_out][has, 2] = 0
+    return got, want, terms
+
+
+@pytest.mark.parametrize("cin,cout,half", [(16, 16, True), (16, 32, True), (32, 32, True), (32, 64, True), (64, 64, True), (64, 128, True),
+                                           (128, 128, True), (4, 16, False), (16, 16, False)])
 def test_an_infinite_weight_reaches_the_rows_that_have_the_neighbour(cin, cout, half):
-    """... and makes no NaN of the others, whose absent neighbours are multiplied as rows of zeros where all weights are finite."""
+    """... and makes no NaN of the others, whose absent neighbours are multiplied as rows of zeros where all weights are finite; the other
+    columns are what they are without it."""
     rng = np.random.default_rng(cin + cout)
     grid, n, mv = (11, 200, 176), 9000, 9100
     coors = np.zeros((mv, 4), np.int32)
     coors[:n] = F.clustered_active_voxels(n, grid, 3, n_blobs=60)
-    feat = rng.uniform(0.5, 1, (mv, cin)).astype(np.float32)
+    feat = O.round_to_half(rng.uniform(0.5, 1, (mv, cin)).astype(np.float32))
     w = O.round_to_half(rng.normal(0, 0.1, (27, cin, cout)).astype(np.float32))
     w[5, 1, 2] = 1e6 if half else np.inf  # (infinite as a half)
     conv = api.SubmConv3d(cin, cout, grid[::-1], w, mv)
     out = to_np(conv(dev(feat, torch.float16 if half else None), dev(coors), dev(np.array([n], np.int32))).float())
-    pairs, num = (to_np(t) for t in conv.export_rulebook())
-    want = np.zeros(n, bool)
-    want[pairs[5, 1, :num[5]]] = True
-    assert want.any() and not want.all()
-    assert np.array_equal(np.isinf(out[:n, 2]), want) and np.isfinite(np.delete(out[:n], 2, 1)).all() and not np.isnan(out).any()
+    got, want, terms = _check_infinite_weight(conv, out, n, feat, w)
+    assert_features_close(got, O.round_to_half(want) if half else want, RTOL_FP16 if half else RTOL_FP32, "%d->%d beside an infinite weight" % (cin, cout),
+                          abs_sum=terms, half=half)
     conv.close()
+
+
+@pytest.mark.parametrize("channels", [64, 128])
+def test_an_infinite_weight_of_the_last_layer_reaches_the_rows_that_have_the_neighbour(channels):
+    """The same for the 3x1x1 layer that ends an FP16 backbone."""
+    layer = SPARSE_LAYERS[3]
+    ig = sparse_input_grid(layer)
+    rng = np.random.default_rng(channels)
+    n, mv = 9000, 18000
+    coors = np.zeros((mv, 4), np.int32)
+    coors[:n] = F.clustered_active_voxels(n, ig, 5, n_blobs=60)
+    feat = O.round_to_half(rng.uniform(0.5, 1, (mv, channels)).astype(np.float32))
+    w = O.round_to_half(rng.normal(0, 0.1, (3, channels, channels)).astype(np.float32))
+    w[1, 1, 2] = 1e6  # (infinite as a half)
+    op = api.SparseConv3d(channels, channels, layer.out_shape, ig[::-1], layer.ksize, layer.stride, layer.padding, w, mv)
+    out, _, num_out = op(dev(feat, torch.float16), dev(coors), dev(np.array([n], np.int32)))
+    got, want, terms = _check_infinite_weight(op, to_np(out.float()), int(to_np(num_out)[0]), feat, w)
+    assert_features_close(got, O.round_to_half(want), RTOL_FP16, "3x1x1 beside an infinite weight", abs_sum=terms, half=True)
+    op.close()
 
 
 @pytest.mark.parametrize("cin,cout,n", [(64, 64, 16384), (64, 64, 16385), (64, 64, 65537), (64, 64, 81920), (64, 64, 81921),

@@ -42,6 +42,10 @@ def test_layers_with_few_channels_run_on_the_matrix_cores_in_large_tensors(fake_
     run_check(fake_hip, "row-limits")
 
 
+def test_layers_with_weights_that_are_not_finite_multiply_no_absent_neighbours(fake_hip):
+    run_check(fake_hip, "weights-not-finite")
+
+
 def test_host_memory_that_runs_out_in_a_frame_is_an_error_code(fake_hip):
     run_check(fake_hip, "host-memory")
 
