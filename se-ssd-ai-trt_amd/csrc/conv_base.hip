@@ -1,7 +1,5 @@
 // conv_base.hip -- what SubmConv3dLayerPlugin and SparseConv3dLayerPlugin share: the device copies
 // of the weights, the fused scale/shift/ReLU epilogue, dtype bookkeeping and the GEMM dispatch.
-#include <cmath>
-
 #include "kernels.h"
 #include "plugins.h"
 
@@ -32,7 +30,12 @@ int ConvPluginBase::uploadWeights(const float* w, size_t count) {
     SESSD_HIP_TRY(hipMemcpy(weights_dev_, w, count * sizeof(float), hipMemcpyHostToDevice));
     std::vector<uint16_t> h(count);
     float value;
-    for (size_t i = 0; i < count; ++i) h[i] = nearest_half(w[i], &value);
+    bool beyond = false;  // (asked here: another pass over the weights is as long as packing them)
+    for (size_t i = 0; i < count; ++i) {
+        h[i] = nearest_half(w[i], &value);
+        beyond |= (h[i] & 0x7c00u) == 0x7c00u;
+    }
+    halves_finite_ = !beyond;
     SESSD_HIP_TRY(hipMalloc(reinterpret_cast<void**>(&weights_half_dev_), count * sizeof(__half)));
     SESSD_HIP_TRY(hipMemcpy(weights_half_dev_, h.data(), count * sizeof(__half), hipMemcpyHostToDevice));
     packed_dtype_ = -1;
@@ -94,11 +97,6 @@ int ConvPluginBase::preparePacked() {
         SESSD_HIP_TRY(hipMalloc(&weights_packed_dev_, bytes));
         SESSD_HIP_TRY(hipMemcpy(weights_packed_dev_, host.data(), bytes, hipMemcpyHostToDevice));
     }
-    packed_finite_ = true;
-    for (float w : weights_data_) {
-        if (compute_type == SESSD_HALF) (void)nearest_half(w, &w);
-        packed_finite_ = packed_finite_ && std::isfinite(w);
-    }
     packed_dtype_ = compute_type;
     return SESSD_OK;
 }
@@ -132,7 +130,7 @@ int ConvPluginBase::runGemm(const void* in_feat, void* out_feat, const int32_t* 
     a.w_f32 = weights_dev_;
     a.w_f16 = weights_half_dev_;
     a.w_packed = weights_packed_dev_;
-    a.w_finite = packed_finite_;
+    a.halves_finite = halves_finite_;
     a.scale = epi_.scale_dev;
     a.shift = epi_.shift_dev;
     a.relu = epi_.relu;

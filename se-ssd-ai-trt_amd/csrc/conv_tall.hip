@@ -314,7 +314,7 @@ int launch_tall(const GemmArgs& a, hipStream_t stream) {
     // (FP32 layers stay on the pair lists: 4 -> 16 and 16 -> 16 are faster this way, at 16 198 rows 5.8 -> 3.6 and 6.6 -> 5.4 us, but what the
     // lists leave of a unit is what the coordinate passes of a frame run in: 20 000 points 263.0 -> 264.9 us, 80 000 408 -> 415)
     // (0 x infinity: with weights that are not finite an absent neighbour may not be a row of zeros)
-    if (!a.w_packed || !a.w_finite || a.K != KC || a.in_type != SESSD_HALF || a.out_type != SESSD_HALF) return SESSD_E_UNSUPPORTED;
+    if (!a.w_packed || !a.halves_finite || a.K != KC || a.in_type != SESSD_HALF || a.out_type != SESSD_HALF) return SESSD_E_UNSUPPORTED;
     if ((reinterpret_cast<uintptr_t>(a.in_feat) | reinterpret_cast<uintptr_t>(a.out_feat)) & 15) return SESSD_E_UNSUPPORTED;
     if (a.cin == 32 && a.cout == 64) return launch<32, 64>(a, stream);
     if (a.cin == 32 && a.cout == 32) return launch<32, 32>(a, stream);

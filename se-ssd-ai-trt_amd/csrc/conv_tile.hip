@@ -380,7 +380,7 @@ bool gemm_runs_tile(int K, int cin, int cout) {
 
 int launch_tile(const GemmArgs& a, hipStream_t stream) {
     // (0 x infinity: with weights that are not finite an absent neighbour may not be a row of zeros)
-    if (!a.w_packed || !a.w_finite || a.in_type != SESSD_HALF || a.out_type != SESSD_HALF) return SESSD_E_UNSUPPORTED;
+    if (!a.w_packed || !a.halves_finite || a.in_type != SESSD_HALF || a.out_type != SESSD_HALF) return SESSD_E_UNSUPPORTED;
     if ((reinterpret_cast<uintptr_t>(a.in_feat) | reinterpret_cast<uintptr_t>(a.out_feat)) & 15) return SESSD_E_UNSUPPORTED;
     if (a.K == 3) {
         if (a.cin == 128 && a.cout == 128) return launch<128, 128, 3>(a, stream);

@@ -102,7 +102,7 @@ class ConvPluginBase {
     __half* weights_half_dev_ = nullptr;  // FP16 copy of the same layout
     void* weights_packed_dev_ = nullptr;  // MFMA B-operand order (see conv_gemm.hip)
     int packed_dtype_ = -1;
-    bool packed_finite_ = false;  // no infinity and no NaN among the packed weights
+    bool halves_finite_ = false;  // no infinity and no NaN among the FP16 weights
     Epilogue epi_;
     int in_type_ = SESSD_FLOAT, out_type_ = SESSD_FLOAT;
     int flags_ = 0;

@@ -46,6 +46,10 @@ def test_layers_with_weights_that_are_not_finite_multiply_no_absent_neighbours(f
     run_check(fake_hip, "weights-not-finite")
 
 
+def test_configuring_a_layer_for_fp16_packs_its_weights_and_no_more(fake_hip):
+    run_check(fake_hip, "first-configure")
+
+
 def test_host_memory_that_runs_out_in_a_frame_is_an_error_code(fake_hip):
     run_check(fake_hip, "host-memory")
 
