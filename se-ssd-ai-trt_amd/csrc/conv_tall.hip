@@ -239,9 +239,8 @@ conv_tall(const int32_t* __restrict__ num_out, const int32_t* __restrict__ nbr, 
         if (PAD && wave >= kWaves) {
             publish();
             lds_barrier();
-            PadRows<__half, COUT> pads(out, n, max_voxels, blockIdx.x * kPadWaves + (wave - kWaves), gridDim.x * kPadWaves);
-            pads.layer(s_epi, t.has_scale, t.has_shift, relu);
-            pads.rest();
+            write_pad_rows<__half, COUT>(out, n, max_voxels, blockIdx.x * (kPadWaves * 64) + (tid - kWaves * 64), gridDim.x * (kPadWaves * 64), s_epi, t.has_scale,
+                                         t.has_shift, relu);
             if (BY > 1) {  // (the barriers below)
                 lds_barrier();
                 lds_barrier();

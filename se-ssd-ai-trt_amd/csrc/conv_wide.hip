@@ -566,10 +566,12 @@ conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles
     if (cut_count == 0) plan = tile_plan(n, walkers, kMaxSplit && lsplit ? kTileRows : S::kWholeRows);
     const int tile_count = cut_count > 0 ? cut_count : (n > 0 ? plan.count : 0);
     bool idle = true;  // (no rows)
-    auto pads = [&]() {
-        if constexpr (PAD) return PadRows<TO, COUT>(out, n, max_voxels, blockIdx.x * kWaves + own_wave, gridDim.x * kWaves);
-        else return NoPadRows();
-    }();
+    // Rows beyond the active ones: beside the products of a workgroup's first tile where there are as many of them as of the others, else
+    // behind its last.  A step is paid for with every block of pairs, whether the wave has anything left to write or not.  Behind / beside:
+    // 64 -> 64 at 30 000 rows, 2 000 to write 29.3 / 29.6 us, 20 000 29.6 / 29.4, 50 000 30.8 / 29.8; 32 -> 32 12.2 / 12.6, 12.5 / 12.7, 13.0 / 12.8;
+    // 4 -> 16 at 8 000 rows, 8 000 to write 5.7 / 5.5, at 50 000 rows 9.7 / 9.8, 150 000 to write 11.2 / 10.8.  In a full tensor 64 -> 64 at
+    // 50 000 rows 45.1 (46.2 with a step for every block).
+    const bool beside = PAD && max_voxels - n >= n && PadRows<TO, COUT>::reach(n, max_voxels);
     for (int tile = first_tile; tile < tile_count; tile += walkers) {
     int run_begin, run_end;
     if (cut_count > 0) {
@@ -622,6 +624,7 @@ conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles
         const_cast<T*>(in), 0, (int)((size_t)max_voxels * S::kRowBytes), kRawBuffer);
     const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<void*>(Wp), 0, (int)((size_t)volume * S::kWeightBytes), kRawBuffer);
+    const bool first = idle;
     idle = false;
     if (tid < 16) s_pair[kMaxK * kTileRows + tid] = kNoPair;
     // zero this wave's partial tile (while the lists are on their way)
@@ -666,11 +669,21 @@ conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles
         s_epi[2 * COUT + tid] = epi_col;
     }
     __syncthreads();
-    pads.layer(s_epi, scale != nullptr, shift != nullptr, relu);
-    if constexpr (kMaxSplit)
-        if (split) multiply<S, COUT, kWgCols / 32>(rs_in, rs_w, s_pair, s_blk, volume, wave, waves, lane, col_first / 16, (rows + 15) >> 4, part, s_part + S::kPartRows * kWgCols, pads);
-    if (!kMaxSplit || !split) multiply<S, COUT, kWgCols / 16>(rs_in, rs_w, s_pair, s_blk, volume, wave, waves, lane, col_first / 16, (rows + 15) >> 4, part, s_part + S::kPartRows * kWgCols, pads);
-    pads.rest();
+    auto products = [&](auto& p) {
+        if constexpr (kMaxSplit)
+            if (split) multiply<S, COUT, kWgCols / 32>(rs_in, rs_w, s_pair, s_blk, volume, wave, waves, lane, col_first / 16, (rows + 15) >> 4, part, s_part + S::kPartRows * kWgCols, p);
+        if (!kMaxSplit || !split) multiply<S, COUT, kWgCols / 16>(rs_in, rs_w, s_pair, s_blk, volume, wave, waves, lane, col_first / 16, (rows + 15) >> 4, part, s_part + S::kPartRows * kWgCols, p);
+    };
+    if (PAD && beside && first) {
+        PadRows<TO, COUT> pads;
+        pads.begin(out, n, max_voxels, blockIdx.x * kWaves + wave, (unsigned)(units * S::kColGroups) * kWaves);
+        pads.layer(s_epi, scale != nullptr, shift != nullptr, relu);
+        products(pads);
+        pads.rest();
+    } else {
+        NoPadRows none;
+        products(none);
+    }
     __syncthreads();
 
     // fixed-order sum of the waves' partial tiles, epilogue, coalesced stores; the sums of kAtOnce vectors are read together
@@ -764,14 +777,16 @@ conv_wide(const int32_t* __restrict__ num_out, const int32_t* __restrict__ tiles
     __syncthreads();  // the next piece reuses the lists and partial tiles
     }
     }
-    if (PAD && idle) {  // (no tile has staged scale and shift)
-        if (thread < COUT) {
-            s_epi[thread] = scale ? scale[thread] : 1.f;
-            s_epi[COUT + thread] = shift ? shift[thread] : 0.f;
+    if (PAD && n < max_voxels && (idle || !beside)) {
+        if (idle) {  // (no tile has staged scale and shift)
+            if (thread < COUT) {
+                s_epi[thread] = scale ? scale[thread] : 1.f;
+                s_epi[COUT + thread] = shift ? shift[thread] : 0.f;
+            }
+            __syncthreads();
         }
-        __syncthreads();
-        pads.layer(s_epi, scale != nullptr, shift != nullptr, relu);
-        pads.rest();
+        write_pad_rows<TO, COUT>(out, n, max_voxels, blockIdx.x * kThreads + thread, (unsigned)(units * S::kColGroups) * kThreads, s_epi, scale != nullptr,
+                                 shift != nullptr, relu);
     }
 }
 
