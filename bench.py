@@ -315,7 +315,7 @@ def measure(config, args, torch, frames=None, points_override=None, deep=True, w
         ach = dom_bytes / (dom_ms * 1e-3) / 1e9
         roof = {"bound": "hbm", "achieved": round(ach, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                 "frac": round(ach / PEAK_HBM_GBS, 4), "traffic": None}
-    # (FP16 3x3x3 layers run on the LDS-ring kernel from 64 channels up, with 32 on the tall-tile one, FP32 on conv_wide)
+    # (FP16 3x3x3 layers run on the LDS-ring kernel from 64 channels up, with 32 on the one that holds all weights in LDS, FP32 on conv_wide)
     kname = (("conv_tile<%d, %d," if dom_c >= 64 else "conv_tall<%d, %d,") if half else "conv_wide<%d, %d,") % (dom_c, dom_c)
     traffic, fresh = profiled_traffic(kname, config, dtype)
     roof["traffic"] = traffic

@@ -197,7 +197,10 @@ int sessd_submconv3d_enqueue(sessd_submconv3d* h, const sessd_tensor_desc* inDes
 /* No counterpart in the reference (it rebuilds the rulebook in every layer although consecutive
  * SubM layers share one coors tensor, se-ssd-ai-trt.cpp:1147-1239): run the layer on the rulebook
  * a previous sessd_submconv3d_enqueue left in `rulebook_workspace` (same coors, same max_voxels,
- * same out_shape).  Only the gather-GEMM kernel is launched. */
+ * same out_shape).  Only the gather-GEMM kernel is launched.  The order in which an element's products are
+ * added may differ from that of sessd_submconv3d_enqueue on the layer's own rulebook: FP32 layers 4->16, 4->32
+ * and 16->16 of at most 8192 rows are multiplied there by the launch that builds the rulebook, and their last
+ * bits can differ.  One entry point with the same tensors gives the same bits each time. */
 int sessd_submconv3d_enqueue_shared(sessd_submconv3d* h, const sessd_tensor_desc* inDesc,
                                     const sessd_tensor_desc* outDesc, const void* const* inputs,
                                     void* const* outputs, const void* rulebook_workspace,

@@ -10,8 +10,10 @@
 //   * A step is four offsets.  Lane (i, q) of a wave requests all 32 or 64 bytes of the neighbour of row i at offset 4 step + q, and the inner
 //     dimension of an MFMA is eight channels of each of the four offsets: the lane's own list entries are all that it needs, no other
 //     lane's, and W is in LDS as the host has packed it (lane (i, q) reads the operand that holds these channels of W[4 step + q]).
-//     Rows are requested two steps (eight offsets) ahead, all of them by straight-line code: the compiler's waits are exact.
-//   * With few rows two or four waves share a block and take every second or fourth step; their sums are added in LDS.
+//     Rows are requested two steps (eight offsets) ahead, with 16 channels three, all of them by straight-line code: the compiler's waits
+//     are exact.
+//   * With few rows (up to four blocks a workgroup, 16 384 rows on 256 units; up to two, 8 192) two or four waves share a block and take
+//     every second or fourth step; their sums are added in LDS.
 //   * W, the row count and, behind that, the lists are on their way together; the first rows are requested in front of the barrier.
 //   * The rows beyond the active ones are written by four waves of their own.
 // What bounds it from some 40 000 rows up are the requests for rows in four cache lookups a row (coalesced ones, with a 4 x 4
@@ -23,7 +25,9 @@
 // 16 -> 16 and 16 -> 32 against conv_wide.hip's pair lists (a quarter of the neighbours is there): 1 947 rows 5.0 -> 2.9 us and 5.2 -> 3.2,
 // 16 198 rows 7.2 -> 3.3 and 8.1 -> 3.7, 60 000 rows 10.4 -> 4.9 and 11.9 -> 5.8; frames of 60 000 points 225.9 -> 215.7.
 // The waves are eight because the coordinate passes beside them need registers (12: the same times, and 504 of 512 taken).
-// Summation order per output element: steps ascending, in a step the channels eight at a time: fixed, run-to-run identical.
+// Summation order per output element: a wave's steps ascending, in a step the channels eight at a time; where waves share a block, to the
+// first one's sum those of the others, the last one's first.  Fixed for a row count and a grid, run-to-run identical; in a launch with more or
+// fewer rows, or on another number of compute units, the same row may be summed in another of the three orders.
 // (The ring of conv_tile.hip, faster from 64 channels up, has too little work per row here.)
 #include <type_traits>
 

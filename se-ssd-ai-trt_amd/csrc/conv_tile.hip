@@ -25,7 +25,7 @@
 // All vector-memory requests of a loading wave are of this one kind and are counted by hand (s_waitcnt vmcnt in issue
 // order).  Summation order per output element: offsets ascending, channels inside the MFMA: fixed, run-to-run identical.
 //
-// Measured against the register-operand kernel of conv_tall.hip, launches back to back: 128 -> 128 at 40 422 rows 47.0
+// Measured against a kernel with its operands in registers (64 or 128 rows, W read once for them), launches back to back: 128 -> 128 at 40 422 rows 47.0
 // -> 34.2 us (1.05 PFLOP/s with the padding pairs; a large FP16 matrix product of the library reaches 1.13: under this
 // load the clock falls to 1.4 .. 1.8 GHz), at 19 825 rows 37.9 -> 21.5, at 2 833 rows 21.5 -> 12.3; 64 -> 64 at 72 854 rows
 // 29.9 -> 24.4, at 26 247 rows 14.9 -> 11.7, at 3 060 rows 9.0 -> 8.5.  Beyond 40 960 rows (Cout 128) the loads bound it.

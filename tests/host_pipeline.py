@@ -399,7 +399,7 @@ def check_first_configure():
                              D.TensorDesc.make((1,), D.SESSD_INT32))
     outs = (D.TensorDesc * 1)(D.TensorDesc.make((1, rows, cout), D.SESSD_HALF))
     packing, configuring = [], []
-    for _ in range(25):
+    for attempt in range(100):
         h = C.c_void_p()
         assert L.sessd_submconv3d_create(C.byref(d), w.ctypes.data, C.byref(h)) == 0, L.sessd_last_error()
         t0 = time.perf_counter()
@@ -409,6 +409,8 @@ def check_first_configure():
         configuring.append(time.perf_counter() - t1)
         packing.append(t1 - t0)
         L.sessd_submconv3d_destroy(h)
+        if attempt >= 24 and min(configuring) < 1.4 * min(packing):  # (more of them where the machine has other work)
+            break
     # (with a second pass over the weights 1.6 to 2 times as long, without 1.1 to 1.2)
     assert min(configuring) < 1.4 * min(packing), (min(configuring), min(packing))
 

@@ -532,9 +532,9 @@ def test_subm_shared_rulebook_skip_pad_and_empty():
 @pytest.mark.parametrize("owner_cout,sharer_cout", [(64, 32), (32, 64)])
 def test_shared_rulebook_between_layers_of_different_tile_capacity(owner_cout, sharer_cout):
     """Two FP16 3x3x3 layers of different widths on one rulebook.  Both run on the kernel of conv_tall.hip, which cuts
-    its own tiles (a rulebook built by such a layer carries no equal-work cuts) and sums a row's offsets in
-    ascending order whatever tile the row falls in: the sharer's output on the owner's rulebook must equal its
-    output on its own bit for bit."""
+    its own tiles (a rulebook built by such a layer carries no equal-work cuts) and whose order of sums follows from the
+    row count alone, the same in both calls: the sharer's output on the owner's rulebook must equal its output on its
+    own bit for bit."""
     grid = (21, 400, 352)
     n, mv, cin = 15000, 16384, 32
     rng = np.random.default_rng(41)
@@ -1018,13 +1018,13 @@ def _fp16_subm_against_oracle(cin, cout, n, mv, grid, seed, clustered=True, epil
     if epilogue:
         o_out = O.scale_shift_relu(o_out, mv, sc, sh, True)
     # every row of the tensor: rows >= n are the epilogue of zero (the reference zero-fills, then BN + ReLU)
-    assert_features_close(to_np(out.float()), O.round_to_half(o_out), RTOL_FP16, "tall fp16 %d->%d, %d rows" % (cin, cout, n))
+    assert_features_close(to_np(out.float()), O.round_to_half(o_out), RTOL_FP16, "fp16 %d->%d, %d rows" % (cin, cout, n))
     conv.close()
 
 
 @pytest.mark.parametrize("cin,cout", [(32, 32), (64, 64), (128, 128)])
 @pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 300])
-def test_tall_fp16_kernel_row_counts_around_its_tiles(cin, cout, n):
+def test_fp16_kernels_row_counts_around_their_tiles(cin, cout, n):
     """A wave of the kernel with all weights in LDS has 16 rows (32 -> 32), a tile of the ring kernel 64 or 32 at these row counts:
     row counts on either side of a block and a tile, down to a single row, against the oracle (pad rows
     included)."""
@@ -1032,7 +1032,7 @@ def test_tall_fp16_kernel_row_counts_around_its_tiles(cin, cout, n):
 
 
 @pytest.mark.parametrize("cin,cout,n", [(32, 32, 66000), (64, 64, 40000), (64, 128, 66000), (128, 128, 40000), (128, 128, 66000)])
-def test_tall_fp16_kernel_with_two_row_blocks_per_wave(cin, cout, n):
+def test_fp16_kernels_with_many_rows(cin, cout, n):
     """Launches of many rows, the last tile partly filled, against the oracle on 16 threads: two or three blocks for a wave, one
     after the other with 32 channels, in one tile on the ring kernel."""
     O.set_threads(16)
@@ -1043,8 +1043,8 @@ def test_tall_fp16_kernel_with_two_row_blocks_per_wave(cin, cout, n):
 
 
 @pytest.mark.parametrize("cout,n", [(32, 81920), (32, 81921), (32, 120000), (32, 163841), (64, 65536), (64, 65537), (64, 100000), (64, 131073)])
-def test_tall_fp16_kernel_with_tall_tiles(cout, n):
-    """Launches of so many rows that every wave walks two to five blocks of 16, some a block more than others."""
+def test_fp16_kernel_with_all_weights_in_lds_whose_waves_walk_many_blocks(cout, n):
+    """Launches of so many rows that every wave walks two to six blocks of 16, some a block more than others."""
     O.set_threads(16)
     try:
         _fp16_subm_against_oracle(32, cout, n, n + 70, (41, 400, 352), 8000 + cout)

@@ -384,8 +384,8 @@ def test_frames_in_flight_give_the_bits_of_one_frame_at_a_time():
     stream.synchronize()
 
 
-def test_fp16_stack_ending_in_a_3x3x3_layer_scatters_from_the_tall_tile_kernel():
-    """A stack whose LAST layer is a 3x3x3 FP16 layer of 32 channels: that layer's kernel (the tall-tile one) also writes
+def test_fp16_stack_ending_in_a_3x3x3_layer_scatters_from_its_own_kernel():
+    """A stack whose LAST layer is a 3x3x3 FP16 layer of 32 channels: that layer's kernel (conv_tall.hip) also writes
     the dense tensor, in both schedules.  Dense tensor, sites and status against the oracle, and each schedule's tensor
     equal to a scatter of its last layer's rows and to the plugin's cell-major pass over them bit for bit."""
     S, P = D.SESSD_LAYER_SUBM, D.SESSD_LAYER_SPARSE
@@ -406,7 +406,7 @@ def test_fp16_stack_ending_in_a_3x3x3_layer_scatters_from_the_tall_tile_kernel()
     assert fused.status() == plain.status() == ref["status"] == 0
     assert [fused.layer_count(l) for l in range(-1, len(layers))] == list(ref["counts"])
     assert np.array_equal(fused.read_layer(len(layers) - 1)[1], ref["coors"])
-    assert_end_to_end_close(to_np(d_fused).astype(np.float32), want, True, "dense from the tall-tile kernel")
+    assert_end_to_end_close(to_np(d_fused).astype(np.float32), want, True, "dense from conv_tall")
     assert torch.equal(d_fused, d_plain)
     for pipe, d in ((fused, d_fused), (plain, d_plain)):
         feat, coors, m = pipe.read_layer(len(layers) - 1)
