@@ -47,7 +47,7 @@
 // they are fewer).  What LDS and registers they leave is what the coordinate passes of a frame's other branch run in: 32 -> 32 with eight waves is the faster launch (15.9 us against 17.1 at
 // 28 043 rows) and makes the slower frame (20 000 points: 283 us against 274); 4 -> 32 likewise (487 against 475).  16 -> 32 with four waves and
 // 3 x 80 rows: 54 613 rows 18.4 -> 17.4 us, but 17 132 rows 9.0 -> 11.4.
-// FP16 features have so little in each block that with up to 32 columns four waves and 64 rows do: four workgroups share a unit, with 40 KB of
+// FP16 features have so little in each block that with up to 32 columns four waves and 64 rows do: four workgroups share a unit, with up to 40 KB of
 // LDS each.  3x3x3 layers are faster without pair lists (16 -> 16 at 60 000 rows 4.9 us on conv_tall.hip, 10.4 here; 32 -> 32 at 49 874 8.4 there,
 // at 45 874 18 here) and come here where a weight is infinite or NaN as a half, and an absent neighbour must not be a row of zeros.
 #include <algorithm>
