@@ -113,10 +113,8 @@ int ConvPluginBase::tilesWide() const {
 }
 int ConvPluginBase::tileRowWeight() const { return 4; }  // (only conv_wide.hip takes cuts)
 
-int ConvPluginBase::runGemm(const void* in_feat, void* out_feat, const int32_t* nbr, const int32_t* tiles,
-                            const int32_t* num_out, hipStream_t stream, const DenseTarget* dense) {
+GemmArgs ConvPluginBase::gemmArgs(const void* in_feat, void* out_feat, const int32_t* nbr, const int32_t* tiles, const int32_t* num_out) const {
     GemmArgs a;
-    if (dense) a.dense = *dense;
     a.in_feat = in_feat;
     a.out_feat = out_feat;
     a.nbr = nbr;
@@ -137,6 +135,13 @@ int ConvPluginBase::runGemm(const void* in_feat, void* out_feat, const int32_t* 
     a.write_pad_rows = (flags_ & SESSD_FLAG_SKIP_PAD_ROWS) ? 0 : 1;
     a.force_valu = (flags_ & SESSD_FLAG_FORCE_VALU) ? 1 : 0;
     a.tiles = tiles;
+    return a;
+}
+
+int ConvPluginBase::runGemm(const void* in_feat, void* out_feat, const int32_t* nbr, const int32_t* tiles,
+                            const int32_t* num_out, hipStream_t stream, const DenseTarget* dense) {
+    GemmArgs a = gemmArgs(in_feat, out_feat, nbr, tiles, num_out);
+    if (dense) a.dense = *dense;
     if (ev_gemm_begin_) SESSD_HIP_TRY(hipEventRecord(ev_gemm_begin_, stream));
     SESSD_TRY(launch_gather_gemm(a, stream));
     if (ev_gemm_end_) SESSD_HIP_TRY(hipEventRecord(ev_gemm_end_, stream));

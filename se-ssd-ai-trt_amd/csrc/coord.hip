@@ -16,6 +16,7 @@
 // Measured (frames without their GEMMs, us; 35 launches, 13, 13 as they are now): 2 000 points 141, 79, 62, 20 000 164, 97, 72, 80 000
 // 231, 127, 95, 60 000 (FP16 configuration) 162, 111, 84, 150 000 221, 147, 111.  A pass is bound by its chain of dependent trips to
 // memory (four to six of 0.7-1 us each) until some 40 000 rows, and by random accesses beyond.
+#include "conv_tall.h"
 #include "coord.h"
 #include "fill.h"
 
@@ -663,16 +664,65 @@ struct FlagsLookups {
     LookupPart look[kMaxLookups];
 };
 
+// Products of a layer that does not need what a pass makes, in the pass's launch (conv_tall.h, a workgroup of four waves for each compute
+// unit): layer 0 beside the numbering of the first strided layer's rows, layer 1 beside the lookups on them.  On a branch of its own either
+// side began 7 us after the other, and the first strided layer 8 to 10 us after the later one.  That layer's products begin, us after the
+// frame: FP32 2 000 points 47.7 -> 41.1, 20 000 55.9 -> 49.9, FP16 60 000 61.8 -> 53.2.  Frames FP32 2 000 points 174.0 -> 167.1, 8 000 210.2 -> 202.8,
+// 20 000 257.6 -> 254.9, 80 000 386 -> 378, FP16 8 000 161.9 -> 151.5, 60 000 196.1 -> 189.6, launched directly 20 000 286.7 -> 276.9.  Two
+// workgroups a unit: the same times but 80 000 points, 1.008x.  The registers are held to what lets five blocks (FP16 lookups: seven) share a unit, so that
+// a pass finds room for its blocks beside the products (with 106 instead of 95 the FP32 lookups had four).  Layers with more weights leave
+// the lookups too little LDS.
+constexpr int kProductWaves = kCoordBlock / 64, kPadBlocks = 256;  // (those write the rows beyond the active ones, behind all others)
+template <int CIN, int COUT, typename T>
+using ProductLds = tall::Lds<CIN, COUT, T, kProductWaves>;
+
+template <int CIN, int COUT, typename T, typename TO>
+__device__ __forceinline__ void products_pass(const TallArgs& g, int block, int blocks, ProductLds<CIN, COUT, T>& lds) {
+    tall::workgroup<CIN, COUT, T, TO, kProductWaves, 0>(g, DenseTarget(), block, blocks, lds);
+}
+template <int CIN, int COUT, typename T, typename TO>
+__device__ __forceinline__ void products_pad_pass(const TallArgs& g, int block, ProductLds<CIN, COUT, T>& lds) {
+    const int n = clamp_rows(g.num_out, g.max_voxels);
+    if (threadIdx.x < COUT) {
+        lds.epi[threadIdx.x] = g.scale ? g.scale[threadIdx.x] : 1.f;
+        lds.epi[COUT + threadIdx.x] = g.shift ? g.shift[threadIdx.x] : 0.f;
+    }
+    __syncthreads();
+    write_pad_rows<TO, COUT>(static_cast<TO*>(g.out), n, g.max_voxels, block * kCoordBlock + threadIdx.x, kPadBlocks * kCoordBlock, lds.epi, g.scale != nullptr,
+                             g.shift != nullptr, g.relu);
+}
+
 // end1 .. end3: where the blocks of the lookups behind the first begin.  (Arguments of their own: those are in registers when the
 // kernel starts.)
 template <bool HASH>
-__global__ void __launch_bounds__(kCoordBlock) flags_lookups(int flag_blocks, int end1, int end2, int end3, FlagsLookups a) {
-    __shared__ LookupLds L;
-    const int b = blockIdx.x;
+__device__ __forceinline__ void flags_lookups_block(int b, int flag_blocks, int end1, int end2, int end3, const FlagsLookups& a, LookupLds& L) {
     if (b < flag_blocks) return sp_flags_pass(a.flags, b, flag_blocks, reinterpret_cast<uint32_t*>(L.sum));
     const int l = __builtin_amdgcn_readfirstlane((b >= end1 ? 1 : 0) + (b >= end2 ? 1 : 0) + (b >= end3 ? 1 : 0));
     static_assert(kMaxLookups == 4, "one argument for each lookup but the first");
     lookup_pass<HASH>(a.look[l], b - (l == 0 ? flag_blocks : (l == 1 ? end1 : (l == 2 ? end2 : end3))), L);
+}
+template <bool HASH>
+__global__ void __launch_bounds__(kCoordBlock) flags_lookups(int flag_blocks, int end1, int end2, int end3, FlagsLookups a) {
+    __shared__ LookupLds L;
+    flags_lookups_block<HASH>(blockIdx.x, flag_blocks, end1, end2, end3, a, L);
+}
+template <int CIN, int COUT, typename T, typename TO>
+__global__ void __launch_bounds__(kCoordBlock, (sizeof(T) == 2 ? 7 : 5)) conv_tall_beside_flags_lookups(int gemm_blocks, int pads_at, int flag_blocks, int end1, int end2,
+                                                                                              int end3, TallArgs g, FlagsLookups a) {
+    __shared__ union {
+        ProductLds<CIN, COUT, T> products;
+        LookupLds lookups;
+    } lds;
+    const int b = blockIdx.x;
+    if (b < gemm_blocks) return products_pass<CIN, COUT, T, TO>(g, b, gemm_blocks, lds.products);
+    if (b >= pads_at) return products_pad_pass<CIN, COUT, T, TO>(g, b - pads_at, lds.products);
+    flags_lookups_block<false>(b - gemm_blocks, flag_blocks, end1, end2, end3, a, lds.lookups);
+}
+
+// the flags alone (where the lookups on the rows behind them run on the other stream)
+__global__ void __launch_bounds__(kCoordBlock) sp_flags(SpPart P) {
+    __shared__ uint32_t lds4[4];
+    sp_flags_pass(P, blockIdx.x, gridDim.x, lds4);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -845,15 +895,18 @@ struct NumberCuts {
     FillPlan<N> also;
 };
 
+struct NumberLds {
+    uint32_t sums[12];
+    int4 rows[kCoordBlock];
+    InsertLds insert;
+};
+
 // end0 .. end3: where the blocks of the cuts end, clean_end: those of the cleaning.
 template <int N>
-__global__ void __launch_bounds__(kCoordBlock) number_cuts(int number_blocks, int has_next, int end0, int end1, int end2, int end3, int clean_end,
-                                                           NumberCuts<N> a) {
-    __shared__ uint32_t lds[12];
-    __shared__ int4 s_rows[kCoordBlock];
-    __shared__ InsertLds L;
-    const int b = blockIdx.x;
-    if (b < number_blocks) return sp_number_pass(a.number, a.next, has_next != 0, b, number_blocks, lds, s_rows, L);
+__device__ __forceinline__ void number_cuts_block(int b, int number_blocks, int has_next, int end0, int end1, int end2, int end3, int clean_end,
+                                                  const NumberCuts<N>& a, NumberLds& L) {
+    uint32_t* const lds = L.sums;
+    if (b < number_blocks) return sp_number_pass(a.number, a.next, has_next != 0, b, number_blocks, lds, L.rows, L.insert);
     static_assert(kMaxCuts == 4, "an argument for each");
     if (b < end3) {
         const int l = __builtin_amdgcn_readfirstlane((b >= end0 ? 1 : 0) + (b >= end1 ? 1 : 0) + (b >= end2 ? 1 : 0));
@@ -861,6 +914,34 @@ __global__ void __launch_bounds__(kCoordBlock) number_cuts(int number_blocks, in
     }
     if (b < clean_end) return clean_pass(a.clean, b - end3);
     fill_pass(a.also, b - clean_end);
+}
+template <int N>
+__global__ void __launch_bounds__(kCoordBlock) number_cuts(int number_blocks, int has_next, int end0, int end1, int end2, int end3, int clean_end,
+                                                           NumberCuts<N> a) {
+    __shared__ NumberLds L;
+    number_cuts_block(blockIdx.x, number_blocks, has_next, end0, end1, end2, end3, clean_end, a, L);
+}
+// ... with a layer's products, whose blocks are the first of the grid or the last: in front is what takes longer (pipeline.hip)
+template <int CIN, int COUT, typename T, typename TO>
+__device__ __forceinline__ void number_and_products(int b, int gemm_at, int gemm_blocks, int pads_at, int number_blocks, int has_next, int end0, int end1, int end2,
+                                                    int end3, int clean_end, const TallArgs& g, const NumberCuts<1>& a) {
+    __shared__ union {
+        ProductLds<CIN, COUT, T> products;
+        NumberLds number;
+    } lds;
+    if (b >= pads_at) return products_pad_pass<CIN, COUT, T, TO>(g, b - pads_at, lds.products);
+    if (b >= gemm_at && b < gemm_at + gemm_blocks) return products_pass<CIN, COUT, T, TO>(g, b - gemm_at, gemm_blocks, lds.products);
+    number_cuts_block(b - (gemm_at ? 0 : gemm_blocks), number_blocks, has_next, end0, end1, end2, end3, clean_end, a, lds.number);
+}
+template <int CIN, int COUT, typename T, typename TO>
+__global__ void __launch_bounds__(kCoordBlock, 5) conv_tall_then_numbering(int gemm_blocks, int pads_at, int number_blocks, int has_next, int end0, int end1, int end2,
+                                                                     int end3, int clean_end, TallArgs g, NumberCuts<1> a) {
+    number_and_products<CIN, COUT, T, TO>(blockIdx.x, 0, gemm_blocks, pads_at, number_blocks, has_next, end0, end1, end2, end3, clean_end, g, a);
+}
+template <int CIN, int COUT, typename T, typename TO>
+__global__ void __launch_bounds__(kCoordBlock, 5) number_cuts_then_conv_tall(int gemm_blocks, int pads_at, int number_blocks, int has_next, int end0, int end1, int end2,
+                                                                        int end3, int clean_end, TallArgs g, NumberCuts<1> a) {
+    number_and_products<CIN, COUT, T, TO>(blockIdx.x, pads_at - gemm_blocks, gemm_blocks, pads_at, number_blocks, has_next, end0, end1, end2, end3, clean_end, g, a);
 }
 
 // rulebook of a strided layer on its own: one store per ticket into the rows sp_number has initialised
@@ -979,7 +1060,15 @@ int launch_sp_insert(const SpPart& s, hipStream_t stream) {
     return SESSD_OK;
 }
 
-int launch_flags_lookups(const SpPart* flags, const LookupPart* lookups, int n, hipStream_t stream) {
+// (finite weights, 32-bit offsets, ... : tall_takes())
+bool number_takes_products(const GemmArgs& a) { return a.cin == 4 && !a.dense.dense && tall_takes(a); }
+bool lookups_take_products(const GemmArgs& a, const LookupPart* lookups, int n) {
+    for (int l = 0; l < n; ++l)
+        if (!lookups[l].t.dense) return false;
+    return n <= kMaxLookups && a.cin == 16 && a.cout == 16 && !a.dense.dense && tall_takes(a);
+}
+
+static int flags_lookups_launch(const SpPart* flags, const LookupPart* lookups, int n, const GemmArgs* products, hipStream_t stream) {
     if (n < 0 || n > kMaxLookups) return fail(SESSD_E_INVALID, "lookups: at most %d in one launch", kMaxLookups);
     FlagsLookups a;
     int flag_blocks = 0;
@@ -1002,7 +1091,19 @@ int launch_flags_lookups(const SpPart* flags, const LookupPart* lookups, int n, 
         }
         end[l] = blocks;
     }
-    if (!blocks) return SESSD_OK;
+    if (!blocks && !products) return SESSD_OK;
+    if (products) {
+        if (!lookups_take_products(*products, lookups, n)) return fail(SESSD_E_UNSUPPORTED, "lookups: a layer's products cannot share this launch");
+        const TallArgs g = tall_args(*products);
+        const int gemm_blocks = gemm_compute_units(), pads_at = gemm_blocks + blocks;
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(pads_at + (products->write_pad_rows ? kPadBlocks : 0)), dim3(kCoordBlock), 0, stream, gemm_blocks, pads_at, flag_blocks, end[0],
+                               end[1], end[2], g, a);
+        };
+        products->in_type == SESSD_HALF ? go(conv_tall_beside_flags_lookups<16, 16, __half, __half>) : go(conv_tall_beside_flags_lookups<16, 16, float, float>);
+        SESSD_HIP_TRY(hipGetLastError());
+        return SESSD_OK;
+    }
     bool hash = false;  // (the flags read either kind of table)
     for (int l = 0; l < n; ++l) hash = hash || !lookups[l].t.dense;
     if (hash) hipLaunchKernelGGL(flags_lookups<true>, dim3(blocks), dim3(kCoordBlock), 0, stream, flag_blocks, end[0], end[1], end[2], a);
@@ -1011,8 +1112,21 @@ int launch_flags_lookups(const SpPart* flags, const LookupPart* lookups, int n, 
     return SESSD_OK;
 }
 
-int launch_number(const SpPart* number, const SpPart* next, const CutPart* cuts, int n_cuts, const CleanPart* clean, const FillArgs* also,
-                  hipStream_t stream) {
+int launch_flags_lookups(const SpPart* flags, const LookupPart* lookups, int n, hipStream_t stream) {
+    return flags_lookups_launch(flags, lookups, n, nullptr, stream);
+}
+int launch_flags_lookups_products(const SpPart* flags, const LookupPart* lookups, int n, const GemmArgs& products, hipStream_t stream) {
+    return flags_lookups_launch(flags, lookups, n, &products, stream);
+}
+
+int launch_sp_flags(const SpPart& s, hipStream_t stream) {
+    hipLaunchKernelGGL(sp_flags, dim3(sp_pass_blocks(s)), dim3(kCoordBlock), 0, stream, s);
+    SESSD_HIP_TRY(hipGetLastError());
+    return SESSD_OK;
+}
+
+static int number_launch(const SpPart* number, const SpPart* next, const CutPart* cuts, int n_cuts, const CleanPart* clean, const FillArgs* also,
+                         const GemmArgs* products, bool products_first, hipStream_t stream) {
     if (n_cuts < 0 || n_cuts > kMaxCuts) return fail(SESSD_E_INVALID, "tile cuts: at most %d in one launch", kMaxCuts);
     NumberCuts<1> a;
     int number_blocks = 0, has_next = 0;
@@ -1045,10 +1159,36 @@ int launch_number(const SpPart* number, const SpPart* next, const CutPart* cuts,
     const int fill_blocks = make_fill_plan(also ? *also : none, a.also);
     if (fill_blocks < 0) return fail(SESSD_E_INVALID, "fill: a region is not 16-byte aligned");
     blocks += fill_blocks;
-    if (!blocks) return SESSD_OK;
-    hipLaunchKernelGGL(number_cuts<1>, dim3(blocks), dim3(kCoordBlock), 0, stream, number_blocks, has_next, end[0], end[1], end[2], end[3], clean_end, a);
+    if (!blocks && !products) return SESSD_OK;
+    if (products) {
+        if (!number_takes_products(*products)) return fail(SESSD_E_UNSUPPORTED, "numbering: a layer's products cannot share this launch");
+        const TallArgs g = tall_args(*products);
+        const int gemm_blocks = gemm_compute_units(), pads_at = gemm_blocks + blocks;
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(pads_at + (products->write_pad_rows ? kPadBlocks : 0)), dim3(kCoordBlock), 0, stream, gemm_blocks, pads_at, number_blocks,
+                               has_next, end[0], end[1], end[2], end[3], clean_end, g, a);
+        };
+        const bool half = products->out_type == SESSD_HALF, narrow = products->cout == 16;
+        if (products_first) {
+            if (half) narrow ? go(conv_tall_then_numbering<4, 16, float, __half>) : go(conv_tall_then_numbering<4, 32, float, __half>);
+            else narrow ? go(conv_tall_then_numbering<4, 16, float, float>) : go(conv_tall_then_numbering<4, 32, float, float>);
+        } else {
+            if (half) narrow ? go(number_cuts_then_conv_tall<4, 16, float, __half>) : go(number_cuts_then_conv_tall<4, 32, float, __half>);
+            else narrow ? go(number_cuts_then_conv_tall<4, 16, float, float>) : go(number_cuts_then_conv_tall<4, 32, float, float>);
+        }
+    } else {
+        hipLaunchKernelGGL(number_cuts<1>, dim3(blocks), dim3(kCoordBlock), 0, stream, number_blocks, has_next, end[0], end[1], end[2], end[3], clean_end, a);
+    }
     SESSD_HIP_TRY(hipGetLastError());
     return SESSD_OK;
+}
+int launch_number(const SpPart* number, const SpPart* next, const CutPart* cuts, int n_cuts, const CleanPart* clean, const FillArgs* also,
+                  hipStream_t stream) {
+    return number_launch(number, next, cuts, n_cuts, clean, also, nullptr, false, stream);
+}
+int launch_number_products(const SpPart* number, const SpPart* next, const CutPart* cuts, int n_cuts, const CleanPart* clean, const FillArgs* also,
+                           const GemmArgs& products, bool products_first, hipStream_t stream) {
+    return number_launch(number, next, cuts, n_cuts, clean, also, &products, products_first, stream);
 }
 
 int launch_sp_scatter(const SpPart& s, hipStream_t stream) {

@@ -18,7 +18,7 @@ struct GemmArgs {
     const float* w_f32;      // [K][cin][cout]
     const __half* w_f16;     // same layout, rounded to half (used when in_type is HALF)
     const void* w_packed;    // MFMA operand order, or null
-    bool halves_finite = false;  // all of w_f16: 0 x w is 0 (an FP16 kernel may multiply absent neighbours as rows of zeros)
+    bool halves_finite = false;  // all of w_f16, hence of w_f32: 0 x w is 0 (a kernel may multiply absent neighbours as rows of zeros)
     const float* scale;      // [cout] or null
     const float* shift;      // [cout] or null
     int relu;

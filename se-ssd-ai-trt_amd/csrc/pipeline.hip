@@ -329,13 +329,12 @@ struct Pipeline {
 
         // Coordinate passes are counted 2i (flags + lookups of stage i) and 2i + 1 (numbering, cuts, builds).  ready[l] = the
         // pass layer l's rulebook is complete after; pass 0 runs on the caller's stream.  works[p]: it does something on the other.
-        const int clean_at = m < 1 ? 0 : 1;  // stage 1's own rulebook is the last reader of the voxels' table
         std::vector<int> ready(stages.size(), 0);
         std::vector<char> works((size_t)(2 * m + 2), 0);
         for (int i = 0; i <= m; ++i) {
             const Stage& sg = cs[(size_t)i];
             works[(size_t)(2 * i)] = i > 0;
-            works[(size_t)(2 * i + 1)] = i < m || i == clean_at || !sg.builds.empty();
+            works[(size_t)(2 * i + 1)] = i < m || i == 1 || m == 0 || !sg.builds.empty();
             for (int l : sg.lookups) {
                 const ConvStage& st = *stages[(size_t)l];
                 const bool cuts = st.subm ? st.subm->wantTileCuts() : st.sparse->wantTileCuts();
@@ -343,6 +342,38 @@ struct Pipeline {
                 if (cuts) works[(size_t)(2 * i + 1)] = 1;
             }
             for (int l : sg.builds) ready[(size_t)l] = 2 * i + 1;
+        }
+        // The first layers and the passes up to the first strided layer's rulebook take about as long as each other, and between two
+        // branches a graph loses 7 us where the second begins and 8 to 10 where one waits for what the other has just done.  So
+        // they share launches on the caller's stream: pass 1 with layer 0's products, where its kernel leaves the pass room, pass 2 with layer 1's
+        // (or, where the first strided layer is next, alone).  The other branch begins behind pass 1, with the flags for pass 3.  The figures
+        // are at the kernels (coord.hip).  (Flags beside the lookups as well, the branch behind pass 2: 2 000 points 1.04x, the passes end too late.)
+        int last_main = 0, clean_at = m < 1 ? 0 : 1;  // (stage 1's own rulebook is the last reader of the voxels' table)
+        int beside[3] = {-1, -1, -1};
+        auto rulebookPass = [&](size_t l) { return ready[(size_t)(stages[l]->rulebook_from >= 0 ? stages[l]->rulebook_from : (int)l)]; };
+        auto productsOf = [&](size_t l) {
+            return stages[l]->subm->sharedGemmArgs(l ? stages[l - 1]->feat.p : vg_voxels.p, stages[l]->feat.p, static_cast<const int32_t*>(vg_num.p),
+                                                   stages[(size_t)(stages[l]->rulebook_from >= 0 ? stages[l]->rulebook_from : (int)l)]->ws.p);
+        };
+        if (m >= 1 && stages.size() > 2 && cs[0].builds.empty() && cs[0].lookups.size() <= (size_t)kMaxCuts && stages[0]->subm && rulebookPass(0) == 0 &&
+            number_takes_products(productsOf(0))) {
+            beside[1] = 0;
+            last_main = 1;
+            bool lookups_alone = cs[1].builds.empty() && cs[1].lookups.size() <= (size_t)kMaxLookups;  // (no cuts, no builds: nothing of pass 3 reads them)
+            for (int l : cs[1].lookups) lookups_alone = lookups_alone && ready[(size_t)l] == 2;
+            if (lookups_alone && rulebookPass(1) == 2) {
+                last_main = 2;
+            } else if (lookups_alone && stages[1]->subm && rulebookPass(1) == 0 && rows[0].table.dense && rows[1].table.dense &&
+                       lookups_take_products(productsOf(1), nullptr, 0)) {
+                beside[2] = 1;
+                last_main = 2;
+            }
+        }
+        const bool fork = aux != nullptr && stages.size() > 0;
+        const bool apart = fork && last_main == 2;  // pass 2 runs beside the passes behind it but for the one that empties the table
+        if (apart && m >= 2) {
+            clean_at = 2;
+            works[5] = 1;
         }
         int last_side = 2 * m + 1;
         while (last_side > 0 && !works[(size_t)last_side]) --last_side;
@@ -353,21 +384,28 @@ struct Pipeline {
         // Each pass by itself / for the branch's end / so, us: the reference's backbone, FP32 2 000 points 183, 178, 178, 20 000 252, 247, 247,
         // FP16 60 000 222, 219, 219 (so is its end); four strided layers more, each with two SubM layers, FP32 2 000 points 343, 371, 330,
         // 20 000 487, 517, 474, FP16 20 000 319, 328, 311; twelve more, FP32 2 000 675, 770, 645.
-        constexpr int kOwnWaits = 4;  // passes that are waited for one by one: to the lookups on the second strided layer's rows
+        // Passes that are waited for one by one: to the lookups on the second strided layer's rows, with few points to their tile cuts (2 000 points
+        // 182 -> 168 us, the branch's end is 15 us away then; 20 000 253.9 -> 258.5).
+        const int kOwnWaits = desc.max_points > 10000 ? 4 : 5;
         constexpr int kAhead = 2, kRest = 4;
-        const bool fork = aux != nullptr && stages.size() > 0;
         hipStream_t side = fork ? aux : stream;
         std::vector<int> wait_for(stages.size(), 0);
         std::vector<char> awaited((size_t)(2 * m + 2), 0);
         bool join = false;  // at the end, for what no layer has waited for
-        int longer = -1;    // passes less layers in front of the last layer that waits by itself for what it needs
+        int longer = -1;    // passes less layers in front of the last layer until the second strided layer's rulebook that needs a pass anew
         if (fork) {
-            int waited = 0;
+            int seen = 0;
             for (size_t l = 0; l < stages.size(); ++l) {
-                const int pass = ready[(size_t)(stages[l]->rulebook_from >= 0 ? stages[l]->rulebook_from : (int)l)];
+                const int pass = rulebookPass(l);
+                if (pass <= seen) continue;
+                seen = pass;
+                if (pass <= 5) longer = pass - (int)l;
+            }
+            int waited = last_main;
+            for (size_t l = 0; l < stages.size(); ++l) {
+                const int pass = rulebookPass(l);
                 if (pass <= waited) continue;
                 waited = pass;
-                if (pass <= kOwnWaits + 1) longer = pass - (int)l;
                 const int end = pass <= kOwnWaits ? pass : (last_side - pass <= kRest ? last_side : pass + kAhead);
                 for (int p = pass + 1; p <= end; ++p) {
                     if (p % 2 && !cs[(size_t)(p / 2)].builds.empty()) break;
@@ -418,11 +456,28 @@ struct Pipeline {
         // 172.8 / 171.0, 12 000 242.5 / 240.8, 177.8 / 174.4, 40 000 331.6 / 320.9, 206.5 / 205.3; one SubM layer in front 5 000 203.9 / 207.8,
         // 165.9 / 169.1, 20 000 244.0 / 245.6, 177.3 / 177.7; four 2 000 189.8 / 182.8, 176.6 / 167.3, 10 000 256.3 / 252.5, 194.3 / 185.8; doubled
         // widths, FP32 5 000 332.6 / 341.4, 20 000 478.4 / 476.3.  The points are those that the tensor holds, which is what the host
-        // knows: a frame of 2 000 points in a tensor for 20 000 takes 184.7, passes first it would be 177.7.
+        // knows: a frame of 2 000 points in a tensor for 20 000 takes 184.7, passes first it would be 177.7.  (Measured while the branches
+        // began behind pass 0.  Where the first layer shares the launch of pass 1 the rule says whose blocks are the first of its grid.)
         const bool chain_first = longer < 0 || desc.max_points > 10000;
+        auto behindPass = [&](int pass) -> int {
+            if (!fork) return SESSD_OK;
+            if (pass == (apart ? 1 : last_main)) {
+                SESSD_HIP_TRY(hipEventRecord(ev_head, stream));
+                SESSD_HIP_TRY(hipStreamWaitEvent(side, ev_head, 0));
+            }
+            if (apart && pass == 2) SESSD_HIP_TRY(hipEventRecord(ev_pass[2], stream));
+            if (pass == last_main && (chain_first || last_main == 2)) return layers(last_main);
+            if (awaited[(size_t)pass]) SESSD_HIP_TRY(hipEventRecord(ev_pass[(size_t)pass], side));
+            return SESSD_OK;
+        };
+        auto launched = [&](int l) {  // (beside a pass)
+            feat = stages[(size_t)l]->feat.p;
+            next_layer = (size_t)l + 1;
+        };
         for (int i = 0; i <= m; ++i) {
             const Stage& sg = cs[(size_t)i];
-            hipStream_t s = i == 0 ? stream : side;
+            hipStream_t s = 2 * i <= last_main ? stream : side, s_number = 2 * i + 1 <= last_main ? stream : side;
+            const int with_lookups = 2 * i <= last_main ? beside[(size_t)(2 * i)] : -1, with_number = 2 * i + 1 <= last_main ? beside[(size_t)(2 * i + 1)] : -1;
             // flags of the next strided layer and the lookups on this stage's rows
             std::vector<LookupPart> looks;
             std::vector<CutPart> cuts;
@@ -439,19 +494,20 @@ struct Pipeline {
                 }
             }
             const SpPart* next = i < m ? &part[(size_t)i + 1] : nullptr;
+            const SpPart* flags = apart && i == 1 ? nullptr : next;
             size_t at = 0;
-            do {
+            if (with_lookups >= 0) {
+                SESSD_TRY(launch_flags_lookups_products(flags, looks.data(), (int)looks.size(), productsOf((size_t)with_lookups), s));
+                launched(with_lookups);
+                at = looks.size();
+            } else do {
                 const size_t n = looks.size() - at < (size_t)kMaxLookups ? looks.size() - at : (size_t)kMaxLookups;
-                SESSD_TRY(launch_flags_lookups(at == 0 ? next : nullptr, looks.data() + at, (int)n, s));
+                SESSD_TRY(launch_flags_lookups(at == 0 ? flags : nullptr, looks.data() + at, (int)n, s));
                 at += n;
             } while (at < looks.size());
-            if (i == 0 && fork) {
-                SESSD_HIP_TRY(hipEventRecord(ev_head, stream));
-                SESSD_HIP_TRY(hipStreamWaitEvent(side, ev_head, 0));
-                if (chain_first) SESSD_TRY(layers(0));
-            } else if (awaited[(size_t)(2 * i)]) {
-                SESSD_HIP_TRY(hipEventRecord(ev_pass[(size_t)(2 * i)], side));
-            }
+            SESSD_TRY(behindPass(2 * i));
+            if (next && !flags) SESSD_TRY(launch_sp_flags(*next, side));
+            if (apart && i == clean_at) SESSD_HIP_TRY(hipStreamWaitEvent(side, ev_pass[2], 0));
             // numbering of the next strided layer's rows (their tickets for the layer behind it), tile cuts
             FillArgs clear;
             CleanPart clean;
@@ -463,10 +519,17 @@ struct Pipeline {
             const SpPart* after = i + 1 < m ? &part[(size_t)i + 2] : nullptr;
             at = 0;
             bool did = false;
+            if (with_number >= 0) {
+                SESSD_TRY(launch_number_products(next, after, cuts.data(), (int)cuts.size(), clean.taken ? &clean : nullptr, &clear, productsOf((size_t)with_number),
+                                                 chain_first, s_number));
+                launched(with_number);
+                at = cuts.size();
+                did = true;
+            }
             while (at < cuts.size() || (!did && (next || i == clean_at))) {
                 const size_t n = cuts.size() - at < (size_t)kMaxCuts ? cuts.size() - at : (size_t)kMaxCuts;
                 SESSD_TRY(launch_number(did ? nullptr : next, did ? nullptr : after, cuts.data() + at, (int)n, did || !clean.taken ? nullptr : &clean,
-                                        did ? nullptr : &clear, side));
+                                        did ? nullptr : &clear, s_number));
                 at += n;
                 did = true;
             }
@@ -474,7 +537,7 @@ struct Pipeline {
                 ConvStage& st = *stages[(size_t)l];
                 SESSD_TRY(st.subm->enqueueBuild(rows[(size_t)i].coors, rows[(size_t)i].num, st.ws.p, side));
             }
-            if (awaited[(size_t)(2 * i + 1)]) SESSD_HIP_TRY(hipEventRecord(ev_pass[(size_t)(2 * i + 1)], side));
+            SESSD_TRY(behindPass(2 * i + 1));
         }
 
         SESSD_TRY(layers(2 * m + 1));

@@ -114,6 +114,7 @@ class ConvPluginBase {
     // `dense`: also scatter the output rows into the dense tensor of a sparse2Dense step (MFMA kernel only)
     int runGemm(const void* in_feat, void* out_feat, const int32_t* nbr, const int32_t* tiles,
                 const int32_t* num_out, hipStream_t stream, const DenseTarget* dense = nullptr);
+    GemmArgs gemmArgs(const void* in_feat, void* out_feat, const int32_t* nbr, const int32_t* tiles, const int32_t* num_out) const;
     // whether a rulebook built by this layer gets equal-work tile cuts: worth two small launches when the
     // GEMM runs on the matrix cores and is not tiny
   public:
@@ -168,6 +169,7 @@ class SubmConv3dLayerPlugin : public ConvPluginBase {
     void collectHeaderFill(void* workspace, FillArgs& f) const;
     int enqueueGemm(const void* in_feat, void* out_feat, const int32_t* voxel_num,
                     const void* rulebook_workspace, hipStream_t stream, const DenseTarget* dense = nullptr);
+    GemmArgs sharedGemmArgs(const void* in_feat, void* out_feat, const int32_t* voxel_num, void* rulebook_workspace) const;
     int exportRulebook(const void* workspace, int32_t* indice_pairs, uint32_t* indice_num,
                        hipStream_t stream) const;
     int countPairs(const void* workspace, uint32_t* indice_num, hipStream_t stream) const;

@@ -540,6 +540,11 @@ int SubmConv3dLayerPlugin::enqueueGemm(const void* in_feat, void* out_feat, cons
     return runGemm(in_feat, out_feat, L.nbr, L.tiles, voxel_num, stream, dense);
 }
 
+GemmArgs SubmConv3dLayerPlugin::sharedGemmArgs(const void* in_feat, void* out_feat, const int32_t* voxel_num, void* rulebook_workspace) const {
+    const Layout L = carve(rulebook_workspace);
+    return gemmArgs(in_feat, out_feat, L.nbr, L.tiles, voxel_num);
+}
+
 int SubmConv3dLayerPlugin::enqueue(const sessd_tensor_desc* inputDesc, const sessd_tensor_desc* outputDesc,
                                    const void* const* inputs, void* const* outputs, void* workspace,
                                    hipStream_t stream) {

@@ -339,6 +339,35 @@ def check_order():
         assert (first[0] < first[1]) == chain, (len(layers), dtype, points, first)
 
 
+def check_shared_launches():
+    """Which of a frame's first layers are multiplied in the launch of a pass over coordinates: the first layer beside the numbering, the
+    second beside the lookups where it has 16 channels and every table is kept; what is left of the passes until the first strided
+    layer's rulebook stays on the caller's stream where nothing else is to do there."""
+    ref = B.reference_layers()
+    one = [ref[0]] + ref[2:]
+    wide = B.reference_layers(width_mult=2)
+    f32, f16 = D.SESSD_FLOAT, D.SESSD_HALF
+    other_grid = B.reference_layers()
+    x, y, z = other_grid[1].out_shape
+    other_grid[1].out_shape = (x + 1, y, z)
+    for layers, dtype, numbering, lookups in ((ref, f32, True, True), (ref, f16, True, True), (one, f32, True, False), (wide, f16, True, False),
+                                              (wide, f32, True, False), (ref[:2], f32, False, False), (other_grid, f32, False, False)):
+        for points in (500, 20000):
+            log = launches(overlapped_frame(layers, dtype, max_points=points))
+            caller = log[0][-1]
+            names = [l[1] for l in log]
+            both = [n for n in names if "conv_tall" in n and ("numbering" in n or "number_cuts" in n)]
+            beside = [n for n in names if "conv_tall" in n and "flags_lookups" in n]
+            assert (len(both), len(beside)) == (int(numbering), int(lookups)), (len(layers), dtype, names)
+            if layers is one:  # (the lookups behind the numbering, then the strided layer: no other stream)
+                assert [l[-1] for l in log[:6]] == [caller] * 6 and "flags_lookups" in names[5], log[:7]
+    # without the kept tables the lookups probe hashes and have no room for products
+    FAKE.fake_largest_allocation(16 << 20)
+    names = [l[1] for l in launches(overlapped_frame(ref, f32))]
+    FAKE.fake_largest_allocation(0)
+    assert not any("conv_tall" in n and "flags_lookups" in n for n in names), names
+
+
 def gemm_kernel(cin, cout, rows, dtype, weight=0.0):
     """The kernel that multiplies in a SubM layer of so many rows, `weight` being one of its weights and the others 0 (nothing runs: the
     addresses are read by nobody)."""
@@ -419,6 +448,7 @@ CHECKS = {
     "first-configure": check_first_configure,
     "weights-not-finite": check_weights_not_finite,
     "events": check_events,
+    "shared-launches": check_shared_launches,
     "waits": check_waits,
     "order": check_order,
     "row-limits": check_row_limits,

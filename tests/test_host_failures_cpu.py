@@ -64,3 +64,7 @@ def test_layers_of_a_deep_backbone_do_not_wait_for_the_whole_coordinate_branch(f
 
 def test_the_longer_branch_of_a_small_frame_is_launched_first(fake_hip):
     run_check(fake_hip, "order")
+
+
+def test_first_layers_share_the_launches_of_coordinate_passes(fake_hip):
+    run_check(fake_hip, "shared-launches")
