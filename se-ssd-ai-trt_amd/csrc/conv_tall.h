@@ -288,19 +288,19 @@ __device__ __forceinline__ void workgroup(const TallArgs& g, const DenseTarget& 
             return;
         }
         const int part = wave % BY;
+        int idx[kSteps];
+        const int first_block = begin + wave / BY;
+        if (first_block < end) ask_lists<BY>(t, tid & 63, first_block * 16, part, idx);
+        publish();  // (in front of the rounds: inside, what it needs stays in registers over all of them)
+        if (first_block >= end) lds_barrier();
         bool first = true;
         for (int at = begin; first || at < end; at += WAVES / BY) {
             const int block = at + wave / BY, row0 = block * 16;
             const bool work = block < end;  // (uniform)
             int lane = tid & 63;
             asm volatile("" : "+v"(lane));  // (or what a round reads from LDS is read in front of the rounds, into registers)
-            int idx[kSteps];
             v4f acc[NB];
-            if (work) ask_lists<BY>(t, lane, row0, part, idx);
-            if (first) {
-                publish();
-                if (!work) lds_barrier();
-            }
+            if (work && !first) ask_lists<BY>(t, lane, row0, part, idx);
             if (work) multiply<CIN, COUT, T, BY>(t, lane, idx, part, s_w, first, acc);
             if constexpr (BY > 1) {  // (there is one round: a workgroup has at most WAVES / BY blocks)
                 float4* const sums = reinterpret_cast<float4*>(s_w);

@@ -669,9 +669,10 @@ struct FlagsLookups {
 // side began 7 us after the other, and the first strided layer 8 to 10 us after the later one.  That layer's products begin, us after the
 // frame: FP32 2 000 points 47.7 -> 41.1, 20 000 55.9 -> 49.9, FP16 60 000 61.8 -> 53.2.  Frames FP32 2 000 points 174.0 -> 167.1, 8 000 210.2 -> 202.8,
 // 20 000 257.6 -> 254.9, 80 000 386 -> 378, FP16 8 000 161.9 -> 151.5, 60 000 196.1 -> 189.6, launched directly 20 000 286.7 -> 276.9.  Two
-// workgroups a unit: the same times but 80 000 points, 1.008x.  The registers are held to what lets five blocks (FP16 lookups: seven) share a unit, so that
-// a pass finds room for its blocks beside the products (with 106 instead of 95 the FP32 lookups had four).  Layers with more weights leave
-// the lookups too little LDS.
+// workgroups a unit: the same times but 80 000 points, 1.008x.  The registers are held to what lets five blocks share a unit (lookups
+// beside FP16 products seven, beside FP32 products four: held to five they need scratch, with which a launch begins 3 us later; frames of 2 000
+// points 169.1 -> 167.2, 20 000 256.2 -> 254.8), so that a pass finds room for its blocks beside the products.  Layers with more weights leave the
+// lookups too little LDS.
 constexpr int kProductWaves = kCoordBlock / 64, kPadBlocks = 256;  // (those write the rows beyond the active ones, behind all others)
 template <int CIN, int COUT, typename T>
 using ProductLds = tall::Lds<CIN, COUT, T, kProductWaves>;
@@ -707,7 +708,7 @@ __global__ void __launch_bounds__(kCoordBlock) flags_lookups(int flag_blocks, in
     flags_lookups_block<HASH>(blockIdx.x, flag_blocks, end1, end2, end3, a, L);
 }
 template <int CIN, int COUT, typename T, typename TO>
-__global__ void __launch_bounds__(kCoordBlock, (sizeof(T) == 2 ? 7 : 5)) conv_tall_beside_flags_lookups(int gemm_blocks, int pads_at, int flag_blocks, int end1, int end2,
+__global__ void __launch_bounds__(kCoordBlock, (sizeof(T) == 2 ? 7 : 4)) conv_tall_beside_flags_lookups(int gemm_blocks, int pads_at, int flag_blocks, int end1, int end2,
                                                                                               int end3, TallArgs g, FlagsLookups a) {
     __shared__ union {
         ProductLds<CIN, COUT, T> products;
