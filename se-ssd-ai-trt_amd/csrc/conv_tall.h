@@ -58,14 +58,15 @@ __device__ __forceinline__ void lds_barrier() {
 __device__ __forceinline__ void store4(__half* dst, const float (&o)[4]) { store4h(dst, o); }
 __device__ __forceinline__ void store4(float* dst, const float (&o)[4]) { *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]); }
 
-template <int CIN, int COUT, typename T, int WAVES>
+// (COUT: columns of a workgroup, COLS: of the layer)
+template <int CIN, int COUT, typename T, int WAVES, int COLS = COUT>
 struct Lds {
     static constexpr int kOffsetBytes = CIN * COUT * (int)sizeof(T);
     static constexpr int kSums = WAVES * (COUT / 16) * 1024;  // of waves that share a block
     static constexpr int kWeights = kSteps * 4 * kOffsetBytes;  // (one offset more than there are, of zeros)
     static_assert(kSteps * 4 == KC + 1, "steps");
     alignas(16) unsigned char w[kWeights > kSums ? kWeights : kSums];
-    float epi[2 * COUT];
+    float epi[2 * COLS];  // (scale and shift of all columns)
 };
 
 template <typename TO>
@@ -125,7 +126,7 @@ __device__ __forceinline__ void multiply(const Tensors<TO>& t, int lane, const i
     for (int m = 0; m < N; ++m, w_at += BY * 4 * NB * kPieces * 256) {
         if (BY > 1 && first + m * BY >= kSteps) break;  // (uniform)
         // (the weights of a piece or two at a time: registers)
-        constexpr int kAtOnce = NB > 2 || !kHalf ? 1 : 2;
+        constexpr int kAtOnce = NB > 2 || !kHalf || (CIN == 32 && NB == 1) ? 1 : 2;
         v4u32 w[2][kAtOnce][NB];
         auto weights = [&](int p, v4u32 (&to)[kAtOnce][NB]) {
 #pragma unroll
@@ -175,8 +176,8 @@ __device__ __forceinline__ void multiply(const Tensors<TO>& t, int lane, const i
 }
 
 // lane (i, q) holds output channels 16nb+4q .. +3 of row i
-template <int COUT, typename TO>
-__device__ __forceinline__ void put(const Tensors<TO>& t, int lane, int row0, const v4f (&acc)[COUT / 16], const float* s_epi, const DenseTarget& dt) {
+template <int COUT, int COLS, typename TO>
+__device__ __forceinline__ void put(const Tensors<TO>& t, int lane, int row0, int col0, const v4f (&acc)[COUT / 16], const float* s_epi, const DenseTarget& dt) {
     constexpr int NB = COUT / 16;
     const int i = lane & 15, q = lane >> 4;
     const int row = row0 + i;
@@ -187,7 +188,7 @@ __device__ __forceinline__ void put(const Tensors<TO>& t, int lane, int row0, co
     if (dt.dense) {  // the sparse2Dense scatter of this row, fused (uniform branch)
         const int4 cc = reinterpret_cast<const int4*>(dt.coors)[row];  // (b,z,y,x)
         if (cc.x != 0 || cc.y < 0 || cc.y >= dt.D || cc.z < 0 || cc.z >= dt.H || cc.w < 0 || cc.w >= dt.W) {
-            if (dt.status && q == 0) atomicOr(dt.status, SESSD_STATUS_BAD_COORD);
+            if (dt.status && q == 0 && col0 == 0) atomicOr(dt.status, SESSD_STATUS_BAD_COORD);
         } else {
             to_dense = true;
             d = static_cast<TO*>(dt.dense) + ((size_t)cc.y * dt.Hp + cc.z + dt.pad_top) * dt.Wp + cc.w + dt.pad_left;
@@ -196,17 +197,17 @@ __device__ __forceinline__ void put(const Tensors<TO>& t, int lane, int row0, co
     }
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-        const int c4 = nb * 16 + q * 4;
+        const int c4 = col0 + nb * 16 + q * 4;
         float o[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             float s = acc[nb][e];
             if (t.has_scale) s = s * s_epi[c4 + e];
-            if (t.has_shift) s = s + s_epi[COUT + c4 + e];
+            if (t.has_shift) s = s + s_epi[COLS + c4 + e];
             if (t.relu) s = s > 0.f ? s : 0.f;
             o[e] = s;
         }
-        store4(t.out + (size_t)row * COUT + c4, o);
+        store4(t.out + (size_t)row * COLS + c4, o);
         if (to_dense) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) d[(size_t)(c4 + e) * plane] = (TO)o[e];
@@ -214,9 +215,10 @@ __device__ __forceinline__ void put(const Tensors<TO>& t, int lane, int row0, co
     }
 }
 
-// Workgroup `group` of `groups`, of WAVES waves that multiply and PADS that write the rows beyond the active ones.
-template <int CIN, int COUT, typename T, typename TO, int WAVES, int PADS>
-__device__ __forceinline__ void workgroup(const TallArgs& g, const DenseTarget& dt, int group, int groups, Lds<CIN, COUT, T, WAVES>& lds) {
+// Workgroup `group` of `groups`, of WAVES waves that multiply columns col0 .. col0 + COUT - 1 and PADS that write the rows beyond the active ones.
+template <int CIN, int COUT, typename T, typename TO, int WAVES, int PADS, int COLS = COUT>
+__device__ __forceinline__ void workgroup(const TallArgs& g, const DenseTarget& dt, int group, int groups, Lds<CIN, COUT, T, WAVES, COLS>& lds, int col0 = 0) {
+    static_assert(COLS == COUT || (CIN * sizeof(T) == 64 && PADS == 0), "columns apart: packed as they are multiplied");
     constexpr int NB = COUT / 16, kThreads = (WAVES + PADS) * 64;
     constexpr int kOffsetBytes = CIN * COUT * (int)sizeof(T), kVectors = KC * kOffsetBytes / 16, kCopies = (kVectors + kThreads - 1) / kThreads;
     unsigned char* const s_w = lds.w;
@@ -227,12 +229,13 @@ __device__ __forceinline__ void workgroup(const TallArgs& g, const DenseTarget& 
 #pragma unroll
     for (int c = 0; c < kCopies; ++c) {
         const int v = c * kThreads + tid;
-        copy[c] = reinterpret_cast<const v4f*>(g.w)[v < kVectors ? v : 0];
+        const int in_w = COLS == COUT ? v : (v / (NB * 64) * (COLS / 16) + col0 / 16) * 64 + v % (NB * 64);  // (offset by offset)
+        copy[c] = reinterpret_cast<const v4f*>(g.w)[v < kVectors ? in_w : 0];
     }
     int n = *g.num_out;
     n = n < 0 ? 0 : (n > g.max_voxels ? g.max_voxels : n);
     float by = 1.f, plus = 0.f;
-    if (tid < COUT) {
+    if (tid < COLS) {
         if (g.scale) by = g.scale[tid];
         if (g.shift) plus = g.shift[tid];
     }
@@ -268,9 +271,9 @@ __device__ __forceinline__ void workgroup(const TallArgs& g, const DenseTarget& 
             }
         }
         if (tid < kOffsetBytes / 16) reinterpret_cast<v4f*>(s_w)[kVectors + tid] = (v4f){0.f, 0.f, 0.f, 0.f};
-        if (tid < COUT) {
+        if (tid < COLS) {
             s_epi[tid] = by;
-            s_epi[COUT + tid] = plus;
+            s_epi[COLS + tid] = plus;
         }
     };
     // BY waves a block
@@ -279,7 +282,7 @@ __device__ __forceinline__ void workgroup(const TallArgs& g, const DenseTarget& 
         if (PADS && wave >= WAVES) {
             publish();
             lds_barrier();
-            write_pad_rows<TO, COUT>(t.out, n, g.max_voxels, group * (PADS * 64) + (tid - WAVES * 64), groups * (PADS * 64), s_epi, t.has_scale,
+            write_pad_rows<TO, COLS>(t.out, n, g.max_voxels, group * (PADS * 64) + (tid - WAVES * 64), groups * (PADS * 64), s_epi, t.has_scale,
                                      t.has_shift, t.relu);
             if (BY > 1) {  // (the barriers below)
                 lds_barrier();
@@ -321,7 +324,7 @@ __device__ __forceinline__ void workgroup(const TallArgs& g, const DenseTarget& 
                             acc[nb][3] += v.w;
                         }
             }
-            if (work && part == 0) put<COUT>(t, lane, row0, acc, s_epi, dt);
+            if (work && part == 0) put<COUT, COLS>(t, lane, row0, col0, acc, s_epi, dt);
             first = false;
         }
     };

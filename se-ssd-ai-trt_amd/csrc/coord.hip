@@ -671,15 +671,21 @@ struct FlagsLookups {
 // 20 000 257.6 -> 254.9, 80 000 386 -> 378, FP16 8 000 161.9 -> 151.5, 60 000 196.1 -> 189.6, launched directly 20 000 286.7 -> 276.9.  Two
 // workgroups a unit: the same times but 80 000 points, 1.008x.  The registers are held to what lets five blocks share a unit (lookups
 // beside FP16 products seven, beside FP32 products four: held to five they need scratch, with which a launch begins 3 us later; frames of 2 000
-// points 169.1 -> 167.2, 20 000 256.2 -> 254.8), so that a pass finds room for its blocks beside the products.  Layers with more weights leave the
-// lookups too little LDS.
+// points 169.1 -> 167.2, 20 000 256.2 -> 254.8), so that a pass finds room for its blocks beside the products.  32 -> 32 in FP16 is
+// multiplied by two workgroups of 16 columns each, which read the rows twice: with 54 KB of weights a unit would have room for two blocks (doubled
+// widths, 30 000 points 284.9 -> 275.8 us, 150 000 0.997x, where the lookups are three rounds of blocks).
 constexpr int kProductWaves = kCoordBlock / 64, kPadBlocks = 256;  // (those write the rows beyond the active ones, behind all others)
 template <int CIN, int COUT, typename T>
-using ProductLds = tall::Lds<CIN, COUT, T, kProductWaves>;
+constexpr int kProductCols = CIN == 32 ? 16 : COUT;
+template <int CIN, int COUT, typename T>
+using ProductLds = tall::Lds<CIN, kProductCols<CIN, COUT, T>, T, kProductWaves, COUT>;
+static int product_blocks(const GemmArgs& a) { return gemm_compute_units() * (a.cin == 32 ? 2 : 1); }
 
 template <int CIN, int COUT, typename T, typename TO>
 __device__ __forceinline__ void products_pass(const TallArgs& g, int block, int blocks, ProductLds<CIN, COUT, T>& lds) {
-    tall::workgroup<CIN, COUT, T, TO, kProductWaves, 0>(g, DenseTarget(), block, blocks, lds);
+    constexpr int kCols = kProductCols<CIN, COUT, T>;
+    const int groups = blocks / (COUT / kCols), part = block / groups;
+    tall::workgroup<CIN, kCols, T, TO, kProductWaves, 0, COUT>(g, DenseTarget(), block - part * groups, groups, lds, part * kCols);
 }
 template <int CIN, int COUT, typename T, typename TO>
 __device__ __forceinline__ void products_pad_pass(const TallArgs& g, int block, ProductLds<CIN, COUT, T>& lds) {
@@ -708,7 +714,7 @@ __global__ void __launch_bounds__(kCoordBlock) flags_lookups(int flag_blocks, in
     flags_lookups_block<HASH>(blockIdx.x, flag_blocks, end1, end2, end3, a, L);
 }
 template <int CIN, int COUT, typename T, typename TO>
-__global__ void __launch_bounds__(kCoordBlock, (sizeof(T) == 2 ? 7 : 4)) conv_tall_beside_flags_lookups(int gemm_blocks, int pads_at, int flag_blocks, int end1, int end2,
+__global__ void __launch_bounds__(kCoordBlock, (sizeof(T) == 4 ? 4 : CIN == 32 ? 5 : 7)) conv_tall_beside_flags_lookups(int gemm_blocks, int pads_at, int flag_blocks, int end1, int end2,
                                                                                               int end3, TallArgs g, FlagsLookups a) {
     __shared__ union {
         ProductLds<CIN, COUT, T> products;
@@ -1066,7 +1072,7 @@ bool number_takes_products(const GemmArgs& a) { return a.cin == 4 && !a.dense.de
 bool lookups_take_products(const GemmArgs& a, const LookupPart* lookups, int n) {
     for (int l = 0; l < n; ++l)
         if (!lookups[l].t.dense) return false;
-    return n <= kMaxLookups && a.cin == 16 && a.cout == 16 && !a.dense.dense && tall_takes(a);
+    return n <= kMaxLookups && a.cin == a.cout && (a.cin == 16 || (a.cin == 32 && a.in_type == SESSD_HALF)) && !a.dense.dense && tall_takes(a);
 }
 
 static int flags_lookups_launch(const SpPart* flags, const LookupPart* lookups, int n, const GemmArgs* products, hipStream_t stream) {
@@ -1096,12 +1102,13 @@ static int flags_lookups_launch(const SpPart* flags, const LookupPart* lookups, 
     if (products) {
         if (!lookups_take_products(*products, lookups, n)) return fail(SESSD_E_UNSUPPORTED, "lookups: a layer's products cannot share this launch");
         const TallArgs g = tall_args(*products);
-        const int gemm_blocks = gemm_compute_units(), pads_at = gemm_blocks + blocks;
+        const int gemm_blocks = product_blocks(*products), pads_at = gemm_blocks + blocks;
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(pads_at + (products->write_pad_rows ? kPadBlocks : 0)), dim3(kCoordBlock), 0, stream, gemm_blocks, pads_at, flag_blocks, end[0],
                                end[1], end[2], g, a);
         };
-        products->in_type == SESSD_HALF ? go(conv_tall_beside_flags_lookups<16, 16, __half, __half>) : go(conv_tall_beside_flags_lookups<16, 16, float, float>);
+        if (products->cin == 32) go(conv_tall_beside_flags_lookups<32, 32, __half, __half>);
+        else products->in_type == SESSD_HALF ? go(conv_tall_beside_flags_lookups<16, 16, __half, __half>) : go(conv_tall_beside_flags_lookups<16, 16, float, float>);
         SESSD_HIP_TRY(hipGetLastError());
         return SESSD_OK;
     }
@@ -1164,7 +1171,7 @@ static int number_launch(const SpPart* number, const SpPart* next, const CutPart
     if (products) {
         if (!number_takes_products(*products)) return fail(SESSD_E_UNSUPPORTED, "numbering: a layer's products cannot share this launch");
         const TallArgs g = tall_args(*products);
-        const int gemm_blocks = gemm_compute_units(), pads_at = gemm_blocks + blocks;
+        const int gemm_blocks = product_blocks(*products), pads_at = gemm_blocks + blocks;
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(pads_at + (products->write_pad_rows ? kPadBlocks : 0)), dim3(kCoordBlock), 0, stream, gemm_blocks, pads_at, number_blocks,
                                has_next, end[0], end[1], end[2], end[3], clean_end, g, a);

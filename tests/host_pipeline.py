@@ -341,7 +341,7 @@ def check_order():
 
 def check_shared_launches():
     """Which of a frame's first layers are multiplied in the launch of a pass over coordinates: the first layer beside the numbering, the
-    second beside the lookups where it has 16 channels and every table is kept; what is left of the passes until the first strided
+    second beside the lookups where it has 16 channels, in FP16 also 32, and every table is kept; what is left of the passes until the first strided
     layer's rulebook stays on the caller's stream where nothing else is to do there."""
     ref = B.reference_layers()
     one = [ref[0]] + ref[2:]
@@ -350,7 +350,7 @@ def check_shared_launches():
     other_grid = B.reference_layers()
     x, y, z = other_grid[1].out_shape
     other_grid[1].out_shape = (x + 1, y, z)
-    for layers, dtype, numbering, lookups in ((ref, f32, True, True), (ref, f16, True, True), (one, f32, True, False), (wide, f16, True, False),
+    for layers, dtype, numbering, lookups in ((ref, f32, True, True), (ref, f16, True, True), (one, f32, True, False), (wide, f16, True, True),
                                               (wide, f32, True, False), (ref[:2], f32, False, False), (other_grid, f32, False, False)):
         for points in (500, 20000):
             log = launches(overlapped_frame(layers, dtype, max_points=points))
