@@ -51,7 +51,7 @@ def kernel_source_hash():
     """Short hash of the gather-GEMM kernels' sources: the committed counter summaries carry the hash of the sources
     they were collected on, so a figure taken from them can be told from a stale one."""
     h = hashlib.sha256()
-    for name in ("conv_tall.hip", "conv_tile.hip", "conv_wide.hip", "pad_rows.h"):
+    for name in ("conv_tall.h", "conv_tall.hip", "conv_tile.hip", "conv_wide.hip", "pad_rows.h"):
         with open(os.path.join(ROOT, "se-ssd-ai-trt_amd", "csrc", name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()[:12]
