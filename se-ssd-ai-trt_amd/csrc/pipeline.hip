@@ -384,9 +384,13 @@ struct Pipeline {
         // Each pass by itself / for the branch's end / so, us: the reference's backbone, FP32 2 000 points 183, 178, 178, 20 000 252, 247, 247,
         // FP16 60 000 222, 219, 219 (so is its end); four strided layers more, each with two SubM layers, FP32 2 000 points 343, 371, 330,
         // 20 000 487, 517, 474, FP16 20 000 319, 328, 311; twelve more, FP32 2 000 675, 770, 645.
-        // Passes that are waited for one by one: to the lookups on the second strided layer's rows, with few points to their tile cuts (2 000 points
-        // 182 -> 168 us, the branch's end is 15 us away then; 20 000 253.9 -> 258.5).
-        const int kOwnWaits = desc.max_points > 10000 ? 4 : 5;
+        // Passes that are waited for one by one: to the lookups on the second strided layer's rows, with few points where pass 2 is on the caller's
+        // stream to their tile cuts.  Four / five so, FP32, us: 2 000 points 179.3 / 165.5 (the branch's end is 15 us away then), 4 000 195.6 / 185.5, 8 000
+        // 204.4 / 201.2, 10 000 213.9 / 212.2, 12 000 220.6 / 222.8, 14 000 221.5 / 223.4, 16 000 229.9 / 224.2, 18 000 233.8 / 231.2, 20 000 253.8 / 255.1, 30 000
+        // to 80 000 five 1.003-1.008x; one SubM layer in front 2 000 179.0 / 164.0, 20 000 251.3 / 245.5; three 2 000 179.8 / 171.1, 8 000 204.7 / 206.5.
+        // Elsewhere: doubled widths 2 000 248.2 / 250.6, 5 000 326.7 / 329.5, 10 000 431.8 / 434.6; without a kept table of the voxels 2 000 183.7 / 187.2, 8 000
+        // 224.9 / 227.9.  FP16 layers need no cuts: the same frames.
+        const int kOwnWaits = apart && desc.max_points <= 10000 ? 5 : 4;
         constexpr int kAhead = 2, kRest = 4;
         hipStream_t side = fork ? aux : stream;
         std::vector<int> wait_for(stages.size(), 0);

@@ -324,6 +324,26 @@ def check_waits():
     assert waits[at] == waits[at - 1] + 1, waits
 
 
+def check_own_waits():
+    """Frames of few points wait for one pass more by itself where a layer's products share the launch of the lookups, and only there:
+    elsewhere the layers wait for the same passes whatever the points."""
+    ref, wide = B.reference_layers(), B.reference_layers(width_mult=2)
+    own_grid = B.reference_layers()
+    x, y, z = own_grid[1].out_shape
+    own_grid[1].out_shape = (x + 1, y, z)
+
+    def awaited(layers, points):  # by each layer, lookups that it is ordered behind, and all waits of the frame
+        log = overlapped_frame(layers, D.SESSD_FLOAT, max_points=points)
+        return passes_before_gemms(log), sum(l[0] == "wait" for l in log)
+
+    assert awaited(ref, 500)[1] == awaited(ref, 10000)[1] == awaited(ref, 10001)[1] + 1 == awaited(ref, 80000)[1] + 1
+    for layers in (wide, own_grid):
+        assert awaited(layers, 500) == awaited(layers, 10000) == awaited(layers, 10001), len(layers)
+    FAKE.fake_largest_allocation(300 << 20)  # (no kept table of the voxels)
+    assert awaited(ref, 500) == awaited(ref, 10001)
+    FAKE.fake_largest_allocation(0)
+
+
 def check_order():
     """Which of an overlapped frame's branches is launched first: with few points the one with more launches until the second strided
     layer's rulebook, else the chain of layers."""
@@ -451,6 +471,7 @@ CHECKS = {
     "shared-launches": check_shared_launches,
     "waits": check_waits,
     "order": check_order,
+    "own-waits": check_own_waits,
     "row-limits": check_row_limits,
     "recovery-direct": lambda: check_recovery(0, enqueue),
     "recovery-overlap": lambda: check_recovery(1, enqueue),

@@ -62,6 +62,10 @@ def test_layers_of_a_deep_backbone_do_not_wait_for_the_whole_coordinate_branch(f
     run_check(fake_hip, "waits")
 
 
+def test_small_frames_wait_for_a_pass_more_only_where_launches_are_shared(fake_hip):
+    run_check(fake_hip, "own-waits")
+
+
 def test_the_longer_branch_of_a_small_frame_is_launched_first(fake_hip):
     run_check(fake_hip, "order")
 
