@@ -348,6 +348,10 @@ struct Pipeline {
         // they share launches on the caller's stream: pass 1 with layer 0's products, where its kernel leaves the pass room, pass 2 with layer 1's
         // (or, where the first strided layer is next, alone).  The other branch begins behind pass 1, with the flags for pass 3.  The figures
         // are at the kernels (coord.hip).  (Flags beside the lookups as well, the branch behind pass 2: 2 000 points 1.04x, the passes end too late.)
+        // Where pass 2 cannot follow on the caller's stream the branches begin behind pass 0 and nothing is shared.  Layer 0 alone beside pass 1, the
+        // branches behind it / so, us: voxels' table not kept, FP32 2 000 points 183.7 / 183.0, 14 000 256.3 / 250.4, 80 000 430.2 / 427.4, FP16 8 000
+        // 178.2 / 174.6, 60 000 225.9 / 221.0; FP32 doubled widths 2 000 248.2 / 246.7, 20 000 564.4 / 558.5, 40 000 717.2 / 714.8, 80 000 973.9 / 978.9.  On one stream
+        // sharing costs no branch anything: FP32 doubled widths 2 000 points 325.2 -> 320.5, 20 000 626.8 -> 623.7.
         int last_main = 0, clean_at = m < 1 ? 0 : 1;  // (stage 1's own rulebook is the last reader of the voxels' table)
         int beside[3] = {-1, -1, -1};
         auto rulebookPass = [&](size_t l) { return ready[(size_t)(stages[l]->rulebook_from >= 0 ? stages[l]->rulebook_from : (int)l)]; };
@@ -355,6 +359,7 @@ struct Pipeline {
             return stages[l]->subm->sharedGemmArgs(l ? stages[l - 1]->feat.p : vg_voxels.p, stages[l]->feat.p, static_cast<const int32_t*>(vg_num.p),
                                                    stages[(size_t)(stages[l]->rulebook_from >= 0 ? stages[l]->rulebook_from : (int)l)]->ws.p);
         };
+        const bool fork = aux != nullptr && stages.size() > 0;
         if (m >= 1 && stages.size() > 2 && cs[0].builds.empty() && cs[0].lookups.size() <= (size_t)kMaxCuts && stages[0]->subm && rulebookPass(0) == 0 &&
             number_takes_products(productsOf(0))) {
             beside[1] = 0;
@@ -368,8 +373,11 @@ struct Pipeline {
                 beside[2] = 1;
                 last_main = 2;
             }
+            if (fork && last_main == 1) {
+                beside[1] = -1;
+                last_main = 0;
+            }
         }
-        const bool fork = aux != nullptr && stages.size() > 0;
         const bool apart = fork && last_main == 2;  // pass 2 runs beside the passes behind it but for the one that empties the table
         if (apart && m >= 2) {
             clean_at = 2;

@@ -260,7 +260,12 @@ def deeper(stages):
 
 def overlapped_frame(layers, dtype, **options):
     """The log of a frame on two streams."""
-    rc, h = create(layers, overlap_streams=1, feature_dtype=dtype, **options)
+    return frame(layers, dtype, overlap_streams=1, **options)
+
+
+def frame(layers, dtype, **options):
+    """The log of a frame, on one stream by default."""
+    rc, h = create(layers, feature_dtype=dtype, **options)
     assert rc == 0, L.sessd_last_error()
     stream = new_stream()
     assert enqueue(h, stream) == 0
@@ -341,7 +346,7 @@ def check_own_waits():
         assert awaited(layers, 500) == awaited(layers, 10000) == awaited(layers, 10001), len(layers)
     FAKE.fake_largest_allocation(300 << 20)  # (no kept table of the voxels)
     assert awaited(ref, 500) == awaited(ref, 10001)
-    FAKE.fake_largest_allocation(0)
+    FAKE.fake_largest_allocation(2 ** 64 - 1)
 
 
 def check_order():
@@ -362,7 +367,8 @@ def check_order():
 def check_shared_launches():
     """Which of a frame's first layers are multiplied in the launch of a pass over coordinates: the first layer beside the numbering, the
     second beside the lookups where it has 16 channels, in FP16 also 32, and every table is kept; what is left of the passes until the first strided
-    layer's rulebook stays on the caller's stream where nothing else is to do there."""
+    layer's rulebook stays on the caller's stream where nothing else is to do there.  On two streams the first layer's launch is shared only
+    where the lookups follow on the caller's stream, on one wherever it can be."""
     ref = B.reference_layers()
     one = [ref[0]] + ref[2:]
     wide = B.reference_layers(width_mult=2)
@@ -371,7 +377,7 @@ def check_shared_launches():
     x, y, z = other_grid[1].out_shape
     other_grid[1].out_shape = (x + 1, y, z)
     for layers, dtype, numbering, lookups in ((ref, f32, True, True), (ref, f16, True, True), (one, f32, True, False), (wide, f16, True, True),
-                                              (wide, f32, True, False), (ref[:2], f32, False, False), (other_grid, f32, False, False)):
+                                              (wide, f32, False, False), (ref[:2], f32, False, False), (other_grid, f32, False, False)):
         for points in (500, 20000):
             log = launches(overlapped_frame(layers, dtype, max_points=points))
             caller = log[0][-1]
@@ -382,10 +388,13 @@ def check_shared_launches():
             if layers is one:  # (the lookups behind the numbering, then the strided layer: no other stream)
                 assert [l[-1] for l in log[:6]] == [caller] * 6 and "flags_lookups" in names[5], log[:7]
     # without the kept tables the lookups probe hashes and have no room for products
+    shared = lambda log: [l[1] for l in launches(log) if "conv_tall" in l[1] and ("numbering" in l[1] or "number_cuts" in l[1] or "lookups" in l[1])]  # noqa: E731
     FAKE.fake_largest_allocation(16 << 20)
-    names = [l[1] for l in launches(overlapped_frame(ref, f32))]
-    FAKE.fake_largest_allocation(0)
-    assert not any("conv_tall" in n and "flags_lookups" in n for n in names), names
+    assert not shared(overlapped_frame(ref, f32)) and not shared(overlapped_frame(ref, f16))
+    assert len(shared(frame(ref, f32))) == 1
+    FAKE.fake_largest_allocation(2 ** 64 - 1)
+    for layers, dtype, n in ((ref, f32, 2), (wide, f32, 1), (wide, f16, 2), (other_grid, f32, 0)):
+        assert len(shared(frame(layers, dtype))) == n, (len(layers), dtype)
 
 
 def gemm_kernel(cin, cout, rows, dtype, weight=0.0):
