@@ -292,7 +292,7 @@ bool number_takes_products(const GemmArgs& a);
 bool lookups_take_products(const GemmArgs& a, const LookupPart* lookups, int n);
 int launch_flags_lookups_products(const SpPart* flags, const LookupPart* lookups, int n, const GemmArgs& products, hipStream_t stream);
 int launch_number_products(const SpPart* number, const SpPart* next, const CutPart* cuts, int n_cuts, const CleanPart* clean, const FillArgs* also,
-                           const GemmArgs& products, bool products_first, hipStream_t stream);
+                           const GemmArgs& products, hipStream_t stream);
 int launch_sp_flags(const SpPart& s, hipStream_t stream);
 int launch_sp_scatter(const SpPart& s, hipStream_t stream);
 int launch_tile_weights(const int32_t* nbr, const int32_t* num_out, int K, int max_voxels, int row_weight, void* region, hipStream_t stream);

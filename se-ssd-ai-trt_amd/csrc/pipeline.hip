@@ -404,7 +404,7 @@ struct Pipeline {
         std::vector<int> wait_for(stages.size(), 0);
         std::vector<char> awaited((size_t)(2 * m + 2), 0);
         bool join = false;  // at the end, for what no layer has waited for
-        int longer = -1;    // passes less layers in front of the last layer until the second strided layer's rulebook that needs a pass anew
+        int longer = -3;    // passes less layers in front of the last layer until the second strided layer's rulebook that needs a pass anew
         if (fork) {
             int seen = 0;
             for (size_t l = 0; l < stages.size(); ++l) {
@@ -460,25 +460,28 @@ struct Pipeline {
             }
             return SESSD_OK;
         };
-        // Of the two branches that begin here the one that is launched first follows at once in a graph, the other 6 us later.  With few
-        // points a layer takes about as long as a pass, so that the longer one until the second strided layer's rulebook is the one with more
-        // launches: the passes in the reference's backbone in FP32 (five for five layers; in FP16, without tile cuts, four), the
-        // chain with four SubM layers in front of the first strided one.  Layers grow with the points and passes hardly.  Passes first /
-        // chain first, us, FP32 and FP16: 2 000 points 177.5 / 184.0, 164.2 / 166.1, 5 000 204.3 / 208.2, 170.3 / 168.7, 8 500 218.9 / 221.7,
-        // 172.8 / 171.0, 12 000 242.5 / 240.8, 177.8 / 174.4, 40 000 331.6 / 320.9, 206.5 / 205.3; one SubM layer in front 5 000 203.9 / 207.8,
-        // 165.9 / 169.1, 20 000 244.0 / 245.6, 177.3 / 177.7; four 2 000 189.8 / 182.8, 176.6 / 167.3, 10 000 256.3 / 252.5, 194.3 / 185.8; doubled
-        // widths, FP32 5 000 332.6 / 341.4, 20 000 478.4 / 476.3.  The points are those that the tensor holds, which is what the host
-        // knows: a frame of 2 000 points in a tensor for 20 000 takes 184.7, passes first it would be 177.7.  (Measured while the branches
-        // began behind pass 0.  Where the first layer shares the launch of pass 1 the rule says whose blocks are the first of its grid.)
-        const bool chain_first = longer < 0 || desc.max_points > 10000;
+        // Of the two branches the one that is launched first follows at once in a graph, the other 6 us later.  Behind shared launches
+        // that is the chain (flags and pass 3 captured in front of pass 2: 2 000 points FP32 165.9 -> 175.6 us, FP16 144.8 -> 152.4, 20 000 252.8 -> 258.2 and 169.6 ->
+        // 178.2).  Elsewhere a layer takes a little less than a pass with few points, and layers grow with the points and passes hardly,
+        // in FP16 a third as fast: it is the passes with up to two SubM layers in front of the first strided one until 50 000 points (FP16 150 000), with
+        // three until 10 000 (30 000), and always the chain with more.  Passes first / chain first, us, FP32 and FP16, the reference's backbone
+        // 2 000 points 172.6 / 176.5, 149.6 / 154.6, 20 000 259.2 / 260.0, 174.1 / 179.6, 40 000 311.0 / 311.6, 60 000 350.0 / 344.3, 191.6 / 196.2, 80 000 387.2 / 384.9, on
+        // hashes 2 000 195.9 / 199.1, 171.3 / 174.9, 20 000 286.0 / 291.5, 205.6 / 210.0, 60 000 FP16 247.1 / 251.4, 80 000 446.8 / 440.8; one SubM layer 5 000 198.6 /
+        // 202.2, 20 000 253.4 / 257.1; three 8 000 215.2 / 215.7, 159.4 / 161.9, 20 000 269.9 / 267.7, 177.8 / 178.8, 40 000 329.9 / 322.3, 60 000 FP16 202.9 / 198.7; four 2 000
+        // 179.5 / 177.2, 156.8 / 155.1, 20 000 276.2 / 272.5, 182.7 / 178.4, 40 000 340.4 / 329.3, 60 000 FP16 209.6 / 197.1; doubled widths 5 000 322.5 / 325.3, 20 000 544.0 /
+        // 550.5, 80 000 978.9 / 969.2, FP16 8 000 220.4 / 223.5, 60 000 303.6 / 302.6, 150 000 425.7 / 429.9.  The points are those that the tensor holds, which is what the host
+        // knows.
+        const bool half = desc.feature_dtype == SESSD_HALF;
+        const int ahead = longer + (half ? 1 : 0);  // (FP16 layers need no tile cuts: one pass less)
+        const bool chain_first = apart || ahead < -1 || desc.max_points > (half ? 3 : 1) * (ahead < 0 ? 10000 : 50000);
         auto behindPass = [&](int pass) -> int {
             if (!fork) return SESSD_OK;
-            if (pass == (apart ? 1 : last_main)) {
+            if (pass == (apart ? 1 : 0)) {
                 SESSD_HIP_TRY(hipEventRecord(ev_head, stream));
                 SESSD_HIP_TRY(hipStreamWaitEvent(side, ev_head, 0));
             }
             if (apart && pass == 2) SESSD_HIP_TRY(hipEventRecord(ev_pass[2], stream));
-            if (pass == last_main && (chain_first || last_main == 2)) return layers(last_main);
+            if (pass == last_main && chain_first) return layers(last_main);
             if (awaited[(size_t)pass]) SESSD_HIP_TRY(hipEventRecord(ev_pass[(size_t)pass], side));
             return SESSD_OK;
         };
@@ -533,7 +536,7 @@ struct Pipeline {
             bool did = false;
             if (with_number >= 0) {
                 SESSD_TRY(launch_number_products(next, after, cuts.data(), (int)cuts.size(), clean.taken ? &clean : nullptr, &clear, productsOf((size_t)with_number),
-                                                 chain_first, s_number));
+                                                 s_number));
                 launched(with_number);
                 at = cuts.size();
                 did = true;

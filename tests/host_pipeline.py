@@ -350,18 +350,33 @@ def check_own_waits():
 
 
 def check_order():
-    """Which of an overlapped frame's branches is launched first: with few points the one with more launches until the second strided
-    layer's rulebook, else the chain of layers."""
+    """Which of an overlapped frame's branches is launched first.  Where the first layers share launches with passes it is the chain of layers,
+    elsewhere, with few points and fewer layers than passes until the second strided layer's rulebook, the other one."""
     ref = B.reference_layers()
     one = [B.Layer("subm0", D.SESSD_LAYER_SUBM, 4, 16, ref[0].out_shape)] + ref[2:]
-    four = ref[:2] + [ref[1]] * 2 + ref[2:]
+    three, four = ref[:2] + [ref[1]] + ref[2:], ref[:2] + [ref[1]] * 2 + ref[2:]
     f32, f16 = D.SESSD_FLOAT, D.SESSD_HALF
-    for layers, dtype, points, chain in ((ref, f32, 500, False), (ref, f32, 10000, False), (ref, f32, 10001, True), (ref, f16, 500, True),
-                                         (one, f32, 500, False), (one, f16, 500, False), (one, f16, 20000, True), (four, f32, 500, True),
-                                         (four, f16, 500, True), (deeper(2), f32, 500, False), (ref[:2], f32, 500, True)):
-        names = [l[1] for l in launches(overlapped_frame(layers, dtype, max_points=points))]
-        first = [i for i, n in enumerate(names) if "conv_" in n][0], [i for i, n in enumerate(names) if "number_cuts" in n][0]
-        assert (first[0] < first[1]) == chain, (len(layers), dtype, points, first)
+
+    def chain_first(layers, dtype, points, shared):
+        log = launches(overlapped_frame(layers, dtype, max_points=points))
+        beside = [i for i, l in enumerate(log) if "conv_tall_then_numbering" in l[1] or "conv_tall_beside" in l[1]]
+        assert bool(beside) == shared, (len(layers), dtype, points, log)
+        layer = [i for i, l in enumerate(log) if "conv_" in l[1] and i not in beside][0]
+        other = [i for i, l in enumerate(log) if l[-1] != log[0][-1]][0]
+        assert log[layer][-1] == log[0][-1]
+        return layer < other
+
+    for layers, dtype, points in ((ref, f32, 500), (ref, f32, 10000), (ref, f32, 10001), (ref, f16, 500), (one, f32, 500), (one, f16, 500),
+                                  (one, f16, 20000), (three, f32, 500), (four, f32, 500), (four, f16, 500), (deeper(2), f32, 500)):
+        assert chain_first(layers, dtype, points, True), (len(layers), dtype, points)
+    assert chain_first(ref[:2], f32, 500, False)  # (no strided layer)
+    FAKE.fake_largest_allocation(40 << 20)  # (no kept tables of the voxels and the first strided layer: nothing is shared)
+    for layers, dtype, points, chain in ((ref, f32, 500, False), (ref, f32, 50000, False), (ref, f32, 50001, True), (ref, f16, 500, False),
+                                         (ref, f16, 150000, False), (ref, f16, 150001, True), (three, f32, 10000, False), (three, f32, 10001, True),
+                                         (three, f16, 30000, False), (three, f16, 30001, True), (four, f32, 500, True), (four, f16, 500, True),
+                                         (deeper(2), f32, 500, False), (ref[:2], f32, 500, True)):
+        assert chain_first(layers, dtype, points, False) == chain, (len(layers), dtype, points)
+    FAKE.fake_largest_allocation(2 ** 64 - 1)
 
 
 def check_shared_launches():
