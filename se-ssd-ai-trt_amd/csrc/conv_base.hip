@@ -129,6 +129,7 @@ GemmArgs ConvPluginBase::gemmArgs(const void* in_feat, void* out_feat, const int
     a.w_f16 = weights_half_dev_;
     a.w_packed = weights_packed_dev_;
     a.halves_finite = halves_finite_;
+    a.strided = strided_;
     a.scale = epi_.scale_dev;
     a.shift = epi_.shift_dev;
     a.relu = epi_.relu;

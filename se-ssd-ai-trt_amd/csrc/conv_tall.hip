@@ -79,6 +79,8 @@ int launch(const GemmArgs& a, hipStream_t stream) {
 
 bool gemm_runs_tall(int K, int cin, int cout) { return K == tall::KC && ((cin == 32 && (cout == 64 || cout == 32)) || (cin == 16 && (cout == 16 || cout == 32))); }
 
+constexpr int kFewStridedRows = 8192;
+
 bool tall_takes(const GemmArgs& a) {
     // (0 x infinity: with weights that are not finite an absent neighbour may not be a row of zeros)
     if (!a.w_packed || !a.halves_finite || a.force_valu || a.K != tall::KC) return false;
@@ -87,7 +89,10 @@ bool tall_takes(const GemmArgs& a) {
     if ((size_t)a.max_voxels * (tall::KC * sizeof(int32_t)) >= tall::kOutOfRange) return false;
     if (a.in_type == SESSD_HALF) return a.out_type == SESSD_HALF && gemm_runs_tall(a.K, a.cin, a.cout);
     if (a.cin == 4) return a.cout == 16 || a.cout == 32;
-    return a.out_type == SESSD_FLOAT && a.cin == 16 && a.cout == 16;
+    // (a strided layer's rows have three or four neighbours: the pair lists are short.  A call, rulebook included, here / there, at a frame's sites
+    // 1 000 rows 21.2 / 22.7 us, 5 000 24.6 / 25.4, 12 000 28.3 / 28.1, 27 585 36.9 / 35.2, 49 642 47.4 / 45.8, 92 422 69.2 / 64.9; isolated ones 5 000 26.7 / 26.6,
+    // 60 000 79.4 / 69.7.  The host knows the rows that the tensors hold.  4 -> 16 at 27 585 32.9 / 34.3, 92 422 62.0 / 64.9, isolated 60 000 70.7 / 69.6)
+    return a.out_type == SESSD_FLOAT && a.cin == 16 && a.cout == 16 && (!a.strided || a.max_voxels <= kFewStridedRows);
 }
 
 TallArgs tall_args(const GemmArgs& a) {

@@ -19,6 +19,7 @@ struct GemmArgs {
     const __half* w_f16;     // same layout, rounded to half (used when in_type is HALF)
     const void* w_packed;    // MFMA operand order, or null
     bool halves_finite = false;  // all of w_f16, hence of w_f32: 0 x w is 0 (a kernel may multiply absent neighbours as rows of zeros)
+    bool strided = false;    // the rows are others than the input's: fewer neighbours each
     const float* scale;      // [cout] or null
     const float* shift;      // [cout] or null
     int relu;

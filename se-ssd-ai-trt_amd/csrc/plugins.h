@@ -103,6 +103,7 @@ class ConvPluginBase {
     void* weights_packed_dev_ = nullptr;  // MFMA B-operand order (see conv_gemm.hip)
     int packed_dtype_ = -1;
     bool halves_finite_ = false;  // no infinity and no NaN among the FP16 weights
+    bool strided_ = false;        // a SparseConv3dLayerPlugin
     Epilogue epi_;
     int in_type_ = SESSD_FLOAT, out_type_ = SESSD_FLOAT;
     int flags_ = 0;
@@ -191,6 +192,7 @@ class SubmConv3dLayerPlugin : public ConvPluginBase {
 // ---------------------------------------------------------------------------------------------
 class SparseConv3dLayerPlugin : public ConvPluginBase {
   public:
+    SparseConv3dLayerPlugin() { strided_ = true; }
     static int create(const sessd_sparseconv3d_desc& d, const float* weights,
                       SparseConv3dLayerPlugin** out);
     static int deserialize(const void* data, size_t length, SparseConv3dLayerPlugin** out);

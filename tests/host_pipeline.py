@@ -456,6 +456,25 @@ def check_weights_not_finite():
             assert "conv_wide" in gemm_kernel(cin, cout, 9000, f32, weight), (cin, cout, weight)
 
 
+def check_strided_few_channels():
+    """A strided FP32 layer 16 -> 16 of more than 8 192 rows multiplies pairs, a smaller one, a SubM layer of its size and strided layers with 4
+    channels or in FP16 all offsets."""
+    ref = B.reference_layers()
+    f32, f16 = D.SESSD_FLOAT, D.SESSD_HALF
+
+    def strided(cin, cout):
+        return B.Layer("strided", D.SESSD_LAYER_SPARSE, cin, cout, ref[2].out_shape, (3, 3, 3), (2, 2, 2), (1, 1, 1))
+
+    for dtype, rows, first, layer, kernel in ((f32, 8193, ref[:1], strided(16, 16), "conv_wideILi16ELi16Eff"), (f32, 8192, ref[:1], strided(16, 16), "conv_tallILi16ELi16Eff"),
+                                              (f16, 8193, ref[:1], strided(16, 16), "conv_tallILi16ELi16E"), (f32, 60000, [], strided(4, 16), "conv_tallILi4ELi16Eff"),
+                                              (f32, 60000, [], strided(4, 32), "conv_tallILi4ELi32Eff")):
+        layers = first + [layer, B.Layer("subm", D.SESSD_LAYER_SUBM, layer.cout, layer.cout, layer.out_shape)]
+        names = [l[1] for l in launches(overlapped_frame(layers, dtype, layer_max_voxels=rows)) if "conv_" in l[1]]
+        assert len(names) == len(layers) and kernel in names[len(first)], names
+        if dtype == f32 and layer.cout == 16:
+            assert "conv_tallILi16ELi16Eff" in names[-1], names
+
+
 def check_first_configure():
     """Configuring a layer for FP16 packs its weights, and does nothing else that takes as long: the first call of a layer waits for it."""
     rng = np.random.default_rng(0)
@@ -497,6 +516,7 @@ CHECKS = {
     "order": check_order,
     "own-waits": check_own_waits,
     "row-limits": check_row_limits,
+    "strided-few-channels": check_strided_few_channels,
     "recovery-direct": lambda: check_recovery(0, enqueue),
     "recovery-overlap": lambda: check_recovery(1, enqueue),
     "recovery-timed": lambda: check_recovery(1, timed),

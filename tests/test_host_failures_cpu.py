@@ -42,6 +42,10 @@ def test_layers_with_few_channels_run_on_the_matrix_cores_in_large_tensors(fake_
     run_check(fake_hip, "row-limits")
 
 
+def test_strided_fp32_layers_with_16_channels_multiply_pairs(fake_hip):
+    run_check(fake_hip, "strided-few-channels")
+
+
 def test_layers_with_weights_that_are_not_finite_multiply_no_absent_neighbours(fake_hip):
     run_check(fake_hip, "weights-not-finite")
 
