@@ -412,7 +412,7 @@ def check_shared_launches():
         assert len(shared(frame(layers, dtype))) == n, (len(layers), dtype)
 
 
-def gemm_kernel(cin, cout, rows, dtype, weight=0.0):
+def gemm_kernel(cin, cout, rows, dtype, weight=0.0, out_dtype=None):
     """The kernel that multiplies in a SubM layer of so many rows, `weight` being one of its weights and the others 0 (nothing runs: the
     addresses are read by nobody)."""
     d = D.SubmConv3dDesc()
@@ -424,7 +424,7 @@ def gemm_kernel(cin, cout, rows, dtype, weight=0.0):
     assert L.sessd_submconv3d_create(C.byref(d), w.ctypes.data, C.byref(h)) == 0, L.sessd_last_error()
     ins = (D.TensorDesc * 3)(D.TensorDesc.make((1, rows, cin), dtype), D.TensorDesc.make((1, rows, 4), D.SESSD_INT32),
                              D.TensorDesc.make((1,), D.SESSD_INT32))
-    outs = (D.TensorDesc * 1)(D.TensorDesc.make((1, rows, cout), dtype))
+    outs = (D.TensorDesc * 1)(D.TensorDesc.make((1, rows, cout), dtype if out_dtype is None else out_dtype))
     assert L.sessd_submconv3d_configure(h, ins, 3, outs, 1) == 0, L.sessd_last_error()
     take_log()
     assert L.sessd_submconv3d_enqueue_shared(h, ins, outs, (C.c_void_p * 3)(4096, 8192, 12288), (C.c_void_p * 1)(16384), 20480, None) == 0
@@ -445,7 +445,8 @@ def check_row_limits():
 
 
 def check_weights_not_finite():
-    """FP16 layers run on the kernels that multiply an absent neighbour as a row of zeros only where all weights are finite as halves."""
+    """FP16 layers, and FP32 ones with few channels, run on the kernels that multiply an absent neighbour as a row of zeros only where all
+    weights are finite as halves."""
     f32, f16 = D.SESSD_FLOAT, D.SESSD_HALF
     for cin, cout in ((16, 16), (16, 32), (32, 32), (32, 64), (64, 64), (64, 128), (128, 128)):
         own = "conv_tile" if cin >= 64 else "conv_tall"
@@ -454,6 +455,13 @@ def check_weights_not_finite():
         for weight in (65520.0, -1e6, np.inf, -np.inf, np.nan):
             assert "conv_wide" in gemm_kernel(cin, cout, 9000, f16, weight), (cin, cout, weight)
             assert "conv_wide" in gemm_kernel(cin, cout, 9000, f32, weight), (cin, cout, weight)
+    for cin, cout, out in ((4, 16, f32), (4, 32, f32), (16, 16, f32), (4, 16, f16), (4, 32, f16)):
+        for weight in (0.0, 65504.0, -65519.0, 1e-30):
+            assert "conv_tall" in gemm_kernel(cin, cout, 9000, f32, weight, out), (cin, cout, out, weight)
+        for weight in (65520.0, -1e6, np.inf, -np.inf, np.nan):
+            assert "conv_wide" in gemm_kernel(cin, cout, 9000, f32, weight, out), (cin, cout, out, weight)
+    for cin, cout in ((16, 32), (32, 32)):
+        assert "conv_wide" in gemm_kernel(cin, cout, 9000, f32), (cin, cout)
 
 
 def check_strided_few_channels():

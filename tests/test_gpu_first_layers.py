@@ -79,11 +79,34 @@ def test_layers_that_share_launches_with_passes(name, dtype):
             assert (rows[pipe.layer_count(l):] == shift).all(), (cells, l)
 
 
+@pytest.mark.parametrize("name,dtype", [("two", "fp32"), ("two", "fp16"), ("wide", "fp16")])
+@pytest.mark.parametrize("cells", [16385, 40000])
+def test_layers_that_share_launches_with_passes_in_several_rounds(name, dtype, cells):
+    """A workgroup of these launches has four waves of 16 rows: with more than 16 384 rows on 256 units it goes on to a second round, with 40 000 to
+    a third.  Tensors for 50 000 points."""
+    layers, half, cap = BACKBONES[name], dtype == "fp16", 45000
+    W = B.random_weights(layers, seed=5, w_std=0.1)
+    if half:
+        W = B.Weights([O.round_to_half(w) for w in W.w], W.scale, W.shift)
+    pipe = api.Pipeline(layers, W, 50000, cap, feature_dtype=dtype, share_rulebooks=True, skip_pad_rows=False, use_graph=True, overlap_streams=True)
+    pts = points_in(cells, cells)
+    p, n = points_input(pts, 50000)
+    dense, stream = pipe.new_dense(), torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        for _ in range(3):
+            pipe.enqueue(p, n, dense, stream)
+    stream.synchronize()
+    assert pipe.layer_count(0) == cells
+    check_frame_against_oracle(pipe, dense, pts, layers, W, cap, cap, half, B.DENSE_SIZE_XYZ)
+
+
 @pytest.mark.parametrize("pad", [False, True])
 @pytest.mark.parametrize("cin,cout", [(4, 16), (4, 32), (16, 16)])
 def test_fp32_layers_with_few_channels(cin, cout, pad):
-    """FP32 3x3x3 layers with all weights in LDS: the orders of sums and the last rows of a block.  1e-4 of an element, and in the norm
-    no further from 64-bit sums than twice a sum of FP32 products one after the other."""
+    """FP32 3x3x3 layers with all weights in LDS: the orders of sums and the last rows of a block.  1e-4 of an element, and in the norm, with
+    thousands of rows, no further from 64-bit sums than the oracle's, which adds each offset's products by themselves: here 0.76 to 0.93 of its
+    distance, one chain over all products 1.06 to 2.6 from 8 193 rows up, a chain for each channel of a piece 1.18 and 1.34 with 16 channels and
+    16 401 and 30 000 rows."""
     rng = np.random.default_rng(cin * cout)
     grid = (12, 60, 70)
     for n in (1, 16, 31, 8192, 8193, 16384, 16401, 30000):
@@ -100,7 +123,7 @@ def test_fp32_layers_with_few_channels(cin, cout, pad):
         want = O.gather_gemm_scatter(fbuf, w, pairs, num, mv)[:n]
         assert_features_close(out[:n], want, RTOL_FP32, "%d rows" % n, abs_sum=abs_sum_of(fbuf, w, pairs, num, mv)[:n])
         exact = sums_in_64_bits(feat, w, pairs, num, n)
-        assert np.linalg.norm(out[:n] - exact) <= 2 * np.linalg.norm(want - exact) + 1e-30
+        assert np.linalg.norm(out[:n] - exact) <= (1 if n > 1000 else 2) * np.linalg.norm(want - exact) + 1e-30
         if pad:
             assert not out[n:].any()
 
