@@ -203,12 +203,12 @@ bool gemm_cuts_own_tiles(int K, int cin, int cout, int in_type, int out_type) {
 }
 
 int launch_gather_gemm(const GemmArgs& a, hipStream_t stream) {
-    if (!a.force_valu) {  // FP16 layers with weights that are finite as halves: 3x3x3 and 3x1x1 from 64 channels up, 3x3x3 with 16 or 32
+    if (!a.force_valu) {  // weights that are finite as halves: FP16 3x3x3 and 3x1x1 from 64 channels up; 3x3x3 in FP16 with 16 or 32, in FP32 with few
         int rc = launch_tile(a, stream);
         if (rc == SESSD_E_UNSUPPORTED) rc = launch_tall(a, stream);
         if (rc != SESSD_E_UNSUPPORTED) return rc;
     }
-    if (!a.force_valu) {  // FP32, an FP16 pipeline's first layer, FP16 layers that the two above do not take
+    if (!a.force_valu) {  // FP32 and FP16 layers that the two above do not take
         const int rc = launch_wide(a, stream);
         if (rc != SESSD_E_UNSUPPORTED) return rc;  // launched (or failed for good)
     }

@@ -14,7 +14,7 @@
 //     In FP32 an MFMA takes one channel of each of the four offsets.  Rows are requested two steps (eight offsets) ahead, those of up to
 //     32 bytes three, all of them by straight-line code: the compiler's waits are exact.
 //   * With few rows (up to four blocks a workgroup, 16 384 rows on 256 units; up to two, 8 192) two or four waves share a block and take
-//     every second or fourth step; their sums are added in LDS.
+//     every second or fourth step; their sums are added in LDS.  (Workgroups of four waves, coord.hip: 8 192 and 4 096 rows.)
 //   * W, the row count and, behind that, the lists are on their way together; the first rows are requested in front of the barrier.
 //   * The rows beyond the active ones are written by four waves of their own.
 // What bounds it from some 40 000 rows up are the requests for rows in four cache lookups a row (coalesced ones, with a 4 x 4
@@ -27,12 +27,20 @@
 // 16 198 rows 7.2 -> 3.3 and 8.1 -> 3.7, 60 000 rows 10.4 -> 4.9 and 11.9 -> 5.8; frames of 60 000 points 225.9 -> 215.7.
 // FP32, launches back to back, pair lists -> here: 4 -> 16 at 933 rows 4.7 -> 3.2 us, 16 569 6.5 -> 4.3, 41 489 9.3 -> 6.2, 92 422 16.0 -> 9.2; 4 -> 32
 // 5.3 -> 3.9, 8.2 -> 5.8, 11.0 -> 8.9, 21.0 -> 13.9; 16 -> 16 4.8 -> 3.7, 7.2 -> 6.8, 10.8 -> 10.1, 20.1 -> 16.8 (16 -> 32 would multiply
-// twelve times its pairs).  Distance from 64-bit sums at 41 489 rows 0.645e-7 -> 0.634e-7, 0.640e-7 -> 0.621e-7, 0.803e-7 -> 0.753e-7.
-// In a frame two of these layers share launches with passes over coordinates (coord.hip).
+// twelve times its pairs).  That is at a frame's sites, where up to a quarter of the neighbours is there.  With all of them 30 000 rows 10.7 -> 4.5, 13.0 -> 6.2,
+// 13.0 -> 7.3; without any 4 -> 16 6.1 -> 4.5, 60 000 rows 8.0 -> 6.8, but 4 -> 32 6.2 -> 6.2 and 8.3 -> 10.0, 16 -> 16 6.7 -> 7.1 and 8.7 -> 11.8: the host knows rows
+// and not neighbours.  Distance from 64-bit sums at 41 489 rows 0.645e-7 -> 0.634e-7, 0.640e-7 -> 0.621e-7, 0.803e-7 -> 0.753e-7, at 933 to 51 443 rows 0.56-0.66e-7 ->
+// 0.55-0.66e-7, 0.54-0.67e-7 -> 0.55-0.64e-7, 0.72-0.81e-7 -> 0.65-0.76e-7 (sites at random, 8 192 rows with a sixth of the neighbours, of a sum's per offset: 0.88 -> 0.92, 0.88 ->
+// 0.93, 0.93 -> 0.79; 30 000 rows 0.76 -> 0.76, 0.77 -> 0.77, 0.83 -> 0.78).
+// In a frame two of these layers share launches with passes over coordinates (coord.hip).  Frames on two streams in which they cannot, here / pair lists there:
+// three SubM layers in front 2 000 points 171.0 / 173.3 us, 20 000 260.7 / 257.6, 80 000 389.0 / 392.7, a SubM layer on a grid of its own 2 000 202.7 / 205.6, 20 000 283.6 /
+// 288.5, 80 000 423.4 / 427.9, on hashes 2 000 197.7 / 195.2, 20 000 291.1 / 290.9, FP16 60 000 points, nothing shared, 194.6 / 202.5.
 // The waves are eight because the coordinate passes beside them need registers (12: the same times, and 504 of 512 taken).
-// Summation order per output element: a wave's steps ascending, in a step the channels eight at a time; where waves share a block, to the
-// first one's sum those of the others, the last one's first.  Fixed for a row count and a grid, run-to-run identical; in a launch with more or
-// fewer rows, or on another number of compute units, the same row may be summed in another of the three orders.
+// Summation order per output element.  FP16: a wave's steps ascending, in a step the channels eight at a time.  FP32: a step has a sum for each of
+// the four channels of a 16-byte piece, over the pieces ascending, of four offsets at a time; (0 + 1) + (2 + 3) goes to one of two totals in turn (4 -> 16: of
+// four), and the totals are added two by two at the end.  Where waves share a block, to the first one's sum those of the others, the last one's
+// first.  Fixed for a row count and a grid, run-to-run identical; in a launch with more or fewer rows, or on another number of compute units or of
+// waves a workgroup, the same row may be summed in another of the three orders.
 // (The ring of conv_tile.hip, faster from 64 channels up, has too little work per row here.)
 #include "conv_tall.h"
 
@@ -89,7 +97,7 @@ bool tall_takes(const GemmArgs& a) {
     if ((size_t)a.max_voxels * (tall::KC * sizeof(int32_t)) >= tall::kOutOfRange) return false;
     if (a.in_type == SESSD_HALF) return a.out_type == SESSD_HALF && gemm_runs_tall(a.K, a.cin, a.cout);
     if (a.cin == 4) return a.cout == 16 || a.cout == 32;
-    // (a strided layer's rows have three or four neighbours: the pair lists are short.  A call, rulebook included, here / there, at a frame's sites
+    // (a strided layer's rows have one to three neighbours at a frame's sites, a SubM layer's up to seven: the pair lists are short.  A call, rulebook included, here / there, at a frame's sites
     // 1 000 rows 21.2 / 22.7 us, 5 000 24.6 / 25.4, 12 000 28.3 / 28.1, 27 585 36.9 / 35.2, 49 642 47.4 / 45.8, 92 422 69.2 / 64.9; isolated ones 5 000 26.7 / 26.6,
     // 60 000 79.4 / 69.7.  The host knows the rows that the tensors hold.  4 -> 16 at 27 585 32.9 / 34.3, 92 422 62.0 / 64.9, isolated 60 000 70.7 / 69.6)
     return a.out_type == SESSD_FLOAT && a.cin == 16 && a.cout == 16 && (!a.strided || a.max_voxels <= kFewStridedRows);

@@ -1,5 +1,5 @@
-// conv_wide.hip -- gather-GEMM of the FP32 layers, of the FP16 layers that conv_tile.hip and conv_tall.hip do not take (kernel
-// volumes other than theirs, weights that are not finite) and of an FP16 pipeline's first layer.
+// conv_wide.hip -- gather-GEMM of the FP32 layers from 16 -> 32 up and of all that conv_tile.hip and conv_tall.hip do not take (kernel
+// volumes other than theirs, weights that are not finite as halves, large strided FP32 layers 16 -> 16).
 //
 //     out[o][:] = epilogue( sum_k  in[nbr[k][o]][:] @ W[k] )
 //
@@ -507,8 +507,8 @@ __device__ __forceinline__ void direct_sum(const float* __restrict__ in, const f
 
 // The number of workgroups and what is done to the sums, in one argument that is in a register when the kernel starts.  As arguments of their own
 // scale, shift and relu were compared with 0 in front of the loops (no store can change them), which was a trip to memory between the cuts and the
-// requests for the lists: frames of 2 000 points 167.0 -> 164.3 us, 5 000 189.0 -> 187.6, 20 000 255.9 -> 254.9, 80 000 381 -> 380 (copies of the
-// pointers inside the loops instead: scalar registers spill, 2 000 points 1.014x).
+// requests for the lists: frames of 2 000 points 167.0 -> 164.3 us, 5 000 189.0 -> 187.6; 20 000 255.9 -> 254.9 and 80 000 381 -> 380, which is within
+// what runs of one side differ by (copies of the pointers inside the loops instead: scalar registers spill, 2 000 points 1.014x).
 constexpr unsigned kUnitsMask = 0xffffffu, kHasScale = 1u << 24, kHasShift = 2u << 24, kRelu = 4u << 24;
 
 // DENSE: the epilogue also scatters the rows into a dense tensor (the layer in front of sparse2Dense).  PAD: the rows beyond the

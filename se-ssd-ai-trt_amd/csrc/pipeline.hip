@@ -268,8 +268,8 @@ struct Pipeline {
 
     // One frame.  The rulebooks depend only on coordinates, the GEMMs on rulebooks + features.  The coordinate chain
     // (coord.h) is  vg_insert | vg_flags | vg_finalize + insert 1 | then per stage i: flags i+1 + lookups on stage i |
-    // number i+1 + insert i+2 + tile cuts of those rulebooks.  With `aux`, everything behind the lookups on the voxels
-    // runs there, and the GEMM chain waits for the passes its layers' rulebooks come from (one by one at first, further on for
+    // number i+1 + insert i+2 + tile cuts of those rulebooks.  With `aux`, everything behind the lookups on the voxels, or behind the
+    // passes that share launches with the first layers, runs there, and the GEMM chain waits for the passes its layers' rulebooks come from (one by one at first, further on for
     // some at once: wait_for), so that the passes of later layers overlap the GEMMs of earlier ones; under stream capture
     // that becomes two branches of the graph.
     int enqueueFrame(const void* points, const void* points_size, void* dense, hipStream_t stream) {

@@ -337,11 +337,13 @@ def check_own_waits():
     x, y, z = own_grid[1].out_shape
     own_grid[1].out_shape = (x + 1, y, z)
 
-    def awaited(layers, points):  # by each layer, lookups that it is ordered behind, and all waits of the frame
-        log = overlapped_frame(layers, D.SESSD_FLOAT, max_points=points)
+    def awaited(layers, points, dtype=D.SESSD_FLOAT):  # by each layer, lookups that it is ordered behind, and all waits of the frame
+        log = overlapped_frame(layers, dtype, max_points=points)
         return passes_before_gemms(log), sum(l[0] == "wait" for l in log)
 
     assert awaited(ref, 500)[1] == awaited(ref, 10000)[1] == awaited(ref, 10001)[1] + 1 == awaited(ref, 80000)[1] + 1
+    for layers in (ref, wide):  # (FP16 layers need no cuts)
+        assert awaited(layers, 500, D.SESSD_HALF) == awaited(layers, 10001, D.SESSD_HALF)
     for layers in (wide, own_grid):
         assert awaited(layers, 500) == awaited(layers, 10000) == awaited(layers, 10001), len(layers)
     FAKE.fake_largest_allocation(300 << 20)  # (no kept table of the voxels)

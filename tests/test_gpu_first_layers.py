@@ -32,7 +32,7 @@ BACKBONES = {
     "one": [subm(4, 16)] + strided(16, 32, 64, 64),                                # pass 2 alone
     "two": [subm(4, 16), subm(16, 16)] + strided(16, 32, 64, 64),                  # passes 1 and 2 with a layer each
     "three": [subm(4, 16), subm(16, 16), subm(16, 16)] + strided(16, 32, 64, 64),  # a layer behind them
-    "wide": [subm(4, 32), subm(32, 32)] + strided(32, 64, 64, 64),                 # pass 1 with a layer
+    "wide": [subm(4, 32), subm(32, 32)] + strided(32, 64, 64, 64),                 # FP16 as "two"; FP32 on one stream pass 1 with a layer
     "own grid": [subm(4, 16), subm(16, 16, (1409, 1600, 41))] + strided(16, 32, 64, 64),
 }
 
